@@ -1,6 +1,6 @@
 """MI355X-native quantized-inference operators behind PyTorch's own op names.
 
-Importing this package loads two in-tree native libraries:
+Importing this package loads three in-tree native libraries:
 
   libtmq.so        hand-written HIP kernels for gfx950 behind the C ABI of
                    ``include/tmq.h`` (quantize / dequantize / min-max, int8 MFMA
@@ -10,6 +10,7 @@ Importing this package loads two in-tree native libraries:
                    ``torch.quantize_per_tensor_dynamic``, ``Tensor.dequantize`` and
                    ``torch.ops.quantized.{linear,linear_relu,linear_prepack,
                    conv2d,conv2d_relu,conv2d_prepack}`` for tensors on the GPU
+  _fastcall.so     native call paths of ``torch.ops.quantized.*`` with packed weights
 
 so that a model written against ``torch.ops.quantized.*`` runs unchanged (the
 counterpart of ``import torch_musa`` for this operator path; reference:
@@ -18,6 +19,7 @@ library is missing the import fails.
 """
 from __future__ import annotations
 
+import functools
 import os
 import warnings
 
@@ -26,8 +28,9 @@ import torch
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_KERNELS = os.path.join(_PKG, "libtmq.so")
 LIB_ATEN = os.path.join(_PKG, "libtmq_aten.so")
+LIB_FASTCALL = os.path.join(_PKG, "_fastcall.so")
 
-__all__ = ["LIB_KERNELS", "LIB_ATEN", "is_loaded", "load", "quantized_device", "quantized_modules_to",
+__all__ = ["LIB_KERNELS", "LIB_ATEN", "LIB_FASTCALL", "is_loaded", "load", "quantized_device", "quantized_modules_to",
            "plain_weight_cache_clear", "plain_weight_cache_counters", "plain_weight_cache_stats",
            "plain_weight_cache_set_max_bytes"]
 
@@ -39,7 +42,7 @@ def load() -> None:
     global _loaded
     if _loaded:
         return
-    for lib in (LIB_KERNELS, LIB_ATEN):
+    for lib in (LIB_KERNELS, LIB_ATEN, LIB_FASTCALL):
         if not os.path.exists(lib):
             raise ImportError(
                 f"{lib} is missing: build the native libraries with "
@@ -49,9 +52,26 @@ def load() -> None:
         # is intended; the dispatcher warns about it once
         warnings.filterwarnings("ignore", message=".*Overriding a previously registered kernel.*")
         torch.ops.load_library(LIB_ATEN)
+    _install_call_paths()
     from . import ao  # the fused SiLU convolution modules, under the reference's torch.ao names
     ao.register()
     _loaded = True
+
+
+def _install_call_paths() -> None:
+    """Give the operator objects ``torch.ops.quantized.{linear, conv2d, ...}`` their native call path.
+
+    The objects stay what they are (same identity, same attributes, still instances of PyTorch's
+    operator class); only calling one goes through ``_fastcall`` first, which hands every call
+    that is not of the plain positional form back to PyTorch's own ``__call__``.
+    """
+    from . import _fastcall
+
+    for name in _fastcall.names():
+        packet = getattr(torch.ops.quantized, name)
+        base = type(packet)
+        native = _fastcall.make(name, functools.partial(base.__call__, packet))
+        packet.__class__ = type(base.__name__, (base,), {"__call__": native, "__module__": base.__module__})
 
 
 def is_loaded() -> bool:

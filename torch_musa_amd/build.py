@@ -4,6 +4,7 @@
   libtmq_bench.so measurement probe behind include/tmq_bench.h (bench.py only)
   libtmq_aten.so  ATen registrations (TORCH_LIBRARY_IMPL + dispatch stubs)
                   that call libtmq.so
+  _fastcall.so    Python callables of the packed-weight operators (host code only)
 
     python torch_musa_amd/build.py [--kernels-only] [--verbose]
 
@@ -25,12 +26,14 @@ OBJ = os.path.join(PKG, "build")
 LIB_KERNELS = os.path.join(PKG, "libtmq.so")
 LIB_ATEN = os.path.join(PKG, "libtmq_aten.so")
 LIB_BENCH = os.path.join(PKG, "libtmq_bench.so")
+LIB_FASTCALL = os.path.join(PKG, "_fastcall.so")
 ARCH = "gfx950"
 
 KERNEL_SOURCES = ["kernels/quantize.hip", "kernels/linear.hip", "kernels/conv2d.hip",
                   "kernels/elementwise.hip"]
 BENCH_SOURCES = ["bench/bench_kernels.hip"]
 ATEN_SOURCES = ["aten/register.cpp"]
+FASTCALL_SOURCE = "python/fastcall.cpp"
 
 # -ffp-contract=off: the requantisation epilogue and the quantizer must round
 # after every fp32 operation, as the CPU ops they mirror do.
@@ -279,11 +282,30 @@ def build_aten(verbose=False):
     return LIB_ATEN
 
 
+def build_fastcall(verbose=False):
+    """A plain CPython extension: the host compiler, as PyTorch's own bindings are built."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension as ce
+
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = ["-I", sysconfig.get_paths()["include"]]
+    for d in ce.include_paths():
+        inc += ["-isystem", d]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + inc
+         + [os.path.join(CSRC, FASTCALL_SOURCE), "-o", LIB_FASTCALL, "-L", tlib, "-ltorch_python", "-ltorch",
+            "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{tlib}"], verbose)
+    return LIB_FASTCALL
+
+
 def build_all(verbose=False, kernels_only=False):
-    out = [build_kernels(verbose), build_bench(verbose)]
-    if not kernels_only and all(os.path.exists(os.path.join(CSRC, s)) for s in ATEN_SOURCES):
-        out.append(build_aten(verbose))
-    return out
+    if kernels_only:
+        return [build_kernels(verbose), build_bench(verbose)]
+    with ThreadPoolExecutor(max_workers=2) as ex:   # host code only: compiles beside the kernels
+        fastcall = ex.submit(build_fastcall, verbose)
+        return [build_kernels(verbose), build_bench(verbose), build_aten(verbose), fastcall.result()]
 
 
 if __name__ == "__main__":
