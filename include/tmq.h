@@ -118,6 +118,20 @@ int tmq_quantize_per_tensor_dev(const float* x, void* q, int64_t n,
 int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int64_t n, int q_signed,
                                         int reduce_range, int rounding, tmq_qparams* qparams,
                                         void* workspace, size_t workspace_bytes, tmq_stream_t stream);
+/* What a kernel tells the host before it ends: pinned host memory that the device
+ * can write (hipHostMalloc), 16-byte aligned.  A word is complete once its upper
+ * half is the ticket of the call -- any number that differs from the one this
+ * memory was last used with. */
+typedef struct tmq_host_report {
+  uint64_t word[2];
+} tmq_host_report;
+/* The same, and the range goes to the host as soon as it is known, before the
+ * codes are written: word[0] and word[1] carry the bits of the fp32 minimum and
+ * maximum (NaNs are passed over; +inf and -inf if there is nothing else).  n > 0. */
+int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, int q_signed,
+                                           int reduce_range, int rounding, tmq_qparams* qparams,
+                                           void* workspace, size_t workspace_bytes,
+                                           tmq_host_report* report, uint32_t ticket, tmq_stream_t stream);
 /* Host-side ChooseQuantizationParams, same arithmetic (pure CPU, no GPU call). */
 int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
                             double* scale, int32_t* zero_point);
@@ -154,6 +168,25 @@ int tmq_dequantize_per_channel_float_qparams(const void* q, float* r, int64_t ou
                                              int64_t channels, int64_t inner,
                                              const float* scales, const float* zero_points,
                                              int q_signed, tmq_stream_t stream);
+
+/* The four functions above as one, with the range check of the zero points on the
+ * device: where `report` is given, word[0] carries 1 if any zero point lies outside
+ * the codes' range, else 0, a few microseconds after the kernel starts.  scales /
+ * zero_points: double / int64, or float / float with float_qparams.  With a report
+ * the tensor must have elements. */
+typedef struct tmq_per_channel_desc {
+  int32_t dequantize; /* 0: fp32 -> codes, 1: codes -> fp32 */
+  int32_t float_qparams;
+  int32_t q_signed;
+  uint32_t ticket;
+  void* fp32;
+  void* codes;
+  int64_t outer, channels, inner;
+  const void* scales;
+  const void* zero_points;
+  tmq_host_report* report; /* or NULL */
+} tmq_per_channel_desc;
+int tmq_per_channel(const tmq_per_channel_desc* desc, tmq_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * quantized::linear weights.

@@ -30,7 +30,9 @@
 #include <torch/library.h>
 
 #include <array>
+#include <condition_variable>
 #include <cstdlib>
+#include <cstring>
 #include <list>
 #include <memory>
 #include <mutex>
@@ -108,6 +110,94 @@ at::Tensor attach_linear_workspace(tmq_linear_desc& d, const at::Tensor& like) {
   return ws;
 }
 
+// What a kernel reports to the host before it ends (tmq_host_report): slots in one page of
+// pinned memory, each held by one call at a time, so that threads and streams do not share
+// one.  A call waits by reading its slot, not for the stream: work queued behind the
+// reporting block goes on meanwhile.
+class HostReport {
+ public:
+  HostReport() {
+    Pool& p = pool();
+    std::unique_lock<std::mutex> lock(p.mu);
+    p.given_back.wait(lock, [&] { return !p.free.empty(); });
+    slot_ = p.free.back();
+    p.free.pop_back();
+    if (++p.ticket == 0) ++p.ticket;  // (fresh memory is zero)
+    ticket_ = p.ticket;
+  }
+  ~HostReport() {
+    if (pending_) return;  // the device may still write to it: not handed out again
+    Pool& p = pool();
+    {
+      std::lock_guard<std::mutex> lock(p.mu);
+      p.free.push_back(slot_);
+    }
+    p.given_back.notify_one();
+  }
+  HostReport(const HostReport&) = delete;
+  HostReport& operator=(const HostReport&) = delete;
+
+  tmq_host_report* memory() { return slot_; }
+  uint32_t ticket() const { return ticket_; }
+  void queued() { pending_ = true; }  // a kernel that will write to the slot is on its stream
+  // Payload of word `i`.
+  uint32_t wait(int i, const c10::hip::HIPStream& stream, const char* what) {
+    const volatile uint64_t* word = &slot_->word[i];
+    for (int spin = 0; spin < kSpins; ++spin) {
+      const uint64_t v = *word;
+      if (static_cast<uint32_t>(v >> 32) == ticket_) return static_cast<uint32_t>(v);
+      __builtin_ia32_pause();
+    }
+    stream.synchronize();  // a long queue ahead of the kernel (or an error, which this raises)
+    const uint64_t v = *word;
+    TORCH_CHECK(static_cast<uint32_t>(v >> 32) == ticket_, what, ": the kernel ended without its report");
+    return static_cast<uint32_t>(v);
+  }
+  void done() { pending_ = false; }
+
+ private:
+  static constexpr int kSlots = 64;     // calls that wait at the same time; more of them queue for a slot
+  static constexpr int kSpins = 20000;  // about a millisecond
+  struct Pool {
+    std::mutex mu;
+    std::condition_variable given_back;
+    std::vector<tmq_host_report*> free;
+    uint32_t ticket = 0;
+    Pool() {
+      void* page = nullptr;
+      TORCH_CHECK(hipHostMalloc(&page, kSlots * kStride, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess,
+                  "hipHostMalloc failed");
+      std::memset(page, 0, kSlots * kStride);
+      for (int i = 0; i < kSlots; ++i)
+        free.push_back(reinterpret_cast<tmq_host_report*>(static_cast<char*>(page) + i * kStride));
+    }
+  };
+  static constexpr size_t kStride = 64;  // a cache line each
+  static Pool& pool() {
+    static Pool* p = new Pool;  // for the life of the process: kernels may hold its address at exit
+    return *p;
+  }
+  tmq_host_report* slot_;
+  uint32_t ticket_;
+  bool pending_ = false;
+};
+
+bool stream_is_capturing(const c10::hip::HIPStream& s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s.stream(), &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;  // unknown: take the safe side
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+// Operators that hand a value of the device to the host cannot be recorded into a graph.
+c10::hip::HIPStream stream_for_report(const at::Tensor& t, const char* what) {
+  const auto stream = c10::hip::getCurrentHIPStream(t.device().index());
+  TORCH_CHECK(!stream_is_capturing(stream), what,
+              ": operation not permitted when stream is capturing (the host needs a value from the device)");
+  return stream;
+}
+
 bool is_signed_qtype(c10::ScalarType t, const char* what) {
   TORCH_CHECK(t == c10::kQInt8 || t == c10::kQUInt8, what, ": only QInt8 and QUInt8 are supported, got ",
               toString(t));
@@ -157,99 +247,64 @@ ChannelView channel_view(const at::Tensor& t, int64_t axis) {
   return v;
 }
 
-struct ChannelParams {
-  at::Tensor scales, zps;
-};
-
-ChannelParams channel_params(const at::Tensor& like, const at::Tensor& scales, const at::Tensor& zps,
-                             int64_t channels, bool sgn) {
-  TORCH_CHECK(scales.numel() == channels && zps.numel() == channels,
+// The per-channel conversions.  The zero points are checked as the reference does
+// (check_zero_points_musa, AffineQuantizer.mu:23-33), by a block of the conversion itself:
+// the call returns once that block has reported, with the conversion still running.
+void convert_per_channel(const at::Tensor& codes, const at::Tensor& fp32, const at::Tensor& scales,
+                         const at::Tensor& zps, int64_t axis, bool dequantize, bool float_qparams, const char* what) {
+  const bool sgn = is_signed_qtype(codes.scalar_type(), what);
+  TORCH_CHECK(fp32.scalar_type() == at::kFloat, what, ": the unquantized side is a Float tensor");
+  const OnDeviceOf on(codes);
+  const ChannelView v = channel_view(codes, axis);
+  TORCH_CHECK(scales.numel() == v.channels && zps.numel() == v.channels,
               "per-channel scales / zero points must have one entry per channel");
-  ChannelParams p;
-  p.scales = scales.to(like.device(), at::kDouble).contiguous();
-  p.zps = zps.to(like.device(), at::kLong).contiguous();
-  // same range check (and the same host synchronisation) as the reference's
-  // check_zero_points_musa, AffineQuantizer.mu:23-33
-  const int64_t qmin = sgn ? -128 : 0, qmax = sgn ? 127 : 255;
-  if (channels > 0) {
-    const bool bad = p.zps.lt(qmin).logical_or(p.zps.gt(qmax)).any().item<bool>();
-    TORCH_CHECK(!bad, "per-channel zero point outside the range of the quantized dtype");
+  const at::Tensor sc = scales.to(codes.device(), float_qparams ? at::kFloat : at::kDouble).contiguous();
+  const at::Tensor zp = zps.to(codes.device(), float_qparams ? at::kFloat : at::kLong).contiguous();
+  if (codes.numel() == 0) {
+    const int64_t qmin = sgn ? -128 : 0, qmax = sgn ? 127 : 255;
+    TORCH_CHECK(v.channels == 0 || !zp.lt(qmin).logical_or(zp.gt(qmax)).any().item<bool>(),
+                "per-channel zero point outside the range of the quantized dtype");
+    return;
   }
-  return p;
+  const auto stream = stream_for_report(codes, what);
+  HostReport report;
+  tmq_per_channel_desc d{};
+  d.dequantize = dequantize;
+  d.float_qparams = float_qparams;
+  d.q_signed = sgn;
+  d.ticket = report.ticket();
+  d.fp32 = fp32.data_ptr();
+  d.codes = codes.data_ptr();
+  d.outer = v.outer;
+  d.channels = v.channels;
+  d.inner = v.inner;
+  d.scales = sc.const_data_ptr();
+  d.zero_points = zp.const_data_ptr();
+  d.report = report.memory();
+  check_status(tmq_per_channel(&d, reinterpret_cast<tmq_stream_t>(stream.stream())), "tmq_per_channel");
+  report.queued();
+  const bool bad = report.wait(0, stream, what) != 0;
+  report.done();
+  TORCH_CHECK(!bad, "per-channel zero point outside the range of the quantized dtype");
 }
 
 void quantize_per_channel_stub(const at::Tensor& r, at::Tensor& q, const at::Tensor& scales,
                                const at::Tensor& zps, int64_t axis) {
-  const bool sgn = is_signed_qtype(q.scalar_type(), "quantize_tensor_per_channel_affine");
-  TORCH_CHECK(r.scalar_type() == at::kFloat, "quantize_tensor_per_channel_affine expects a Float tensor");
-  const OnDeviceOf on(q);
-  const ChannelView v = channel_view(q, axis);
-  const ChannelParams p = channel_params(q, scales, zps, v.channels, sgn);
-  check_status(tmq_quantize_per_channel(cptr<float>(r), q.data_ptr(), v.outer, v.channels, v.inner,
-                                        cptr<double>(p.scales), cptr<int64_t>(p.zps),
-                                        sgn, current_stream(q)),
-               "tmq_quantize_per_channel");
+  convert_per_channel(q, r, scales, zps, axis, false, false, "quantize_tensor_per_channel_affine");
 }
-
 void dequantize_per_channel_stub(const at::Tensor& q, at::Tensor& r, const at::Tensor& scales,
                                  const at::Tensor& zps, int64_t axis) {
-  const bool sgn = is_signed_qtype(q.scalar_type(), "dequantize_tensor_per_channel_affine");
-  TORCH_CHECK(r.scalar_type() == at::kFloat, "dequantize_tensor_per_channel_affine writes a Float tensor");
-  const OnDeviceOf on(q);
-  const ChannelView v = channel_view(q, axis);
-  const ChannelParams p = channel_params(q, scales, zps, v.channels, sgn);
-  check_status(tmq_dequantize_per_channel(q.data_ptr(), mptr<float>(r), v.outer, v.channels, v.inner,
-                                          cptr<double>(p.scales), cptr<int64_t>(p.zps),
-                                          sgn, current_stream(q)),
-               "tmq_dequantize_per_channel");
+  convert_per_channel(q, r, scales, zps, axis, true, false, "dequantize_tensor_per_channel_affine");
 }
-
 // Float scales and float zero points (qscheme per_channel_affine_float_qparams,
-// AffineQuantizer.mu:259-336), with the reference's range check of the zero
-// points (check_zero_points_musa, :23-33) and its host synchronisation.
-struct FloatChannelParams {
-  at::Tensor scales, zps;
-};
-
-FloatChannelParams float_channel_params(const at::Tensor& like, const at::Tensor& scales,
-                                        const at::Tensor& zps, int64_t channels, bool sgn) {
-  TORCH_CHECK(scales.numel() == channels && zps.numel() == channels,
-              "per-channel scales / zero points must have one entry per channel");
-  FloatChannelParams p;
-  p.scales = scales.to(like.device(), at::kFloat).contiguous();
-  p.zps = zps.to(like.device(), at::kFloat).contiguous();
-  const int64_t qmin = sgn ? -128 : 0, qmax = sgn ? 127 : 255;
-  if (channels > 0) {
-    const bool bad = p.zps.lt(qmin).logical_or(p.zps.gt(qmax)).any().item<bool>();
-    TORCH_CHECK(!bad, "per-channel zero point outside the range of the quantized dtype");
-  }
-  return p;
-}
-
+// AffineQuantizer.mu:259-336).
 void quantize_per_channel_float_qparams_stub(const at::Tensor& r, at::Tensor& q, const at::Tensor& scales,
                                              const at::Tensor& zps, int64_t axis) {
-  const bool sgn = is_signed_qtype(q.scalar_type(), "quantize_tensor_per_channel_float_qparams");
-  TORCH_CHECK(r.scalar_type() == at::kFloat, "quantize_tensor_per_channel_float_qparams expects a Float tensor");
-  const OnDeviceOf on(q);
-  const ChannelView v = channel_view(q, axis);
-  const FloatChannelParams p = float_channel_params(q, scales, zps, v.channels, sgn);
-  check_status(tmq_quantize_per_channel_float_qparams(cptr<float>(r), q.data_ptr(), v.outer, v.channels,
-                                                      v.inner, cptr<float>(p.scales), cptr<float>(p.zps), sgn,
-                                                      current_stream(q)),
-               "tmq_quantize_per_channel_float_qparams");
+  convert_per_channel(q, r, scales, zps, axis, false, true, "quantize_tensor_per_channel_float_qparams");
 }
-
 void dequantize_per_channel_float_qparams_stub(const at::Tensor& q, at::Tensor& r, const at::Tensor& scales,
                                                const at::Tensor& zps, int64_t axis) {
-  const bool sgn = is_signed_qtype(q.scalar_type(), "dequantize_tensor_per_channel_float_qparams");
-  TORCH_CHECK(r.scalar_type() == at::kFloat, "dequantize_tensor_per_channel_float_qparams writes a Float tensor");
-  const OnDeviceOf on(q);
-  const ChannelView v = channel_view(q, axis);
-  const FloatChannelParams p = float_channel_params(q, scales, zps, v.channels, sgn);
-  check_status(tmq_dequantize_per_channel_float_qparams(q.data_ptr(), mptr<float>(r), v.outer, v.channels,
-                                                        v.inner, cptr<float>(p.scales), cptr<float>(p.zps), sgn,
-                                                        current_stream(q)),
-               "tmq_dequantize_per_channel_float_qparams");
+  convert_per_channel(q, r, scales, zps, axis, true, true, "dequantize_tensor_per_channel_float_qparams");
 }
 
 // The stub objects live in libtorch; overriding their GPU slot at load time is
@@ -299,37 +354,48 @@ at::Tensor dequantize_run(const at::Tensor& self) {
 }
 
 // ---------------------------------------------------------------------------
-// aten::quantize_per_tensor_dynamic: one min/max pass, one small copy to the
-// host (the quantizer object keeps the scale on the host), one quantize pass.
+// aten::quantize_per_tensor_dynamic: range, parameters and codes in one chain on the
+// stream.  The quantizer object keeps the scale on the host, so the host waits for the
+// range, which the chain reports as soon as it is known.
 // ---------------------------------------------------------------------------
 at::Tensor quantize_per_tensor_dynamic(const at::Tensor& self, at::ScalarType dtype, bool reduce_range) {
+  const char* what = "quantize_per_tensor_dynamic";
   TORCH_CHECK(dtype == at::kQInt8 || dtype == at::kQUInt8 || dtype == at::kHalf,
               "dtype ", dtype, " not supported");
   const OnDeviceOf on(self);
-  at::Tensor x = self.contiguous();
-  if (dtype == at::kHalf) return x.to(at::kHalf);
-  if (x.scalar_type() != at::kFloat) x = x.to(at::kFloat);
+  if (dtype == at::kHalf) return self.contiguous().to(at::kHalf);
+  // in the tensor's own memory format, which the result keeps
+  const auto fmt = self.suggest_memory_format();
+  const at::Tensor x = (self.scalar_type() == at::kFloat ? self : self.to(at::kFloat)).contiguous(fmt);
   if (reduce_range && at::globalContext().qEngine() == at::QEngine::QNNPACK) reduce_range = false;
   const bool sgn = dtype == at::kQInt8;
-  float mm[2] = {0.f, 0.f};
-  if (x.numel() > 0) {
-    at::Tensor ws = at::empty({static_cast<int64_t>(tmq_minmax_workspace_bytes(x.numel()))},
-                              x.options().dtype(at::kByte));
-    at::Tensor out = at::empty({2}, x.options());
-    check_status(tmq_minmax(cptr<float>(x), x.numel(), mptr<float>(out), ws.data_ptr(),
-                            static_cast<size_t>(ws.numel()), current_stream(x)),
-                 "tmq_minmax");
-    const at::Tensor host = out.cpu();
-    mm[0] = cptr<float>(host)[0];
-    mm[1] = cptr<float>(host)[1];
-  }
-  TORCH_CHECK(mm[0] <= mm[1], "In ChooseQuantizationParams, min should be less than or equal to max");
   double scale = 0;
   int32_t zp = 0;
-  check_status(tmq_choose_qparams_host(mm[0], mm[1], sgn, reduce_range, &scale, &zp),
-               "tmq_choose_qparams_host");
-  // quantize the original tensor, so that its memory format carries over
-  return at::quantize_per_tensor(self.scalar_type() == at::kFloat ? self : self.to(at::kFloat), scale, zp, dtype);
+  if (x.numel() == 0) {
+    check_status(tmq_choose_qparams_host(0.f, 0.f, sgn, reduce_range, &scale, &zp), "tmq_choose_qparams_host");
+    return empty_quantized(x.sizes(), x, dtype, scale, zp, fmt);
+  }
+  const auto stream = stream_for_report(x, what);
+  at::Tensor q = empty_quantized(x.sizes(), x, dtype, 1.0, 0, fmt);
+  const int64_t range_bytes = static_cast<int64_t>(tmq_minmax_workspace_bytes(x.numel()));
+  const at::Tensor scratch = empty_bytes(range_bytes + static_cast<int64_t>(sizeof(tmq_qparams)), x);
+  auto* ws = static_cast<uint8_t*>(scratch.data_ptr());
+  HostReport report;
+  check_status(tmq_quantize_per_tensor_dynamic_report(
+                   cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
+                   reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes),
+                   report.memory(), report.ticket(), reinterpret_cast<tmq_stream_t>(stream.stream())),
+               "tmq_quantize_per_tensor_dynamic_report");
+  report.queued();
+  const uint32_t lo = report.wait(0, stream, what), hi = report.wait(1, stream, what);
+  report.done();
+  float mn, mx;
+  std::memcpy(&mn, &lo, 4);
+  std::memcpy(&mx, &hi, 4);
+  TORCH_CHECK(mn <= mx, "In ChooseQuantizationParams, min should be less than or equal to max");
+  check_status(tmq_choose_qparams_host(mn, mx, sgn, reduce_range, &scale, &zp), "tmq_choose_qparams_host");
+  at::get_qtensorimpl(q)->set_quantizer_(at::make_per_tensor_affine_quantizer(scale, zp, dtype));
+  return q;
 }
 
 // ---------------------------------------------------------------------------
@@ -1210,15 +1276,6 @@ struct PlainWeightEntry {
   c10::hip::HIPStream stream;
   int64_t bytes = 0;
 };
-
-bool stream_is_capturing(const c10::hip::HIPStream& s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s.stream(), &st) != hipSuccess) {
-    (void)hipGetLastError();
-    return true;  // unknown: take the safe side
-  }
-  return st != hipStreamCaptureStatusNone;
-}
 
 class PlainWeightCache {
  public:

@@ -110,6 +110,23 @@ __device__ __forceinline__ void resolve(const QParamsArg& a, float& inv, float& 
   }
 }
 
+// What the host waits for goes to it as one or two 8-byte words in pinned host memory, a
+// ticket in the upper half and the payload in the lower one: each word is a single store,
+// so the host needs no order between them and the device no fence (a system-scope release
+// would write back the L2s first).
+__device__ __forceinline__ void report_word(uint64_t* word, uint32_t ticket, uint32_t payload) {
+  __hip_atomic_store(word, (static_cast<uint64_t>(ticket) << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+struct RangeReport {
+  tmq_host_report* to;
+  uint32_t ticket;
+};
+__device__ __forceinline__ void report_range(const RangeReport& r, float mn, float mx) {
+  if (r.to == nullptr) return;
+  report_word(&r.to->word[0], r.ticket, __builtin_bit_cast(uint32_t, mn));
+  report_word(&r.to->word[1], r.ticket, __builtin_bit_cast(uint32_t, mx));
+}
+
 // x4/q4 view the first 4*n4 elements; the block with index 0 also converts the
 // n - 4*n4 (< 4) trailing elements one by one.
 // The fp32 input is read once and never again: non-temporal loads keep it out of
@@ -330,7 +347,7 @@ __global__ void choose_qparams_kernel(const float* __restrict__ minmax, int qmin
 // Last stage of the min/max reduction and ChooseQuantizationParams in one block.
 __global__ __launch_bounds__(kThreads) void minmax_final_choose_kernel(
     const float* __restrict__ partials, int count, int qmin, int qmax, int reduce_range,
-    float* __restrict__ minmax_out, tmq_qparams* __restrict__ out) {
+    tmq_qparams* __restrict__ out, RangeReport report) {
   __shared__ float s_mm[2];
   float mn = std::numeric_limits<float>::infinity();
   float mx = -std::numeric_limits<float>::infinity();
@@ -346,10 +363,7 @@ __global__ __launch_bounds__(kThreads) void minmax_final_choose_kernel(
     out->scale = s;
     out->zero_point = z;
     out->reserved = 0;
-    if (minmax_out != nullptr) {
-      minmax_out[0] = s_mm[0];
-      minmax_out[1] = s_mm[1];
-    }
+    report_range(report, s_mm[0], s_mm[1]);
   }
 }
 
@@ -370,7 +384,7 @@ template <bool SIGNED, bool FUSED>
 __global__ __launch_bounds__(kThreads) void quantize_after_minmax_kernel(
     const v4f* __restrict__ x4, uint32_t* __restrict__ q4, int64_t n4, const float* __restrict__ x,
     uint8_t* __restrict__ q, int64_t n, const float* __restrict__ partials, int count, int qmin, int qmax,
-    int reduce_range, tmq_qparams* __restrict__ out) {
+    int reduce_range, tmq_qparams* __restrict__ out, RangeReport report) {
   __shared__ float s_mm[2];
   __shared__ float s_inv, s_zp;
   constexpr int U = kUnrollQD;
@@ -402,6 +416,7 @@ __global__ __launch_bounds__(kThreads) void quantize_after_minmax_kernel(
     s_inv = 1.0f / static_cast<float>(sc);  // IEEE division, as resolve()
     s_zp = static_cast<float>(z);
     if (blockIdx.x == 0) {
+      report_range(report, s_mm[0], s_mm[1]);
       out->scale = sc;
       out->zero_point = z;
       out->reserved = 0;
@@ -439,7 +454,7 @@ constexpr int64_t kDynSmallMax = 32768;
 template <bool SIGNED, bool FUSED>
 __global__ __launch_bounds__(kDynSmallThreads) void dynamic_quantize_small_kernel(
     const float* __restrict__ x, uint8_t* __restrict__ q, int64_t n, int qmin, int qmax,
-    int reduce_range, bool vec, tmq_qparams* __restrict__ out) {
+    int reduce_range, bool vec, tmq_qparams* __restrict__ out, RangeReport report) {
   __shared__ float s_mn[kDynSmallThreads / kWave], s_mx[kDynSmallThreads / kWave];
   __shared__ float s_inv, s_zp;
   const int t = threadIdx.x;
@@ -481,6 +496,7 @@ __global__ __launch_bounds__(kDynSmallThreads) void dynamic_quantize_small_kerne
       mn = fminf(mn, s_mn[w]);
       mx = fmaxf(mx, s_mx[w]);
     }
+    report_range(report, mn, mx);
     double s;
     int32_t z;
     choose_qparams(mn, mx, qmin, qmax, reduce_range != 0, &s, &z);
@@ -503,60 +519,21 @@ __global__ __launch_bounds__(kDynSmallThreads) void dynamic_quantize_small_kerne
 }
 
 // ---------------------------------------------------------------------------
-// Per-channel kernels over [outer, C, inner], element-indexed: the channel of
-// an element comes from its flat index.  They serve short rows (inner < 64,
-// e.g. a channel axis that is the last dimension); longer rows take
-// pc_rows_kernel below.  VEC = 4 when inner % 4 == 0 and the pointers are
-// 16-byte aligned (a group of 4 never straddles a channel).
+// Per-channel kernels over [outer, C, inner].  One Op per conversion (double or float
+// parameters, either direction); which kernel walks the tensor depends on where the
+// channels lie:
+//   inner == 1 (a channel axis that is the last dimension in memory): pc_cols_kernel,
+//     a thread keeps its channels and walks down the rows;
+//   inner % 4 == 0, inner >= 64: pc_rows_kernel, the channel is a property of the block;
+//   other inner >= 4: pc_flat_kernel, 16-byte accesses over the flat tensor, a group of
+//     four lies in at most two channels;
+//   inner 2 and 3: pc_element_kernel.
 // ---------------------------------------------------------------------------
-template <bool SIGNED, int VEC>
-__global__ __launch_bounds__(kThreads) void quantize_pc_kernel(
-    const float* __restrict__ x, uint8_t* __restrict__ q, int64_t n, int64_t C, int64_t inner,
-    const double* __restrict__ scales, const int64_t* __restrict__ zps) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * VEC;
-  for (int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC; i < n;
-       i += stride) {
-    const int64_t c = (i / inner) % C;
-    const float inv = 1.0f / static_cast<float>(scales[c]);
-    const float zp_f = static_cast<float>(zps[c]);
-    if constexpr (VEC == 4) {
-      const v4f v = *reinterpret_cast<const v4f*>(x + i);
-      *reinterpret_cast<uint32_t*>(q + i) = quantize_four<SIGNED>(v, inv, zp_f);
-    } else {
-      q[i] = static_cast<uint8_t>(quantize_one<SIGNED>(x[i], inv, zp_f));
-    }
-  }
-}
-
 template <bool SIGNED>
 __device__ __forceinline__ float dequantize_pc_one(uint32_t byte, float zp_f, double scale) {
   const int v = SIGNED ? static_cast<int>(static_cast<int8_t>(byte)) : static_cast<int>(byte);
   const float d = static_cast<float>(v) - zp_f;
   return static_cast<float>(static_cast<double>(d) * scale);
-}
-
-template <bool SIGNED, int VEC>
-__global__ __launch_bounds__(kThreads) void dequantize_pc_kernel(
-    const uint8_t* __restrict__ q, float* __restrict__ r, int64_t n, int64_t C, int64_t inner,
-    const double* __restrict__ scales, const int64_t* __restrict__ zps) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * VEC;
-  for (int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC; i < n;
-       i += stride) {
-    const int64_t c = (i / inner) % C;
-    const double scale = scales[c];
-    const float zp_f = static_cast<float>(zps[c]);
-    if constexpr (VEC == 4) {
-      const uint32_t w = *reinterpret_cast<const uint32_t*>(q + i);
-      v4f o;
-      o.x = dequantize_pc_one<SIGNED>(w & 0xffu, zp_f, scale);
-      o.y = dequantize_pc_one<SIGNED>((w >> 8) & 0xffu, zp_f, scale);
-      o.z = dequantize_pc_one<SIGNED>((w >> 16) & 0xffu, zp_f, scale);
-      o.w = dequantize_pc_one<SIGNED>(w >> 24, zp_f, scale);
-      *reinterpret_cast<v4f*>(r + i) = o;
-    } else {
-      r[i] = dequantize_pc_one<SIGNED>(q[i], zp_f, scale);
-    }
-  }
 }
 
 // Per-channel quantizer with float scales and float zero points
@@ -570,28 +547,6 @@ __device__ __forceinline__ uint32_t quantize_fq_one(float x, float inv, float zp
   return static_cast<uint32_t>(static_cast<int>(r)) & 0xffu;
 }
 
-template <bool SIGNED, int VEC>
-__global__ __launch_bounds__(kThreads) void quantize_pcf_kernel(
-    const float* __restrict__ x, uint8_t* __restrict__ q, int64_t n, int64_t C, int64_t inner,
-    const float* __restrict__ scales, const float* __restrict__ zps) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * VEC;
-  for (int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC; i < n;
-       i += stride) {
-    const int64_t c = (i / inner) % C;
-    const float sc = scales[c];
-    const float inv = sc == 0.f ? 1.0f : 1.0f / sc;
-    const float zp = zps[c];
-    if constexpr (VEC == 4) {
-      const v4f v = *reinterpret_cast<const v4f*>(x + i);
-      *reinterpret_cast<uint32_t*>(q + i) =
-          quantize_fq_one<SIGNED>(v.x, inv, zp) | (quantize_fq_one<SIGNED>(v.y, inv, zp) << 8) |
-          (quantize_fq_one<SIGNED>(v.z, inv, zp) << 16) | (quantize_fq_one<SIGNED>(v.w, inv, zp) << 24);
-    } else {
-      q[i] = static_cast<uint8_t>(quantize_fq_one<SIGNED>(x[i], inv, zp));
-    }
-  }
-}
-
 template <bool SIGNED>
 __device__ __forceinline__ float dequantize_fq_one(uint32_t byte, float zp, float scale) {
   const int v = SIGNED ? static_cast<int>(static_cast<int8_t>(byte)) : static_cast<int>(byte);
@@ -599,43 +554,8 @@ __device__ __forceinline__ float dequantize_fq_one(uint32_t byte, float zp, floa
   return d * scale;
 }
 
-template <bool SIGNED, int VEC>
-__global__ __launch_bounds__(kThreads) void dequantize_pcf_kernel(
-    const uint8_t* __restrict__ q, float* __restrict__ r, int64_t n, int64_t C, int64_t inner,
-    const float* __restrict__ scales, const float* __restrict__ zps) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * VEC;
-  for (int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC; i < n;
-       i += stride) {
-    const int64_t c = (i / inner) % C;
-    const float scale = scales[c], zp = zps[c];
-    if constexpr (VEC == 4) {
-      const uint32_t w = *reinterpret_cast<const uint32_t*>(q + i);
-      v4f o;
-      o.x = dequantize_fq_one<SIGNED>(w & 0xffu, zp, scale);
-      o.y = dequantize_fq_one<SIGNED>((w >> 8) & 0xffu, zp, scale);
-      o.z = dequantize_fq_one<SIGNED>((w >> 16) & 0xffu, zp, scale);
-      o.w = dequantize_fq_one<SIGNED>(w >> 24, zp, scale);
-      *reinterpret_cast<v4f*>(r + i) = o;
-    } else {
-      r[i] = dequantize_fq_one<SIGNED>(q[i], zp, scale);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Per-channel kernels for inner >= kPcRowsMinInner: the channel is a property of
-// the block, not of the element.  The tensor is `rows` = outer * C rows of
-// `inner` elements; a block takes RB = A >> lg_us consecutive rows (A accesses per thread) x one
-// segment of US = 1 << lg_us runs of 256 lanes x VEC elements, i.e. eight
-// accesses per thread whatever the row length (a row of 4096 floats is four
-// 16-byte accesses per thread, so a quantizing block takes two rows).  Row and channel come
-// from blockIdx with one division per block; the parameters of a row are
-// wave-uniform (scalar loads); the element loop has no division at all.
-// Loads are batched ahead of the stores and carry the same cache hints as the
-// per-tensor kernels.
-// ---------------------------------------------------------------------------
-constexpr int kPcRowsMinInner = 64;
-
+// An Op: P, the parameters of a channel; load4 / load1, conv4 (four values of up to four
+// channels), conv1, put4 / put1; zp_outside, the range check of a channel's zero point.
 template <bool SIGNED>
 struct PcQuantize {
   // fp32 -> codes, double scales, int64 zero points
@@ -647,17 +567,28 @@ struct PcQuantize {
   struct P { float inv, zp; };
   using In4 = v4f;
   using In1 = float;
+  using Out4 = uint32_t;
   __device__ __forceinline__ P params(int64_t c) const {
     return {1.0f / static_cast<float>(scales[c]), static_cast<float>(zps[c])};
+  }
+  __device__ __forceinline__ bool zp_outside(int64_t c) const {
+    const int64_t z = zps[c];
+    return z < (SIGNED ? -128 : 0) || z > (SIGNED ? 127 : 255);
   }
   __device__ __forceinline__ In4 load4(int64_t i) const {
     return __builtin_nontemporal_load(reinterpret_cast<const v4f*>(x + i));
   }
   __device__ __forceinline__ In1 load1(int64_t i) const { return x[i]; }
-  __device__ __forceinline__ void store4(int64_t i, In4 v, P p) const {
-    *reinterpret_cast<uint32_t*>(q + i) = quantize_four<SIGNED>(v, p.inv, p.zp);
+  __device__ __forceinline__ Out4 conv4(In4 v, const P (&p)[4]) const {
+    uint32_t packed = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)  // (as quantize_four)
+      packed = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_rintf(v[j] * p[j].inv) + (SIGNED ? p[j].zp + 128.f : p[j].zp), j,
+                                              packed);
+    return SIGNED ? packed ^ 0x80808080u : packed;
   }
-  __device__ __forceinline__ void store1(int64_t i, In1 v, P p) const {
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
+  __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_one<SIGNED>(v, p.inv, p.zp));
   }
 };
@@ -673,20 +604,26 @@ struct PcDequantize {
   struct P { double scale; float zp; };
   using In4 = uint32_t;
   using In1 = uint32_t;
+  using Out4 = v4f;
   __device__ __forceinline__ P params(int64_t c) const { return {scales[c], static_cast<float>(zps[c])}; }
+  __device__ __forceinline__ bool zp_outside(int64_t c) const {
+    const int64_t z = zps[c];
+    return z < (SIGNED ? -128 : 0) || z > (SIGNED ? 127 : 255);
+  }
   __device__ __forceinline__ In4 load4(int64_t i) const { return *reinterpret_cast<const uint32_t*>(q + i); }
   __device__ __forceinline__ In1 load1(int64_t i) const { return q[i]; }
-  __device__ __forceinline__ void store4(int64_t i, In4 w, P p) const {
+  __device__ __forceinline__ Out4 conv4(In4 w, const P (&p)[4]) const {
     v4f o;
-    o.x = dequantize_pc_one<SIGNED>(w & 0xffu, p.zp, p.scale);
-    o.y = dequantize_pc_one<SIGNED>((w >> 8) & 0xffu, p.zp, p.scale);
-    o.z = dequantize_pc_one<SIGNED>((w >> 16) & 0xffu, p.zp, p.scale);
-    o.w = dequantize_pc_one<SIGNED>(w >> 24, p.zp, p.scale);
+    o.x = dequantize_pc_one<SIGNED>(w & 0xffu, p[0].zp, p[0].scale);
+    o.y = dequantize_pc_one<SIGNED>((w >> 8) & 0xffu, p[1].zp, p[1].scale);
+    o.z = dequantize_pc_one<SIGNED>((w >> 16) & 0xffu, p[2].zp, p[2].scale);
+    o.w = dequantize_pc_one<SIGNED>(w >> 24, p[3].zp, p[3].scale);
+    return o;
+  }
+  __device__ __forceinline__ void put4(int64_t i, Out4 o) const {
     __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(r + i));
   }
-  __device__ __forceinline__ void store1(int64_t i, In1 b, P p) const {
-    r[i] = dequantize_pc_one<SIGNED>(b, p.zp, p.scale);
-  }
+  __device__ __forceinline__ void put1(int64_t i, In1 b, P p) const { r[i] = dequantize_pc_one<SIGNED>(b, p.zp, p.scale); }
 };
 
 template <bool SIGNED>
@@ -700,20 +637,24 @@ struct PcfQuantize {
   struct P { float inv, zp; };
   using In4 = v4f;
   using In1 = float;
+  using Out4 = uint32_t;
   __device__ __forceinline__ P params(int64_t c) const {
     const float sc = scales[c];
     return {sc == 0.f ? 1.0f : 1.0f / sc, zps[c]};
+  }
+  __device__ __forceinline__ bool zp_outside(int64_t c) const {
+    return zps[c] < (SIGNED ? -128.f : 0.f) || zps[c] > (SIGNED ? 127.f : 255.f);
   }
   __device__ __forceinline__ In4 load4(int64_t i) const {
     return __builtin_nontemporal_load(reinterpret_cast<const v4f*>(x + i));
   }
   __device__ __forceinline__ In1 load1(int64_t i) const { return x[i]; }
-  __device__ __forceinline__ void store4(int64_t i, In4 v, P p) const {
-    *reinterpret_cast<uint32_t*>(q + i) =
-        quantize_fq_one<SIGNED>(v.x, p.inv, p.zp) | (quantize_fq_one<SIGNED>(v.y, p.inv, p.zp) << 8) |
-        (quantize_fq_one<SIGNED>(v.z, p.inv, p.zp) << 16) | (quantize_fq_one<SIGNED>(v.w, p.inv, p.zp) << 24);
+  __device__ __forceinline__ Out4 conv4(In4 v, const P (&p)[4]) const {
+    return quantize_fq_one<SIGNED>(v.x, p[0].inv, p[0].zp) | (quantize_fq_one<SIGNED>(v.y, p[1].inv, p[1].zp) << 8) |
+           (quantize_fq_one<SIGNED>(v.z, p[2].inv, p[2].zp) << 16) | (quantize_fq_one<SIGNED>(v.w, p[3].inv, p[3].zp) << 24);
   }
-  __device__ __forceinline__ void store1(int64_t i, In1 v, P p) const {
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
+  __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_fq_one<SIGNED>(v, p.inv, p.zp));
   }
 };
@@ -729,41 +670,77 @@ struct PcfDequantize {
   struct P { float scale, zp; };
   using In4 = uint32_t;
   using In1 = uint32_t;
+  using Out4 = v4f;
   __device__ __forceinline__ P params(int64_t c) const { return {scales[c], zps[c]}; }
+  __device__ __forceinline__ bool zp_outside(int64_t c) const {
+    return zps[c] < (SIGNED ? -128.f : 0.f) || zps[c] > (SIGNED ? 127.f : 255.f);
+  }
   __device__ __forceinline__ In4 load4(int64_t i) const { return *reinterpret_cast<const uint32_t*>(q + i); }
   __device__ __forceinline__ In1 load1(int64_t i) const { return q[i]; }
-  __device__ __forceinline__ void store4(int64_t i, In4 w, P p) const {
+  __device__ __forceinline__ Out4 conv4(In4 w, const P (&p)[4]) const {
     v4f o;
-    o.x = dequantize_fq_one<SIGNED>(w & 0xffu, p.zp, p.scale);
-    o.y = dequantize_fq_one<SIGNED>((w >> 8) & 0xffu, p.zp, p.scale);
-    o.z = dequantize_fq_one<SIGNED>((w >> 16) & 0xffu, p.zp, p.scale);
-    o.w = dequantize_fq_one<SIGNED>(w >> 24, p.zp, p.scale);
+    o.x = dequantize_fq_one<SIGNED>(w & 0xffu, p[0].zp, p[0].scale);
+    o.y = dequantize_fq_one<SIGNED>((w >> 8) & 0xffu, p[1].zp, p[1].scale);
+    o.z = dequantize_fq_one<SIGNED>((w >> 16) & 0xffu, p[2].zp, p[2].scale);
+    o.w = dequantize_fq_one<SIGNED>(w >> 24, p[3].zp, p[3].scale);
+    return o;
+  }
+  __device__ __forceinline__ void put4(int64_t i, Out4 o) const {
     __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(r + i));
   }
-  __device__ __forceinline__ void store1(int64_t i, In1 b, P p) const {
-    r[i] = dequantize_fq_one<SIGNED>(b, p.zp, p.scale);
-  }
+  __device__ __forceinline__ void put1(int64_t i, In1 b, P p) const { r[i] = dequantize_fq_one<SIGNED>(b, p.zp, p.scale); }
 };
 
-// Accesses per thread (Op::kAccesses), all in flight before the first store: four for
-// the quantizers, two for the dequantizers, in blocks of two waves -- the shape the
-// per-tensor kernels settled on as well.  At fp32 [11008, 4096], axis 0, inputs and
+// The range check of the zero points, which the caller has to raise an error for before it
+// returns: the first block of the conversion does nothing else, so the answer is out a few
+// microseconds after the kernel starts, while the other blocks convert, and the host goes on
+// without waiting for them.  (As a chain of its own, two comparisons, their union and a
+// reduction read back by the host, it took 16 us of GPU time and left the queue empty.)
+struct PcCheck {
+  tmq_host_report* report;
+  uint32_t ticket;
+};
+template <class Op>
+__device__ __forceinline__ void pc_check_block(const Op& op, int64_t C, const PcCheck& check) {
+  int bad = 0;
+  for (int64_t c = threadIdx.x; c < C; c += blockDim.x) bad |= op.zp_outside(c) ? 1 : 0;
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) report_word(&check.report->word[0], check.ticket, bad != 0 ? 1u : 0u);
+}
+// This block's index among the converting ones; negative: it was the checking one.
+template <class Op>
+__device__ __forceinline__ int64_t pc_block(const Op& op, int64_t C, const PcCheck& check) {
+  if (check.report == nullptr) return blockIdx.x;
+  if (blockIdx.x == 0) pc_check_block(op, C, check);
+  return static_cast<int64_t>(blockIdx.x) - 1;
+}
+
+constexpr int kPcRowsMinInner = 64;
+
+// pc_rows_kernel: the tensor is `rows` = outer * C rows of `inner` elements; a block takes
+// RB = A >> lg_us consecutive rows (A accesses per thread) x one segment of US = 1 << lg_us
+// runs of 128 lanes x 4 elements.  Row and channel come from blockIdx with one division per
+// block; the parameters of a row are wave-uniform (scalar loads); the element loop has no
+// division at all.  Accesses per thread (Op::kAccesses), all in flight before the first
+// store: four for the quantizers, two for the dequantizers, in blocks of two waves -- the
+// shape the per-tensor kernels settled on as well.  At fp32 [11008, 4096], axis 0, inputs and
 // outputs rotating over more bytes than the last-level cache holds: quantize 39.8 us
 // (per-tensor kernel on as many elements: 38.4 us), dequantize 37.6 us (35.4 us);
 // the dequantizer took 42.2 us with a parameter request per access, each waiting for
 // the one before it, 39.4 us with one per row in blocks of four waves x four accesses.
 constexpr int kPcThreads = 128;
-template <class Op, int VEC>
+template <class Op>
 __global__ __launch_bounds__(kPcThreads) void pc_rows_kernel(Op op, int64_t rows, int64_t C, int64_t inner,
-                                                           int lg_us, uint32_t segs) {
-  using In = std::conditional_t<VEC == 4, typename Op::In4, typename Op::In1>;
-  constexpr int kPcAccesses = Op::kAccesses;
-  const uint32_t rg = blockIdx.x / segs, seg = blockIdx.x - rg * segs;
+                                                           int lg_us, uint32_t segs, PcCheck check) {
+  constexpr int kPcAccesses = Op::kAccesses, VEC = 4;
+  const int64_t block = pc_block(op, C, check);
+  if (block < 0) return;
+  const uint32_t rg = static_cast<uint32_t>(block) / segs, seg = static_cast<uint32_t>(block) - rg * segs;
   const int us_mask = (1 << lg_us) - 1;
   const int64_t row0 = static_cast<int64_t>(rg) * (kPcAccesses >> lg_us);
   const int64_t c0 = row0 % C;  // once per block, wave-uniform
   const int64_t col0 = (static_cast<int64_t>(seg) << lg_us) * (kPcThreads * VEC) + threadIdx.x * VEC;
-  In held[kPcAccesses];
+  typename Op::In4 held[kPcAccesses];
   bool live[kPcAccesses];
   // a block that lies inside the tensor as a whole (all but the last row group and the
   // last segment of a row) loads and stores without a condition per access
@@ -780,11 +757,8 @@ __global__ __launch_bounds__(kPcThreads) void pc_rows_kernel(Op op, int64_t rows
 #pragma unroll
         for (int r = 0; r < kRows; ++r)
 #pragma unroll
-          for (int k = 0; k < kRuns; ++k) {
-            const int64_t at = (row0 + r) * inner + col0 + static_cast<int64_t>(k) * (kPcThreads * VEC);
-            if constexpr (VEC == 4) held[r * kRuns + k] = op.load4(at);
-            else held[r * kRuns + k] = op.load1(at);
-          }
+          for (int k = 0; k < kRuns; ++k)
+            held[r * kRuns + k] = op.load4((row0 + r) * inner + col0 + static_cast<int64_t>(k) * (kPcThreads * VEC));
         typename Op::P prm[kRows];
 #pragma unroll
         for (int r = 0; r < kRows; ++r) {
@@ -797,8 +771,7 @@ __global__ __launch_bounds__(kPcThreads) void pc_rows_kernel(Op op, int64_t rows
 #pragma unroll
           for (int k = 0; k < kRuns; ++k) {
             const int64_t at = (row0 + r) * inner + col0 + static_cast<int64_t>(k) * (kPcThreads * VEC);
-            if constexpr (VEC == 4) op.store4(at, held[r * kRuns + k], prm[r]);
-            else op.store1(at, held[r * kRuns + k], prm[r]);
+            op.put4(at, op.conv4(held[r * kRuns + k], {prm[r], prm[r], prm[r], prm[r]}));
           }
       }
     };
@@ -815,10 +788,7 @@ __global__ __launch_bounds__(kPcThreads) void pc_rows_kernel(Op op, int64_t rows
     const int64_t row = row0 + (u >> lg_us);
     const int64_t col = col0 + static_cast<int64_t>(u & us_mask) * (kPcThreads * VEC);
     live[u] = row < rows && col < inner;
-    if (live[u]) {
-      if constexpr (VEC == 4) held[u] = op.load4(row * inner + col);
-      else held[u] = op.load1(row * inner + col);
-    }
+    if (live[u]) held[u] = op.load4(row * inner + col);
   }
 #pragma unroll
   for (int u = 0; u < kPcAccesses; ++u) {
@@ -828,32 +798,114 @@ __global__ __launch_bounds__(kPcThreads) void pc_rows_kernel(Op op, int64_t rows
     while (c >= C) c -= C;   // at most A - 1 rows past c0: uniform, a few scalar steps
     const typename Op::P p = op.params(c);
     const int64_t col = col0 + static_cast<int64_t>(u & us_mask) * (kPcThreads * VEC);
-    if (live[u]) {
-      if constexpr (VEC == 4) op.store4(row * inner + col, held[u], p);
-      else op.store1(row * inner + col, held[u], p);
+    if (live[u]) op.put4(row * inner + col, op.conv4(held[u], {p, p, p, p}));
+  }
+}
+
+// Quotient and remainder of non-negative 32-bit values by a divisor whose fp32 reciprocal is
+// at hand; exact for quotients below 2**20 (the estimate is off by one at most).
+__device__ __forceinline__ void divmod_by(int a, int d, float inv_d, int& quo, int& rem) {
+  quo = static_cast<int>(static_cast<float>(a) * inv_d);
+  rem = a - quo * d;
+  if (rem < 0) {
+    --quo;
+    rem += d;
+  } else if (rem >= d) {
+    ++quo;
+    rem -= d;
+  }
+}
+
+// pc_flat_kernel: rows that no 16-byte access divides (a weight of 5411 columns, 3 x 3 x 3
+// taps) as one flat run.  A thread's group of four values begins in channel c and may run
+// into c + 1; one 64-bit division per block, float-reciprocal ones per group, and each
+// thread's own channel parameters from the caches while its values are on their way.
+// Bound by memory like the row kernel: fp32 [8328, 5411] axis 0 (quantize) runs at the
+// row kernel's rate, where the 4-byte accesses it replaces reached half of it.
+constexpr int kPcFlatGroups = 4;  // groups of four values per thread
+constexpr int64_t kPcFlatSpan = kPcThreads * kPcFlatGroups * 4;
+constexpr int64_t kPcFlatMaxExtent = int64_t{1} << 30;  // inner and C within 32-bit arithmetic
+template <class Op, bool VEC>
+__global__ __launch_bounds__(kPcThreads) void pc_flat_kernel(Op op, int64_t n, int32_t C, int32_t inner, float inv_c,
+                                                           float inv_inner, PcCheck check) {
+  const int64_t block = pc_block(op, C, check);
+  if (block < 0) return;
+  const int64_t start = block * kPcFlatSpan;
+  typename Op::In4 held[kPcFlatGroups];
+  const int at0 = static_cast<int>(threadIdx.x) * 4;
+#pragma unroll
+  for (int u = 0; u < kPcFlatGroups; ++u) {
+    const int64_t i = start + u * (kPcThreads * 4) + at0;
+    if (VEC && i + 4 <= n) held[u] = op.load4(i);
+  }
+  const int64_t row0 = start / inner;
+  const int rem0 = static_cast<int>(start - row0 * inner);
+  const int c0 = static_cast<int>(row0 % C);
+#pragma unroll
+  for (int u = 0; u < kPcFlatGroups; ++u) {
+    const int local = u * (kPcThreads * 4) + at0;
+    const int64_t i = start + local;
+    if (i >= n) break;
+    int row, rem, wraps, c;
+    divmod_by(rem0 + local, inner, inv_inner, row, rem);
+    divmod_by(c0 + row, C, inv_c, wraps, c);
+    const int first = inner - rem;  // values of this group that belong to channel c
+    const typename Op::P a = op.params(c);
+    typename Op::P b = a;
+    if (first < 4) b = op.params(c + 1 == C ? 0 : c + 1);
+    if (VEC && i + 4 <= n) {
+      op.put4(i, op.conv4(held[u], {a, first > 1 ? a : b, first > 2 ? a : b, first > 3 ? a : b}));
+    } else {
+      for (int j = 0; j < 4 && i + j < n; ++j) op.put1(i + j, op.load1(i + j), j < first ? a : b);
     }
   }
 }
 
-// Launches pc_rows_kernel if the shape suits it; returns false if the caller
-// should use the element-indexed kernels (short rows, or a grid beyond 2**31).
+// pc_cols_kernel: `rows` x C values whose channel is the column.  A block takes the columns
+// [col0, col0 + width) of kPcColsRows runs of rows; its threads stand on `lanes` = width / VEC column
+// groups x 256 / lanes rows, so every thread keeps its columns and their parameters.
+constexpr int kPcColsThreads = 256;
+constexpr int kPcColsSteps = 8;  // rows per thread
+template <class Op, int VEC>
+__global__ __launch_bounds__(kPcColsThreads) void pc_cols_kernel(Op op, int64_t rows, int64_t C, int32_t lanes,
+                                                               uint32_t col_blocks, PcCheck check) {
+  const int64_t block = pc_block(op, C, check);
+  if (block < 0) return;
+  const uint32_t rb = static_cast<uint32_t>(block) / col_blocks, cb = static_cast<uint32_t>(block) - rb * col_blocks;
+  const int per = kPcColsThreads / lanes;  // rows side by side
+  const int mine = static_cast<int>(threadIdx.x) / lanes;
+  const int64_t col = (static_cast<int64_t>(cb) * lanes + (static_cast<int>(threadIdx.x) - mine * lanes)) * VEC;
+  if (mine >= per || col >= C) return;
+  const int64_t row0 = static_cast<int64_t>(rb) * (per * kPcColsSteps) + mine;
+  std::conditional_t<VEC == 4, typename Op::In4, typename Op::In1> held[kPcColsSteps];
+#pragma unroll
+  for (int u = 0; u < kPcColsSteps; ++u) {
+    const int64_t row = row0 + u * per;
+    if (row < rows) {
+      if constexpr (VEC == 4) held[u] = op.load4(row * C + col);
+      else held[u] = op.load1(row * C + col);
+    }
+  }
+  typename Op::P p[4];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) p[j] = op.params(col + j);
+#pragma unroll
+  for (int u = 0; u < kPcColsSteps; ++u) {
+    const int64_t row = row0 + u * per;
+    if (row < rows) {
+      if constexpr (VEC == 4) op.put4(row * C + col, op.conv4(held[u], p));
+      else op.put1(row * C + col, held[u], p[0]);
+    }
+  }
+}
+
 template <class Op>
-bool launch_pc_rows(const Op& op, int64_t outer, int64_t C, int64_t inner, bool vec, hipStream_t s) {
-  if (inner < kPcRowsMinInner) return false;
-  constexpr int kPcAccesses = Op::kAccesses;
-  const int64_t per_run = kPcThreads * (vec ? 4 : 1);
-  int lg_us = 0;
-  while ((2 << lg_us) <= kPcAccesses && (per_run << lg_us) < inner) ++lg_us;
-  const int64_t rows = outer * C;
-  const int64_t segs = ceil_div(inner, per_run << lg_us);
-  const int64_t row_groups = ceil_div(rows, kPcAccesses >> lg_us);
-  if (segs > 0x7fffffff || row_groups > 0x7fffffff / segs) return false;
-  const dim3 grid(static_cast<unsigned>(row_groups * segs));
-  if (vec)
-    pc_rows_kernel<Op, 4><<<grid, dim3(kPcThreads), 0, s>>>(op, rows, C, inner, lg_us, static_cast<uint32_t>(segs));
-  else
-    pc_rows_kernel<Op, 1><<<grid, dim3(kPcThreads), 0, s>>>(op, rows, C, inner, lg_us, static_cast<uint32_t>(segs));
-  return true;
+__global__ __launch_bounds__(kThreads) void pc_element_kernel(Op op, int64_t n, int64_t C, int64_t inner, PcCheck check) {
+  const int64_t block = pc_block(op, C, check);
+  if (block < 0) return;
+  const int64_t stride = (static_cast<int64_t>(gridDim.x) - (check.report != nullptr ? 1 : 0)) * kThreads;
+  for (int64_t i = block * kThreads + threadIdx.x; i < n; i += stride)
+    op.put1(i, op.load1(i), op.params((i / inner) % C));
 }
 
 inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t cap) {
@@ -861,6 +913,57 @@ inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t cap) {
   if (g < 1) g = 1;
   if (g > cap) g = cap;
   return static_cast<unsigned>(g);
+}
+
+// `vec`: both pointers take 16-byte accesses of fp32 and 4-byte accesses of codes.
+template <class Op>
+int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bool vec, const PcCheck& check,
+                       hipStream_t s) {
+  const int64_t n = outer * C * inner, extra = check.report != nullptr ? 1 : 0;
+  if (n == 0) return TMQ_OK;
+  if (inner == 1) {
+    const bool v4 = vec && C % 4 == 0;
+    const int64_t groups = v4 ? C / 4 : C;
+    // as few column blocks as 256 threads allow, of equal width
+    const int64_t col_blocks = ceil_div(groups, kPcColsThreads), lanes = ceil_div(groups, col_blocks);
+    const int64_t blocks = ceil_div(outer, kPcColsThreads / lanes * kPcColsSteps) * col_blocks;
+    if (blocks < 0x7fffffff) {
+      const dim3 grid(static_cast<unsigned>(blocks + extra));
+      if (v4)
+        pc_cols_kernel<Op, 4><<<grid, dim3(kPcColsThreads), 0, s>>>(op, outer, C, static_cast<int32_t>(lanes),
+                                                                    static_cast<uint32_t>(col_blocks), check);
+      else
+        pc_cols_kernel<Op, 1><<<grid, dim3(kPcColsThreads), 0, s>>>(op, outer, C, static_cast<int32_t>(lanes),
+                                                                    static_cast<uint32_t>(col_blocks), check);
+      return launch_status();
+    }
+  }
+  if (vec && inner % 4 == 0 && inner >= kPcRowsMinInner) {
+    constexpr int kPcAccesses = Op::kAccesses;
+    const int64_t per_run = kPcThreads * 4;
+    int lg_us = 0;
+    while ((2 << lg_us) <= kPcAccesses && (per_run << lg_us) < inner) ++lg_us;
+    const int64_t segs = ceil_div(inner, per_run << lg_us);
+    const int64_t row_groups = ceil_div(outer * C, kPcAccesses >> lg_us);
+    if (segs < 0x7fffffff && row_groups < 0x7fffffff / segs) {
+      pc_rows_kernel<Op><<<dim3(static_cast<unsigned>(row_groups * segs + extra)), dim3(kPcThreads), 0, s>>>(
+          op, outer * C, C, inner, lg_us, static_cast<uint32_t>(segs), check);
+      return launch_status();
+    }
+  }
+  if (inner >= 4 && inner <= kPcFlatMaxExtent && C <= kPcFlatMaxExtent && ceil_div(n, kPcFlatSpan) < 0x7fffffff) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(n, kPcFlatSpan) + extra));
+    const int32_t c32 = static_cast<int32_t>(C), inner32 = static_cast<int32_t>(inner);
+    const float inv_c = 1.0f / static_cast<float>(C), inv_inner = 1.0f / static_cast<float>(inner);
+    if (vec)
+      pc_flat_kernel<Op, true><<<grid, dim3(kPcThreads), 0, s>>>(op, n, c32, inner32, inv_c, inv_inner, check);
+    else
+      pc_flat_kernel<Op, false><<<grid, dim3(kPcThreads), 0, s>>>(op, n, c32, inner32, inv_c, inv_inner, check);
+    return launch_status();
+  }
+  const unsigned g = grid_for(n, kThreads, 1 << 20);
+  pc_element_kernel<Op><<<dim3(g + static_cast<unsigned>(extra)), dim3(kThreads), 0, s>>>(op, n, C, inner, check);
+  return launch_status();
 }
 
 template <bool SIGNED, bool FUSED>
@@ -990,9 +1093,11 @@ TMQ_EXPORT int tmq_choose_qparams_dev(const float* minmax, int q_signed, int red
   return launch_status();
 }
 
-TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int64_t n, int q_signed,
-                                                   int reduce_range, int rounding, tmq_qparams* qparams,
-                                                   void* workspace, size_t workspace_bytes, tmq_stream_t stream) {
+namespace tmq {
+namespace {
+int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduce_range, int rounding,
+                     tmq_qparams* qparams, void* workspace, size_t workspace_bytes, RangeReport report,
+                     tmq_stream_t stream) {
   if (n < 0 || qparams == nullptr || (n > 0 && (x == nullptr || q == nullptr))) return TMQ_ERR_INVALID_ARGUMENT;
   if (rounding != TMQ_ROUND_PRODUCT && rounding != TMQ_ROUND_FUSED) return TMQ_ERR_INVALID_ARGUMENT;
   const bool fused = rounding == TMQ_ROUND_FUSED;
@@ -1004,13 +1109,13 @@ TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int6
     uint8_t* qb = static_cast<uint8_t*>(q);
     const dim3 one(1), block(kDynSmallThreads);
     if (q_signed && fused)
-      dynamic_quantize_small_kernel<true, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams);
+      dynamic_quantize_small_kernel<true, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
     else if (q_signed)
-      dynamic_quantize_small_kernel<true, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams);
+      dynamic_quantize_small_kernel<true, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
     else if (fused)
-      dynamic_quantize_small_kernel<false, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams);
+      dynamic_quantize_small_kernel<false, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
     else
-      dynamic_quantize_small_kernel<false, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams);
+      dynamic_quantize_small_kernel<false, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
     return launch_status();
   }
   if (workspace == nullptr || workspace_bytes < tmq_minmax_workspace_bytes(n) || !aligned(workspace, 4))
@@ -1031,13 +1136,13 @@ TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int6
     uint8_t* qb = static_cast<uint8_t*>(q);
     const int cnt = static_cast<int>(g);
     if (q_signed && fused)
-      quantize_after_minmax_kernel<true, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams);
+      quantize_after_minmax_kernel<true, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, report);
     else if (q_signed)
-      quantize_after_minmax_kernel<true, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams);
+      quantize_after_minmax_kernel<true, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, report);
     else if (fused)
-      quantize_after_minmax_kernel<false, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams);
+      quantize_after_minmax_kernel<false, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, report);
     else
-      quantize_after_minmax_kernel<false, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams);
+      quantize_after_minmax_kernel<false, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, report);
     return launch_status();
   }
   // larger inputs (streamed past the caches) and unaligned buffers: range, parameters and
@@ -1051,13 +1156,31 @@ TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int6
                                                            n, partials);
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   minmax_final_choose_kernel<<<dim3(1), dim3(kThreads), 0, s>>>(partials, static_cast<int>(g), qmin, qmax,
-                                                                reduce_range, nullptr, qparams);
+                                                                reduce_range, qparams, report);
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   QParamsArg qp;
   qp.inv = 0.f;
   qp.zp_f = 0.f;
   qp.dev = qparams;
   return quantize_launch(x, q, n, qp, q_signed, s, fused);
+}
+}  // namespace
+}  // namespace tmq
+
+TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int64_t n, int q_signed,
+                                                   int reduce_range, int rounding, tmq_qparams* qparams,
+                                                   void* workspace, size_t workspace_bytes, tmq_stream_t stream) {
+  return quantize_dynamic(x, q, n, q_signed, reduce_range, rounding, qparams, workspace, workspace_bytes,
+                          RangeReport{nullptr, 0}, stream);
+}
+
+TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, int q_signed,
+                                                      int reduce_range, int rounding, tmq_qparams* qparams,
+                                                      void* workspace, size_t workspace_bytes,
+                                                      tmq_host_report* report, uint32_t ticket, tmq_stream_t stream) {
+  if (report == nullptr || n <= 0) return TMQ_ERR_INVALID_ARGUMENT;
+  return quantize_dynamic(x, q, n, q_signed, reduce_range, rounding, qparams, workspace, workspace_bytes,
+                          RangeReport{report, ticket}, stream);
 }
 
 TMQ_EXPORT int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
@@ -1068,13 +1191,44 @@ TMQ_EXPORT int tmq_choose_qparams_host(float min, float max, int q_signed, int r
   return TMQ_OK;
 }
 
+TMQ_EXPORT int tmq_per_channel(const tmq_per_channel_desc* d, tmq_stream_t stream) {
+  if (d == nullptr || d->outer < 0 || d->channels < 0 || d->inner < 0) return TMQ_ERR_INVALID_ARGUMENT;
+  if (d->outer == 0 || d->channels == 0 || d->inner == 0) return d->report == nullptr ? TMQ_OK : TMQ_ERR_INVALID_ARGUMENT;
+  if (d->fp32 == nullptr || d->codes == nullptr || d->scales == nullptr || d->zero_points == nullptr)
+    return TMQ_ERR_INVALID_ARGUMENT;
+  hipStream_t s = as_stream(stream);
+  const PcCheck check{d->report, d->ticket};
+  auto* f = static_cast<float*>(d->fp32);
+  auto* q = static_cast<uint8_t*>(d->codes);
+  const bool vec = aligned(f, 16) && aligned(q, 4);
+  auto go = [&](const auto& op) { return launch_per_channel(op, d->outer, d->channels, d->inner, vec, check, s); };
+  if (d->float_qparams) {
+    auto* sc = static_cast<const float*>(d->scales);
+    auto* zp = static_cast<const float*>(d->zero_points);
+    if (d->dequantize) return d->q_signed ? go(PcfDequantize<true>{q, f, sc, zp}) : go(PcfDequantize<false>{q, f, sc, zp});
+    return d->q_signed ? go(PcfQuantize<true>{f, q, sc, zp}) : go(PcfQuantize<false>{f, q, sc, zp});
+  }
+  auto* sc = static_cast<const double*>(d->scales);
+  auto* zp = static_cast<const int64_t*>(d->zero_points);
+  if (d->dequantize) return d->q_signed ? go(PcDequantize<true>{q, f, sc, zp}) : go(PcDequantize<false>{q, f, sc, zp});
+  return d->q_signed ? go(PcQuantize<true>{f, q, sc, zp}) : go(PcQuantize<false>{f, q, sc, zp});
+}
+
 namespace {
-bool pc_args_ok(const void* a, const void* b, int64_t outer, int64_t C, int64_t inner,
-                const double* scales, const int64_t* zps) {
-  if (outer < 0 || C < 0 || inner < 0) return false;
-  const bool empty = outer == 0 || C == 0 || inner == 0;
-  if (!empty && (a == nullptr || b == nullptr || scales == nullptr || zps == nullptr)) return false;
-  return true;
+int per_channel(int dequantize, int float_qparams, const void* fp32, const void* codes, int64_t outer, int64_t channels,
+                int64_t inner, const void* scales, const void* zero_points, int q_signed, tmq_stream_t stream) {
+  tmq_per_channel_desc d{};
+  d.dequantize = dequantize;
+  d.float_qparams = float_qparams;
+  d.q_signed = q_signed;
+  d.fp32 = const_cast<void*>(fp32);
+  d.codes = const_cast<void*>(codes);
+  d.outer = outer;
+  d.channels = channels;
+  d.inner = inner;
+  d.scales = scales;
+  d.zero_points = zero_points;
+  return tmq_per_channel(&d, stream);
 }
 }  // namespace
 
@@ -1082,118 +1236,28 @@ TMQ_EXPORT int tmq_quantize_per_channel(const float* x, void* q, int64_t outer, 
                                         int64_t inner, const double* scales,
                                         const int64_t* zero_points, int q_signed,
                                         tmq_stream_t stream) {
-  if (!pc_args_ok(x, q, outer, channels, inner, scales, zero_points))
-    return TMQ_ERR_INVALID_ARGUMENT;
-  const int64_t n = outer * channels * inner;
-  if (n == 0) return TMQ_OK;
-  hipStream_t s = as_stream(stream);
-  uint8_t* qb = static_cast<uint8_t*>(q);
-  const bool vec = inner % 4 == 0 && aligned(x, 16) && aligned(q, 4);
-  if (q_signed ? launch_pc_rows(PcQuantize<true>{x, qb, scales, zero_points}, outer, channels, inner, vec, s)
-               : launch_pc_rows(PcQuantize<false>{x, qb, scales, zero_points}, outer, channels, inner, vec, s))
-    return launch_status();
-  const unsigned g = grid_for(n, kThreads * (vec ? 4 : 1), 1 << 20);
-  if (vec) {
-    if (q_signed)
-      quantize_pc_kernel<true, 4><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-    else
-      quantize_pc_kernel<false, 4><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-  } else {
-    if (q_signed)
-      quantize_pc_kernel<true, 1><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-    else
-      quantize_pc_kernel<false, 1><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-  }
-  return launch_status();
+  return per_channel(0, 0, x, q, outer, channels, inner, scales, zero_points, q_signed, stream);
 }
 
 TMQ_EXPORT int tmq_dequantize_per_channel(const void* q, float* r, int64_t outer, int64_t channels,
                                           int64_t inner, const double* scales,
                                           const int64_t* zero_points, int q_signed,
                                           tmq_stream_t stream) {
-  if (!pc_args_ok(q, r, outer, channels, inner, scales, zero_points))
-    return TMQ_ERR_INVALID_ARGUMENT;
-  const int64_t n = outer * channels * inner;
-  if (n == 0) return TMQ_OK;
-  hipStream_t s = as_stream(stream);
-  const uint8_t* qb = static_cast<const uint8_t*>(q);
-  const bool vec = inner % 4 == 0 && aligned(r, 16) && aligned(q, 4);
-  if (q_signed ? launch_pc_rows(PcDequantize<true>{qb, r, scales, zero_points}, outer, channels, inner, vec, s)
-               : launch_pc_rows(PcDequantize<false>{qb, r, scales, zero_points}, outer, channels, inner, vec, s))
-    return launch_status();
-  const unsigned g = grid_for(n, kThreads * (vec ? 4 : 1), 1 << 20);
-  if (vec) {
-    if (q_signed)
-      dequantize_pc_kernel<true, 4><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-    else
-      dequantize_pc_kernel<false, 4><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-  } else {
-    if (q_signed)
-      dequantize_pc_kernel<true, 1><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-    else
-      dequantize_pc_kernel<false, 1><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-  }
-  return launch_status();
+  return per_channel(1, 0, r, q, outer, channels, inner, scales, zero_points, q_signed, stream);
 }
 
 TMQ_EXPORT int tmq_quantize_per_channel_float_qparams(const float* x, void* q, int64_t outer,
                                                       int64_t channels, int64_t inner,
                                                       const float* scales, const float* zero_points,
                                                       int q_signed, tmq_stream_t stream) {
-  if (outer < 0 || channels < 0 || inner < 0) return TMQ_ERR_INVALID_ARGUMENT;
-  const int64_t n = outer * channels * inner;
-  if (n == 0) return TMQ_OK;
-  if (x == nullptr || q == nullptr || scales == nullptr || zero_points == nullptr)
-    return TMQ_ERR_INVALID_ARGUMENT;
-  hipStream_t s = as_stream(stream);
-  uint8_t* qb = static_cast<uint8_t*>(q);
-  const bool vec = inner % 4 == 0 && aligned(x, 16) && aligned(q, 4);
-  if (q_signed ? launch_pc_rows(PcfQuantize<true>{x, qb, scales, zero_points}, outer, channels, inner, vec, s)
-               : launch_pc_rows(PcfQuantize<false>{x, qb, scales, zero_points}, outer, channels, inner, vec, s))
-    return launch_status();
-  const unsigned g = grid_for(n, kThreads * (vec ? 4 : 1), 1 << 20);
-  if (vec) {
-    if (q_signed)
-      quantize_pcf_kernel<true, 4><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-    else
-      quantize_pcf_kernel<false, 4><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-  } else {
-    if (q_signed)
-      quantize_pcf_kernel<true, 1><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-    else
-      quantize_pcf_kernel<false, 1><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, channels, inner, scales, zero_points);
-  }
-  return launch_status();
+  return per_channel(0, 1, x, q, outer, channels, inner, scales, zero_points, q_signed, stream);
 }
 
 TMQ_EXPORT int tmq_dequantize_per_channel_float_qparams(const void* q, float* r, int64_t outer,
                                                         int64_t channels, int64_t inner,
                                                         const float* scales, const float* zero_points,
                                                         int q_signed, tmq_stream_t stream) {
-  if (outer < 0 || channels < 0 || inner < 0) return TMQ_ERR_INVALID_ARGUMENT;
-  const int64_t n = outer * channels * inner;
-  if (n == 0) return TMQ_OK;
-  if (r == nullptr || q == nullptr || scales == nullptr || zero_points == nullptr)
-    return TMQ_ERR_INVALID_ARGUMENT;
-  hipStream_t s = as_stream(stream);
-  const uint8_t* qb = static_cast<const uint8_t*>(q);
-  const bool vec = inner % 4 == 0 && aligned(r, 16) && aligned(q, 4);
-  if (q_signed ? launch_pc_rows(PcfDequantize<true>{qb, r, scales, zero_points}, outer, channels, inner, vec, s)
-               : launch_pc_rows(PcfDequantize<false>{qb, r, scales, zero_points}, outer, channels, inner, vec, s))
-    return launch_status();
-  const unsigned g = grid_for(n, kThreads * (vec ? 4 : 1), 1 << 20);
-  if (vec) {
-    if (q_signed)
-      dequantize_pcf_kernel<true, 4><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-    else
-      dequantize_pcf_kernel<false, 4><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-  } else {
-    if (q_signed)
-      dequantize_pcf_kernel<true, 1><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-    else
-      dequantize_pcf_kernel<false, 1><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, channels, inner, scales, zero_points);
-  }
-  return launch_status();
+  return per_channel(1, 1, r, q, outer, channels, inner, scales, zero_points, q_signed, stream);
 }
 
 TMQ_EXPORT const char* tmq_status_string(int status) {
