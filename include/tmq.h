@@ -132,6 +132,13 @@ int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, i
                                            int reduce_range, int rounding, tmq_qparams* qparams,
                                            void* workspace, size_t workspace_bytes,
                                            tmq_host_report* report, uint32_t ticket, tmq_stream_t stream);
+/* The same for M rows of K values -> rows of `pitch` codes, pitch a multiple of
+ * 16 that is at least K: what tmq_linear wants of activations whose K is not.
+ * The codes behind a row's end are undefined (the packed weights are zero there).
+ * Two launches; `workspace` 8-byte aligned. */
+int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
+                                  int reduce_range, int rounding, tmq_qparams* qparams,
+                                  void* workspace, size_t workspace_bytes, tmq_stream_t stream);
 /* Host-side ChooseQuantizationParams, same arithmetic (pure CPU, no GPU call). */
 int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
                             double* scale, int32_t* zero_point);
@@ -256,6 +263,12 @@ int tmq_linear(const tmq_linear_desc* desc, tmq_stream_t stream);
  * anyway.  No counterpart in the reference: muDNN allocates its own scratch
  * through the InternalMemAlloc callback (torch_musa/csrc/aten/utils/Utils.cpp:79-153). */
 int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* Everything the call can make use of as `workspace`: the above, and for
+ * activations off the 16-byte grid (K no multiple of 16, or on_grid == 0: their
+ * pointer or row pitch is none) room for a copy of the rows on it, which lets the
+ * vector kernels run them.  Without it such products fall back to a byte-wise
+ * kernel, a hundred times slower; up to 16 rows of 16 and more bytes need none. */
+int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid);
 /* The split behind that figure: *splits runs of *stages k-stages (64 bytes of K
  * each), the last run taking everything that is left; *splits == 1: no split.
  * Pure host arithmetic, no GPU call. */
@@ -283,7 +296,9 @@ typedef struct tmq_linear_choice {
 enum tmq_linear_output_kind { TMQ_LINEAR_OUT_BYTES = 0, TMQ_LINEAR_OUT_F32 = 1, TMQ_LINEAR_OUT_ACC32 = 2 };
 /* flags: bits 0-1 a tmq_linear_output_kind; bit 2: a workspace of
  * tmq_linear_workspace_bytes(M, N, K) is attached; bit 3: K, the row pitch or
- * the activation pointer is not a multiple of 16 (the plain kernel's case).
+ * the activation pointer is not a multiple of 16 (without scratch: the plain
+ * kernel's case, which is what is reported; with tmq_linear_scratch_bytes the
+ * kernel of the shape with K rounded up to 16 runs).
  * forced_kernel: tmq_linear_desc::kernel (0 = automatic).  compute_units: of
  * the device the product would run on (the persistent kernel's grid follows it). */
 int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t ldx, int32_t flags, int32_t forced_kernel,

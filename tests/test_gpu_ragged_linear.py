@@ -1,0 +1,53 @@
+"""quantized::linear and linear_dynamic on feature counts and pointers off the 16-byte grid, against PyTorch's CPU
+operators: the streaming kernel on unaligned rows, the copy onto the grid, the one-launch dynamic kernels."""
+import pytest
+import torch
+import torch_musa_amd  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+OPS = torch.ops.quantized
+
+SHAPES = [(1, 16, 5), (1, 17, 3), (16, 31, 16), (2, 63, 17), (7, 65, 33), (16, 1000, 40), (3, 4100, 64), (5, 8191, 20),
+          (1, 1, 4), (16, 15, 9), (17, 7, 5), (17, 17, 18), (33, 100, 64), (64, 129, 63), (65, 1000, 130),
+          (130, 2051, 100), (517, 1000, 2051), (70, 8200, 96), (300, 72, 1000)]
+
+
+def _weight(n, k, per_channel, gen):
+    w = torch.randn(n, k, generator=gen) * 0.02
+    if per_channel:
+        return torch.quantize_per_channel(w, w.abs().amax(1).double().clamp_min(1e-6) / 127,
+                                          torch.zeros(n, dtype=torch.long), 0, torch.qint8)
+    return torch.quantize_per_tensor(w, float(w.abs().max()) / 127, 0, torch.qint8)
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("per_channel", [True, False])
+def test_static(m, k, n, per_channel):
+    gen = torch.Generator().manual_seed(m * 7919 + k * 31 + n)
+    w, b = _weight(n, k, per_channel, gen), torch.randn(n, generator=gen)
+    x = torch.quantize_per_tensor(torch.randn(m, k, generator=gen), 0.03, 121, torch.quint8)
+    scale = 0.03 * max(k, 4) ** 0.5
+    op = OPS.linear_relu if m % 2 else OPS.linear
+    want = op(x, OPS.linear_prepack(w, b), scale, 99).int_repr()
+    packed = OPS.linear_prepack(w.cuda(), b.cuda())
+    print("[case]", m, k, n, per_channel, flush=True)
+    got = op(x.cuda(), packed, scale, 99).int_repr().cpu()
+    assert torch.equal(got, want)
+    # the same rows one byte into their storage
+    codes = torch.empty(m * k + 1, dtype=torch.uint8, device="cuda")[1:].view(m, k).copy_(x.int_repr().cuda())
+    view = torch._make_per_tensor_quantized_tensor(codes, 0.03, 121)
+    assert torch.equal(op(view, packed, scale, 99).int_repr().cpu(), want)
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES + [(16, 1022, 33), (16, 2047, 20), (4, 8190, 33), (1, 16383, 17)])
+def test_dynamic(m, k, n):
+    gen = torch.Generator().manual_seed(m * 104729 + k * 17 + n)
+    w, b = _weight(n, k, m % 3 == 0, gen), torch.randn(n, generator=gen)
+    x = torch.randn(m, k, generator=gen) + 0.5
+    want = OPS.linear_dynamic(x, OPS.linear_prepack(w, b), False)
+    print("[case]", m, k, n, flush=True)
+    packed = OPS.linear_prepack(w.cuda(), b.cuda())
+    got = OPS.linear_dynamic(x.cuda(), packed, False).cpu()
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5 * float(want.abs().max()) + 1e-7)
+    view = torch.empty(m * k + 1, device="cuda")[1:].view(m, k).copy_(x.cuda())
+    assert torch.equal(OPS.linear_dynamic(view, packed, False).cpu(), got)

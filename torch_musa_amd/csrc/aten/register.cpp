@@ -98,11 +98,12 @@ void check_status(int status, const char* what) {
   TORCH_CHECK(status == TMQ_OK, what, " failed: ", tmq_status_string(status));
 }
 
-// Scratch memory for the split-K schedule of products with a few hundred rows:
-// allocated through the caching allocator (stream-ordered reuse), attached to
+// Scratch memory for the split-K schedule of products with a few hundred rows and
+// for activations off the 16-byte grid: allocated through the caching allocator (stream-ordered reuse), attached to
 // the descriptor, kept alive by the returned tensor until the call is queued.
 at::Tensor attach_linear_workspace(tmq_linear_desc& d, const at::Tensor& like) {
-  const int64_t bytes = tmq_linear_workspace_bytes(d.M, d.N, d.K);
+  const bool on_grid = d.ldx % 16 == 0 && reinterpret_cast<uintptr_t>(d.x) % 16 == 0;
+  const int64_t bytes = tmq_linear_scratch_bytes(d.M, d.N, d.K, on_grid);
   if (bytes <= 0) return at::Tensor();
   at::Tensor ws = empty_bytes(bytes, like);
   d.workspace = ws.data_ptr();
@@ -521,7 +522,7 @@ struct PackedLinearWeightTmq final : public LinearPackedParamsBase {
       return relu ? y.clamp_min_(0) : y;
     }
     const auto stream = current_stream(x);
-    if (tmq_linear_dynamic_small_takes(M, N_, K_) != 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0) {
+    if (tmq_linear_dynamic_small_takes(M, N_, K_) != 0) {
       // a handful of rows: range, parameters, codes and product in one launch
       tmq_linear_desc d{};
       d.M = M;
@@ -537,23 +538,29 @@ struct PackedLinearWeightTmq final : public LinearPackedParamsBase {
                    "tmq_linear_dynamic_small");
       return y;
     }
-    // one allocation: the codes, the partial ranges, the parameters
-    const int64_t code_bytes = (x.numel() + 255) / 256 * 256;
+    // one allocation: the codes (rows on the 16-byte grid), the partial ranges, the parameters
+    const int64_t pitch = (K_ + 15) / 16 * 16;
+    const int64_t code_bytes = (M * pitch + 255) / 256 * 256;
     const int64_t range_bytes = (static_cast<int64_t>(tmq_minmax_workspace_bytes(x.numel())) + 255) / 256 * 256;
     const at::Tensor scratch = empty_bytes(code_bytes + range_bytes + static_cast<int64_t>(sizeof(tmq_qparams)), x);
     auto* xq = static_cast<uint8_t*>(scratch.data_ptr());
     auto* qpd = reinterpret_cast<tmq_qparams*>(xq + code_bytes + range_bytes);
     // the CPU op quantizes the activations while packing them, with product and
     // zero point rounded once
-    check_status(tmq_quantize_per_tensor_dynamic_dev(cptr<float>(x), xq, x.numel(), 0, reduce_range, TMQ_ROUND_FUSED, qpd,
-                                                     xq + code_bytes, static_cast<size_t>(range_bytes), stream),
-                 "tmq_quantize_per_tensor_dynamic_dev");
+    check_status(pitch == K_
+                     ? tmq_quantize_per_tensor_dynamic_dev(cptr<float>(x), xq, x.numel(), 0, reduce_range,
+                                                           TMQ_ROUND_FUSED, qpd, xq + code_bytes,
+                                                           static_cast<size_t>(range_bytes), stream)
+                     : tmq_quantize_rows_dynamic_dev(cptr<float>(x), xq, M, K_, pitch, 0, reduce_range,
+                                                     TMQ_ROUND_FUSED, qpd, xq + code_bytes,
+                                                     static_cast<size_t>(range_bytes), stream),
+                 "quantized::linear_dynamic: quantizing the activations");
     tmq_linear_desc d{};
     d.M = M;
     d.N = N_;
-    d.K = K_;
+    d.K = pitch;  // (the packed weights are zero from K on)
     d.x = xq;
-    d.ldx = K_;
+    d.ldx = pitch;
     d.x_signed = 0;
     d.x_scale = 1.f;  // unused: read from qp on the device
     d.w_packed = packed_.const_data_ptr();

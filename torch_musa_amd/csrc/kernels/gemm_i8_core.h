@@ -165,6 +165,29 @@ struct __attribute__((packed, aligned(1))) V4iAnyAlignment {
 };
 __device__ __forceinline__ void st16_any(void* p, v4i v) { reinterpret_cast<V4iAnyAlignment*>(p)->v = v; }
 __device__ __forceinline__ v4i ld16_any(const void* p) { return reinterpret_cast<const V4iAnyAlignment*>(p)->v; }
+// Bytes s ... 15 of a 16-byte value moved to its front, zeros behind them (s = 0 ... 15).  The last 16-byte
+// chunk of a row whose length is no multiple of 16 is read as the row's last 16 bytes and shifted down,
+// so that nothing outside the row is touched.
+__device__ __forceinline__ v4i shift_down_bytes(v4i v, int s) {
+  const uint64_t lo = (static_cast<uint64_t>(static_cast<uint32_t>(v.y)) << 32) | static_cast<uint32_t>(v.x);
+  const uint64_t hi = (static_cast<uint64_t>(static_cast<uint32_t>(v.w)) << 32) | static_cast<uint32_t>(v.z);
+  const int b = 8 * s;  // 0 ... 120
+  const uint64_t nlo = b == 0 ? lo : b < 64 ? (lo >> b) | (hi << (64 - b)) : hi >> (b - 64);
+  const uint64_t nhi = b < 64 ? hi >> b : 0;
+  return v4i{static_cast<int>(nlo), static_cast<int>(nlo >> 32), static_cast<int>(nhi), static_cast<int>(nhi >> 32)};
+}
+// Four fp32 values 4 c4 ... 4 c4 + 3 of a row of K >= 4 values (4-byte aligned), zeros behind its
+// end, by the same clamped load.  (A zero does not change the range of a dynamic quantization:
+// ChooseQuantizationParams extends every range to hold 0.)
+struct __attribute__((packed, aligned(4))) V4fRow {
+  v4f v;
+};
+__device__ __forceinline__ v4f load_row4(const float* row, int c4, int K) {
+  const int at = 4 * c4 < K - 4 ? 4 * c4 : K - 4, s = 4 * c4 - at;
+  const v4f v = reinterpret_cast<const V4fRow*>(row + at)->v;
+  return v4f{s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w, s == 0 ? v.y : s == 1 ? v.z : s == 2 ? v.w : 0.f,
+             s == 0 ? v.z : s == 1 ? v.w : 0.f, s == 0 ? v.w : 0.f};
+}
 typedef int v2i __attribute__((ext_vector_type(2)));
 struct __attribute__((packed, aligned(1))) V2iAnyAlignment {
   v2i v;

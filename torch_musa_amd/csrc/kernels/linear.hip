@@ -112,7 +112,11 @@ constexpr int kDecodeRowsAuto = 16;  // up to here the automatic choice always s
 // results 4.5 us (the store's acknowledgement ends the kernel); one or two
 // accumulators and 4 / 8 / 16 waves all stay within 0.1 us.
 // flags: bits 0-7 M, bit 8 per-channel weight scales, bit 9 unsigned activations.
-template <int MODE, int MG>
+// RAGGED: K (>= 16), the row pitch or the activation pointer is no multiple of 16.  The
+// activation requests are the same 16 bytes per lane at whatever address the row has, the
+// last chunk of a row is shifted into place; one launch instead of a pass that copies the rows onto
+// the 16-byte grid first (that pass is what more rows take, and the vector path it then needs).
+template <int MODE, int MG, bool RAGGED = false>
 __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
     const uint8_t* __restrict__ w_packed, const uint8_t* __restrict__ x, const int32_t* __restrict__ colsum,
     const float* __restrict__ w_scales, const float* __restrict__ bias, int32_t K, int32_t ldx, int32_t N,
@@ -170,6 +174,20 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
   }
   const int xor_word = (flags >> 9) & 1 ? static_cast<int>(0x80808080u) : 0;
   const v4i xmask = {xor_word, xor_word, xor_word, xor_word};
+  // This lane's 16-byte piece of k-block kb of its row; `ok`: the piece has bytes of the row.
+  auto piece = [&](const uint8_t* row, int kb, bool ok) {
+    const int at = ok ? kb * 64 + sp * 16 : 0;
+    if constexpr (RAGGED) return ld16_any(row + (at <= K - 16 ? at : K - 16));
+    else return ld16(row + at);
+  };
+  // (behind the load, in the k-block that ends the row)
+  auto settle = [&](v4i v, int kb) {
+    if constexpr (RAGGED) {
+      const int over = kb * 64 + sp * 16 - (K - 16);
+      return over > 0 && over < 16 ? shift_down_bytes(v, over) : v;
+    }
+    return v;
+  };
   // Two accumulators per row group, used in turn: a multiply-accumulate does not
   // wait for the one before it.
   v4i acc2[MG][2];
@@ -195,7 +213,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
 #pragma unroll
         for (int mg = 0; mg < MG; ++mg) {
           xok[mg][u] = kb < KB && xrow[mg] && (kb * 64 + sp * 16 < K);
-          xf[mg][u] = ld16(xp[mg] + (xok[mg][u] ? kb * 64 + sp * 16 : 0));
+          xf[mg][u] = piece(xp[mg], kb, xok[mg][u]);
         }
       }
     }
@@ -208,7 +226,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
 #pragma unroll
         for (int mg = 0; mg < MG; ++mg) {
           xok[mg][u] = kb < KB && xrow[mg] && (kb * 64 + sp * 16 < K);
-          xf[mg][u] = ld16(xp[mg] + (xok[mg][u] ? kb * 64 + sp * 16 : 0));
+          xf[mg][u] = piece(xp[mg], kb, xok[mg][u]);
         }
       }
     }
@@ -216,7 +234,9 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
     for (int u = 0; u < kBatch; ++u)
 #pragma unroll
       for (int mg = 0; mg < MG; ++mg) {
-        const v4i xs = xok[mg][u] ? (xf[mg][u] ^ xmask) : v4i{0, 0, 0, 0};
+        v4i xw = xf[mg][u];
+        if (RAGGED && kb0 + u * kWaves == KB - 1) xw = settle(xw, KB - 1);  // (the same for the whole wave)
+        const v4i xs = xok[mg][u] ? (xw ^ xmask) : v4i{0, 0, 0, 0};
         v4i xv;
 #pragma unroll
         for (int c = 0; c < 4; ++c) xv[c] = __builtin_amdgcn_ds_bpermute(perm_addr, xs[c]);
@@ -307,7 +327,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
   constexpr int kWaves = kDecodeWaves;
   constexpr int kBatch = 8;
   static_assert(kHeld * 4 * kWaves * kWave <= kDynSmallMaxValues, "held values");
-  extern __shared__ __attribute__((aligned(16))) uint8_t sx[];  // [M][K + 16] activation codes
+  extern __shared__ __attribute__((aligned(16))) uint8_t sx[];  // [M][pitch] activation codes
   __shared__ int s_sum[4][kWave];  // the waves' partial sums, added with LDS atomics (see linear_decode_kernel)
   __shared__ float s_mn[kWaves], s_mx[kWaves];
   __shared__ float s_scale, s_inv, s_zp;
@@ -315,7 +335,8 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
   const int lr = lane & 15, lc = lane >> 4;
   const int64_t nb = blockIdx.x;
   const int64_t KB = ceil_div(a.K, 64);
-  const int pitch = static_cast<int>(a.K) + 16;  // rows 16 bytes apart in the banks
+  const int K = static_cast<int>(a.K);
+  const int pitch = (K + 15) / 16 * 16 + 16;  // rows 16 bytes apart in the banks
   const uint8_t* wp = a.w_packed + nb * a.w_kchunks * 256 + lc * 256 + lr * 16;
   // per-channel constants of the 64 finishing threads, requested first
   const int fm = t >> 2, fg = t & 3;
@@ -334,7 +355,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
   // ---- the input: requested first (loads return in order: behind the weight
   // stream it would arrive only after it), held in registers between the range
   // pass and the quantization
-  const int k4 = static_cast<int>(a.K / 4);
+  const int k4 = (K + 3) / 4;
   const int total4 = static_cast<int>(a.M) * k4;
   v4f held[kHeld];
 #pragma unroll
@@ -342,7 +363,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
     const int e = t + u * (kWaves * kWave);
     const int ec = e < total4 ? e : 0;  // unconditional loads keep the load counter exact
     const int row = ec / k4, c4 = ec - row * k4;
-    held[u] = *reinterpret_cast<const v4f*>(x + row * ldxf + c4 * 4);
+    held[u] = load_row4(x + row * ldxf, c4, K);
   }
   // then the first batch of weights: on its way while the input is processed
   v4i wf[kBatch];
@@ -426,7 +447,8 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
     for (int u = 0; u < kBatch; ++u) {
       const int64_t kb = kb0 + u * kWaves;
       const bool xok = kb < KB && xrow && (kb * 64 + lc * 16 < a.K);
-      // (weights of a block past K were loaded from a clamped address: the zero
+      // (bytes of LDS past the end of a row meet the zeros the packed weights end in;
+      // weights of a block past K were loaded from a clamped address: the zero
       // activation operand removes them from the sum, x ^ 0x80 alone would not)
       const v4i xf = xok ? ld16(xp + kb * 64) ^ xmask : v4i{0, 0, 0, 0};
       const v4i wv = kb < KB ? wf[u] : v4i{0, 0, 0, 0};
@@ -457,7 +479,33 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
 }
 
 // ---------------------------------------------------------------------------
-// Plain kernel: any K, any alignment.  One thread per (m, group of 4 channels).
+// Activation rows onto the 16-byte grid: K bytes at any address and pitch -> `chunks`
+// 16-byte chunks, zeros past K.  The copy that lets every vector kernel run a product whose
+// K or pointer is off that grid: M x K bytes in and out (the product reads them many times
+// over), against the plain kernel's byte-wise loop, which is all such products had: 517 rows
+// quantized, through 1000 -> 2051 -> 1000 features and dequantized: 4014 -> 27 us.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void regrid_rows_kernel(const uint8_t* __restrict__ x, int64_t ldx, int32_t K,
+                                                          uint32_t chunks, uint32_t total, v4i* __restrict__ out) {
+  const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= total) return;
+  const uint32_t row = id / chunks;
+  const int k0 = static_cast<int>(id - row * chunks) * 16;
+  const uint8_t* src = x + static_cast<int64_t>(row) * ldx;
+  v4i v = {0, 0, 0, 0};
+  if (K >= 16) {
+    const int at = k0 <= K - 16 ? k0 : K - 16;
+    v = shift_down_bytes(ld16_any(src + at), k0 - at);
+  } else {
+    uint32_t w[4] = {0, 0, 0, 0};
+    for (int b = 0; b < K; ++b) w[b >> 2] |= static_cast<uint32_t>(src[b]) << (8 * (b & 3));
+    v = v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
+  }
+  out[id] = v;
+}
+
+// ---------------------------------------------------------------------------
+// Plain kernel: any K, any alignment, no scratch memory.  One thread per (m, group of 4 channels).
 // ---------------------------------------------------------------------------
 template <int MODE>
 __global__ __launch_bounds__(256) void linear_plain_kernel(GemmArgs a, XLinear xs, int x_signed) {
@@ -598,6 +646,30 @@ int launch_gemm_persistent(const GemmArgs& a, const XLinear& xs, hipStream_t s) 
   } else {
     return TMQ_ERR_UNSUPPORTED;
   }
+}
+
+// Scratch for activation rows that are off the 16-byte grid (regrid_rows_kernel).
+int64_t regrid_pitch(int64_t K) { return round_up(K, 16); }
+int64_t regrid_bytes(int64_t M, int64_t K) { return round_up(M * regrid_pitch(K), 256); }
+// (the copy's index arithmetic is 32 bits wide: up to 32 GiB of activations)
+bool regrid_limits_ok(int64_t M, int64_t K) { return K > 0 && K <= 0x7fffff00 && M * (regrid_pitch(K) / 16) <= 0x7fffff00; }
+int launch_regrid(const XLinear& xs, int64_t M, int64_t K, void* out, hipStream_t s) {
+  const int64_t chunks = regrid_pitch(K) / 16, total = M * chunks;
+  regrid_rows_kernel<<<dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s>>>(
+      xs.x, xs.ldx, static_cast<int32_t>(K), static_cast<uint32_t>(chunks), static_cast<uint32_t>(total),
+      static_cast<v4i*>(out));
+  return launch_status();
+}
+
+// Weight streaming for up to 16 rows that are off the 16-byte grid.
+template <int MODE>
+int launch_linear_decode_ragged(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
+  const uint32_t flags = static_cast<uint32_t>(a.M) | (a.w_scale_stride != 0 ? 0x100u : 0u) |
+                         (a.x_xor != 0 ? 0x200u : 0u);
+  linear_decode_kernel<MODE, 1, true><<<dim3(static_cast<unsigned>(ceil_div(a.N, 16))), dim3(kDecodeWaves * kWave), 0, s>>>(
+      a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, static_cast<int32_t>(a.K), static_cast<int32_t>(xs.ldx),
+      static_cast<int32_t>(a.N), flags, a);
+  return launch_status();
 }
 
 // Weight streaming for up to 64 rows: one block per 16 channels.
@@ -1179,6 +1251,25 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
   q.workspace_attached = workspace != nullptr;
   q.workspace_bytes = workspace != nullptr && aligned(workspace, 16) ? workspace_bytes : 0;
   if (a.splits != 1) return TMQ_ERR_INVALID_ARGUMENT;  // the split is this function's to plan
+  if (!vec_ok && forced < 0) {
+    // Off the 16-byte grid: up to 16 rows stream the weights as they are (the copy would cost a
+    // launch, more than any other kernel's advantage at so few rows); more rows are copied onto
+    // the grid if the caller left room for that, and take the kernel of the padded shape.
+    if (a.M <= kDecodeRowsAuto && a.K >= 16 && stream_limits_ok(q) && a.w_kchunks == packed_kchunks(a.K))
+      return launch_linear_decode_ragged<MODE>(a, xs, s);
+    const int64_t room = regrid_bytes(a.M, a.K);
+    if (regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room) {
+      const int rc = launch_regrid(xs, a.M, a.K, workspace, s);
+      if (rc != TMQ_OK) return rc;
+      GemmArgs b = a;
+      b.K = regrid_pitch(a.K);  // (the packed weights are zero from K on, up to a multiple of 128)
+      const XLinear on_grid{static_cast<const uint8_t*>(workspace), b.K};
+      const bool rest = workspace_bytes > room;
+      return dispatch_linear<MODE>(b, on_grid, x_signed, true, forced, s,
+                                   rest ? static_cast<uint8_t*>(workspace) + room : nullptr,
+                                   rest ? workspace_bytes - room : 0);
+    }
+  }
   const LinearChoice c = choose_linear(q, forced);
   switch (c.cfg) {
     case 9: {
@@ -1297,6 +1388,13 @@ TMQ_EXPORT int tmq_linear_unpack(const void* packed, int64_t N, int64_t K, int8_
 TMQ_EXPORT int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return split_workspace_bytes(plan_split(M, N, K), M);
+}
+
+TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (K % 16 == 0 && on_grid) return tmq_linear_workspace_bytes(M, N, K);
+  if ((M <= kDecodeRowsAuto && K >= 16) || !regrid_limits_ok(M, K)) return 0;
+  return regrid_bytes(M, K) + tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
 }
 
 TMQ_EXPORT int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int32_t* stages) {
@@ -1504,11 +1602,19 @@ TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qpa
 // CU then reads 256 KB of rows: 14.2 us against 11.0 us for the two launches at N = 4096).
 constexpr int64_t kDynResidentMaxValues = 32768;
 
+namespace {
+// Groups of four values, the last one of a row perhaps partly behind its end.
+int64_t dyn_groups(int64_t M, int64_t K) { return M * ceil_div(K, 4); }
+bool dyn_resident_ok(int64_t M, int64_t N, int64_t K, int cus) {
+  return 4 * dyn_groups(M, K) <= kDynResidentMaxValues && resident_limits_ok(M, N, round_up(K, 16), K, cus);
+}
+}  // namespace
+
 TMQ_EXPORT int tmq_linear_dynamic_small_takes(int64_t M, int64_t N, int64_t K) {
-  if (M < 1 || M > 16 || N < 1 || K < 16 || K % 16 != 0 || ceil_div(N, 16) > 0x7fffffff) return 0;
-  if (M * K <= kDynSmallMaxValues) return 1;
+  if (M < 1 || M > 16 || N < 1 || K < 16 || ceil_div(N, 16) > 0x7fffffff) return 0;
+  if (4 * dyn_groups(M, K) <= kDynSmallMaxValues) return 1;
   const int cus = cu_count();
-  return M * K <= kDynResidentMaxValues && resident_limits_ok(M, N, K, K, cus > 0 ? cus : 256) ? 1 : 0;
+  return dyn_resident_ok(M, N, K, cus > 0 ? cus : 256) ? 1 : 0;
 }
 
 TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x, int64_t ldx, int reduce_range,
@@ -1516,11 +1622,11 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
   if (d == nullptr) return TMQ_ERR_INVALID_ARGUMENT;
   if (d->M < 0 || d->N < 0 || d->K < 0) return TMQ_ERR_INVALID_ARGUMENT;
   if (d->M == 0 || d->N == 0) return TMQ_OK;
-  if (d->M > 16 || d->K < 16 || d->K % 16 != 0) return TMQ_ERR_UNSUPPORTED;
+  if (d->M > 16 || d->K < 16) return TMQ_ERR_UNSUPPORTED;
   if (x == nullptr || y == nullptr || d->w_packed == nullptr || d->w_colsum == nullptr || d->w_scales == nullptr)
     return TMQ_ERR_INVALID_ARGUMENT;
   if (ldx < d->K || ldy < d->N) return TMQ_ERR_INVALID_ARGUMENT;
-  if (!aligned(x, 16) || ldx % 4 != 0 || !aligned(d->w_packed, 16) || !aligned(y, 4)) return TMQ_ERR_UNSUPPORTED;
+  if (!aligned(x, 4) || !aligned(d->w_packed, 16) || !aligned(y, 4)) return TMQ_ERR_UNSUPPORTED;
   const int64_t blocks = ceil_div(d->N, 16);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   GemmArgs a{};
@@ -1541,8 +1647,8 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
   // one block per CU that does it once for all its channel groups (up to 32768 values, K <= 8192).
   // desc->kernel pins one for tests: 9 the first, 29 the second.
   const int cus = cu_count();
-  const bool resident_ok = d->M * d->K <= kDynResidentMaxValues && resident_limits_ok(d->M, d->N, d->K, d->K, cus);
-  const bool small_ok = d->M * d->K <= kDynSmallMaxValues;
+  const bool resident_ok = dyn_resident_ok(d->M, d->N, d->K, cus);
+  const bool small_ok = 4 * dyn_groups(d->M, d->K) <= kDynSmallMaxValues;
   if ((d->kernel == 9 && !small_ok) || (d->kernel == 29 && !resident_ok) || (!small_ok && !resident_ok))
     return TMQ_ERR_UNSUPPORTED;
   const bool resident =
@@ -1550,7 +1656,7 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
   if (resident) {
     const XLinear none{nullptr, 0};
     const dim3 grid(static_cast<unsigned>(blocks < cus ? blocks : cus)), block(kResidentThreads);
-    const int64_t held = ceil_div(d->M * d->K / 4, kResidentThreads);  // float4 per thread
+    const int64_t held = ceil_div(dyn_groups(d->M, d->K), kResidentThreads);  // float4 per thread
     if (held <= 2)
       linear_resident_kernel<kOutF32, 1, kResidentWaves, 2><<<grid, block, 0, s>>>(a, none, x, ldx, reduce_range);
     else if (held <= 4)
@@ -1559,9 +1665,9 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
       linear_resident_kernel<kOutF32, 1, kResidentWaves, 8><<<grid, block, 0, s>>>(a, none, x, ldx, reduce_range);
     return launch_status();
   }
-  const size_t lds = static_cast<size_t>(d->M) * static_cast<size_t>(d->K + 16);
+  const size_t lds = static_cast<size_t>(d->M) * static_cast<size_t>(round_up(d->K, 16) + 16);
   const dim3 grid(static_cast<unsigned>(blocks)), block(kDecodeWaves * kWave);
-  const int64_t groups = ceil_div(d->M * d->K / 4, kDecodeWaves * kWave);  // float4 per thread
+  const int64_t groups = ceil_div(dyn_groups(d->M, d->K), kDecodeWaves * kWave);  // float4 per thread
   if (groups <= 1)
     linear_decode_dynamic_kernel<1><<<grid, block, lds, s>>>(a, x, ldx, reduce_range);
   else if (groups <= 2)

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
   const int lr = lane & 15, lc = lane >> 4;
   const int K = static_cast<int>(a.K), M = static_cast<int>(a.M), N = static_cast<int>(a.N);
   const int KB = (K + 63) >> 6;                    // 64-byte k-blocks
-  const int KC = K >> 4;                           // 16-byte chunks (K is a multiple of 16)
+  const int KC = K >> 4;                           // 16-byte chunks of a row of codes (K is a multiple of 16 there)
   const int NG = (N + 15) >> 4;                    // channel groups
   const int G = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
   const int ngb = (NG - b + G - 1) / G;            // groups of this block (G <= NG: at least one)
@@ -90,14 +90,14 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
   constexpr int kHeldN = HELD > 0 ? HELD : 1;
   v4f held[kHeldN];
   const int sr = lane >> 2, sp = lane & 3;
-  const int k4 = K >> 2, total4 = M * k4;          // (dynamic form) groups of four float values
+  const int k4 = (K + 3) >> 2, total4 = M * k4;    // (dynamic form) groups of four float values
   if constexpr (HELD > 0) {
 #pragma unroll
     for (int u = 0; u < HELD; ++u) {
       const int e = t + u * kThreads;
       const int ec = e < total4 ? e : 0;           // unconditional loads keep the load counter exact
       const int row = ec / k4, c4 = ec - row * k4;
-      held[u] = *reinterpret_cast<const v4f*>(xf + row * ldxf + c4 * 4);
+      held[u] = load_row4(xf + row * ldxf, c4, K);
     }
   } else {
 #pragma unroll

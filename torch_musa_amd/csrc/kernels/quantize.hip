@@ -443,6 +443,61 @@ __global__ __launch_bounds__(kThreads) void quantize_after_minmax_kernel(
   }
 }
 
+// The same for rows that the product behind it wants on the 16-byte grid: `M` rows of K values
+// -> rows of `pitch` codes (a multiple of 16, less than 16 over K), a word of four codes per lane.
+// The codes behind a row's end are whatever the last values give; they meet zero weights.
+template <bool SIGNED, bool FUSED>
+__global__ __launch_bounds__(kThreads) void quantize_rows_after_minmax_kernel(
+    const float* __restrict__ x, uint32_t* __restrict__ q4, int64_t M, int32_t K, int32_t pitch4,
+    const float* __restrict__ partials, int count, int qmin, int qmax, int reduce_range, tmq_qparams* __restrict__ out) {
+  __shared__ float s_mm[2];
+  __shared__ float s_inv, s_zp;
+  float mn = std::numeric_limits<float>::infinity();
+  float mx = -std::numeric_limits<float>::infinity();
+  for (int i = threadIdx.x; i < count; i += kThreads) {
+    const float2 p = *reinterpret_cast<const float2*>(partials + 2 * i);
+    mn = fminf(mn, p.x);
+    mx = fmaxf(mx, p.y);
+  }
+  block_minmax_store(mn, mx, s_mm);
+  if (threadIdx.x == 0) {
+    double sc;
+    int32_t z;
+    choose_qparams(s_mm[0], s_mm[1], qmin, qmax, reduce_range != 0, &sc, &z);
+    s_inv = 1.0f / static_cast<float>(sc);  // IEEE division, as resolve()
+    s_zp = static_cast<float>(z);
+    if (blockIdx.x == 0) {
+      out->scale = sc;
+      out->zero_point = z;
+      out->reserved = 0;
+    }
+  }
+  __syncthreads();
+  const float inv = s_inv, zp_f = s_zp;
+  const int64_t total = M * pitch4, step = static_cast<int64_t>(gridDim.x) * kThreads;
+  int64_t g = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  int64_t row = g / pitch4;
+  int c4 = static_cast<int>(g - row * pitch4);
+  const int64_t step_rows = step / pitch4;  // (one division each, not one per word)
+  const int step_c4 = static_cast<int>(step - step_rows * pitch4);
+  for (; g < total; g += step) {
+    const float* src = x + row * K;
+    v4f v = {0.f, 0.f, 0.f, 0.f};
+    if (4 * c4 + 4 <= K) {
+      __builtin_memcpy(&v, src + 4 * c4, 16);
+    } else {
+      for (int j = 0; 4 * c4 + j < K; ++j) v[j] = src[4 * c4 + j];
+    }
+    q4[g] = quantize_four<SIGNED, FUSED>(v, inv, zp_f);
+    row += step_rows;
+    c4 += step_c4;
+    if (c4 >= pitch4) {
+      c4 -= pitch4;
+      ++row;
+    }
+  }
+}
+
 // Dynamic quantization of a small tensor in one launch: one block finds the
 // range, chooses the parameters and converts.  A decode-sized activation
 // ([1..16, 4096] floats) is a few tens of KB: three dependent launches would
@@ -1181,6 +1236,38 @@ TMQ_EXPORT int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, i
   if (report == nullptr || n <= 0) return TMQ_ERR_INVALID_ARGUMENT;
   return quantize_dynamic(x, q, n, q_signed, reduce_range, rounding, qparams, workspace, workspace_bytes,
                           RangeReport{report, ticket}, stream);
+}
+
+TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
+                                             int reduce_range, int rounding, tmq_qparams* qparams, void* workspace,
+                                             size_t workspace_bytes, tmq_stream_t stream) {
+  if (M < 1 || K < 1 || K > 0x7fffff00 || pitch % 16 != 0 || pitch < K || x == nullptr || q == nullptr || qparams == nullptr)
+    return TMQ_ERR_INVALID_ARGUMENT;
+  if (rounding != TMQ_ROUND_PRODUCT && rounding != TMQ_ROUND_FUSED) return TMQ_ERR_INVALID_ARGUMENT;
+  if (!aligned(x, 4) || !aligned(q, 4)) return TMQ_ERR_ALIGNMENT;
+  if (workspace == nullptr || workspace_bytes < tmq_minmax_workspace_bytes(M * K) || !aligned(workspace, 8))
+    return TMQ_ERR_WORKSPACE;
+  hipStream_t s = as_stream(stream);
+  const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
+  float* partials = static_cast<float*>(workspace);
+  const int64_t n = M * K;
+  const uintptr_t mis = reinterpret_cast<uintptr_t>(x) & 15u;
+  int64_t head = mis == 0 ? 0 : static_cast<int64_t>((16 - mis) / 4);
+  if (head > n) head = n;
+  const int64_t n4 = (n - head) / 4;
+  const int count = static_cast<int>(grid_for(n4, kThreads * kUnroll, kDynPartials));
+  minmax_partial_kernel<true><<<dim3(count), dim3(kThreads), 0, s>>>(reinterpret_cast<const v4f*>(x + head), n4, x, head, n,
+                                                                    partials);
+  if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
+  const dim3 grid(grid_for(M * (pitch / 4), kThreads * 2, kDynQBlocks)), block(kThreads);
+  auto go = [&](auto kernel) {
+    kernel<<<grid, block, 0, s>>>(x, static_cast<uint32_t*>(q), M, static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4),
+                                  partials, count, qmin, qmax, reduce_range, qparams);
+    return launch_status();
+  };
+  const bool fused = rounding == TMQ_ROUND_FUSED;
+  if (q_signed) return fused ? go(quantize_rows_after_minmax_kernel<true, true>) : go(quantize_rows_after_minmax_kernel<true, false>);
+  return fused ? go(quantize_rows_after_minmax_kernel<false, true>) : go(quantize_rows_after_minmax_kernel<false, false>);
 }
 
 TMQ_EXPORT int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
