@@ -344,10 +344,15 @@ int tmq_linear_acc32(const tmq_linear_desc* desc, int32_t* acc, int64_t ldacc,
  * seeing the parameters. */
 int tmq_linear_f32(const tmq_linear_desc* desc, const tmq_qparams* x_qparams_dev, float* y,
                    int64_t ldy, tmq_stream_t stream);
+/* The same with the results stored as fp32, bfloat16 or fp16 (rounded to nearest
+ * even from the fp32 value); ldy in elements. */
+enum tmq_float_kind { TMQ_FLOAT_F32 = 0, TMQ_FLOAT_BF16 = 1, TMQ_FLOAT_F16 = 2 };
+int tmq_linear_float(const tmq_linear_desc* desc, const tmq_qparams* x_qparams_dev, void* y, int64_t ldy, int kind,
+                     tmq_stream_t stream);
 
 /* The whole dynamically quantized linear for a handful of rows in one launch:
- * fp32 x [M, ldx] -> fp32 y [M, ldy] with M <= 16, K a multiple of 16, x 16-byte
- * aligned, ldx a multiple of 4, and either M * K <= 16384 (every block of the
+ * fp32 x [M, ldx] -> fp32 y [M, ldy] with M <= 16, K >= 16, and (K rounded up to
+ * a multiple of 4) either M * K <= 16384 (every block of the
  * weight-streaming kernel derives the activation range, parameters and codes
  * itself while its weights are on their way) or M * K <= 32768 with
  * 64 <= K <= 8192 (one block per CU does so once, keeps the codes in LDS and

@@ -51,3 +51,16 @@ def test_dynamic(m, k, n):
     assert torch.allclose(got, want, rtol=1e-5, atol=1e-5 * float(want.abs().max()) + 1e-7)
     view = torch.empty(m * k + 1, device="cuda")[1:].view(m, k).copy_(x.cuda())
     assert torch.equal(OPS.linear_dynamic(view, packed, False).cpu(), got)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 5), (7, 100, 33), (100, 320, 18), (300, 1024, 257), (64, 4096, 96),
+                                   (512, 64, 4099), (2600, 320, 1920)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_plain_tensor_linear_in_16_bits(m, k, n, dtype):
+    """The 16-bit outputs are the fp32 output rounded once."""
+    gen = torch.Generator().manual_seed(m + k + n)
+    x = torch.randint(0, 256, (m, k), dtype=torch.uint8, generator=gen).cuda()
+    w = torch.randint(-127, 128, (k, n), dtype=torch.int8, generator=gen).cuda()
+    ws, wz = (torch.rand(n, generator=gen) * 1e-3).cuda(), torch.zeros(n, dtype=torch.long).cuda()
+    call = lambda out: OPS.linear_per_tensor(x, 0.02, 120, w, ws, wz, None, 1.0, 0, out, "relu", [], "")  # noqa: E731
+    assert torch.equal(call(dtype), call(torch.float32).to(dtype))

@@ -1413,11 +1413,14 @@ at::Tensor qlinear_per_tensor_run(at::Tensor act, double act_scale, int64_t act_
     TORCH_CHECK(bias->numel() == N, what, ": bias must have ", N, " elements");
     b = bias->to(act.device(), at::kFloat).contiguous();
   }
-  const bool float_path = !o.is_int || post == "tanh" || post == "gelu";
-  at::Tensor y = empty_plain({M, N}, float_path ? at::kFloat : o.dtype, act);
+  // the product leaves the kernel in the output's type; only a post operation that the kernel does
+  // not have works on its fp32 value
+  const bool more = post == "tanh" || post == "gelu";
+  const bool float_path = !o.is_int || more;
+  at::Tensor y = empty_plain({M, N}, more ? at::kFloat : o.dtype, act);
   const auto stream = current_stream(act);
   const at::Tensor x = act.contiguous();
-  if (y.numel() == 0) return float_path ? plain_requant(y, output_scale, output_zero_point, o) : y;
+  if (y.numel() == 0) return more ? plain_requant(y, output_scale, output_zero_point, o) : y;
   // weight side: re-tiled copy, column sums and fp32 scales, made once per weight
   at::Tensor packed, colsum, ws;
   const std::array<int64_t, 8> geom{0, N, K, act.device().index(), 0, 0, 0, 0};
@@ -1452,7 +1455,9 @@ at::Tensor qlinear_per_tensor_run(at::Tensor act, double act_scale, int64_t act_
   d.bias = b.has_value() ? cptr<float>(*b) : nullptr;
   const at::Tensor split_ws = attach_linear_workspace(d, act);
   if (float_path) {
-    check_status(tmq_linear_f32(&d, nullptr, mptr<float>(y), N, stream), "tmq_linear_f32");
+    const int kind = y.scalar_type() == at::kBFloat16 ? TMQ_FLOAT_BF16 : y.scalar_type() == at::kHalf ? TMQ_FLOAT_F16 : TMQ_FLOAT_F32;
+    check_status(tmq_linear_float(&d, nullptr, y.data_ptr(), N, kind, stream), "tmq_linear_float");
+    if (!more) return y;
     if (post == "tanh") y = at::tanh(y);
     if (post == "gelu") y = at::gelu(y);
     return plain_requant(y, output_scale, output_zero_point, o);

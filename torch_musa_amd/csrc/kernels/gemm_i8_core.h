@@ -121,6 +121,8 @@ struct GemmArgs {
   // null: x_scale and acc_coef above hold.  acc_base is acc_coef + zero point.
   const tmq_qparams* x_qp_dev = nullptr;
   int32_t acc_base = 0;
+  // kOutF32: what the results are stored as (tmq_float_kind: fp32, bfloat16, fp16)
+  int32_t f_kind = 0;
   // Split K (raw int32 output of plain activation rows only): block row
   // blockIdx.y multiplies stages [y * split_stages, (y + 1) * split_stages) of
   // the k loop -- the last one everything from y * split_stages on -- and
@@ -140,21 +142,54 @@ __device__ __forceinline__ XQuant x_quant(const GemmArgs& a) {
   return XQuant{a.x_scale, a.acc_coef};
 }
 
-// Four float results of one output row (kOutF32), channels n .. n+3.
+// bfloat16 and fp16 bits of an fp32 value, rounded to nearest even (NaN: the quiet one).
+__device__ __forceinline__ uint32_t bf16_bits(float f) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, f);
+  return f != f ? 0x7fc0u : (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+__device__ __forceinline__ uint32_t fp16_bits(float f) {
+  return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
+}
+// Stores four results of one output row, channels n .. n+3 (those below N), as a.f_kind asks.
+// STREAM: past the caches.  The 16-bit kinds leave the kernel instead of an fp32 tensor that
+// a second launch reads and converts.
+template <bool STREAM = false>
+__device__ __forceinline__ void put_f32x4(const GemmArgs& a, int64_t m, int64_t n, v4f v) {
+  const int64_t at = m * a.ldy + a.n_off + n;
+  if (a.f_kind == TMQ_FLOAT_F32) {
+    float* dst = static_cast<float*>(a.y) + at;
+    if (n + 3 < a.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+      if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(dst));
+      else *reinterpret_cast<v4f*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < a.N) dst[j] = v[j];
+    }
+    return;
+  }
+  uint32_t h[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = a.f_kind == TMQ_FLOAT_BF16 ? bf16_bits(v[j]) : fp16_bits(v[j]);
+  uint16_t* dst = static_cast<uint16_t*>(a.y) + at;
+  if (n + 3 < a.N && (reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+    const v2u w = {h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    if constexpr (STREAM) __builtin_nontemporal_store(w, reinterpret_cast<v2u*>(dst));
+    else *reinterpret_cast<v2u*>(dst) = w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (n + j < a.N) dst[j] = static_cast<uint16_t>(h[j]);
+  }
+}
 __device__ __forceinline__ void store_f32x4(const GemmArgs& a, int64_t m, int64_t n, const int (&raw)[4],
                                             v4f mult, v4f bias) {
-  float* dst = static_cast<float*>(a.y) + m * a.ldy + a.n_off + n;
   v4f v;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     v[j] = __builtin_fmaxf(__builtin_fmaf(static_cast<float>(raw[j]), mult[j], bias[j]), a.lo_f);
-  if (n + 3 < a.N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-    *reinterpret_cast<v4f*>(dst) = v;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (n + j < a.N) dst[j] = v[j];
-  }
+  put_f32x4(a, m, n, v);
 }
 
 __device__ __forceinline__ v4i ld16(const void* p) { return *reinterpret_cast<const v4i*>(p); }
@@ -1086,8 +1121,6 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
     // write their rows into LDS, then all threads copy whole rows out, 16 B per
     // lane on consecutive addresses (a lane's own four floats of 32 different
     // rows would make 32 partial lines per store instruction).
-    float* const yf = static_cast<float*>(a.y) + a.n_off;
-    const bool vec_ok = ((a.ldy & 3) == 0) && ((reinterpret_cast<uintptr_t>(yf) & 15) == 0);
     constexpr int kRowChunks = BN / 4;
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
@@ -1117,15 +1150,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
         const int lr = id / kRowChunks, cc = id % kRowChunks;
         const int64_t m = m0 + (lr / 32) * WTM + tm * 32 + (lr % 32), n = n0 + cc * 4;
         if (m >= a.M || n >= a.N) continue;
-        const v4f v = *reinterpret_cast<const v4f*>(&smem[lr * kF32Pitch + cc * 16]);
-        float* dst = yf + m * a.ldy + n;
-        if (vec_ok && n + 4 <= a.N) {
-          *reinterpret_cast<v4f*>(dst) = v;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (n + j < a.N) dst[j] = v[j];
-        }
+        put_f32x4(a, m, n, *reinterpret_cast<const v4f*>(&smem[lr * kF32Pitch + cc * 16]));
       }
     }
   } else {

@@ -216,23 +216,13 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
       *reinterpret_cast<v4f*>(&sW[(wm0 + li) * kPitch + nl * 4]) = v;
     }
     __syncthreads();
-    float* const yf = static_cast<float*>(a.y) + a.n_off;
-    const bool vec_ok = ((a.ldy & 3) == 0) && ((reinterpret_cast<uintptr_t>(yf) & 15) == 0);
     constexpr int kRowChunks = BN / 4;
 #pragma unroll
     for (int id = t; id < BM * kRowChunks; id += 256) {
       const int row = id / kRowChunks, cc = id % kRowChunks;
       const int64_t m = m0 + row, n = n0 + cc * 4;
       if (m >= a.M || n >= a.N) continue;
-      const v4f v = *reinterpret_cast<const v4f*>(&sW[row * kPitch + cc * 16]);
-      float* dst = yf + m * a.ldy + n;
-      if (vec_ok && n + 4 <= a.N) {
-        *reinterpret_cast<v4f*>(dst) = v;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (n + j < a.N) dst[j] = v[j];
-      }
+      put_f32x4(a, m, n, *reinterpret_cast<const v4f*>(&sW[row * kPitch + cc * 16]));
     }
   } else {
     constexpr int kPitch = BN + 16;
@@ -305,19 +295,12 @@ __device__ __forceinline__ void ksplit_finish_four(const GemmArgs& a, const uint
     }
   }
   if constexpr (MODE == kOutF32 || MODE == kOutAcc32) {
-    float* const dst = static_cast<float*>(a.y) + a.n_off + m * a.ldy + n;
     v4f v;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       v[j] = MODE == kOutAcc32 ? __int_as_float(raw[j])
                                : __builtin_fmaxf(__builtin_fmaf(static_cast<float>(raw[j]), mult[j], bdiv[j]), a.lo_f);
-    if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0 && n + 4 <= a.N) {
-      *reinterpret_cast<v4f*>(dst) = v;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n + j < a.N) dst[j] = v[j];
-    }
+    put_f32x4(a, m, n, v);
   } else {
     const float bmul = bias_mul(a.w_scale_stride == 0, xq.scale * __int_as_float(s_raw[1][0]));
     const bool plain_u8 = MODE == kOutU8 && a.lo_f <= 0.f && a.hi_f >= 255.f;

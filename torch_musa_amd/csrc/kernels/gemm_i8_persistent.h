@@ -272,8 +272,6 @@ __global__ __launch_bounds__(kPersistThreads, 1) void gemm_i8_persistent_kernel(
   // (8 lanes per row, 8 rows per store instruction)
   auto epilogue_f32 = [&](int m0, int n0, int par) {
     uint8_t* const sF = smem + kStagingOff + wave * kFBytes;
-    float* const yf = static_cast<float*>(a.y);
-    const bool fvec_ok = ((a.ldy & 3) == 0) && ((reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
 #pragma unroll
@@ -297,18 +295,10 @@ __global__ __launch_bounds__(kPersistThreads, 1) void gemm_i8_persistent_kernel(
           const int p = pass * 8 + (lane >> 3), cq = lane & 7;
           const v4f v = *reinterpret_cast<const v4f*>(sF + p * kFPitch + cq * 16);
           const int64_t m = m0 + wm0 + tm * 32 + p, n = n0 + wn0 + tn * 32 + cq * 4;
-          if (m < a.M && n < a.N) {
-            float* dst = yf + m * a.ldy + n;
-            if (fvec_ok && n + 4 <= a.N) {
-              // (four times the bytes of the operands and read by nobody in this launch: past
-              // the caches, which hold the operands -- 210 -> 204 us for the dynamic linear at
-              // M = K = 4096, N = 11008; the byte outputs measure the same either way)
-              __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(dst));
-            } else {
-              for (int j = 0; j < 4; ++j)
-                if (n + j < a.N) dst[j] = v[j];
-            }
-          }
+          // (four times the bytes of the operands and read by nobody in this launch: past
+          // the caches, which hold the operands -- 210 -> 204 us for the dynamic linear at
+          // M = K = 4096, N = 11008; the byte outputs measure the same either way)
+          if (m < a.M && n < a.N) put_f32x4<true>(a, m, n, v);
         }
         wave_sync_lds();  // the staging rows are rewritten by the next tile
       }

@@ -1572,8 +1572,9 @@ TMQ_EXPORT int tmq_linear_acc32(const tmq_linear_desc* d, int32_t* acc, int64_t 
                                     d->workspace_bytes);
 }
 
-TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qparams_dev, float* y,
-                              int64_t ldy, tmq_stream_t stream) {
+TMQ_EXPORT int tmq_linear_float(const tmq_linear_desc* d, const tmq_qparams* x_qparams_dev, void* y, int64_t ldy,
+                                int kind, tmq_stream_t stream) {
+  if (kind != TMQ_FLOAT_F32 && kind != TMQ_FLOAT_BF16 && kind != TMQ_FLOAT_F16) return TMQ_ERR_INVALID_ARGUMENT;
   GemmArgs a{};
   XLinear xs{};
   bool vec_ok = false;
@@ -1581,7 +1582,8 @@ TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qpa
   if (rc != TMQ_OK || d->M == 0 || d->N == 0) return rc;
   if (y == nullptr || d->w_scales == nullptr || ldy < d->N) return TMQ_ERR_INVALID_ARGUMENT;
   if (x_qparams_dev == nullptr && !(d->x_scale > 0.f)) return TMQ_ERR_INVALID_ARGUMENT;
-  if (!aligned(y, 4)) return TMQ_ERR_ALIGNMENT;
+  if (!aligned(y, kind == TMQ_FLOAT_F32 ? 4 : 2)) return TMQ_ERR_ALIGNMENT;
+  a.f_kind = kind;
   a.w_scales = d->w_scales;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
   a.bias = d->bias;
@@ -1595,6 +1597,11 @@ TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qpa
   a.ldy = ldy;
   return dispatch_linear<kOutF32>(a, xs, d->x_signed, vec_ok, d->kernel - 1, as_stream(stream), d->workspace,
                                   d->workspace_bytes);
+}
+
+TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qparams_dev, float* y,
+                              int64_t ldy, tmq_stream_t stream) {
+  return tmq_linear_float(d, x_qparams_dev, y, ldy, TMQ_FLOAT_F32, stream);
 }
 
 // The float rows of the one-launch dynamic linear as the resident kernel holds them: 16 waves x 64

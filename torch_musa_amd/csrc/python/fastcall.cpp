@@ -14,6 +14,7 @@
 // tensor subclasses, a torch-function mode, tracing, stand-in objects of the export
 // machinery, numbers of other types -- goes to PyTorch's own callable, which is kept
 // as `self` of the function, and has its results and its errors.
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/api/object.h>
@@ -57,6 +58,44 @@ bool take(PyObject* o, bool* out) {
   *out = o == Py_True;
   return true;
 }
+bool take(PyObject* o, std::optional<at::Tensor>* out) {
+  if (o == Py_None) {
+    out->reset();
+    return true;
+  }
+  at::Tensor t;
+  if (!take(o, &t)) return false;
+  *out = std::move(t);
+  return true;
+}
+bool take(PyObject* o, std::optional<at::ScalarType>* out) {
+  if (o == Py_None) {
+    out->reset();
+    return true;
+  }
+  if (!THPDtype_Check(o)) return false;
+  *out = reinterpret_cast<THPDtype*>(o)->scalar_type;
+  return true;
+}
+bool take(PyObject* o, c10::string_view* out) {  // a view into the string object, which the caller holds
+  if (!PyUnicode_CheckExact(o)) return false;
+  Py_ssize_t n = 0;
+  const char* s = PyUnicode_AsUTF8AndSize(o, &n);
+  if (s == nullptr) {
+    PyErr_Clear();
+    return false;
+  }
+  *out = c10::string_view(s, static_cast<size_t>(n));
+  return true;
+}
+// The argument lists of post operations: only empty ones come this way.
+struct NoScalars {
+  torch::List<std::optional<at::Scalar>> list;
+};
+bool take(PyObject* o, NoScalars*) { return PyList_CheckExact(o) && PyList_GET_SIZE(o) == 0; }
+template <typename T>
+T& passed(T& v) { return v; }
+torch::List<std::optional<at::Scalar>>& passed(NoScalars& v) { return v.list; }
 template <typename Base>
 bool take(PyObject* o, c10::intrusive_ptr<Base>* out) {
   if (Py_TYPE(o) != g_script_object) return false;
@@ -91,7 +130,7 @@ struct Op {
         at::Tensor result;
         {
           py::gil_scoped_release no_gil;
-          result = std::apply([](auto&&... a) { return handle->call(a...); }, v);
+          result = std::apply([](auto&&... a) { return handle->call(passed(a)...); }, v);
         }
         return THPVariable_Wrap(std::move(result));
       }
@@ -124,6 +163,15 @@ using ConvAddOp = Op<ID, at::Tensor(at::Tensor, at::Tensor, const ConvPtr&, doub
 template <int ID>
 using AddOp = Op<ID, at::Tensor(at::Tensor, at::Tensor, double, int64_t), at::Tensor, at::Tensor, double, int64_t>;
 
+template <int ID>
+using PlainLinearOp =
+    Op<ID,
+       at::Tensor(at::Tensor, double, int64_t, at::Tensor, at::Tensor, at::Tensor, std::optional<at::Tensor>, double,
+                  int64_t, std::optional<at::ScalarType>, c10::string_view, torch::List<std::optional<at::Scalar>>,
+                  c10::string_view),
+       at::Tensor, double, int64_t, at::Tensor, at::Tensor, at::Tensor, std::optional<at::Tensor>, double, int64_t,
+       std::optional<at::ScalarType>, c10::string_view, NoScalars, c10::string_view>;
+
 struct Entry {
   PyMethodDef def;
   const char* qualified;
@@ -146,6 +194,7 @@ Entry g_entries[] = {
     {{"conv2d_add_silu"}, "quantized::conv2d_add_silu", "", 5, &ConvAddOp<11>::make},
     {{"add"}, "quantized::add", "", 4, &AddOp<12>::make},
     {{"add_relu"}, "quantized::add_relu", "", 4, &AddOp<13>::make},
+    {{"linear_per_tensor"}, "quantized::linear_per_tensor", "", 13, &PlainLinearOp<14>::make},
 };
 
 // make(name, fallback) -> the native callable of quantized::<name>; `fallback` takes the same arguments
