@@ -125,13 +125,17 @@ int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int64_t n, int 
 typedef struct tmq_host_report {
   uint64_t word[2];
 } tmq_host_report;
+#define TMQ_HOST_REPORTS 64
 /* The same, and the range goes to the host as soon as it is known, before the
- * codes are written: word[0] and word[1] carry the bits of the fp32 minimum and
+ * codes are written.  `slot` < TMQ_HOST_REPORTS numbers the reports of the calls
+ * that are in flight on a device at the same time (the library counts the blocks
+ * of the range pass by it).  word[0] and word[1] carry the bits of the fp32 minimum and
  * maximum (NaNs are passed over; +inf and -inf if there is nothing else).  n > 0. */
 int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, int q_signed,
                                            int reduce_range, int rounding, tmq_qparams* qparams,
                                            void* workspace, size_t workspace_bytes,
-                                           tmq_host_report* report, uint32_t ticket, tmq_stream_t stream);
+                                           tmq_host_report* report, uint32_t ticket, uint32_t slot,
+                                           tmq_stream_t stream);
 /* The same for M rows of K values -> rows of `pitch` codes, pitch a multiple of
  * 16 that is at least K: what tmq_linear wants of activations whose K is not.
  * The codes behind a row's end are undefined (the packed weights are zero there).

@@ -139,6 +139,9 @@ class HostReport {
   HostReport& operator=(const HostReport&) = delete;
 
   tmq_host_report* memory() { return slot_; }
+  uint32_t number() const {
+    return static_cast<uint32_t>((reinterpret_cast<char*>(slot_) - static_cast<char*>(pool().page)) / kStride);
+  }
   uint32_t ticket() const { return ticket_; }
   void queued() { pending_ = true; }  // a kernel that will write to the slot is on its stream
   // Payload of word `i`.
@@ -157,15 +160,15 @@ class HostReport {
   void done() { pending_ = false; }
 
  private:
-  static constexpr int kSlots = 64;     // calls that wait at the same time; more of them queue for a slot
+  static constexpr int kSlots = TMQ_HOST_REPORTS;  // calls that wait at the same time; more of them queue for a slot
   static constexpr int kSpins = 20000;  // about a millisecond
   struct Pool {
     std::mutex mu;
     std::condition_variable given_back;
     std::vector<tmq_host_report*> free;
     uint32_t ticket = 0;
+    void* page = nullptr;
     Pool() {
-      void* page = nullptr;
       TORCH_CHECK(hipHostMalloc(&page, kSlots * kStride, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess,
                   "hipHostMalloc failed");
       std::memset(page, 0, kSlots * kStride);
@@ -385,7 +388,7 @@ at::Tensor quantize_per_tensor_dynamic(const at::Tensor& self, at::ScalarType dt
   check_status(tmq_quantize_per_tensor_dynamic_report(
                    cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
                    reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes),
-                   report.memory(), report.ticket(), reinterpret_cast<tmq_stream_t>(stream.stream())),
+                   report.memory(), report.ticket(), report.number(), reinterpret_cast<tmq_stream_t>(stream.stream())),
                "tmq_quantize_per_tensor_dynamic_report");
   report.queued();
   const uint32_t lo = report.wait(0, stream, what), hi = report.wait(1, stream, what);
