@@ -583,10 +583,13 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
   };
   const auto launch_tiles = [&](auto nt_tag) {
     if constexpr (MODE != kOutAcc32) {
-      if (po.any()) return launch(std::true_type{}, nt_tag, std::false_type{});
-      if (plain_bytes<MODE>(zp_f, lo_f, hi_f)) return launch(std::false_type{}, nt_tag, std::true_type{});
+      const bool plain = plain_bytes<MODE>(zp_f, lo_f, hi_f);
+      if (po.silu) return launch(std::integral_constant<int, 2>{}, nt_tag, std::false_type{});
+      if (po.any() && plain) return launch(std::integral_constant<int, 1>{}, nt_tag, std::true_type{});
+      if (po.any()) return launch(std::integral_constant<int, 1>{}, nt_tag, std::false_type{});
+      if (plain) return launch(std::integral_constant<int, 0>{}, nt_tag, std::true_type{});
     }
-    launch(std::false_type{}, nt_tag, std::false_type{});
+    launch(std::integral_constant<int, 0>{}, nt_tag, std::false_type{});
   };
   if (nt == 2)
     launch_tiles(std::integral_constant<int, 2>{});
@@ -599,8 +602,17 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
 // (conv_runs_pointwise_kernel); false when the layer is not one of them.
 bool pointwise_rows_ok(const tmq_conv2d_geom& g, const ConvShape& s) {
   return g.groups == 1 && s.KH == 1 && s.KW == 1 && s.sh == 1 && s.sw == 1 && s.ph == 0 && s.pw == 0 && s.runs_KS > 0 &&
-         conv_runs_pointwise_lds(s.OC, s.runs_KS) <= kCrPointwiseLdsMax;
+         s.B * s.H * s.W <= 0x7fffff00 && s.OC <= 65536;
 }
+
+// Where it is ahead of everything else that runs the layer (us, it | the best other): always with a residual (batch
+// 32, 256 -> 512 on 28 x 28 15.1 | 18.6; 128 -> 768 on 53 x 109 at batch 6 17.7 | 28.8; one image, 96 -> 576 on
+// 14 x 14 4.4 | 5.3), up to 128 input channels (batch 32: 128 -> 512 on 28 x 28 10.6 | 10.8, 96 -> 576 on 14 x 14
+// 5.3 | 6.4; one image: 64 -> 256 on 56 x 56 4.2 | 4.5), and up to 160 output channels (256 -> 64 on 56 x 56 10.9 |
+// 11.0, 144 -> 24 on one image of 57 x 43 4.2 | 4.7).  More of both without a residual is the linear kernels'
+// (256 -> 512 on 28 x 28 14.4 | 12.7, 256 -> 1024 on 14 x 14 9.9 | 8.4): every wave would read the pixels again for
+// its 64 channels.
+bool pointwise_rows_first(const ConvShape& s, bool post) { return post || s.runs_KS <= 2 || s.OC <= 160; }
 
 template <int MODE>
 int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, const PostOps& po, float zp_f, float lo_f,
@@ -619,7 +631,6 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.sh = a.sw = 1;
   a.RL = static_cast<int>(s.runs_RL); a.RP = static_cast<int>(s.runs_RP); a.KS = static_cast<int>(s.runs_KS);
   const int64_t pieces = ceil_div(s.B * s.H * s.W, 16);
-  if (pieces > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   a.tiles = static_cast<int32_t>(pieces);
   a.vec = aligned(out, 16) && s.OC % (MODE == kOutAcc32 ? 4 : 16) == 0 ? 1 : 0;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
@@ -630,39 +641,37 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.zp_f = zp_f; a.lo_f = lo_f; a.hi_f = hi_f;
   a.post = po;
   const int nt = conv_runs_tiles(s.OC);
-  const int64_t lds = conv_runs_pointwise_lds(s.OC, s.runs_KS);
-  // as many blocks per CU as their registers and weights allow (three),
-  // each walking the pieces its waves are dealt
-  int64_t per_cu = (160 * 1024) / (lds + 512);
-  const int64_t by_registers = 3;
-  per_cu = per_cu < 1 ? 1 : per_cu > by_registers ? by_registers : per_cu;
-  const int64_t want = ceil_div(pieces, kCrWaves), cap = 256 * per_cu;
-  const dim3 grid(static_cast<unsigned>(want < cap ? want : cap)), block(kCrThreads);
+  // one wave per channel block and run of pieces, as many as the chip holds at once (their registers), but at least
+  // one per channel block
+  const int64_t nblk = ceil_div(s.OC, 16 * nt), cap = 256 * (s.runs_KS > 2 ? 2 : 3) * kCrWaves;
+  int64_t groups = cap / nblk < 1 ? 1 : cap / nblk;
+  if (groups > pieces) groups = pieces;
+  const dim3 grid(static_cast<unsigned>(ceil_div(groups * nblk, kCrWaves))), block(kCrThreads);
   const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
-    auto* const kernel = conv_runs_pointwise_kernel<MODE, decltype(post_tag)::value, decltype(nt_tag)::value,
-                                                    decltype(plain_tag)::value>;
-    // the kernel's LDS allowance is a per-device attribute: set once per device (and kernel)
-    static std::atomic<uint64_t> done{0};
-    const int dev = current_device();
-    if (dev < 0) return false;
-    if ((done.load(std::memory_order_acquire) >> dev & 1) == 0) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              kCrPointwiseLdsMax) != hipSuccess)
-        return false;
-      done.fetch_or(uint64_t{1} << dev, std::memory_order_release);
-    }
-    kernel<<<grid, block, static_cast<size_t>(lds), stream>>>(a);
-    return true;
+    constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;
+    constexpr bool kPlain = decltype(plain_tag)::value;
+    if (s.runs_KS == 1)
+      conv_runs_pointwise_kernel<MODE, kP, kNT, 1, kPlain><<<grid, block, 0, stream>>>(a);
+    else if (s.runs_KS == 2)
+      conv_runs_pointwise_kernel<MODE, kP, kNT, 2, kPlain><<<grid, block, 0, stream>>>(a);
+    else
+      conv_runs_pointwise_kernel<MODE, kP, kNT, 4, kPlain><<<grid, block, 0, stream>>>(a);
   };
   const auto launch_tiles = [&](auto nt_tag) {
     if constexpr (MODE != kOutAcc32) {
-      if (po.any()) return launch(std::true_type{}, nt_tag, std::false_type{});
-      if (plain_bytes<MODE>(zp_f, lo_f, hi_f)) return launch(std::false_type{}, nt_tag, std::true_type{});
+      const bool plain = plain_bytes<MODE>(zp_f, lo_f, hi_f);
+      if (po.silu) return launch(std::integral_constant<int, 2>{}, nt_tag, std::false_type{});
+      if (po.any() && plain) return launch(std::integral_constant<int, 1>{}, nt_tag, std::true_type{});
+      if (po.any()) return launch(std::integral_constant<int, 1>{}, nt_tag, std::false_type{});
+      if (plain) return launch(std::integral_constant<int, 0>{}, nt_tag, std::true_type{});
     }
-    return launch(std::false_type{}, nt_tag, std::false_type{});
+    launch(std::integral_constant<int, 0>{}, nt_tag, std::false_type{});
   };
-  const bool ok = nt == 2 ? launch_tiles(std::integral_constant<int, 2>{}) : launch_tiles(std::integral_constant<int, 4>{});
-  return ok ? launch_status() : TMQ_ERR_LAUNCH;
+  if (nt == 2)
+    launch_tiles(std::integral_constant<int, 2>{});
+  else
+    launch_tiles(std::integral_constant<int, 4>{});
+  return launch_status();
 }
 
 // Depthwise layers on the vector ALU (conv_depthwise.h).
@@ -814,7 +823,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     // 28 x 28 14.3 against 18.0 us)
     // (a detection head's 255 channels count as wide: 128 -> 255 on 80 x 80 at batch 8 18.0 -> 15.2 us)
     const bool wide = s.IC >= 128 && s.OC >= 224 && rows * s.IC * s.OC >= 1000000000;
-    if (forced == 5 || (forced < 0 && pointwise && (rows <= kPointwiseAsLinearRows || wide))) {
+    if (forced == 5 || (forced < 0 && pointwise && (rows <= kPointwiseAsLinearRows || wide) &&
+                        !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, false)))) {
       return run_as_linear(d, rows, s.OC, s.IC, d->x, relu, out, stream);
     }
   }
@@ -873,17 +883,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   {
     const bool rows_ok = pointwise_rows_ok(d->geom, s) && (MODE != kOutAcc32 || aligned(out, 4));
     if (forced == 9 && !rows_ok) return TMQ_ERR_UNSUPPORTED;
-    // Automatic where the image offers enough 16-pixel pieces for the chip's waves and few enough channel blocks
-    // for a wave to run them all (batch 32, against the halo tiles or the byte-run kernel: 32 -> 16 channels on
-    // 112 x 112 19.3 -> 10 us, 24 -> 144 on 56 x 56 21.5 -> 11.5 us, 16 -> 96 on 112 x 112 31 -> 25 us, 256 -> 128 on
-    // 56 x 56 18.6 -> 15.6 us, 192 -> 32 on 28 x 28 4.7 -> 4.0 us; 128 -> 512 on 28 x 28 10.5 against 12.5 us and
-    // 96 -> 576 on 14 x 14 5.8 against 11.4 us stay where they were).
-    const int64_t pieces = ceil_div(s.B * s.H * s.W, 16), blocks = ceil_div(s.OC, 16 * conv_runs_tiles(s.OC));
-    // (one channel block: from 128 pieces on -- one image, 32 -> 16 channels on 112 x 112 4.3 -> 3.7 us; and whenever the
-    // channel count leaves only the byte-run kernel: one image, 24 -> 144 on 56 x 56 6.6 -> 5.0 us)
-    const bool worth = (pieces >= 1024 && (blocks <= 3 || (pieces >= 4096 && blocks <= 4))) ||
-                       (pieces >= 128 && blocks == 1) || !mfma_ok;
-    if (forced == 9 || (forced < 0 && rows_ok && worth))
+    if (forced == 9 || (forced < 0 && rows_ok && (pointwise_rows_first(s, po.any()) || !mfma_ok)))
       return launch_conv_pointwise_rows<MODE>(d, s, po, zp_f, lo_f, hi_f, out, stream);
   }
   // depthwise layers: four channels per lane on the vector ALU

@@ -95,9 +95,43 @@ __device__ __forceinline__ v4i conv_runs_slot(const int8_t* __restrict__ w, int6
 // MFMAs of its NT channel tiles, and store them at element offset `off` of the output: one store of 4 NT
 // bytes where all the channels exist.  mult / bdiv: the constants of channel cb onwards.  PLAIN: the host found
 // requant_plain_u8 to hold (zero point 0 for unsigned bytes, -128 for signed ones, no bounds inside the range).
-template <int MODE, bool POST, int NT, bool PLAIN = false>
+// POST: 0 no post operations, 1 a residual and no SiLU, 2 SiLU (a residual if there is one); accw: the residual
+// bytes of the lane's channels (runs_residual).
+template <int NT>
+struct RunsResidual {
+  uint32_t w[NT];
+};
+template <int NT>
+__device__ __forceinline__ RunsResidual<NT> runs_residual(const ConvRunArgs& a, int64_t off, int cb) {
+  // one load of 4 NT bytes at any alignment where all the channels exist (a dword per four channels
+  // took four requests, each waited for by itself)
+  RunsResidual<NT> r;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) r.w[nt] = 0;
+  const uint8_t* const src = a.post.accum + off;
+  if (cb + 4 * NT <= a.OC) {
+    if constexpr (NT == 4) {
+      const v4i v = ld16_any(src);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) r.w[nt] = static_cast<uint32_t>(v[nt]);
+    } else {
+      const v2i v = reinterpret_cast<const V2iAnyAlignment*>(src)->v;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) r.w[nt] = static_cast<uint32_t>(v[nt]);
+    }
+  } else {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int left = a.OC - (cb + 4 * nt);
+      if (left > 0) r.w[nt] = load_accum4(a.post, off + 4 * nt, left < 4 ? left : 4);
+    }
+  }
+  return r;
+}
+template <int MODE, int POST, int NT, bool PLAIN = false>
 __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v4i (&acc)[NT], int64_t off, int cb,
-                                                   const float* mult_cb, const float* bdiv_cb, float bmul) {
+                                                   const float* mult_cb, const float* bdiv_cb, float bmul,
+                                                   const RunsResidual<NT>& accw) {
   constexpr int kLaneCh = 4 * NT;
   uint32_t packed[NT];
 #pragma unroll
@@ -113,14 +147,10 @@ __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v
           if (cb + 4 * nt + r < a.OC) dst[r] = raw[r];
       }
     } else {
-      const v4f mult = *reinterpret_cast<const v4f*>(mult_cb + 4 * nt);
-      const v4f bdiv = *reinterpret_cast<const v4f*>(bdiv_cb + 4 * nt);
-      if constexpr (POST) {
-        const int left = a.OC - (cb + 4 * nt);
-        const int nvalid = left < 0 ? 0 : (left < 4 ? left : 4);
-        const uint32_t accw =
-            a.post.accum != nullptr && nvalid > 0 ? load_accum4(a.post, off + 4 * nt, nvalid) : 0u;
-        packed[nt] = requant4_post<MODE>(raw, bdiv, bmul, mult, a.post, accw, a.zp_f, a.lo_f, a.hi_f);
+      const v4f mult = {mult_cb[4 * nt], mult_cb[4 * nt + 1], mult_cb[4 * nt + 2], mult_cb[4 * nt + 3]};
+      const v4f bdiv = {bdiv_cb[4 * nt], bdiv_cb[4 * nt + 1], bdiv_cb[4 * nt + 2], bdiv_cb[4 * nt + 3]};
+      if constexpr (POST != 0) {
+        packed[nt] = requant4_post<MODE, POST, PLAIN>(raw, bdiv, bmul, mult, a.post, accw.w[nt], a.zp_f, a.lo_f, a.hi_f);
       } else {
         packed[nt] = requant4<MODE, true, PLAIN ? 1 : 0>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
       }
@@ -152,7 +182,7 @@ __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v
   }
 }
 
-template <int MODE, bool POST, int NT, bool PLAIN = false>
+template <int MODE, int POST, int NT, bool PLAIN = false>
 __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a) {
   constexpr int kCrBN = 16 * NT;  // output channels per block (grid y)
   constexpr int kLaneCh = 4 * NT; // consecutive channels of one pixel in a lane
@@ -354,7 +384,9 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
       const int cb = n0 + kLaneCh * pq;
       if (cb >= a.OC) continue;
       const int64_t off = opix * a.OC + cb;
-      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, &s_mult[kLaneCh * pq], &s_bdiv[kLaneCh * pq], bmul);
+      RunsResidual<NT> accw{};
+      if (POST == 1 || (POST == 2 && a.post.accum != nullptr)) accw = runs_residual<NT>(a, off, cb);
+      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, &s_mult[kLaneCh * pq], &s_bdiv[kLaneCh * pq], bmul, accw);
     }
     __syncthreads();  // the staged rows are overwritten by the next tile
   }
@@ -364,72 +396,91 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
 // on the same per-lane weight layout: here a pixel's IC bytes *are* the run, a lane's MFMA
 // operand for pixel p and k-step ks is the 16 bytes at p * IC + 64 ks + 16 (lane / 16) of the
 // input -- straight from memory, any alignment, no staging -- and what it picks up past the
-// pixel's last channel (the next pixel's bytes) meets zero weights.  The weights of all output
-// channels sit in LDS as MFMA operands; a wave walks 16-pixel pieces of the image on its own
-// (no barrier after set-up), asks for the next piece's bytes before it works on the current
-// one's, and runs every 16 NT-channel block of the output over the piece in hand: the input is
-// read once whatever OC is.  a.tiles: the number of 16-pixel pieces.
-constexpr int kCrPointwiseLdsMax = 144 * 1024;
-__host__ __device__ inline int64_t conv_runs_pointwise_lds(int64_t OC, int64_t KS) {
-  const int64_t nt = conv_runs_tiles(OC), nblk = (OC + 16 * nt - 1) / (16 * nt);
-  return nblk * nt * KS * 1024 + nblk * 16 * nt * 12;
-}
+// pixel's last channel (the next pixel's bytes) meets zero weights.
+//
+// A wave owns one channel block for the whole launch, its weights (NT x KSN operands) and the
+// requantisation constants of the lane's 4 NT channels in registers, and walks every G-th 16-pixel
+// piece of the image, D pieces' bytes (input and residual) on their way: a load per k-step, the MFMAs,
+// eight vector instructions per value and one store, no LDS and no barrier behind the set-up.  The waves
+// of neighbouring channel blocks read the same pieces at the same time, from one L1.  What bounds it is the
+// requantisation, then memory: 64 -> 256 channels with a residual on 56 x 56 at batch 32 (58 MB) takes
+// 14.4 us; with the weights and constants in LDS and every channel block over a piece in turn, the LDS
+// reads were a third of its instructions and the residual a latency per block: 27.9 us.
+// a.tiles: the number of 16-pixel pieces.
+template <int KSN>
+constexpr int kCrPointwiseDepth = KSN == 1 ? 4 : 2;
 
-template <int MODE, bool POST, int NT, bool PLAIN = false>
-__global__ __launch_bounds__(kCrThreads, 3) void conv_runs_pointwise_kernel(ConvRunArgs a) {
+template <int MODE, int POST, int NT, int KSN, bool PLAIN = false>
+__global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointwise_kernel(ConvRunArgs a) {
   constexpr int kCrBN = 16 * NT;   // output channels per channel block
   constexpr int kLaneCh = 4 * NT;  // consecutive channels of one pixel in a lane
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int D = kCrPointwiseDepth<KSN>;
+  // constants of the channels of this block's waves: at most four channel blocks
+  __shared__ __attribute__((aligned(16))) int s_acc0[kCrWaves * kCrBN];
+  __shared__ __attribute__((aligned(16))) float s_mult[kCrWaves * kCrBN];
+  __shared__ __attribute__((aligned(16))) float s_bdiv[kCrWaves * kCrBN];
   const int t = threadIdx.x, lane = t % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int pj = lane & 15, pq = lane >> 4;
   const int KS = a.KS;
   const int nblk = (a.OC + kCrBN - 1) / kCrBN;
-  const int wslots = nblk * NT * KS * kWave;  // 16-byte operands
-  int* const s_acc0 = reinterpret_cast<int*>(lds + wslots * 16);
-  float* const s_mult = reinterpret_cast<float*>(s_acc0 + nblk * kCrBN);
-  float* const s_bdiv = s_mult + nblk * kCrBN;
-  const int64_t npix = static_cast<int64_t>(a.B) * a.H * a.W, x_bytes = npix * a.IC;
-  // this lane's 16 bytes of every k-step for the pixel pj of a piece (zeros where the piece has no such pixel or the
-  // k-step no such bytes; the tensor's last few bytes one by one)
-  const auto fetch = [&](int64_t piece, v4i (&xv)[kCrMaxKS]) {
-    const int64_t pix = piece * 16 + pj;
+  const int groups = static_cast<int>(gridDim.x) * kCrWaves / nblk;  // waves on one channel block
+  const int w = static_cast<int>(blockIdx.x) * kCrWaves + wave;
+  const int g = w / nblk, cb = w - g * nblk;
+  const int npix = a.B * a.H * a.W;
+  const int64_t x_bytes = static_cast<int64_t>(npix) * a.IC;
+  const bool works = g < groups && g < a.tiles;  // (the same for the whole wave)
+
+  // this lane's 16 bytes of every k-step for the pixel pj of a piece; a pixel or bytes that do not exist: any
+  // others (nothing of them is stored, or their weights are zero)
+  const auto fetch = [&](int piece, v4i (&xv)[KSN]) {
+    const int pix = piece * 16 + pj < npix ? piece * 16 + pj : npix - 1;
+    const int64_t row = static_cast<int64_t>(pix) * a.IC;
 #pragma unroll
-    for (int ks = 0; ks < kCrMaxKS; ++ks) {
-      xv[ks] = v4i{0, 0, 0, 0};
+    for (int ks = 0; ks < KSN; ++ks) {
       const int k0 = ks * 64 + pq * 16;
-      if (ks < KS && pix < npix && k0 < a.RP) {
-        const int64_t o = pix * a.IC + k0;
-        if (o + 16 <= x_bytes) {
-          xv[ks] = ld16_any(a.x + o);
-        } else {
-          uint32_t words[4] = {0, 0, 0, 0};
-          for (int b = 0; b < 16; ++b)
-            if (o + b < x_bytes) words[b >> 2] |= static_cast<uint32_t>(a.x[o + b]) << (8 * (b & 3));
-          xv[ks] = v4i{static_cast<int>(words[0]), static_cast<int>(words[1]), static_cast<int>(words[2]), static_cast<int>(words[3])};
-        }
+      const int64_t o = row + (k0 < a.RP ? k0 : 0);
+      if (o + 16 <= x_bytes) {
+        xv[ks] = ld16_any(a.x + o);
+      } else {  // the tensor's last few bytes, one by one
+        uint32_t words[4] = {0, 0, 0, 0};
+        for (int b = 0; b < 16; ++b)
+          if (o + b < x_bytes) words[b >> 2] |= static_cast<uint32_t>(a.x[o + b]) << (8 * (b & 3));
+        xv[ks] = v4i{static_cast<int>(words[0]), static_cast<int>(words[1]), static_cast<int>(words[2]), static_cast<int>(words[3])};
       }
     }
   };
-  // the first pieces' bytes are asked for before the weights and constants are set up: their latencies overlap
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kCrWaves;
-  int64_t piece = static_cast<int64_t>(blockIdx.x) * kCrWaves + wave;
-  // (KS == 1: pre[i] is the one k-step of the i-th piece ahead, four pieces in flight; otherwise the next piece's k-steps)
-  static_assert(kCrMaxKS == 4, "the ring of four pieces shares the registers of one piece's four k-steps");
-  v4i pre[kCrMaxKS] = {};
-  if (KS == 1) {
+  const bool residual = POST == 1 || (POST == 2 && a.post.accum != nullptr);
+  const int cl = cb * kCrBN + kLaneCh * pq;  // this lane's first channel
+  const auto fetch_residual = [&](int piece, RunsResidual<NT>& r) {
+    const int pix = piece * 16 + pj;
+    if (residual && pix < npix && cl < a.OC) r = runs_residual<NT>(a, static_cast<int64_t>(pix) * a.OC + cl, cl);
+  };
+  // the first pieces' bytes and the weights are asked for before the constants are set up
+  v4i xr[D][KSN];
+  RunsResidual<NT> rr[D];
+  v4i wreg[NT][KSN];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (piece + i * stride < a.tiles) {
-        v4i tmp[kCrMaxKS];
-        fetch(piece + i * stride, tmp);
-        pre[i] = tmp[0];
-      }
-  } else if (piece < a.tiles) {
-    fetch(piece, pre);
+  for (int i = 0; i < D; ++i) {
+#pragma unroll
+    for (int ks = 0; ks < KSN; ++ks) xr[i][ks] = v4i{0, 0, 0, 0};
+    rr[i] = RunsResidual<NT>{};
+    if (works && g + i * groups < a.tiles) {
+      fetch(g + i * groups, xr[i]);
+      fetch_residual(g + i * groups, rr[i]);
+    }
   }
-  for (int i = t; i < wslots; i += kCrThreads) *reinterpret_cast<v4i*>(lds + i * 16) = ld16(a.w_runs + static_cast<int64_t>(i) * 16);
-  for (int n = t; n < nblk * kCrBN; n += kCrThreads) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int ks = 0; ks < KSN; ++ks)
+      wreg[nt][ks] = works && ks < KS ? ld16(a.w_runs + ((static_cast<int64_t>(cb) * NT + nt) * KS + ks) * (kWave * 16) + lane * 16)
+                                      : v4i{0, 0, 0, 0};
+  // the constants of the block's four waves' channels, a channel per thread (two IEEE divisions each; in registers
+  // of every lane they would be 32 per lane)
+  for (int i = t; i < kCrWaves * kCrBN; i += kCrThreads) {
+    const int wv = static_cast<int>(blockIdx.x) * kCrWaves + i / kCrBN;
+    const int n = (wv % nblk) * kCrBN + i % kCrBN;
     int acc0 = 0;
     float mult = 0.f, bdiv = 0.f;
     if (n < a.OC) {
@@ -440,63 +491,54 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_pointwise_kernel(Conv
         bdiv = a.bias != nullptr ? bias_term(a.w_scale_stride == 0, a.bias[n], atw) : 0.f;
       }
     }
-    s_acc0[n] = acc0;
-    s_mult[n] = mult;
-    s_bdiv[n] = bdiv;
+    s_acc0[i] = acc0;
+    s_mult[i] = mult;
+    s_bdiv[i] = bdiv;
   }
   __syncthreads();
+  if (!works) return;
   float bmul = 1.0f;
   if constexpr (MODE != kOutAcc32) bmul = bias_mul(a.w_scale_stride == 0, a.x_scale * a.w_scales[0]);
-
-  // every channel block over the piece in hand (xv: its bytes, sign flip applied)
-  const auto multiply = [&](int64_t piece, const v4i (&xv)[kCrMaxKS]) {
-    const int64_t pix = piece * 16 + pj;
-    for (int cbi = 0; cbi < nblk; ++cbi) {
-      const int cl = cbi * kCrBN + kLaneCh * pq;  // this lane's first channel of the block
-      v4i acc[NT];
+  v4i acc0[NT];
+  float mult[kLaneCh], bdiv[kLaneCh];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[nt] = *reinterpret_cast<const v4i*>(&s_acc0[cl + 4 * nt]);
+  for (int nt = 0; nt < NT; ++nt) {
+    const int at = wave * kCrBN + kLaneCh * pq + 4 * nt;
+    acc0[nt] = *reinterpret_cast<const v4i*>(&s_acc0[at]);
+    const v4f m = *reinterpret_cast<const v4f*>(&s_mult[at]), b = *reinterpret_cast<const v4f*>(&s_bdiv[at]);
 #pragma unroll
-      for (int ks = 0; ks < kCrMaxKS; ++ks) {
-        if (ks < KS) {
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) {
-            const v4i w = *reinterpret_cast<const v4i*>(lds + ((((cbi * NT + nt) * KS + ks) * kWave + lane) << 4));
-            acc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, xv[ks], acc[nt], 0, 0, 0);
-          }
-        }
-      }
-      if (pix < npix && cl < a.OC)
-        runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, pix * a.OC + cl, cl, &s_mult[cl], &s_bdiv[cl], bmul);
+    for (int r = 0; r < 4; ++r) {
+      mult[4 * nt + r] = m[r];
+      bdiv[4 * nt + r] = b[r];
     }
-  };
+  }
   const int xo = static_cast<int>(a.x_xor);
   const v4i flip = {xo, xo, xo, xo};
-  if (KS == 1) {
-    // At most 64 input channels: one load per piece, four pieces' loads in flight per wave.
-    while (piece < a.tiles) {
+  for (int piece = g; piece < a.tiles;) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (piece < a.tiles) {
-          const v4i xv[kCrMaxKS] = {pre[i] ^ flip, v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
-          if (piece + 4 * stride < a.tiles) {
-            v4i tmp[kCrMaxKS];
-            fetch(piece + 4 * stride, tmp);
-            pre[i] = tmp[0];
-          }
-          multiply(piece, xv);
-          piece += stride;
+    for (int i = 0; i < D; ++i) {
+      if (piece < a.tiles) {
+        v4i acc[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[nt] = acc0[nt];
+#pragma unroll
+        for (int ks = 0; ks < KSN; ++ks) {
+          const v4i xv = xr[i][ks] ^ flip;
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt)
+            acc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[nt][ks], xv, acc[nt], 0, 0, 0);
         }
+        const RunsResidual<NT> accw = rr[i];
+        if (piece + D * groups < a.tiles) {
+          fetch(piece + D * groups, xr[i]);
+          fetch_residual(piece + D * groups, rr[i]);
+        }
+        const int pix = piece * 16 + pj;
+        if (pix < npix && cl < a.OC)
+          runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, static_cast<int64_t>(pix) * a.OC + cl, cl, mult, bdiv, bmul, accw);
+        piece += groups;
       }
     }
-    return;
-  }
-  for (; piece < a.tiles; piece += stride) {
-    v4i xv[kCrMaxKS];
-#pragma unroll
-    for (int ks = 0; ks < kCrMaxKS; ++ks) xv[ks] = pre[ks] ^ flip;
-    if (piece + stride < a.tiles) fetch(piece + stride, pre);
-    multiply(piece, xv);
   }
 }
 
