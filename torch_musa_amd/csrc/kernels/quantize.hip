@@ -540,46 +540,57 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_after_minmax_kernel(
   }
 }
 
-// Dynamic quantization of a small tensor in one launch: one block finds the
-// range, chooses the parameters and converts.  A decode-sized activation
-// ([1..16, 4096] floats) is a few tens of KB: three dependent launches would
-// cost several times what the work does.
-constexpr int kDynSmallThreads = 1024;
-// (elements.  From 32 Ki on the two-launch chain below is faster than one block pulling the
-// whole input: a dynamically quantized linear of 16 x 4096 values takes 11.1 instead of 12.6 us.)
-constexpr int64_t kDynSmallMax = 32768;
+// Dynamic quantization of a small tensor in one launch.  Every block reads the whole input and
+// finds the range for itself -- the same lines for all of them, from the L2s -- and converts its
+// own 1024 words of four codes; a block converts what it reads at its own position, so nothing is
+// read twice by a block.  No block waits for another.  The read bounds it: 96 Ki values are 384 KB
+// into every CU, 2.7 us at 64 bytes a clock, about what the launch and the gap between two launches
+// cost (a dynamically quantized linear of 55 rows, 704 -> 480: 12.2 -> 8.6 us; of 283 rows, 392 -> 192,
+// 111 Ki values: level; quantize and dequantize of 130 x 384 values 16.7 -> 15.6 us, of 581 x 221
+// 16.3 -> 17.4 us, hence the limit).
+// Rows: `K` values each, written at a pitch of 4 pitch4 codes (pitch4 = 0: one row, no pitch).  x is read as
+// 16 bytes at any 4-byte alignment.
+constexpr int kDynRepeatThreads = 1024;
+constexpr int64_t kDynRepeatMax = 98304;
 template <bool SIGNED, bool FUSED>
-__global__ __launch_bounds__(kDynSmallThreads) void dynamic_quantize_small_kernel(
-    const float* __restrict__ x, uint8_t* __restrict__ q, int64_t n, int qmin, int qmax,
-    int reduce_range, bool vec, tmq_qparams* __restrict__ out, RangeReport report) {
-  __shared__ float s_mn[kDynSmallThreads / kWave], s_mx[kDynSmallThreads / kWave];
+__global__ __launch_bounds__(kDynRepeatThreads) void dynamic_quantize_repeat_kernel(
+    const float* __restrict__ x, uint8_t* __restrict__ q, int32_t n, int32_t K, int32_t pitch4, int qmin, int qmax,
+    int reduce_range, bool words, tmq_qparams* __restrict__ out, RangeReport report) {
+  constexpr int kWaves = kDynRepeatThreads / kWave, kAhead = 8;
+  __shared__ float s_mn[kWaves], s_mx[kWaves];
   __shared__ float s_inv, s_zp;
-  const int t = threadIdx.x;
-  const int64_t n4 = vec ? n / 4 : 0;
-  const v4f* x4 = reinterpret_cast<const v4f*>(x);
-  // the whole input fits the block's registers (kDynSmallMax / 4 / threads = 8
-  // groups of four per thread): memory is read once, all loads in flight together
-  constexpr int kHeld = static_cast<int>(kDynSmallMax / 4 / kDynSmallThreads);
-  v4f held[kHeld];
-#pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int64_t i = t + static_cast<int64_t>(u) * kDynSmallThreads;
-    if (i < n4) held[u] = x4[i];
-  }
+  const int t = threadIdx.x, own = static_cast<int>(blockIdx.x);
+  struct __attribute__((packed, aligned(4))) Four {
+    v4f v;
+  };
+  // group i of the input: values 4 i ... 4 i + 3; the last one begins where four values are left (some are then
+  // seen twice, which no minimum or maximum minds)
+  const auto group = [&](int i) { return reinterpret_cast<const Four*>(x + (4 * i + 4 <= n ? 4 * i : n - 4))->v; };
   float mn = std::numeric_limits<float>::infinity();
   float mx = -std::numeric_limits<float>::infinity();
+  v4f mine = {0.f, 0.f, 0.f, 0.f};
+  const int groups = (n + 3) / 4;
+  if (n >= 4 && groups <= kDynRepeatThreads) {
+    mine = group(t < groups ? t : groups - 1);
+    mn = fminf(fminf(mine.x, mine.y), fminf(mine.z, mine.w));
+    mx = fmaxf(fmaxf(mine.x, mine.y), fmaxf(mine.z, mine.w));
+  } else if (n >= 4) {
+    for (int u0 = 0; u0 * kDynRepeatThreads < groups; u0 += kAhead) {
+      v4f v[kAhead];
 #pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int64_t i = t + static_cast<int64_t>(u) * kDynSmallThreads;
-    if (i < n4) {
-      const v4f v = held[u];
-      mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
-      mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
+      for (int u = 0; u < kAhead; ++u) {
+        const int i = (u0 + u) * kDynRepeatThreads + t;
+        v[u] = group(i < groups ? i : groups - 1);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        mn = fminf(fminf(mn, v[u].x), fminf(v[u].y, fminf(v[u].z, v[u].w)));
+        mx = fmaxf(fmaxf(mx, v[u].x), fmaxf(v[u].y, fmaxf(v[u].z, v[u].w)));
+        if (u0 + u == own) mine = v[u];
+      }
     }
-  }
-  for (int64_t i = 4 * n4 + t; i < n; i += kDynSmallThreads) {
-    mn = fminf(mn, x[i]);
-    mx = fmaxf(mx, x[i]);
+  } else if (t < n) {
+    mn = mx = x[t];
   }
   wave_minmax(mn, mx);
   if (t % kWave == 0) {
@@ -587,32 +598,53 @@ __global__ __launch_bounds__(kDynSmallThreads) void dynamic_quantize_small_kerne
     s_mx[t / kWave] = mx;
   }
   __syncthreads();
-  if (t == 0) {
-#pragma unroll
-    for (int w = 1; w < kDynSmallThreads / kWave; ++w) {
-      mn = fminf(mn, s_mn[w]);
-      mx = fmaxf(mx, s_mx[w]);
+  if (t < kWave) {
+    mn = t < kWaves ? s_mn[t] : std::numeric_limits<float>::infinity();
+    mx = t < kWaves ? s_mx[t] : -std::numeric_limits<float>::infinity();
+    wave_minmax(mn, mx);
+    if (t == 0) {
+      double s;
+      int32_t z;
+      if (own == 0) report_range(report, mn, mx);
+      choose_qparams(mn, mx, qmin, qmax, reduce_range != 0, &s, &z);
+      if (own == 0) {
+        out->scale = s;
+        out->zero_point = z;
+        out->reserved = 0;
+      }
+      s_inv = 1.0f / static_cast<float>(s);  // IEEE division, as in resolve()
+      s_zp = static_cast<float>(z);
     }
-    report_range(report, mn, mx);
-    double s;
-    int32_t z;
-    choose_qparams(mn, mx, qmin, qmax, reduce_range != 0, &s, &z);
-    out->scale = s;
-    out->zero_point = z;
-    out->reserved = 0;
-    s_inv = 1.0f / static_cast<float>(s);  // IEEE division, as in resolve()
-    s_zp = static_cast<float>(z);
   }
   __syncthreads();
   const float inv = s_inv, zp_f = s_zp;
-  uint32_t* q4 = reinterpret_cast<uint32_t*>(q);
-#pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int64_t i = t + static_cast<int64_t>(u) * kDynSmallThreads;
-    if (i < n4) q4[i] = quantize_four<SIGNED, FUSED>(held[u], inv, zp_f);
+  const int g = own * kDynRepeatThreads + t;  // this thread's word
+  if (pitch4 == 0) {
+    if (4 * g + 4 <= n && words) {
+      reinterpret_cast<uint32_t*>(q)[g] = quantize_four<SIGNED, FUSED>(mine, inv, zp_f);
+    } else {
+      for (int j = 4 * g; j < 4 * g + 4 && j < n; ++j) q[j] = static_cast<uint8_t>(quantize_one<SIGNED, FUSED>(x[j], inv, zp_f));
+    }
+    return;
   }
-  for (int64_t i = 4 * n4 + t; i < n; i += kDynSmallThreads)
-    q[i] = static_cast<uint8_t>(quantize_one<SIGNED, FUSED>(x[i], inv, zp_f));
+  const int row = g / pitch4, c = 4 * (g - row * pitch4);
+  if (row * K >= n) return;
+  v4f v = {0.f, 0.f, 0.f, 0.f};
+  if (c + 4 <= K) {
+    v = reinterpret_cast<const Four*>(x + row * K + c)->v;
+  } else {
+    for (int j = 0; c + j < K; ++j) v[j] = x[row * K + c + j];
+  }
+  reinterpret_cast<uint32_t*>(q)[g] = quantize_four<SIGNED, FUSED>(v, inv, zp_f);
+}
+template <class... Args>
+int launch_dynamic_repeat(bool q_signed, bool fused, int64_t words, hipStream_t s, Args... args) {
+  const dim3 grid(static_cast<unsigned>((words + kDynRepeatThreads - 1) / kDynRepeatThreads)), block(kDynRepeatThreads);
+  if (q_signed && fused) dynamic_quantize_repeat_kernel<true, true><<<grid, block, 0, s>>>(args...);
+  else if (q_signed) dynamic_quantize_repeat_kernel<true, false><<<grid, block, 0, s>>>(args...);
+  else if (fused) dynamic_quantize_repeat_kernel<false, true><<<grid, block, 0, s>>>(args...);
+  else dynamic_quantize_repeat_kernel<false, false><<<grid, block, 0, s>>>(args...);
+  return launch_status();
 }
 
 // ---------------------------------------------------------------------------
@@ -1217,19 +1249,11 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   if (!aligned(x, 4)) return TMQ_ERR_ALIGNMENT;
   hipStream_t s = as_stream(stream);
   const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
-  if (n <= kDynSmallMax) {
-    const bool vec = aligned(x, 16) && aligned(q, 4);
-    uint8_t* qb = static_cast<uint8_t*>(q);
-    const dim3 one(1), block(kDynSmallThreads);
-    if (q_signed && fused)
-      dynamic_quantize_small_kernel<true, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
-    else if (q_signed)
-      dynamic_quantize_small_kernel<true, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
-    else if (fused)
-      dynamic_quantize_small_kernel<false, true><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
-    else
-      dynamic_quantize_small_kernel<false, false><<<one, block, 0, s>>>(x, qb, n, qmin, qmax, reduce_range, vec, qparams, report);
-    return launch_status();
+  if (n <= kDynRepeatMax) {
+    const int32_t n32 = static_cast<int32_t>(n);
+    // (nothing to quantize: one block still publishes the parameters)
+    return launch_dynamic_repeat(q_signed != 0, fused, n > 0 ? ceil_div(n, 4) : 1, s, x, static_cast<uint8_t*>(q), n32, n32, 0,
+                                 qmin, qmax, reduce_range, aligned(q, 4), qparams, report);
   }
   if (workspace == nullptr || workspace_bytes < tmq_minmax_workspace_bytes(n) ||
       !aligned(workspace, report.to != nullptr ? 8 : 4))
@@ -1311,8 +1335,13 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
     return TMQ_ERR_WORKSPACE;
   hipStream_t s = as_stream(stream);
   const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
-  float* partials = static_cast<float*>(workspace);
+  const bool fused = rounding == TMQ_ROUND_FUSED;
   const int64_t n = M * K;
+  if (n <= kDynRepeatMax)
+    return launch_dynamic_repeat(q_signed != 0, fused, M * (pitch / 4), s, x, static_cast<uint8_t*>(q), static_cast<int32_t>(n),
+                                 static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4), qmin, qmax, reduce_range, true,
+                                 qparams, RangeReport{nullptr, 0, 0});
+  float* partials = static_cast<float*>(workspace);
   const uintptr_t mis = reinterpret_cast<uintptr_t>(x) & 15u;
   int64_t head = mis == 0 ? 0 : static_cast<int64_t>((16 - mis) / 4);
   if (head > n) head = n;
@@ -1327,7 +1356,6 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
                                   partials, count, qmin, qmax, reduce_range, qparams);
     return launch_status();
   };
-  const bool fused = rounding == TMQ_ROUND_FUSED;
   if (q_signed) return fused ? go(quantize_rows_after_minmax_kernel<true, true>) : go(quantize_rows_after_minmax_kernel<true, false>);
   return fused ? go(quantize_rows_after_minmax_kernel<false, true>) : go(quantize_rows_after_minmax_kernel<false, false>);
 }
