@@ -9,6 +9,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "conv_image.h"
 #include "conv_runs.h"
 #include "conv_depthwise.h"
 #include "conv_tile.h"
@@ -37,6 +38,7 @@ struct ConvShape {
   // the second weight layout, behind the first, for the kernel of conv_runs.h: k-steps
   // (0: the shape is not that kernel's), run bytes, padded run bytes, offset and size in bytes
   int64_t runs_KS, runs_RL, runs_RP, runs_off, runs_bytes;
+  bool pixels4;  // ... laid out for the kernel of conv_image.h, three channels as four-byte pixels
   // depthwise layers over a multiple of 4 channels: a [channel][kernel row][taps padded to a multiple
   // of 4] copy of the weight for the kernel of conv_depthwise.h in the same place (0: not such a layer)
   int64_t taps_bytes;
@@ -83,9 +85,11 @@ int make_shape(const tmq_conv2d_geom* g, ConvShape* s) {
   s->KC = packed_kchunks(s->Kp);
   s->group_bytes = ceil_div(s->OCg, 16) * s->KC * 256;
   s->runs_KS = s->runs_RL = s->runs_RP = s->runs_bytes = 0;
+  s->pixels4 = false;
   s->runs_off = s->groups * s->group_bytes;
   if (g->groups == 1 && g->dil_h == 1 && g->dil_w == 1) {
-    const int64_t RL = g->KW * g->IC, RP = round_up(RL, 16);
+    s->pixels4 = g->IC == 3 && g->KH * round_up(g->KW * 4, 16) <= 64 * kCrMaxKS && !(g->KH == 1 && g->KW == 1);
+    const int64_t RL = g->KW * (s->pixels4 ? 4 : g->IC), RP = round_up(RL, 16);
     if (g->KH * RP <= 64 * kCrMaxKS) {
       s->runs_RL = RL;
       s->runs_RP = RP;
@@ -137,7 +141,9 @@ __global__ __launch_bounds__(256) void conv_prepack_runs_kernel(const int8_t* __
   const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (id >= total) return;
   *reinterpret_cast<v4i*>(dst + id * 16) =
-      conv_runs_slot(w, id, static_cast<int>(s.OC), static_cast<int>(s.KH), static_cast<int>(s.runs_RL),
+      s.pixels4 ? conv_image_slot(w, id, static_cast<int>(s.OC), static_cast<int>(s.KH), static_cast<int>(s.KW),
+                                  static_cast<int>(s.runs_RP), static_cast<int>(s.runs_KS))
+                : conv_runs_slot(w, id, static_cast<int>(s.OC), static_cast<int>(s.KH), static_cast<int>(s.runs_RL),
                      static_cast<int>(s.runs_RP), static_cast<int>(s.runs_KS));
 }
 
@@ -508,8 +514,39 @@ int launch_conv_tiles(const ConvShape& s, const TilePlan& p, const ConvTileArgs&
 struct RunPlan {
   int RL, RP, KS, TR, TW, mtw, rows_in, pitch, lds;
 };
+// The same for three channels as four-byte pixels (conv_image.h).  The cost of a schedule: rounds of tiles
+// over the blocks the chip holds (three per CU) times a block's turns -- ten for each 16-pixel piece of its
+// waves, two for each group of its threads, fifteen for the set-up of a round.
+bool plan_image(const ConvShape& s, int forced_rows, RunPlan* p) {
+  if (!s.pixels4 || s.B * s.H * s.W * 3 < 12) return false;
+  constexpr int64_t kSlots = 3 * 256, kMaxGroups = int64_t{kCiUnits} * kCrThreads, kMaxLds = 48 * 1024;
+  const int64_t by = ceil_div(s.OC, 16 * conv_runs_tiles(s.OC));
+  int64_t best = -1;
+  for (int64_t TW = s.OW < 256 ? s.OW : 256;; TW = round_up(TW / 2, 16)) {
+    const int64_t mtw = ceil_div(TW, 16), G = ceil_div((TW - 1) * s.sw + s.runs_RP / 4, 4);
+    for (int64_t TR = 1; TR <= s.OH && TR <= 16; ++TR) {
+      const int64_t rows_in = (TR - 1) * s.sh + s.KH;
+      if (rows_in * G > kMaxGroups || rows_in * G * 16 > kMaxLds) break;
+      if (forced_rows > 0 && TR != forced_rows) continue;
+      const int64_t tiles = s.B * ceil_div(s.OH, TR) * ceil_div(s.OW, TW);
+      if (tiles > 0x7fffffff) continue;
+      const int64_t cost = ceil_div(tiles * by, kSlots) *
+                           (ceil_div(TR * mtw, kCrWaves) * 10 + ceil_div(rows_in * G, kCrThreads) * 2 + 15);
+      if (best < 0 || cost < best) {
+        best = cost;
+        p->RL = static_cast<int>(s.runs_RL); p->RP = static_cast<int>(s.runs_RP); p->KS = static_cast<int>(s.runs_KS);
+        p->TR = static_cast<int>(TR); p->TW = static_cast<int>(TW); p->mtw = static_cast<int>(mtw);
+        p->rows_in = static_cast<int>(rows_in); p->pitch = static_cast<int>(G * 16);
+        p->lds = static_cast<int>(rows_in * G * 16);
+      }
+    }
+    if (TW <= 16) break;
+  }
+  return best >= 0;
+}
 bool plan_runs(const ConvShape& s, int forced_rows, RunPlan* p) {
   if (s.runs_KS == 0) return false;
+  if (s.pixels4) return plan_image(s, forced_rows, p);
   const int64_t RL = s.runs_RL, RP = s.runs_RP, KS = s.runs_KS;
   // Tile = TR output rows x TW columns.  The staged image rows of a tile pass through
   // registers in units of 1 KB of a row, at most kCrUnits per wave; among the shapes that
@@ -575,10 +612,25 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
   const int64_t by = ceil_div(s.OC, 16 * nt);
   if (by > 65535) return TMQ_ERR_UNSUPPORTED;
   // three blocks per CU (their registers), each with its weights in registers for every tile it walks
-  const int64_t bx = a.tiles < 768 ? a.tiles : 768;  // (plan_runs: kSlots)
+  const int64_t slots = s.pixels4 ? std::max<int64_t>(768 / by, 1) : 768;  // (plan_runs, plan_image: kSlots)
+  const int64_t bx = a.tiles < slots ? a.tiles : slots;
   const dim3 grid(static_cast<unsigned>(bx), static_cast<unsigned>(by)), block(kCrThreads);
   const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
-    conv_runs_kernel<MODE, decltype(post_tag)::value, decltype(nt_tag)::value, decltype(plain_tag)::value>
+    constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;
+    constexpr bool kPlain = decltype(plain_tag)::value;
+    const auto image = [&](auto ks_tag) {
+      constexpr int kKS = decltype(ks_tag)::value;
+      if (s.sw % 2 == 0)
+        conv_image_kernel<MODE, kP, kNT, kKS, true, kPlain><<<grid, block, p.lds, stream>>>(a);
+      else
+        conv_image_kernel<MODE, kP, kNT, kKS, false, kPlain><<<grid, block, p.lds, stream>>>(a);
+    };
+    if (s.pixels4 && s.runs_KS == 1)
+      image(std::integral_constant<int, 1>{});
+    else if (s.pixels4)
+      image(std::integral_constant<int, kCrMaxKS>{});
+    else
+      conv_runs_kernel<MODE, decltype(post_tag)::value, decltype(nt_tag)::value, decltype(plain_tag)::value>
         <<<grid, block, p.lds, stream>>>(a);
   };
   const auto launch_tiles = [&](auto nt_tag) {
@@ -602,7 +654,7 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
 // (conv_runs_pointwise_kernel); false when the layer is not one of them.
 bool pointwise_rows_ok(const tmq_conv2d_geom& g, const ConvShape& s) {
   return g.groups == 1 && s.KH == 1 && s.KW == 1 && s.sh == 1 && s.sw == 1 && s.ph == 0 && s.pw == 0 && s.runs_KS > 0 &&
-         s.B * s.H * s.W <= 0x7fffff00 && s.OC <= 65536;
+         s.B * s.H * s.W <= 0x7fffff00 && s.B * s.H * s.W * s.IC >= 16 && s.OC <= 65536;
 }
 
 // Where it is ahead of everything else that runs the layer (us, it | the best other): always with a residual (batch

@@ -91,6 +91,9 @@ __device__ __forceinline__ v4i conv_runs_slot(const int8_t* __restrict__ w, int6
              static_cast<int>(words[3])};
 }
 
+struct __attribute__((packed, aligned(1))) U32AnyAlignment {
+  uint32_t v;
+};
 // Requantise (or pass on) the 4 NT consecutive channels cb ... of one pixel that a lane holds after the
 // MFMAs of its NT channel tiles, and store them at element offset `off` of the output: one store of 4 NT
 // bytes where all the channels exist.  mult / bdiv: the constants of channel cb onwards.  PLAIN: the host found
@@ -175,9 +178,18 @@ __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v
           st8_any(dst, all);
       }
     } else {
+      // a lane at the end of the channels: a word where four exist, else bytes
 #pragma unroll
-      for (int c = 0; c < kLaneCh; ++c)
-        if (cb + c < a.OC) dst[c] = static_cast<uint8_t>(packed[c >> 2] >> (8 * (c & 3)));
+      for (int nt = 0; nt < NT; ++nt) {
+        const int left = a.OC - (cb + 4 * nt);
+        if (left >= 4) {
+          reinterpret_cast<U32AnyAlignment*>(dst + 4 * nt)->v = packed[nt];
+        } else if (left > 0) {
+          dst[4 * nt] = static_cast<uint8_t>(packed[nt]);
+          if (left > 1) dst[4 * nt + 1] = static_cast<uint8_t>(packed[nt] >> 8);
+          if (left > 2) dst[4 * nt + 2] = static_cast<uint8_t>(packed[nt] >> 16);
+        }
+      }
     }
   }
 }
@@ -440,14 +452,9 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
     for (int ks = 0; ks < KSN; ++ks) {
       const int k0 = ks * 64 + pq * 16;
       const int64_t o = row + (k0 < a.RP ? k0 : 0);
-      if (o + 16 <= x_bytes) {
-        xv[ks] = ld16_any(a.x + o);
-      } else {  // the tensor's last few bytes, one by one
-        uint32_t words[4] = {0, 0, 0, 0};
-        for (int b = 0; b < 16; ++b)
-          if (o + b < x_bytes) words[b >> 2] |= static_cast<uint32_t>(a.x[o + b]) << (8 * (b & 3));
-        xv[ks] = v4i{static_cast<int>(words[0]), static_cast<int>(words[1]), static_cast<int>(words[2]), static_cast<int>(words[3])};
-      }
+      const int over = static_cast<int>(o + 16 - x_bytes);  // (the host: a tensor of at least 16 bytes)
+      xv[ks] = ld16_any(a.x + (over > 0 ? o - over : o));
+      if (over > 0) xv[ks] = shift_down_bytes(xv[ks], over);  // the tensor's last few bytes
     }
   };
   const bool residual = POST == 1 || (POST == 2 && a.post.accum != nullptr);

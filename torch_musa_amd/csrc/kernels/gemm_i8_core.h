@@ -211,6 +211,15 @@ __device__ __forceinline__ v4i shift_down_bytes(v4i v, int s) {
   const uint64_t nhi = b < 64 ? hi >> b : 0;
   return v4i{static_cast<int>(nlo), static_cast<int>(nlo >> 32), static_cast<int>(nhi), static_cast<int>(nhi >> 32)};
 }
+// The other way: bytes 0 ... 15 - s moved up by s, zeros in front of them.
+__device__ __forceinline__ v4i shift_up_bytes(v4i v, int s) {
+  const uint64_t lo = (static_cast<uint64_t>(static_cast<uint32_t>(v.y)) << 32) | static_cast<uint32_t>(v.x);
+  const uint64_t hi = (static_cast<uint64_t>(static_cast<uint32_t>(v.w)) << 32) | static_cast<uint32_t>(v.z);
+  const int b = 8 * s;  // 0 ... 120
+  const uint64_t nhi = b == 0 ? hi : b < 64 ? (hi << b) | (lo >> (64 - b)) : lo << (b - 64);
+  const uint64_t nlo = b < 64 ? lo << b : 0;
+  return v4i{static_cast<int>(nlo), static_cast<int>(nlo >> 32), static_cast<int>(nhi), static_cast<int>(nhi >> 32)};
+}
 // Four fp32 values 4 c4 ... 4 c4 + 3 of a row of K >= 4 values (4-byte aligned), zeros behind its
 // end, by the same clamped load.  (A zero does not change the range of a dynamic quantization:
 // ChooseQuantizationParams extends every range to hold 0.)
