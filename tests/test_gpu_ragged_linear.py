@@ -64,3 +64,25 @@ def test_plain_tensor_linear_in_16_bits(m, k, n, dtype):
     ws, wz = (torch.rand(n, generator=gen) * 1e-3).cuda(), torch.zeros(n, dtype=torch.long).cuda()
     call = lambda out: OPS.linear_per_tensor(x, 0.02, 120, w, ws, wz, None, 1.0, 0, out, "relu", [], "")  # noqa: E731
     assert torch.equal(call(dtype), call(torch.float32).to(dtype))
+
+
+@pytest.mark.parametrize("m,k,n", [
+    # an odd or short run of stages shared by two wave groups: 20, 21 (the last one 16 bytes), 33, 103 stages
+    (64, 1280, 64), (130, 1296, 100), (517, 2064, 70), (266, 6592, 130),
+    # rows read where they lie: the last chunk 1 ... 15 bytes, one stage, one and two wave groups, edges of tiles
+    (17, 17, 65), (129, 65, 1), (65, 127, 64), (400, 1279, 66), (64, 1281, 65), (70, 2049, 129), (300, 8191, 67)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_tiles_of_64_in_wave_groups_and_on_rows_off_the_grid(m, k, n, relu):
+    """Exact integer sums and the requantisation of the CPU operator: the same bytes."""
+    gen = torch.Generator().manual_seed(m * 7919 + k * 31 + n)
+    w, b = _weight(n, k, n % 2 == 0, gen), torch.randn(n, generator=gen)
+    x = torch.quantize_per_tensor(torch.randn(m, k, generator=gen), 0.03, 121, torch.quint8)
+    scale = 0.03 * max(k, 4) ** 0.5
+    op = OPS.linear_relu if relu else OPS.linear
+    want = op(x, OPS.linear_prepack(w, b), scale, 99).int_repr()
+    packed = OPS.linear_prepack(w.cuda(), b.cuda())
+    print("[case]", m, k, n, relu, flush=True)
+    for at in (0, 1, 8):  # the rows at this byte of their storage
+        codes = torch.empty(m * k + at, dtype=torch.uint8, device="cuda")[at:].view(m, k).copy_(x.int_repr().cuda())
+        view = torch._make_per_tensor_quantized_tensor(codes, 0.03, 121)
+        assert torch.equal(op(view, packed, scale, 99).int_repr().cpu(), want)

@@ -50,6 +50,13 @@ struct XLinear {
   int64_t ldx;
 };
 
+// The same rows at any address and pitch, of any K >= 16 (register staging only).
+struct XLinearRagged {
+  static constexpr bool kPostOps = false;
+  const uint8_t* x;
+  int64_t ldx;
+};
+
 struct XConv {
   static constexpr bool kPostOps = true;
   const uint8_t* x;  // NHWC
@@ -287,6 +294,14 @@ struct XLoader<XLinear> {
 };
 
 template <>
+struct XLoader<XLinearRagged> {
+  const uint8_t* p;
+  __device__ __forceinline__ void init(const XLinearRagged& s, int64_t m, int64_t M) {
+    p = s.x + (m < M ? m : M - 1) * s.ldx;
+  }
+};
+
+template <>
 struct XLoader<XConv> {
   const uint8_t* img;  // first byte of this row's image (+ group channel offset)
   int ih0, iw0;        // top-left input coordinate of the receptive field
@@ -322,6 +337,20 @@ struct KCursor<XLinear> {
     int64_t k = static_cast<int64_t>(kc) * 16;
     k = k < K ? k : K - 16;
     return ld16(row.p + k);
+  }
+};
+
+// (a chunk that reaches past K is read as the row's last 16 bytes and shifted to its place
+// when it is stored: no byte outside the row is touched)
+template <>
+struct KCursor<XLinearRagged> {
+  int kc;
+  int c;
+  __device__ __forceinline__ void init(const XLinearRagged&, int c_) { c = c_; kc = c_; }
+  __device__ __forceinline__ void seek(const XLinearRagged&, int kt) { kc = kt * kChunks + c; }
+  __device__ __forceinline__ v4i load(const XLinearRagged&, const XLoader<XLinearRagged>& row, int64_t K) const {
+    const int64_t k = static_cast<int64_t>(kc) * 16;
+    return ld16_any(row.p + (k + 16 <= K ? k : K - 16));
   }
 };
 
@@ -526,13 +555,15 @@ __device__ __forceinline__ uint32_t requant4_post(const int (&raw)[4], v4f bdiv,
 // fragment reads behind it.
 //
 // KW > 1 (register staging only): KW groups of WM x WN
-// waves share one output tile and split its k loop into KW equal runs of
+// waves share one output tile and split its k loop into KW runs of
 // stages, each group with its own LDS stages and registers; after the loop the
 // groups' accumulators are added through LDS and group 0 runs the epilogue.
 // For grids far smaller than the chip: a lone block per CU spends most of a
 // stage waiting on its own chain LDS store -> barrier -> LDS read -> MFMA, and
-// the other groups' waves fill those gaps.  The host sends only k loops whose
-// stage count KW divides.
+// the other groups' waves fill those gaps.  The groups share the barriers, so
+// all walk the longest run; a group whose run is shorter (the stage count is no
+// multiple of KW) stores zeros for the activations of the stages it lacks.  Every
+// group has at least one stage of its own.
 template <int BM, int BN, int WM, int WN, int MODE, class XSRC, int PD = 4, bool WDMA = false, int KW = 1,
           bool XWIDE = false>
 __global__ __launch_bounds__(WM* WN* KW* kWave, (WDMA && WM * WN == 4 && (BM / WM) * (BN / WN) <= 128 * 64) ? 2 : 1)
@@ -541,13 +572,20 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
   constexpr int NTB = NT * KW;          // threads of the block
   static_assert(KW >= 1 && (KW == 1 || !WDMA), "k-split groups: register staging only");
   const int kg = KW == 1 ? 0 : static_cast<int>(threadIdx.x) / NT;  // this thread's group
+  constexpr bool kRagged = std::is_same<XSRC, XLinearRagged>::value;
+  constexpr bool kRows = kRagged || std::is_same<XSRC, XLinear>::value;
+  static_assert(!kRagged || !WDMA, "rows off the 16-byte grid: register staging only");
+  int run_stages = 0;                   // KW > 1: stages of the longest run
   if constexpr (KW > 1) {  // this group's share of K: move the operands, shorten K
-    const int64_t per = ceil_div(a.K, kBK) / KW;
-    const int64_t k0 = kg * per * kBK;
+    const int all = static_cast<int>(ceil_div(a.K, kBK)), per = all / KW, longer = all - per * KW;
+    const int64_t first = kg * per + (kg < longer ? kg : longer);
+    const int64_t mine = per + (kg < longer ? 1 : 0);
+    const int64_t k0 = first * kBK;
     const int64_t left = a.K - k0;
-    a.K = left < per * kBK ? left : per * kBK;
-    a.w_packed += kg * per * (kChunks * 256);
-    if constexpr (std::is_same<XSRC, XLinear>::value)
+    run_stages = per + (longer > 0 ? 1 : 0);
+    a.K = left < mine * kBK ? left : mine * kBK;
+    a.w_packed += first * (kChunks * 256);
+    if constexpr (kRows)
       xsrc.x += k0;
     else
       xsrc.kc0 += static_cast<int>(k0 / 16);
@@ -1004,12 +1042,26 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       xreg[set][k - NW] = kcur.load(xsrc, xl[k - NW], a.K);
     }
   };
-  // k-th LDS store of a stage
-  auto store_one = [&](int set, int buf, int k) {
-    if (k < NW)
+  // k-th LDS store of stage kt
+  int tail_shift = 0;  // kRagged: bytes this thread's chunk of the last stage was read too early
+  if constexpr (kRagged) {
+    const int past = (KT - 1) * kBK + (t & 3) * 16 - (static_cast<int>(a.K) - 16);
+    tail_shift = past > 0 && past < 16 ? past : 0;  // (16 and more: all of it past K, against zero weights)
+  }
+  auto store_one = [&](int set, int buf, int k, int kt) {
+    if (k < NW) {
       *reinterpret_cast<v4i*>(&gmem[buf * kWStage + wdst[k]]) = wreg[set][k];
-    else
-      *reinterpret_cast<v4i*>(&gmem[buf * kXStage + xdst[k - NW]]) = xreg[set][k - NW] ^ xmask;
+    } else {
+      v4i v = xreg[set][k - NW];
+      if constexpr (kRagged)
+        if (kt == KT - 1) v = shift_down_bytes(v, tail_shift);
+      v ^= xmask;
+      if constexpr (KW > 1) {
+        const int keep = kt < KT ? -1 : 0;
+        v &= v4i{keep, keep, keep, keep};
+      }
+      *reinterpret_cast<v4i*>(&gmem[buf * kXStage + xdst[k - NW]]) = v;
+    }
   };
 
   // ---- software pipeline.
@@ -1050,7 +1102,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
 #pragma unroll
       for (int o = q * (NF + NG) / Q; o < (q + 1) * (NF + NG) / Q; ++o) {
         if (o < NF) read_one(buf ^ 1, buf ^ 1, 0, o, wf0, xf0);
-        else store_one(store_set, buf, o - NF);
+        else store_one(store_set, buf, o - NF, kt + 2);
       }
       mfma(q, wf1, xf1);
       __builtin_amdgcn_sched_barrier(0);
@@ -1063,26 +1115,27 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
 #pragma unroll
   for (int k = 0; k < NG; ++k) load_one(1 % NSET, clampk(1), k);
 #pragma unroll
-  for (int k = 0; k < NG; ++k) store_one(0, 0, k);
+  for (int k = 0; k < NG; ++k) store_one(0, 0, k, 0);
 #pragma unroll
   for (int s = 2; s < PD; ++s)
 #pragma unroll
     for (int k = 0; k < NG; ++k) load_one(s % NSET, clampk(s), k);
   // (with NSET == 2 the loads of stage 2 reuse set 0, already stored above)
 #pragma unroll
-  for (int k = 0; k < NG; ++k) store_one(1 % NSET, 1, k);
+  for (int k = 0; k < NG; ++k) store_one(1 % NSET, 1, k, 1);
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < NF; ++j) read_one(0, 0, 0, j, wf0, xf0);
 
+  const int KTR = KW > 1 ? run_stages : KT;  // stages this group walks: all groups the same
   int kt0 = 0;
-  for (; kt0 + NSET <= KT; kt0 += NSET) {
+  for (; kt0 + NSET <= KTR; kt0 += NSET) {
 #pragma unroll
     for (int j = 0; j < NSET; ++j) stage(kt0 + j, (j + 1) % NSET, (j + 2) % NSET);
   }
 #pragma unroll
   for (int j = 0; j < NSET - 1; ++j)
-    if (kt0 + j < KT) stage(kt0 + j, (j + 1) % NSET, (j + 2) % NSET);
+    if (kt0 + j < KTR) stage(kt0 + j, (j + 1) % NSET, (j + 2) % NSET);
   }
 
   if constexpr (KW > 1) {

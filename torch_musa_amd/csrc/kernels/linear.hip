@@ -557,12 +557,13 @@ __global__ __launch_bounds__(256) void linear_plain_kernel(GemmArgs a, XLinear x
   }
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, int PD = 4, bool WDMA = false, int KW = 1, bool XWIDE = false>
-int launch_gemm(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
+template <int BM, int BN, int WM, int WN, int MODE, int PD = 4, bool WDMA = false, int KW = 1, bool XWIDE = false,
+          class XSRC = XLinear>
+int launch_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  if (KW > 1 && ceil_div(a.K, kBK) % KW != 0) return TMQ_ERR_UNSUPPORTED;  // equal runs of stages only
-  gemm_i8_kernel<BM, BN, WM, WN, MODE, XLinear, PD, WDMA, KW, XWIDE>
+  if (ceil_div(a.K, kBK) < KW) return TMQ_ERR_UNSUPPORTED;  // a stage for every wave group
+  gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, PD, WDMA, KW, XWIDE>
       <<<dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s>>>(a, xs);
   return launch_status();
 }
@@ -769,9 +770,13 @@ constexpr int64_t kSplitMinStages = 16;  // shortest run of stages per split
 //    18.0 against 15.5 us streaming).
 enum class SmallRows { kStream, kTiles, kSplit };
 
+// 64 x 64 tiles whose k loop two wave groups share: at most one block per CU and a loop long enough to
+// pay for adding the groups' sums (us, one group | two: K = 6592, N = 1600, M = 266 21.3 | 16.2; K = 4160,
+// N = 4096, M = 256 14.8 | 12.2; K = 2064, N = 1000, M = 517 9.0 | 8.1; K = 1536, N = 2048, M = 300 7.4 | 6.7;
+// K = 1344, N = 168, M = 2017 7.1 | 6.7; K = 1088, N = 1024, M = 200 5.9 | 5.9; 275 tiles, K = 1600 9.8 | 10.2;
+// four groups are behind two at all of these).
 bool two_wave_groups_fit(int64_t M, int64_t N, int64_t K) {
-  const int64_t stages = ceil_div(K, kBK);
-  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && stages >= 32 && stages % 2 == 0;
+  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && ceil_div(K, kBK) >= 20;
 }
 
 SplitPlan plan_split_tiles(int64_t M, int64_t N, int64_t K);
@@ -1005,6 +1010,7 @@ struct LinearQuery {
 constexpr int kNoKernel = -2;
 struct LinearChoice {
   int cfg = kNoKernel;
+  int groups = 1;  // wave groups that share the k loop of a 64 x 64 tile (cfg 2; cfg 14 always has two)
   SplitPlan split;
 };
 
@@ -1194,8 +1200,10 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     else if (nblk(64, 64) <= 256 && ceil_div(K, kBK) >= 32 && ceil_div(K, kBK) % 2 == 0)
       cfg = 14;  // at most one block per CU and a long k loop: two wave groups halve it (14.7 -> 11.7 us
                  // at M = 128, K = N = 4096; four groups run into the L2's bandwidth: 12.3 us)
-    else
+    else {
       cfg = 2;
+      c.groups = two_wave_groups_fit(M, N, K) ? 2 : 1;  // (an odd number of stages, or a shorter loop)
+    }
   }
   const bool wide_ok = wide_limits_ok(K, q.ldx);
   if (cfg == 19 && !wide_ok) cfg = 17;
@@ -1237,6 +1245,22 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
   return c;
 }
 
+// More than 16 rows off the 16-byte grid: 64 x 64 tiles that read the rows where they lie, or a copy
+// onto the grid and the padded shape's own kernel.  The copy is a launch (2.2 us and a scratch
+// allocation); the larger tiles it opens earn that back from 512 tiles on, later where K is short
+// (us, direct | copy: M = 517: K = 1000, N = 2051 7.9 | 10.1, K = 2051, N = 1000 8.8 | 11.4; K = 3907,
+// N = 193, M = 2889 12.7 | 23.8; K = 4100, N = 3900, M = 500 (488 tiles) 21.1 | 24.4; K = 2051, N = 2051,
+// M = 1000 (528) 18.2 | 16.9; K = 700, N = 2000: M = 2048 (1024) 10.1 | 10.7; K = 1500, N = 2000, M = 2000
+// (1024) 19.6 | 16.4; K = 500, N = 2000, M = 3000 (1504) 12.5 | 12.2; K = 100, N = 1000, M = 8000 (2000)
+// 10.1 | 12.9; K = 120, N = 8000, M = 4096 (8000) 26.6 | 22.9).  Rows few enough for the streaming kernel
+// keep it (M = 40, K = 4100, N = 512 12.0 | 10.6).
+bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
+  if (K < 16 || K > 0x7fffff00) return false;
+  if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return false;
+  const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64);
+  return tiles <= (K <= 128 ? 3072 : K <= 768 ? 1024 : 512);
+}
+
 template <int MODE>
 int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec_ok, int forced,
                     hipStream_t s, void* workspace = nullptr, int64_t workspace_bytes = 0) {
@@ -1253,10 +1277,16 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
   if (a.splits != 1) return TMQ_ERR_INVALID_ARGUMENT;  // the split is this function's to plan
   if (!vec_ok && forced < 0) {
     // Off the 16-byte grid: up to 16 rows stream the weights as they are (the copy would cost a
-    // launch, more than any other kernel's advantage at so few rows); more rows are copied onto
-    // the grid if the caller left room for that, and take the kernel of the padded shape.
+    // launch, more than any other kernel's advantage at so few rows); more rows take 64 x 64 tiles
+    // that read them where they lie, or are copied onto the grid if the caller left room for that
+    // and take the kernel of the padded shape.
     if (a.M <= kDecodeRowsAuto && a.K >= 16 && stream_limits_ok(q) && a.w_kchunks == packed_kchunks(a.K))
       return launch_linear_decode_ragged<MODE>(a, xs, s);
+    if (ragged_tiles_preferred(a.M, a.N, a.K)) {
+      const XLinearRagged rows{xs.x, xs.ldx};
+      return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
+                                                : launch_gemm<64, 64, 2, 2, MODE>(a, rows, s);
+    }
     const int64_t room = regrid_bytes(a.M, a.K);
     if (regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room) {
       const int rc = launch_regrid(xs, a.M, a.K, workspace, s);
@@ -1294,7 +1324,8 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     case 13: return run_split<MODE>(a, xs, c.split, workspace, dma_limits_ok(a.K, xs.ldx), s);
     case 0: return launch_gemm<256, 256, 2, 2, MODE>(a, xs, s);
     case 1: return launch_gemm<128, 128, 2, 2, MODE>(a, xs, s);
-    case 2: return launch_gemm<64, 64, 2, 2, MODE>(a, xs, s);
+    case 2: return c.groups == 2 ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s)
+                                 : launch_gemm<64, 64, 2, 2, MODE>(a, xs, s);
     case 3: return launch_gemm<256, 256, 2, 4, MODE, 3>(a, xs, s);
     case 4: return launch_gemm<128, 256, 2, 2, MODE>(a, xs, s);
     case 5: return launch_gemm<256, 128, 2, 2, MODE>(a, xs, s);
@@ -1393,7 +1424,7 @@ TMQ_EXPORT int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (K % 16 == 0 && on_grid) return tmq_linear_workspace_bytes(M, N, K);
-  if ((M <= kDecodeRowsAuto && K >= 16) || !regrid_limits_ok(M, K)) return 0;
+  if ((M <= kDecodeRowsAuto && K >= 16) || ragged_tiles_preferred(M, N, K) || !regrid_limits_ok(M, K)) return 0;
   return regrid_bytes(M, K) + tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
 }
 
@@ -1431,7 +1462,8 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     case 0: bm = 256, bn = 256; break;
     case 3: case 6: case 20: bm = 256, bn = 256, waves = 8; break;
     case 1: case 7: case 13: bm = 128, bn = 128; break;
-    case 2: case 21: bm = 64, bn = 64; break;
+    case 2: bm = 64, bn = 64, waves = 4 * c.groups; break;
+    case 21: bm = 64, bn = 64; break;
     case 14: bm = 64, bn = 64, waves = 8; break;
     case 4: bm = 128, bn = 256; break;
     case 17: case 19: bm = 128, bn = 256, waves = 8; break;
