@@ -69,10 +69,12 @@ def test_plain_tensor_linear_in_16_bits(m, k, n, dtype):
 @pytest.mark.parametrize("m,k,n", [
     # an odd or short run of stages shared by two wave groups: 20, 21 (the last one 16 bytes), 33, 103 stages
     (64, 1280, 64), (130, 1296, 100), (517, 2064, 70), (266, 6592, 130),
+    # 64 x 128 tiles with all of K in LDS: one chunk, two to four phases, edges of tiles
+    (129, 16, 10000), (1030, 272, 1001), (384, 768, 3072), (500, 784, 3000), (65, 1024, 16100),
     # rows read where they lie: the last chunk 1 ... 15 bytes, one stage, one and two wave groups, edges of tiles
     (17, 17, 65), (129, 65, 1), (65, 127, 64), (400, 1279, 66), (64, 1281, 65), (70, 2049, 129), (300, 8191, 67)])
 @pytest.mark.parametrize("relu", [False, True])
-def test_tiles_of_64_in_wave_groups_and_on_rows_off_the_grid(m, k, n, relu):
+def test_tiles_of_64_rows(m, k, n, relu):
     """Exact integer sums and the requantisation of the CPU operator: the same bytes."""
     gen = torch.Generator().manual_seed(m * 7919 + k * 31 + n)
     w, b = _weight(n, k, n % 2 == 0, gen), torch.randn(n, generator=gen)

@@ -13,7 +13,8 @@
 // synchronisation; behind the barrier that ends phase p the buffer it used takes
 // phase p + 4.
 //
-// The automatic choice sends K <= 1024 here (grids of at most 256 tiles; up to 512
+// The automatic choice sends K <= 1024 here (grids of at most 256 tiles; where 64 x 64 tiles are
+// more than that and 64 x 128 ones are not, those: 384 x 768 x 3072, 6.6 -> 5.8 us; up to 512
 // tiles of 32 x 32 go to gemm_i8_ksplit_kernel at the end of this file).  Longer
 // K runs (any K, for tests) but does not pay: with cold weights a phase then
 // waits for memory, 96 KB in flight per CU against about 2 us of latency, and
@@ -43,12 +44,17 @@ __device__ __forceinline__ void lds_dma4(const void* base, uint32_t off, uint32_
                : "memory", "m0");
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinear xs) {
-  constexpr int BM = 64, BN = 64;
+// BN = 128 (eight waves of the same 32 x 32, a ring of three phases, 144 KB): for grids whose 64 x 64 tiles
+// are a little more than the chip holds and would need a second round.
+template <int MODE, int BN = 64>
+__global__ __launch_bounds__(BN * 4) void gemm_i8_onepass_kernel(GemmArgs a, XLinear xs) {
+  constexpr int BM = 64, kThreads = BN * 4, kWaves = kThreads / kWave;
   constexpr int kPhaseChunks = 16;                 // k-chunks per barrier: 256 bytes of K
-  constexpr int kRing = 4;                         // phases the LDS buffers hold
-  constexpr int kCopiesPerPhase = 8;               // per wave: 4 weight chunks + 4 activation row groups
+  constexpr int kRing = BN == 64 ? 4 : 3;          // phases the LDS buffers hold
+  constexpr int NX = 16 / kWaves;                  // activation copies (four rows each) per wave and phase
+  constexpr int kCopiesPerPhase = 4 + NX;          // per wave: 4 weight copies + the activation copies
+  constexpr int kHalves = BN / 64;                 // weight copies (64 rows of one k-chunk each) per k-chunk
+  static_assert(kPhaseChunks * kHalves == 4 * kWaves, "weight copies per wave");
   __shared__ __attribute__((aligned(16))) uint8_t sW[kRing * kPhaseChunks * BN * 16];
   __shared__ __attribute__((aligned(16))) uint8_t sX[kRing * BM * 256];
   __shared__ __attribute__((aligned(16))) int s_raw[3][BN];  // colsum, weight scale, bias as fetched
@@ -69,61 +75,66 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
 
   // ---- requests, oldest first: the tile's per-channel constants (wave 0), then
   // phase by phase the weight chunks and activation row groups of this wave
-  if (wave_u == 0) {
-    const int64_t n = n0 + lane < a.N ? n0 + lane : a.N - 1;
-    const uint32_t np = static_cast<uint32_t>(n + a.n_off);
-    lds_dma4(a.colsum, np * 4u, lds_address(&s_raw[0][0]));
+  if (wave_u < kHalves) {
+    const int64_t nl = n0 + wave_u * kWave + lane;
+    const uint32_t np = static_cast<uint32_t>((nl < a.N ? nl : a.N - 1) + a.n_off);
+    lds_dma4(a.colsum, np * 4u, lds_address(&s_raw[0][wave_u * kWave]));
     if constexpr (MODE != kOutAcc32) {  // (raw accumulators: the caller passes no scales)
-      lds_dma4(a.w_scales, np * static_cast<uint32_t>(a.w_scale_stride) * 4u, lds_address(&s_raw[1][0]));
+      lds_dma4(a.w_scales, np * static_cast<uint32_t>(a.w_scale_stride) * 4u, lds_address(&s_raw[1][wave_u * kWave]));
       lds_dma4(a.bias != nullptr ? a.bias : a.w_scales, a.bias != nullptr ? np * 4u : 0u,
-               lds_address(&s_raw[2][0]));
+               lds_address(&s_raw[2][wave_u * kWave]));
     }
   }
   const int64_t NB = ceil_div(a.N, 16);
   const int64_t nb_last = NB - 1 - n0 / 16;        // 16-row blocks past N: clamped, never stored
   const uint8_t* const wtile = a.w_packed + (n0 / 16) * a.w_kchunks * 256;
-  const int64_t rb = (lane >> 4) < nb_last ? (lane >> 4) : nb_last;
-  const uint32_t woff = static_cast<uint32_t>(rb * a.w_kchunks * 256 + (lane & 15) * 16);
+  uint32_t woff[kHalves];
+#pragma unroll
+  for (int h = 0; h < kHalves; ++h) {
+    const int64_t rb = 4 * h + (lane >> 4) < nb_last ? 4 * h + (lane >> 4) : nb_last;
+    woff[h] = static_cast<uint32_t>(rb * a.w_kchunks * 256 + (lane & 15) * 16);
+  }
   const int kc_last = static_cast<int>(a.w_kchunks) - 1;
   const uint8_t* const xtile = xs.x + m0 * xs.ldx;
   const int64_t m_last = a.M - 1 - m0;             // rows past M: clamped, never stored
   const uint32_t ldsW = lds_address(sW), ldsX = lds_address(sX);
-  uint32_t xrow_off[4];                            // this lane's row of the wave's four activation copies
-  int xslot[4];
+  uint32_t xrow_off[NX];                           // this lane's row of the wave's activation copies
+  int xslot[NX];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 4 * (4 * wave_u + i) + (lane >> 4);
+  for (int i = 0; i < NX; ++i) {
+    const int r = 4 * (NX * wave_u + i) + (lane >> 4);
     const int64_t rc = r < m_last ? r : m_last;
     xrow_off[i] = static_cast<uint32_t>(rc * xs.ldx);
     xslot[i] = (lane & 15) ^ (r & 15);
   }
-  // the eight copies of this wave for phase p, into ring buffer p % kRing
+  // the copies of this wave for phase p, into ring buffer p % kRing
   auto issue = [&](int p) {
-    const int b = p & (kRing - 1);
+    const int b = p % kRing;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int kc = p * kPhaseChunks + 4 * wave_u + i;
+      const int wc = (4 * wave_u + i) / kHalves, h = i % kHalves;
+      const int kc = p * kPhaseChunks + wc;
       const int kcc = kc < kc_last ? kc : kc_last;   // (chunks past the packed pitch are never multiplied)
-      lds_dma16(wtile + static_cast<int64_t>(kcc) * 256, woff,
-                ldsW + static_cast<uint32_t>(b * kPhaseChunks + 4 * wave_u + i) * 1024u);
+      lds_dma16(wtile + static_cast<int64_t>(kcc) * 256, woff[h],
+                ldsW + static_cast<uint32_t>((b * kPhaseChunks + wc) * kHalves + h) * 1024u);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NX; ++i) {
       const int cc = p * kPhaseChunks + xslot[i];
       // chunks past K: any bytes of the row will do, they meet a zeroed operand or zero weights
       const int ccc = cc < KC ? cc : KC - 1;
       lds_dma16(xtile, xrow_off[i] + static_cast<uint32_t>(ccc) * 16u,
-                ldsX + static_cast<uint32_t>(b * BM + 4 * (4 * wave_u + i)) * 256u);
+                ldsX + static_cast<uint32_t>(b * BM + 4 * (NX * wave_u + i)) * 256u);
     }
   };
   // waits until at most `phases` phases of this wave's copies (the youngest) are outstanding
   auto wait_phases = [&](int phases) {
-    static_assert(kCopiesPerPhase == 8, "the wait counts below are multiples of the copies per phase");
+    constexpr int C1 = kCopiesPerPhase, C2 = 2 * C1, C3 = 3 * C1;  // (lgkmcnt and expcnt are left alone)
     switch (phases) {
-      case 0: __builtin_amdgcn_s_waitcnt((0 & 15) | ((0 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
-      case 1: __builtin_amdgcn_s_waitcnt((8 & 15) | ((8 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
-      case 2: __builtin_amdgcn_s_waitcnt((16 & 15) | ((16 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
-      default: __builtin_amdgcn_s_waitcnt((24 & 15) | ((24 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
+      case 0: __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); break;
+      case 1: __builtin_amdgcn_s_waitcnt((C1 & 15) | ((C1 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
+      case 2: __builtin_amdgcn_s_waitcnt((C2 & 15) | ((C2 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
+      default: __builtin_amdgcn_s_waitcnt((C3 & 15) | ((C3 >> 4) << 14) | (7 << 4) | (15 << 8)); break;
     }
   };
 
@@ -163,7 +174,7 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
   }
 
   for (int p = 0; p < NP; ++p) {
-    const int b = p & (kRing - 1);
+    const int b = p % kRing;
     const int left = S - p * (kPhaseChunks / 2);
     const int nsteps = left < kPhaseChunks / 2 ? left : kPhaseChunks / 2;
     // (k-steps past the end of K in the last phase read whatever the buffers
@@ -183,7 +194,7 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
     }
     if (p + 1 < NP) {
       // Phase p+1 must have landed; what this wave may still have on its way are
-      // the phases after it that were already requested (up to p+3).  Behind the
+      // the phases after it that were already requested (up to p + kRing - 1).  Behind the
       // barrier every wave is done with buffer p % kRing, which takes phase p+kRing.
       const int youngest = p + kRing - 1 < NP - 1 ? p + kRing - 1 : NP - 1;
       wait_phases(youngest - (p + 1));
@@ -218,7 +229,7 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
     __syncthreads();
     constexpr int kRowChunks = BN / 4;
 #pragma unroll
-    for (int id = t; id < BM * kRowChunks; id += 256) {
+    for (int id = t; id < BM * kRowChunks; id += kThreads) {
       const int row = id / kRowChunks, cc = id % kRowChunks;
       const int64_t m = m0 + row, n = n0 + cc * 4;
       if (m >= a.M || n >= a.N) continue;
@@ -246,7 +257,7 @@ __global__ __launch_bounds__(256) void gemm_i8_onepass_kernel(GemmArgs a, XLinea
     uint8_t* const y = static_cast<uint8_t*>(a.y) + a.n_off;
     const bool vec_ok = ((a.ldy & 15) == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
     constexpr int kRowChunks = BN / 16;
-    const int row = t / kRowChunks, cc = t % kRowChunks;   // 256 threads: one 16-byte piece each
+    const int row = t / kRowChunks, cc = t % kRowChunks;   // four threads per channel: one 16-byte piece each
     const int64_t m = m0 + row, n = n0 + cc * 16;
     if (m < a.M && n < a.N) {
       const v4i v = ld16(&sW[row * kPitch + cc * 16]);

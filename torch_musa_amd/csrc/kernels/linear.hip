@@ -568,13 +568,13 @@ int launch_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   return launch_status();
 }
 
-// 64 x 64 tiles with all of K in LDS (K <= 1024; the caller checked the address ranges).
-template <int MODE>
+// 64 x 64 (64 x 128) tiles with all of K in LDS (K <= 1024; the caller checked the address ranges).
+template <int MODE, int BN = 64>
 int launch_gemm_onepass(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
-  const int64_t tiles_m = ceil_div(a.M, 64), tiles_n = ceil_div(a.N, 64);
+  const int64_t tiles_m = ceil_div(a.M, 64), tiles_n = ceil_div(a.N, BN);
   if (tiles_n > 0x7fffffff || tiles_m > 65535) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_onepass_kernel<MODE>
-      <<<dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(256), 0, s>>>(a, xs);
+  gemm_i8_onepass_kernel<MODE, BN>
+      <<<dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(BN * 4), 0, s>>>(a, xs);
   return launch_status();
 }
 
@@ -1011,6 +1011,7 @@ constexpr int kNoKernel = -2;
 struct LinearChoice {
   int cfg = kNoKernel;
   int groups = 1;  // wave groups that share the k loop of a 64 x 64 tile (cfg 2; cfg 14 always has two)
+  bool onepass = false;  // 64 x 128 tiles with all of K in LDS (cfg 23)
   SplitPlan split;
 };
 
@@ -1075,6 +1076,17 @@ bool dynamic_resident_preferred(int64_t M, int64_t N, int64_t K) {
   return !(M <= 2 && N <= 4096 && K > 2048 && K <= 4096);
 }
 
+// 64 x 128 tiles with all of K in LDS, where 64 x 64 ones would need a second round of blocks and these fit
+// one (us, these | the pipelined tiles: K = 768, N = 3072: M = 384 5.8 | 6.6, M = 512 5.8 | 6.7, M = 640 5.9 | 6.8;
+// K = 256, N = 2000, M = 1000 4.3 | 5.6; K = 64, N = 1000, M = 2000 4.7 | 6.7; K = 512, N = 1024, M = 2048 5.1 | 6.1;
+// two rounds of them, K = 640, N = 1500, M = 1500: 10.4 | 8.2).  A K of four phases waits for the ring once:
+// K = 1024: N = 1024, M = 2048 (512 tiles of 64 x 64) 6.9 | 7.5, N = 300, M = 4096 (320) 7.2 | 7.7, N = 1600,
+// M = 700 (275) 7.8 | 7.3; K = 1008, N = 2051, M = 517 (297) 8.4 | 7.5.
+bool onepass_wide_preferred(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64);
+  return K <= kOnePassMaxK && tiles > (K <= 768 ? 256 : 300) && ceil_div(M, 64) * ceil_div(N, 128) <= 256;
+}
+
 // forced: tmq_linear_desc::kernel - 1 (-1 = automatic choice).
 LinearChoice choose_linear(const LinearQuery& q, int forced) {
   LinearChoice c;
@@ -1117,6 +1129,9 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     // whose waves split K spread the copies over more CUs (3.8 us; M = 512: 5.7 -> 4.4 us;
     // N = 4096, K = 512, M = 128: 4.4 -> 4.3 us; 640 tiles and more, or K <= 256: slower)
     cfg = K > 256 && ceil_div(M, 32) * ceil_div(N, 32) <= 512 ? 24 : 21;
+  } else if (cfg < 0 && onepass_ok && onepass_wide_preferred(M, N, K)) {
+    cfg = 23;
+    c.onepass = true;
   } else if (cfg < 0 && onepass_ok && wstream_tile(M, N, K) != 0) {
     // K up to 4096 on a grid of 32 x 32 tiles that the chip holds at once: the waves split
     // K and take their weights through registers (cold weights, K = N = 4096, M = 64:
@@ -1336,7 +1351,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     case 19: return launch_gemm<128, 256, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
     case 20: return launch_gemm_persistent<MODE>(a, xs, s);
     case 22: return launch_gemm<128, 64, 2, 2, MODE>(a, xs, s);
-    case 23: return launch_gemm<64, 128, 2, 2, MODE>(a, xs, s);
+    case 23: return c.onepass ? launch_gemm_onepass<MODE, 128>(a, xs, s) : launch_gemm<64, 128, 2, 2, MODE>(a, xs, s);
     case 21: return launch_gemm_onepass<MODE>(a, xs, s);
     case 24: return launch_gemm_ksplit<MODE>(a, xs, s);
     case 25: return launch_gemm_wstream<MODE>(a, xs, false, s);
@@ -1469,7 +1484,7 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     case 17: case 19: bm = 128, bn = 256, waves = 8; break;
     case 5: bm = 256, bn = 128; break;
     case 22: bm = 128, bn = 64; break;
-    case 23: bm = 64, bn = 128; break;
+    case 23: bm = 64, bn = 128, waves = c.onepass ? 8 : 4; break;
     case 24: case 25: bm = 32, bn = 32; break;
     case 26: bm = 32, bn = 64, waves = 8; break;
     case 27: bm = 64, bn = 64, waves = 8; break;
