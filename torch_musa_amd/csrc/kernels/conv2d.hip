@@ -39,7 +39,7 @@ struct ConvShape {
   // (0: the shape is not that kernel's), run bytes, padded run bytes, offset and size in bytes
   int64_t runs_KS, runs_RL, runs_RP, runs_off, runs_bytes;
   bool pixels4;  // ... laid out for the kernel of conv_image.h, three channels as four-byte pixels
-  // depthwise layers over a multiple of 4 channels: a [channel][kernel row][taps padded to a multiple
+  // depthwise layers over a multiple of 4 or at least 16 channels: a [channel][kernel row][taps padded to a multiple
   // of 4] copy of the weight for the kernel of conv_depthwise.h in the same place (0: not such a layer)
   int64_t taps_bytes;
 };
@@ -99,7 +99,7 @@ int make_shape(const tmq_conv2d_geom* g, ConvShape* s) {
     }
   }
   s->taps_bytes = 0;
-  if (g->groups > 1 && g->groups == g->IC && g->IC == g->OC && g->IC % 4 == 0)
+  if (g->groups > 1 && g->groups == g->IC && g->IC == g->OC && (g->IC % 4 == 0 || g->IC >= 16))
     s->taps_bytes = round_up(g->IC * g->KH * round_up(g->KW, 4), 16);
   // 32-bit index arithmetic inside the kernels
   if (g->H > (1 << 24) || g->W > (1 << 24) || g->IC > (1 << 24) || s->Kp > (1 << 30) ||
@@ -756,10 +756,10 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
   if (!pinned_strip && s.KH >= 5 && s.OH > 8) strip = ceil_div(s.OH, s.OH <= 14 ? 2 : ceil_div(s.OH, 14));
   const int64_t lanes_wanted = int64_t{1} << (s.KH == 7 && s.KW == 7 ? 15 : 16);
   if (!pinned_strip)
-    while (strip > 1 && s.B * ceil_div(s.OH, strip) * s.OW * (s.IC / 4) < lanes_wanted) strip = ceil_div(strip, 2);
+    while (strip > 1 && s.B * ceil_div(s.OH, strip) * s.OW * ceil_div(s.IC, 4) < lanes_wanted) strip = ceil_div(strip, 2);
   if (strip > s.OH) strip = s.OH;
   a.strip = static_cast<int>(strip);
-  const int64_t per_image = ceil_div(s.OH, strip) * s.OW * (s.IC / 4);
+  const int64_t per_image = ceil_div(s.OH, strip) * s.OW * ceil_div(s.IC, 4);
   const int64_t blocks_per_image = ceil_div(per_image, kDwThreads);
   a.per_image = static_cast<uint32_t>(per_image);
   a.blocks_per_image = static_cast<uint32_t>(blocks_per_image);
@@ -943,8 +943,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     // (32-bit byte offsets into the input and the output, also for the rows a window reaches past the image)
     const bool lanes_ok = s.taps_bytes > 0 && s.B * s.H * s.W * s.IC < (int64_t{1} << 31) &&
                           (s.H + s.KH * s.dh + s.sh + 8) * s.W * s.IC < (int64_t{1} << 31) &&
-                          s.B * s.OH * s.OW * s.OC < (int64_t{1} << (MODE == kOutAcc32 ? 29 : 31)) && aligned(d->x, 4) && aligned(out, MODE == kOutAcc32 ? 16 : 4) &&
-                          (po.accum == nullptr || aligned(po.accum, 4));
+                          s.B * s.OH * s.OW * s.OC < (int64_t{1} << (MODE == kOutAcc32 ? 29 : 31)) && aligned(out, MODE == kOutAcc32 ? 4 : 1);
     if (forced == 7 && !lanes_ok) return TMQ_ERR_UNSUPPORTED;
     // Also where the groups would merge into 16-channel blocks for the matrix pipe, for the kernel sizes with a
     // register window (batch 32, against the merged groups on the halo tiles or the implicit GEMM: 3 x 3, 32
