@@ -507,6 +507,9 @@ int tmq_qcat_rows(const void* x, void* y, int64_t outer, int64_t in_row, int64_t
                   int64_t out_col_offset, float in_scale, int32_t in_zero_point, float out_scale,
                   int32_t out_zero_point, int q_signed, tmq_stream_t stream);
 
+/* B images of three planes of `pixels` bytes each -> pixels of three bytes (NCHW to NHWC); at least 16 pixels. */
+int tmq_planes_to_pixels(const void* x, void* y, int64_t B, int64_t pixels, tmq_stream_t stream);
+
 /* Max pooling over NHWC codes (replaces MaxPool2dQuantized /
  * QuantizedMaxPool2dImpl, torch_musa/csrc/aten/quantized/Pool.cpp:80-130,178-247,
  * muDNN Pooling): y[b,oh,ow,c] = max over the window's in-image positions of

@@ -2,6 +2,7 @@
 of four pixels over the image's edges and the tensor's ends, channel tails, one and several k-steps, tiles in columns."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from gpu_util import say
@@ -34,3 +35,24 @@ def test_image_conv(cabi, spec, x_signed):  # noqa: F811
     want = oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
                          c["out_zp"], relu=c["relu"], nthreads=8)
     _check(y, want, "image conv")
+
+
+@pytest.mark.parametrize("size", [(1, 3, 5), (1, 4, 4), (2, 1, 17), (3, 7, 11), (2, 64, 48), (1, 3, 4099)])
+@pytest.mark.parametrize("at", [0, 1])
+def test_planes_to_pixels(cabi, size, at):
+    b, h, w = size
+    x = torch.randint(0, 256, (b * 3 * h * w + at,), dtype=torch.uint8).cuda()[at:].view(b, 3, h, w)
+    print("[case]", size, at, flush=True)
+    y = torch.full((b, h, w, 3), 77, dtype=torch.uint8, device="cuda")
+    rc = cabi.lib().tmq_planes_to_pixels(x.data_ptr(), y.data_ptr(), b, h * w, cabi.stream_ptr())
+    assert rc == (0 if h * w >= 16 else 2)  # fewer than 16 pixels are refused
+    assert torch.equal(y, x.permute(0, 2, 3, 1)) if rc == 0 else bool((y == 77).all())
+
+
+def test_image_in_nchw_memory_gives_the_same_bytes(cabi):
+    x = torch.quantize_per_tensor(torch.randn(2, 3, 33, 29).cuda(), 0.03, 128, torch.quint8)
+    w = torch.quantize_per_tensor(torch.randn(24, 3, 3, 3).cuda(), 0.02, 0, torch.qint8)
+    packed = torch.ops.quantized.conv2d_prepack(w, None, [2, 2], [1, 1], [1, 1], 1)
+    y = torch.ops.quantized.conv2d(x, packed, 0.1, 100)
+    z = torch.ops.quantized.conv2d(x.contiguous(memory_format=torch.channels_last), packed, 0.1, 100)
+    assert torch.equal(y.int_repr(), z.int_repr())

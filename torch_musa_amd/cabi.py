@@ -28,7 +28,7 @@ DECLARED_SYMBOLS = [
     "tmq_quantize_per_tensor_dynamic_report", "tmq_quantize_rows_dynamic_dev", "tmq_linear_scratch_bytes", "tmq_linear_float", "tmq_per_channel",
     "tmq_conv2d_packed_bytes", "tmq_conv2d_prepack", "tmq_conv2d_out_hw", "tmq_conv2d_workspace_bytes",
     "tmq_conv2d", "tmq_conv2d_acc32", "tmq_conv2d_fused",
-    "tmq_qadd", "tmq_qrelu", "tmq_qcat_rows", "tmq_qmaxpool2d", "tmq_qadaptive_avgpool2d", "tmq_qunary",
+    "tmq_qadd", "tmq_qrelu", "tmq_qcat_rows", "tmq_planes_to_pixels", "tmq_qmaxpool2d", "tmq_qadaptive_avgpool2d", "tmq_qunary",
 ]
 
 
@@ -150,6 +150,7 @@ def lib() -> C.CDLL:
         l.tmq_qrelu.argtypes = [v, v, C.c_int64, C.c_int32, C.c_int, v]
         l.tmq_qcat_rows.argtypes = [v, v, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_float, C.c_int32,
                                     C.c_float, C.c_int32, C.c_int, v]
+        l.tmq_planes_to_pixels.argtypes = [v, v, C.c_int64, C.c_int64, v]
         l.tmq_qmaxpool2d.argtypes = [v, v] + [C.c_int64] * 4 + [C.c_int32] * 8 + [C.c_int64] * 2 + [C.c_int, v]
         l.tmq_qadaptive_avgpool2d.argtypes = [v, v] + [C.c_int64] * 6 + [C.c_int32, C.c_int, v]
         l.tmq_qunary.argtypes = [v, v, C.c_int64, C.c_int, C.c_float, C.c_int32, C.c_float, C.c_int32, C.c_int, v]

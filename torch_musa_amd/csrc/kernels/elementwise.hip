@@ -392,6 +392,35 @@ __global__ __launch_bounds__(kEwThreads) void qmaxpool_k3_rows_kernel(const uint
   store_codes16(y + ((b * OH + oh) * OW + ow) * static_cast<int64_t>(C) + c, m.result());
 }
 
+// Three planes of bytes to pixels of three (an image in NCHW on its way into a convolution or a pooling).
+// A thread takes 16 pixels: three 16-byte loads and three 16-byte stores at whatever address they have, the
+// bytes interleaved in registers, six permutes for four pixels; the last 16 pixels of an image overlap the 16
+// before them (the same bytes).  Memory bounds it.
+__global__ __launch_bounds__(kEwThreads) void planes_to_pixels_kernel(const uint8_t* __restrict__ x, uint8_t* __restrict__ y,
+                                                                      int64_t pixels, int64_t groups, int64_t total) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kEwThreads + threadIdx.x;
+  if (i >= total) return;
+  const int64_t b = i / groups;
+  const int64_t p = group_channel<16>(i - b * groups, pixels);
+  const uint8_t* const src = x + b * 3 * pixels + p;
+  const v4i r = load_codes16(src), g = load_codes16(src + pixels), u = load_codes16(src + 2 * pixels);
+  uint32_t out[12];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // (v_perm_b32: bytes 0 ... 3 of a selector are those of the second word, 4 ... 7 those of the first)
+    const uint32_t rj = static_cast<uint32_t>(r[j]), gj = static_cast<uint32_t>(g[j]), bj = static_cast<uint32_t>(u[j]);
+    const uint32_t rg01 = __builtin_amdgcn_perm(gj, rj, 0x05010400u), rg23 = __builtin_amdgcn_perm(gj, rj, 0x07030602u);
+    out[3 * j] = __builtin_amdgcn_perm(bj, rg01, 0x02040100u);
+    out[3 * j + 1] = __builtin_amdgcn_perm(rg23, __builtin_amdgcn_perm(bj, rg01, 0x00000503u), 0x05040100u);
+    out[3 * j + 2] = __builtin_amdgcn_perm(bj, rg23, 0x07030206u);
+  }
+  uint8_t* const dst = y + (b * pixels + p) * 3;
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    store_codes16(dst + 16 * j, v4i{static_cast<int>(out[4 * j]), static_cast<int>(out[4 * j + 1]),
+                                    static_cast<int>(out[4 * j + 2]), static_cast<int>(out[4 * j + 3])});
+}
+
 // Adaptive average pooling: output pixel (oh, ow) averages the input window
 // rows floor(oh*H/OH) .. ceil((oh+1)*H/OH)-1 (likewise columns).  VEC = 4: a
 // thread owns four consecutive channels (one 32-bit word per input pixel).
@@ -610,6 +639,18 @@ TMQ_EXPORT int tmq_qcat_rows(const void* x, void* y, int64_t outer, int64_t in_r
     else
       qcat_rows_kernel<false, 1><<<grid, block, 0, s>>>(xb, yb, outer, in_row, out_row, out_col_offset, p);
   }
+  return launch_status();
+}
+
+TMQ_EXPORT int tmq_planes_to_pixels(const void* x, void* y, int64_t B, int64_t pixels, tmq_stream_t stream) {
+  if (B < 0 || pixels < 0) return TMQ_ERR_INVALID_ARGUMENT;
+  if (B == 0 || pixels == 0) return TMQ_OK;
+  if (x == nullptr || y == nullptr) return TMQ_ERR_INVALID_ARGUMENT;
+  if (pixels < 16) return TMQ_ERR_UNSUPPORTED;
+  const int64_t groups = ceil_div(pixels, 16), blocks = ceil_div(B * groups, kEwThreads);
+  if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
+  planes_to_pixels_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kEwThreads), 0, as_stream(stream)>>>(
+      static_cast<const uint8_t*>(x), static_cast<uint8_t*>(y), pixels, groups, B * groups);
   return launch_status();
 }
 
