@@ -1297,7 +1297,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     // and take the kernel of the padded shape.
     if (a.M <= kDecodeRowsAuto && a.K >= 16 && stream_limits_ok(q) && a.w_kchunks == packed_kchunks(a.K))
       return launch_linear_decode_ragged<MODE>(a, xs, s);
-    if (ragged_tiles_preferred(a.M, a.N, a.K)) {
+    if (ragged_tiles_preferred(a.M, a.N, a.K) && a.w_kchunks == packed_kchunks(a.K)) {
       const XLinearRagged rows{xs.x, xs.ldx};
       return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
                                                 : launch_gemm<64, 64, 2, 2, MODE>(a, rows, s);
