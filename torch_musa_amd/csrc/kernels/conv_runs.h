@@ -31,6 +31,7 @@
 #pragma once
 
 #include "gemm_i8_core.h"
+#include "tail_read.h"
 
 namespace tmq {
 
@@ -451,10 +452,9 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
 #pragma unroll
     for (int ks = 0; ks < KSN; ++ks) {
       const int k0 = ks * 64 + pq * 16;
-      const int64_t o = row + (k0 < a.RP ? k0 : 0);
-      const int over = static_cast<int>(o + 16 - x_bytes);  // (the host: a tensor of at least 16 bytes)
-      xv[ks] = ld16_any(a.x + (over > 0 ? o - over : o));
-      if (over > 0) xv[ks] = shift_down_bytes(xv[ks], over);  // the tensor's last few bytes
+      const TailRead r = tail_read16(row + (k0 < a.RP ? k0 : 0), x_bytes);  // (the host: a tensor of at least 16 bytes)
+      xv[ks] = ld16_any(a.x + r.at);
+      if (r.shift > 0) xv[ks] = shift_down_bytes(xv[ks], r.shift);  // the tensor's last few bytes
     }
   };
   const bool residual = POST == 1 || (POST == 2 && a.post.accum != nullptr);
