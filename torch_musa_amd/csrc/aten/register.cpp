@@ -30,15 +30,16 @@
 #include <torch/library.h>
 
 #include <array>
-#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <list>
 #include <memory>
 #include <mutex>
 #include <tuple>
+#include <utility>
 #include <vector>
 
+#include "report_slots.h"
 #include "tmq.h"
 
 namespace {
@@ -126,78 +127,66 @@ at::Tensor channels_last(const at::Tensor& act) {
 }
 
 // What a kernel reports to the host before it ends (tmq_host_report): slots in one page of
-// pinned memory, each held by one call at a time, so that threads and streams do not share
-// one.  A call waits by reading its slot, not for the stream: work queued behind the
+// pinned memory, each held by one call at a time (report_slots.h), so that threads and streams do
+// not share one.  A call waits by reading its slot, not for the stream: work queued behind the
 // reporting block goes on meanwhile.
 class HostReport {
  public:
-  HostReport() {
-    Pool& p = pool();
-    std::unique_lock<std::mutex> lock(p.mu);
-    p.given_back.wait(lock, [&] { return !p.free.empty(); });
-    slot_ = p.free.back();
-    p.free.pop_back();
-    if (++p.ticket == 0) ++p.ticket;  // (fresh memory is zero)
-    ticket_ = p.ticket;
+  HostReport(const c10::hip::HIPStream& stream, const char* what) : stream_(stream), what_(what), hold_(pool().slots) {
+    TORCH_CHECK(hold_.slot() >= 0, what_, ": every report slot was lost to a failed call");
+    slot_ = reinterpret_cast<tmq_host_report*>(static_cast<char*>(pool().page) + hold_.slot() * kStride);
   }
-  ~HostReport() {
-    if (pending_) return;  // the device may still write to it: not handed out again
-    Pool& p = pool();
-    {
-      std::lock_guard<std::mutex> lock(p.mu);
-      p.free.push_back(slot_);
-    }
-    p.given_back.notify_one();
-  }
-  HostReport(const HostReport&) = delete;
-  HostReport& operator=(const HostReport&) = delete;
 
   tmq_host_report* memory() { return slot_; }
-  uint32_t number() const {
-    return static_cast<uint32_t>((reinterpret_cast<char*>(slot_) - static_cast<char*>(pool().page)) / kStride);
+  uint32_t number() const { return static_cast<uint32_t>(hold_.slot()); }
+  uint32_t ticket() const { return hold_.ticket(); }
+  // Queues the kernels that write to the slot: `call` returns the library's status.
+  template <class Call>
+  void queue(Call&& call) {
+    check_status(hold_.queue(std::forward<Call>(call),
+                             [&] {
+                               const bool idle = hipStreamSynchronize(stream_.stream()) == hipSuccess;
+                               (void)hipGetLastError();
+                               return idle;
+                             }),
+                 what_);
   }
-  uint32_t ticket() const { return ticket_; }
-  void queued() { pending_ = true; }  // a kernel that will write to the slot is on its stream
   // Payload of word `i`.
-  uint32_t wait(int i, const c10::hip::HIPStream& stream, const char* what) {
+  uint32_t wait(int i) {
     const volatile uint64_t* word = &slot_->word[i];
     for (int spin = 0; spin < kSpins; ++spin) {
       const uint64_t v = *word;
-      if (static_cast<uint32_t>(v >> 32) == ticket_) return static_cast<uint32_t>(v);
+      if (static_cast<uint32_t>(v >> 32) == ticket()) return static_cast<uint32_t>(v);
       __builtin_ia32_pause();
     }
-    stream.synchronize();  // a long queue ahead of the kernel (or an error, which this raises)
+    stream_.synchronize();  // a long queue ahead of the kernel (or an error, which this raises)
     const uint64_t v = *word;
-    TORCH_CHECK(static_cast<uint32_t>(v >> 32) == ticket_, what, ": the kernel ended without its report");
+    TORCH_CHECK(static_cast<uint32_t>(v >> 32) == ticket(), what_, ": the kernel ended without its report");
     return static_cast<uint32_t>(v);
   }
-  void done() { pending_ = false; }
+  void done() { hold_.done(); }
 
  private:
   static constexpr int kSlots = TMQ_HOST_REPORTS;  // calls that wait at the same time; more of them queue for a slot
   static constexpr int kSpins = 20000;  // about a millisecond
+  static constexpr size_t kStride = 64;  // a cache line each
   struct Pool {
-    std::mutex mu;
-    std::condition_variable given_back;
-    std::vector<tmq_host_report*> free;
-    uint32_t ticket = 0;
+    tmq::ReportSlots slots{kSlots};
     void* page = nullptr;
     Pool() {
       TORCH_CHECK(hipHostMalloc(&page, kSlots * kStride, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess,
                   "hipHostMalloc failed");
       std::memset(page, 0, kSlots * kStride);
-      for (int i = 0; i < kSlots; ++i)
-        free.push_back(reinterpret_cast<tmq_host_report*>(static_cast<char*>(page) + i * kStride));
     }
   };
-  static constexpr size_t kStride = 64;  // a cache line each
   static Pool& pool() {
     static Pool* p = new Pool;  // for the life of the process: kernels may hold its address at exit
     return *p;
   }
+  const c10::hip::HIPStream stream_;
+  const char* const what_;
+  tmq::ReportHold hold_;
   tmq_host_report* slot_;
-  uint32_t ticket_;
-  bool pending_ = false;
 };
 
 bool stream_is_capturing(const c10::hip::HIPStream& s) {
@@ -285,7 +274,7 @@ void convert_per_channel(const at::Tensor& codes, const at::Tensor& fp32, const 
     return;
   }
   const auto stream = stream_for_report(codes, what);
-  HostReport report;
+  HostReport report(stream, what);
   tmq_per_channel_desc d{};
   d.dequantize = dequantize;
   d.float_qparams = float_qparams;
@@ -299,9 +288,8 @@ void convert_per_channel(const at::Tensor& codes, const at::Tensor& fp32, const 
   d.scales = sc.const_data_ptr();
   d.zero_points = zp.const_data_ptr();
   d.report = report.memory();
-  check_status(tmq_per_channel(&d, reinterpret_cast<tmq_stream_t>(stream.stream())), "tmq_per_channel");
-  report.queued();
-  const bool bad = report.wait(0, stream, what) != 0;
+  report.queue([&] { return tmq_per_channel(&d, reinterpret_cast<tmq_stream_t>(stream.stream())); });
+  const bool bad = report.wait(0) != 0;
   report.done();
   TORCH_CHECK(!bad, "per-channel zero point outside the range of the quantized dtype");
 }
@@ -398,14 +386,14 @@ at::Tensor quantize_per_tensor_dynamic(const at::Tensor& self, at::ScalarType dt
   const int64_t range_bytes = static_cast<int64_t>(tmq_minmax_workspace_bytes(x.numel()));
   const at::Tensor scratch = empty_bytes(range_bytes + static_cast<int64_t>(sizeof(tmq_qparams)), x);
   auto* ws = static_cast<uint8_t*>(scratch.data_ptr());
-  HostReport report;
-  check_status(tmq_quantize_per_tensor_dynamic_report(
-                   cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
-                   reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes),
-                   report.memory(), report.ticket(), report.number(), reinterpret_cast<tmq_stream_t>(stream.stream())),
-               "tmq_quantize_per_tensor_dynamic_report");
-  report.queued();
-  const uint32_t lo = report.wait(0, stream, what), hi = report.wait(1, stream, what);
+  HostReport report(stream, what);
+  report.queue([&] {
+    return tmq_quantize_per_tensor_dynamic_report(
+        cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
+        reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes), report.memory(),
+        report.ticket(), report.number(), reinterpret_cast<tmq_stream_t>(stream.stream()));
+  });
+  const uint32_t lo = report.wait(0), hi = report.wait(1);
   report.done();
   float mn, mx;
   std::memcpy(&mn, &lo, 4);
