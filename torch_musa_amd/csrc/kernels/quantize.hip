@@ -347,6 +347,9 @@ __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
   }
   __syncthreads();
   if (!s_last) return;
+  // The other blocks' pairs are read behind the count that says they are there.  (Acquire: this wave's later
+  // loads are issued after it and find no older copy in a cache; nothing is written back.)
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   mn = std::numeric_limits<float>::infinity();
   mx = -std::numeric_limits<float>::infinity();
   for (unsigned i = threadIdx.x; i < gridDim.x; i += kThreads) {
