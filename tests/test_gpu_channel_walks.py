@@ -50,6 +50,24 @@ def test_dynamic_range_report(n):
         torch.quantize_per_tensor_dynamic(torch.full((n,), float("nan"), device="cuda"), torch.quint8, False)
 
 
+@pytest.mark.parametrize("n,offset", [
+    (98305, 0), (1 << 21, 0),                                           # reported by the range pass
+    ((1 << 21) + 4, 0), ((1 << 21) + 7, 0), ((1 << 24) + 1, 0), (1 << 25, 0),  # by the quantizer's first block
+    (98305, 1), ((1 << 21) + 6, 1),                                     # values off the 16-byte grid: by the pass between
+])
+@pytest.mark.parametrize("dtype", [torch.quint8, torch.qint8])
+def test_dynamic_range_report_by_each_pass(n, offset, dtype):
+    x = torch.randn(n, generator=torch.Generator().manual_seed(n)) * 2
+    x[n - 1], x[n // 2] = 31.0, -47.0    # the range's ends: the last value and one in the middle
+    xg = torch.empty(n + offset, device="cuda")[offset:].copy_(x.cuda())
+    want = torch.quantize_per_tensor_dynamic(x, dtype, False)
+    got = torch.quantize_per_tensor_dynamic(xg, dtype, False)
+    assert got.q_scale() == want.q_scale() and got.q_zero_point() == want.q_zero_point()
+    assert torch.equal(got.int_repr().cpu(), want.int_repr())
+    with pytest.raises(RuntimeError, match="min should be"):
+        torch.quantize_per_tensor_dynamic(xg.fill_(float("nan")), dtype, False)
+
+
 def test_dynamic_keeps_the_memory_format():
     x = torch.randn(2, 5, 6, 7).contiguous(memory_format=torch.channels_last)
     got = torch.quantize_per_tensor_dynamic(x.cuda(), torch.qint8, True)
