@@ -931,7 +931,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   }
   const bool mfma_ok = s.ICg % 16 == 0 && aligned(d->x, 16);
   if ((forced == 1 || forced == 2) && !mfma_ok) return TMQ_ERR_UNSUPPORTED;
-  // pointwise layers over few input channels: pixels straight from memory against weights in LDS
+  // pointwise layers over few input channels: pixels straight from memory against weights in registers
   {
     const bool rows_ok = pointwise_rows_ok(d->geom, s) && (MODE != kOutAcc32 || aligned(out, 4));
     if (forced == 9 && !rows_ok) return TMQ_ERR_UNSUPPORTED;

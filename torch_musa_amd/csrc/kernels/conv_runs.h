@@ -415,10 +415,13 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
 // requantisation constants of the lane's 4 NT channels in registers, and walks every G-th 16-pixel
 // piece of the image, D pieces' bytes (input and residual) on their way: a load per k-step, the MFMAs,
 // eight vector instructions per value and one store, no LDS and no barrier behind the set-up.  The waves
-// of neighbouring channel blocks read the same pieces at the same time, from one L1.  What bounds it is the
-// requantisation, then memory: 64 -> 256 channels with a residual on 56 x 56 at batch 32 (58 MB) takes
-// 14.4 us; with the weights and constants in LDS and every channel block over a piece in turn, the LDS
-// reads were a third of its instructions and the residual a latency per block: 27.9 us.
+// of neighbouring channel blocks read the same pieces at the same time, from one L1.  With few k-steps the
+// requantisation bounds it: 64 -> 256 channels with a residual on 56 x 56 at batch 32 (58 MB) takes 14.2 us, each of a
+// SIMD's three waves issuing vector instructions in 27 % of its cycles; with the weights and constants in LDS and
+// every channel block over a piece in turn, the LDS reads were a third of its instructions and the residual a
+// latency per block: 27.9 us.  With four k-steps and one channel block the loads' latency does: 256 -> 64 on the
+// same image (32 MB) takes 9.8 us, its two waves a SIMD wait in 49 % of their cycles and issue vector instructions in
+// 15 % (four pieces ahead instead of two: 9.3 against 8.9 us, no gain).
 // a.tiles: the number of 16-pixel pieces.
 template <int KSN>
 constexpr int kCrPointwiseDepth = KSN == 1 ? 4 : 2;

@@ -13,7 +13,9 @@
 // A call that is not of the plain form -- keywords, another number of arguments,
 // tensor subclasses, a torch-function mode, tracing, stand-in objects of the export
 // machinery, numbers of other types -- goes to PyTorch's own callable, which is kept
-// as `self` of the function, and has its results and its errors.
+// as `self` of the function, and has its results and its errors.  Some of PyTorch's modules
+// are among those: quantized.dynamic.Linear passes reduce_range by name, QFunctional.add its
+// scale and zero point.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
