@@ -343,13 +343,14 @@ __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("" ::"v"(before) : "memory");  // (waits for the answer)
     const unsigned int last = gridDim.x - 1;
-    s_last = atomicInc(&g_range_arrivals[report.slot], last) == last;
+    const bool is_last = atomicInc(&g_range_arrivals[report.slot], last) == last;
+    // The other blocks' pairs are read behind the count that says they are there: the barrier hands this
+    // acquire on to the block's other waves.  (Later loads find no older copy in a cache; nothing is written back.)
+    if (is_last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    s_last = is_last;
   }
   __syncthreads();
   if (!s_last) return;
-  // The other blocks' pairs are read behind the count that says they are there.  (Acquire: this wave's later
-  // loads are issued after it and find no older copy in a cache; nothing is written back.)
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   mn = std::numeric_limits<float>::infinity();
   mx = -std::numeric_limits<float>::infinity();
   for (unsigned i = threadIdx.x; i < gridDim.x; i += kThreads) {
