@@ -121,7 +121,8 @@ int tmq_quantize_per_tensor_dynamic_dev(const float* x, void* q, int64_t n, int 
 /* What a kernel tells the host before it ends: pinned host memory that the device
  * can write (hipHostMalloc), 16-byte aligned.  A word is complete once its upper
  * half is the ticket of the call -- any number that differs from the one this
- * memory was last used with. */
+ * memory was last used with.  A call that fails may have queued kernels that still
+ * write to it: wait for the stream before the memory or its slot is used again. */
 typedef struct tmq_host_report {
   uint64_t word[2];
 } tmq_host_report;
@@ -139,7 +140,7 @@ int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, i
 /* The same for M rows of K values -> rows of `pitch` codes, pitch a multiple of
  * 16 that is at least K: what tmq_linear wants of activations whose K is not.
  * The codes behind a row's end are undefined (the packed weights are zero there).
- * Two launches; `workspace` 8-byte aligned. */
+ * One launch up to 98304 values, else two; `workspace` 8-byte aligned. */
 int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
                                   int reduce_range, int rounding, tmq_qparams* qparams,
                                   void* workspace, size_t workspace_bytes, tmq_stream_t stream);

@@ -420,7 +420,7 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
 // SIMD's three waves issuing vector instructions in 27 % of its cycles; with the weights and constants in LDS and
 // every channel block over a piece in turn, the LDS reads were a third of its instructions and the residual a
 // latency per block: 27.9 us.  With four k-steps and one channel block the loads' latency does: 256 -> 64 on the
-// same image (32 MB) takes 9.8 us, its two waves a SIMD wait in 49 % of their cycles and issue vector instructions in
+// same image (32 MB) takes 10.0 us, its two waves a SIMD wait in 49 % of their cycles and issue vector instructions in
 // 15 % (four pieces ahead instead of two: 9.3 against 8.9 us, no gain).
 // a.tiles: the number of 16-pixel pieces.
 template <int KSN>
