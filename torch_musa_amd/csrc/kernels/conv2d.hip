@@ -666,6 +666,15 @@ bool pointwise_rows_ok(const tmq_conv2d_geom& g, const ConvShape& s) {
 // its 64 channels.
 bool pointwise_rows_first(const ConvShape& s, bool post) { return post || s.runs_KS <= 2 || s.OC <= 160; }
 
+// The 16-pixel pieces whose reads and stores the kernel makes without a check: all 16 pixels exist, and the last pixel's
+// 16-byte reads (to RP >= IC bytes behind its first) end inside the tensor.  None where a lane's residual bytes are more
+// than a pixel has.
+int64_t pointwise_whole_pieces(int64_t pixels, int64_t IC, int64_t RP, bool short_residual) {
+  const int64_t last = pixels * IC - RP - 15 * IC;  // first byte of the last piece that may be read so
+  if (short_residual || last < 0) return 0;
+  return std::min(pixels / 16, last / (16 * IC) + 1);
+}
+
 template <int MODE>
 int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, const PostOps& po, float zp_f, float lo_f,
                                float hi_f, void* out, hipStream_t stream) {
@@ -693,11 +702,16 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.zp_f = zp_f; a.lo_f = lo_f; a.hi_f = hi_f;
   a.post = po;
   const int nt = conv_runs_tiles(s.OC);
+  a.whole = static_cast<int32_t>(pointwise_whole_pieces(s.B * s.H * s.W, s.IC, s.runs_RP, po.accum != nullptr && s.OC < 4 * nt));
   // one wave per channel block and run of pieces, as many as the chip holds at once (their registers), but at least
   // one per channel block
   const int64_t nblk = ceil_div(s.OC, 16 * nt), cap = 256 * (s.runs_KS > 2 ? 2 : 3) * kCrWaves;
   int64_t groups = cap / nblk < 1 ? 1 : cap / nblk;
   if (groups > pieces) groups = pieces;
+  a.nblk = static_cast<int>(nblk);
+  a.groups = static_cast<int>(groups);
+  // (exact while waves x nblk < 2**32: at most 3072 waves, or nblk <= 2048 of them)
+  a.nblk_magic = static_cast<uint32_t>(((int64_t{1} << 32) + nblk - 1) / nblk);
   const dim3 grid(static_cast<unsigned>(ceil_div(groups * nblk, kCrWaves))), block(kCrThreads);
   const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
     constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;

@@ -55,6 +55,9 @@ struct ConvRunArgs {
   int rows_in, pitch;        // staged image rows, LDS bytes per staged row (multiple of 16)
   int tiles_h, tiles_w;
   int vec;                   // 16-byte (int32 mode: per 4 channels) stores are aligned
+  int whole;                 // (pointwise) pieces all of whose reads and stores lie inside the tensors
+  int nblk, groups;          // (pointwise) channel blocks, and waves on each of them
+  uint32_t nblk_magic;       // w / nblk = (w * nblk_magic) >> 32 for the waves w of the launch (nblk > 1)
   int32_t w_scale_stride;
   uint32_t x_xor, pad_word;  // pad_word: the activation zero point in 4 bytes, before the xor
   int32_t acc_coef;
@@ -132,66 +135,72 @@ __device__ __forceinline__ RunsResidual<NT> runs_residual(const ConvRunArgs& a, 
   }
   return r;
 }
+template <int MODE, int POST, int NT, bool PLAIN>
+__device__ __forceinline__ void runs_requant(const ConvRunArgs& a, const v4i (&acc)[NT], const float* mult_cb,
+                                             const float* bdiv_cb, float bmul, const RunsResidual<NT>& accw,
+                                             uint32_t (&packed)[NT]) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int raw[4] = {acc[nt][0], acc[nt][1], acc[nt][2], acc[nt][3]};
+    const v4f mult = {mult_cb[4 * nt], mult_cb[4 * nt + 1], mult_cb[4 * nt + 2], mult_cb[4 * nt + 3]};
+    const v4f bdiv = {bdiv_cb[4 * nt], bdiv_cb[4 * nt + 1], bdiv_cb[4 * nt + 2], bdiv_cb[4 * nt + 3]};
+    if constexpr (POST != 0) {
+      packed[nt] = requant4_post<MODE, POST, PLAIN>(raw, bdiv, bmul, mult, a.post, accw.w[nt], a.zp_f, a.lo_f, a.hi_f);
+    } else {
+      packed[nt] = requant4<MODE, true, PLAIN ? 1 : 0>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
+    }
+  }
+}
+// One store of a lane's 4 NT bytes, at any alignment (the same instruction as an aligned one).
+template <int NT>
+__device__ __forceinline__ void runs_store(uint8_t* dst, const uint32_t (&packed)[NT]) {
+  if constexpr (NT == 4) {
+    st16_any(dst, v4i{static_cast<int>(packed[0]), static_cast<int>(packed[1]), static_cast<int>(packed[2]),
+                      static_cast<int>(packed[3])});
+  } else {
+    static_assert(NT == 2, "channel tiles per block: 2 or 4");
+    st8_any(dst, v2i{static_cast<int>(packed[0]), static_cast<int>(packed[1])});
+  }
+}
+// A lane at the end of the channels, `left` of whose 4 NT exist: a word where four do, else bytes.
+template <int NT>
+__device__ __forceinline__ void runs_store_some(uint8_t* dst, const uint32_t (&packed)[NT], int left) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt, left -= 4) {
+    if (left >= 4) {
+      reinterpret_cast<U32AnyAlignment*>(dst + 4 * nt)->v = packed[nt];
+    } else if (left > 0) {
+      dst[4 * nt] = static_cast<uint8_t>(packed[nt]);
+      if (left > 1) dst[4 * nt + 1] = static_cast<uint8_t>(packed[nt] >> 8);
+      if (left > 2) dst[4 * nt + 2] = static_cast<uint8_t>(packed[nt] >> 16);
+    }
+  }
+}
 template <int MODE, int POST, int NT, bool PLAIN = false>
 __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v4i (&acc)[NT], int64_t off, int cb,
                                                    const float* mult_cb, const float* bdiv_cb, float bmul,
                                                    const RunsResidual<NT>& accw) {
   constexpr int kLaneCh = 4 * NT;
-  uint32_t packed[NT];
+  if constexpr (MODE == kOutAcc32) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int raw[4] = {acc[nt][0], acc[nt][1], acc[nt][2], acc[nt][3]};
-    if constexpr (MODE == kOutAcc32) {
+    for (int nt = 0; nt < NT; ++nt) {
       int32_t* const dst = static_cast<int32_t*>(a.y) + off + 4 * nt;
       if (a.vec && cb + 4 * nt + 4 <= a.OC) {
-        *reinterpret_cast<v4i*>(dst) = v4i{raw[0], raw[1], raw[2], raw[3]};
+        *reinterpret_cast<v4i*>(dst) = acc[nt];
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (cb + 4 * nt + r < a.OC) dst[r] = raw[r];
-      }
-    } else {
-      const v4f mult = {mult_cb[4 * nt], mult_cb[4 * nt + 1], mult_cb[4 * nt + 2], mult_cb[4 * nt + 3]};
-      const v4f bdiv = {bdiv_cb[4 * nt], bdiv_cb[4 * nt + 1], bdiv_cb[4 * nt + 2], bdiv_cb[4 * nt + 3]};
-      if constexpr (POST != 0) {
-        packed[nt] = requant4_post<MODE, POST, PLAIN>(raw, bdiv, bmul, mult, a.post, accw.w[nt], a.zp_f, a.lo_f, a.hi_f);
-      } else {
-        packed[nt] = requant4<MODE, true, PLAIN ? 1 : 0>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
+          if (cb + 4 * nt + r < a.OC) dst[r] = acc[nt][r];
       }
     }
-  }
-  if constexpr (MODE != kOutAcc32) {
+  } else {
+    uint32_t packed[NT];
+    runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult_cb, bdiv_cb, bmul, accw, packed);
     uint8_t* const dst = static_cast<uint8_t*>(a.y) + off;
-    if (cb + kLaneCh <= a.OC) {  // one store of 4 NT bytes; any alignment unless the host found the rows aligned
-      if constexpr (NT == 4) {
-        const v4i all = {static_cast<int>(packed[0]), static_cast<int>(packed[1]), static_cast<int>(packed[2]),
-                         static_cast<int>(packed[3])};
-        if (a.vec)
-          *reinterpret_cast<v4i*>(dst) = all;
-        else
-          st16_any(dst, all);
-      } else {
-        static_assert(NT == 2, "channel tiles per block: 2 or 4");
-        const v2i all = {static_cast<int>(packed[0]), static_cast<int>(packed[1])};
-        if (a.vec)
-          *reinterpret_cast<v2i*>(dst) = all;
-        else
-          st8_any(dst, all);
-      }
-    } else {
-      // a lane at the end of the channels: a word where four exist, else bytes
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int left = a.OC - (cb + 4 * nt);
-        if (left >= 4) {
-          reinterpret_cast<U32AnyAlignment*>(dst + 4 * nt)->v = packed[nt];
-        } else if (left > 0) {
-          dst[4 * nt] = static_cast<uint8_t>(packed[nt]);
-          if (left > 1) dst[4 * nt + 1] = static_cast<uint8_t>(packed[nt] >> 8);
-          if (left > 2) dst[4 * nt + 2] = static_cast<uint8_t>(packed[nt] >> 16);
-        }
-      }
-    }
+    if (cb + kLaneCh <= a.OC)
+      runs_store<NT>(dst, packed);
+    else
+      runs_store_some<NT>(dst, packed, a.OC - cb);
   }
 }
 
@@ -414,14 +423,20 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
 // A wave owns one channel block for the whole launch, its weights (NT x KSN operands) and the
 // requantisation constants of the lane's 4 NT channels in registers, and walks every G-th 16-pixel
 // piece of the image, D pieces' bytes (input and residual) on their way: a load per k-step, the MFMAs,
-// eight vector instructions per value and one store, no LDS and no barrier behind the set-up.  The waves
-// of neighbouring channel blocks read the same pieces at the same time, from one L1.  With few k-steps the
-// requantisation bounds it: 64 -> 256 channels with a residual on 56 x 56 at batch 32 (58 MB) takes 14.2 us, each of a
-// SIMD's three waves issuing vector instructions in 27 % of its cycles; with the weights and constants in LDS and
-// every channel block over a piece in turn, the LDS reads were a third of its instructions and the residual a
-// latency per block: 27.9 us.  With four k-steps and one channel block the loads' latency does: 256 -> 64 on the
-// same image (32 MB) takes 10.0 us, its two waves a SIMD wait in 49 % of their cycles and issue vector instructions in
-// 15 % (four pieces ahead instead of two: 9.3 against 8.9 us, no gain).
+// eight vector instructions per value (four without a residual) and one store, no LDS and no barrier.  The waves
+// of neighbouring channel blocks read the same pieces at the same time, from one L1.  With the weights and constants in
+// LDS and every channel block over a piece in turn, the LDS reads were a third of its instructions and the residual a
+// latency per block (64 -> 256 channels with a residual on 56 x 56 at batch 32, 58 MB: 27.9 us).
+//
+// A launch has a handful of pieces per wave, so what bounds it is a wave's chain: arguments, set-up, first bytes, then
+// pieces whose loads, products and stores follow one another.  Hence all requests of the set-up leave together, the
+// constants first and each wave's its own (the bias used to be asked for after the scales had come, and the block met
+// at a barrier), the wave's place in the grid is a multiplication, not a division, and a piece that lies inside the
+// tensors takes its addresses from the scalar unit and keeps an exact count of the requests on their way.  us, before |
+// after: the layer above 15.2 | 13.7, 256 -> 64 on the same image (32 MB) 9.6 | 8.0, 24 -> 144 there 10.2 | 9.5 and on
+// one image of 57 x 43 4.0 | 3.2, 16 -> 96 on 112 x 112 at batch 32 18.0 | 15.3, 512 channels with a residual from 128
+// on 28 x 28 at batch 8 7.2 | 6.2.
+// (256 -> 64 with four pieces ahead instead of two: 9.3 against 8.9 us.)
 // a.tiles: the number of 16-pixel pieces.
 template <int KSN>
 constexpr int kCrPointwiseDepth = KSN == 1 ? 4 : 2;
@@ -431,7 +446,7 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
   constexpr int kCrBN = 16 * NT;   // output channels per channel block
   constexpr int kLaneCh = 4 * NT;  // consecutive channels of one pixel in a lane
   constexpr int D = kCrPointwiseDepth<KSN>;
-  // constants of the channels of this block's waves: at most four channel blocks
+  // constants of the channels of this block's waves, each wave its own
   __shared__ __attribute__((aligned(16))) int s_acc0[kCrWaves * kCrBN];
   __shared__ __attribute__((aligned(16))) float s_mult[kCrWaves * kCrBN];
   __shared__ __attribute__((aligned(16))) float s_bdiv[kCrWaves * kCrBN];
@@ -439,32 +454,61 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int pj = lane & 15, pq = lane >> 4;
   const int KS = a.KS;
-  const int nblk = (a.OC + kCrBN - 1) / kCrBN;
-  const int groups = static_cast<int>(gridDim.x) * kCrWaves / nblk;  // waves on one channel block
-  const int w = static_cast<int>(blockIdx.x) * kCrWaves + wave;
-  const int g = w / nblk, cb = w - g * nblk;
+  const int nblk = a.nblk, groups = a.groups;
+  const uint32_t w = blockIdx.x * kCrWaves + static_cast<uint32_t>(wave);
+  const int g = static_cast<int>(nblk == 1 ? w : __umulhi(w, a.nblk_magic));
+  const int cb = static_cast<int>(w) - g * nblk;
+  if (g >= groups || g >= a.tiles) return;  // (no barrier below: the waves share nothing)
+
+  // Every request of the set-up leaves before anything is waited for, the constants first: with the bias behind a
+  // branch of its own its latency (cold: most of a microsecond) came on top of the scales'.
+  const int ci = lane % kCrBN;
+  const int cn = cb * kCrBN + ci < a.OC ? cb * kCrBN + ci : 0;
+  const int c_cs = a.colsum[cn];
+  float c_ws = 1.f, c_b = 0.f;
+  if constexpr (MODE != kOutAcc32) {
+    c_ws = a.w_scales[cn * a.w_scale_stride];
+    const float* const bsrc = a.bias != nullptr ? a.bias : a.w_scales;  // a load that always has an address
+    c_b = bsrc[a.bias != nullptr ? cn : 0];
+  }
   const int npix = a.B * a.H * a.W;
   const int64_t x_bytes = static_cast<int64_t>(npix) * a.IC;
-  const bool works = g < groups && g < a.tiles;  // (the same for the whole wave)
-
-  // this lane's 16 bytes of every k-step for the pixel pj of a piece; a pixel or bytes that do not exist: any
-  // others (nothing of them is stored, or their weights are zero)
-  const auto fetch = [&](int piece, v4i (&xv)[KSN]) {
-    const int pix = piece * 16 + pj < npix ? piece * 16 + pj : npix - 1;
-    const int64_t row = static_cast<int64_t>(pix) * a.IC;
-#pragma unroll
-    for (int ks = 0; ks < KSN; ++ks) {
-      const int k0 = ks * 64 + pq * 16;
-      const TailRead r = tail_read16(row + (k0 < a.RP ? k0 : 0), x_bytes);  // (the host: a tensor of at least 16 bytes)
-      xv[ks] = ld16_any(a.x + r.at);
-      if (r.shift > 0) xv[ks] = shift_down_bytes(xv[ks], r.shift);  // the tensor's last few bytes
-    }
-  };
+  // A piece all of whose bytes exist (the first a.whole ones): addresses are the piece's, the same for the whole wave,
+  // plus an offset of the lane that never changes, so that a piece costs no vector instruction for them.
   const bool residual = POST == 1 || (POST == 2 && a.post.accum != nullptr);
   const int cl = cb * kCrBN + kLaneCh * pq;  // this lane's first channel
-  const auto fetch_residual = [&](int piece, RunsResidual<NT>& r) {
-    const int pix = piece * 16 + pj;
-    if (residual && pix < npix && cl < a.OC) r = runs_residual<NT>(a, static_cast<int64_t>(pix) * a.OC + cl, cl);
+  const bool all_ch = (cb + 1) * kCrBN <= a.OC;  // every lane of the wave has its 4 NT channels
+  const uint32_t yo = static_cast<uint32_t>(pj * a.OC + cl);
+  // (a lane at the end of the channels reads its residual bytes as the pixel's last 4 NT and shifts them down)
+  const int over = cl + kLaneCh - a.OC;
+  const uint32_t ro = yo - static_cast<uint32_t>(over > 0 && over < kLaneCh ? over : over > 0 ? cl : 0);
+  uint32_t xo[KSN];
+#pragma unroll
+  for (int ks = 0; ks < KSN; ++ks) {
+    const int k0 = ks * 64 + pq * 16;
+    xo[ks] = static_cast<uint32_t>(pj * a.IC + (k0 < a.RP ? k0 : 0));
+  }
+  // Piece number i of this wave.  A number past the last asks for the first piece's first bytes instead, the same for all
+  // lanes: the count of requests on their way stays exact, which one under a condition would end (the compiler then
+  // waits for all of them), and it costs next to nothing.
+  const int mine = g < a.whole ? (a.whole - g + groups - 1) / groups : 0;  // whole pieces of this wave
+  const auto fetch = [&](int i, v4i (&xv)[KSN], RunsResidual<NT>& r) {
+    const int64_t first = i < mine ? (g + i * groups) * int64_t{16} : 0;
+    const uint32_t keep = i < mine ? ~0u : 0u;
+    const uint8_t* const src = a.x + first * a.IC;
+#pragma unroll
+    for (int ks = 0; ks < KSN; ++ks) xv[ks] = ld16_any(src + (xo[ks] & keep));
+    if (!residual) return;
+    const uint8_t* const rsrc = a.post.accum + first * a.OC + (ro & keep);
+    if constexpr (NT == 4) {
+      const v4i v = ld16_any(rsrc);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) r.w[nt] = static_cast<uint32_t>(v[nt]);
+    } else {
+      const v2i v = reinterpret_cast<const V2iAnyAlignment*>(rsrc)->v;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) r.w[nt] = static_cast<uint32_t>(v[nt]);
+    }
   };
   // the first pieces' bytes and the weights are asked for before the constants are set up
   v4i xr[D][KSN];
@@ -475,40 +519,32 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
 #pragma unroll
     for (int ks = 0; ks < KSN; ++ks) xr[i][ks] = v4i{0, 0, 0, 0};
     rr[i] = RunsResidual<NT>{};
-    if (works && g + i * groups < a.tiles) {
-      fetch(g + i * groups, xr[i]);
-      fetch_residual(g + i * groups, rr[i]);
-    }
+  }
+  if (mine > 0) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) fetch(i, xr[i], rr[i]);
   }
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int ks = 0; ks < KSN; ++ks)
-      wreg[nt][ks] = works && ks < KS ? ld16(a.w_runs + ((static_cast<int64_t>(cb) * NT + nt) * KS + ks) * (kWave * 16) + lane * 16)
+      wreg[nt][ks] = ks < KS ? ld16(a.w_runs + ((static_cast<int64_t>(cb) * NT + nt) * KS + ks) * (kWave * 16) + lane * 16)
                                       : v4i{0, 0, 0, 0};
-  // the constants of the block's four waves' channels, a channel per thread (two IEEE divisions each; in registers
-  // of every lane they would be 32 per lane)
-  for (int i = t; i < kCrWaves * kCrBN; i += kCrThreads) {
-    const int wv = static_cast<int>(blockIdx.x) * kCrWaves + i / kCrBN;
-    const int n = (wv % nblk) * kCrBN + i % kCrBN;
-    int acc0 = 0;
-    float mult = 0.f, bdiv = 0.f;
-    if (n < a.OC) {
-      acc0 = a.acc_coef * a.colsum[n];
-      if constexpr (MODE != kOutAcc32) {
-        const float atw = a.x_scale * a.w_scales[n * a.w_scale_stride];
-        mult = atw / a.out_scale;
-        bdiv = a.bias != nullptr ? bias_term(a.w_scale_stride == 0, a.bias[n], atw) : 0.f;
-      }
-    }
-    s_acc0[i] = acc0;
-    s_mult[i] = mult;
-    s_bdiv[i] = bdiv;
-  }
-  __syncthreads();
-  if (!works) return;
+  // the wave's constants, a channel per lane (two IEEE divisions each), then to the lanes that want them
   float bmul = 1.0f;
-  if constexpr (MODE != kOutAcc32) bmul = bias_mul(a.w_scale_stride == 0, a.x_scale * a.w_scales[0]);
+  {
+    float mult = 0.f, bdiv = 0.f;
+    if constexpr (MODE != kOutAcc32) {
+      const float atw = a.x_scale * c_ws;
+      mult = atw / a.out_scale;
+      bdiv = a.bias != nullptr ? bias_term(a.w_scale_stride == 0, c_b, atw) : 0.f;
+      bmul = bias_mul(a.w_scale_stride == 0, atw);  // (per tensor: the same for every channel)
+    }
+    s_acc0[wave * kCrBN + ci] = a.acc_coef * c_cs;
+    s_mult[wave * kCrBN + ci] = mult;
+    s_bdiv[wave * kCrBN + ci] = bdiv;
+    wave_sync_lds();
+  }
   v4i acc0[NT];
   float mult[kLaneCh], bdiv[kLaneCh];
 #pragma unroll
@@ -522,32 +558,81 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
       bdiv[4 * nt + r] = b[r];
     }
   }
-  const int xo = static_cast<int>(a.x_xor);
-  const v4i flip = {xo, xo, xo, xo};
-  for (int piece = g; piece < a.tiles;) {
+  const int flip_word = static_cast<int>(a.x_xor);
+  const v4i flip = {flip_word, flip_word, flip_word, flip_word};
+  const auto multiply = [&](const v4i (&xv)[KSN], v4i (&acc)[NT]) {
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      if (piece < a.tiles) {
-        v4i acc[NT];
+    for (int ks = 0; ks < KSN; ++ks) {
+      const v4i xf = xv[ks] ^ flip;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[nt] = acc0[nt];
+      for (int nt = 0; nt < NT; ++nt)
+        acc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[nt][ks], xf, ks == 0 ? acc0[nt] : acc[nt], 0, 0, 0);
+    }
+  };
+  const auto whole_piece = [&](int i, int n, auto all_ch_tag) {
+    v4i acc[NT];
+    multiply(xr[i], acc);
+    RunsResidual<NT> accw = rr[i];
+    fetch(n + D, xr[i], rr[i]);
+    const int64_t base = static_cast<int64_t>(g + n * groups) * (16 * a.OC);
+    if constexpr (MODE == kOutAcc32) {
+      if (cl < a.OC) runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, base + yo, cl, mult, bdiv, bmul, accw);
+    } else {
+      uint32_t packed[NT];
+      uint8_t* const dst = static_cast<uint8_t*>(a.y) + base;
+      if constexpr (decltype(all_ch_tag)::value) {
+        runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
+        runs_store<NT>(dst + yo, packed);
+      } else {
+        if (residual && over > 0 && over < kLaneCh) {
+          v4i v = {0, 0, 0, 0};
 #pragma unroll
-        for (int ks = 0; ks < KSN; ++ks) {
-          const v4i xv = xr[i][ks] ^ flip;
+          for (int nt = 0; nt < NT; ++nt) v[nt] = static_cast<int>(accw.w[nt]);
+          v = shift_down_bytes(v, over);
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            acc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[nt][ks], xv, acc[nt], 0, 0, 0);
+          for (int nt = 0; nt < NT; ++nt) accw.w[nt] = static_cast<uint32_t>(v[nt]);
         }
-        const RunsResidual<NT> accw = rr[i];
-        if (piece + D * groups < a.tiles) {
-          fetch(piece + D * groups, xr[i]);
-          fetch_residual(piece + D * groups, rr[i]);
-        }
-        const int pix = piece * 16 + pj;
-        if (pix < npix && cl < a.OC)
-          runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, static_cast<int64_t>(pix) * a.OC + cl, cl, mult, bdiv, bmul, accw);
-        piece += groups;
+        runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
+        if (over <= 0)
+          runs_store<NT>(dst + yo, packed);
+        else if (over < kLaneCh)
+          runs_store_some<NT>(dst + yo, packed, kLaneCh - over);
       }
+    }
+  };
+  // (one copy of the D pieces, left at any of them: waves with a piece or two would pay for fetching a second one)
+  const auto walk = [&](auto all_ch_tag) {
+    for (int n = 0;; n += D) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        if (n + i >= mine) return;
+        whole_piece(i, n + i, all_ch_tag);
+      }
+    }
+  };
+  if (MODE != kOutAcc32 && all_ch)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
+  // what is left at the tensor's end (one piece or two of the launch): every address checked
+  for (int piece = g + mine * groups; piece < a.tiles; piece += groups) {
+    const int pix = piece * 16 + pj < npix ? piece * 16 + pj : npix - 1;
+    const int64_t row = static_cast<int64_t>(pix) * a.IC;
+    v4i xv[KSN], acc[NT];
+#pragma unroll
+    for (int ks = 0; ks < KSN; ++ks) {
+      // (a pixel or bytes that do not exist: any others -- nothing of them is stored, or their weights are zero)
+      const int k0 = ks * 64 + pq * 16;
+      const TailRead r = tail_read16(row + (k0 < a.RP ? k0 : 0), x_bytes);  // (the host: a tensor of at least 16 bytes)
+      xv[ks] = ld16_any(a.x + r.at);
+      if (r.shift > 0) xv[ks] = shift_down_bytes(xv[ks], r.shift);  // the tensor's last few bytes
+    }
+    multiply(xv, acc);
+    if (piece * 16 + pj < npix && cl < a.OC) {
+      const int64_t off = static_cast<int64_t>(pix) * a.OC + cl;
+      RunsResidual<NT> accw{};
+      if (residual) accw = runs_residual<NT>(a, off, cl);
+      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cl, mult, bdiv, bmul, accw);
     }
   }
 }

@@ -511,7 +511,7 @@ __device__ __forceinline__ uint32_t requant4_post(const int (&raw)[4], v4f bdiv,
   // per byte): a signed byte s equals (s ^ 0x80) - 128, so the word is flipped
   // once and 128 joins the zero point.  Both terms of the difference are small
   // integers, exact in fp32, so it equals float(q - zero_point).
-  const uint32_t accu = p.accum_signed ? accw ^ 0x80808080u : accw;
+  const uint32_t accu = accw ^ (p.accum_signed ? 0x80808080u : 0u);
   const float acc_zp_f = static_cast<float>(p.accum_zp + (p.accum_signed ? 128 : 0));
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
