@@ -98,6 +98,12 @@ constexpr int kDecodeMaxRows = 64;
 constexpr int kDecodeRowsAuto = 16;  // up to here the automatic choice always streams the weights
 // MG = groups of 16 activation rows (M <= 16 * MG): the weight operands are
 // loaded once and multiplied with every group.
+// ROWS = 4 (one group of at most four rows): a request for activations brings four k-blocks of the
+// wave at once, so that a batch holds 8 registers of them instead of 32 and six waves fit a SIMD
+// instead of five: 688 blocks (N = 11008) are then on the chip together instead of 512 and a rest
+// (us, rows one to four, 16-row requests | these: K = 4096, N = 11008 11.2 | 9.6, N = 12288 12.5 | 10.3;
+// K = 11008, N = 4096 9.8 | 9.1; K = 8192, N = 2048 6.9 | 6.0; K = 192, N = 8192 4.9 | 4.1; a kernel that only reads
+// 45 MB takes 7.5).  Requests of two k-blocks for eight rows gain nothing (9.8 | 9.9).
 //
 // The 14 dwords in front of GemmArgs are everything the kernel's loads need.  The
 // library is compiled with kernel-argument preloading, which hands up to 14
@@ -105,7 +111,8 @@ constexpr int kDecodeRowsAuto = 16;  // up to here the automatic choice always s
 // requests leave without waiting for a read of the argument buffer; the rest of
 // the arguments is fetched under the weight stream.  The finishing threads'
 // per-channel constants are requested first (cold, and memory serves requests
-// in the order issued), then each k-block's weights (HBM) and activations (L2).
+// in the order issued) and worked out under the first batch's requests, not behind its products; then each
+// k-block's weights (HBM) and activations (L2).
 // Measured at K = N = 4096 in a replayed graph of 40 cold weights: 5.25 us at
 // M = 1, of which 1.9 us are what an empty kernel costs there, a kernel that
 // only reads the 16.8 MB takes 4.1 us, and the one that also stores 4 KB of
@@ -116,19 +123,22 @@ constexpr int kDecodeRowsAuto = 16;  // up to here the automatic choice always s
 // activation requests are the same 16 bytes per lane at whatever address the row has, the
 // last chunk of a row is shifted into place; one launch instead of a pass that copies the rows onto
 // the 16-byte grid first (that pass is what more rows take, and the vector path it then needs).
-template <int MODE, int MG, bool RAGGED = false>
-__global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
+template <int MODE, int MG, bool RAGGED = false, int ROWS = 16>
+__global__ __launch_bounds__(kDecodeWaves* kWave, ROWS == 4 ? 6 : 1) void linear_decode_kernel(
     const uint8_t* __restrict__ w_packed, const uint8_t* __restrict__ x, const int32_t* __restrict__ colsum,
     const float* __restrict__ w_scales, const float* __restrict__ bias, int32_t K, int32_t ldx, int32_t N,
     uint32_t flags, GemmArgs a) {
   constexpr int kWaves = kDecodeWaves;
   constexpr int kBatch = 8;  // 64-byte k-blocks in flight per wave: 64 KB of weights per block
+  constexpr int kSpan = 16 / ROWS;  // k-blocks whose activations one request brings
+  static_assert(MG == 1 || ROWS == 16, "fewer than 16 rows: one group");
+  static_assert(kBatch % kSpan == 0, "whole requests");
   // The eight waves' partial sums meet in one [4 registers][64 lanes] array per row group:
   // every wave adds its accumulators with LDS atomics as it finishes (a wave instruction covers
   // 64 consecutive words: no bank conflicts, and the early waves' additions are off the block's
   // critical path), and the 64 finishing threads read four words each instead of 32.
   __shared__ int s_sum[MG][4][kWave];
-  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+  const int t = threadIdx.x, lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int lr = lane & 15, lc = lane >> 4;
   const int nb = blockIdx.x;
   const int M = static_cast<int>(flags & 0xffu);
@@ -152,19 +162,20 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
       c_cs[j] = colsum[np];
       if (MODE != kOutAcc32) {
         c_ws[j] = w_scales[np * ws_stride];
-        const float bv = bsrc[bias != nullptr ? np : 0];
-        c_b[j] = bias != nullptr ? bv : 0.f;
+        c_b[j] = bsrc[bias != nullptr ? np : 0];  // (looked at in `constants`: a select here would wait for it)
       }
     }
   }
   const uint8_t* wp = w_packed + static_cast<int64_t>(nb) * (packed_kchunks(K) * 256) + lc * 256 + lr * 16;
   // Activations are loaded with four consecutive lanes on the 64 bytes one row
   // contributes to a k-block (lane -> row lane / 4, 16-byte piece lane % 4): a
-  // quad of lanes then asks for one cache line instead of four.  The multiply
+  // quad of lanes then asks for one cache line instead of four.  With at most ROWS < 16 rows
+  // the other lanes take the same rows of the wave's next k-blocks.  The multiply
   // wants row lane % 16 and piece lane / 16, so every loaded register goes
-  // through one cross-lane permutation (lane l takes from lane 4 (l % 16) + l / 16).
-  const int sr = lane >> 2, sp = lane & 3;
-  const int perm_addr = (4 * lr + lc) * 4;
+  // through cross-lane permutations (for k-block i of a request, lane l takes from lane
+  // 4 (ROWS i + l % ROWS) + l / 16; rows ROWS ... 15 repeat others and are not stored).
+  const int sr = (lane >> 2) & (ROWS - 1), sp = lane & 3, sk = lane / (4 * ROWS);
+  const int perm_addr = (4 * (lr & (ROWS - 1)) + lc) * 4;
   bool xrow[MG];
   const uint8_t* xp[MG];
 #pragma unroll
@@ -198,52 +209,78 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
   // load), so that the counts of outstanding loads are exact and the k-blocks are
   // multiplied one by one as they arrive; with a load under a condition the
   // compiler waits for all of them before the first product.
-  auto batch = [&](int kb0) {
-    v4i wf[kBatch], xf[MG][kBatch];
-    bool xok[MG][kBatch];
-    // Requests are counted back in the order issued.  With one group of rows the weights
+  // `meanwhile` runs under the latency of the requests.
+  auto batch = [&](int kb0, auto meanwhile) {
+    constexpr int kReq = kBatch / kSpan;  // activation requests per row group
+    v4i wf[kBatch], xf[MG][kReq];
+    bool xok[MG][kReq];
+    const auto request_x = [&](int mg, int q) {
+      const int kb = kb0 + (q * kSpan + sk) * kWaves;
+      xok[mg][q] = kb < KB && xrow[mg] && (kb * 64 + sp * 16 < K);
+      xf[mg][q] = piece(xp[mg], kb, xok[mg][q]);
+    };
+    // Requests are counted back in the order issued.  With one group of 16 rows the weights
     // (memory, the critical path) go first, each followed by its activations; with more
-    // groups the activations (L2) all go first, so that their cross-lane permutations run
-    // while the weights are still on their way (K = N = 4096: M = 1 5.25 against 5.46 us
+    // groups, or where a request serves several k-blocks, the activations (L2) all go first, so that their
+    // cross-lane permutations run while the weights are still on their way (K = N = 4096: M = 1 5.25 against 5.46 us
     // the other way round, M = 32 7.5 against 7.8 us).
-    if constexpr (MG >= 2) {
+    constexpr bool kFirst = MG >= 2 || kSpan > 1;
+    if constexpr (kFirst) {
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int kb = kb0 + u * kWaves;
+      for (int q = 0; q < kReq; ++q)
 #pragma unroll
-        for (int mg = 0; mg < MG; ++mg) {
-          xok[mg][u] = kb < KB && xrow[mg] && (kb * 64 + sp * 16 < K);
-          xf[mg][u] = piece(xp[mg], kb, xok[mg][u]);
-        }
-      }
+        for (int mg = 0; mg < MG; ++mg) request_x(mg, q);
     }
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int kb = kb0 + u * kWaves;
       const int kbc = kb < KB ? kb : KB - 1;
       wf[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wp + static_cast<int64_t>(kbc) * 1024));
-      if constexpr (MG < 2) {
-#pragma unroll
-        for (int mg = 0; mg < MG; ++mg) {
-          xok[mg][u] = kb < KB && xrow[mg] && (kb * 64 + sp * 16 < K);
-          xf[mg][u] = piece(xp[mg], kb, xok[mg][u]);
-        }
-      }
+      if constexpr (!kFirst) request_x(0, u);
     }
+    meanwhile();
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
 #pragma unroll
       for (int mg = 0; mg < MG; ++mg) {
-        v4i xw = xf[mg][u];
-        if (RAGGED && kb0 + u * kWaves == KB - 1) xw = settle(xw, KB - 1);  // (the same for the whole wave)
-        const v4i xs = xok[mg][u] ? (xw ^ xmask) : v4i{0, 0, 0, 0};
+        const int q = u / kSpan;
+        if (u % kSpan == 0) {
+          v4i xw = xf[mg][q];
+          // (the k-block that ends the rows: the same for the whole wave with one k-block per request)
+          if (RAGGED && kb0 + (u + kSpan - 1) * kWaves >= KB - 1) xw = settle(xw, kb0 + (u + sk) * kWaves);
+          xf[mg][q] = xok[mg][q] ? (xw ^ xmask) : v4i{0, 0, 0, 0};
+        }
         v4i xv;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) xv[c] = __builtin_amdgcn_ds_bpermute(perm_addr, xs[c]);
+        for (int c = 0; c < 4; ++c)
+          xv[c] = __builtin_amdgcn_ds_bpermute(perm_addr + (u % kSpan) * (16 * ROWS), xf[mg][q][c]);
         acc2[mg][u & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[u], xv, acc2[mg][u & 1], 0, 0, 0);
       }
   };
-  for (int kb0 = wave; kb0 < KB; kb0 += kWaves * kBatch) batch(kb0);
+  // requantisation constants, by the wave that finishes the block, under its first requests
+  v4f bdiv = {0.f, 0.f, 0.f, 0.f}, mult = {0.f, 0.f, 0.f, 0.f};
+  float bmul = 1.f;
+  int acc0[4] = {0, 0, 0, 0};
+  auto constants = [&]() {
+    if (wave != 0) return;
+    const XQuant xq = x_quant(a);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc0[j] = xq.coef * c_cs[j];
+      if (MODE == kOutF32) {
+        mult[j] = xq.scale * c_ws[j];
+        bdiv[j] = a.bias != nullptr ? c_b[j] : 0.f;
+      } else if (MODE != kOutAcc32) {
+        const float atw = xq.scale * c_ws[j];
+        mult[j] = atw / a.out_scale;
+        bdiv[j] = a.bias != nullptr ? bias_term(a.w_scale_stride == 0, c_b[j], atw) : 0.f;
+        bmul = bias_mul(a.w_scale_stride == 0, atw);  // (per tensor: the same for every j)
+      }
+    }
+  };
+  // (two copies of the batch: with the constants inside the loop the registers of one copy hold fewer waves)
+  if (wave < KB) batch(wave, constants);  // (K >= 1: wave 0 has a k-block)
+  for (int kb0 = wave + kWaves * kBatch; kb0 < KB; kb0 += kWaves * kBatch) batch(kb0, []() {});
   v4i acc[MG];
 #pragma unroll
   for (int mg = 0; mg < MG; ++mg) acc[mg] = acc2[mg][0] + acc2[mg][1];
@@ -252,26 +289,6 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       __hip_atomic_fetch_add(&s_sum[mg][r][lane], acc[mg][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  // requantisation constants, before the barrier: off the block's critical path
-  v4f bdiv = {0.f, 0.f, 0.f, 0.f}, mult = {0.f, 0.f, 0.f, 0.f};
-  float bmul = 1.f;
-  int acc0[4] = {0, 0, 0, 0};
-  if (t < 64) {
-    const XQuant xq = x_quant(a);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc0[j] = xq.coef * c_cs[j];
-      if (MODE == kOutF32) {
-        mult[j] = xq.scale * c_ws[j];
-        bdiv[j] = c_b[j];
-      } else if (MODE != kOutAcc32) {
-        const float atw = xq.scale * c_ws[j];
-        mult[j] = atw / a.out_scale;
-        bdiv[j] = a.bias != nullptr ? bias_term(a.w_scale_stride == 0, c_b[j], atw) : 0.f;
-        bmul = bias_mul(a.w_scale_stride == 0, atw);  // (per tensor: the same for every j)
-      }
-    }
-  }
   __syncthreads();
   if (t < 64) {
     const int g = fg;
@@ -667,9 +684,14 @@ template <int MODE>
 int launch_linear_decode_ragged(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const uint32_t flags = static_cast<uint32_t>(a.M) | (a.w_scale_stride != 0 ? 0x100u : 0u) |
                          (a.x_xor != 0 ? 0x200u : 0u);
-  linear_decode_kernel<MODE, 1, true><<<dim3(static_cast<unsigned>(ceil_div(a.N, 16))), dim3(kDecodeWaves * kWave), 0, s>>>(
-      a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, static_cast<int32_t>(a.K), static_cast<int32_t>(xs.ldx),
-      static_cast<int32_t>(a.N), flags, a);
+  const auto launch = [&](auto rows_tag) {
+    linear_decode_kernel<MODE, 1, true, decltype(rows_tag)::value>
+        <<<dim3(static_cast<unsigned>(ceil_div(a.N, 16))), dim3(kDecodeWaves * kWave), 0, s>>>(
+            a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, static_cast<int32_t>(a.K), static_cast<int32_t>(xs.ldx),
+            static_cast<int32_t>(a.N), flags, a);
+  };
+  if (a.M <= 4) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 16>{});
   return launch_status();
 }
 
@@ -684,7 +706,12 @@ int launch_linear_decode(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const uint32_t flags = static_cast<uint32_t>(a.M) | (a.w_scale_stride != 0 ? 0x100u : 0u) |
                          (a.x_xor != 0 ? 0x200u : 0u);
   switch ((a.M + 15) / 16) {
-    case 1: linear_decode_kernel<MODE, 1><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
+    case 1:
+      if (a.M <= 4)
+        linear_decode_kernel<MODE, 1, false, 4><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
+      else
+        linear_decode_kernel<MODE, 1><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
+      break;
     case 2: linear_decode_kernel<MODE, 2><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
     case 3: linear_decode_kernel<MODE, 3><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
     default: linear_decode_kernel<MODE, 4><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
