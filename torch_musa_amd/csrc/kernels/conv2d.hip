@@ -311,8 +311,8 @@ template <int BM, int BN, int WM, int WN, int MODE, int KW = 1>
 int launch_conv_gemm(const GemmArgs& a, const XConv& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_kernel<BM, BN, WM, WN, MODE, XConv, 4, false, KW>
-      <<<dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s>>>(a, xs);
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XConv, 4, false, KW>,
+          dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s, a, xs);
   return launch_status();
 }
 
@@ -465,8 +465,8 @@ int launch_conv_tiles_variant(const ConvShape& s, const TilePlan& p, const ConvT
   }
   const int64_t bx = s.B * a.tiles_h * a.tiles_w, by = static_cast<int64_t>(a.n_tiles) * s.groups;
   if (bx > 0x7fffffff || by > 65535) return TMQ_ERR_UNSUPPORTED;
-  conv_tile_kernel<MODE, KIND, VEC><<<dim3(static_cast<unsigned>(bx), static_cast<unsigned>(by)),
-                                      dim3(kCtThreads), p.lds_total, stream>>>(a);
+  enqueue(conv_tile_kernel<MODE, KIND, VEC>,
+          dim3(static_cast<unsigned>(bx), static_cast<unsigned>(by)), dim3(kCtThreads), p.lds_total, stream, a);
   return launch_status();
 }
 
@@ -621,17 +621,16 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
     const auto image = [&](auto ks_tag) {
       constexpr int kKS = decltype(ks_tag)::value;
       if (s.sw % 2 == 0)
-        conv_image_kernel<MODE, kP, kNT, kKS, true, kPlain><<<grid, block, p.lds, stream>>>(a);
+        enqueue(conv_image_kernel<MODE, kP, kNT, kKS, true, kPlain>, grid, block, p.lds, stream, a);
       else
-        conv_image_kernel<MODE, kP, kNT, kKS, false, kPlain><<<grid, block, p.lds, stream>>>(a);
+        enqueue(conv_image_kernel<MODE, kP, kNT, kKS, false, kPlain>, grid, block, p.lds, stream, a);
     };
     if (s.pixels4 && s.runs_KS == 1)
       image(std::integral_constant<int, 1>{});
     else if (s.pixels4)
       image(std::integral_constant<int, kCrMaxKS>{});
     else
-      conv_runs_kernel<MODE, decltype(post_tag)::value, decltype(nt_tag)::value, decltype(plain_tag)::value>
-        <<<grid, block, p.lds, stream>>>(a);
+      enqueue(conv_runs_kernel<MODE, decltype(post_tag)::value, decltype(nt_tag)::value, decltype(plain_tag)::value>, grid, block, p.lds, stream, a);
   };
   const auto launch_tiles = [&](auto nt_tag) {
     if constexpr (MODE != kOutAcc32) {
@@ -717,11 +716,11 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
     constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;
     constexpr bool kPlain = decltype(plain_tag)::value;
     if (s.runs_KS == 1)
-      conv_runs_pointwise_kernel<MODE, kP, kNT, 1, kPlain><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 1, kPlain>, grid, block, 0, stream, a);
     else if (s.runs_KS == 2)
-      conv_runs_pointwise_kernel<MODE, kP, kNT, 2, kPlain><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 2, kPlain>, grid, block, 0, stream, a);
     else
-      conv_runs_pointwise_kernel<MODE, kP, kNT, 4, kPlain><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 4, kPlain>, grid, block, 0, stream, a);
   };
   const auto launch_tiles = [&](auto nt_tag) {
     if constexpr (MODE != kOutAcc32) {
@@ -791,13 +790,13 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
   const auto launch = [&](auto post_tag) {
     constexpr bool kP = decltype(post_tag)::value;
     if (s.KH == 3 && s.KW == 3)
-      conv_depthwise_kernel<MODE, kP, 3><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 3>, grid, block, 0, stream, a);
     else if (s.KH == 5 && s.KW == 5)
-      conv_depthwise_kernel<MODE, kP, 5><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 5>, grid, block, 0, stream, a);
     else if (s.KH == 7 && s.KW == 7)
-      conv_depthwise_kernel<MODE, kP, 7><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 7>, grid, block, 0, stream, a);
     else
-      conv_depthwise_kernel<MODE, kP, 0><<<grid, block, 0, stream>>>(a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 0>, grid, block, 0, stream, a);
   };
   if constexpr (MODE != kOutAcc32) {
     if (po.any()) {
@@ -908,9 +907,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
       if (forced == 6 && !use) return TMQ_ERR_UNSUPPORTED;
       if (use) {
         const int64_t chunks = need / 16;
-        conv_patch_rows_kernel<<<dim3(static_cast<unsigned>(ceil_div(chunks, 256))), dim3(256), 0, stream>>>(
-            static_cast<const uint8_t*>(d->x), s, chunks,
-            0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point)), static_cast<uint8_t*>(d->workspace));
+        enqueue(conv_patch_rows_kernel, dim3(static_cast<unsigned>(ceil_div(chunks, 256))), dim3(256), 0, stream,
+                static_cast<const uint8_t*>(d->x), s, chunks,
+                0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point)), static_cast<uint8_t*>(d->workspace));
         if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
         return run_as_linear(d, rows, s.OC, s.Kp, d->workspace, relu, out, stream);
       }
@@ -929,9 +928,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     if (forced == 8 && !use) return TMQ_ERR_UNSUPPORTED;
     if (use) {
       const int64_t chunks = need / 16;
-      conv_pad_channels_kernel<<<dim3(static_cast<unsigned>(ceil_div(chunks, 256))), dim3(256), 0, stream>>>(
-          static_cast<const uint8_t*>(d->x), static_cast<int>(s.IC), static_cast<int>(ceil_div(s.IC, 16)), chunks,
-          static_cast<uint8_t*>(d->workspace));
+      enqueue(conv_pad_channels_kernel, dim3(static_cast<unsigned>(ceil_div(chunks, 256))), dim3(256), 0, stream,
+              static_cast<const uint8_t*>(d->x), static_cast<int>(s.IC), static_cast<int>(ceil_div(s.IC, 16)), chunks,
+              static_cast<uint8_t*>(d->workspace));
       if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
       tmq_conv2d_desc padded = *d;
       padded.x = d->workspace;
@@ -992,7 +991,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     p.post = po;
     const int64_t blocks = ceil_div(rows * s.OC, 256);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-    conv_plain_kernel<MODE><<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(s, p);
+    enqueue(conv_plain_kernel<MODE>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, s, p);
     return launch_status();
   }
 
@@ -1164,23 +1163,23 @@ TMQ_EXPORT int tmq_conv2d_prepack(const int8_t* w_ohwi, const tmq_conv2d_geom* g
   const int64_t total = s.groups * s.group_bytes / 16;
   int64_t blocks = ceil_div(total, 256);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  conv_prepack_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, hs>>>(
-      w_ohwi, s, total, static_cast<uint8_t*>(packed));
+  enqueue(conv_prepack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, hs,
+          w_ohwi, s, total, static_cast<uint8_t*>(packed));
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   if (s.runs_bytes > 0) {
     const int64_t slots = s.runs_bytes / 16;
-    conv_prepack_runs_kernel<<<dim3(static_cast<unsigned>(ceil_div(slots, 256))), dim3(256), 0, hs>>>(
-        w_ohwi, s, slots, static_cast<uint8_t*>(packed) + s.runs_off);
+    enqueue(conv_prepack_runs_kernel, dim3(static_cast<unsigned>(ceil_div(slots, 256))), dim3(256), 0, hs,
+            w_ohwi, s, slots, static_cast<uint8_t*>(packed) + s.runs_off);
     if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   }
   if (s.taps_bytes > 0) {
-    conv_prepack_taps_kernel<<<dim3(static_cast<unsigned>(ceil_div(s.taps_bytes, 256))), dim3(256), 0, hs>>>(
-        w_ohwi, s.IC, s.KH, s.KW, s.taps_bytes, static_cast<uint8_t*>(packed) + s.runs_off);
+    enqueue(conv_prepack_taps_kernel, dim3(static_cast<unsigned>(ceil_div(s.taps_bytes, 256))), dim3(256), 0, hs,
+            w_ohwi, s.IC, s.KH, s.KW, s.taps_bytes, static_cast<uint8_t*>(packed) + s.runs_off);
     if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   }
   blocks = ceil_div(s.OC, 256 / kWave);
-  conv_colsum_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, hs>>>(
-      w_ohwi, s.OC, s.KH * s.KW * s.ICgo, colsum);
+  enqueue(conv_colsum_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, hs,
+          w_ohwi, s.OC, s.KH * s.KW * s.ICgo, colsum);
   return launch_status();
 }
 

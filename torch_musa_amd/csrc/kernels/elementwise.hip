@@ -540,12 +540,12 @@ int launch_add(const void* a, const void* b, void* out, int64_t n, const AddPara
     const int64_t n16 = n / 16;
     const int64_t blocks = n16 == 0 ? 1 : ceil_div(n16, kEwThreads * kEwUnroll);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-    qadd_vec_kernel<SIGNED, RELU><<<dim3(static_cast<unsigned>(blocks)), dim3(kEwThreads), 0, s>>>(
-        static_cast<const v4i*>(a), static_cast<const v4i*>(b), static_cast<v4i*>(out), n16, ab, bb, ob, n, p);
+    enqueue(qadd_vec_kernel<SIGNED, RELU>, dim3(static_cast<unsigned>(blocks)), dim3(kEwThreads), 0, s,
+            static_cast<const v4i*>(a), static_cast<const v4i*>(b), static_cast<v4i*>(out), n16, ab, bb, ob, n, p);
   } else {
     int64_t g = ceil_div(n, kEwThreads);
     g = g > 65536 ? 65536 : g;
-    qadd_scalar_kernel<SIGNED, RELU><<<dim3(static_cast<unsigned>(g)), dim3(kEwThreads), 0, s>>>(ab, bb, ob, n, p);
+    enqueue(qadd_scalar_kernel<SIGNED, RELU>, dim3(static_cast<unsigned>(g)), dim3(kEwThreads), 0, s, ab, bb, ob, n, p);
   }
   return launch_status();
 }
@@ -589,17 +589,19 @@ TMQ_EXPORT int tmq_qrelu(const void* x, void* y, int64_t n, int32_t zero_point, 
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
     const dim3 grid(static_cast<unsigned>(blocks)), block(kEwThreads);
     if (q_signed)
-      qrelu_vec_kernel<true><<<grid, block, 0, s>>>(static_cast<const v4i*>(x), static_cast<v4i*>(y), n16, xb, yb, n, zero_point);
+      enqueue(qrelu_vec_kernel<true>, grid, block, 0, s,
+              static_cast<const v4i*>(x), static_cast<v4i*>(y), n16, xb, yb, n, zero_point);
     else
-      qrelu_vec_kernel<false><<<grid, block, 0, s>>>(static_cast<const v4i*>(x), static_cast<v4i*>(y), n16, xb, yb, n, zero_point);
+      enqueue(qrelu_vec_kernel<false>, grid, block, 0, s,
+              static_cast<const v4i*>(x), static_cast<v4i*>(y), n16, xb, yb, n, zero_point);
   } else {
     int64_t g = ceil_div(n, kEwThreads);
     g = g > 65536 ? 65536 : g;
     const dim3 grid(static_cast<unsigned>(g)), block(kEwThreads);
     if (q_signed)
-      qrelu_scalar_kernel<true><<<grid, block, 0, s>>>(xb, yb, n, zero_point);
+      enqueue(qrelu_scalar_kernel<true>, grid, block, 0, s, xb, yb, n, zero_point);
     else
-      qrelu_scalar_kernel<false><<<grid, block, 0, s>>>(xb, yb, n, zero_point);
+      enqueue(qrelu_scalar_kernel<false>, grid, block, 0, s, xb, yb, n, zero_point);
   }
   return launch_status();
 }
@@ -630,14 +632,14 @@ TMQ_EXPORT int tmq_qcat_rows(const void* x, void* y, int64_t outer, int64_t in_r
   uint8_t* yb = static_cast<uint8_t*>(y);
   if (vec) {
     if (q_signed)
-      qcat_rows_kernel<true, 16><<<grid, block, 0, s>>>(xb, yb, outer, in_row, out_row, out_col_offset, p);
+      enqueue(qcat_rows_kernel<true, 16>, grid, block, 0, s, xb, yb, outer, in_row, out_row, out_col_offset, p);
     else
-      qcat_rows_kernel<false, 16><<<grid, block, 0, s>>>(xb, yb, outer, in_row, out_row, out_col_offset, p);
+      enqueue(qcat_rows_kernel<false, 16>, grid, block, 0, s, xb, yb, outer, in_row, out_row, out_col_offset, p);
   } else {
     if (q_signed)
-      qcat_rows_kernel<true, 1><<<grid, block, 0, s>>>(xb, yb, outer, in_row, out_row, out_col_offset, p);
+      enqueue(qcat_rows_kernel<true, 1>, grid, block, 0, s, xb, yb, outer, in_row, out_row, out_col_offset, p);
     else
-      qcat_rows_kernel<false, 1><<<grid, block, 0, s>>>(xb, yb, outer, in_row, out_row, out_col_offset, p);
+      enqueue(qcat_rows_kernel<false, 1>, grid, block, 0, s, xb, yb, outer, in_row, out_row, out_col_offset, p);
   }
   return launch_status();
 }
@@ -649,8 +651,8 @@ TMQ_EXPORT int tmq_planes_to_pixels(const void* x, void* y, int64_t B, int64_t p
   if (pixels < 16) return TMQ_ERR_UNSUPPORTED;
   const int64_t groups = ceil_div(pixels, 16), blocks = ceil_div(B * groups, kEwThreads);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  planes_to_pixels_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kEwThreads), 0, as_stream(stream)>>>(
-      static_cast<const uint8_t*>(x), static_cast<uint8_t*>(y), pixels, groups, B * groups);
+  enqueue(planes_to_pixels_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kEwThreads), 0, as_stream(stream),
+          static_cast<const uint8_t*>(x), static_cast<uint8_t*>(y), pixels, groups, B * groups);
   return launch_status();
 }
 
@@ -683,18 +685,18 @@ TMQ_EXPORT int tmq_qmaxpool2d(const void* x, void* y, int64_t B, int64_t H, int6
     const int h = static_cast<int>(H), w = static_cast<int>(W), c = static_cast<int>(C);
     const int oh = static_cast<int>(OH), ow = static_cast<int>(OW);
     if (q_signed)
-      qmaxpool_k3_rows_kernel<true><<<rgrid, block, 0, hs>>>(xb, yb, h, w, c, oh, ow, stride_h, stride_w, pad_h, pad_w);
+      enqueue(qmaxpool_k3_rows_kernel<true>, rgrid, block, 0, hs, xb, yb, h, w, c, oh, ow, stride_h, stride_w, pad_h, pad_w);
     else
-      qmaxpool_k3_rows_kernel<false><<<rgrid, block, 0, hs>>>(xb, yb, h, w, c, oh, ow, stride_h, stride_w, pad_h, pad_w);
+      enqueue(qmaxpool_k3_rows_kernel<false>, rgrid, block, 0, hs, xb, yb, h, w, c, oh, ow, stride_h, stride_w, pad_h, pad_w);
   } else if (vec && kh == 3 && kw == 3 && dil_h == 1 && dil_w == 1) {
-    if (q_signed) qmaxpool_k3_kernel<true><<<grid, block, 0, hs>>>(xb, yb, s);
-    else qmaxpool_k3_kernel<false><<<grid, block, 0, hs>>>(xb, yb, s);
+    if (q_signed) enqueue(qmaxpool_k3_kernel<true>, grid, block, 0, hs, xb, yb, s);
+    else enqueue(qmaxpool_k3_kernel<false>, grid, block, 0, hs, xb, yb, s);
   } else if (vec) {
-    if (q_signed) qmaxpool_kernel<true, 16><<<grid, block, 0, hs>>>(xb, yb, s);
-    else qmaxpool_kernel<false, 16><<<grid, block, 0, hs>>>(xb, yb, s);
+    if (q_signed) enqueue(qmaxpool_kernel<true, 16>, grid, block, 0, hs, xb, yb, s);
+    else enqueue(qmaxpool_kernel<false, 16>, grid, block, 0, hs, xb, yb, s);
   } else {
-    if (q_signed) qmaxpool_kernel<true, 1><<<grid, block, 0, hs>>>(xb, yb, s);
-    else qmaxpool_kernel<false, 1><<<grid, block, 0, hs>>>(xb, yb, s);
+    if (q_signed) enqueue(qmaxpool_kernel<true, 1>, grid, block, 0, hs, xb, yb, s);
+    else enqueue(qmaxpool_kernel<false, 1>, grid, block, 0, hs, xb, yb, s);
   }
   return launch_status();
 }
@@ -718,11 +720,11 @@ TMQ_EXPORT int tmq_qadaptive_avgpool2d(const void* x, void* y, int64_t B, int64_
   const uint8_t* xb = static_cast<const uint8_t*>(x);
   uint8_t* yb = static_cast<uint8_t*>(y);
   if (vec) {
-    if (q_signed) qadaptive_avgpool_kernel<true, 4><<<grid, block, 0, hs>>>(xb, yb, s, zero_point);
-    else qadaptive_avgpool_kernel<false, 4><<<grid, block, 0, hs>>>(xb, yb, s, zero_point);
+    if (q_signed) enqueue(qadaptive_avgpool_kernel<true, 4>, grid, block, 0, hs, xb, yb, s, zero_point);
+    else enqueue(qadaptive_avgpool_kernel<false, 4>, grid, block, 0, hs, xb, yb, s, zero_point);
   } else {
-    if (q_signed) qadaptive_avgpool_kernel<true, 1><<<grid, block, 0, hs>>>(xb, yb, s, zero_point);
-    else qadaptive_avgpool_kernel<false, 1><<<grid, block, 0, hs>>>(xb, yb, s, zero_point);
+    if (q_signed) enqueue(qadaptive_avgpool_kernel<true, 1>, grid, block, 0, hs, xb, yb, s, zero_point);
+    else enqueue(qadaptive_avgpool_kernel<false, 1>, grid, block, 0, hs, xb, yb, s, zero_point);
   }
   return launch_status();
 }
@@ -749,7 +751,7 @@ TMQ_EXPORT int tmq_qunary(const void* x, void* y, int64_t n, int kind, float in_
   uint8_t* yb = static_cast<uint8_t*>(y);
   const v4i* x16 = vec ? static_cast<const v4i*>(x) : nullptr;
   v4i* y16 = vec ? static_cast<v4i*>(y) : nullptr;
-  if (q_signed) qunary_lut_kernel<true><<<grid, block, 0, s>>>(x16, y16, n16, xb, yb, n, p);
-  else qunary_lut_kernel<false><<<grid, block, 0, s>>>(x16, y16, n16, xb, yb, n, p);
+  if (q_signed) enqueue(qunary_lut_kernel<true>, grid, block, 0, s, x16, y16, n16, xb, yb, n, p);
+  else enqueue(qunary_lut_kernel<false>, grid, block, 0, s, x16, y16, n16, xb, yb, n, p);
   return launch_status();
 }

@@ -580,8 +580,8 @@ int launch_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   if (ceil_div(a.K, kBK) < KW) return TMQ_ERR_UNSUPPORTED;  // a stage for every wave group
-  gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, PD, WDMA, KW, XWIDE>
-      <<<dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s>>>(a, xs);
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, PD, WDMA, KW, XWIDE>,
+          dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s, a, xs);
   return launch_status();
 }
 
@@ -590,8 +590,8 @@ template <int MODE, int BN = 64>
 int launch_gemm_onepass(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 64), tiles_n = ceil_div(a.N, BN);
   if (tiles_n > 0x7fffffff || tiles_m > 65535) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_onepass_kernel<MODE, BN>
-      <<<dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(BN * 4), 0, s>>>(a, xs);
+  enqueue(gemm_i8_onepass_kernel<MODE, BN>,
+          dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(BN * 4), 0, s, a, xs);
   return launch_status();
 }
 
@@ -600,8 +600,8 @@ template <int MODE>
 int launch_gemm_ksplit(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, 32);
   if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > kOnePassMaxK) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_ksplit_kernel<MODE>
-      <<<dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(256), 0, s>>>(a, xs);
+  enqueue(gemm_i8_ksplit_kernel<MODE>,
+          dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(256), 0, s, a, xs);
   return launch_status();
 }
 
@@ -613,11 +613,11 @@ int launch_gemm_wstream(const GemmArgs& a, const XLinear& xs, bool wide, hipStre
   if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > 4096) return TMQ_ERR_UNSUPPORTED;
   const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
   if (!wide && a.K <= 2048)
-    gemm_i8_wstream_kernel<MODE, 16><<<grid, dim3(256), 0, s>>>(a, xs);
+    enqueue(gemm_i8_wstream_kernel<MODE, 16>, grid, dim3(256), 0, s, a, xs);
   else if (!wide)
-    gemm_i8_wstream_kernel<MODE, 32><<<grid, dim3(256), 0, s>>>(a, xs);
+    enqueue(gemm_i8_wstream_kernel<MODE, 32>, grid, dim3(256), 0, s, a, xs);
   else
-    gemm_i8_wstream_kernel<MODE, 16, 2, 8><<<grid, dim3(512), 0, s>>>(a, xs);
+    enqueue(gemm_i8_wstream_kernel<MODE, 16, 2, 8>, grid, dim3(512), 0, s, a, xs);
   return launch_status();
 }
 
@@ -627,8 +627,8 @@ template <int MODE>
 int launch_gemm_wring(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 64), tiles_n = ceil_div(a.N, 64);
   if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > kWringMaxK || a.K % 16 != 0) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_wring_kernel<MODE><<<dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)),
-                               dim3(kWringThreads), 0, s>>>(a, xs);
+  enqueue(gemm_i8_wring_kernel<MODE>,
+          dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(kWringThreads), 0, s, a, xs);
   return launch_status();
 }
 
@@ -659,7 +659,7 @@ int launch_gemm_persistent(const GemmArgs& a, const XLinear& xs, hipStream_t s) 
     // several rounds: a multiple of 8 blocks, so that the tile sequence deals
     // every XCD its own run of tiles
     const int64_t grid = tiles <= cus ? tiles : cus / 8 * 8;
-    gemm_i8_persistent_kernel<MODE><<<dim3(static_cast<unsigned>(grid)), dim3(kPersistThreads), 0, s>>>(a, xs);
+    enqueue(gemm_i8_persistent_kernel<MODE>, dim3(static_cast<unsigned>(grid)), dim3(kPersistThreads), 0, s, a, xs);
     return launch_status();
   } else {
     return TMQ_ERR_UNSUPPORTED;
@@ -673,9 +673,9 @@ int64_t regrid_bytes(int64_t M, int64_t K) { return round_up(M * regrid_pitch(K)
 bool regrid_limits_ok(int64_t M, int64_t K) { return K > 0 && K <= 0x7fffff00 && M * (regrid_pitch(K) / 16) <= 0x7fffff00; }
 int launch_regrid(const XLinear& xs, int64_t M, int64_t K, void* out, hipStream_t s) {
   const int64_t chunks = regrid_pitch(K) / 16, total = M * chunks;
-  regrid_rows_kernel<<<dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s>>>(
-      xs.x, xs.ldx, static_cast<int32_t>(K), static_cast<uint32_t>(chunks), static_cast<uint32_t>(total),
-      static_cast<v4i*>(out));
+  enqueue(regrid_rows_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s,
+          xs.x, xs.ldx, static_cast<int32_t>(K), static_cast<uint32_t>(chunks), static_cast<uint32_t>(total),
+          static_cast<v4i*>(out));
   return launch_status();
 }
 
@@ -685,8 +685,8 @@ int launch_linear_decode_ragged(const GemmArgs& a, const XLinear& xs, hipStream_
   const uint32_t flags = static_cast<uint32_t>(a.M) | (a.w_scale_stride != 0 ? 0x100u : 0u) |
                          (a.x_xor != 0 ? 0x200u : 0u);
   const auto launch = [&](auto rows_tag) {
-    linear_decode_kernel<MODE, 1, true, decltype(rows_tag)::value>
-        <<<dim3(static_cast<unsigned>(ceil_div(a.N, 16))), dim3(kDecodeWaves * kWave), 0, s>>>(
+    enqueue(linear_decode_kernel<MODE, 1, true, decltype(rows_tag)::value>,
+            dim3(static_cast<unsigned>(ceil_div(a.N, 16))), dim3(kDecodeWaves * kWave), 0, s,
             a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, static_cast<int32_t>(a.K), static_cast<int32_t>(xs.ldx),
             static_cast<int32_t>(a.N), flags, a);
   };
@@ -708,13 +708,18 @@ int launch_linear_decode(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   switch ((a.M + 15) / 16) {
     case 1:
       if (a.M <= 4)
-        linear_decode_kernel<MODE, 1, false, 4><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
+        enqueue(linear_decode_kernel<MODE, 1, false, 4>, grid, block, 0, s,
+                a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
       else
-        linear_decode_kernel<MODE, 1><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
+        enqueue(linear_decode_kernel<MODE, 1>, grid, block, 0, s,
+                a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a);
       break;
-    case 2: linear_decode_kernel<MODE, 2><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
-    case 3: linear_decode_kernel<MODE, 3><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
-    default: linear_decode_kernel<MODE, 4><<<grid, block, 0, s>>>(a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
+    case 2: enqueue(linear_decode_kernel<MODE, 2>, grid, block, 0, s,
+            a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
+    case 3: enqueue(linear_decode_kernel<MODE, 3>, grid, block, 0, s,
+            a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
+    default: enqueue(linear_decode_kernel<MODE, 4>, grid, block, 0, s,
+            a.w_packed, xs.x, a.colsum, a.w_scales, a.bias, k32, ldx32, n32, flags, a); break;
   }
   return launch_status();
 }
@@ -746,15 +751,15 @@ int launch_linear_resident(const GemmArgs& a, const XLinear& xs, hipStream_t s) 
   const int64_t groups = ceil_div(a.N, 16);
   if (resident_pair(a.M, a.N, a.K, cus)) {
     const dim3 grid(static_cast<unsigned>(groups < 2 * cus ? groups : 2 * cus)), block(8 * kWave);
-    linear_resident_kernel<MODE, 1, 8><<<grid, block, 0, s>>>(a, xs, nullptr, 0, 0);
+    enqueue(linear_resident_kernel<MODE, 1, 8>, grid, block, 0, s, a, xs, nullptr, 0, 0);
     return launch_status();
   }
   const dim3 grid(static_cast<unsigned>(groups < cus ? groups : cus)), block(kResidentThreads);
   switch ((a.M + 15) / 16) {
-    case 1: linear_resident_kernel<MODE, 1><<<grid, block, 0, s>>>(a, xs, nullptr, 0, 0); break;
-    case 2: linear_resident_kernel<MODE, 2><<<grid, block, 0, s>>>(a, xs, nullptr, 0, 0); break;
-    case 3: linear_resident_kernel<MODE, 3><<<grid, block, 0, s>>>(a, xs, nullptr, 0, 0); break;
-    default: linear_resident_kernel<MODE, 4><<<grid, block, 0, s>>>(a, xs, nullptr, 0, 0); break;
+    case 1: enqueue(linear_resident_kernel<MODE, 1>, grid, block, 0, s, a, xs, nullptr, 0, 0); break;
+    case 2: enqueue(linear_resident_kernel<MODE, 2>, grid, block, 0, s, a, xs, nullptr, 0, 0); break;
+    case 3: enqueue(linear_resident_kernel<MODE, 3>, grid, block, 0, s, a, xs, nullptr, 0, 0); break;
+    default: enqueue(linear_resident_kernel<MODE, 4>, grid, block, 0, s, a, xs, nullptr, 0, 0); break;
   }
   return launch_status();
 }
@@ -989,8 +994,8 @@ template <int BM, int BN, int WM, int WN, int PD = 4, bool WDMA = false, bool XW
 int launch_gemm_split(const GemmArgs& a, const XLinear& xs, const SplitPlan& p, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  gemm_i8_kernel<BM, BN, WM, WN, kOutAcc32, XLinear, PD, WDMA, 1, XWIDE>
-      <<<dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(p.splits)), dim3(WM * WN * kWave), 0, s>>>(a, xs);
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, kOutAcc32, XLinear, PD, WDMA, 1, XWIDE>,
+          dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(p.splits)), dim3(WM * WN * kWave), 0, s, a, xs);
   return launch_status();
 }
 
@@ -1013,8 +1018,8 @@ int run_split(const GemmArgs& a, const XLinear& xs, const SplitPlan& p, void* wo
   const int rows = a.M <= 256 ? 4 : 16;
   const int64_t bx = ceil_div(a.N, 256), by = ceil_div(a.M, rows);
   if (bx > 0x7fffffff || by > 65535) return TMQ_ERR_UNSUPPORTED;  // a split product has a few hundred rows
-  splitk_finish_kernel<MODE><<<dim3(static_cast<unsigned>(bx), static_cast<unsigned>(by)), dim3(256), 0, s>>>(
-      a, static_cast<const int32_t*>(workspace), p.splits, p.ldp, a.M * p.ldp, rows);
+  enqueue(splitk_finish_kernel<MODE>, dim3(static_cast<unsigned>(bx), static_cast<unsigned>(by)), dim3(256), 0, s,
+          a, static_cast<const int32_t*>(workspace), p.splits, p.ldp, a.M * p.ldp, rows);
   return launch_status();
 }
 
@@ -1354,7 +1359,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
       const int64_t work = a.M * ceil_div(a.N, 4);
       const int64_t blocks = ceil_div(work, 256);
       if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-      linear_plain_kernel<MODE><<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(b, xs, x_signed);
+      enqueue(linear_plain_kernel<MODE>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, b, xs, x_signed);
       return launch_status();
     }
     case 8: return launch_linear_decode<MODE>(a, xs, s);
@@ -1436,13 +1441,13 @@ TMQ_EXPORT int tmq_linear_prepack(const int8_t* w, int64_t N, int64_t K, int64_t
   if (total > 0) {
     const int64_t blocks = ceil_div(total, 256);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-    prepack_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(
-        w, N, K, ldw, KC, total, vec, static_cast<uint8_t*>(packed));
+    enqueue(prepack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
+            w, N, K, ldw, KC, total, vec, static_cast<uint8_t*>(packed));
     if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   }
   const int64_t blocks = ceil_div(N, 256 / kWave);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  colsum_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(w, N, K, ldw, vec, colsum);
+  enqueue(colsum_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, w, N, K, ldw, vec, colsum);
   return launch_status();
 }
 
@@ -1453,8 +1458,8 @@ TMQ_EXPORT int tmq_linear_unpack(const void* packed, int64_t N, int64_t K, int8_
   if (packed == nullptr || w == nullptr) return TMQ_ERR_INVALID_ARGUMENT;
   const int64_t blocks = ceil_div(N * K, 256);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  unpack_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream)>>>(
-      static_cast<const uint8_t*>(packed), N, K, ldw, packed_kchunks(K), w);
+  enqueue(unpack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream),
+          static_cast<const uint8_t*>(packed), N, K, ldw, packed_kchunks(K), w);
   return launch_status();
 }
 
@@ -1739,23 +1744,23 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
     const dim3 grid(static_cast<unsigned>(blocks < cus ? blocks : cus)), block(kResidentThreads);
     const int64_t held = ceil_div(dyn_groups(d->M, d->K), kResidentThreads);  // float4 per thread
     if (held <= 2)
-      linear_resident_kernel<kOutF32, 1, kResidentWaves, 2><<<grid, block, 0, s>>>(a, none, x, ldx, reduce_range);
+      enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 2>, grid, block, 0, s, a, none, x, ldx, reduce_range);
     else if (held <= 4)
-      linear_resident_kernel<kOutF32, 1, kResidentWaves, 4><<<grid, block, 0, s>>>(a, none, x, ldx, reduce_range);
+      enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 4>, grid, block, 0, s, a, none, x, ldx, reduce_range);
     else
-      linear_resident_kernel<kOutF32, 1, kResidentWaves, 8><<<grid, block, 0, s>>>(a, none, x, ldx, reduce_range);
+      enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 8>, grid, block, 0, s, a, none, x, ldx, reduce_range);
     return launch_status();
   }
   const size_t lds = static_cast<size_t>(d->M) * static_cast<size_t>(round_up(d->K, 16) + 16);
   const dim3 grid(static_cast<unsigned>(blocks)), block(kDecodeWaves * kWave);
   const int64_t groups = ceil_div(dyn_groups(d->M, d->K), kDecodeWaves * kWave);  // float4 per thread
   if (groups <= 1)
-    linear_decode_dynamic_kernel<1><<<grid, block, lds, s>>>(a, x, ldx, reduce_range);
+    enqueue(linear_decode_dynamic_kernel<1>, grid, block, lds, s, a, x, ldx, reduce_range);
   else if (groups <= 2)
-    linear_decode_dynamic_kernel<2><<<grid, block, lds, s>>>(a, x, ldx, reduce_range);
+    enqueue(linear_decode_dynamic_kernel<2>, grid, block, lds, s, a, x, ldx, reduce_range);
   else if (groups <= 4)
-    linear_decode_dynamic_kernel<4><<<grid, block, lds, s>>>(a, x, ldx, reduce_range);
+    enqueue(linear_decode_dynamic_kernel<4>, grid, block, lds, s, a, x, ldx, reduce_range);
   else
-    linear_decode_dynamic_kernel<8><<<grid, block, lds, s>>>(a, x, ldx, reduce_range);
+    enqueue(linear_decode_dynamic_kernel<8>, grid, block, lds, s, a, x, ldx, reduce_range);
   return launch_status();
 }

@@ -644,10 +644,10 @@ __global__ __launch_bounds__(kDynRepeatThreads) void dynamic_quantize_repeat_ker
 template <class... Args>
 int launch_dynamic_repeat(bool q_signed, bool fused, int64_t words, hipStream_t s, Args... args) {
   const dim3 grid(static_cast<unsigned>((words + kDynRepeatThreads - 1) / kDynRepeatThreads)), block(kDynRepeatThreads);
-  if (q_signed && fused) dynamic_quantize_repeat_kernel<true, true><<<grid, block, 0, s>>>(args...);
-  else if (q_signed) dynamic_quantize_repeat_kernel<true, false><<<grid, block, 0, s>>>(args...);
-  else if (fused) dynamic_quantize_repeat_kernel<false, true><<<grid, block, 0, s>>>(args...);
-  else dynamic_quantize_repeat_kernel<false, false><<<grid, block, 0, s>>>(args...);
+  if (q_signed && fused) enqueue(dynamic_quantize_repeat_kernel<true, true>, grid, block, 0, s, args...);
+  else if (q_signed) enqueue(dynamic_quantize_repeat_kernel<true, false>, grid, block, 0, s, args...);
+  else if (fused) enqueue(dynamic_quantize_repeat_kernel<false, true>, grid, block, 0, s, args...);
+  else enqueue(dynamic_quantize_repeat_kernel<false, false>, grid, block, 0, s, args...);
   return launch_status();
 }
 
@@ -1079,11 +1079,11 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
     if (blocks < 0x7fffffff) {
       const dim3 grid(static_cast<unsigned>(blocks + extra));
       if (v4)
-        pc_cols_kernel<Op, 4><<<grid, dim3(kPcColsThreads), 0, s>>>(op, outer, C, static_cast<int32_t>(lanes),
-                                                                    static_cast<uint32_t>(col_blocks), check);
+        enqueue(pc_cols_kernel<Op, 4>, grid, dim3(kPcColsThreads), 0, s, op, outer, C, static_cast<int32_t>(lanes),
+                static_cast<uint32_t>(col_blocks), check);
       else
-        pc_cols_kernel<Op, 1><<<grid, dim3(kPcColsThreads), 0, s>>>(op, outer, C, static_cast<int32_t>(lanes),
-                                                                    static_cast<uint32_t>(col_blocks), check);
+        enqueue(pc_cols_kernel<Op, 1>, grid, dim3(kPcColsThreads), 0, s, op, outer, C, static_cast<int32_t>(lanes),
+                static_cast<uint32_t>(col_blocks), check);
       return launch_status();
     }
   }
@@ -1095,8 +1095,8 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
     const int64_t segs = ceil_div(inner, per_run << lg_us);
     const int64_t row_groups = ceil_div(outer * C, kPcAccesses >> lg_us);
     if (segs < 0x7fffffff && row_groups < 0x7fffffff / segs) {
-      pc_rows_kernel<Op><<<dim3(static_cast<unsigned>(row_groups * segs + extra)), dim3(kPcThreads), 0, s>>>(
-          op, outer * C, C, inner, lg_us, static_cast<uint32_t>(segs), check);
+      enqueue(pc_rows_kernel<Op>, dim3(static_cast<unsigned>(row_groups * segs + extra)), dim3(kPcThreads), 0, s,
+              op, outer * C, C, inner, lg_us, static_cast<uint32_t>(segs), check);
       return launch_status();
     }
   }
@@ -1105,13 +1105,13 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
     const int32_t c32 = static_cast<int32_t>(C), inner32 = static_cast<int32_t>(inner);
     const float inv_c = 1.0f / static_cast<float>(C), inv_inner = 1.0f / static_cast<float>(inner);
     if (vec)
-      pc_flat_kernel<Op, true><<<grid, dim3(kPcThreads), 0, s>>>(op, n, c32, inner32, inv_c, inv_inner, check);
+      enqueue(pc_flat_kernel<Op, true>, grid, dim3(kPcThreads), 0, s, op, n, c32, inner32, inv_c, inv_inner, check);
     else
-      pc_flat_kernel<Op, false><<<grid, dim3(kPcThreads), 0, s>>>(op, n, c32, inner32, inv_c, inv_inner, check);
+      enqueue(pc_flat_kernel<Op, false>, grid, dim3(kPcThreads), 0, s, op, n, c32, inner32, inv_c, inv_inner, check);
     return launch_status();
   }
   const unsigned g = grid_for(n, kThreads, 1 << 20);
-  pc_element_kernel<Op><<<dim3(g + static_cast<unsigned>(extra)), dim3(kThreads), 0, s>>>(op, n, C, inner, check);
+  enqueue(pc_element_kernel<Op>, dim3(g + static_cast<unsigned>(extra)), dim3(kThreads), 0, s, op, n, C, inner, check);
   return launch_status();
 }
 
@@ -1123,14 +1123,14 @@ int quantize_launch_as(const float* x, void* q, int64_t n, QParamsArg qp, hipStr
     const int64_t blocks = n4 == 0 ? 1 : ceil_div(n4, kQThreads * kUnrollQD);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
     if (n >= kStreamOutCodes)
-      quantize_vec_kernel<SIGNED, FUSED, true><<<dim3(blocks), dim3(kQThreads), 0, s>>>(
-          reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
+      enqueue(quantize_vec_kernel<SIGNED, FUSED, true>, dim3(blocks), dim3(kQThreads), 0, s,
+              reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
     else
-      quantize_vec_kernel<SIGNED, FUSED><<<dim3(blocks), dim3(kQThreads), 0, s>>>(
-          reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
+      enqueue(quantize_vec_kernel<SIGNED, FUSED>, dim3(blocks), dim3(kQThreads), 0, s,
+              reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
   } else {
     const unsigned g = grid_for(n, kThreads, 65536);
-    quantize_scalar_kernel<SIGNED, FUSED><<<dim3(g), dim3(kThreads), 0, s>>>(x, qb, n, qp);
+    enqueue(quantize_scalar_kernel<SIGNED, FUSED>, dim3(g), dim3(kThreads), 0, s, x, qb, n, qp);
   }
   return launch_status();
 }
@@ -1191,15 +1191,15 @@ TMQ_EXPORT int tmq_dequantize_per_tensor(const void* q, float* r, int64_t n, dou
     auto* q4 = reinterpret_cast<const uint32_t*>(q);
     auto* r4 = reinterpret_cast<v4f*>(r);
     if (q_signed)
-      dequantize_vec_kernel<true><<<dim3(blocks), dim3(kDqThreads), 0, s>>>(q4, r4, n4, qb, r, n, scale_f, zp);
+      enqueue(dequantize_vec_kernel<true>, dim3(blocks), dim3(kDqThreads), 0, s, q4, r4, n4, qb, r, n, scale_f, zp);
     else
-      dequantize_vec_kernel<false><<<dim3(blocks), dim3(kDqThreads), 0, s>>>(q4, r4, n4, qb, r, n, scale_f, zp);
+      enqueue(dequantize_vec_kernel<false>, dim3(blocks), dim3(kDqThreads), 0, s, q4, r4, n4, qb, r, n, scale_f, zp);
   } else {
     const unsigned g = grid_for(n, kThreads, 65536);
     if (q_signed)
-      dequantize_scalar_kernel<true><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, scale_f, zp);
+      enqueue(dequantize_scalar_kernel<true>, dim3(g), dim3(kThreads), 0, s, qb, r, n, scale_f, zp);
     else
-      dequantize_scalar_kernel<false><<<dim3(g), dim3(kThreads), 0, s>>>(qb, r, n, scale_f, zp);
+      enqueue(dequantize_scalar_kernel<false>, dim3(g), dim3(kThreads), 0, s, qb, r, n, scale_f, zp);
   }
   return launch_status();
 }
@@ -1227,18 +1227,18 @@ TMQ_EXPORT int tmq_minmax(const float* x, int64_t n, float* minmax, void* worksp
   }
   const int64_t n4 = (n - head) / 4;
   const unsigned g = grid_for(n4, kThreads * kUnroll, kMinMaxMaxBlocks);
-  minmax_partial_kernel<false><<<dim3(g), dim3(kThreads), 0, s>>>(
-      reinterpret_cast<const v4f*>(x + head), n4, x, head, n, partials, RangeReport{nullptr, 0, 0});
+  enqueue(minmax_partial_kernel<false>, dim3(g), dim3(kThreads), 0, s,
+          reinterpret_cast<const v4f*>(x + head), n4, x, head, n, partials, RangeReport{nullptr, 0, 0});
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
-  minmax_final_kernel<<<dim3(1), dim3(kThreads), 0, s>>>(partials, static_cast<int>(g), minmax);
+  enqueue(minmax_final_kernel, dim3(1), dim3(kThreads), 0, s, partials, static_cast<int>(g), minmax);
   return launch_status();
 }
 
 TMQ_EXPORT int tmq_choose_qparams_dev(const float* minmax, int q_signed, int reduce_range,
                                       tmq_qparams* qparams, tmq_stream_t stream) {
   if (minmax == nullptr || qparams == nullptr) return TMQ_ERR_INVALID_ARGUMENT;
-  choose_qparams_kernel<<<dim3(1), dim3(kWave), 0, as_stream(stream)>>>(
-      minmax, q_signed ? -128 : 0, q_signed ? 127 : 255, reduce_range, qparams);
+  enqueue(choose_qparams_kernel, dim3(1), dim3(kWave), 0, as_stream(stream),
+          minmax, q_signed ? -128 : 0, q_signed ? 127 : 255, reduce_range, qparams);
   return launch_status();
 }
 
@@ -1273,20 +1273,24 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
     const int64_t n4 = n / 4;
     const unsigned g = grid_for(n4, kThreads * kUnroll, kDynPartials);
     const v4f* x4 = reinterpret_cast<const v4f*>(x);
-    minmax_partial_kernel<true><<<dim3(g), dim3(kThreads), 0, s>>>(x4, n4, x, 0, n, partials, early);
+    enqueue(minmax_partial_kernel<true>, dim3(g), dim3(kThreads), 0, s, x4, n4, x, 0, n, partials, early);
     if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
     const dim3 grid(grid_for(n4, kThreads * kUnrollQD, kDynQBlocks)), block(kThreads);
     uint32_t* q4 = static_cast<uint32_t*>(q);
     uint8_t* qb = static_cast<uint8_t*>(q);
     const int cnt = static_cast<int>(g);
     if (q_signed && fused)
-      quantize_after_minmax_kernel<true, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
+      enqueue(quantize_after_minmax_kernel<true, true>, grid, block, 0, s,
+              x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
     else if (q_signed)
-      quantize_after_minmax_kernel<true, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
+      enqueue(quantize_after_minmax_kernel<true, false>, grid, block, 0, s,
+              x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
     else if (fused)
-      quantize_after_minmax_kernel<false, true><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
+      enqueue(quantize_after_minmax_kernel<false, true>, grid, block, 0, s,
+              x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
     else
-      quantize_after_minmax_kernel<false, false><<<grid, block, 0, s>>>(x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
+      enqueue(quantize_after_minmax_kernel<false, false>, grid, block, 0, s,
+              x4, q4, n4, x, qb, n, partials, cnt, qmin, qmax, reduce_range, qparams, late);
     return launch_status();
   }
   // larger inputs (streamed past the caches) and unaligned buffers: range, parameters and
@@ -1296,11 +1300,11 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   if (head > n) head = n;
   const int64_t n4 = (n - head) / 4;
   const unsigned g = grid_for(n4, kThreads * kUnroll, kMinMaxMaxBlocks);
-  minmax_partial_kernel<false><<<dim3(g), dim3(kThreads), 0, s>>>(reinterpret_cast<const v4f*>(x + head), n4, x, head,
-                                                           n, partials, none);
+  enqueue(minmax_partial_kernel<false>, dim3(g), dim3(kThreads), 0, s, reinterpret_cast<const v4f*>(x + head), n4, x, head,
+          n, partials, none);
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
-  minmax_final_choose_kernel<<<dim3(1), dim3(kThreads), 0, s>>>(partials, static_cast<int>(g), qmin, qmax,
-                                                                reduce_range, qparams, report);
+  enqueue(minmax_final_choose_kernel, dim3(1), dim3(kThreads), 0, s, partials, static_cast<int>(g), qmin, qmax,
+          reduce_range, qparams, report);
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   QParamsArg qp;
   qp.inv = 0.f;
@@ -1351,13 +1355,14 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
   if (head > n) head = n;
   const int64_t n4 = (n - head) / 4;
   const int count = static_cast<int>(grid_for(n4, kThreads * kUnroll, kDynPartials));
-  minmax_partial_kernel<true><<<dim3(count), dim3(kThreads), 0, s>>>(reinterpret_cast<const v4f*>(x + head), n4, x, head, n,
-                                                                    partials, RangeReport{nullptr, 0, 0});
+  enqueue(minmax_partial_kernel<true>, dim3(count), dim3(kThreads), 0, s,
+          reinterpret_cast<const v4f*>(x + head), n4, x, head, n,
+          partials, RangeReport{nullptr, 0, 0});
   if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
   const dim3 grid(grid_for(M * (pitch / 4), kThreads * 2, kDynQBlocks)), block(kThreads);
   auto go = [&](auto kernel) {
-    kernel<<<grid, block, 0, s>>>(x, static_cast<uint32_t*>(q), M, static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4),
-                                  partials, count, qmin, qmax, reduce_range, qparams);
+    enqueue(kernel, grid, block, 0, s, x, static_cast<uint32_t*>(q), M, static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4),
+            partials, count, qmin, qmax, reduce_range, qparams);
     return launch_status();
   };
   if (q_signed) return fused ? go(quantize_rows_after_minmax_kernel<true, true>) : go(quantize_rows_after_minmax_kernel<true, false>);
