@@ -307,13 +307,25 @@ __global__ __launch_bounds__(256) void conv_plain_kernel(ConvShape s, PlainArgs 
   }
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, int KW = 1>
-int launch_conv_gemm(const GemmArgs& a, const XConv& xs, hipStream_t s) {
+template <int BM, int BN, int WM, int WN, int MODE, int KW = 1, class XSRC>
+int launch_conv_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XConv, 4, false, KW>,
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, 4, false, KW>,
           dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s, a, xs);
   return launch_status();
+}
+
+// Tiles of one group's product: wave_groups and tall_tiles (128 x 64, one or two groups) go with small products only.
+template <int MODE, class XSRC>
+int launch_conv_gemm_tiles(const GemmArgs& a, const XSRC& xs, int wave_groups, bool tall_tiles, hipStream_t s) {
+  if (a.N > 64 && a.M >= 128 * 128) return launch_conv_gemm<128, 128, 2, 2, MODE>(a, xs, s);
+  if (a.M >= 256 * 256) return launch_conv_gemm<256, 64, 4, 1, MODE>(a, xs, s);
+  if (tall_tiles && wave_groups == 2) return launch_conv_gemm<128, 64, 2, 2, MODE, 2>(a, xs, s);
+  if (tall_tiles) return launch_conv_gemm<128, 64, 2, 2, MODE>(a, xs, s);
+  if (wave_groups == 4) return launch_conv_gemm<64, 64, 2, 2, MODE, 4>(a, xs, s);
+  if (wave_groups == 2) return launch_conv_gemm<64, 64, 2, 2, MODE, 2>(a, xs, s);
+  return launch_conv_gemm<64, 64, 2, 2, MODE>(a, xs, s);
 }
 
 // Patch shape and LDS layout of the halo-tiled kernel for one problem.
@@ -1043,7 +1055,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     return launch_conv_tiles<MODE>(s, plan, t, stream);
   }
 
-  XConv xs{};
+  XConvTable xs{};
   xs.x = static_cast<const uint8_t*>(d->x);
   xs.H = static_cast<int>(s.H); xs.W = static_cast<int>(s.W); xs.IC = static_cast<int>(s.IC);
   xs.OH = static_cast<int>(s.OH); xs.OW = static_cast<int>(s.OW);
@@ -1052,6 +1064,10 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   xs.pad_h = static_cast<int>(s.ph); xs.pad_w = static_cast<int>(s.pw);
   xs.dil_h = static_cast<int>(s.dh); xs.dil_w = static_cast<int>(s.dw);
   xs.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
+  xs.KH = static_cast<int>(s.KH);
+  xs.chunks = static_cast<int>(s.Kp / 16);
+  // (beyond the table's limits -- a 7 x 7 kernel over more than 334 channels, an 8 x 8 one -- the cursor that walks)
+  const bool table = s.KH * s.KW <= kConvMaxTaps && s.Kp / 16 <= kConvMaxChunks;
   xs.step_w = static_cast<int>(s.dw * s.IC - 16 * (s.ICgp / 16));
   xs.step_h = static_cast<int>(s.dh * s.W * s.IC - s.KW * s.dw * s.IC);
 
@@ -1104,20 +1120,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     a.w_packed = static_cast<const uint8_t*>(d->w_packed) + g * s.group_bytes;
     a.n_off = static_cast<int32_t>(g * s.OCg);
     xs.ic_off = static_cast<int>(g * s.ICg);
-    if (s.OCg > 64 && rows >= 128 * 128)
-      rc = launch_conv_gemm<128, 128, 2, 2, MODE>(a, xs, stream);
-    else if (rows >= 256 * 256)
-      rc = launch_conv_gemm<256, 64, 4, 1, MODE>(a, xs, stream);
-    else if (tall_tiles && wave_groups == 2)
-      rc = launch_conv_gemm<128, 64, 2, 2, MODE, 2>(a, xs, stream);
-    else if (tall_tiles)
-      rc = launch_conv_gemm<128, 64, 2, 2, MODE>(a, xs, stream);
-    else if (wave_groups == 4)
-      rc = launch_conv_gemm<64, 64, 2, 2, MODE, 4>(a, xs, stream);
-    else if (wave_groups == 2)
-      rc = launch_conv_gemm<64, 64, 2, 2, MODE, 2>(a, xs, stream);
-    else
-      rc = launch_conv_gemm<64, 64, 2, 2, MODE>(a, xs, stream);
+    rc = table ? launch_conv_gemm_tiles<MODE>(a, xs, wave_groups, tall_tiles, stream)
+               : launch_conv_gemm_tiles<MODE>(a, static_cast<const XConv&>(xs), wave_groups, tall_tiles, stream);
     if (rc != TMQ_OK) return rc;
   }
   return TMQ_OK;
