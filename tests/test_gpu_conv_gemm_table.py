@@ -4,8 +4,8 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_util import say
-from test_gpu_conv import _check, _conv_case, _run, cabi  # noqa: F401
+from gpu_util import dev, host, say
+from test_gpu_conv import LSB_TOL, _check, _conv_case, _run, cabi  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -21,6 +21,14 @@ pytestmark = pytest.mark.gpu
     ((3, 8, 8, 64, 64, 4, 1, 2, 1, 1), 2, 0),
     ((3, 8, 8, 64, 130, 4, 1, 2, 1, 1), 4, 0),
     ((3, 8, 8, 64, 64, 4, 2, 2, 1, 1), 2, 128),
+    ((1, 9, 9, 160, 70, 3, 1, 1, 1, 1), 1, 0),       # copies into LDS, 64 x 64 tiles
+    ((5, 7, 7, 48, 130, 3, 1, 1, 1, 1), 0, 128),     # 128 x 128: three images per tile, channels one past the tile
+    ((140, 3, 3, 64, 33, 3, 3, 1, 1, 1), 0, 128),    # an image per row and partly padding
+    ((3, 9, 10, 64, 257, 3, 2, 1, 1, 1), 0, 256),    # 128 x 256
+    ((1, 12, 11, 208, 250, 1, 1, 0, 1, 1), 0, 256),  # one tap, rows and channels just past and short of the tile
+    ((2, 11, 12, 96, 96, 3, 1, 2, 1, 2), 0, 256),    # two groups
+    ((1, 13, 10, 144, 16, 1, 1, 0, 1, 1), 0, 128),   # three stages, the copies' ring
+    ((1, 13, 10, 128, 16, 1, 1, 0, 1, 1), 0, 128),   # two: the cursor
     ((1, 9, 9, 320, 64, 7, 1, 3, 1, 1), 0, 0),       # 980 chunks
     ((1, 4, 5, 1024, 20, 4, 1, 2, 1, 1), 4, 0),      # 1024: the whole table
     ((1, 4, 5, 1040, 20, 4, 1, 2, 1, 1), 4, 0),      # 1040: past it
@@ -41,3 +49,33 @@ def test_conv_gemm_table(cabi, spec, wave_groups, tile_rows, x_signed):  # noqa:
     np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
     _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
                             c["out_zp"], relu=c["relu"], nthreads=8), "table")
+
+
+@pytest.mark.parametrize("ic,oc,height,tile_rows", [(272, 70, 9, 0), (464, 256, 17, 128), (1024, 40, 8, 256),
+                                                    (320, 320, 57, -1), (464, 300, 81, -1), (784, 64, 129, -1)])
+@pytest.mark.parametrize("residual,activation", [(False, "relu"), (False, "silu"), (True, "relu"), (True, "silu")])
+def test_wide_pointwise(cabi, ic, oc, height, tile_rows, residual, activation):  # noqa: F811
+    """Wide pointwise layers with residual and SiLU in the GEMM's epilogue: pinned, and (-1) by the rule's own choice."""
+    say("wide pointwise", ic, oc, height, tile_rows, residual, activation)
+    rng = np.random.default_rng(ic + oc)
+    c = _conv_case(1, height, 131, ic, oc, 1, 1, 0, 1, 1, seed=ic)
+    acc = rng.integers(0, 256, (1, height, 131, oc), dtype=np.uint8) if residual else None
+    g = cabi.conv_geom(c["xq"].shape, c["wq"].shape, (1, 1), (0, 0), (1, 1), 1)
+    pw = cabi.PackedConv2d(dev(c["wq"]), g)
+    if tile_rows >= 0:
+        cabi.force_conv_path(2)
+        cabi.force_conv_tile(tile_rows, 0)
+    try:
+        y = host(cabi.conv2d_fused(dev(c["xq"]), pw, g, c["x_scale"], c["x_zp"], dev(c["w_scales"].astype(np.float32)),
+                                   dev(c["bias"]), c["out_scale"], 20, accum=None if acc is None else dev(acc),
+                                   accum_scale=0.35, accum_zp=110, activation=activation))
+    finally:
+        cabi.force_conv_path(-1)
+        cabi.force_conv_tile(0, 0)
+    want = oracle.conv2d_fused(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], (1, 1), (0, 0), (1, 1), 1,
+                               c["out_scale"], 20, accum=acc, accum_scale=0.35, accum_zp=110, activation=activation, nthreads=8)
+    d = np.abs(y.astype(np.int32) - want.astype(np.int32))
+    if activation == "silu":  # expf on the device and on the host may differ in the last bit
+        assert d.max() <= LSB_TOL and np.count_nonzero(d) <= max(2, 0.001 * d.size), (d.max(), np.count_nonzero(d))
+    else:
+        assert d.max() == 0, (np.count_nonzero(d), d.max())

@@ -24,10 +24,10 @@ namespace {
 
 constexpr int64_t kKPad = 128;
 constexpr int64_t kTwoGroupTiles = 512;          // 64 x 64 tiles up to which the implicit GEMM splits K over two wave groups
-constexpr int64_t kFourGroupTiles = 256;         // ... over four (K of 64 stages and more)
-constexpr int64_t kPointwiseAsLinearRows = 8192;
+constexpr int64_t kPointwiseAsLinearRows = 8192;  // pixels up to which a pointwise layer runs as a linear layer
 constexpr int64_t kPatchRowsMax = 512;           // output pixels up to which a layer may run on its patch rows (workspace)
-constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on  // pixels up to which a pointwise layer runs as a linear layer
+constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on ...
+constexpr int64_t kPatchRowsMaxK = 4096;         // ... up to which it may (64 pixels: any K)
 inline int64_t packed_kchunks(int64_t K) { return (K + kKPad - 1) / kKPad * (kKPad / 16); }
 
 struct ConvShape {
@@ -207,7 +207,7 @@ int64_t patch_rows_bytes(const tmq_conv2d_geom& g, const ConvShape& s, bool pinn
       // 1024 -> 2048: 9.9 -> 8.8 us; 256 -> 512 on 56 x 56 level at batch 32 and behind at batch 8, 8.8 against 9.4 us).
       // (eight images, 512 -> 1024 on 28 x 28: 9.0 against 7.9 us on the implicit GEMM)
       if (s.IC < 512 || rows * s.IC * s.OC < (s.IC >= 1024 ? 500000000 : 2000000000)) return 0;
-    } else if (rows > kPatchRowsMax || s.Kp < kPatchRowsMinK) {
+    } else if (rows > (s.Kp <= kPatchRowsMaxK ? kPatchRowsMax : 64) || s.Kp < kPatchRowsMinK) {
       return 0;
     }
   }
@@ -307,25 +307,96 @@ __global__ __launch_bounds__(256) void conv_plain_kernel(ConvShape s, PlainArgs 
   }
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, int KW = 1, class XSRC>
+template <int BM, int BN, int WM, int WN, int MODE, bool DMA, int KW = 1, class XSRC>
 int launch_conv_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, 4, false, KW>,
-          dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s, a, xs);
+  uint32_t lds = 0;
+  if constexpr (std::is_same<XSRC, XConvTable>::value) lds = conv_table_bytes(xs.chunks);
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, DMA ? 3 : 4, DMA, KW>,
+          dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), lds, s, a, xs);
   return launch_status();
 }
 
-// Tiles of one group's product: wave_groups and tall_tiles (128 x 64, one or two groups) go with small products only.
-template <int MODE, class XSRC>
-int launch_conv_gemm_tiles(const GemmArgs& a, const XSRC& xs, int wave_groups, bool tall_tiles, hipStream_t s) {
-  if (a.N > 64 && a.M >= 128 * 128) return launch_conv_gemm<128, 128, 2, 2, MODE>(a, xs, s);
-  if (a.M >= 256 * 256) return launch_conv_gemm<256, 64, 4, 1, MODE>(a, xs, s);
-  if (tall_tiles && wave_groups == 2) return launch_conv_gemm<128, 64, 2, 2, MODE, 2>(a, xs, s);
-  if (tall_tiles) return launch_conv_gemm<128, 64, 2, 2, MODE>(a, xs, s);
-  if (wave_groups == 4) return launch_conv_gemm<64, 64, 2, 2, MODE, 4>(a, xs, s);
-  if (wave_groups == 2) return launch_conv_gemm<64, 64, 2, 2, MODE, 2>(a, xs, s);
-  return launch_conv_gemm<64, 64, 2, 2, MODE>(a, xs, s);
+// Tiles of the implicit GEMM.  kConvGroups2/4, kConvTall2: k-split wave groups, register staging (64 x 64 and 128 x 64).
+enum ConvGemmTile { kConv64, kConvGroups2, kConvGroups4, kConvTall2, kConv128, kConv256 };
+
+// The one expected to end first, by times measured on 3 x 3 layers over 176 .. 1024 channels and 49 .. 40960 pixels (us;
+// u = tiles / 256 CUs, st = stages of 64 k-bytes):
+//   64 x 64      4.0 + 0.25 u + st max(0.19 up to one tile per CU or else 0.24, 0.08 + 0.112 u)
+//   128 x 128    5.0 + st (0.28 for u <= 1, 0.35 + 0.1 u for u <= 2, 0.3 + 0.19 u for u <= 3: three blocks on a CU)
+//   128 x 256    5.0 + st (0.36 + 0.08 u for u <= 1, 0.52 + 0.23 u for u <= 2: two blocks on a CU), and per round of those;
+//                a residual or SiLU in the epilogue costs the lone block of a big tile 2 and 3.5 more
+//   128 x 64, two wave groups: 5.5 + 0.195 st for up to 256 tiles and K from 32 stages on; 64 x 64 with two: 4.3 + 0.14 st
+//                (four groups from 128 stages on: 1024 -> 1024 on 14 x 14 23.7 -> 22.3)
+// What the rule changed, from 64 x 64 by fewer than 16384 pixels and 128 x 128 beyond: 512 -> 512 on 9 x 33 x 30 47 -> 34,
+// on 16 x 28 x 28 62 -> 36, on 32 x 28 x 28 88 -> 67 (128 x 256); 384 -> 384 on 9 x 33 x 30 29 -> 22 (128 x 128).
+ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
+  const auto tiles = [&](int64_t bm, int64_t bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
+  const double st = static_cast<double>(stages), cus = 256.0;
+  const int64_t t64 = tiles(64, 64);
+  if (stages >= 128 && stages % 4 == 0 && t64 <= 128) return kConvGroups4;
+  if (stages >= 32 && stages % 2 == 0 && t64 <= 256) return kConvGroups2;
+  const double u64 = t64 / cus;
+  double best = 4.0 + 0.25 * u64 + st * std::max(t64 <= 256 ? 0.19 : 0.24, 0.08 + 0.112 * u64);
+  ConvGemmTile tile = kConv64;
+  const auto offer = [&](ConvGemmTile t, double us) {
+    if (us < best) {
+      best = us;
+      tile = t;
+    }
+  };
+  if (stages >= 32 && stages % 2 == 0 && tiles(128, 64) <= 256) offer(kConvTall2, 5.5 + 0.195 * st);
+  {
+    const int64_t t = tiles(128, 128), last = t % 768;
+    const double u = last / cus;
+    const double rate = u <= 1.0 ? 0.28 : u <= 2.0 ? 0.35 + 0.1 * u : 0.3 + 0.19 * u;
+    offer(kConv128, 1.3 + (post ? 2.0 : 0.0) + t / 768 * (5.0 + 0.8 * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
+  }
+  {
+    const int64_t t = tiles(128, 256), last = t % 512;
+    const double u = last / cus;
+    const double rate = u <= 1.0 ? 0.36 + 0.08 * u : 0.52 + 0.23 * u;
+    offer(kConv256, 1.0 + (post ? 3.5 : 0.0) + t / 512 * (5.0 + 0.9 * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
+  }
+  return tile;
+}
+
+// Pointwise layers whose weight slice leaves the halo tiles one block on a CU, or whose SiLU they cannot hide behind
+// another block's loads (us, halo tiles | implicit GEMM).  SiLU: 320 -> 320 on 32 x 14 x 14 8.8 | 6.8, 896 -> 256 on
+// 14 x 80 x 24 44.5 | 17.6, on 32 x 56 x 56 142 | 53, 448 -> 448 there 111 | 73; level at 448 -> 448 on 5 x 23 x 27
+// (6.9 | 7.0) and behind below.  A residual alone costs the GEMM's epilogue scattered reads: 288 -> 288 on 4 x 75 x 66
+// 13.1 | 14.9, on 14 x 80 x 24 19.0 | 17.6; 448 -> 448 on 32 x 14 x 14 7.9 | 8.9, on 9 x 33 x 30 12.5 | 10.1; 512 -> 1024 on
+// 32 x 14 x 14 15.0 | 15.7, on 32 x 56 x 56 224 | 148.  Neither, and at most 64 output channels (more go to the linear
+// kernels): 1024 -> 64 on 4 x 75 x 66 11.5 | 7.6, on 32 x 56 x 56 39 | 24, but 288 -> 64 there 9.5 | 11.5.
+bool pointwise_gemm_first(const ConvShape& s, const PostOps& po) {
+  if (s.KH != 1 || s.KW != 1 || s.groups != 1 || s.IC <= 256) return false;
+  const int64_t rows = s.B * s.OH * s.OW, products = rows * s.IC * s.OC;
+  if (po.silu) return products >= 150000000;
+  if (po.accum != nullptr) return rows >= 8192 && products >= (s.IC < 448 ? 2100000000 : 1700000000);
+  return s.IC >= 768 && s.OC <= 64 && rows >= 16384;
+}
+
+template <int MODE>
+int launch_conv_gemm_tile(ConvGemmTile tile, const GemmArgs& a, const XConvTable& xs, hipStream_t s) {
+  switch (tile) {
+    case kConv64: return launch_conv_gemm<64, 64, 2, 2, MODE, true>(a, xs, s);
+    case kConvGroups2: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
+    case kConvGroups4: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 4>(a, xs, s);
+    case kConvTall2: return launch_conv_gemm<128, 64, 2, 2, MODE, false, 2>(a, xs, s);
+    case kConv128: return launch_conv_gemm<128, 128, 2, 2, MODE, true>(a, xs, s);
+    case kConv256: return launch_conv_gemm<128, 256, 2, 4, MODE, true>(a, xs, s);
+  }
+  return TMQ_ERR_UNSUPPORTED;
+}
+
+// Layers the table does not take: the cursor that walks.
+template <int MODE>
+int launch_conv_gemm_walk(const GemmArgs& a, const XConv& xs, hipStream_t s) {
+  if (a.N > 64 && a.M >= 128 * 128) return launch_conv_gemm<128, 128, 2, 2, MODE, false>(a, xs, s);
+  if (ceil_div(a.K, kBK) >= 32 && ceil_div(a.M, 64) * ceil_div(a.N, 64) <= kTwoGroupTiles)
+    return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
+  return launch_conv_gemm<64, 64, 2, 2, MODE, false>(a, xs, s);
 }
 
 // Patch shape and LDS layout of the halo-tiled kernel for one problem.
@@ -899,7 +970,11 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     // channels on either side stay with the tiles: 256 -> 64 on 56 x 56 11.7 against 19.9 us, 96 -> 576 on
     // 28 x 28 14.3 against 18.0 us)
     // (a detection head's 255 channels count as wide: 128 -> 255 on 80 x 80 at batch 8 18.0 -> 15.2 us)
-    const bool wide = s.IC >= 128 && s.OC >= 224 && rows * s.IC * s.OC >= 1000000000;
+    // (narrow outputs behind wide inputs: 768 -> 192 on 16 x 28 x 28 10.9 -> 7.3 us, on 32 x 56 x 56 69 -> 32.5, 512 -> 160
+    // there 45 -> 26, 384 -> 96 there 23.3 -> 16.3; 768 -> 192 on 9 x 33 x 30 6.7 against 7.1)
+    const int64_t products = rows * s.IC * s.OC;
+    const bool wide = (s.IC >= 128 && s.OC >= 224 && products >= 1000000000) ||
+                      (s.IC >= 384 && s.OC > 64 && products >= 1500000000);
     if (forced == 5 || (forced < 0 && pointwise && (rows <= kPointwiseAsLinearRows || wide) &&
                         !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, false)))) {
       return run_as_linear(d, rows, s.OC, s.IC, d->x, relu, out, stream);
@@ -907,9 +982,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   }
   // Few output pixels against a long K and a weight slice the halo tiles cannot hold: with a
   // workspace the patch rows are written out and the product runs on the linear kernels
-  // (3 x 3, 256 -> 256 channels, one 14 x 14 image: 13.1 -> 10.1 us; 512 -> 512, one 7 x 7 image:
-  // 19.8 -> 16.1 us, eight of them 19.7 -> 17.2 us; from about a thousand pixels on the implicit
-  // GEMM with its wave groups is ahead: 1568 pixels, 256 -> 256: 13.6 against 15.4 us).
+  // (3 x 3 at 196 pixels, patch rows | implicit GEMM with its wave groups: 256 -> 256 channels 8.9 | 9.5 us, 384 -> 384
+  // 10.3 | 11.8, 448 -> 448 10.4 | 15.1, 512 -> 512 16.2 | 14.2; at 480: 384 -> 384 11.8 | 11.8, 512 -> 512 17.5 | 14.3;
+  // 1024 -> 1024 at 196 26.7 | 22.3, at 49 19.8 | 21.9; 512 -> 512 at 49 14.1 | 14.0).
   if constexpr (MODE != kOutAcc32) {
     if (forced == 6 || forced < 0) {
       const int64_t need = po.any() || !aligned(d->x, 16) ? 0 : patch_rows_bytes(d->geom, s, forced == 6);
@@ -1008,7 +1083,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   }
 
   TilePlan plan;
-  const bool tiles_ok = forced != 2 && plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan);
+  const bool tiles_ok = forced != 2 && !(forced < 0 && pointwise_gemm_first(s, po)) &&
+                        plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan);
   if (forced == 1 && !tiles_ok) return TMQ_ERR_UNSUPPORTED;
   if (tiles_ok) {
     ConvTileArgs t{};
@@ -1066,8 +1142,11 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   xs.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
   xs.KH = static_cast<int>(s.KH);
   xs.chunks = static_cast<int>(s.Kp / 16);
-  // (beyond the table's limits -- a 7 x 7 kernel over more than 334 channels, an 8 x 8 one -- the cursor that walks)
-  const bool table = s.KH * s.KW <= kConvMaxTaps && s.Kp / 16 <= kConvMaxChunks;
+  // (Beyond the table's limits -- a 7 x 7 kernel over more than 334 channels, an 8 x 8 one -- the cursor that walks; also
+  // where K ends before the copies' ring of three stages is full, and where the images of a tile's 128 rows reach past
+  // the 32 bits of its offsets.)
+  const bool table = s.KH * s.KW <= kConvMaxTaps && s.Kp / 16 <= kConvMaxChunks && s.Kp > 2 * kBK &&
+                     (128 / (s.OH * s.OW) + 2) * s.H * s.W * s.IC < (int64_t{1} << 31);
   xs.step_w = static_cast<int>(s.dw * s.IC - 16 * (s.ICgp / 16));
   xs.step_h = static_cast<int>(s.dh * s.W * s.IC - s.KW * s.dw * s.IC);
 
@@ -1088,40 +1167,22 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   a.y = out;
   a.ldy = s.OC;
   a.post = po;
-  // Few 64 x 64 tiles against a long K (3 x 3 layers over hundreds of channels on small images):
-  // two or four wave groups per block walk a half or a quarter of K each, as in quantized::linear.
-  // (pinned for tests: tile_cols = 1, 2 or 4 groups)
+  // (pinned for tests: tile_cols = 1, 2 or 4 wave groups, tile_rows = 128: tiles of 128 rows, 256: the 128 x 256 tile)
   const int64_t stages = ceil_div(s.Kp, kBK);
-  const int64_t tiles64 = ceil_div(rows, 64) * ceil_div(s.OCg, 64) * s.groups;
-  const bool small_tiles = !(s.OCg > 64 && rows >= 128 * 128) && rows < 256 * 256;
-  int wave_groups = 1;
-  if (forced == 2 && d->tile_cols > 0) {
-    wave_groups = d->tile_cols;
-    if (wave_groups != 1 && ((wave_groups != 2 && wave_groups != 4) || !small_tiles || stages % wave_groups != 0))
-      return TMQ_ERR_UNSUPPORTED;
-  } else if (small_tiles && stages >= 32) {
-    // (four groups from 64 stages on: K = 4608, 200 tiles: 20.9 against 21.9 us with two, 56 tiles: 19.7 against
-    // 20.4 us; K = 2304: level at 100 tiles, 27 against 20.7 us at 392)
-    if (stages % 4 == 0 && stages >= 64 && tiles64 <= kFourGroupTiles)
-      wave_groups = 4;
-    else if (stages % 2 == 0 && tiles64 <= kTwoGroupTiles)
-      wave_groups = 2;
-  }
-  // More 64 x 64 tiles than CUs, at most two per CU: the second round would run half empty.  Tiles of 128 rows
-  // make it one round (256 -> 256 channels, 3 x 3, 14 x 14 at batch 32, 392 tiles: 19.7 -> 17.0 us; 512 -> 512 on
-  // 7 x 7 at batch 64: 29.7 -> 28.6 us).  (pinned for tests: tile_rows = 128)
-  bool tall_tiles = small_tiles && forced == 2 && d->tile_rows == 128 && wave_groups <= 2;
-  if (!(forced == 2 && (d->tile_cols > 0 || d->tile_rows > 0)) && small_tiles && stages >= 32 && stages % 2 == 0 &&
-      tiles64 > 256 && tiles64 <= 512) {
-    tall_tiles = true;
-    wave_groups = 2;
+  ConvGemmTile tile = conv_gemm_tile(rows, s.OCg, stages, po.any());
+  if (forced == 2 && (d->tile_cols > 0 || d->tile_rows > 0)) {
+    const int groups = d->tile_cols > 0 ? d->tile_cols : 1;
+    if ((groups != 1 && groups != 2 && groups != 4) || stages % groups != 0) return TMQ_ERR_UNSUPPORTED;
+    if (d->tile_rows >= 128 && groups <= 2)
+      tile = groups == 2 ? kConvTall2 : d->tile_rows == 256 ? kConv256 : kConv128;
+    else
+      tile = groups == 4 ? kConvGroups4 : groups == 2 ? kConvGroups2 : kConv64;
   }
   for (int64_t g = 0; g < s.groups; ++g) {
     a.w_packed = static_cast<const uint8_t*>(d->w_packed) + g * s.group_bytes;
     a.n_off = static_cast<int32_t>(g * s.OCg);
     xs.ic_off = static_cast<int>(g * s.ICg);
-    rc = table ? launch_conv_gemm_tiles<MODE>(a, xs, wave_groups, tall_tiles, stream)
-               : launch_conv_gemm_tiles<MODE>(a, static_cast<const XConv&>(xs), wave_groups, tall_tiles, stream);
+    rc = table ? launch_conv_gemm_tile<MODE>(tile, a, xs, stream) : launch_conv_gemm_walk<MODE>(a, xs, stream);
     if (rc != TMQ_OK) return rc;
   }
   return TMQ_OK;

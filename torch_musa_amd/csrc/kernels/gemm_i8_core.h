@@ -76,8 +76,9 @@ struct XConv {
 // The same with the k order in a table in LDS, one entry per 16-byte k-chunk: a stage's address is one LDS read, a bit of
 // the row's mask and two additions instead of the cursor's walk (30 vector instructions a stage and wave of a 64 x 64
 // tile for 126, beside four matrix instructions).  For kernels of at most kConvMaxTaps taps and kConvMaxChunks chunks;
-// XConv has no limits.  3 x 3, 256 -> 256 channels, 32 x 14 x 14: 20.2 -> 14.1 us, 32 x 28 x 28: 34.5 -> 26.8,
-// 448 -> 448 on 14 x 80 x 24: 116 -> 89 (both with the pad put in at the LDS store and the weights through the caches).
+// XConv has no limits.  3 x 3, 256 -> 256 channels, 32 x 14 x 14: 20.2 -> 14.1 us, 32 x 28 x 28: 34.5 -> 26.8 (both with
+// the pad put in at the LDS store and the weights through the caches), with direct copies in place of registers and the
+// tiles chosen by conv_gemm_tile 13.0 and 22.0.
 struct XConvTable : XConv {
   int KH, chunks;    // kernel rows, k-chunks that carry weights
 };
@@ -86,6 +87,11 @@ struct ConvChunk {
   int off;           // bytes from the window's corner
   int tap;           // kConvMaxTaps: no tap, outside every image
 };
+
+// The table's bytes of dynamic LDS: two stages of entries past the end of K (KCursor::seek), and three for the lanes' chunk.
+inline uint32_t conv_table_bytes(int chunks) {
+  return static_cast<uint32_t>((round_up(chunks, kChunks) + 3 * kChunks) * sizeof(ConvChunk));
+}
 
 // Optional work between the requantisation's multiply and its rounding:
 //   t += float(accum_q - accum_zp) * amult     (quantized residual, output-scale units)
@@ -587,7 +593,7 @@ __device__ __forceinline__ uint32_t requant4_post(const int (&raw)[4], v4f bdiv,
 // stages: the global loads of stage t+PD are issued while stage t is being
 // multiplied, so PD-1 stages of 16-byte loads are in flight per thread.
 //
-// WDMA = true (quantized::linear only): no operand passes through registers on
+// WDMA = true (rows of quantized::linear, convolutions by their table): no operand passes through registers on
 // its way to LDS.  Each wave copies 1 KB per instruction straight from global
 // memory into LDS (global_load_lds_dwordx4: lane L's 16 bytes land in slot L
 // of the 1 KB destination), kDmaBufs stages ahead, into a ring of kDmaBufs
@@ -613,8 +619,10 @@ __global__ __launch_bounds__(WM* WN* KW* kWave, (WDMA && WM * WN == 4 && (BM / W
 void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
   constexpr int NT = WM * WN * kWave;   // threads of one group
   constexpr int NTB = NT * KW;          // threads of the block
+  constexpr bool kTable = std::is_same<XSRC, XConvTable>::value;
   static_assert(KW >= 1 && (KW == 1 || !WDMA), "k-split groups: register staging only");
-  const int kg = KW == 1 ? 0 : static_cast<int>(threadIdx.x) / NT;  // this thread's group
+  // (this thread's group; made a scalar with readfirstlane it costs two groups a tenth: M = 76, K = 5808, N = 128 14.5 -> 16.0 us)
+  const int kg = KW == 1 ? 0 : static_cast<int>(threadIdx.x) / NT;
   constexpr bool kRagged = std::is_same<XSRC, XLinearRagged>::value;
   constexpr bool kRows = kRagged || std::is_same<XSRC, XLinear>::value;
   static_assert(!kRagged || !WDMA, "rows off the 16-byte grid: register staging only");
@@ -661,11 +669,10 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
   constexpr int NDW = kChunks * (BN / 64) / NWAVES;  // weight copies per wave per stage
   constexpr int NDX = (BM / 16) / NWAVES;            // activation copies per wave per stage
   constexpr int ND = NDW + NDX;
-  static_assert(!WDMA || std::is_same<XSRC, XLinear>::value, "direct copies need plain activation rows");
+  static_assert(!WDMA || kTable || std::is_same<XSRC, XLinear>::value, "direct copies: plain rows or a table");
   static_assert(!WDMA || (BN % 64 == 0 && kChunks * (BN / 64) % NWAVES == 0 && BM % 16 == 0 &&
                           (BM / 16) % NWAVES == 0),
                 "direct copies do not divide among the waves");
-  static_assert(!WDMA || (TN + TM <= TN * TM && ND <= TN * TM), "one LDS read and one copy per MFMA at most");
   constexpr int kWBufs = WDMA ? kDmaBufs : 2, kXBufs = WDMA ? kDmaBufs : 2;
   static_assert(!XWIDE || (WDMA && PD == 3 && KW == 1 && (BM / 8) % (2 * NWAVES) == 0),
                 "wide activation copies: three-stage direct-copy ring only");
@@ -686,8 +693,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
   __shared__ __attribute__((aligned(16))) int s_acc0[BN];
   __shared__ __attribute__((aligned(16))) float s_mult[BN];
   __shared__ __attribute__((aligned(16))) float s_bdiv[BN];
-  constexpr bool kTable = std::is_same<XSRC, XConvTable>::value;
-  __shared__ ConvChunk s_chunks[kTable ? kConvMaxChunks + 3 * kChunks : 1];
+  extern __shared__ __attribute__((aligned(16))) ConvChunk s_chunks[];  // kTable: conv_table_bytes() of them
   uint8_t* const gmem = smem + kg * kMainBytes;  // this group's stages
   uint8_t* const sW = gmem;                      // [kWBufs][kWStage]
   uint8_t* const sX = gmem + kWBufs * kWStage;   // [kXBufs][kXStage]
@@ -768,6 +774,21 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
         for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[tn][tm][r] = 0;
+    }
+  };
+
+  // the k order of a convolution (all of K, whichever share a wave group has; two stages past its end)
+  auto build_table = [&]() {
+    if constexpr (kTable) {
+      for (int kc = tb; kc < static_cast<int>(round_up(xsrc.chunks, kChunks)) + 2 * kChunks; kc += NTB) {
+        ConvChunk e{0, kConvMaxTaps};
+        if (kc < xsrc.chunks) {
+          e.tap = static_cast<int>(static_cast<uint32_t>(kc) / static_cast<uint32_t>(xsrc.icb));
+          const int kh = static_cast<int>(static_cast<uint32_t>(e.tap) / static_cast<uint32_t>(xsrc.KW));
+          e.off = (kh * xsrc.dil_h * xsrc.W + (e.tap - kh * xsrc.KW) * xsrc.dil_w) * xsrc.IC + (kc - e.tap * xsrc.icb) * 16;
+        }
+        s_chunks[kc] = e;
+      }
     }
   };
 
@@ -950,7 +971,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
     // scalar bases move, no vector instruction is spent on addresses.  The host
     // keeps 256 rows of either operand within 32 bits of the tile's base.
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const uint32_t lds0 = lds_address(smem);
+    const uint32_t lds0 = lds_address(gmem);
     // weight copy i of wave w: k-chunk w & 3, 64-row group (w >> 2) + i * NWAVES / 4
     static_assert(NWAVES % 4 == 0, "weight copies: one k-chunk per wave");
     const uint8_t* const wtile = a.w_packed + (n0 / 16) * a.w_kchunks * 256;
@@ -966,18 +987,39 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
     const uint32_t wdma_lds = lds0 + ((wave_u & 3) * BN + (wave_u >> 2) * 64) * 16;
     // activation copy i of wave w: rows 16 (w + i NWAVES) .. + 15, four lanes per
     // row; the lane of slot sl fetches the k-chunk that the swizzle puts there
-    const uint8_t* const xtile = xsrc.x + m0 * xsrc.ldx;
-    const int64_t m_last = a.M - 1 - m0;
-    const int ktail = static_cast<int>(a.K) - 16 - (KT - 1) * kBK;  // last chunk inside K of the last stage
+    const uint8_t* xtile;
     uint32_t xdma_off[NDX], xdma_off_last[NDX];
+    // convolutions: offsets of the rows' windows from the tile's first image, the taps of each inside the image, and
+    // for every buffer which of this lane's copies lie outside (bit i)
+    uint64_t inside[NDX];
+    uint32_t outside[kDmaBufs];
+    KCursor<XSRC> kcur;
+    if constexpr (kTable) {
+      build_table();
+      __syncthreads();
+      const uint32_t image = static_cast<uint32_t>(m0) / static_cast<uint32_t>(xsrc.OH * xsrc.OW);
+      xtile = xsrc.x + static_cast<int64_t>(image) * xsrc.H * xsrc.W * xsrc.IC + xsrc.ic_off;
 #pragma unroll
-    for (int i = 0; i < NDX; ++i) {
-      const int row = (wave_u + i * NWAVES) * 16 + (lane >> 2);
-      const int64_t r = row < m_last ? row : m_last;
-      const int kc = ((lane & 3) ^ x_swizzle(row)) * 16;
-      xdma_off[i] = static_cast<uint32_t>(r * xsrc.ldx + kc);
-      // chunks past K: any valid bytes will do, the packed weight is zero there
-      xdma_off_last[i] = static_cast<uint32_t>(r * xsrc.ldx + (kc < ktail ? kc : ktail));
+      for (int i = 0; i < NDX; ++i) {
+        XLoader<XSRC> row;
+        row.init(xsrc, m0 + (wave_u + i * NWAVES) * 16 + (lane >> 2), a.M);
+        xdma_off[i] = static_cast<uint32_t>(row.img - xtile) + static_cast<uint32_t>(row.off0);
+        inside[i] = row.inside;
+      }
+      kcur.init(xsrc, (lane & 3) ^ x_swizzle(lane >> 2), s_chunks);
+    } else {
+      xtile = xsrc.x + m0 * xsrc.ldx;
+      const int64_t m_last = a.M - 1 - m0;
+      const int ktail = static_cast<int>(a.K) - 16 - (KT - 1) * kBK;  // last chunk inside K of the last stage
+#pragma unroll
+      for (int i = 0; i < NDX; ++i) {
+        const int row = (wave_u + i * NWAVES) * 16 + (lane >> 2);
+        const int64_t r = row < m_last ? row : m_last;
+        const int kc = ((lane & 3) ^ x_swizzle(row)) * 16;
+        xdma_off[i] = static_cast<uint32_t>(r * xsrc.ldx + kc);
+        // chunks past K: any valid bytes will do, the packed weight is zero there
+        xdma_off_last[i] = static_cast<uint32_t>(r * xsrc.ldx + (kc < ktail ? kc : ktail));
+      }
     }
     const uint32_t xdma_lds = lds0 + kWBufs * kWStage + wave_u * 1024;
     auto dma = [&](const uint8_t* base, uint32_t off, uint32_t lds_dst) { lds_dma16(base, off, lds_dst); };
@@ -988,8 +1030,32 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
             wdma_lds + b * kWStage + i * (NWAVES / 4) * 64 * 16);
       } else {
         const int j = i - NDW;
-        dma(xtile + static_cast<int64_t>(kt) * kBK, kt == KT - 1 ? xdma_off_last[j] : xdma_off[j],
-            xdma_lds + b * kXStage + j * NWAVES * 1024);
+        if constexpr (kTable) {
+          if (j == 0) {
+            kcur.seek(xsrc, kt);
+            outside[b] = 0;
+          }
+          const uint32_t in = static_cast<uint32_t>(inside[j] >> kcur.cur.tap) & 1u;
+          outside[b] |= (in ^ 1u) << j;
+          dma(xtile, (xdma_off[j] + static_cast<uint32_t>(kcur.cur.off)) & (0u - in),
+              xdma_lds + b * kXStage + j * NWAVES * 1024);
+        } else {
+          dma(xtile + static_cast<int64_t>(kt) * kBK, kt == KT - 1 ? xdma_off_last[j] : xdma_off[j],
+              xdma_lds + b * kXStage + j * NWAVES * 1024);
+        }
+      }
+    };
+    // Chunks outside the image arrive as some bytes of it; once they have, the lane that asked for one puts the zero
+    // point in its place.
+    auto pad_outside = [&](int b) {
+      if constexpr (kTable) {
+        if (outside[b] != 0) {
+          const int pad = static_cast<int>(xsrc.pad_word);
+#pragma unroll
+          for (int j = 0; j < NDX; ++j)
+            if ((outside[b] >> j) & 1u)
+              *reinterpret_cast<v4i*>(&sX[b * kXStage + (wave + j * NWAVES) * 1024 + lane * 16]) = v4i{pad, pad, pad, pad};
+        }
       }
     };
     auto wait_loads = [&](auto left_tag) {  // s_waitcnt vmcnt(left) only
@@ -998,12 +1064,15 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       __builtin_amdgcn_s_waitcnt((kLeft & 15) | ((kLeft >> 4) << 14) | (7 << 4) | (15 << 8));
     };
     auto flip = [&](v4i& f) { f ^= xmask; };
+    // LDS reads and copies per MFMA
+    constexpr int kReads = (NF + Q - 1) / Q, kCopies = (ND + Q - 1) / Q;
     // b = kt % kDmaBufs as a compile-time constant
     auto stage = [&](int kt, int b) {
       const int bn = (b + 1) % kDmaBufs;
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        if (q < NF) read_one(b, b, 1, q, wf1, xf1);
+#pragma unroll
+        for (int o = q * kReads; o < NF && o < (q + 1) * kReads; ++o) read_one(b, b, 1, o, wf1, xf1);
         mfma(q, wf0, xf0);
         if (q + 1 < TM) flip(xf0[q + 1]);
         if (q == Q - 1) flip(xf1[0]);
@@ -1011,6 +1080,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       }
       // only the copies of stages t+2 .. t+kDmaBufs-1 may still be outstanding
       wait_loads(std::integral_constant<int, (kDmaBufs - 2) * ND>{});
+      pad_outside(bn);
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
       const int kload = clampk(kt + kDmaBufs);
@@ -1018,8 +1088,11 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       constexpr int kFirstDma = (TM - 1 < Q - 1 - ND) ? TM - 1 : (Q - 1 - ND > 0 ? Q - 1 - ND : 0);
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        if (q < NF) read_one(bn, bn, 0, q, wf0, xf0);
-        if (q >= kFirstDma && q - kFirstDma < ND) dma_one(kload, b, q - kFirstDma);
+#pragma unroll
+        for (int o = q * kReads; o < NF && o < (q + 1) * kReads; ++o) read_one(bn, bn, 0, o, wf0, xf0);
+#pragma unroll
+        for (int i = (q - kFirstDma) * kCopies; i < ND && i < (q - kFirstDma + 1) * kCopies; ++i)
+          if (i >= 0) dma_one(kload, b, i);
         mfma(q, wf1, xf1);
         if (q + 1 < TM) flip(xf1[q + 1]);
         if (q == Q - 1) flip(xf0[0]);
@@ -1033,6 +1106,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       for (int i = 0; i < ND; ++i) dma_one(clampk(st), st, i);
     init_tile();
     wait_loads(std::integral_constant<int, (kDmaBufs - 1) * ND>{});
+    pad_outside(0);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < NF; ++j) read_one(0, 0, 0, j, wf0, xf0);
@@ -1052,17 +1126,7 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
     // the LDS is reused below or handed to another block
     wait_loads(std::integral_constant<int, 0>{});
   } else {
-  if constexpr (kTable) {  // (all of K, whichever share a wave group has; two stages past its end)
-    for (int kc = tb; kc < static_cast<int>(round_up(xsrc.chunks, kChunks)) + 2 * kChunks; kc += NTB) {
-      ConvChunk e{0, kConvMaxTaps};
-      if (kc < xsrc.chunks) {
-        e.tap = static_cast<int>(static_cast<uint32_t>(kc) / static_cast<uint32_t>(xsrc.icb));
-        const int kh = static_cast<int>(static_cast<uint32_t>(e.tap) / static_cast<uint32_t>(xsrc.KW));
-        e.off = (kh * xsrc.dil_h * xsrc.W + (e.tap - kh * xsrc.KW) * xsrc.dil_w) * xsrc.IC + (kc - e.tap * xsrc.icb) * 16;
-      }
-      s_chunks[kc] = e;
-    }
-  }
+  build_table();
   init_tile();  // (ends the table too: its barrier)
   // ---- staging assignments (weight rows past N are clamped: never stored)
   const uint8_t* wsrc[NW];
