@@ -1033,7 +1033,8 @@ struct LinearQuery {
   bool workspace_attached = false;
   int64_t workspace_bytes = 0;   // usable (16-byte aligned) split-K scratch
 };
-// cfg: tmq_linear_desc::kernel - 1.  0-7, 14, 17, 19, 22, 23: tiles of gemm_i8_kernel; 8: weight
+// cfg: tmq_linear_desc::kernel - 1.  0-7, 14, 17, 19, 22, 23: tiles of gemm_i8_kernel (1, 2, 6, 7, 17, 19: copied straight
+// into LDS where K and the pitch allow it); 8: weight
 // streaming; 9: plain kernel; 13: split K (plan in `split`); 20: persistent 256 x 256 tiles;
 // 21 / 24: all of K in LDS (64 x 64 / 32 x 32 tiles); 25 / 26: weights through registers
 // (32 x 32 / 32 x 64 tiles); 27: the same with 64 x 64 tiles and the activations in a ring
@@ -1109,7 +1110,7 @@ bool dynamic_resident_preferred(int64_t M, int64_t N, int64_t K) {
 }
 
 // 64 x 128 tiles with all of K in LDS, where 64 x 64 ones would need a second round of blocks and these fit
-// one (us, these | the pipelined tiles: K = 768, N = 3072: M = 384 5.8 | 6.6, M = 512 5.8 | 6.7, M = 640 5.9 | 6.8;
+// one, up to K = 256 (beyond, tile_by_rounds finds better ones; raw accumulators keep them; us, these | the pipelined tiles: K = 768, N = 3072: M = 384 5.8 | 6.6, M = 512 5.8 | 6.7, M = 640 5.9 | 6.8;
 // K = 256, N = 2000, M = 1000 4.3 | 5.6; K = 64, N = 1000, M = 2000 4.7 | 6.7; K = 512, N = 1024, M = 2048 5.1 | 6.1;
 // two rounds of them, K = 640, N = 1500, M = 1500: 10.4 | 8.2).  A K of four phases waits for the ring once:
 // K = 1024: N = 1024, M = 2048 (512 tiles of 64 x 64) 6.9 | 7.5, N = 300, M = 4096 (320) 7.2 | 7.7, N = 1600,
@@ -1117,6 +1118,72 @@ bool dynamic_resident_preferred(int64_t M, int64_t N, int64_t K) {
 bool onepass_wide_preferred(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64);
   return K <= kOnePassMaxK && tiles > (K <= 768 ? 256 : 300) && ceil_div(M, 64) * ceil_div(N, 128) <= 256;
+}
+
+// Tiles of products over K <= kRoundsMaxK by the time their rounds take (us, u = tiles / 256 CUs, st = stages of 64 k-bytes):
+//   start + round max(floor, by_u u) + full rounds of `on_cu` tiles per CU at fill + rate st each, start holding the fill of
+// the last one: per_u u and max(floor, rate0 + rate1 u) st.  The constants are fitted to 1100 shapes drawn over M = 24 .. 110000,
+// N = 64 .. 12288 and K = 64 .. 3600 (weights in the cache of the memory side; mean error 5 to 7 %); the tile they name is 2 %
+// behind the best of all kernels on average, where the thresholds below, fitted to few sizes, are 11 % behind (14 % at
+// K <= 128).  Gained (us): M = 603, N = 2304, K = 768 6.1 -> 5.3 (64 x 64 copies for 64 x 128 with all of K in LDS);
+// M = 642, N = 2304, K = 1920 12.1 -> 8.6, M = 2417, N = 832, K = 1344 9.4 -> 7.8 (for 128 x 128); M = 1690, N = 2616,
+// K = 112 8.3 -> 6.5 (64 x 64 for 128 x 128 by registers); weights from memory, M = 460, N = 1728, K = 960 8.0 -> 6.0.
+struct TileRate {
+  int cfg, bm, bn;
+  double on_cu, start, per_u, floor, rate0, rate1, fill, full;
+};
+constexpr int64_t kRoundsMaxK = 3600;
+// A lone 64 x 64 tile on a CU has room for a ring of six stages: nothing where its weights come from a cache, but from
+// memory M = 131, N = 3845, K = 2128 13.3 -> 9.5 us and M = 176, N = 2880, K = 2496 14.7 -> 10.9 (eight stages: 9.6 and 11.0).
+bool one_round_ring(int64_t M, int64_t N, int64_t K) {
+  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && K > 5 * kBK;
+}
+constexpr TileRate kShortRates[] = {
+    // one or two stages: register staging
+    {2, 64, 64, 6, 3.27, 0.47, 0.19, 0.0, 0.106, 3.14, 0.57},
+    {3, 256, 256, 1, 6.11, 2.59, 0.81, 0.0, 1.05, 6.14, 0.82},
+};
+constexpr TileRate kRates[] = {
+    // three and more: direct copies (2: 64 x 64, 1 / 7: 128 x 128 with copies of one / two stages)
+    {2, 64, 64, 4, 3.14, 0.305, 0.116, 0.0, 0.119, 1.72, 0.45},
+    {1, 128, 128, 1, 4.28, 0.66, 0.181, 0.138, 0.164, 1.40, 0.274},
+    {7, 128, 128, 1, 4.51, 0.85, 0.177, 0.146, 0.128, 2.03, 0.238},
+    {17, 128, 256, 1, 4.44, 1.97, 0.327, 0.0, 0.470, 2.67, 0.428},
+    {6, 256, 256, 1, 7.35, 1.37, 0.489, 0.274, 0.601, 6.94, 0.767},
+};
+double rounds_time(const TileRate& r, int64_t M, int64_t N, int64_t K) {
+  const double st = static_cast<double>(ceil_div(K, kBK)), round = 256.0 * r.on_cu;
+  const int64_t tiles = ceil_div(M, r.bm) * ceil_div(N, r.bn);
+  const int64_t full = (tiles - 1) / static_cast<int64_t>(round);
+  const double u = (static_cast<double>(tiles) - static_cast<double>(full) * round) / 256.0;
+  return r.start + r.per_u * u + static_cast<double>(full) * (r.fill + r.full * st) + st * std::max(r.floor, r.rate0 + r.rate1 * u);
+}
+// Beyond K = 2560 only one round of 64 x 64 tiles (weights from memory: M = 783, N = 1856, K = 3584, 377 tiles, 18.8
+// against 19.9 us), and no few rows (two wave groups are ahead: M = 57, N = 10915, K = 2816 9.8 against 11.6).
+bool rounds_modelled(int64_t M, int64_t N, int64_t K) {
+  if (N > 16384) return false;  // (beyond what was fitted)
+  return K <= 2560 || (K <= kRoundsMaxK && M > 64 && ceil_div(M, 64) * ceil_div(N, 64) <= 256);
+}
+// cfg: what the thresholds chose.  It stays where it is one of the modelled tiles and less than 5 % behind (the kernels with
+// all of K in LDS up to K = 256 are ahead: M = 1502, N = 768, K = 256 3.9 against 4.1 us).
+int tile_by_rounds(int cfg, bool onepass, int64_t M, int64_t N, int64_t K) {
+  const bool tile = cfg == 1 || cfg == 2 || cfg == 3 || cfg == 6 || cfg == 7 || cfg == 14 || cfg == 17 || cfg == 19 ||
+                    cfg == 22 || cfg == 27 || (cfg == 23 && (!onepass || K > 256)) || (cfg == 21 && K > 256 && K <= kOnePassMaxK);
+  if (!tile || !rounds_modelled(M, N, K)) return cfg;
+  int best = cfg;
+  double least = 1e30;
+  const auto offer = [&](const TileRate& r) {
+    const double us = rounds_time(r, M, N, K) * (r.cfg == cfg || (r.cfg == 17 && cfg == 19) ? 0.95 : 1.0);
+    if (us < least) {
+      least = us;
+      best = r.cfg;
+    }
+  };
+  if (K <= 2 * kBK)
+    for (const TileRate& r : kShortRates) offer(r);
+  else
+    for (const TileRate& r : kRates) offer(r);
+  return best == 17 && cfg == 19 ? 19 : best;
 }
 
 // forced: tmq_linear_desc::kernel - 1 (-1 = automatic choice).
@@ -1159,7 +1226,7 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     // short K on a grid no larger than the chip: one latency instead of one per stage
     // (M = 128, K = N = 1024: 6.0 -> 5.6 us with cold weights); up to 512 tiles of 32 x 32
     // whose waves split K spread the copies over more CUs (3.8 us; M = 512: 5.7 -> 4.4 us;
-    // N = 4096, K = 512, M = 128: 4.4 -> 4.3 us; 640 tiles and more, or K <= 256: slower)
+    // N = 4096, K = 512, M = 128: 4.4 -> 4.3 us; 640 tiles and more: tile_by_rounds; K <= 256: slower)
     cfg = K > 256 && ceil_div(M, 32) * ceil_div(N, 32) <= 512 ? 24 : 21;
   } else if (cfg < 0 && onepass_ok && onepass_wide_preferred(M, N, K)) {
     cfg = 23;
@@ -1251,6 +1318,12 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
       cfg = 2;
       c.groups = two_wave_groups_fit(M, N, K) ? 2 : 1;  // (an odd number of stages, or a shorter loop)
     }
+  }
+  if (forced < 0 && q.mode != kOutAcc32 && dma_limits_ok(std::max<int64_t>(K, 3 * kBK), q.ldx)) {
+    const int by_rounds = tile_by_rounds(cfg, c.onepass, M, N, K);
+    if (by_rounds != cfg) c.onepass = false;
+    if (by_rounds == 2 && rounds_modelled(M, N, K)) c.groups = 1;
+    cfg = by_rounds;
   }
   const bool wide_ok = wide_limits_ok(K, q.ldx);
   if (cfg == 19 && !wide_ok) cfg = 17;
@@ -1370,9 +1443,13 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     }
     case 13: return run_split<MODE>(a, xs, c.split, workspace, dma_limits_ok(a.K, xs.ldx), s);
     case 0: return launch_gemm<256, 256, 2, 2, MODE>(a, xs, s);
-    case 1: return launch_gemm<128, 128, 2, 2, MODE>(a, xs, s);
-    case 2: return c.groups == 2 ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s)
-                                 : launch_gemm<64, 64, 2, 2, MODE>(a, xs, s);
+    case 1: return dma_limits_ok(a.K, xs.ldx) ? launch_gemm<128, 128, 2, 2, MODE, 3, true>(a, xs, s)
+                                              : launch_gemm<128, 128, 2, 2, MODE>(a, xs, s);
+    case 2: return c.groups == 2                  ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s)
+                   : one_round_ring(a.M, a.N, a.K) && dma_limits_ok(a.K, xs.ldx)
+                       ? launch_gemm<64, 64, 2, 2, MODE, 6, true>(a, xs, s)
+                   : dma_limits_ok(a.K, xs.ldx) ? launch_gemm<64, 64, 2, 2, MODE, 3, true>(a, xs, s)
+                                                : launch_gemm<64, 64, 2, 2, MODE>(a, xs, s);
     case 3: return launch_gemm<256, 256, 2, 4, MODE, 3>(a, xs, s);
     case 4: return launch_gemm<128, 256, 2, 2, MODE>(a, xs, s);
     case 5: return launch_gemm<256, 128, 2, 2, MODE>(a, xs, s);
