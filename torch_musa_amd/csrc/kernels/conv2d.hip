@@ -223,25 +223,33 @@ int64_t padded_input_bytes(const tmq_conv2d_geom& g, const ConvShape& s, bool pi
   if (g.groups != 1 || s.IC % 16 == 0) return 0;
   if (!pinned && s.runs_KS != 0) return 0;
   const int64_t pixels = s.B * s.H * s.W, blocks = ceil_div(s.IC, 16);
-  if (pixels == 0 || pixels * blocks > 0x7fffffff) return 0;
+  if (pixels * s.IC < 16 || pixels * blocks > 0x7fffffff) return 0;
   return pixels * blocks * 16;
 }
 
-// One thread per 16-byte block of the padded copy.
+// kPadBlocks 16-byte blocks of the padded copy per thread, each read as 16 bytes wherever they lie (the last block of a
+// pixel runs on into the next pixel's bytes; the tensor's last ones are read from its last 16 bytes).  Bound by memory:
+// 582 channels on 22 x 38 x 81, 39 MB in and 40 out, 41.8 us with sixteen byte loads per block and a 64-bit division, 11.8 so.
+constexpr int kPadBlocks = 4;
 __global__ __launch_bounds__(256) void conv_pad_channels_kernel(const uint8_t* __restrict__ x, int IC, int blocks,
-                                                                int64_t total, uint8_t* __restrict__ dst) {
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (id >= total) return;
-  const int64_t pixel = id / blocks;
-  const int c0 = static_cast<int>(id - pixel * blocks) * 16;
-  const uint8_t* src = x + pixel * IC + c0;
-  const int n = IC - c0 < 16 ? IC - c0 : 16;
-  uint32_t words[4] = {0, 0, 0, 0};
+                                                                uint32_t total, int64_t bytes, uint8_t* __restrict__ dst) {
+  const uint32_t id0 = blockIdx.x * (256u * kPadBlocks) + threadIdx.x;
+  v4i v[kPadBlocks];
+  int past[kPadBlocks];  // bytes a block was read too early
 #pragma unroll
-  for (int b = 0; b < 16; ++b)
-    if (b < n) words[b >> 2] |= static_cast<uint32_t>(src[b]) << (8 * (b & 3));
-  *reinterpret_cast<v4i*>(dst + id * 16) = v4i{static_cast<int>(words[0]), static_cast<int>(words[1]),
-                                               static_cast<int>(words[2]), static_cast<int>(words[3])};
+  for (int u = 0; u < kPadBlocks; ++u) {
+    const uint32_t id = id0 + u * 256u < total ? id0 + u * 256u : total - 1;
+    const uint32_t pixel = id / static_cast<uint32_t>(blocks);
+    const int64_t off = static_cast<int64_t>(pixel) * IC + (id - pixel * static_cast<uint32_t>(blocks)) * 16;
+    const int64_t at = off + 16 <= bytes ? off : bytes - 16;
+    past[u] = static_cast<int>(off - at);
+    v[u] = ld16_any(x + at);
+  }
+#pragma unroll
+  for (int u = 0; u < kPadBlocks; ++u) {
+    const uint32_t id = id0 + u * 256u;
+    if (id < total) *reinterpret_cast<v4i*>(dst + static_cast<int64_t>(id) * 16) = past[u] > 0 ? shift_down_bytes(v[u], past[u]) : v[u];
+  }
 }
 
 struct PlainArgs {
@@ -1015,9 +1023,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     if (forced == 8 && !use) return TMQ_ERR_UNSUPPORTED;
     if (use) {
       const int64_t chunks = need / 16;
-      enqueue(conv_pad_channels_kernel, dim3(static_cast<unsigned>(ceil_div(chunks, 256))), dim3(256), 0, stream,
-              static_cast<const uint8_t*>(d->x), static_cast<int>(s.IC), static_cast<int>(ceil_div(s.IC, 16)), chunks,
-              static_cast<uint8_t*>(d->workspace));
+      enqueue(conv_pad_channels_kernel, dim3(static_cast<unsigned>(ceil_div(chunks, 256 * kPadBlocks))), dim3(256), 0, stream,
+              static_cast<const uint8_t*>(d->x), static_cast<int>(s.IC), static_cast<int>(ceil_div(s.IC, 16)),
+              static_cast<uint32_t>(chunks), s.B * s.H * s.W * s.IC, static_cast<uint8_t*>(d->workspace));
       if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
       tmq_conv2d_desc padded = *d;
       padded.x = d->workspace;
