@@ -50,3 +50,25 @@ def test_pieces(cabi, height, width, ic, oc, x_signed, offset):  # noqa: F811
                 assert d.max() == 0, (activation, np.count_nonzero(d), d.max())
     finally:
         cabi.force_conv_path(-1)
+
+
+@pytest.mark.parametrize("ic,oc,height,width", [(24, 512, 1, 17), (24, 513, 9, 31), (100, 1030, 40, 41),  # eight channel blocks and more
+                                                (192, 320, 30, 30), (144, 768, 40, 45), (150, 190, 91, 91),  # three k-steps
+                                                (200, 200, 128, 128), (256, 330, 127, 129), (256, 512, 33, 31)])  # four
+def test_many_blocks_and_choice(cabi, ic, oc, height, width):  # noqa: F811
+    """Waves placed by XCD, and wide layers by the automatic choice, against the oracle."""
+    say("pointwise blocks", ic, oc, height, width)
+    c = _conv_case(1, height, width, ic, oc, 1, 1, 0, 1, 1, seed=ic + oc, relu=True)
+    args = (c["stride"], c["padding"], c["dilation"], c["groups"])
+    g = cabi.conv_geom(c["xq"].shape, c["wq"].shape, *args)
+    pw, ws, bias = cabi.PackedConv2d(dev(c["wq"]), g), dev(c["w_scales"].astype(np.float32)), dev(c["bias"])
+    want = oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
+                         c["out_zp"], relu=True, nthreads=8)
+    for path in (9, -1):
+        cabi.force_conv_path(path)
+        try:
+            got = host(cabi.conv2d(dev(c["xq"]), pw, g, c["x_scale"], c["x_zp"], ws, bias, c["out_scale"], c["out_zp"],
+                                   relu=True))
+        finally:
+            cabi.force_conv_path(-1)
+        np.testing.assert_array_equal(got, want)

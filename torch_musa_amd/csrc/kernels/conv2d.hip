@@ -747,14 +747,21 @@ bool pointwise_rows_ok(const tmq_conv2d_geom& g, const ConvShape& s) {
          s.B * s.H * s.W <= 0x7fffff00 && s.B * s.H * s.W * s.IC >= 16 && s.OC <= 65536;
 }
 
-// Where it is ahead of everything else that runs the layer (us, it | the best other): always with a residual (batch
-// 32, 256 -> 512 on 28 x 28 15.1 | 18.6; 128 -> 768 on 53 x 109 at batch 6 17.7 | 28.8; one image, 96 -> 576 on
+// Where it is ahead of everything else that runs the layer (us, it | the best other): always with a residual or SiLU
+// (batch 32, 256 -> 512 on 28 x 28 15.1 | 18.6; 128 -> 768 on 53 x 109 at batch 6 17.7 | 28.8; one image, 96 -> 576 on
 // 14 x 14 4.4 | 5.3), up to 128 input channels (batch 32: 128 -> 512 on 28 x 28 10.6 | 10.8, 96 -> 576 on 14 x 14
 // 5.3 | 6.4; one image: 64 -> 256 on 56 x 56 4.2 | 4.5), and up to 160 output channels (256 -> 64 on 56 x 56 10.9 |
-// 11.0, 144 -> 24 on one image of 57 x 43 4.2 | 4.7).  More of both without a residual is the linear kernels'
-// (256 -> 512 on 28 x 28 14.4 | 12.7, 256 -> 1024 on 14 x 14 9.9 | 8.4): every wave would read the pixels again for
-// its 64 channels.
-bool pointwise_rows_first(const ConvShape& s, bool post) { return post || s.runs_KS <= 2 || s.OC <= 160; }
+// 11.0, 144 -> 24 on one image of 57 x 43 4.2 | 4.7).  Of more of both, up to 192 input channels by the pixels: 1024 and
+// fewer (192 -> 320 on 30 x 30 3.5 | 3.7), 8192 and more (144 -> 864 on 4 x 103 x 91 17.8 | 22.8, 192 -> 320 on
+// 32 x 56 x 56 16.0 | 24.5), between them from 768 output channels on (3600: 192 -> 1152 5.5 | 6.7, but 144 -> 512 4.7 |
+// 4.3); beyond 192 from 16384 on (256 -> 256 on 32 x 56 x 56 18.5 | 22.3, 256 -> 512 on 4 x 75 x 66 9.9 | 10.9; on
+// 8 x 40 x 40 8.0 | 7.5).  The rest is the linear kernels': every wave would read the pixels again for its 64 channels.
+bool pointwise_rows_first(const ConvShape& s, bool post) {
+  const int64_t pixels = s.B * s.H * s.W;
+  if (post || s.runs_KS <= 2 || s.OC <= 160) return true;
+  if (s.runs_KS == 3) return pixels <= 1024 || pixels >= 8192 || s.OC >= 768;
+  return pixels >= 16384;
+}
 
 // The 16-pixel pieces whose reads and stores the kernel makes without a check: all 16 pixels exist, and the last pixel's
 // 16-byte reads (to RP >= IC bytes behind its first) end inside the tensor.  None where a lane's residual bytes are more

@@ -455,7 +455,13 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
   const int pj = lane & 15, pq = lane >> 4;
   const int KS = a.KS;
   const int nblk = a.nblk, groups = a.groups;
-  const uint32_t w = blockIdx.x * kCrWaves + static_cast<uint32_t>(wave);
+  // With eight and more channel blocks the waves of one group of pixels sit in several blocks: on one XCD they share the
+  // pixels' bytes and the output lines where two channel blocks meet (97 -> 582 channels on 22 x 38 x 81 34.9 -> 30.8 us,
+  // 128 -> 768 on 11 x 17 x 48 8.4 -> 8.0; fewer share nothing and stream worse: 24 -> 144 at batch 32 9.9 -> 12.2, 128 ->
+  // 273 with a residual 7.3 -> 8.0).
+  const uint32_t blocks = (static_cast<uint32_t>(groups * nblk) + kCrWaves - 1) / kCrWaves;
+  const uint32_t block = nblk >= 8 ? xcd_contiguous(blockIdx.x, blocks) : blockIdx.x;
+  const uint32_t w = block * kCrWaves + static_cast<uint32_t>(wave);
   const int g = static_cast<int>(nblk == 1 ? w : __umulhi(w, a.nblk_magic));
   const int cb = static_cast<int>(w) - g * nblk;
   if (g >= groups || g >= a.tiles) return;  // (no barrier below: the waves share nothing)
