@@ -137,6 +137,16 @@ int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, i
                                            void* workspace, size_t workspace_bytes,
                                            tmq_host_report* report, uint32_t ticket, uint32_t slot,
                                            tmq_stream_t stream);
+/* The same, where the range may come in parts: *count of them, each the minimum (lower half) and maximum (upper half)
+ * of some of the values as one word of `parts`, TMQ_HOST_PARTS words of pinned host memory that the caller has set to
+ * TMQ_HOST_PART_EMPTY (two NaNs, which no part is).  *count = 0: the range goes to `report` as a whole. */
+#define TMQ_HOST_PARTS 64
+#define TMQ_HOST_PART_EMPTY 0xffffffffffffffffull
+int tmq_quantize_per_tensor_dynamic_parts(const float* x, void* q, int64_t n, int q_signed,
+                                          int reduce_range, int rounding, tmq_qparams* qparams,
+                                          void* workspace, size_t workspace_bytes,
+                                          tmq_host_report* report, uint32_t ticket, uint32_t slot,
+                                          uint64_t* parts, int32_t* count, tmq_stream_t stream);
 /* The same for M rows of K values -> rows of `pitch` codes, pitch a multiple of
  * 16 that is at least K: what tmq_linear wants of activations whose K is not.
  * The codes behind a row's end are undefined (the packed weights are zero there).

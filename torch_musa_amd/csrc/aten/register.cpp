@@ -135,6 +135,7 @@ class HostReport {
   HostReport(const c10::hip::HIPStream& stream, const char* what) : stream_(stream), what_(what), hold_(pool().slots) {
     TORCH_CHECK(hold_.slot() >= 0, what_, ": every report slot was lost to a failed call");
     slot_ = reinterpret_cast<tmq_host_report*>(static_cast<char*>(pool().page) + hold_.slot() * kStride);
+    parts_ = reinterpret_cast<uint64_t*>(slot_) + kPartsAt / sizeof(uint64_t);
   }
 
   tmq_host_report* memory() { return slot_; }
@@ -164,12 +165,48 @@ class HostReport {
     TORCH_CHECK(static_cast<uint32_t>(v >> 32) == ticket(), what_, ": the kernel ended without its report");
     return static_cast<uint32_t>(v);
   }
+  // A range that may come in parts (tmq_quantize_per_tensor_dynamic_parts): emptied before the call ...
+  uint64_t* empty_parts() {
+    for (int i = 0; i < TMQ_HOST_PARTS; ++i) parts_[i] = TMQ_HOST_PART_EMPTY;
+    return parts_;
+  }
+  // ... and put together behind it.
+  void wait_range(int count, float* mn, float* mx) {
+    if (count == 0) {
+      const uint32_t lo = wait(0), hi = wait(1);
+      std::memcpy(mn, &lo, 4);
+      std::memcpy(mx, &hi, 4);
+      return;
+    }
+    *mn = std::numeric_limits<float>::infinity();
+    *mx = -std::numeric_limits<float>::infinity();
+    int spin = 0;
+    bool waited = false;
+    for (int i = 0; i < count;) {
+      const uint64_t v = *static_cast<const volatile uint64_t*>(&parts_[i]);
+      if (v != TMQ_HOST_PART_EMPTY) {
+        const uint32_t lo = static_cast<uint32_t>(v), hi = static_cast<uint32_t>(v >> 32);
+        float a, b;
+        std::memcpy(&a, &lo, 4);
+        std::memcpy(&b, &hi, 4);
+        *mn = std::min(*mn, a);
+        *mx = std::max(*mx, b);
+        ++i;
+      } else if (++spin < kSpins) {
+        __builtin_ia32_pause();
+      } else {
+        TORCH_CHECK(!waited, what_, ": the kernel ended without its report");
+        stream_.synchronize();
+        waited = true;
+      }
+    }
+  }
   void done() { hold_.done(); }
 
  private:
   static constexpr int kSlots = TMQ_HOST_REPORTS;  // calls that wait at the same time; more of them queue for a slot
   static constexpr int kSpins = 20000;  // about a millisecond
-  static constexpr size_t kStride = 64;  // a cache line each
+  static constexpr size_t kPartsAt = 64, kStride = kPartsAt + TMQ_HOST_PARTS * sizeof(uint64_t);  // cache lines of their own
   struct Pool {
     tmq::ReportSlots slots{kSlots};
     void* page = nullptr;
@@ -187,6 +224,7 @@ class HostReport {
   const char* const what_;
   tmq::ReportHold hold_;
   tmq_host_report* slot_;
+  uint64_t* parts_;
 };
 
 bool stream_is_capturing(const c10::hip::HIPStream& s) {
@@ -387,17 +425,17 @@ at::Tensor quantize_per_tensor_dynamic(const at::Tensor& self, at::ScalarType dt
   const at::Tensor scratch = empty_bytes(range_bytes + static_cast<int64_t>(sizeof(tmq_qparams)), x);
   auto* ws = static_cast<uint8_t*>(scratch.data_ptr());
   HostReport report(stream, what);
+  uint64_t* const parts = report.empty_parts();
+  int32_t count = 0;
   report.queue([&] {
-    return tmq_quantize_per_tensor_dynamic_report(
+    return tmq_quantize_per_tensor_dynamic_parts(
         cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
         reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes), report.memory(),
-        report.ticket(), report.number(), reinterpret_cast<tmq_stream_t>(stream.stream()));
+        report.ticket(), report.number(), parts, &count, reinterpret_cast<tmq_stream_t>(stream.stream()));
   });
-  const uint32_t lo = report.wait(0), hi = report.wait(1);
-  report.done();
   float mn, mx;
-  std::memcpy(&mn, &lo, 4);
-  std::memcpy(&mx, &hi, 4);
+  report.wait_range(count, &mn, &mx);
+  report.done();
   TORCH_CHECK(mn <= mx, "In ChooseQuantizationParams, min should be less than or equal to max");
   check_status(tmq_choose_qparams_host(mn, mx, sgn, reduce_range, &scale, &zp), "tmq_choose_qparams_host");
   at::get_qtensorimpl(q)->set_quantizer_(at::make_per_tensor_affine_quantizer(scale, zp, dtype));
