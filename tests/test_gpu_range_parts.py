@@ -11,7 +11,7 @@ import torch_musa_amd  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [98305, 98306, 98307, 98308, 128 * 1024, 262144 - 1, 262144, 262144 + 5, 262144 + 4096 * 4 + 3, 1 << 20, (1 << 21) - 3, 1 << 21, (1 << 21) + 1]
+SIZES = [65536, 65537, 65539, 81920, 98304, 98305, 98306, 98307, 98308, 128 * 1024, 262144 - 1, 262144, 262144 + 5, 262144 + 4096 * 4 + 3, 1 << 20, (1 << 21) - 3, 1 << 21, (1 << 21) + 1]
 
 
 @pytest.mark.parametrize("n", SIZES)

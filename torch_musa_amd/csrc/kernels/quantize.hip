@@ -367,9 +367,11 @@ __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
 // block tells the host the range of its own part with one store, and the host puts the parts together.  The kernel above
 // spends two trips to where all XCDs see its count, and a third to read the other blocks' pairs, before the host hears a word;
 // here the host reads up to eight cache lines instead.  (quantize_per_tensor_dynamic and dequantize of 128 x 1024 values
-// 16.6 -> 15.6 us, of 1000 x 1000 17.9 -> 16.4, of 2048 x 1024 19.2 -> 16.7.)
+// 16.6 -> 15.6 us, of 1000 x 1000 17.9 -> 16.4, of 2048 x 1024 19.2 -> 16.7.  Against the one launch of
+// dynamic_quantize_repeat_kernel, whose blocks each read everything before the first of them reports: 32 Ki values 15.9 | 14.9,
+// 64 Ki level at 16.0, 80 Ki 15.8 | 16.9, 96 Ki 15.9 | 17.0.)
 constexpr int kPartsThreads = 1024;
-constexpr int64_t kPartsMax = int64_t{1} << 21;
+constexpr int64_t kPartsMin = int64_t{1} << 16, kPartsMax = int64_t{1} << 21;
 __global__ __launch_bounds__(kPartsThreads) void minmax_parts_kernel(const v4f* __restrict__ x4, int32_t n4,
                                                                      const float* __restrict__ x, int32_t n,
                                                                      float* __restrict__ partials, uint64_t* parts) {
@@ -1306,7 +1308,9 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   if (!aligned(x, 4)) return TMQ_ERR_ALIGNMENT;
   hipStream_t s = as_stream(stream);
   const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
-  if (n <= kDynRepeatMax) {
+  const bool vec_ok = aligned(x, 16) && aligned(q, 4);
+  const bool two_ok = workspace != nullptr && workspace_bytes >= tmq_minmax_workspace_bytes(n) && aligned(workspace, 8);
+  if (n <= kDynRepeatMax && !(parts != nullptr && n > kPartsMin && vec_ok && two_ok)) {
     const int32_t n32 = static_cast<int32_t>(n);
     // (nothing to quantize: one block still publishes the parameters)
     return launch_dynamic_repeat(q_signed != 0, fused, n > 0 ? ceil_div(n, 4) : 1, s, x, static_cast<uint8_t*>(q), n32, n32, 0,
@@ -1317,7 +1321,7 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
     return TMQ_ERR_WORKSPACE;
   float* partials = static_cast<float*>(workspace);
   const RangeReport none{nullptr, 0, 0};
-  if (n <= kDynKeepMax && aligned(x, 16) && aligned(q, 4) && aligned(workspace, 8)) {
+  if (n <= kDynKeepMax && vec_ok && two_ok) {
     // Inputs that fit the last-level cache with room to spare (where the launches, not the
     // bytes, are what counts): two launches -- partial ranges, read with ordinary loads so
     // that the second pass finds the input cached, then the quantizer whose blocks finish
