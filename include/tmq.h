@@ -435,7 +435,8 @@ typedef struct tmq_conv2d_desc {
    * to a multiple of 16, then whatever the library chooses for that, 9 a pointwise
    * layer over at most 256 input channels with its pixels straight from memory
    * (TMQ_ERR_UNSUPPORTED when the family cannot run the problem).  tile_rows / tile_cols > 0 pin the halo
-   * kernel's patch height / bound its patch width. */
+   * kernel's patch height / bound its patch width; for the implicit GEMM tile_rows = 128 pins tiles of 128
+   * rows, 256 the tile of 128 rows x 256 channels, tile_cols = 1, 2 or 4 the wave groups that share K. */
   int32_t kernel;
   int32_t tile_rows, tile_cols;
   int32_t reserved;
