@@ -79,3 +79,30 @@ def test_wide_pointwise(cabi, ic, oc, height, tile_rows, residual, activation): 
         assert d.max() <= LSB_TOL and np.count_nonzero(d) <= max(2, 0.001 * d.size), (d.max(), np.count_nonzero(d))
     else:
         assert d.max() == 0, (np.count_nonzero(d), d.max())
+
+
+@pytest.mark.parametrize("spec", [
+    # layers without a table, by the rule's own choice
+    (1, 9, 9, 32, 20, 9, 1, 4, 1, 1),          # 41 stages: four wave groups, ten stages each and eleven
+    (2, 10, 9, 64, 70, 9, 2, 4, 1, 2),         # the same over two groups
+    (1, 6, 7, 32, 33, 8, 1, 6, 2, 1),          # 32 stages, windows reaching past the image on all sides
+    (5, 36, 34, 32, 130, 8, 1, 3, 1, 1),       # 5775 pixels x 130 channels: 128 x 64 tiles, two groups of 16 stages
+    (1, 40, 52, 48, 72, 9, 1, 4, 1, 1),        # 61 stages
+    (1, 30, 31, 16, 40, 8, 1, 4, 1, 1),        # 16 stages: one group
+    (1, 129, 130, 32, 70, 1, 1, 0, 1, 1),      # one stage, 128 x 128 tiles
+    (1, 257, 257, 32, 48, 1, 1, 0, 1, 1),      # one stage, 256 x 64 tiles
+    (1, 513, 515, 112, 64, 1, 2, 0, 1, 1),     # two, every second pixel
+])
+@pytest.mark.parametrize("x_signed", [False, True])
+def test_conv_gemm_walk(cabi, spec, x_signed):  # noqa: F811
+    say("conv gemm walk", spec, x_signed)
+    c = _conv_case(*spec, seed=sum(spec), x_signed=x_signed, relu=x_signed)
+    cabi.force_conv_path(2)
+    try:
+        y, acc, _ = _run(cabi, c)
+    finally:
+        cabi.force_conv_path(-1)
+    args = (c["stride"], c["padding"], c["dilation"], c["groups"])
+    np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
+    _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
+                            c["out_zp"], relu=c["relu"], nthreads=8), "walk")

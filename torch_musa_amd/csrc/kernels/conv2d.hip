@@ -23,11 +23,10 @@ namespace tmq {
 namespace {
 
 constexpr int64_t kKPad = 128;
-constexpr int64_t kTwoGroupTiles = 512;          // 64 x 64 tiles up to which the implicit GEMM splits K over two wave groups
 constexpr int64_t kPointwiseAsLinearRows = 8192;  // pixels up to which a pointwise layer runs as a linear layer
 constexpr int64_t kPatchRowsMax = 512;           // output pixels up to which a layer may run on its patch rows (workspace)
 constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on ...
-constexpr int64_t kPatchRowsMaxK = 4096;         // ... up to which it may (64 pixels: any K)
+constexpr int64_t kPatchRowsMaxK = 4096;         // ... up to which it may (64 pixels, or no table for the layer: any K)
 inline int64_t packed_kchunks(int64_t K) { return (K + kKPad - 1) / kKPad * (kKPad / 16); }
 
 struct ConvShape {
@@ -170,6 +169,14 @@ __global__ __launch_bounds__(256) void conv_colsum_kernel(const int8_t* __restri
   if (lane == 0) colsum[n] = s;
 }
 
+// Whether the implicit GEMM has the layer's k order in a table (XConvTable); the rest walks it (XConv): kernels of 8 x 8 and
+// more, K that ends before the copies' ring of three stages is full, and images of which a tile's 128 rows reach past the
+// 32 bits of its offsets.
+bool conv_table_takes(const ConvShape& s) {
+  return s.KH * s.KW <= kConvMaxTaps && s.Kp / 16 <= kConvMaxChunks && s.Kp > 2 * kBK &&
+         (128 / (s.OH * s.OW) + 2) * s.H * s.W * s.IC < (int64_t{1} << 31);
+}
+
 // Patch rows (im2col) of a convolution over whole 16-channel blocks, one group: row m = output
 // pixel (b, oh, ow), k = (kh, kw, ic) as in the packed weight; one thread per 16-byte chunk.
 // Taps outside the image are the activation zero point.
@@ -207,7 +214,7 @@ int64_t patch_rows_bytes(const tmq_conv2d_geom& g, const ConvShape& s, bool pinn
       // 1024 -> 2048: 9.9 -> 8.8 us; 256 -> 512 on 56 x 56 level at batch 32 and behind at batch 8, 8.8 against 9.4 us).
       // (eight images, 512 -> 1024 on 28 x 28: 9.0 against 7.9 us on the implicit GEMM)
       if (s.IC < 512 || rows * s.IC * s.OC < (s.IC >= 1024 ? 500000000 : 2000000000)) return 0;
-    } else if (rows > (s.Kp <= kPatchRowsMaxK ? kPatchRowsMax : 64) || s.Kp < kPatchRowsMinK) {
+    } else if (rows > (s.Kp <= kPatchRowsMaxK || !conv_table_takes(s) ? kPatchRowsMax : 64) || s.Kp < kPatchRowsMinK) {
       return 0;
     }
   }
@@ -327,7 +334,7 @@ int launch_conv_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
 }
 
 // Tiles of the implicit GEMM.  kConvGroups2/4, kConvTall2: k-split wave groups, register staging (64 x 64 and 128 x 64).
-enum ConvGemmTile { kConv64, kConvGroups2, kConvGroups4, kConvTall2, kConv128, kConv256 };
+enum ConvGemmTile { kConv64, kConvGroups2, kConvGroups4, kConvTall2, kConvRows256, kConv128, kConv256 };
 
 // The one expected to end first, by times measured on 3 x 3 layers over 176 .. 1024 channels and 49 .. 40960 pixels (us;
 // u = tiles / 256 CUs, st = stages of 64 k-bytes):
@@ -394,17 +401,36 @@ int launch_conv_gemm_tile(ConvGemmTile tile, const GemmArgs& a, const XConvTable
     case kConvTall2: return launch_conv_gemm<128, 64, 2, 2, MODE, false, 2>(a, xs, s);
     case kConv128: return launch_conv_gemm<128, 128, 2, 2, MODE, true>(a, xs, s);
     case kConv256: return launch_conv_gemm<128, 256, 2, 4, MODE, true>(a, xs, s);
+    case kConvRows256: break;
   }
   return TMQ_ERR_UNSUPPORTED;
 }
 
-// Layers the table does not take: the cursor that walks.
+// Tiles of the layers that walk (conv_table_takes).  Up to 256 tiles of 64 x 64 four wave groups (us, one group | two |
+// four: 8 x 8 over 256 channels, N = 256, 196 pixels 82 | 48 | 42, 3136 pixels 84 | 51 | 45; 11 x 11 over 32, N = 64, 6272
+// pixels 28.3 | 21.1 | 20.8), up to 512 tiles of 128 x 64 with two (9 x 9 over 48, N = 64, 25088 pixels: 26.9 against 32.0 with
+// 64 x 64 and two); beyond those, and on K short of 32 stages, 128 x 128 behind more than 64 channels (K = 4096, N = 256, 25088
+// pixels 44.6, as 64 x 64 69; K = 128, N = 256, 401408 pixels 77 | 101) and 256 x 64 for up to 64 from 65536 pixels on
+// (K = 3872, 100352 pixels 60 against 92 as 64 x 64; K = 32, N = 48: 9.1 | 11.5, 50176 pixels level).
+ConvGemmTile conv_walk_tile(int64_t M, int64_t N, int64_t stages) {
+  const int64_t t64 = ceil_div(M, 64) * ceil_div(N, 64);
+  if (stages >= 32 && t64 <= 512) return t64 <= 256 ? kConvGroups4 : kConvTall2;
+  if (N > 64) return M >= 128 * 128 || stages >= 32 ? kConv128 : kConv64;
+  return M >= 256 * 256 ? kConvRows256 : kConv64;
+}
+
 template <int MODE>
-int launch_conv_gemm_walk(const GemmArgs& a, const XConv& xs, hipStream_t s) {
-  if (a.N > 64 && a.M >= 128 * 128) return launch_conv_gemm<128, 128, 2, 2, MODE, false>(a, xs, s);
-  if (ceil_div(a.K, kBK) >= 32 && ceil_div(a.M, 64) * ceil_div(a.N, 64) <= kTwoGroupTiles)
-    return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
-  return launch_conv_gemm<64, 64, 2, 2, MODE, false>(a, xs, s);
+int launch_conv_gemm_walk(ConvGemmTile tile, const GemmArgs& a, const XConv& xs, hipStream_t s) {
+  switch (tile) {
+    case kConv64: return launch_conv_gemm<64, 64, 2, 2, MODE, false>(a, xs, s);
+    case kConvGroups2: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
+    case kConvGroups4: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 4>(a, xs, s);
+    case kConvTall2: return launch_conv_gemm<128, 64, 2, 2, MODE, false, 2>(a, xs, s);
+    case kConvRows256: return launch_conv_gemm<256, 64, 4, 1, MODE, false>(a, xs, s);
+    case kConv128: return launch_conv_gemm<128, 128, 2, 2, MODE, false>(a, xs, s);
+    case kConv256: break;
+  }
+  return TMQ_ERR_UNSUPPORTED;
 }
 
 // Patch shape and LDS layout of the halo-tiled kernel for one problem.
@@ -999,7 +1025,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   // workspace the patch rows are written out and the product runs on the linear kernels
   // (3 x 3 at 196 pixels, patch rows | implicit GEMM with its wave groups: 256 -> 256 channels 8.9 | 9.5 us, 384 -> 384
   // 10.3 | 11.8, 448 -> 448 10.4 | 15.1, 512 -> 512 16.2 | 14.2; at 480: 384 -> 384 11.8 | 11.8, 512 -> 512 17.5 | 14.3;
-  // 1024 -> 1024 at 196 26.7 | 22.3, at 49 19.8 | 21.9; 512 -> 512 at 49 14.1 | 14.0).
+  // 1024 -> 1024 at 196 26.7 | 22.3, at 49 19.8 | 21.9; 512 -> 512 at 49 14.1 | 14.0; layers that walk: 8 x 8, 256 -> 256 at
+  // 196 37.3 | 42.1, 11 x 11, 96 -> 96 at 196 29.4 | 31.8, at 784 34.5 | 32.4).
   if constexpr (MODE != kOutAcc32) {
     if (forced == 6 || forced < 0) {
       const int64_t need = po.any() || !aligned(d->x, 16) ? 0 : patch_rows_bytes(d->geom, s, forced == 6);
@@ -1157,11 +1184,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   xs.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
   xs.KH = static_cast<int>(s.KH);
   xs.chunks = static_cast<int>(s.Kp / 16);
-  // (Beyond the table's limits -- a 7 x 7 kernel over more than 334 channels, an 8 x 8 one -- the cursor that walks; also
-  // where K ends before the copies' ring of three stages is full, and where the images of a tile's 128 rows reach past
-  // the 32 bits of its offsets.)
-  const bool table = s.KH * s.KW <= kConvMaxTaps && s.Kp / 16 <= kConvMaxChunks && s.Kp > 2 * kBK &&
-                     (128 / (s.OH * s.OW) + 2) * s.H * s.W * s.IC < (int64_t{1} << 31);
+  const bool table = conv_table_takes(s);
   xs.step_w = static_cast<int>(s.dw * s.IC - 16 * (s.ICgp / 16));
   xs.step_h = static_cast<int>(s.dh * s.W * s.IC - s.KW * s.dw * s.IC);
 
@@ -1184,7 +1207,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   a.post = po;
   // (pinned for tests: tile_cols = 1, 2 or 4 wave groups, tile_rows = 128: tiles of 128 rows, 256: the 128 x 256 tile)
   const int64_t stages = ceil_div(s.Kp, kBK);
-  ConvGemmTile tile = conv_gemm_tile(rows, s.OCg, stages, po.any());
+  ConvGemmTile tile = table ? conv_gemm_tile(rows, s.OCg, stages, po.any()) : conv_walk_tile(rows, s.OCg, stages);
   if (forced == 2 && (d->tile_cols > 0 || d->tile_rows > 0)) {
     const int groups = d->tile_cols > 0 ? d->tile_cols : 1;
     if ((groups != 1 && groups != 2 && groups != 4) || stages % groups != 0) return TMQ_ERR_UNSUPPORTED;
@@ -1197,7 +1220,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     a.w_packed = static_cast<const uint8_t*>(d->w_packed) + g * s.group_bytes;
     a.n_off = static_cast<int32_t>(g * s.OCg);
     xs.ic_off = static_cast<int>(g * s.ICg);
-    rc = table ? launch_conv_gemm_tile<MODE>(tile, a, xs, stream) : launch_conv_gemm_walk<MODE>(a, xs, stream);
+    rc = table ? launch_conv_gemm_tile<MODE>(tile, a, xs, stream) : launch_conv_gemm_walk<MODE>(tile, a, xs, stream);
     if (rc != TMQ_OK) return rc;
   }
   return TMQ_OK;
