@@ -436,7 +436,9 @@ typedef struct tmq_conv2d_desc {
    * layer over at most 256 input channels with its pixels straight from memory
    * (TMQ_ERR_UNSUPPORTED when the family cannot run the problem).  tile_rows / tile_cols > 0 pin the halo
    * kernel's patch height / bound its patch width; for the implicit GEMM tile_rows = 128 pins tiles of 128
-   * rows, 256 the tile of 128 rows x 256 channels, tile_cols = 1, 2 or 4 the wave groups that share K. */
+   * rows, 256 the tile of 128 rows x 256 channels, tile_cols = 1, 2 or 4 the wave groups that share K: four with
+   * tile_rows = 0 only, none with 256, and only where they divide the 64-byte stages of K.  Any other value is
+   * TMQ_ERR_UNSUPPORTED, and so are 256 rows for a kernel of more than 63 taps or a K of at most 128. */
   int32_t kernel;
   int32_t tile_rows, tile_cols;
   int32_t reserved;

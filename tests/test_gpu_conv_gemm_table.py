@@ -106,3 +106,44 @@ def test_conv_gemm_walk(cabi, spec, x_signed):  # noqa: F811
     np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
     _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
                             c["out_zp"], relu=c["relu"], nthreads=8), "walk")
+
+
+@pytest.mark.parametrize("spec,wave_groups,tile_rows", [
+    ((1, 9, 9, 64, 64, 3, 1, 1, 1, 1), 4, 128),    # no such tile
+    ((1, 9, 9, 128, 64, 3, 1, 1, 1, 1), 2, 256),   # 128 x 256: one group
+    ((1, 9, 9, 64, 64, 3, 1, 1, 1, 1), 0, 64),     # no such height
+    ((1, 9, 9, 64, 64, 3, 1, 1, 1, 1), 0, 192),
+    ((1, 9, 9, 192, 64, 3, 1, 1, 1, 1), 3, 0),     # three groups
+    ((1, 9, 9, 64, 64, 3, 1, 1, 1, 1), 2, 0),      # nine stages
+    ((1, 9, 9, 32, 64, 9, 1, 4, 1, 1), 2, 0),      # 41, without a table
+    ((1, 9, 9, 16, 64, 8, 1, 4, 1, 1), 0, 256),    # 128 x 256 without a table
+    ((1, 9, 9, 128, 64, 1, 1, 0, 1, 1), 0, 256),
+])
+def test_conv_gemm_pins_refused(cabi, spec, wave_groups, tile_rows):  # noqa: F811
+    say("conv gemm pins refused", spec, wave_groups, tile_rows)
+    c = _conv_case(*spec, seed=sum(spec))
+    cabi.force_conv_path(2)
+    cabi.force_conv_tile(tile_rows, wave_groups)
+    try:
+        with pytest.raises(cabi.TmqError):
+            _run(cabi, c)
+    finally:
+        cabi.force_conv_path(-1)
+        cabi.force_conv_tile(0, 0)
+
+
+@pytest.mark.parametrize("wave_groups,tile_rows", [(1, 0), (2, 0), (4, 0), (2, 128), (1, 128)])
+def test_conv_gemm_walk_pinned(cabi, wave_groups, tile_rows):  # noqa: F811
+    say("conv gemm walk pinned", wave_groups, tile_rows)
+    c = _conv_case(2, 11, 12, 80, 70, 8, 1, 4, 1, 1, seed=wave_groups + tile_rows)
+    cabi.force_conv_path(2)
+    cabi.force_conv_tile(tile_rows, wave_groups)
+    try:
+        y, acc, _ = _run(cabi, c)
+    finally:
+        cabi.force_conv_path(-1)
+        cabi.force_conv_tile(0, 0)
+    args = (c["stride"], c["padding"], c["dilation"], c["groups"])
+    np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
+    _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
+                            c["out_zp"], relu=c["relu"], nthreads=8), "walk pinned")

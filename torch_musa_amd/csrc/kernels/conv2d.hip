@@ -433,6 +433,23 @@ int launch_conv_gemm_walk(ConvGemmTile tile, const GemmArgs& a, const XConv& xs,
   return TMQ_ERR_UNSUPPORTED;
 }
 
+// The tile that tmq_conv2d_desc's tile_rows and tile_cols (wave groups) pin, if they do; false when there is none such.
+// (The launch refuses what the table, or the walk, does not have.)
+bool pinned_conv_tile(int32_t tile_rows, int32_t tile_cols, int64_t stages, ConvGemmTile* tile) {
+  if (tile_rows <= 0 && tile_cols <= 0) return true;
+  const int groups = tile_cols > 0 ? tile_cols : 1;
+  if (stages % groups != 0) return false;
+  if (tile_rows <= 0 && (groups == 1 || groups == 2 || groups == 4))
+    *tile = groups == 1 ? kConv64 : groups == 2 ? kConvGroups2 : kConvGroups4;
+  else if (tile_rows == 128 && (groups == 1 || groups == 2))
+    *tile = groups == 1 ? kConv128 : kConvTall2;
+  else if (tile_rows == 256 && groups == 1)
+    *tile = kConv256;
+  else
+    return false;
+  return true;
+}
+
 // Patch shape and LDS layout of the halo-tiled kernel for one problem.
 struct TilePlan {
   int TH, TW, HH, HW, pitch, KS;
@@ -1205,17 +1222,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   a.y = out;
   a.ldy = s.OC;
   a.post = po;
-  // (pinned for tests: tile_cols = 1, 2 or 4 wave groups, tile_rows = 128: tiles of 128 rows, 256: the 128 x 256 tile)
   const int64_t stages = ceil_div(s.Kp, kBK);
   ConvGemmTile tile = table ? conv_gemm_tile(rows, s.OCg, stages, po.any()) : conv_walk_tile(rows, s.OCg, stages);
-  if (forced == 2 && (d->tile_cols > 0 || d->tile_rows > 0)) {
-    const int groups = d->tile_cols > 0 ? d->tile_cols : 1;
-    if ((groups != 1 && groups != 2 && groups != 4) || stages % groups != 0) return TMQ_ERR_UNSUPPORTED;
-    if (d->tile_rows >= 128 && groups <= 2)
-      tile = groups == 2 ? kConvTall2 : d->tile_rows == 256 ? kConv256 : kConv128;
-    else
-      tile = groups == 4 ? kConvGroups4 : groups == 2 ? kConvGroups2 : kConv64;
-  }
+  if (forced == 2 && !pinned_conv_tile(d->tile_rows, d->tile_cols, stages, &tile)) return TMQ_ERR_UNSUPPORTED;
   for (int64_t g = 0; g < s.groups; ++g) {
     a.w_packed = static_cast<const uint8_t*>(d->w_packed) + g * s.group_bytes;
     a.n_off = static_cast<int32_t>(g * s.OCg);
