@@ -147,3 +147,26 @@ def test_conv_gemm_walk_pinned(cabi, wave_groups, tile_rows):  # noqa: F811
     np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
     _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
                             c["out_zp"], relu=c["relu"], nthreads=8), "walk pinned")
+
+
+@pytest.mark.parametrize("spec", [
+    (1, 7, 9, 320, 33, 3, 1, 1, 1, 1),     # 45 stages: two wave groups, 23 and 22
+    (2, 9, 10, 448, 70, 3, 2, 2, 2, 2),    # 32 stages each (31.5) over two groups
+    (1, 8, 9, 192, 40, 7, 1, 3, 1, 1),     # 147: four, 37, 37, 37 and 36
+    (1, 7, 7, 912, 20, 3, 1, 1, 1, 1),     # 129 (128.25): 33, 32, 32 and 32
+    (5, 35, 33, 320, 130, 3, 1, 1, 1, 1),  # 45 over 128 x 64 tiles
+])
+@pytest.mark.parametrize("x_signed", [False, True])
+def test_conv_gemm_uneven_groups(cabi, spec, x_signed):  # noqa: F811
+    """Stage counts that the wave groups do not divide, by the rule's own choice."""
+    say("conv gemm uneven groups", spec, x_signed)
+    c = _conv_case(*spec, seed=sum(spec), x_signed=x_signed, relu=x_signed)
+    cabi.force_conv_path(2)
+    try:
+        y, acc, _ = _run(cabi, c)
+    finally:
+        cabi.force_conv_path(-1)
+    args = (c["stride"], c["padding"], c["dilation"], c["groups"])
+    np.testing.assert_array_equal(acc, oracle.conv2d_acc32(c["xq"], c["wq"], *args, c["x_zp"], nthreads=8))
+    _check(y, oracle.conv2d(c["xq"], c["x_scale"], c["x_zp"], c["wq"], c["w_scales"], c["bias"], *args, c["out_scale"],
+                            c["out_zp"], relu=c["relu"], nthreads=8), "uneven groups")

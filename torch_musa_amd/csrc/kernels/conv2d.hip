@@ -343,15 +343,15 @@ enum ConvGemmTile { kConv64, kConvGroups2, kConvGroups4, kConvTall2, kConvRows25
 //   128 x 256    5.0 + st (0.36 + 0.08 u for u <= 1, 0.52 + 0.23 u for u <= 2: two blocks on a CU), and per round of those;
 //                a residual or SiLU in the epilogue costs the lone block of a big tile 2 and 3.5 more
 //   128 x 64, two wave groups: 5.5 + 0.195 st for up to 256 tiles and K from 32 stages on; 64 x 64 with two: 4.3 + 0.14 st
-//                (four groups from 128 stages on: 1024 -> 1024 on 14 x 14 23.7 -> 22.3)
+//                (four groups from 128 stages on: 1024 -> 1024 on 14 x 14 23.7 -> 22.3; K = 9216, 176 tiles 23.7 -> 23.3);
+//                the groups' runs may differ by a stage (147 stages, 56 tiles: one group 33.2, two 24.5, four 24.0)
 // What the rule changed, from 64 x 64 by fewer than 16384 pixels and 128 x 128 beyond: 512 -> 512 on 9 x 33 x 30 47 -> 34,
 // on 16 x 28 x 28 62 -> 36, on 32 x 28 x 28 88 -> 67 (128 x 256); 384 -> 384 on 9 x 33 x 30 29 -> 22 (128 x 128).
 ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
   const auto tiles = [&](int64_t bm, int64_t bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
   const double st = static_cast<double>(stages), cus = 256.0;
   const int64_t t64 = tiles(64, 64);
-  if (stages >= 128 && stages % 4 == 0 && t64 <= 128) return kConvGroups4;
-  if (stages >= 32 && stages % 2 == 0 && t64 <= 256) return kConvGroups2;
+  if (stages >= 32 && t64 <= 256) return stages >= 128 ? kConvGroups4 : kConvGroups2;
   const double u64 = t64 / cus;
   double best = 4.0 + 0.25 * u64 + st * std::max(t64 <= 256 ? 0.19 : 0.24, 0.08 + 0.112 * u64);
   ConvGemmTile tile = kConv64;
@@ -361,7 +361,7 @@ ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
       tile = t;
     }
   };
-  if (stages >= 32 && stages % 2 == 0 && tiles(128, 64) <= 256) offer(kConvTall2, 5.5 + 0.195 * st);
+  if (stages >= 32 && tiles(128, 64) <= 256) offer(kConvTall2, 5.5 + 0.195 * st);
   {
     const int64_t t = tiles(128, 128), last = t % 768;
     const double u = last / cus;
