@@ -1,5 +1,5 @@
 """The implicit GEMM's k order in a table: channel blocks that do not fill a stage, strides, dilations, groups, the table's
-limits (63 taps, 16 KiB of K) and what lies beyond them, against the oracle."""
+limits (63 taps, 8128 chunks of 16 bytes) and what lies beyond them, against the oracle."""
 import numpy as np
 import pytest
 
@@ -30,8 +30,12 @@ pytestmark = pytest.mark.gpu
     ((1, 13, 10, 144, 16, 1, 1, 0, 1, 1), 0, 128),   # three stages, the copies' ring
     ((1, 13, 10, 128, 16, 1, 1, 0, 1, 1), 0, 128),   # two: the cursor
     ((1, 9, 9, 320, 64, 7, 1, 3, 1, 1), 0, 0),       # 980 chunks
-    ((1, 4, 5, 1024, 20, 4, 1, 2, 1, 1), 4, 0),      # 1024: the whole table
-    ((1, 4, 5, 1040, 20, 4, 1, 2, 1, 1), 4, 0),      # 1040: past it
+    ((1, 4, 5, 1024, 20, 4, 1, 2, 1, 1), 4, 0),      # 1024
+    ((1, 4, 5, 1040, 20, 4, 1, 2, 1, 1), 4, 0),      # 1040
+    ((1, 4, 5, 2048, 70, 3, 1, 2, 2, 1), 0, 128),    # 1152: dilated, direct copies
+    ((1, 3, 4, 8128, 20, 4, 1, 2, 1, 1), 4, 0),      # 8128: the whole table
+    ((1, 3, 4, 8128, 20, 4, 1, 2, 1, 1), 0, 256),    # ... beside the largest tile's stages
+    ((1, 3, 4, 8144, 20, 4, 1, 2, 1, 1), 4, 0),      # 8144: past it
     ((1, 9, 9, 16, 64, 8, 1, 4, 1, 1), 2, 0),        # 64 taps: past it
 ])
 @pytest.mark.parametrize("x_signed", [False, True])

@@ -23,6 +23,7 @@ namespace tmq {
 namespace {
 
 constexpr int64_t kKPad = 128;
+constexpr int64_t kCuLds = 160 * 1024;            // LDS of a CU, what blocks that run on it at once share
 constexpr int64_t kPointwiseAsLinearRows = 8192;  // pixels up to which a pointwise layer runs as a linear layer
 constexpr int64_t kPatchRowsMax = 512;           // output pixels up to which a layer may run on its patch rows (workspace)
 constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on ...
@@ -336,17 +337,23 @@ int launch_conv_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
 // Tiles of the implicit GEMM.  kConvGroups2/4, kConvTall2: k-split wave groups, register staging (64 x 64 and 128 x 64).
 enum ConvGemmTile { kConv64, kConvGroups2, kConvGroups4, kConvTall2, kConvRows256, kConv128, kConv256 };
 
-// The one expected to end first, by times measured on 3 x 3 layers over 176 .. 1024 channels and 49 .. 40960 pixels (us;
-// u = tiles / 256 CUs, st = stages of 64 k-bytes):
+// The one expected to end first, by times measured on 3 x 3 layers over 176 .. 4096 channels, 5 x 5 and 7 x 7 ones over up
+// to 1024, and 49 .. 40960 pixels (us; u = tiles / 256 CUs, st = stages of 64 k-bytes):
 //   64 x 64      4.0 + 0.25 u + st max(0.19 up to one tile per CU or else 0.24, 0.08 + 0.112 u)
-//   128 x 128    5.0 + st (0.28 for u <= 1, 0.35 + 0.1 u for u <= 2, 0.3 + 0.19 u for u <= 3: three blocks on a CU)
-//   128 x 256    5.0 + st (0.36 + 0.08 u for u <= 1, 0.52 + 0.23 u for u <= 2: two blocks on a CU), and per round of those;
-//                a residual or SiLU in the epilogue costs the lone block of a big tile 2 and 3.5 more
-//   128 x 64, two wave groups: 5.5 + 0.195 st for up to 256 tiles and K from 32 stages on; 64 x 64 with two: 4.3 + 0.14 st
-//                (four groups from 128 stages on: 1024 -> 1024 on 14 x 14 23.7 -> 22.3; K = 9216, 176 tiles 23.7 -> 23.3);
-//                the groups' runs may differ by a stage (147 stages, 56 tiles: one group 33.2, two 24.5, four 24.0)
+//   128 x 64, two wave groups: 5.5 + 0.195 st for up to 256 tiles and K from 32 stages on
+//   128 x 128    1.3, for each full round of the chip (three blocks on a CU, two or one where the table's LDS leaves no room
+//                for more) 5.0 + 0.8, 0.55 or 0.28 st, for the last one 5.0 + st (0.28 for u <= 1, 0.35 + 0.1 u for u <= 2,
+//                0.3 + 0.19 u for u <= 3)
+//   128 x 256    1.0, for each full round (two blocks on a CU or one) 5.0 + 0.9 or 0.44 st, for the last one
+//                5.0 + st (0.36 + 0.08 u for u <= 1, 0.52 + 0.23 u for u <= 2)
+//                (a residual or SiLU in the epilogue costs the lone block of a big tile 2 and 3.5 more)
+// and by tile count alone, up to 256 tiles of 64 x 64: four wave groups from 128 stages on (1024 -> 1024 on 14 x 14 23.7 with
+// two, 22.3 with four; K = 9216, 176 tiles 23.7, 23.3), two from 32 on.  The groups' runs may differ by a stage (147 stages,
+// 56 tiles: one group 33.2, two 24.5, four 24.0).
 // What the rule changed, from 64 x 64 by fewer than 16384 pixels and 128 x 128 beyond: 512 -> 512 on 9 x 33 x 30 47 -> 34,
-// on 16 x 28 x 28 62 -> 36, on 32 x 28 x 28 88 -> 67 (128 x 256); 384 -> 384 on 9 x 33 x 30 29 -> 22 (128 x 128).
+// on 16 x 28 x 28 62 -> 36, on 32 x 28 x 28 88 -> 67 (128 x 256); 384 -> 384 on 9 x 33 x 30 29 -> 22 (128 x 128).  On 90 random
+// layers with K from 10800 to 37632 and 49 to 18424 pixels it took the fastest of the six tiles each time, on 70 with an odd
+// stage count from 25 to 147 it was 1.5 % behind that one on average and 9 % at most (25 stages, where two groups are ahead).
 ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
   const auto tiles = [&](int64_t bm, int64_t bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
   const double st = static_cast<double>(stages), cus = 256.0;
@@ -362,17 +369,24 @@ ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
     }
   };
   if (stages >= 32 && tiles(128, 64) <= 256) offer(kConvTall2, 5.5 + 0.195 * st);
+  // blocks of a direct-copy tile on a CU: three stages, the channels' constants and the table
+  const auto fit = [&](int64_t rows, int64_t cols, int64_t most) {
+    const int64_t lds = 3 * kBK * (rows + cols) + 12 * cols + conv_table_bytes(static_cast<int>(stages * kChunks));
+    return std::max<int64_t>(1, std::min(most, kCuLds / lds));
+  };
   {
-    const int64_t t = tiles(128, 128), last = t % 768;
+    const int64_t n = fit(128, 128, 3), t = tiles(128, 128), last = t % (256 * n);
     const double u = last / cus;
+    const double full = n == 3 ? 0.8 : n == 2 ? 0.55 : 0.28;
     const double rate = u <= 1.0 ? 0.28 : u <= 2.0 ? 0.35 + 0.1 * u : 0.3 + 0.19 * u;
-    offer(kConv128, 1.3 + (post ? 2.0 : 0.0) + t / 768 * (5.0 + 0.8 * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
+    offer(kConv128, 1.3 + (post ? 2.0 : 0.0) + t / (256 * n) * (5.0 + full * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
   }
   {
-    const int64_t t = tiles(128, 256), last = t % 512;
+    const int64_t n = fit(128, 256, 2), t = tiles(128, 256), last = t % (256 * n);
     const double u = last / cus;
+    const double full = n == 2 ? 0.9 : 0.44;
     const double rate = u <= 1.0 ? 0.36 + 0.08 * u : 0.52 + 0.23 * u;
-    offer(kConv256, 1.0 + (post ? 3.5 : 0.0) + t / 512 * (5.0 + 0.9 * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
+    offer(kConv256, 1.0 + (post ? 3.5 : 0.0) + t / (256 * n) * (5.0 + full * st) + (last == 0 ? 0.0 : 5.0 + rate * st));
   }
   return tile;
 }
@@ -511,7 +525,6 @@ bool plan_tiles(const ConvShape& s, bool forced, int forced_rows, int forced_col
   if (w_bytes > 96 * 1024 || icb > 64) return false;
   const int64_t pitch = (icb | 1) * 16;
   const int64_t n_tiles = ceil_div(s.OCg, kCtBN);
-  constexpr int64_t kCuLds = 160 * 1024;
   // patch widths: the whole row or a power of two, and the row cut into 2..8 equal parts
   int64_t widths[14];
   int nw = 0;

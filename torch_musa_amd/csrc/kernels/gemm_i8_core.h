@@ -75,23 +75,25 @@ struct XConv {
 
 // The same with the k order in a table in LDS, one entry per 16-byte k-chunk: a stage's address is one LDS read, a bit of
 // the row's mask and two additions instead of the cursor's walk (30 vector instructions a stage and wave of a 64 x 64
-// tile for 126, beside four matrix instructions).  For kernels of at most kConvMaxTaps taps and kConvMaxChunks chunks;
+// tile for 126, beside four matrix instructions).  For kernels of at most kConvMaxTaps taps (the bits of a row's
+// mask) and kConvMaxChunks chunks (the 64 KiB of dynamic LDS that any launch may ask for; every tile has room for them);
 // XConv has no limits.  3 x 3, 256 -> 256 channels, 32 x 14 x 14: 20.2 -> 14.1 us, 32 x 28 x 28: 34.5 -> 26.8 (both with
 // the pad put in at the LDS store and the weights through the caches), with direct copies in place of registers and the
 // tiles chosen by conv_gemm_tile 13.0 and 22.0.
 struct XConvTable : XConv {
   int KH, chunks;    // kernel rows, k-chunks that carry weights
 };
-constexpr int kConvMaxTaps = 63, kConvMaxChunks = 1024;
+constexpr int kConvMaxTaps = 63, kConvMaxChunks = 8128;
 struct ConvChunk {
   int off;           // bytes from the window's corner
   int tap;           // kConvMaxTaps: no tap, outside every image
 };
 
 // The table's bytes of dynamic LDS: two stages of entries past the end of K (KCursor::seek), and three for the lanes' chunk.
-inline uint32_t conv_table_bytes(int chunks) {
-  return static_cast<uint32_t>((round_up(chunks, kChunks) + 3 * kChunks) * sizeof(ConvChunk));
+constexpr uint32_t conv_table_bytes(int chunks) {
+  return static_cast<uint32_t>(((chunks + kChunks - 1) / kChunks + 3) * kChunks * sizeof(ConvChunk));
 }
+static_assert(conv_table_bytes(kConvMaxChunks) <= 64 * 1024, "dynamic LDS without an attribute of the kernel");
 
 // Optional work between the requantisation's multiply and its rounding:
 //   t += float(accum_q - accum_zp) * amult     (quantized residual, output-scale units)
