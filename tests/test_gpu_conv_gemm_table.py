@@ -56,7 +56,7 @@ def test_conv_gemm_table(cabi, spec, wave_groups, tile_rows, x_signed):  # noqa:
 
 
 @pytest.mark.parametrize("ic,oc,height,tile_rows", [(272, 70, 9, 0), (464, 256, 17, 128), (1024, 40, 8, 256),
-                                                    (320, 320, 57, -1), (464, 300, 81, -1), (784, 64, 129, -1)])
+                                                    (304, 130, 11, -1), (320, 320, 57, -1), (464, 300, 81, -1), (784, 64, 129, -1)])
 @pytest.mark.parametrize("residual,activation", [(False, "relu"), (False, "silu"), (True, "relu"), (True, "silu")])
 def test_wide_pointwise(cabi, ic, oc, height, tile_rows, residual, activation):  # noqa: F811
     """Wide pointwise layers with residual and SiLU in the GEMM's epilogue: pinned, and (-1) by the rule's own choice."""

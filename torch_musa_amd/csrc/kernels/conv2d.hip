@@ -24,7 +24,6 @@ namespace {
 
 constexpr int64_t kKPad = 128;
 constexpr int64_t kCuLds = 160 * 1024;            // LDS of a CU, what blocks that run on it at once share
-constexpr int64_t kPointwiseAsLinearRows = 8192;  // pixels up to which a pointwise layer runs as a linear layer
 constexpr int64_t kPatchRowsMax = 512;           // output pixels up to which a layer may run on its patch rows (workspace)
 constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on ...
 constexpr int64_t kPatchRowsMaxK = 4096;         // ... up to which it may (64 pixels, or no table for the layer: any K)
@@ -391,19 +390,18 @@ ConvGemmTile conv_gemm_tile(int64_t M, int64_t N, int64_t stages, bool post) {
   return tile;
 }
 
-// Pointwise layers whose weight slice leaves the halo tiles one block on a CU, or whose SiLU they cannot hide behind
-// another block's loads (us, halo tiles | implicit GEMM).  SiLU: 320 -> 320 on 32 x 14 x 14 8.8 | 6.8, 896 -> 256 on
-// 14 x 80 x 24 44.5 | 17.6, on 32 x 56 x 56 142 | 53, 448 -> 448 there 111 | 73; level at 448 -> 448 on 5 x 23 x 27
-// (6.9 | 7.0) and behind below.  A residual alone costs the GEMM's epilogue scattered reads: 288 -> 288 on 4 x 75 x 66
-// 13.1 | 14.9, on 14 x 80 x 24 19.0 | 17.6; 448 -> 448 on 32 x 14 x 14 7.9 | 8.9, on 9 x 33 x 30 12.5 | 10.1; 512 -> 1024 on
-// 32 x 14 x 14 15.0 | 15.7, on 32 x 56 x 56 224 | 148.  Neither, and at most 64 output channels (more go to the linear
-// kernels): 1024 -> 64 on 4 x 75 x 66 11.5 | 7.6, on 32 x 56 x 56 39 | 24, but 288 -> 64 there 9.5 | 11.5.
-bool pointwise_gemm_first(const ConvShape& s, const PostOps& po) {
+// Pointwise layers over more than 256 channels: halo tiles or this kernel, by the rounds that the former's blocks take (one
+// block on a CU next to such a weight slice, so a second round is the whole chain again).  Halo time over this kernel's,
+// 240 random layers from 272 to 2048 channels, geometric mean (least .. most):
+//   residual alone           one round 0.89 (0.80 .. 0.95); two and three 1.21 (1.01 .. 1.45) from 384 channels on, 0.96
+//                            (0.81 .. 1.21) below, where four are level (1.01, 1.03) and more 1.36
+//   residual and SiLU        one round 0.97 (0.90 .. 1.06), more 1.38 (1.22 .. 1.58)
+//   SiLU                     two rounds 1.49 (1.35 .. 1.61); one: up to 150 million products 1.00 (0.95 .. 1.06), beyond 1.02
+//                            (0.93 .. 1.18; 1.09 from a billion on)
+bool pointwise_gemm_first(const ConvShape& s, const PostOps& po, int64_t halo_rounds) {
   if (s.KH != 1 || s.KW != 1 || s.groups != 1 || s.IC <= 256) return false;
-  const int64_t rows = s.B * s.OH * s.OW, products = rows * s.IC * s.OC;
-  if (po.silu) return products >= 150000000;
-  if (po.accum != nullptr) return rows >= 8192 && products >= (s.IC < 448 ? 2100000000 : 1700000000);
-  return s.IC >= 768 && s.OC <= 64 && rows >= 16384;
+  if (po.silu && po.accum == nullptr && s.B * s.OH * s.OW * s.IC * s.OC >= 150000000) return true;
+  return halo_rounds > (po.silu || s.IC >= 384 ? 1 : 4);
 }
 
 template <int MODE>
@@ -468,6 +466,7 @@ bool pinned_conv_tile(int32_t tile_rows, int32_t tile_cols, int64_t stages, Conv
 struct TilePlan {
   int TH, TW, HH, HW, pitch, KS;
   int row_slots;  // 16-byte LDS slots per halo row, padding included
+  int64_t rounds;  // of blocks, as many at once as fit the CUs' LDS
   int lds_x, lds_t, lds_tab, lds_total;
 };
 
@@ -588,6 +587,7 @@ bool plan_tiles(const ConvShape& s, bool forced, int forced_rows, int forced_col
         best->HH = static_cast<int>(HH); best->HW = static_cast<int>(HWd);
         best->pitch = static_cast<int>(pitch); best->KS = static_cast<int>(KS);
         best->row_slots = static_cast<int>(row_slots);
+        best->rounds = ceil_div(per_cu, together);
         best->lds_x = static_cast<int>(w_bytes);
         best->lds_t = static_cast<int>(w_bytes + x_bytes);
         best->lds_tab = best->lds_t + kCtWaves * kCtTBytes;
@@ -803,20 +803,20 @@ bool pointwise_rows_ok(const tmq_conv2d_geom& g, const ConvShape& s) {
          s.B * s.H * s.W <= 0x7fffff00 && s.B * s.H * s.W * s.IC >= 16 && s.OC <= 65536;
 }
 
-// Where it is ahead of everything else that runs the layer (us, it | the best other): always with a residual or SiLU
-// (batch 32, 256 -> 512 on 28 x 28 15.1 | 18.6; 128 -> 768 on 53 x 109 at batch 6 17.7 | 28.8; one image, 96 -> 576 on
-// 14 x 14 4.4 | 5.3), up to 128 input channels (batch 32: 128 -> 512 on 28 x 28 10.6 | 10.8, 96 -> 576 on 14 x 14
-// 5.3 | 6.4; one image: 64 -> 256 on 56 x 56 4.2 | 4.5), and up to 160 output channels (256 -> 64 on 56 x 56 10.9 |
-// 11.0, 144 -> 24 on one image of 57 x 43 4.2 | 4.7).  Of more of both, up to 192 input channels by the pixels: 1024 and
-// fewer (192 -> 320 on 30 x 30 3.5 | 3.7), 8192 and more (144 -> 864 on 4 x 103 x 91 17.8 | 22.8, 192 -> 320 on
-// 32 x 56 x 56 16.0 | 24.5), between them from 768 output channels on (3600: 192 -> 1152 5.5 | 6.7, but 144 -> 512 4.7 |
-// 4.3); beyond 192 from 16384 on (256 -> 256 on 32 x 56 x 56 18.5 | 22.3, 256 -> 512 on 4 x 75 x 66 9.9 | 10.9; on
-// 8 x 40 x 40 8.0 | 7.5).  The rest is the linear kernels': every wave would read the pixels again for its 64 channels.
+// Where it is ahead of everything else that runs the layer (us, it | the best other): with a residual or SiLU (batch 32,
+// 256 -> 512 on 28 x 28 15.1 | 18.6; 128 -> 768 on 53 x 109 at batch 6 17.7 | 28.8; one image, 96 -> 576 on 14 x 14 4.4 | 5.3),
+// up to 128 input channels (batch 32: 128 -> 512 on 28 x 28 10.6 | 10.8; one image: 64 -> 256 on 56 x 56 4.2 | 4.5) and up to
+// 32 output channels (144 -> 24 on one image of 57 x 43 4.2 | 4.7).  Of more of both, against the linear kernels, by the
+// pieces of 16 pixels times the blocks of 64 channels: up to 1024, one for each SIMD (208 -> 1024 on 560 pixels 3.65 | 3.9,
+// 192 -> 192 on 4899 3.5 | 3.9), and again from where the linear kernels are past what they do at once: 2048, or 3072 where
+// more than four channel blocks read the same pixels (192 -> 128 on 50176 6.9 | 7.4, 208 -> 1024 on 9792 8.7 | 11.4; in between
+// 240 -> 64 on 25088 4.65 | 4.4, 192 -> 960 on 2812 5.4 | 5.1); over 256 channels, whole 128-byte lines to the linear kernels,
+// 8192, or 4096 for one block (256 -> 512 on 4761 6.2 | 5.1, on 21312 10.8 | 11.6; 256 -> 64 on 50176 6.7 | 6.4, on 100352 8.4 |
+// 9.3).  On 570 random layers the choice is 0.1 % behind the better of the two on average and 7 % at most.
 bool pointwise_rows_first(const ConvShape& s, bool post) {
-  const int64_t pixels = s.B * s.H * s.W;
-  if (post || s.runs_KS <= 2 || s.OC <= 160) return true;
-  if (s.runs_KS == 3) return pixels <= 1024 || pixels >= 8192 || s.OC >= 768;
-  return pixels >= 16384;
+  if (post || s.runs_KS <= 2 || s.OC <= 32) return true;
+  const int64_t blocks = ceil_div(s.OC, 64), units = ceil_div(s.B * s.H * s.W, 16) * blocks;
+  return units <= 1024 || units > (s.IC == 256 ? (blocks == 1 ? 4096 : 8192) : blocks <= 4 ? 2048 : 3072);
 }
 
 // The 16-pixel pieces whose reads and stores the kernel makes without a check: all 16 pixels exist, and the last pixel's
@@ -1029,25 +1029,16 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   const int forced = d->kernel > 0 ? d->kernel : -1;
   // A pointwise layer (1 x 1, stride 1, no padding, one group) is a linear layer over the
   // pixels: rows = pixels, K = input channels, and the packed weight is the linear one
-  // (same 16-channel blocks, same k padding).  With few pixels -- the late stages of an
-  // image network -- the linear kernels' choice for short M is ahead of the halo tiles
-  // (1024 -> 256 channels on 14 x 14, batch 32: 12.8 -> 7.8 us; 512 -> 2048 on 7 x 7: 11.7 -> 7.1 us).
+  // (same 16-channel blocks, same k padding), and the linear kernels take it unless pointwise_rows_first says otherwise:
+  // over more than 256 channels the best other kernel took 1.11 to 1.5 times as long on most of 180 random layers (288 -> 64
+  // on 23326 pixels 5.0 | 4.5 us, 512 -> 64 on 20880 5.7 | 4.9, 640 -> 32 on 46176 8.5 | 6.7, 768 -> 80 on 8460 6.0 | 5.1, 1024
+  // -> 112 on 8844 7.7 | 6.0, 1024 -> 256 on 14 x 14 at batch 32 12.8 | 7.8); where it was ahead (272 -> 48 on 102144 8.7 | 9.2),
+  // by 5 % at most.
   if constexpr (MODE != kOutAcc32) {
     const bool pointwise = s.KH == 1 && s.KW == 1 && s.sh == 1 && s.sw == 1 && s.ph == 0 && s.pw == 0 &&
                            d->geom.groups == 1 && s.IC % 16 == 0 && aligned(d->x, 16) && !po.any();
     if (forced == 5 && !pointwise) return TMQ_ERR_UNSUPPORTED;
-    // (and with 128 input and 256 output channels or more from about a billion products on: 256 -> 256 on
-    // 56 x 56 at batch 32 35.9 -> 25.8 us, 512 -> 512 on 28 x 28 25.0 -> 16.1 us, 128 -> 512 13.7 -> 11.6 us; fewer
-    // channels on either side stay with the tiles: 256 -> 64 on 56 x 56 11.7 against 19.9 us, 96 -> 576 on
-    // 28 x 28 14.3 against 18.0 us)
-    // (a detection head's 255 channels count as wide: 128 -> 255 on 80 x 80 at batch 8 18.0 -> 15.2 us)
-    // (narrow outputs behind wide inputs: 768 -> 192 on 16 x 28 x 28 10.9 -> 7.3 us, on 32 x 56 x 56 69 -> 32.5, 512 -> 160
-    // there 45 -> 26, 384 -> 96 there 23.3 -> 16.3; 768 -> 192 on 9 x 33 x 30 6.7 against 7.1)
-    const int64_t products = rows * s.IC * s.OC;
-    const bool wide = (s.IC >= 128 && s.OC >= 224 && products >= 1000000000) ||
-                      (s.IC >= 384 && s.OC > 64 && products >= 1500000000);
-    if (forced == 5 || (forced < 0 && pointwise && (rows <= kPointwiseAsLinearRows || wide) &&
-                        !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, false)))) {
+    if (forced == 5 || (forced < 0 && pointwise && !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, false)))) {
       return run_as_linear(d, rows, s.OC, s.IC, d->x, relu, out, stream);
     }
   }
@@ -1155,8 +1146,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   }
 
   TilePlan plan;
-  const bool tiles_ok = forced != 2 && !(forced < 0 && pointwise_gemm_first(s, po)) &&
-                        plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan);
+  const bool tiles_ok = forced != 2 && plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan) &&
+                        !(forced < 0 && pointwise_gemm_first(s, po, plan.rounds));
   if (forced == 1 && !tiles_ok) return TMQ_ERR_UNSUPPORTED;
   if (tiles_ok) {
     ConvTileArgs t{};
