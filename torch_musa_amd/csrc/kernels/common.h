@@ -39,13 +39,6 @@ static inline bool aligned(const void* p, uintptr_t a) {
   return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 
-// Workgroups are dealt round-robin to the 8 XCDs, each with an L2 of its own: the place of block b of n in a sequence of which
-// every XCD has one contiguous run, so that neighbours share what they read, and the lines that both write, in one L2.
-__device__ static inline uint32_t xcd_contiguous(uint32_t b, uint32_t n) {
-  const uint32_t q = n / 8, rem = n % 8, xcd = b % 8;
-  return xcd * q + (xcd < rem ? xcd : rem) + b / 8;
-}
-
 __host__ __device__ static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 __host__ __device__ static inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 

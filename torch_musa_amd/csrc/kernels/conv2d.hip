@@ -861,11 +861,22 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   const int64_t nblk = ceil_div(s.OC, 16 * nt), cap = 256 * (s.runs_KS > 2 ? 2 : 3) * kCrWaves;
   int64_t groups = cap / nblk < 1 ? 1 : cap / nblk;
   if (groups > pieces) groups = pieces;
+  // groups dealt to the XCDs where some have a piece more than the rest, as many to each if that costs no further piece
+  const int64_t even = groups < 8 ? groups : groups - groups % 8;
+  const bool by_xcd = nblk >= kCrXcdBlocks, deal = by_xcd && pieces % groups != 0 && ceil_div(pieces, even) == ceil_div(pieces, groups);
+  if (deal) groups = even;
+  const int64_t blocks = deal ? 8 * ceil_div(ceil_div(groups, 8) * nblk, kCrWaves) : ceil_div(groups * nblk, kCrWaves);
   a.nblk = static_cast<int>(nblk);
   a.groups = static_cast<int>(groups);
   // (exact while waves x nblk < 2**32: at most 3072 waves, or nblk <= 2048 of them)
   a.nblk_magic = static_cast<uint32_t>(((int64_t{1} << 32) + nblk - 1) / nblk);
-  const dim3 grid(static_cast<unsigned>(ceil_div(groups * nblk, kCrWaves))), block(kCrThreads);
+  a.xcd_mask = by_xcd ? 7 : 0;
+  a.xcd_shift = by_xcd ? 3 : 0;
+  a.xcd_blocks = by_xcd && !deal ? static_cast<uint32_t>(blocks / 8) : 0;
+  a.xcd_longer = by_xcd && !deal ? static_cast<uint32_t>(blocks % 8) : 0;
+  a.deal_shift = deal ? 3 : 0;
+  a.deal_mask = deal ? 7 : 0;
+  const dim3 grid(static_cast<unsigned>(blocks)), block(kCrThreads);
   const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
     constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;
     constexpr bool kPlain = decltype(plain_tag)::value;

@@ -51,9 +51,17 @@ struct ConvRunArgs {
   int B, H, W, IC, OH, OW, OC, KH, KW;
   int sh, sw, ph, pw;
   int RL, RP, KS;            // run bytes, padded run bytes, k-steps (KH * RP <= 64 KS)
-  int TR, TW, mtw;           // output rows and columns per tile, 16-pixel pieces per tile row
-  int rows_in, pitch;        // staged image rows, LDS bytes per staged row (multiple of 16)
-  int tiles_h, tiles_w;
+  union {                    // (both sets side by side cost every pointwise layer 0.05 us more)
+    struct {
+      int TR, TW, mtw;       // output rows and columns per tile, 16-pixel pieces per tile row
+      int rows_in, pitch;    // staged image rows, LDS bytes per staged row (multiple of 16)
+      int tiles_h, tiles_w;
+    };
+    struct {                 // (pointwise) blockIdx -> XCD and place in it, blocks of an XCD's run (xcd_longer of the runs
+                             // have one more), groups dealt to the XCDs
+      uint32_t xcd_mask, xcd_shift, xcd_blocks, xcd_longer, deal_shift, deal_mask;
+    };
+  };
   int vec;                   // 16-byte (int32 mode: per 4 channels) stores are aligned
   int whole;                 // (pointwise) pieces all of whose reads and stores lie inside the tensors
   int nblk, groups;          // (pointwise) channel blocks, and waves on each of them
@@ -440,6 +448,7 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
 // a.tiles: the number of 16-pixel pieces.
 template <int KSN>
 constexpr int kCrPointwiseDepth = KSN == 1 ? 4 : 2;
+constexpr int kCrXcdBlocks = 8;  // channel blocks from which on the waves of a group of pixels sit on one XCD
 
 template <int MODE, int POST, int NT, int KSN, bool PLAIN = false>
 __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointwise_kernel(ConvRunArgs a) {
@@ -458,12 +467,15 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
   // With eight and more channel blocks the waves of one group of pixels sit in several blocks: on one XCD they share the
   // pixels' bytes and the output lines where two channel blocks meet (97 -> 582 channels on 22 x 38 x 81 34.9 -> 30.8 us,
   // 128 -> 768 on 11 x 17 x 48 8.4 -> 8.0; fewer share nothing and stream worse: 24 -> 144 at batch 32 9.9 -> 12.2, 128 ->
-  // 273 with a residual 7.3 -> 8.0).
-  const uint32_t blocks = (static_cast<uint32_t>(groups * nblk) + kCrWaves - 1) / kCrWaves;
-  const uint32_t block = nblk >= 8 ? xcd_contiguous(blockIdx.x, blocks) : blockIdx.x;
+  // 273 with a residual 7.3 -> 8.0).  Where some groups, the first ones, have a piece more than the rest, the groups are
+  // dealt to the XCDs in turn: in one run they kept one XCD busy for longer (96 -> 512 with SiLU on 2 x 59 x 59, 436 pieces
+  // for 384 groups: 8.8 -> 7.5 us).
+  const uint32_t xcd = blockIdx.x & a.xcd_mask;
+  const uint32_t block = xcd * a.xcd_blocks + (xcd < a.xcd_longer ? xcd : a.xcd_longer) + (blockIdx.x >> a.xcd_shift);
   const uint32_t w = block * kCrWaves + static_cast<uint32_t>(wave);
-  const int g = static_cast<int>(nblk == 1 ? w : __umulhi(w, a.nblk_magic));
-  const int cb = static_cast<int>(w) - g * nblk;
+  const int in_run = static_cast<int>(nblk == 1 ? w : __umulhi(w, a.nblk_magic));
+  const int cb = static_cast<int>(w) - in_run * nblk;
+  const int g = (in_run << a.deal_shift) + static_cast<int>(xcd & a.deal_mask);
   if (g >= groups || g >= a.tiles) return;  // (no barrier below: the waves share nothing)
 
   // Every request of the set-up leaves before anything is waited for, the constants first: with the bias behind a
