@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <tuple>
+#include <utility>
 
 #include "tmq.h"
 
@@ -26,7 +27,8 @@ static inline int launch_status() {
 // operator takes.  launch_status() has the outcome.
 template <class... P, class... A>
 static inline void enqueue(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A&&... args) {
-  std::tuple<P...> values(static_cast<P>(args)...);  // what the kernel's parameters are
+  // what the kernel's parameters are; braces: an argument that one of them is too narrow for does not compile
+  std::tuple<P...> values{P{std::forward<A>(args)}...};
   std::apply(
       [&](P&... v) {
         void* pointers[] = {const_cast<void*>(static_cast<const void*>(&v))..., nullptr};
