@@ -139,8 +139,11 @@ int tmq_quantize_per_tensor_dynamic_report(const float* x, void* q, int64_t n, i
                                            tmq_stream_t stream);
 /* The same, where the range may come in parts: *count of them, each the minimum (lower half) and maximum (upper half)
  * of some of the values as one word of `parts`, TMQ_HOST_PARTS words of pinned host memory that the caller has set to
- * TMQ_HOST_PART_EMPTY (two NaNs, which no part is).  *count = 0: the range goes to `report` as a whole. */
+ * TMQ_HOST_PART_EMPTY (two NaNs, which no part is).  *count = 0: the range goes to `report` as a whole, as it does
+ * wherever n is not above TMQ_HOST_PARTS_ABOVE and up to TMQ_HOST_PARTS_UP_TO. */
 #define TMQ_HOST_PARTS 64
+#define TMQ_HOST_PARTS_ABOVE 65536
+#define TMQ_HOST_PARTS_UP_TO 2097152
 #define TMQ_HOST_PART_EMPTY 0xffffffffffffffffull
 int tmq_quantize_per_tensor_dynamic_parts(const float* x, void* q, int64_t n, int q_signed,
                                           int reduce_range, int rounding, tmq_qparams* qparams,

@@ -5,6 +5,7 @@ import threading
 import pytest
 import torch
 import torch_musa_amd  # noqa: F401
+from torch_musa_amd import cabi
 
 pytestmark = pytest.mark.gpu
 
@@ -51,7 +52,7 @@ def test_dynamic_range_report(n):
 
 
 @pytest.mark.parametrize("n,offset", [
-    (98305, 0), (1 << 21, 0),                                           # reported by the range pass
+    (98305, 0), (1 << 21, 0),                                           # by each block of the range pass
     ((1 << 21) + 4, 0), ((1 << 21) + 7, 0), ((1 << 24) + 1, 0), (1 << 25, 0),  # by the quantizer's first block
     (98305, 1), ((1 << 21) + 6, 1),                                     # values off the 16-byte grid: by the pass between
 ])
@@ -66,6 +67,26 @@ def test_dynamic_range_report_by_each_pass(n, offset, dtype):
     assert torch.equal(got.int_repr().cpu(), want.int_repr())
     with pytest.raises(RuntimeError, match="min should be"):
         torch.quantize_per_tensor_dynamic(xg.fill_(float("nan")), dtype, False)
+
+
+@pytest.mark.parametrize("n,offset", [(1, 0), (65537, 0), (98304, 0),            # by the one launch
+                                      (98305, 0), (200003, 0), (1 << 21, 0),     # by the range pass's last block
+                                      ((1 << 21) + 1, 0), (98305, 1)])
+def test_range_reported_as_a_whole(n, offset):
+    """The C entry point whose range comes in one piece at every size."""
+    x = torch.randn(n, generator=torch.Generator().manual_seed(n)) * 2
+    x[n - 1], x[n // 2] = 31.0, -47.0
+    xg = torch.empty(n + offset, device="cuda")[offset:].copy_(x.cuda())
+    want = torch.quantize_per_tensor_dynamic(x, torch.quint8, False)
+    report = torch.zeros(2, dtype=torch.int64).pin_memory()
+    for ticket in (7, 8):     # the block count of the slot is ready for the next call
+        q, qp = cabi.quantize_per_tensor_dynamic_report(xg, False, False, report, ticket, 63)
+        torch.cuda.synchronize()
+        assert [w >> 32 for w in report.tolist()] == [ticket, ticket]
+        bits = torch.tensor([w & 0xffffffff for w in report.tolist()], dtype=torch.int64).to(torch.uint32)
+        assert bits.view(torch.float32).tolist() == [x.min().item(), x.max().item()]
+        assert cabi.read_qparams(qp) == (want.q_scale(), want.q_zero_point())
+        assert torch.equal(q.cpu(), want.int_repr())
 
 
 def test_dynamic_keeps_the_memory_format():

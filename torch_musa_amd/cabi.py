@@ -140,6 +140,8 @@ def lib() -> C.CDLL:
         l.tmq_linear_dynamic_small.argtypes = [C.POINTER(LinearDesc), v, C.c_int64, C.c_int, v, C.c_int64, v]
         l.tmq_linear_dynamic_small_takes.argtypes = [C.c_int64, C.c_int64, C.c_int64]
         l.tmq_quantize_per_tensor_dynamic_dev.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v]
+        l.tmq_quantize_per_tensor_dynamic_report.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v,
+                                                             C.c_uint32, C.c_uint32, v]
         l.tmq_conv2d_prepack.argtypes = [v, C.POINTER(Conv2dGeom), v, v, v]
         l.tmq_conv2d_out_hw.argtypes = [C.POINTER(Conv2dGeom), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]
         l.tmq_conv2d.argtypes = [C.POINTER(Conv2dDesc), v]
@@ -249,6 +251,21 @@ def quantize_per_tensor_dynamic_dev(x: torch.Tensor, signed: bool, reduce_range:
     check(lib().tmq_quantize_per_tensor_dynamic_dev(x.data_ptr(), q.data_ptr(), x.numel(), int(signed),
                                                     int(reduce_range), int(fused), qp.data_ptr(), ws.data_ptr(),
                                                     ws.numel(), stream_ptr()), "tmq_quantize_per_tensor_dynamic_dev")
+    return q, qp
+
+
+def quantize_per_tensor_dynamic_report(x: torch.Tensor, signed: bool, reduce_range: bool, report: torch.Tensor,
+                                       ticket: int, slot: int):
+    """As quantize_per_tensor_dynamic_dev, the range also to `report` (two int64 of pinned host memory, upper halves
+    `ticket` once they are complete)."""
+    assert x.dtype == torch.float32 and x.is_contiguous() and report.is_pinned() and report.dtype == torch.int64
+    q = torch.empty(x.shape, dtype=torch.int8 if signed else torch.uint8, device=x.device)
+    qp = torch.empty(16, dtype=torch.uint8, device=x.device)
+    ws = minmax_workspace(x.device)
+    check(lib().tmq_quantize_per_tensor_dynamic_report(x.data_ptr(), q.data_ptr(), x.numel(), int(signed),
+                                                       int(reduce_range), 0, qp.data_ptr(), ws.data_ptr(), ws.numel(),
+                                                       report.data_ptr(), ticket, slot, stream_ptr()),
+          "tmq_quantize_per_tensor_dynamic_report")
     return q, qp
 
 

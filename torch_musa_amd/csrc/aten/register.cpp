@@ -425,14 +425,23 @@ at::Tensor quantize_per_tensor_dynamic(const at::Tensor& self, at::ScalarType dt
   const at::Tensor scratch = empty_bytes(range_bytes + static_cast<int64_t>(sizeof(tmq_qparams)), x);
   auto* ws = static_cast<uint8_t*>(scratch.data_ptr());
   HostReport report(stream, what);
-  uint64_t* const parts = report.empty_parts();
+  auto* const qp = reinterpret_cast<tmq_qparams*>(ws + range_bytes);
+  const auto s = reinterpret_cast<tmq_stream_t>(stream.stream());
   int32_t count = 0;
-  report.queue([&] {
-    return tmq_quantize_per_tensor_dynamic_parts(
-        cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range, TMQ_ROUND_PRODUCT,
-        reinterpret_cast<tmq_qparams*>(ws + range_bytes), ws, static_cast<size_t>(range_bytes), report.memory(),
-        report.ticket(), report.number(), parts, &count, reinterpret_cast<tmq_stream_t>(stream.stream()));
-  });
+  if (x.numel() > TMQ_HOST_PARTS_ABOVE && x.numel() <= TMQ_HOST_PARTS_UP_TO) {
+    uint64_t* const parts = report.empty_parts();
+    report.queue([&] {
+      return tmq_quantize_per_tensor_dynamic_parts(cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range,
+                                                   TMQ_ROUND_PRODUCT, qp, ws, static_cast<size_t>(range_bytes),
+                                                   report.memory(), report.ticket(), report.number(), parts, &count, s);
+    });
+  } else {
+    report.queue([&] {
+      return tmq_quantize_per_tensor_dynamic_report(cptr<float>(x), q.data_ptr(), x.numel(), sgn, reduce_range,
+                                                    TMQ_ROUND_PRODUCT, qp, ws, static_cast<size_t>(range_bytes),
+                                                    report.memory(), report.ticket(), report.number(), s);
+    });
+  }
   float mn, mx;
   report.wait_range(count, &mn, &mx);
   report.done();

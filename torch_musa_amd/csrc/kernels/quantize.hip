@@ -371,7 +371,7 @@ __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
 // dynamic_quantize_repeat_kernel, whose blocks each read everything before the first of them reports: 32 Ki values 15.9 | 14.9,
 // 64 Ki level at 16.0, 80 Ki 15.8 | 16.9, 96 Ki 15.9 | 17.0.)
 constexpr int kPartsThreads = 1024;
-constexpr int64_t kPartsMin = int64_t{1} << 16, kPartsMax = int64_t{1} << 21;
+constexpr int64_t kPartsMin = TMQ_HOST_PARTS_ABOVE, kPartsMax = TMQ_HOST_PARTS_UP_TO;
 __global__ __launch_bounds__(kPartsThreads) void minmax_parts_kernel(const v4f* __restrict__ x4, int32_t n4,
                                                                      const float* __restrict__ x, int32_t n,
                                                                      float* __restrict__ partials, uint64_t* parts) {
