@@ -1368,12 +1368,16 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
 // More than 16 rows off the 16-byte grid: 64 x 64 tiles that read the rows where they lie, or a copy
 // onto the grid and the padded shape's own kernel.  The copy is a launch (2.2 us and a scratch
 // allocation); the larger tiles it opens earn that back from 512 tiles on, later where K is short
-// (us, direct | copy: M = 517: K = 1000, N = 2051 7.9 | 10.1, K = 2051, N = 1000 8.8 | 11.4; K = 3907,
-// N = 193, M = 2889 12.7 | 23.8; K = 4100, N = 3900, M = 500 (488 tiles) 21.1 | 24.4; K = 2051, N = 2051,
-// M = 1000 (528) 18.2 | 16.9; K = 700, N = 2000: M = 2048 (1024) 10.1 | 10.7; K = 1500, N = 2000, M = 2000
-// (1024) 19.6 | 16.4; K = 500, N = 2000, M = 3000 (1504) 12.5 | 12.2; K = 100, N = 1000, M = 8000 (2000)
-// 10.1 | 12.9; K = 120, N = 8000, M = 4096 (8000) 26.6 | 22.9).  Rows few enough for the streaming kernel
-// keep it (M = 40, K = 4100, N = 512 12.0 | 10.6).
+// (us, direct | copy, weights in the caches: M = 517: K = 1000, N = 2051 8.1 | 9.8, K = 2051, N = 1000 9.3 | 10.7; K = 3907,
+// N = 193, M = 2889 13.6 | 25.3; K = 4100, N = 3900, M = 500 (488 tiles) 22.6 | 23.9; K = 2051, N = 2051, M = 1000 (528)
+// 19.4 | 18.6; K = 1480, N = 5664, M = 611 (890) 18.9 | 14.7; K = 700, N = 2000, M = 2048 (1024) 11.3 | 12.6; K = 741,
+// N = 3952, M = 1560 (1550) 21.4 | 14.8; K = 500, N = 2000, M = 3000 (1504) 12.8 | 12.3; K = 100, N = 1000, M = 8000 (2000)
+// 10.4 | 12.8; K = 120, N = 8000, M = 4096 (8000) 26.3 | 22.1).  Few outputs leave the copy behind further on (K = 1204,
+// N = 646, M = 2983, 517 tiles, 11.3 | 14.9).  Few rows against K beyond 1200 have kernels on the grid that make up for it
+// on the device (M = 67, N = 2383, K = 2901 11.1 | 9.0, M = 40, N = 1308, K = 1413 7.7 | 6.8), but not on the host, which
+// takes longer over the copy's launch and memory than the device gains: two layers, quantize and dequantize, M = 67,
+// 2901 -> 2383 -> 1001 25.1 | 25.0, M = 40, 1413 -> 1308 -> 1413 18.7 | 25.4, M = 109, 3298 -> 74 -> 3298 20.3 | 24.5.  Rows few
+// enough for the streaming kernel keep it (M = 40, K = 4100, N = 512: 10.5).
 bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
   if (K < 16 || K > 0x7fffff00) return false;
   if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return false;
