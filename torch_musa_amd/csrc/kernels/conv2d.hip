@@ -24,9 +24,8 @@ namespace {
 
 constexpr int64_t kKPad = 128;
 constexpr int64_t kCuLds = 160 * 1024;            // LDS of a CU, what blocks that run on it at once share
-constexpr int64_t kPatchRowsMax = 512;           // output pixels up to which a layer may run on its patch rows (workspace)
-constexpr int64_t kPatchRowsMinK = 2048;         // and the K from which on ...
-constexpr int64_t kPatchRowsMaxK = 4096;         // ... up to which it may (64 pixels, or no table for the layer: any K)
+constexpr int64_t kPatchRowsMinK = 2048;         // K from which on a layer may run on its patch rows (workspace) ...
+constexpr int64_t kPatchRowsMaxK = 4096;         // ... and up to which it may at more pixels (patch_rows_max)
 inline int64_t packed_kchunks(int64_t K) { return (K + kKPad - 1) / kKPad * (kKPad / 16); }
 
 struct ConvShape {
@@ -199,6 +198,12 @@ __global__ __launch_bounds__(256) void conv_patch_rows_kernel(const uint8_t* __r
   *reinterpret_cast<v4i*>(rows + id * 16) = v;
 }
 
+// Output pixels up to which a layer's patch rows are ahead of the implicit GEMM (run_conv has the figures).
+int64_t patch_rows_max(const ConvShape& s) {
+  const bool short_k = s.Kp <= kPatchRowsMaxK;
+  return conv_table_takes(s) ? (short_k ? 512 : 64) : (short_k ? 1024 : 512);
+}
+
 // Whether a layer may run on its patch rows, and the bytes they take: one group over whole
 // 16-channel blocks, few output pixels, a long K, and no halo tiles for it.
 int64_t patch_rows_bytes(const tmq_conv2d_geom& g, const ConvShape& s, bool pinned) {
@@ -214,7 +219,7 @@ int64_t patch_rows_bytes(const tmq_conv2d_geom& g, const ConvShape& s, bool pinn
       // 1024 -> 2048: 9.9 -> 8.8 us; 256 -> 512 on 56 x 56 level at batch 32 and behind at batch 8, 8.8 against 9.4 us).
       // (eight images, 512 -> 1024 on 28 x 28: 9.0 against 7.9 us on the implicit GEMM)
       if (s.IC < 512 || rows * s.IC * s.OC < (s.IC >= 1024 ? 500000000 : 2000000000)) return 0;
-    } else if (rows > (s.Kp <= kPatchRowsMaxK || !conv_table_takes(s) ? kPatchRowsMax : 64) || s.Kp < kPatchRowsMinK) {
+    } else if (rows > patch_rows_max(s) || s.Kp < kPatchRowsMinK) {
       return 0;
     }
   }
@@ -1058,7 +1063,8 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   // (3 x 3 at 196 pixels, patch rows | implicit GEMM with its wave groups: 256 -> 256 channels 8.9 | 9.5 us, 384 -> 384
   // 10.3 | 11.8, 448 -> 448 10.4 | 15.1, 512 -> 512 16.2 | 14.2; at 480: 384 -> 384 11.8 | 11.8, 512 -> 512 17.5 | 14.3;
   // 1024 -> 1024 at 196 26.7 | 22.3, at 49 19.8 | 21.9; 512 -> 512 at 49 14.1 | 14.0; layers that walk: 8 x 8, 256 -> 256 at
-  // 196 37.3 | 42.1, 11 x 11, 96 -> 96 at 196 29.4 | 31.8, at 784 34.5 | 32.4).
+  // 196 37.3 | 42.1, 11 x 11, 96 -> 96 at 196 29.4 | 31.8, at 784 34.5 | 32.4; 11 x 11, 32 -> 64 at 784 11.7 | 20.0, at 3136
+  // 21.3 | 20.6, 8 x 8, 64 -> 256 at 784 15.0 | 16.0, at 1568 18.3 | 16.3).
   if constexpr (MODE != kOutAcc32) {
     if (forced == 6 || forced < 0) {
       const int64_t need = po.any() || !aligned(d->x, 16) ? 0 : patch_rows_bytes(d->geom, s, forced == 6);
