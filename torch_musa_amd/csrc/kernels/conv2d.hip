@@ -1163,7 +1163,9 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   }
 
   TilePlan plan;
-  const bool tiles_ok = forced != 2 && plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan) &&
+  // (what needs no plan first: that takes the host 0.5 to 3 us)
+  const bool tiles_ok = forced != 2 && !(forced < 0 && pointwise_gemm_first(s, po, 0)) &&
+                        plan_tiles(s, forced == 1, d->tile_rows, d->tile_cols, &plan) &&
                         !(forced < 0 && pointwise_gemm_first(s, po, plan.rounds));
   if (forced == 1 && !tiles_ok) return TMQ_ERR_UNSUPPORTED;
   if (tiles_ok) {
