@@ -54,6 +54,7 @@ def test_pieces(cabi, height, width, ic, oc, x_signed, offset):  # noqa: F811
 
 @pytest.mark.parametrize("ic,oc,height,width", [(24, 512, 1, 17), (24, 513, 9, 31), (100, 1030, 40, 41),  # eight channel blocks and more
                                                 (96, 512, 59, 118), (16, 570, 73, 75),  # ... a piece more for some groups
+                                                (16, 24576, 7, 19), (16, 32770, 5, 23),  # eight groups, and five
                                                 (192, 320, 30, 30), (144, 768, 40, 45), (150, 190, 91, 91),  # three k-steps
                                                 (200, 200, 128, 128), (256, 330, 127, 129), (256, 512, 33, 31)])  # four
 def test_many_blocks_and_choice(cabi, ic, oc, height, width):  # noqa: F811

@@ -867,8 +867,9 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   int64_t groups = cap / nblk < 1 ? 1 : cap / nblk;
   if (groups > pieces) groups = pieces;
   // groups dealt to the XCDs where some have a piece more than the rest, as many to each if that costs no further piece
-  const int64_t even = groups < 8 ? groups : groups - groups % 8;
-  const bool by_xcd = nblk >= kCrXcdBlocks, deal = by_xcd && pieces % groups != 0 && ceil_div(pieces, even) == ceil_div(pieces, groups);
+  const bool by_xcd = nblk >= kCrXcdBlocks;
+  const int64_t even = groups - groups % 8;
+  const bool deal = by_xcd && groups >= 8 && pieces % groups != 0 && ceil_div(pieces, even) == ceil_div(pieces, groups);
   if (deal) groups = even;
   const int64_t blocks = deal ? 8 * ceil_div(ceil_div(groups, 8) * nblk, kCrWaves) : ceil_div(groups * nblk, kCrWaves);
   a.nblk = static_cast<int>(nblk);
@@ -1061,7 +1062,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
   // Few output pixels against a long K and a weight slice the halo tiles cannot hold: with a
   // workspace the patch rows are written out and the product runs on the linear kernels
   // (3 x 3 at 196 pixels, patch rows | implicit GEMM with its wave groups: 256 -> 256 channels 8.9 | 9.5 us, 384 -> 384
-  // 10.3 | 11.8, 448 -> 448 10.4 | 15.1, 512 -> 512 16.2 | 14.2; at 480: 384 -> 384 11.8 | 11.8, 512 -> 512 17.5 | 14.3;
+  // 10.3 | 11.8, 448 -> 448 10.4 | 13.3, 512 -> 512 16.2 | 14.2; at 480: 384 -> 384 11.8 | 11.8, 512 -> 512 17.5 | 14.3;
   // 1024 -> 1024 at 196 26.7 | 22.3, at 49 19.8 | 21.9; 512 -> 512 at 49 14.1 | 14.0; layers that walk: 8 x 8, 256 -> 256 at
   // 196 37.3 | 42.1, 11 x 11, 96 -> 96 at 196 29.4 | 31.8, at 784 34.5 | 32.4; 11 x 11, 32 -> 64 at 784 11.7 | 20.0, at 3136
   // 21.3 | 20.6, 8 x 8, 64 -> 256 at 784 15.0 | 16.0, at 1568 18.3 | 16.3).

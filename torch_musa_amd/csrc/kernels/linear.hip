@@ -1122,10 +1122,11 @@ bool onepass_wide_preferred(int64_t M, int64_t N, int64_t K) {
 
 // Tiles of products over K <= kRoundsMaxK by the time their rounds take (us, u = tiles / 256 CUs, st = stages of 64 k-bytes):
 //   start + round max(floor, by_u u) + full rounds of `on_cu` tiles per CU at fill + rate st each, start holding the fill of
-// the last one: per_u u and max(floor, rate0 + rate1 u) st.  The constants are fitted to 1100 shapes drawn over M = 24 .. 110000,
-// N = 64 .. 12288 and K = 64 .. 3600 (weights in the cache of the memory side; mean error 5 to 7 %); the tile they name is 2 %
-// behind the best of all kernels on average, where the thresholds below, fitted to few sizes, are 11 % behind (14 % at
-// K <= 128).  Gained (us): M = 603, N = 2304, K = 768 6.1 -> 5.3 (64 x 64 copies for 64 x 128 with all of K in LDS);
+// the last one: per_u u and max(floor, rate0 + rate1 u) st.  The constants are fitted to shapes drawn over M = 24 .. 110000,
+// N = 64 .. 12288 and K = 64 .. 3600 (weights in the cache of the memory side; mean error 5 to 7 %), because the thresholds
+// below, fitted to few sizes, miss by a tenth between those.  On 43 shapes with K from 64 to 3584 and weights from memory the
+// tile they name is 1.5 % behind the best of all kernels on average, 17 % at most (M = 783, N = 1856, K = 3584 19.5 against
+// 16.7 us for 128 x 64; M = 8000, N = 1000, K = 128 9.5 | 8.1 for 64 x 128).  Gained (us): M = 603, N = 2304, K = 768 6.1 -> 5.3 (64 x 64 copies for 64 x 128 with all of K in LDS);
 // M = 642, N = 2304, K = 1920 12.1 -> 8.6, M = 2417, N = 832, K = 1344 9.4 -> 7.8 (for 128 x 128); M = 1690, N = 2616,
 // K = 112 8.3 -> 6.5 (64 x 64 for 128 x 128 by registers); weights from memory, M = 460, N = 1728, K = 960 8.0 -> 6.0.
 struct TileRate {
