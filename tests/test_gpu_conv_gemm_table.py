@@ -91,6 +91,7 @@ def test_wide_pointwise(cabi, ic, oc, height, tile_rows, residual, activation): 
     (2, 10, 9, 64, 70, 9, 2, 4, 1, 2),         # the same over two groups
     (1, 6, 7, 32, 33, 8, 1, 6, 2, 1),          # 32 stages, windows reaching past the image on all sides
     (5, 36, 34, 32, 130, 8, 1, 3, 1, 1),       # 5775 pixels x 130 channels: 128 x 64 tiles, two groups of 16 stages
+    (5, 36, 34, 32, 130, 9, 1, 4, 1, 1),       # the same of 21 and 20
     (1, 40, 52, 48, 72, 9, 1, 4, 1, 1),        # 61 stages
     (1, 30, 31, 16, 40, 8, 1, 4, 1, 1),        # 16 stages: one group
     (1, 129, 130, 32, 70, 1, 1, 0, 1, 1),      # one stage, 128 x 128 tiles
