@@ -1,5 +1,6 @@
-"""Pointwise convolutions over inputs of more than 2 GiB and 4 GiB: the same bytes as the same images in batches that
-stay below 2 GiB (whose results the other tests compare with the oracle)."""
+"""Inputs past the lines that a size draws: the same bytes as the same input in smaller pieces (whose results the other
+tests compare with the oracle).  Pointwise convolutions over more than 2 GiB and 4 GiB; the quantizer on either side of
+the codes that it still writes with ordinary stores."""
 import numpy as np
 import pytest
 import torch
@@ -42,3 +43,15 @@ def test_pointwise_beyond_32_bits(batch, channels, residual):
         hi = min(lo + step, batch)
         assert torch.equal(whole[lo:hi], run(lo, hi)), (lo, hi)
     assert whole[0].unique().numel() > 100
+
+
+@pytest.mark.parametrize("n", [2**28, 2**28 + 4, 2**28 + 1031])
+@pytest.mark.parametrize("dtype", [torch.quint8, torch.qint8])
+def test_quantize_around_a_cache_of_codes(n, dtype):
+    say("quantize", n, dtype)
+    gen = torch.Generator("cuda").manual_seed(n % 9973)
+    x = torch.randn(n, device="cuda", generator=gen)
+    whole = torch.quantize_per_tensor(x, 0.03, 5, dtype).int_repr()
+    cut = 2**27 + 12  # off the blocks' grid
+    assert torch.equal(whole[:cut], torch.quantize_per_tensor(x[:cut], 0.03, 5, dtype).int_repr())
+    assert torch.equal(whole[cut:], torch.quantize_per_tensor(x[cut:], 0.03, 5, dtype).int_repr())

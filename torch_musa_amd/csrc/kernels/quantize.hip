@@ -133,15 +133,17 @@ __device__ __forceinline__ void report_range(const RangeReport& r, float mn, flo
 // The fp32 input is read once and never again: non-temporal loads keep it out of
 // the caches.  The codes are written with ordinary stores, so a consumer that
 // follows on the stream (dequantize, a GEMM) finds them in the last-level cache --
-// unless there are more of them than that cache holds (STREAM_OUT, 128 MiB and
-// up): then they leave with non-temporal stores as well (2**28 elements into a
-// different output buffer every launch: 211 -> 205.5 us).
+// unless there are more of them than that cache has bytes, 256 Mi: then they leave
+// with non-temporal stores as well (STREAM_OUT).  Quantize and dequantize of 2**28
+// values, us, non-temporal | ordinary: 407 | 375 with one buffer of codes call after
+// call, 405 | 386 with three in turn (2**27: 204 | 195; the quantizer by itself,
+// three buffers: 199 | 208); of 1.5 * 2**28: 606 | 640, 2**29: 808 | 853.
 // Blocks of two waves, as for the dequantizer below: of 128 / 256 / 512 threads with two
 // or four accesses each, two waves x two accesses moved 2**28 elements fastest (213 us
 // against 219-225 us in one run).
 constexpr int kQThreads = 128;
 
-constexpr int64_t kStreamOutCodes = int64_t{1} << 27;
+constexpr int64_t kStreamOutCodes = int64_t{1} << 28;  // the last-level cache, in bytes
 template <bool SIGNED, bool FUSED = false, bool STREAM_OUT = false>
 __global__ __launch_bounds__(kQThreads) void quantize_vec_kernel(
     const v4f* __restrict__ x4, uint32_t* __restrict__ q4, int64_t n4,
@@ -192,10 +194,11 @@ __global__ __launch_bounds__(kThreads) void quantize_scalar_kernel(
 // the last-level cache from the kernel that produced them); the fp32 output is
 // four times larger and streams out with non-temporal stores so that it does
 // not evict them.
-// Blocks of two waves: the kernel is bound by the write stream (four of every
-// five bytes; a plain 1 GiB fill reaches 4.5-5 TB/s on this part), and of the
+// Blocks of two waves: the kernel is bound by the mix of reads and writes at memory (6.5 TB/s of both, 7.1 where the codes
+// are still in the last-level cache; a fill of 1 GiB 6.6), and of the
 // block sizes 64 ... 1024 two waves with two accesses per thread sustained the
-// most over 2**28 elements (204.8 us against 210-240 us for the others).
+// most over 2**28 elements (204.8 us against 210-240 us for the others).  Stores past the L2s (sc1 nt) with four waves
+// take 3 to 6 % off this kernel alone and add up to a fifth to the quantizer beside it; persistent blocks are behind.
 constexpr int kDqThreads = 128;
 
 template <bool SIGNED>
@@ -1177,7 +1180,7 @@ int quantize_launch_as(const float* x, void* q, int64_t n, QParamsArg qp, hipStr
     const int64_t n4 = n / 4;
     const int64_t blocks = n4 == 0 ? 1 : ceil_div(n4, kQThreads * kUnrollQD);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
-    if (n >= kStreamOutCodes)
+    if (n > kStreamOutCodes)
       enqueue(quantize_vec_kernel<SIGNED, FUSED, true>, dim3(blocks), dim3(kQThreads), 0, s,
               reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
     else
