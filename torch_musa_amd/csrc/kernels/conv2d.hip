@@ -729,6 +729,36 @@ bool plan_runs(const ConvShape& s, int forced_rows, RunPlan* p) {
   return best >= 0;
 }
 
+// Which layers' stores the L2s pass on at once (st16_through).  Off the 16-channel grid the lines are written in parts by
+// different instructions, and each part goes to memory by itself (24 -> 40 channels on 32 x 56 x 56 5.9 -> 10.3 us).
+int64_t out_bytes(const ConvShape& s) { return s.B * s.OH * s.OW * s.OC; }
+bool lanes_on_grid(const ConvShape& s, const void* out) { return aligned(out, 16) && s.OC % (s.OC <= 32 ? 8 : 16) == 0; }
+// From an image, of any size (us without | with them: 3 -> 64, 7 x 7, [32, 3, 224, 224] 19.4 | 15.9, one image 5.2 | 4.9;
+// 3 -> 32, 3 x 3, 12.6 | 9.4 and 4.2 | 4.0).
+bool image_through(const ConvShape& s, const void* out) { return lanes_on_grid(s, out); }
+// Pointwise rows: 64 -> 64 with a residual 6.4 MB 8.2 | 6.6, 64 -> 128 12.8 MB 13.1 | 10.0, 256 -> 128 12.5 | 10.7.  Where the
+// lines leave the L2s during the kernel anyway, past 20 MB, those that several CUs write leave more than once (64 -> 384
+// 38.5 MB 14.4 | 15.3); not so where a pixel's channel blocks are one CU's (64 -> 256 25.7 MB 15.2 | 14.4, 24 -> 512 19.7 |
+// 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6; 256 -> 384 23.3 | 21.9).  Blocks that
+// begin inside a line, past 12 MB (24 -> 112 11.2 MB 9.6 | 6.2, 24 -> 144 14.5 MB 9.9 | 11.2, 144 -> 864 18.3 MB 13.3 | 15.0).
+bool pointwise_through(const ConvShape& s, bool silu, const void* out) {
+  const int64_t bytes = out_bytes(s);
+  const bool lines = s.OC % 64 == 0;
+  return lanes_on_grid(s, out) &&
+         (silu || bytes <= int64_t{lines ? 20 : 12} << 20 || s.OC % 256 == 0 || (lines && s.runs_KS > 2));
+}
+// Halo tiles: a block has 64 channels of its pixels.  64 -> 64 on 32 x 56 x 56 11.6 | 10.2, on 16 x 56 x 56 7.2 | 6.7, one
+// image 5.2 | 5.1; where other blocks write the rest of a line, up to 8 MB (96 channels 4.8 MB 11.3 | 9.7, 9.6 MB 16.8 | 17.4).
+bool tiles_through(const ConvShape& s, const void* out) {
+  return aligned(out, 16) && s.OC % 16 == 0 && (s.OC <= 64 || s.OC % 64 == 0 || out_bytes(s) <= int64_t{8} << 20);
+}
+// Depthwise, four bytes a lane: 96 channels on 4 x 56 x 56 1.2 MB 4.9 | 5.4, 60 on 32 x 56 x 56 6 MB 10.0 | 8.4, 144 on
+// 16 x 56 x 56 7.2 MB 11.1 | 9.6, 192 on 32 x 56 x 56 19.3 MB 15.3 | 15.8.
+bool depthwise_through(const ConvShape& s, const void* out) {
+  const int64_t bytes = out_bytes(s);
+  return aligned(out, 4) && s.OC % 4 == 0 && bytes >= int64_t{9} << 19 && bytes <= int64_t{16} << 20;
+}
+
 template <int MODE>
 int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan& p, const PostOps& po, float zp_f,
                      float lo_f, float hi_f, void* out, hipStream_t stream) {
@@ -751,7 +781,10 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
   a.tiles_h = static_cast<int>(ceil_div(s.OH, p.TR));
   a.tiles_w = static_cast<int>(ceil_div(s.OW, p.TW));
   a.tiles = static_cast<int32_t>(s.B * a.tiles_h * a.tiles_w);
-  a.vec = aligned(out, 16) && s.OC % (MODE == kOutAcc32 ? 4 : 16) == 0 ? 1 : 0;
+  if constexpr (MODE == kOutAcc32)
+    a.vec = aligned(out, 16) && s.OC % 4 == 0 ? 1 : 0;
+  else
+    a.through = (s.pixels4 ? image_through(s, out) : pointwise_through(s, po.silu, out)) ? 1 : 0;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
   a.x_xor = d->x_signed ? 0u : 0x80808080u;
   a.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
@@ -851,7 +884,10 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.RL = static_cast<int>(s.runs_RL); a.RP = static_cast<int>(s.runs_RP); a.KS = static_cast<int>(s.runs_KS);
   const int64_t pieces = ceil_div(s.B * s.H * s.W, 16);
   a.tiles = static_cast<int32_t>(pieces);
-  a.vec = aligned(out, 16) && s.OC % (MODE == kOutAcc32 ? 4 : 16) == 0 ? 1 : 0;
+  if constexpr (MODE == kOutAcc32)
+    a.vec = aligned(out, 16) && s.OC % 4 == 0 ? 1 : 0;
+  else
+    a.through = pointwise_through(s, po.silu, out) ? 1 : 0;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
   a.x_xor = d->x_signed ? 0u : 0x80808080u;
   a.acc_coef = (d->x_signed ? 0 : 128) - d->x_zero_point;
@@ -958,16 +994,22 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
   const int64_t blocks = s.B * blocks_per_image;
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kDwThreads);
-  const auto launch = [&](auto post_tag) {
-    constexpr bool kP = decltype(post_tag)::value;
+  const auto launch_as = [&](auto post_tag, auto through_tag) {
+    constexpr bool kP = decltype(post_tag)::value, kThrough = decltype(through_tag)::value;
     if (s.KH == 3 && s.KW == 3)
-      enqueue(conv_depthwise_kernel<MODE, kP, 3>, grid, block, 0, stream, a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 3, kThrough>, grid, block, 0, stream, a);
     else if (s.KH == 5 && s.KW == 5)
-      enqueue(conv_depthwise_kernel<MODE, kP, 5>, grid, block, 0, stream, a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 5, kThrough>, grid, block, 0, stream, a);
     else if (s.KH == 7 && s.KW == 7)
-      enqueue(conv_depthwise_kernel<MODE, kP, 7>, grid, block, 0, stream, a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 7, kThrough>, grid, block, 0, stream, a);
     else
-      enqueue(conv_depthwise_kernel<MODE, kP, 0>, grid, block, 0, stream, a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 0, false>, grid, block, 0, stream, a);
+  };
+  const auto launch = [&](auto post_tag) {
+    if constexpr (MODE != kOutAcc32) {
+      if (depthwise_through(s, out)) return launch_as(post_tag, std::true_type{});
+    }
+    launch_as(post_tag, std::false_type{});
   };
   if constexpr (MODE != kOutAcc32) {
     if (po.any()) {
@@ -1193,6 +1235,7 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     t.tiles_h = static_cast<int>(ceil_div(s.OH, plan.TH));
     t.tiles_w = static_cast<int>(ceil_div(s.OW, plan.TW));
     t.lds_x = plan.lds_x; t.lds_t = plan.lds_t; t.lds_tab = plan.lds_tab;
+    t.through = MODE != kOutAcc32 && tiles_through(s, out) ? 1 : 0;
     t.w_scale_stride = d->w_per_channel ? 1 : 0;
     t.x_xor = d->x_signed ? 0u : 0x80808080u;
     t.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));

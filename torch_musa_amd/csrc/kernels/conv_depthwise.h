@@ -84,7 +84,8 @@ __device__ __forceinline__ void transpose_4x4_bytes(uint32_t a0, uint32_t a1, ui
 // the image still loads -- from row 0 / column 0 of the lane's image in its place, so that no
 // load sits behind a branch -- and the zero point replaces what came back, chosen by bits (a
 // select would let the compiler move the load behind a branch again).
-template <int MODE, bool POST, int KS>
+// THROUGH: bytes on the 4-byte grid leave past the L2 (a branch on that in the row loop costs 0.6 of 6.4 us).
+template <int MODE, bool POST, int KS, bool THROUGH>
 __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_depthwise_kernel(DepthwiseArgs a) {
   const uint32_t b = blockIdx.x / a.blocks_per_image;
   const uint32_t q0 = (blockIdx.x - b * a.blocks_per_image) * kDwThreads, q = q0 + threadIdx.x;
@@ -180,7 +181,9 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
       } else {
         packed = requant4<MODE, true, 2>(acc, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);  // (tested here: 11.8 -> 10.8 us where it holds, level where not)
       }
-      reinterpret_cast<DwWord*>(static_cast<uint8_t*>(a.y) + yoff)->v = packed;
+      uint8_t* const dst = static_cast<uint8_t*>(a.y) + yoff;
+      if constexpr (THROUGH) st4_through(dst, packed);
+      else reinterpret_cast<DwWord*>(dst)->v = packed;
     }
     yoff += ystep;
   };

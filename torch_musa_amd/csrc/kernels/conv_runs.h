@@ -62,7 +62,10 @@ struct ConvRunArgs {
       uint32_t xcd_mask, xcd_shift, xcd_blocks, xcd_longer, deal_shift, deal_mask;
     };
   };
-  int vec;                   // 16-byte (int32 mode: per 4 channels) stores are aligned
+  union {
+    int vec;                 // (int32 outputs) 16-byte stores per 4 channels are aligned
+    int through;             // (bytes) the stores of whole lanes are st16_through / st8_through
+  };
   int whole;                 // (pointwise) pieces all of whose reads and stores lie inside the tensors
   int nblk, groups;          // (pointwise) channel blocks, and waves on each of them
   uint32_t nblk_magic;       // w / nblk = (w * nblk_magic) >> 32 for the waves w of the launch (nblk > 1)
@@ -159,15 +162,19 @@ __device__ __forceinline__ void runs_requant(const ConvRunArgs& a, const v4i (&a
     }
   }
 }
-// One store of a lane's 4 NT bytes, at any alignment (the same instruction as an aligned one).
+// One store of a lane's 4 NT bytes, at any alignment (the same instruction as an aligned one); through: see common.h, dst
+// on the grid of 4 NT bytes.
 template <int NT>
-__device__ __forceinline__ void runs_store(uint8_t* dst, const uint32_t (&packed)[NT]) {
+__device__ __forceinline__ void runs_store(uint8_t* dst, const uint32_t (&packed)[NT], bool through) {
   if constexpr (NT == 4) {
-    st16_any(dst, v4i{static_cast<int>(packed[0]), static_cast<int>(packed[1]), static_cast<int>(packed[2]),
-                      static_cast<int>(packed[3])});
+    const v4i v = {static_cast<int>(packed[0]), static_cast<int>(packed[1]), static_cast<int>(packed[2]),
+                   static_cast<int>(packed[3])};
+    if (through) st16_through(dst, v);
+    else st16_any(dst, v);
   } else {
     static_assert(NT == 2, "channel tiles per block: 2 or 4");
-    st8_any(dst, v2i{static_cast<int>(packed[0]), static_cast<int>(packed[1])});
+    if (through) st8_through(dst, (static_cast<uint64_t>(packed[1]) << 32) | packed[0]);
+    else st8_any(dst, v2i{static_cast<int>(packed[0]), static_cast<int>(packed[1])});
   }
 }
 // A lane at the end of the channels, `left` of whose 4 NT exist: a word where four do, else bytes.
@@ -206,7 +213,7 @@ __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v
     runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult_cb, bdiv_cb, bmul, accw, packed);
     uint8_t* const dst = static_cast<uint8_t*>(a.y) + off;
     if (cb + kLaneCh <= a.OC)
-      runs_store<NT>(dst, packed);
+      runs_store<NT>(dst, packed, a.through != 0);
     else
       runs_store_some<NT>(dst, packed, a.OC - cb);
   }
@@ -600,7 +607,7 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
       uint8_t* const dst = static_cast<uint8_t*>(a.y) + base;
       if constexpr (decltype(all_ch_tag)::value) {
         runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
-        runs_store<NT>(dst + yo, packed);
+        runs_store<NT>(dst + yo, packed, a.through != 0);
       } else {
         if (residual && over > 0 && over < kLaneCh) {
           v4i v = {0, 0, 0, 0};
@@ -612,7 +619,7 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
         }
         runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
         if (over <= 0)
-          runs_store<NT>(dst + yo, packed);
+          runs_store<NT>(dst + yo, packed, a.through != 0);
         else if (over < kLaneCh)
           runs_store_some<NT>(dst + yo, packed, kLaneCh - over);
       }

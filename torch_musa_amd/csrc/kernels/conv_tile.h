@@ -56,6 +56,7 @@ struct ConvTileArgs {
   int xdstep;                // and the LDS bytes between them
   int tiles_h, tiles_w;
   int lds_x, lds_t, lds_tab;
+  int through;               // (bytes on the 16-byte grid) stores that the L2 passes on at once
   int32_t w_scale_stride;
   uint32_t x_xor;            // 0x80808080 for quint8 activations
   uint32_t pad_word;         // activation zero point in 4 bytes (before the xor)
@@ -406,7 +407,8 @@ __global__ __launch_bounds__(kCtThreads) void conv_tile_kernel(ConvTileArgs a) {
           if (op >= 0 && n < a.OCg) {
             uint8_t* dst = y + static_cast<int64_t>(op) * a.OC + ch0 + cq * 16;
             if (vec_ok) {
-              *reinterpret_cast<v4i*>(dst) = v;
+              if (a.through) st16_through(dst, v);
+              else *reinterpret_cast<v4i*>(dst) = v;
             } else if (n + 16 <= a.OCg) {
               st16_any(dst, v);
             } else {

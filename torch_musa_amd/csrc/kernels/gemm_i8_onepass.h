@@ -263,7 +263,7 @@ __global__ __launch_bounds__(BN * 4) void gemm_i8_onepass_kernel(GemmArgs a, XLi
       const v4i v = ld16(&sW[row * kPitch + cc * 16]);
       uint8_t* dst = y + m * a.ldy + n;
       if (vec_ok && n + 16 <= a.N) {
-        *reinterpret_cast<v4i*>(dst) = v;
+        st16_through(dst, v);
       } else if (n + 16 <= a.N) {
         st16_any(dst, v);  // (a row pitch or pointer off the 16-byte grid)
       } else {

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kPersistThreads, 1) void gemm_i8_persistent_kernel(
         if (m < a.M && n < a.N) {
           uint8_t* dst = ybase + m * a.ldy + n;
           if (vec_ok && n + 16 <= a.N) {
-            *reinterpret_cast<v4i*>(dst) = v;
+            st16_through(dst, v);  // (4096 x 1024 -> 4096 23.2 -> 21.3 us, 4096 x 11008 -> 4096 149.5 -> 147.7)
           } else if (n + 16 <= a.N) {
             st16_any(dst, v);  // (a row pitch or pointer off the 16-byte grid)
           } else {
