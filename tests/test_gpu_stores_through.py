@@ -82,3 +82,28 @@ def test_linear(m, k, n):
     for lo in range(0, m, step):
         assert torch.equal(whole[lo:lo + step], OPS.linear(x[lo:lo + step], packed, scale, 128).int_repr()), lo
     assert whole.unique().numel() > 100
+
+
+@pytest.mark.parametrize("rows,cols,axis", [(7168, 4096, 0), (7167, 4096, 0), (4100, 8196, 0), (28001, 1050, 0)])
+def test_quantize(rows, cols, axis):
+    say("quantize", rows, cols)
+    gen = torch.Generator("cuda").manual_seed(rows)
+    x = torch.randn(rows, cols, device="cuda", generator=gen)
+    scales = x.abs().amax(1).double() / 127
+    zps = torch.zeros(rows, dtype=torch.long, device="cuda")
+    whole, channels = torch.quantize_per_tensor(x, 0.03, 5, torch.qint8), torch.quantize_per_channel(x, scales, zps, axis, torch.qint8)
+    step = 3001
+    for lo in range(0, rows, step):
+        part = x[lo:lo + step].contiguous()
+        assert torch.equal(whole.int_repr()[lo:lo + step], torch.quantize_per_tensor(part, 0.03, 5, torch.qint8).int_repr())
+        few = torch.quantize_per_channel(part, scales[lo:lo + step].contiguous(), zps[lo:lo + step].contiguous(), axis, torch.qint8)
+        assert torch.equal(channels.int_repr()[lo:lo + step], few.int_repr())
+
+
+@pytest.mark.parametrize("c", [48, 56])
+def test_max_pool(c):
+    gen = torch.Generator("cuda").manual_seed(c)
+    x = feature_map(gen, 9, 147, 159, c)  # 2.6 and 3.1 MB of maxima in all
+    whole = torch.nn.functional.max_pool2d(x, 3, 2, 1).int_repr()
+    for i in range(9):
+        assert torch.equal(whole[i:i + 1], torch.nn.functional.max_pool2d(x[i:i + 1], 3, 2, 1).int_repr())

@@ -144,7 +144,8 @@ __device__ __forceinline__ void report_range(const RangeReport& r, float mn, flo
 constexpr int kQThreads = 128;
 
 constexpr int64_t kStreamOutCodes = int64_t{1} << 28;  // the last-level cache, in bytes
-template <bool SIGNED, bool FUSED = false, bool STREAM_OUT = false>
+enum QStore { kQCached, kQThrough, kQStream };
+template <bool SIGNED, bool FUSED = false, int STORE = kQCached>
 __global__ __launch_bounds__(kQThreads) void quantize_vec_kernel(
     const v4f* __restrict__ x4, uint32_t* __restrict__ q4, int64_t n4,
     const float* __restrict__ x, uint8_t* __restrict__ q, int64_t n, QParamsArg qp) {
@@ -158,7 +159,8 @@ __global__ __launch_bounds__(kQThreads) void quantize_vec_kernel(
 #pragma unroll
     for (int u = 0; u < kUnrollQD; ++u) {
       const uint32_t codes = quantize_four<SIGNED, FUSED>(v[u], inv, zp_f);
-      if constexpr (STREAM_OUT) __builtin_nontemporal_store(codes, &q4[base + u * kQThreads]);
+      if constexpr (STORE == kQStream) __builtin_nontemporal_store(codes, &q4[base + u * kQThreads]);
+      else if constexpr (STORE == kQThrough) st4_through(&q4[base + u * kQThreads], codes);
       else q4[base + u * kQThreads] = codes;
     }
   } else {
@@ -747,7 +749,7 @@ __device__ __forceinline__ float dequantize_fq_one(uint32_t byte, float zp, floa
 
 // An Op: P, the parameters of a channel; load4 / load1, conv4 (four values of up to four
 // channels), conv1, put4 / put1; zp_outside, the range check of a channel's zero point.
-template <bool SIGNED>
+template <bool SIGNED, bool THROUGH = false>
 struct PcQuantize {
   // fp32 -> codes, double scales, int64 zero points
   static constexpr int kAccesses = 4;
@@ -778,7 +780,10 @@ struct PcQuantize {
                                               packed);
     return SIGNED ? packed ^ 0x80808080u : packed;
   }
-  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const {
+    if constexpr (THROUGH) st4_through(q + i, v);
+    else *reinterpret_cast<uint32_t*>(q + i) = v;
+  }
   __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_one<SIGNED>(v, p.inv, p.zp));
   }
@@ -817,7 +822,7 @@ struct PcDequantize {
   __device__ __forceinline__ void put1(int64_t i, In1 b, P p) const { r[i] = dequantize_pc_one<SIGNED>(b, p.zp, p.scale); }
 };
 
-template <bool SIGNED>
+template <bool SIGNED, bool THROUGH = false>
 struct PcfQuantize {
   // fp32 -> codes, float scales and float zero points
   static constexpr int kAccesses = 4;
@@ -844,7 +849,10 @@ struct PcfQuantize {
     return quantize_fq_one<SIGNED>(v.x, p[0].inv, p[0].zp) | (quantize_fq_one<SIGNED>(v.y, p[1].inv, p[1].zp) << 8) |
            (quantize_fq_one<SIGNED>(v.z, p[2].inv, p[2].zp) << 16) | (quantize_fq_one<SIGNED>(v.w, p[3].inv, p[3].zp) << 24);
   }
-  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const {
+    if constexpr (THROUGH) st4_through(q + i, v);
+    else *reinterpret_cast<uint32_t*>(q + i) = v;
+  }
   __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_fq_one<SIGNED>(v, p.inv, p.zp));
   }
@@ -1122,6 +1130,11 @@ inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t cap) {
   return static_cast<unsigned>(g);
 }
 
+bool pc_rows_take(int64_t inner) { return inner % 4 == 0 && inner >= kPcRowsMinInner; }
+// Codes that leave past the L2s, us without | with them, both directions: [11008, 4096] 69.3 | 67.1, [12288, 8192] 146.8 | 144.7,
+// [12288, 12288] 217.9 | 215.1; [4096, 4096] level, [4096, 2048] 25.4 | 28.8 (as for the per-tensor quantizer above).
+bool pc_through(int64_t n) { return n >= (int64_t{28} << 20); }
+
 // `vec`: both pointers take 16-byte accesses of fp32 and 4-byte accesses of codes.
 template <class Op>
 int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bool vec, const PcCheck& check,
@@ -1145,7 +1158,7 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
       return launch_status();
     }
   }
-  if (vec && inner % 4 == 0 && inner >= kPcRowsMinInner) {
+  if (vec && pc_rows_take(inner)) {
     constexpr int kPcAccesses = Op::kAccesses;
     const int64_t per_run = kPcThreads * 4;
     int lg_us = 0;
@@ -1173,6 +1186,11 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
   return launch_status();
 }
 
+// Codes that leave past the L2s (st4_through), us without | with them, quantize and dequantize: 32 Mi values 51.6 | 49.7, 48 Mi
+// 74.6 | 73.2, 64 Mi 97.5 | 96.8, 128 Mi 191.0 | 191.2.  Fewer than the L2s hold stay in them for a dequantizer, whose blocks
+// read what the same XCD wrote (24 Mi 36.8 | 38.1, 8 Mi 13.7 | 15.0).
+bool quantize_through(int64_t n) { return n >= (int64_t{28} << 20) && n < (int64_t{96} << 20); }
+
 template <bool SIGNED, bool FUSED>
 int quantize_launch_as(const float* x, void* q, int64_t n, QParamsArg qp, hipStream_t s) {
   uint8_t* qb = static_cast<uint8_t*>(q);
@@ -1181,7 +1199,10 @@ int quantize_launch_as(const float* x, void* q, int64_t n, QParamsArg qp, hipStr
     const int64_t blocks = n4 == 0 ? 1 : ceil_div(n4, kQThreads * kUnrollQD);
     if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
     if (n > kStreamOutCodes)
-      enqueue(quantize_vec_kernel<SIGNED, FUSED, true>, dim3(blocks), dim3(kQThreads), 0, s,
+      enqueue(quantize_vec_kernel<SIGNED, FUSED, kQStream>, dim3(blocks), dim3(kQThreads), 0, s,
+              reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
+    else if (quantize_through(n))
+      enqueue(quantize_vec_kernel<SIGNED, FUSED, kQThrough>, dim3(blocks), dim3(kQThreads), 0, s,
               reinterpret_cast<const v4f*>(x), reinterpret_cast<uint32_t*>(q), n4, x, qb, n, qp);
     else
       enqueue(quantize_vec_kernel<SIGNED, FUSED>, dim3(blocks), dim3(kQThreads), 0, s,
@@ -1466,16 +1487,19 @@ TMQ_EXPORT int tmq_per_channel(const tmq_per_channel_desc* d, tmq_stream_t strea
   auto* f = static_cast<float*>(d->fp32);
   auto* q = static_cast<uint8_t*>(d->codes);
   const bool vec = aligned(f, 16) && aligned(q, 4);
+  const bool through = !d->dequantize && vec && pc_rows_take(d->inner) && pc_through(d->outer * d->channels * d->inner);
   auto go = [&](const auto& op) { return launch_per_channel(op, d->outer, d->channels, d->inner, vec, check, s); };
   if (d->float_qparams) {
     auto* sc = static_cast<const float*>(d->scales);
     auto* zp = static_cast<const float*>(d->zero_points);
     if (d->dequantize) return d->q_signed ? go(PcfDequantize<true>{q, f, sc, zp}) : go(PcfDequantize<false>{q, f, sc, zp});
+    if (through) return d->q_signed ? go(PcfQuantize<true, true>{f, q, sc, zp}) : go(PcfQuantize<false, true>{f, q, sc, zp});
     return d->q_signed ? go(PcfQuantize<true>{f, q, sc, zp}) : go(PcfQuantize<false>{f, q, sc, zp});
   }
   auto* sc = static_cast<const double*>(d->scales);
   auto* zp = static_cast<const int64_t*>(d->zero_points);
   if (d->dequantize) return d->q_signed ? go(PcDequantize<true>{q, f, sc, zp}) : go(PcDequantize<false>{q, f, sc, zp});
+  if (through) return d->q_signed ? go(PcQuantize<true, true>{f, q, sc, zp}) : go(PcQuantize<false, true>{f, q, sc, zp});
   return d->q_signed ? go(PcQuantize<true>{f, q, sc, zp}) : go(PcQuantize<false>{f, q, sc, zp});
 }
 
