@@ -162,7 +162,7 @@ __device__ __forceinline__ void runs_requant(const ConvRunArgs& a, const v4i (&a
     }
   }
 }
-// One store of a lane's 4 NT bytes, at any alignment (the same instruction as an aligned one); through: see common.h, dst
+// One store of a lane's 4 NT bytes, at any alignment (the same instruction as an aligned one); through: stores_through.h, dst
 // on the grid of 4 NT bytes.
 template <int NT>
 __device__ __forceinline__ void runs_store(uint8_t* dst, const uint32_t (&packed)[NT], bool through) {

@@ -12,6 +12,7 @@
 //   q = clamp(rne(c * fl(1 / out_scale)) + out_zp)
 // every step in fp32.
 #include "common.h"
+#include "stores_through.h"
 
 namespace tmq {
 namespace {

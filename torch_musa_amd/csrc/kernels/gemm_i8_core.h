@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "stores_through.h"
 
 namespace tmq {
 

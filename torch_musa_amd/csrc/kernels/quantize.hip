@@ -15,6 +15,7 @@
 
 #include "common.h"
 #include "qparams.h"
+#include "stores_through.h"
 
 namespace tmq {
 namespace {
