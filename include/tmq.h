@@ -300,7 +300,8 @@ int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int3
  * here so that the choice and every kernel's preconditions can be swept on the
  * host over thousands of shapes. */
 typedef struct tmq_linear_choice {
-  int32_t kernel;        /* value that pins this kernel in tmq_linear_desc::kernel (configuration + 1);
+  int32_t kernel;        /* value that pins this kernel in tmq_linear_desc::kernel (configuration + 1; 3 with tiles of
+                            32 rows: 30 pins those of 32 channels, 31 those of 64);
                             0: no kernel takes the shape (TMQ_ERR_UNSUPPORTED from the call) */
   int32_t tile_rows;     /* activation rows per workgroup tile (0: plain kernel) */
   int32_t tile_channels; /* output channels per workgroup tile */

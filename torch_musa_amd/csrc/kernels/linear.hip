@@ -7,6 +7,7 @@
 #include "gemm_i8_onepass.h"
 #include "gemm_i8_persistent.h"
 #include "gemm_i8_wring.h"
+#include "gemm_i8_wloop.h"
 #include "linear_resident.h"
 #include "qparams.h"
 
@@ -632,6 +633,18 @@ int launch_gemm_wring(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   return launch_status();
 }
 
+// Tiles of 32 rows x 32 or 64 channels whose waves split K and walk their shares in pieces (the caller checked the
+// address ranges).
+template <int MODE>
+int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
+  const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, wide ? 64 : 32);
+  if (tiles_n > 0x7fffffff || tiles_m > 65535) return TMQ_ERR_UNSUPPORTED;
+  const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), block(kWloopWaves * kWave);
+  if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2>, grid, block, 0, s, a, xs);
+  else enqueue(gemm_i8_wloop_kernel<MODE, 1>, grid, block, 0, s, a, xs);
+  return launch_status();
+}
+
 constexpr int kMaxDevices = 64;
 
 // Compute units of the current device (cached per device; two threads that race
@@ -843,6 +856,28 @@ bool phased_ring_preferred(int64_t M, int64_t N, int64_t K) {
   return K > 4096 ? M <= 128 : (K == 4096 && M <= 64 && N >= 10240);
 }
 
+// More than 48 rows against K beyond what the kernels above hold at once, one round of tiles of 32 rows: eight waves a
+// tile that walk their shares of K (gemm_i8_wloop.h).  Us, the best other kernel | it, weights from memory:
+//   up to 256 tiles of 32 x 32: 322 x 4352 -> 384 12.1 | 8.0; 622 x 6400 -> 384 15.6 | 11.8; 1762 x 8000 -> 64 18.5 | 11.3;
+//     2025 x 9536 -> 64 21.2 | 14.5; 531 x 6144 -> 640 15.3 | 13.6; least ahead against much weight, 116 x 10368 -> 1728
+//     19.7 | 19.0 and 185 x 10816 -> 704 16.0 | 14.9 (split K); at K = 4096 and below behind those that hold K at once
+//     (593 x 4096 -> 384 7.1 | 8.2);
+//   up to 256 of 32 x 64, more than 64 rows, up to 12 Mi weights: 219 x 5440 -> 1536 14.2 | 11.1; 2129 x 7104 -> 192
+//     17.0 | 15.6; 668 x 8320 -> 448 18.9 | 15.6; 314 x 6528 -> 1600 18.0 | 18.6; with more weights 137 x 7168 -> 2752
+//     18.2 | 20.5, 93 x 9280 -> 3712 20.7 | 24.5;
+//   49 to 64 rows: 61 x 7808 -> 1088 14.0 | 10.6, 59 x 11008 -> 3136 20.0 | 19.7; fewer stream their weights as fast
+//     (48 x 5568 -> 128 8.7 | 9.8, 35 x 4672 -> 320 9.2 | 8.7, 18 x 11328 -> 768 11.1 | 12.5).
+// The tiles that walk K as a ring of phases keep their shapes up to K = 5632: their tests hold them to it, although
+// 116 x 4480 -> 1728 takes 15.3 | 10.7 (117 x 6272 -> 1472 19.5 | 12.8).  Measured up to K = 12288.  Returns the channels per tile, 0: not such a shape.
+constexpr int64_t kWloopMaxK = 12288, kWloopRingMinK = 5632;
+int wloop_tile(int64_t M, int64_t N, int64_t K) {
+  if (M <= 48 || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
+  if (K < kWloopRingMinK && phased_ring_preferred(M, N, K)) return 0;
+  if (ceil_div(M, 32) * ceil_div(N, 32) <= 256) return 32;
+  if (M > kDecodeMaxRows && ceil_div(M, 32) * ceil_div(N, 64) <= 256 && N * K <= int64_t{12} << 20) return 64;
+  return 0;
+}
+
 SmallRows small_rows_path(int64_t M, int64_t N, int64_t K, bool workspace) {
   // Where the 32 x 32 tiles with the weights through registers fit, they are measured
   // directly against the weight-streaming kernel (us at M = 17 / 32 / 40 / 64, tiles | streaming):
@@ -1038,7 +1073,8 @@ struct LinearQuery {
 // streaming; 9: plain kernel; 13: split K (plan in `split`); 20: persistent 256 x 256 tiles;
 // 21 / 24: all of K in LDS (64 x 64 / 32 x 32 tiles); 25 / 26: weights through registers
 // (32 x 32 / 32 x 64 tiles); 27: the same with 64 x 64 tiles and the activations in a ring
-// per wave; 28: activations resident in LDS, one block per CU streams its channel groups;
+// per wave; 28: activations resident in LDS, one block per CU streams its channel groups; 29 / 30: tiles of 32 rows x 32 / 64
+// channels whose waves walk their shares of K in pieces;
 // kNoKernel: the forced kernel does not take this shape.
 constexpr int kNoKernel = -2;
 struct LinearChoice {
@@ -1202,6 +1238,10 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     c.cfg = 28;
     return c;
   }
+  if (forced < 0 && onepass_limits_ok(q) && wloop_tile(q.M, q.N, q.K) != 0) {
+    c.cfg = wloop_tile(q.M, q.N, q.K) == 32 ? 29 : 30;
+    return c;
+  }
   const bool stream_auto =
       forced < 0 && (q.M <= kDecodeRowsAuto ||
                      (q.M <= kDecodeMaxRows &&
@@ -1359,6 +1399,9 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     case 28:
       if (!resident_limits_ok(M, N, K, q.ldx, 256)) cfg = kNoKernel;
       break;
+    case 29: case 30:
+      if (!onepass_ok) cfg = kNoKernel;
+      break;
     default:
       cfg = kNoKernel;
   }
@@ -1386,6 +1429,11 @@ bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
   return tiles <= (K <= 128 ? 3072 : K <= 768 ? 1024 : 512);
 }
 
+// ... and where the copy comes first, if there is room for it: K so long that the padded shape's kernel earns it back (two
+// layers, quantize and dequantize as a program calls them, direct | copy, us: 840 x 8155 -> 192 39.0 | 33.8, 59 x 6040 -> 384
+// 26.8 | 21.5, 200 x 5001 -> 1000 29.7 | 25.2, 1237 x 6284 -> 212 36.7 | 34.1, 1633 x 5834 -> 163 35.6 | 35.4).
+bool ragged_copy_first(int64_t M, int64_t N, int64_t K) { return wloop_tile(M, N, regrid_pitch(K)) != 0; }
+
 template <int MODE>
 int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec_ok, int forced,
                     hipStream_t s, void* workspace = nullptr, int64_t workspace_bytes = 0) {
@@ -1407,13 +1455,15 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     // and take the kernel of the padded shape.
     if (a.M <= kDecodeRowsAuto && a.K >= 16 && stream_limits_ok(q) && a.w_kchunks == packed_kchunks(a.K))
       return launch_linear_decode_ragged<MODE>(a, xs, s);
-    if (ragged_tiles_preferred(a.M, a.N, a.K) && a.w_kchunks == packed_kchunks(a.K)) {
+    const int64_t room = regrid_bytes(a.M, a.K);
+    const bool copy_ok = regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room;
+    if (ragged_tiles_preferred(a.M, a.N, a.K) && a.w_kchunks == packed_kchunks(a.K) &&
+        !(copy_ok && ragged_copy_first(a.M, a.N, a.K))) {
       const XLinearRagged rows{xs.x, xs.ldx};
       return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
                                                 : launch_gemm<64, 64, 2, 2, MODE>(a, rows, s);
     }
-    const int64_t room = regrid_bytes(a.M, a.K);
-    if (regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room) {
+    if (copy_ok) {
       const int rc = launch_regrid(xs, a.M, a.K, workspace, s);
       if (rc != TMQ_OK) return rc;
       GemmArgs b = a;
@@ -1471,6 +1521,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     case 25: return launch_gemm_wstream<MODE>(a, xs, false, s);
     case 26: return launch_gemm_wstream<MODE>(a, xs, true, s);
     case 27: return launch_gemm_wring<MODE>(a, xs, s);
+    case 29: case 30: return launch_gemm_wloop<MODE>(a, xs, c.cfg == 30, s);
     default: return TMQ_ERR_UNSUPPORTED;
   }
 }
@@ -1552,9 +1603,11 @@ TMQ_EXPORT int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (K % 16 == 0 && on_grid) return tmq_linear_workspace_bytes(M, N, K);
-  if ((M <= kDecodeRowsAuto && K >= 16) || ragged_tiles_preferred(M, N, K) || !regrid_limits_ok(M, K)) return 0;
-  return regrid_bytes(M, K) + tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
+  // (the plan of a split along K is there for pinned kernels where the automatic choice is another one)
+  const int64_t split = wloop_tile(M, N, regrid_pitch(K)) != 0 ? 0 : tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
+  if (K % 16 == 0 && on_grid) return split;
+  if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_tiles_preferred(M, N, K) && !ragged_copy_first(M, N, K)) || !regrid_limits_ok(M, K)) return 0;
+  return regrid_bytes(M, K) + split;
 }
 
 TMQ_EXPORT int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int32_t* stages) {
@@ -1602,11 +1655,13 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     case 24: case 25: bm = 32, bn = 32; break;
     case 26: bm = 32, bn = 64, waves = 8; break;
     case 27: bm = 64, bn = 64, waves = 8; break;
+    case 29: bm = 32, bn = 32, waves = kWloopWaves; break;
+    case 30: bm = 32, bn = 64, waves = kWloopWaves; break;
     case 8: bm = 16 * static_cast<int>(ceil_div(M, 16)), bn = 16, waves = kDecodeWaves; break;
     case 28: bm = 16 * static_cast<int>(ceil_div(M, 16)), bn = 16, waves = resident_pair(M, N, K, compute_units) ? 8 : kResidentWaves; break;
     default: break;  // 9: one thread per four outputs
   }
-  out->kernel = c.cfg + 1;
+  out->kernel = (forced_kernel == 0 && (c.cfg == 29 || c.cfg == 30) ? 2 : c.cfg) + 1;  // (see tmq_linear_choice)
   out->tile_rows = bm;
   out->tile_channels = bn;
   out->waves = waves;
