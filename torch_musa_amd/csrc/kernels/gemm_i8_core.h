@@ -890,6 +890,8 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       else
         xf[j - TN] = ld16(&sX[xb * kXStage + (wm0 + (j - TN) * 32 + li) * (2 * kBK) + (((4 * p + c) ^ xswz8) << 4)]);
     };
+    constexpr int kReads = (NF + Q - 1) / Q;  // LDS reads per MFMA
+    static_assert(ND <= Q, "a copy per MFMA at most");
     // ph = kt % 6 as a compile-time constant
     auto stage = [&](int kt, int ph) {
       const int wb = ph % 3, xb = (ph >> 1) % 3, p = ph & 1;
@@ -897,7 +899,8 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       const int wbn = phn % 3, xbn = (phn >> 1) % 3, pn = phn & 1;
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        if (q < NF) read_w(wb, xb, p, 1, q, wf1, xf1);
+#pragma unroll
+        for (int o = q * kReads; o < NF && o < (q + 1) * kReads; ++o) read_w(wb, xb, p, 1, o, wf1, xf1);
         mfma(q, wf0, xf0);
         if (q + 1 < TM) flip(xf0[q + 1]);
         if (q == Q - 1) flip(xf1[0]);
@@ -914,7 +917,8 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       constexpr int kFirstDma = (TM - 1 < Q - 1 - ND) ? TM - 1 : (Q - 1 - ND > 0 ? Q - 1 - ND : 0);
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        if (q < NF) read_w(wbn, xbn, pn, 0, q, wf0, xf0);
+#pragma unroll
+        for (int o = q * kReads; o < NF && o < (q + 1) * kReads; ++o) read_w(wbn, xbn, pn, 0, o, wf0, xf0);
         if (q >= kFirstDma && q - kFirstDma < ND) {
           const int i = q - kFirstDma;
           if (i < NDW) dma_w(kload, wb, i);

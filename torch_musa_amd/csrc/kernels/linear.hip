@@ -1188,6 +1188,21 @@ constexpr TileRate kRates[] = {
     {17, 128, 256, 1, 4.44, 1.97, 0.327, 0.0, 0.470, 2.67, 0.428},
     {6, 256, 256, 1, 7.35, 1.37, 0.489, 0.274, 0.601, 6.94, 0.767},
 };
+// Tiles of 64 x 128 and 128 x 64, copied straight into a ring of six stages where one round of them has a block per CU:
+// a lone block's three stages in registers are what it waits for (us, registers | ring: M = 641, N = 1600, K = 8064 32.1 |
+// 24.5; M = 133, N = 9984, K = 11776 52.0 | 42.1; M = 440, N = 2752, K = 3136 13.7 | 11.7; M = 514, N = 2432, K = 7104 128 x 64
+// 29.0 | 23.7).  128 x 64 is two thirds activations, whose copies of 64 bytes touch two lines each off the 64-byte grid:
+// no gain there (M = 261, N = 3712, K = 5200 23.0 | 24.2; M = 189, N = 6656, K = 4080 18.8 | 19.0).
+bool oblong_ring(int64_t M, int64_t N, int64_t K, int64_t ldx, int bm, int bn) {
+  return ceil_div(M, bm) * ceil_div(N, bn) <= 256 && K > 5 * kBK && dma_limits_ok(K, ldx) && (bm == 64 || K % kBK == 0);
+}
+// ... and ahead of every other tile there from K = 1280 on, where 64 x 64 tiles are more than a round (us, the choice before |
+// 64 x 128 in a ring: M = 1829, N = 800, K = 1552 9.9 | 8.3; M = 875, N = 1600, K = 1680 10.8 | 8.8; M = 2718, N = 304, K = 3024
+// 14.8 | 11.5; M = 3628, N = 432, K = 5360 26.1 | 17.6; level at M = 731, N = 1472, K = 1856 9.1 | 8.9; behind below, M = 1135,
+// N = 1024, K = 1216 7.2 | 7.4, and where a round of 64 x 64 tiles holds the product, M = 182, N = 4480, K = 1984 7.6 | 9.1).
+bool oblong_ring_first(int64_t M, int64_t N, int64_t K, int64_t ldx) {
+  return K >= 1280 && ceil_div(M, 64) * ceil_div(N, 64) > 256 && oblong_ring(M, N, K, ldx, 64, 128);
+}
 double rounds_time(const TileRate& r, int64_t M, int64_t N, int64_t K) {
   const double st = static_cast<double>(ceil_div(K, kBK)), round = 256.0 * r.on_cu;
   const int64_t tiles = ceil_div(M, r.bm) * ceil_div(N, r.bn);
@@ -1366,6 +1381,11 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     if (by_rounds == 2 && rounds_modelled(M, N, K)) c.groups = 1;
     cfg = by_rounds;
   }
+  if (forced < 0 && q.mode != kOutAcc32 && (cfg == 1 || cfg == 2 || cfg == 7 || cfg == 14 || cfg == 17) &&
+      oblong_ring_first(M, N, K, q.ldx)) {
+    cfg = 23;
+    c.groups = 1;
+  }
   const bool wide_ok = wide_limits_ok(K, q.ldx);
   if (cfg == 19 && !wide_ok) cfg = 17;
   // 256 x 256 tiles with byte or float outputs: the persistent kernel, which hides each
@@ -1509,13 +1529,23 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     case 4: return launch_gemm<128, 256, 2, 2, MODE>(a, xs, s);
     case 5: return launch_gemm<256, 128, 2, 2, MODE>(a, xs, s);
     case 6: return launch_gemm<256, 256, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
-    case 7: return launch_gemm<128, 128, 2, 2, MODE, 3, true, 1, true>(a, xs, s);
+    // (a block per CU: eight waves, so that one's fragment reads run beside another's products, and from K = 1536 on a ring
+    // of six stages where the copies of 64 activation bytes lie in one line each.  Us, four waves | eight | eight and six
+    // stages: M = 1160, N = 2048, K = 11008 59.4 | 58 | 41.7; M = 1062, N = 2496, K = 6016 35.5 | - | 26.8; M = 617, N = 5952,
+    // K = 1728 14.2 | 13.7 | 13.0; M = 752, N = 4800, K = 960 8.7 | 8.0 | 8.4; M = 254, N = 11264, K = 2480 20.3 | 19.8 | 23.5)
+    case 7: return ceil_div(a.M, 128) * ceil_div(a.N, 128) > 256
+                       ? launch_gemm<128, 128, 2, 2, MODE, 3, true, 1, true>(a, xs, s)
+                   : a.K >= 1536 && a.K % kBK == 0 ? launch_gemm<128, 128, 2, 4, MODE, 6, true>(a, xs, s)
+                                                   : launch_gemm<128, 128, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
     case 14: return launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s);
     case 17: return launch_gemm<128, 256, 2, 4, MODE, 3, true>(a, xs, s);
     case 19: return launch_gemm<128, 256, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
     case 20: return launch_gemm_persistent<MODE>(a, xs, s);
-    case 22: return launch_gemm<128, 64, 2, 2, MODE>(a, xs, s);
-    case 23: return c.onepass ? launch_gemm_onepass<MODE, 128>(a, xs, s) : launch_gemm<64, 128, 2, 2, MODE>(a, xs, s);
+    case 22: return oblong_ring(a.M, a.N, a.K, xs.ldx, 128, 64) ? launch_gemm<128, 64, 2, 2, MODE, 6, true>(a, xs, s)
+                                                                : launch_gemm<128, 64, 2, 2, MODE>(a, xs, s);
+    case 23: return c.onepass ? launch_gemm_onepass<MODE, 128>(a, xs, s)
+                    : oblong_ring(a.M, a.N, a.K, xs.ldx, 64, 128) ? launch_gemm<64, 128, 2, 2, MODE, 6, true>(a, xs, s)
+                                                                  : launch_gemm<64, 128, 2, 2, MODE>(a, xs, s);
     case 21: return launch_gemm_onepass<MODE>(a, xs, s);
     case 24: return launch_gemm_ksplit<MODE>(a, xs, s);
     case 25: return launch_gemm_wstream<MODE>(a, xs, false, s);
@@ -1643,7 +1673,8 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
   switch (c.cfg) {
     case 0: bm = 256, bn = 256; break;
     case 3: case 6: case 20: bm = 256, bn = 256, waves = 8; break;
-    case 1: case 7: case 13: bm = 128, bn = 128; break;
+    case 1: case 13: bm = 128, bn = 128; break;
+    case 7: bm = 128, bn = 128, waves = ceil_div(M, 128) * ceil_div(N, 128) <= 256 ? 8 : 4; break;
     case 2: bm = 64, bn = 64, waves = 4 * c.groups; break;
     case 21: bm = 64, bn = 64; break;
     case 14: bm = 64, bn = 64, waves = 8; break;
