@@ -41,7 +41,9 @@ def test_piece_and_tile_edges(cabi, cfg, k, m, n):  # noqa: F811
     (256, 1024, 4112), (257, 1024, 4112), (2048, 128, 12288), (300, 700, 12304),                  # 256 tiles of 32 x 32, the end of K
     (512, 1024, 5120), (513, 1024, 5120), (288, 1800, 6400), (288, 1800, 7168),                   # 256 of 32 x 64, 12 Mi weights
     # off the 16-byte grid: the copy comes first where the padded shape is one of these
-    (49, 33, 4097), (840, 192, 8155), (513, 70, 4111), (300, 500, 12287), (300, 500, 12290)])
+    (49, 33, 4097), (840, 192, 8155), (513, 70, 4111), (300, 500, 12287), (300, 500, 12290),
+    # ... or 64 x 128 tiles in a ring
+    (700, 1500, 2303), (700, 1500, 2305), (500, 3900, 4100)])
 @pytest.mark.parametrize("x_signed", [False, True])
 def test_the_choice(cabi, m, n, k, x_signed):  # noqa: F811
     say("linear pieces, the choice", m, n, k, x_signed)

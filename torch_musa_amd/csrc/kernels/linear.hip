@@ -1450,9 +1450,14 @@ bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
 }
 
 // ... and where the copy comes first, if there is room for it: K so long that the padded shape's kernel earns it back (two
-// layers, quantize and dequantize as a program calls them, direct | copy, us: 840 x 8155 -> 192 39.0 | 33.8, 59 x 6040 -> 384
-// 26.8 | 21.5, 200 x 5001 -> 1000 29.7 | 25.2, 1237 x 6284 -> 212 36.7 | 34.1, 1633 x 5834 -> 163 35.6 | 35.4).
-bool ragged_copy_first(int64_t M, int64_t N, int64_t K) { return wloop_tile(M, N, regrid_pitch(K)) != 0; }
+// layers, quantize and dequantize as a program calls them, direct | copy, us).  Waves that walk their shares of K: 840 x 8155
+// -> 192 39.0 | 33.8, 59 x 6040 -> 384 26.8 | 21.5, 200 x 5001 -> 1000 29.7 | 25.2, 1237 x 6284 -> 212 36.7 | 34.1, 1633 x
+// 5834 -> 163 35.6 | 35.4.  64 x 128 tiles in a ring: 600 x 6001 -> 2000 45.3 | 34.6, 700 x 3001 -> 1500 30.8 | 26.8, 1500 x
+// 2501 -> 900 31.4 | 29.7; 1000 x 2051 -> 2051 28.5 | 29.3, 2048 x 1310 -> 1024 25.6 | 26.9.
+bool ragged_copy_first(int64_t M, int64_t N, int64_t K) {
+  const int64_t pitch = regrid_pitch(K);
+  return wloop_tile(M, N, pitch) != 0 || (K >= 2304 && oblong_ring_first(M, N, pitch, pitch));
+}
 
 template <int MODE>
 int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec_ok, int forced,
