@@ -39,11 +39,16 @@ def test_piece_and_tile_edges(cabi, cfg, k, m, n):  # noqa: F811
 @pytest.mark.parametrize("m,n,k", [
     (48, 320, 4112), (49, 320, 4112), (49, 320, 4096), (64, 4096, 4400), (64, 4128, 4400),        # few rows
     (256, 1024, 4112), (257, 1024, 4112), (2048, 128, 12288), (300, 700, 12304),                  # 256 tiles of 32 x 32, the end of K
-    (512, 1024, 5120), (513, 1024, 5120), (288, 1800, 6400), (288, 1800, 7168),                   # 256 of 32 x 64, 12 Mi weights
+    (512, 1024, 5120), (513, 1024, 5120), (288, 1800, 6400), (288, 1800, 7168),                   # 256 of 32 x 64
+    (100, 3740, 8960), (100, 3750, 8960), (100, 2270, 9216), (100, 2280, 9216),                   # 32 and 20 Mi weights
+    (32, 320, 7680), (33, 320, 7680), (33, 320, 7664),                                            # more than 32 rows
     # off the 16-byte grid: the copy comes first where the padded shape is one of these
     (49, 33, 4097), (840, 192, 8155), (513, 70, 4111), (300, 500, 12287), (300, 500, 12290),
     # ... or 64 x 128 tiles in a ring
-    (700, 1500, 2303), (700, 1500, 2305), (500, 3900, 4100)])
+    (700, 1500, 2303), (700, 1500, 2305), (500, 3900, 4100),
+    # tiles dealt to the XCDs in runs, on either side of 900 KB of weights, of all row tiles' remainders
+    (129, 3040, 656), (129, 3072, 656), (64, 1360, 672), (64, 1376, 672), (33, 1376, 672), (300, 950, 1024),
+    (70, 5184, 1280), (65, 950, 1040), (129, 1100, 2064), (1129, 448, 3072), (40, 4200, 4096)])
 @pytest.mark.parametrize("x_signed", [False, True])
 def test_the_choice(cabi, m, n, k, x_signed):  # noqa: F811
     say("linear pieces, the choice", m, n, k, x_signed)

@@ -44,6 +44,26 @@ __device__ __forceinline__ void lds_dma4(const void* base, uint32_t off, uint32_
                : "memory", "m0");
 }
 
+// The tile of a block of grids smaller than the chip (channel tiles, row tiles).  Blocks are dealt to the 8 XCDs in turn, so
+// where the channel tiles are no multiple of 8 the row tiles over the same weights lie on different ones and each fetches
+// the weights from memory.  RUNS: each XCD takes one run of the tiles instead, rows before channels (us, in the grid's order |
+// in runs, weights from memory: gemm_i8_wloop_kernel, M = 314, N = 1600, K = 6528 18.6 | 11.7, M = 173, N = 1600, K = 4544
+// 13.2 | 9.3).  The division takes 0.1 us and a test for it in the kernel as much, which shows in the kernels for short K
+// (M = 128, N = K = 1024 3.7 | 3.8), so the host tells (tile_runs).
+struct TileAt {
+  int64_t m0, n0;
+};
+template <int BM, int BN, bool RUNS>
+__device__ __forceinline__ TileAt tile_of_block(const GemmArgs& a) {
+  if constexpr (!RUNS) return TileAt{static_cast<int64_t>(blockIdx.y) * BM, static_cast<int64_t>(blockIdx.x) * BN};
+  const uint32_t tiles_m = static_cast<uint32_t>(ceil_div(a.M, BM)), tiles_n = static_cast<uint32_t>(ceil_div(a.N, BN));
+  const uint32_t id = blockIdx.y * tiles_n + blockIdx.x, all = tiles_m * tiles_n;
+  const uint32_t share = all / 8, rest = all % 8, xcd = id % 8;
+  const uint32_t tile = xcd * share + (xcd < rest ? xcd : rest) + id / 8;
+  const uint32_t tile_n = __builtin_amdgcn_readfirstlane(tile / tiles_m);  // (the division is the vector unit's)
+  return TileAt{static_cast<int64_t>(tile - tile_n * tiles_m) * BM, static_cast<int64_t>(tile_n) * BN};
+}
+
 // BN = 128 (eight waves of the same 32 x 32, a ring of three phases, 144 KB): for grids whose 64 x 64 tiles
 // are a little more than the chip holds and would need a second round.
 template <int MODE, int BN = 64>
@@ -356,7 +376,7 @@ __device__ __forceinline__ void ksplit_finish(const GemmArgs& a, const uint8_t* 
 // LDS of wave w:  weights [k-step][k-chunk of the step][32 rows][16 B] (a copy
 // instruction moves one k-step: two 16-row blocks of two k-chunks of the packed
 // layout), activations [32 rows][256 B] with the slot swizzle of the kernel above.
-template <int MODE>
+template <int MODE, bool RUNS>
 __global__ __launch_bounds__(256) void gemm_i8_ksplit_kernel(GemmArgs a, XLinear xs) {
   constexpr int BM = 32, BN = 32;
   constexpr int kWaveSteps = 8;                    // 32-byte k-steps a wave can hold: 256 bytes of K
@@ -369,8 +389,8 @@ __global__ __launch_bounds__(256) void gemm_i8_ksplit_kernel(GemmArgs a, XLinear
   const int t = threadIdx.x, lane = t % kWave;
   const int wave_u = __builtin_amdgcn_readfirstlane(t / kWave);
   const int li = lane & 31, half = lane >> 5;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BM;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * BN;
+  const TileAt at = tile_of_block<BM, BN, RUNS>(a);
+  const int64_t m0 = at.m0, n0 = at.n0;
   const int KC = static_cast<int>(a.K >> 4);       // k-chunks (K is a multiple of 16, at most 1024)
   const int S = (KC + 1) >> 1;                     // 32-byte k-steps, at most 32
   const int sp = (S + 3) >> 2;                     // k-steps per wave
@@ -476,7 +496,7 @@ __global__ __launch_bounds__(256) void gemm_i8_ksplit_kernel(GemmArgs a, XLinear
 // that 32 x 32 tiles would overfill) and WAVES = 8 splits K eight ways, which keeps
 // the weight fragments of two channel tiles within the register file at K up to
 // 4096 (four waves with two channel tiles each measured 9.4 us where eight take 7.3).
-template <int MODE, int STEPS, int CT = 1, int WAVES = 4>
+template <int MODE, bool RUNS, int STEPS, int CT = 1, int WAVES = 4>
 __global__ __launch_bounds__(WAVES* kWave) void gemm_i8_wstream_kernel(GemmArgs a, XLinear xs) {
   constexpr int BM = 32, BN = 32 * CT;
   constexpr int SEGS = STEPS / 8;                  // 256-byte segments of K per wave
@@ -489,8 +509,8 @@ __global__ __launch_bounds__(WAVES* kWave) void gemm_i8_wstream_kernel(GemmArgs 
   const int t = threadIdx.x, lane = t % kWave;
   const int wave_u = __builtin_amdgcn_readfirstlane(t / kWave);
   const int li = lane & 31, half = lane >> 5;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BM;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * BN;
+  const TileAt at = tile_of_block<BM, BN, RUNS>(a);
+  const int64_t m0 = at.m0, n0 = at.n0;
   const int KC = static_cast<int>(a.K >> 4);       // k-chunks (K is a multiple of 16)
   const int S = (KC + 1) >> 1;                     // 32-byte k-steps, at most WAVES * STEPS
   const int sp = (S + WAVES - 1) / WAVES;          // k-steps per wave, at most STEPS

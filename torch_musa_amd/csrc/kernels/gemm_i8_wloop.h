@@ -42,8 +42,8 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   const int t = threadIdx.x, lane = t % kWave;
   const int wave_u = __builtin_amdgcn_readfirstlane(t / kWave);
   const int li = lane & 31, half = lane >> 5;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BM;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * BN;
+  const TileAt at = tile_of_block<BM, BN, true>(a);
+  const int64_t m0 = at.m0, n0 = at.n0;
   const int K = static_cast<int>(a.K);
   const int KC = K >> 4;                     // 16-byte chunks of a row (K is a multiple of 16)
   const int pieces = (K + PB - 1) / PB;

@@ -596,30 +596,45 @@ int launch_gemm_onepass(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   return launch_status();
 }
 
+// Whether the XCDs take runs of a small grid's tiles (tile_of_block): several row tiles over 900 KB of weights and more that
+// the grid's order would spread over the XCDs (us, weights from memory, without | with: 129 x 656 -> 3040 5.7 | 4.7, 137 x 688 ->
+// 2272 5.3 | 4.7, 70 x 1280 -> 5184 7.3 | 6.3, 1129 x 3072 -> 448 8.6 | 7.8; 277 x 704 -> 640 3.8 | 4.2).
+bool tile_runs(int64_t tiles_m, int64_t tiles_n, const GemmArgs& a) {
+  return tiles_m > 1 && tiles_n % 8 != 0 && a.N * a.K >= 900 * 1024;
+}
+
 // 32 x 32 tiles whose four waves split K (K <= 1024; the caller checked the address ranges).
 template <int MODE>
 int launch_gemm_ksplit(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, 32);
   if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > kOnePassMaxK) return TMQ_ERR_UNSUPPORTED;
-  enqueue(gemm_i8_ksplit_kernel<MODE>,
-          dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(256), 0, s, a, xs);
+  const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
+  if (tiles_n * tiles_m <= 0x7fffffff && tile_runs(tiles_m, tiles_n, a))
+    enqueue(gemm_i8_ksplit_kernel<MODE, true>, grid, dim3(256), 0, s, a, xs);
+  else
+    enqueue(gemm_i8_ksplit_kernel<MODE, false>, grid, dim3(256), 0, s, a, xs);
   return launch_status();
 }
 
 // Tiles of 32 rows whose waves split K, weights through registers (K <= 4096; the caller
 // checked the address ranges).  wide: 64 channels per tile instead of 32.
+template <int MODE, bool RUNS>
+int launch_gemm_wstream_as(const GemmArgs& a, const XLinear& xs, bool wide, dim3 grid, hipStream_t s) {
+  if (!wide && a.K <= 2048)
+    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 16>, grid, dim3(256), 0, s, a, xs);
+  else if (!wide)
+    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 32>, grid, dim3(256), 0, s, a, xs);
+  else
+    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 16, 2, 8>, grid, dim3(512), 0, s, a, xs);
+  return launch_status();
+}
 template <int MODE>
 int launch_gemm_wstream(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, wide ? 64 : 32);
   if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > 4096) return TMQ_ERR_UNSUPPORTED;
   const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
-  if (!wide && a.K <= 2048)
-    enqueue(gemm_i8_wstream_kernel<MODE, 16>, grid, dim3(256), 0, s, a, xs);
-  else if (!wide)
-    enqueue(gemm_i8_wstream_kernel<MODE, 32>, grid, dim3(256), 0, s, a, xs);
-  else
-    enqueue(gemm_i8_wstream_kernel<MODE, 16, 2, 8>, grid, dim3(512), 0, s, a, xs);
-  return launch_status();
+  return tiles_n * tiles_m <= 0x7fffffff && tile_runs(tiles_m, tiles_n, a) ? launch_gemm_wstream_as<MODE, true>(a, xs, wide, grid, s)
+                                                                           : launch_gemm_wstream_as<MODE, false>(a, xs, wide, grid, s);
 }
 
 // 64 x 64 tiles whose eight waves split K, weights through registers, activations through
@@ -638,7 +653,7 @@ int launch_gemm_wring(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
 template <int MODE>
 int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
   const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, wide ? 64 : 32);
-  if (tiles_n > 0x7fffffff || tiles_m > 65535) return TMQ_ERR_UNSUPPORTED;
+  if (tiles_n * tiles_m > 0x7fffffff || tiles_m > 65535) return TMQ_ERR_UNSUPPORTED;
   const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), block(kWloopWaves * kWave);
   if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2>, grid, block, 0, s, a, xs);
   else enqueue(gemm_i8_wloop_kernel<MODE, 1>, grid, block, 0, s, a, xs);
@@ -856,25 +871,25 @@ bool phased_ring_preferred(int64_t M, int64_t N, int64_t K) {
   return K > 4096 ? M <= 128 : (K == 4096 && M <= 64 && N >= 10240);
 }
 
-// More than 48 rows against K beyond what the kernels above hold at once, one round of tiles of 32 rows: eight waves a
+// More than 48 (32) rows against K beyond what the kernels above hold at once, one round of tiles of 32 rows: eight waves a
 // tile that walk their shares of K (gemm_i8_wloop.h).  Us, the best other kernel | it, weights from memory:
-//   up to 256 tiles of 32 x 32: 322 x 4352 -> 384 12.1 | 8.0; 622 x 6400 -> 384 15.6 | 11.8; 1762 x 8000 -> 64 18.5 | 11.3;
-//     2025 x 9536 -> 64 21.2 | 14.5; 531 x 6144 -> 640 15.3 | 13.6; least ahead against much weight, 116 x 10368 -> 1728
-//     19.7 | 19.0 and 185 x 10816 -> 704 16.0 | 14.9 (split K); at K = 4096 and below behind those that hold K at once
-//     (593 x 4096 -> 384 7.1 | 8.2);
-//   up to 256 of 32 x 64, more than 64 rows, up to 12 Mi weights: 219 x 5440 -> 1536 14.2 | 11.1; 2129 x 7104 -> 192
-//     17.0 | 15.6; 668 x 8320 -> 448 18.9 | 15.6; 314 x 6528 -> 1600 18.0 | 18.6; with more weights 137 x 7168 -> 2752
-//     18.2 | 20.5, 93 x 9280 -> 3712 20.7 | 24.5;
-//   49 to 64 rows: 61 x 7808 -> 1088 14.0 | 10.6, 59 x 11008 -> 3136 20.0 | 19.7; fewer stream their weights as fast
-//     (48 x 5568 -> 128 8.7 | 9.8, 35 x 4672 -> 320 9.2 | 8.7, 18 x 11328 -> 768 11.1 | 12.5).
-// The tiles that walk K as a ring of phases keep their shapes up to K = 5632: their tests hold them to it, although
-// 116 x 4480 -> 1728 takes 15.3 | 10.7 (117 x 6272 -> 1472 19.5 | 12.8).  Measured up to K = 12288.  Returns the channels per tile, 0: not such a shape.
+//   up to 256 tiles of 32 x 32: 526 x 11936 -> 464 33.3 | 16.5; 373 x 8832 -> 576 19.9 | 11.5; 322 x 4352 -> 384 12.1 | 8.0;
+//     58 x 11840 -> 2944 20.3 | 18.3; 53 x 10832 -> 96 level at 13.0; at K = 4096 and below behind those that hold K at
+//     once (593 x 4096 -> 384 7.1 | 8.3);
+//   up to 256 of 32 x 64: 225 x 4992 -> 1392 13.3 | 10.6; 250 x 6720 -> 1216 19.8 | 12.7; 111 x 7808 -> 2576 21.2 | 16.3;
+//     289 x 12128 -> 1600 28.6 | 21.5; not for more than 32 Mi weights, near level (54 x 5440 -> 7616 18.2 | 17.1), nor
+//     from K = 9216 on more than 20 Mi, where a split along K into two launches is ahead (114 x 10576 -> 2304 20.6 | 22.3);
+//   up to 48 rows weights stream as fast (41 x 5712 -> 144 9.0 | 10.0, 37 x 6592 -> 1664 10.6 | 12.0, 23 x 8128 -> 448
+//     8.5 | 9.9) but for more than 32 from K = 7680 on: 38 x 9408 -> 432 14.4 | 12.2, 46 x 8960 -> 768 13.7 | 10.6.
+// The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and 32 Mi weights: their tests hold them to it, although
+// 116 x 4480 -> 1728 takes 15.3 | 10.7 (117 x 6272 -> 1472 19.5 | 12.8).  Measured up to K = 12288.  Returns the channels per
+// tile, 0: not such a shape.
 constexpr int64_t kWloopMaxK = 12288, kWloopRingMinK = 5632;
 int wloop_tile(int64_t M, int64_t N, int64_t K) {
-  if (M <= 48 || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
+  if (M <= (K >= 7680 ? 32 : 48) || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
   if (K < kWloopRingMinK && phased_ring_preferred(M, N, K)) return 0;
   if (ceil_div(M, 32) * ceil_div(N, 32) <= 256) return 32;
-  if (M > kDecodeMaxRows && ceil_div(M, 32) * ceil_div(N, 64) <= 256 && N * K <= int64_t{12} << 20) return 64;
+  if (M > 48 && ceil_div(M, 32) * ceil_div(N, 64) <= 256 && N * K <= int64_t{K < 9216 ? 32 : 20} << 20) return 64;
   return 0;
 }
 
