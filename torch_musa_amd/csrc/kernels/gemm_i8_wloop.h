@@ -11,8 +11,8 @@
 // as it has been multiplied the piece after the next is requested into the same registers.
 // The sign flip of unsigned activations and the zeros behind K are applied on the way into LDS.
 //
-// Measured (us, weights from memory, the best other kernel | this one): M = 174, N = 1088, K = 4544 12.5 | 9.4;
-// M = 102, N = 1280, K = 6784 16.2 | 10.1; M = 267, N = 256, K = 8704 20.8 | 10.3; M = 364, N = 320, K = 11968 24.6 | 15.2.
+// Measured (us, weights from memory, the best other kernel | this one): M = 174, N = 1088, K = 4544 12.5 | 8.6;
+// M = 102, N = 1280, K = 6784 16.2 | 10.1; M = 267, N = 256, K = 8704 19.6 | 10.3; M = 364, N = 320, K = 11968 24.7 | 14.8.
 // At those a block pulls 64 K bytes at 48 ... 60 bytes a nanosecond behind 2 us of launch and first bytes.  Tried: 64 x 64
 // tiles the same way (never the best: M = 561, N = 1920, K = 6528 33 against 27); rows off the 16-byte grid read where
 // they lie (M = 1633, N = 163, K = 5834 20.9 against 17.2 for the tiles that stage them), which are copied onto the grid

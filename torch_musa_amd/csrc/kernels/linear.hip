@@ -882,7 +882,7 @@ bool phased_ring_preferred(int64_t M, int64_t N, int64_t K) {
 //   up to 48 rows weights stream as fast (41 x 5712 -> 144 9.0 | 10.0, 37 x 6592 -> 1664 10.6 | 12.0, 23 x 8128 -> 448
 //     8.5 | 9.9) but for more than 32 from K = 7680 on: 38 x 9408 -> 432 14.4 | 12.2, 46 x 8960 -> 768 13.7 | 10.6.
 // The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and 32 Mi weights: their tests hold them to it, although
-// 116 x 4480 -> 1728 takes 15.3 | 10.7 (117 x 6272 -> 1472 19.5 | 12.8).  Measured up to K = 12288.  Returns the channels per
+// 116 x 4480 -> 1728 takes 15.2 | 12.2 (117 x 6272 -> 1472 15.5 | 10.4).  Measured up to K = 12288.  Returns the channels per
 // tile, 0: not such a shape.
 constexpr int64_t kWloopMaxK = 12288, kWloopRingMinK = 5632;
 int wloop_tile(int64_t M, int64_t N, int64_t K) {
