@@ -37,7 +37,7 @@ def test_ring_and_tile_edges(cabi, cfg, k, m, n):  # noqa: F811
     (1024, 1024, 1280), (1025, 1024, 1280),                                              # ... in one
     (422, 3904, 5824), (422, 3904, 5808), (133, 4100, 4112),                             # 128 x 64
     (512, 8192, 1536), (513, 8192, 1536), (500, 8100, 1520), (254, 11264, 1552),         # 128 x 128, a round and more
-    (1535, 2900, 4112), (1537, 2900, 4112), (1537, 2900, 8208), (887, 5280, 2576),       # ... or 128 x 256, half a round
+    (1535, 2900, 4112), (1537, 2900, 4112), (1537, 2900, 8208), (887, 5280, 2576), (575, 8100, 4112), (577, 8100, 4112),       # ... or 128 x 256, half a round
     (900, 8100, 1088), (900, 8100, 1104)])
 @pytest.mark.parametrize("x_signed", [False, True])
 def test_the_choice(cabi, m, n, k, x_signed):  # noqa: F811

@@ -1354,9 +1354,9 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     else if (t128x256 > 256 && rows_used(256))
       cfg = t256 > 256 && t256 <= 400 ? 17 : 6;  // 6: 8 waves of 128x64, operands copied straight into LDS
     else if (t128x256 >= 160 && rows_used(128))
-      // (barely more than half a round of them, against a long K and fewer than 1536 rows: 128x128 tiles, at most 304,
+      // (barely more than half a round of them, against a long K and fewer than 1536 rows: 128x128 tiles, at most 320 (304),
       // all resident at once; the branch of 128x128 tiles below has the figures)
-      cfg = K >= 4096 && nblk(128, 128) <= 304 && (M < 1536 || K > 8192) ? 7 : cfg128x256;
+      cfg = K >= 4096 && nblk(128, 128) <= (M < 576 ? 304 : 320) && (M < 1536 || K > 8192) ? 7 : cfg128x256;
     else if (N >= 2048 && (N >= 4096 || K >= 4096) && nblk(64, 64) > 256 && (nblk(64, 128) <= 256 || M <= 64))
       // a few hundred rows whose 128 x 128 tiles would leave half the chip idle and whose
       // 64 x 64 tiles need a second round: 64 rows x 128 channels, one round (K = N = 4096,
@@ -1372,12 +1372,13 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     else if (nblk(128, 128) >= 128 && M > 64)  // (64 tiles: 64x64 wins, 15.2 against 17.9 us at M = 256, K = N = 4096;
                                                // up to 64 rows half of every tile is padding: M = 64, N = 16384, K = 4096:
                                                // 27.5 us against 17.5 us for the 64 x 64 tiles that walk K in phases)
-      // (just past a round of them 128 x 256 ones are more than half a round: behind up to 304 tiles of fewer rows against
-      // many channels or of K beyond 8192, 128 x 128 | 128 x 256: M = 374, N = 12208, K = 8304 65 | 76, M = 887, N = 5280,
-      // K = 3520 28.7 | 30.3, M = 1234, N = 3440, K = 4992 33.8 | 36.5, M = 1650, N = 2512, K = 8960 55.2 | 61.3; ahead with
+      // (just past a round of them 128 x 256 ones are more than half a round: behind up to 320 tiles (304 below 576 rows) of
+      // fewer rows against many channels or of K beyond 8192, 128 x 128 | 128 x 256: M = 374, N = 12208, K = 8304 65 | 76, M = 887, N = 5280,
+      // K = 3520 28.7 | 30.3, M = 1234, N = 3440, K = 4992 33.8 | 36.5, M = 640, N = 8192, K = 4096 29.3 | 31.3, M = 1650, N = 2512, K = 8960 55.2 | 61.3; ahead with
       // more rows or tiles: M = 3613, N = 1216, K = 4288 33.5 | 26.3, M = 2547, N = 1680, K = 4592 39.0 | 27.9, M = 4591,
-      // N = 944, K = 7552 45.8 | 40.6, M = 479, N = 9984, K = 2816 27.8 | 24.9, M = 695, N = 8688, K = 5824 53.1 | 47.2)
-      cfg = K > 2560 && nblk(128, 128) > 256 && rows_used(128) && (nblk(128, 128) > 304 || (M >= 1536 && K <= 8192)) ? cfg128x256 : 7;
+      // N = 944, K = 7552 45.8 | 40.6, M = 479, N = 9984, K = 2816 27.8 | 24.9, M = 490, N = 10032, K = 5440
+      // 50.1 | 46.0, M = 695, N = 8688, K = 5824 53.1 | 47.2)
+      cfg = K > 2560 && nblk(128, 128) > 256 && rows_used(128) && (nblk(128, 128) > (M < 576 ? 304 : 320) || (M >= 1536 && K <= 8192)) ? cfg128x256 : 7;
     else if (onepass_ok && K >= 3072 && K <= kWringMaxK && nblk(64, 64) <= 256 && N * K <= (int64_t{3} << 23))
       // one round of 64 x 64 tiles against a long K: eight waves split K, weights through
       // registers, activations through a ring per wave, no barrier before the partial tiles
