@@ -270,7 +270,7 @@ def main():
                   (2017, 168, 1344), (300, 2048, 1536), (642, 2304, 1920), (1024, 2048, 2048), (4096, 2048, 2048),
                   (131, 3845, 2128), (176, 2880, 2496), (512, 2560, 2560), (2560, 2560, 2560), (783, 1856, 3584),
                   (192, 3072, 3584)]
-        candidates = (1, 2, 3, 6, 7, 8, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28)
+        candidates = (1, 2, 3, 6, 7, 8, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30)
         rows = []
         for (Ms, Ns, Ks) in shapes:
             sets = max(2, min(40, (600 << 20) // (Ns * Ks)))
@@ -312,7 +312,7 @@ def main():
                 c_ = cabi.linear_kernel_choice(Ms, Ns, Ks, workspace=wbytes > 0, forced=cfg + 1)
                 if c_["kernel"] - 1 != cfg or cfg == auto["kernel"] - 1:
                     continue          # refused, or replaced by another kernel
-                if c_["blocks"] > 8192 or (cfg in (2, 14, 21, 24, 25, 26, 27) and Ms * Ns > 1 << 22):
+                if c_["blocks"] > 8192 or (cfg in (2, 14, 21, 24, 25, 26, 27, 29, 30) and Ms * Ns > 1 << 22):
                     continue          # small tiles on a large product: not a candidate
                 others[cfg] = round(timed(cfg), 2)
             best = min(others, key=others.get) if others else None

@@ -276,9 +276,9 @@ typedef struct tmq_linear_desc {
 
 int tmq_linear(const tmq_linear_desc* desc, tmq_stream_t stream);
 
-/* Bytes of workspace that tmq_linear / tmq_linear_f32 / tmq_linear_acc32 can
- * use for this problem size; 0 when the single-launch kernels are chosen
- * anyway.  No counterpart in the reference: muDNN allocates its own scratch
+/* Bytes of workspace for a split along K of this problem size; 0 where it is
+ * never split.  tmq_linear / tmq_linear_f32 / tmq_linear_acc32 split where no
+ * single-launch kernel is ahead of that, and always when the split is pinned.  No counterpart in the reference: muDNN allocates its own scratch
  * through the InternalMemAlloc callback (torch_musa/csrc/aten/utils/Utils.cpp:79-153). */
 int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /* Everything the call can make use of as `workspace`: the above, and for
@@ -300,8 +300,7 @@ int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int3
  * here so that the choice and every kernel's preconditions can be swept on the
  * host over thousands of shapes. */
 typedef struct tmq_linear_choice {
-  int32_t kernel;        /* value that pins this kernel in tmq_linear_desc::kernel (configuration + 1; 3 with tiles of
-                            32 rows: 30 pins those of 32 channels, 31 those of 64);
+  int32_t kernel;        /* value that pins this kernel in tmq_linear_desc::kernel (configuration + 1);
                             0: no kernel takes the shape (TMQ_ERR_UNSUPPORTED from the call) */
   int32_t tile_rows;     /* activation rows per workgroup tile (0: plain kernel) */
   int32_t tile_channels; /* output channels per workgroup tile */

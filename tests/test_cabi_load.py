@@ -226,6 +226,11 @@ def _check_choice(c, m, n, k, ldx, out, workspace, misaligned, forced=0, cus=256
         if forced == 0:                             # rows that share the streamed weights, or a short K
             assert k >= 1024 and m <= 32 and (m <= 16 or 10240 <= n <= 20480), what
         return
+    elif cfg in (29, 30):                           # 32 rows, eight waves walk their shares of K in pieces: 32-bit offsets
+        assert (bm, bn) == (32, 32 * (cfg - 28)) and c["waves"] == 8 and c["blocks"] == tiles, what    # over a tile's rows
+        assert k <= 2 ** 23 and ldx <= 2 ** 23 and n < 2 ** 29 and _ceil(m, 32) <= 65535, what
+        if forced == 0:                             # one round, K beyond the kernels that hold a wave's share at once
+            assert 4096 < k <= 12288 and m > 32 and tiles <= 256, what
     else:                                           # register-staged tiles take any aligned shape
         assert cfg in (0, 1, 2, 3, 4, 5, 22, 23), what
     if forced == 0 and cfg in (22, 23):             # a few hundred rows: one round of oblong tiles; up to 64 rows: any number
@@ -259,6 +264,10 @@ def test_automatic_kernel_choice_keeps_every_kernels_preconditions():
                 assert c["kernel"] != 0, (m, n, k, ldx, out, workspace)      # the automatic choice always runs
                 _check_choice(c, m, n, k, ldx, out, workspace, False)
                 seen.add(c["kernel"] - 1)
+                # the reported value pins what was reported
+                pinned = cabi.linear_kernel_choice(m, n, k, ldx, out, workspace, forced=c["kernel"])
+                assert [pinned[f] for f in ("kernel", "tile_rows", "tile_channels", "splits", "split_stages", "blocks")] == \
+                    [c[f] for f in ("kernel", "tile_rows", "tile_channels", "splits", "split_stages", "blocks")], (m, n, k, c)
     # huge pitches and K: the 32-bit offset limits of the direct-copy kernels
     for m, n, k, ldx in ((4096, 11008, 4096, 2 ** 23 + 16), (4096, 11008, 2 ** 23 + 64, 2 ** 23 + 64),
                          (512, 4096, 4096, 2 ** 24), (128, 1024, 1024, 2 ** 23 + 16), (64, 4096, 4096, 2 ** 23 + 16)):
@@ -269,7 +278,7 @@ def test_automatic_kernel_choice_keeps_every_kernels_preconditions():
             seen.add(c["kernel"] - 1)
     c = cabi.linear_kernel_choice(300, 500, 4096, misaligned=True)
     assert c["kernel"] == 10
-    assert seen >= {2, 3, 7, 8, 9, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28}, sorted(seen)
+    assert seen >= {2, 3, 7, 8, 9, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30}, sorted(seen)
     # the benchmark configurations
     assert cabi.linear_kernel_choice(4096, 11008, 4096)["kernel"] - 1 == 20
     assert cabi.linear_kernel_choice(4096, 11008, 4096)["blocks"] == 256
@@ -285,7 +294,7 @@ def test_forced_kernels_run_inside_their_preconditions_or_not_at_all():
     rng = np.random.default_rng(21)
     refused = 0
     for m, n, k, ldx in _random_linear_shapes(rng, 1500):
-        for cfg in (0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28):
+        for cfg in (0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 14, 17, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30):
             for out in ("bytes", "acc32"):
                 c = cabi.linear_kernel_choice(m, n, k, ldx, out, workspace=True, forced=cfg + 1)
                 if c["kernel"] == 0:

@@ -1720,7 +1720,7 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     case 28: bm = 16 * static_cast<int>(ceil_div(M, 16)), bn = 16, waves = resident_pair(M, N, K, compute_units) ? 8 : kResidentWaves; break;
     default: break;  // 9: one thread per four outputs
   }
-  out->kernel = (forced_kernel == 0 && (c.cfg == 29 || c.cfg == 30) ? 2 : c.cfg) + 1;  // (see tmq_linear_choice)
+  out->kernel = c.cfg + 1;
   out->tile_rows = bm;
   out->tile_channels = bn;
   out->waves = waves;
