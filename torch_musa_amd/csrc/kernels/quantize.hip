@@ -750,7 +750,7 @@ __device__ __forceinline__ float dequantize_fq_one(uint32_t byte, float zp, floa
 
 // An Op: P, the parameters of a channel; load4 / load1, conv4 (four values of up to four
 // channels), conv1, put4 / put1; zp_outside, the range check of a channel's zero point.
-template <bool SIGNED, bool THROUGH = false>
+template <bool SIGNED>
 struct PcQuantize {
   // fp32 -> codes, double scales, int64 zero points
   static constexpr int kAccesses = 4;
@@ -781,10 +781,7 @@ struct PcQuantize {
                                               packed);
     return SIGNED ? packed ^ 0x80808080u : packed;
   }
-  __device__ __forceinline__ void put4(int64_t i, Out4 v) const {
-    if constexpr (THROUGH) st4_through(q + i, v);
-    else *reinterpret_cast<uint32_t*>(q + i) = v;
-  }
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
   __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_one<SIGNED>(v, p.inv, p.zp));
   }
@@ -823,7 +820,7 @@ struct PcDequantize {
   __device__ __forceinline__ void put1(int64_t i, In1 b, P p) const { r[i] = dequantize_pc_one<SIGNED>(b, p.zp, p.scale); }
 };
 
-template <bool SIGNED, bool THROUGH = false>
+template <bool SIGNED>
 struct PcfQuantize {
   // fp32 -> codes, float scales and float zero points
   static constexpr int kAccesses = 4;
@@ -850,10 +847,7 @@ struct PcfQuantize {
     return quantize_fq_one<SIGNED>(v.x, p[0].inv, p[0].zp) | (quantize_fq_one<SIGNED>(v.y, p[1].inv, p[1].zp) << 8) |
            (quantize_fq_one<SIGNED>(v.z, p[2].inv, p[2].zp) << 16) | (quantize_fq_one<SIGNED>(v.w, p[3].inv, p[3].zp) << 24);
   }
-  __device__ __forceinline__ void put4(int64_t i, Out4 v) const {
-    if constexpr (THROUGH) st4_through(q + i, v);
-    else *reinterpret_cast<uint32_t*>(q + i) = v;
-  }
+  __device__ __forceinline__ void put4(int64_t i, Out4 v) const { *reinterpret_cast<uint32_t*>(q + i) = v; }
   __device__ __forceinline__ void put1(int64_t i, In1 v, P p) const {
     q[i] = static_cast<uint8_t>(quantize_fq_one<SIGNED>(v, p.inv, p.zp));
   }
@@ -889,6 +883,13 @@ struct PcfDequantize {
     __builtin_nontemporal_store(o, reinterpret_cast<v4f*>(r + i));
   }
   __device__ __forceinline__ void put1(int64_t i, In1 b, P p) const { r[i] = dequantize_fq_one<SIGNED>(b, p.zp, p.scale); }
+};
+
+// A quantizer whose codes leave past the L2s.
+template <class Op>
+struct PcThrough : Op {
+  explicit PcThrough(const Op& op) : Op(op) {}
+  __device__ __forceinline__ void put4(int64_t i, typename Op::Out4 v) const { st4_through(this->q + i, v); }
 };
 
 // The range check of the zero points, which the caller has to raise an error for before it
@@ -1131,7 +1132,6 @@ inline unsigned grid_for(int64_t work_items, int64_t per_block, int64_t cap) {
   return static_cast<unsigned>(g);
 }
 
-bool pc_rows_take(int64_t inner) { return inner % 4 == 0 && inner >= kPcRowsMinInner; }
 // Codes that leave past the L2s, us without | with them, both directions: [11008, 4096] 69.3 | 67.1, [12288, 8192] 146.8 | 144.7,
 // [12288, 12288] 217.9 | 215.1; [4096, 4096] level, [4096, 2048] 25.4 | 28.8 (as for the per-tensor quantizer above).
 bool pc_through(int64_t n) { return n >= (int64_t{28} << 20); }
@@ -1159,7 +1159,7 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
       return launch_status();
     }
   }
-  if (vec && pc_rows_take(inner)) {
+  if (vec && inner % 4 == 0 && inner >= kPcRowsMinInner) {
     constexpr int kPcAccesses = Op::kAccesses;
     const int64_t per_run = kPcThreads * 4;
     int lg_us = 0;
@@ -1167,9 +1167,15 @@ int launch_per_channel(const Op& op, int64_t outer, int64_t C, int64_t inner, bo
     const int64_t segs = ceil_div(inner, per_run << lg_us);
     const int64_t row_groups = ceil_div(outer * C, kPcAccesses >> lg_us);
     if (segs < 0x7fffffff && row_groups < 0x7fffffff / segs) {
-      enqueue(pc_rows_kernel<Op>, dim3(static_cast<unsigned>(row_groups * segs + extra)), dim3(kPcThreads), 0, s,
-              op, outer * C, C, inner, lg_us, static_cast<uint32_t>(segs), check);
-      return launch_status();
+      const auto rows = [&](const auto& stores) {
+        enqueue(pc_rows_kernel<std::decay_t<decltype(stores)>>, dim3(static_cast<unsigned>(row_groups * segs + extra)),
+                dim3(kPcThreads), 0, s, stores, outer * C, C, inner, lg_us, static_cast<uint32_t>(segs), check);
+        return launch_status();
+      };
+      if constexpr (std::is_same_v<typename Op::Out4, uint32_t>) {  // a quantizer
+        if (pc_through(n)) return rows(PcThrough<Op>(op));
+      }
+      return rows(op);
     }
   }
   if (inner >= 4 && inner <= kPcFlatMaxExtent && C <= kPcFlatMaxExtent && ceil_div(n, kPcFlatSpan) < 0x7fffffff) {
@@ -1488,19 +1494,16 @@ TMQ_EXPORT int tmq_per_channel(const tmq_per_channel_desc* d, tmq_stream_t strea
   auto* f = static_cast<float*>(d->fp32);
   auto* q = static_cast<uint8_t*>(d->codes);
   const bool vec = aligned(f, 16) && aligned(q, 4);
-  const bool through = !d->dequantize && vec && pc_rows_take(d->inner) && pc_through(d->outer * d->channels * d->inner);
   auto go = [&](const auto& op) { return launch_per_channel(op, d->outer, d->channels, d->inner, vec, check, s); };
   if (d->float_qparams) {
     auto* sc = static_cast<const float*>(d->scales);
     auto* zp = static_cast<const float*>(d->zero_points);
     if (d->dequantize) return d->q_signed ? go(PcfDequantize<true>{q, f, sc, zp}) : go(PcfDequantize<false>{q, f, sc, zp});
-    if (through) return d->q_signed ? go(PcfQuantize<true, true>{f, q, sc, zp}) : go(PcfQuantize<false, true>{f, q, sc, zp});
     return d->q_signed ? go(PcfQuantize<true>{f, q, sc, zp}) : go(PcfQuantize<false>{f, q, sc, zp});
   }
   auto* sc = static_cast<const double*>(d->scales);
   auto* zp = static_cast<const int64_t*>(d->zero_points);
   if (d->dequantize) return d->q_signed ? go(PcDequantize<true>{q, f, sc, zp}) : go(PcDequantize<false>{q, f, sc, zp});
-  if (through) return d->q_signed ? go(PcQuantize<true, true>{f, q, sc, zp}) : go(PcQuantize<false, true>{f, q, sc, zp});
   return d->q_signed ? go(PcQuantize<true>{f, q, sc, zp}) : go(PcQuantize<false>{f, q, sc, zp});
 }
 
