@@ -61,26 +61,63 @@ def test_conv(b, h, w, ic, oc, k, groups, post):
     assert whole.unique().numel() > 50
 
 
-@pytest.mark.parametrize("m,k,n", [
-    (1000, 512, 1600),    # 1.6 MB: tiles
-    (1000, 512, 1568),    # just below
-    (1000, 512, 1610),    # off the 16-channel grid
-    (700, 1024, 2304),
-    (4133, 1024, 1040),   # a last row tile and a last 16 channels
-    (5000, 1024, 4096),   # persistent
-    (2048, 128, 2048),    # one or two stages
-    (401, 4096, 4096),
+# Products whose tiles may write outputs of any size: past the L2s up to 24 MiB, where channels lie on the 64-byte grid up to
+# 52 MiB (256 x 256 tiles there at any size), against the plain kernel, which has ordinary stores only.
+@pytest.mark.parametrize("n,rows", [(272, (92521, 92522)), (4096, (13312, 13313))])
+@pytest.mark.parametrize("cfg,k", [(1, 384), (2, 384), (3, 384), (7, 384), (17, 384), (20, 384), (1, 64), (2, 64)])
+@pytest.mark.parametrize("x_signed", [False, True])
+def test_products_on_either_side_of_the_lines(n, rows, cfg, k, x_signed):
+    from torch_musa_amd import cabi
+    lo, hi, dt = (-128, 128, torch.int8) if x_signed else (0, 256, torch.uint8)
+    gen = torch.Generator("cuda").manual_seed(n + k)
+    pw = cabi.PackedLinear(torch.randint(-127, 128, (n, k), generator=gen, device="cuda").to(torch.int8))
+    ws = torch.rand(n, generator=gen, device="cuda") * 1e-3 + 1e-4
+    bias = torch.randn(n, generator=gen, device="cuda")
+    for m in rows:
+        x = torch.randint(lo, hi, (m, k), generator=gen, device="cuda").to(dt)
+        for pitch in {n, 272 if n == 272 else 4160}:   # rows of a wider output as well
+            say("product", m, n, k, cfg, x_signed, pitch)
+            outs = []
+            for pin in (9, cfg):
+                y = torch.full((m, pitch), 77, dtype=dt, device="cuda")
+                cabi.force_linear_config(pin)
+                try:
+                    outs.append(cabi.linear(x, pw, 0.05, 3, ws, bias, k ** 0.5 / 100, 10 if x_signed else 100, out=y[:, :n]))
+                finally:
+                    cabi.force_linear_config(-1)
+                assert bool((y[:, n:] == 77).all())
+            assert torch.equal(*outs)
+            assert outs[0].unique().numel() > 100
+
+
+# Implicit GEMMs likewise: two images past the line (ordinary stores), each by itself below it.
+@pytest.mark.parametrize("h,w,ic,oc,tile", [
+    (217, 214, 288, 272, (0, 1)), (217, 214, 288, 272, (128, 1)), (217, 214, 288, 272, (256, 1)),
+    (653, 653, 144, 64, (128, 1)),                                       # whole lines
+    (513, 512, 32, 48, (0, 0)), (397, 397, 32, 80, (0, 0)),              # the k order walked, 256 x 64 and 128 x 128
 ])
-def test_linear(m, k, n):
-    say("linear", m, k, n)
-    gen = torch.Generator("cuda").manual_seed(m + n)
-    x = torch.quantize_per_tensor(torch.randn(m, k, device="cuda", generator=gen), 8.0 / 255, 128, torch.quint8)
-    packed = OPS.linear_prepack(weight(gen, n, k), torch.randn(n, device="cuda", generator=gen))
-    scale = 8 * k ** 0.5 / 255
-    whole = OPS.linear(x, packed, scale, 128).int_repr()
-    step = max(1, (1 << 20) // n)
-    for lo in range(0, m, step):
-        assert torch.equal(whole[lo:lo + step], OPS.linear(x[lo:lo + step], packed, scale, 128).int_repr()), lo
+def test_implicit_gemm_on_either_side_of_the_lines(h, w, ic, oc, tile):
+    from torch_musa_amd import cabi
+    say("implicit GEMM", h, w, ic, oc, tile)
+    gen = torch.Generator("cuda").manual_seed(oc + ic)
+    x = torch.randint(0, 256, (2, h, w, ic), generator=gen, device="cuda").to(torch.uint8)
+    wq = torch.randint(-127, 128, (oc, 1, 1, ic), generator=gen, device="cuda").to(torch.int8)
+    ws = torch.rand(oc, generator=gen, device="cuda") * 1e-3 + 1e-4
+    bias = torch.randn(oc, generator=gen, device="cuda") * 0.1
+
+    def run(xs):
+        g = cabi.conv_geom(tuple(xs.shape), tuple(wq.shape), (1, 1), (0, 0), (1, 1), 1)
+        cabi.force_conv_path(2)
+        cabi.force_conv_tile(*tile)
+        try:
+            return cabi.conv2d(xs, cabi.PackedConv2d(wq, g), g, 0.03, 60, ws, bias, ic ** 0.5 / 400, 100)
+        finally:
+            cabi.force_conv_path(-1)
+            cabi.force_conv_tile(0, 0)
+
+    whole = run(x)
+    for i in range(2):
+        assert torch.equal(whole[i:i + 1], run(x[i:i + 1].contiguous()))
     assert whole.unique().numel() > 100
 
 

@@ -327,15 +327,23 @@ __global__ __launch_bounds__(256) void conv_plain_kernel(ConvShape s, PlainArgs 
   }
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, bool DMA, int KW = 1, class XSRC>
+template <int BM, int BN, int WM, int WN, int MODE, bool DMA, int KW = 1, bool THROUGH = true, class XSRC>
 int launch_conv_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   uint32_t lds = 0;
   if constexpr (std::is_same<XSRC, XConvTable>::value) lds = conv_table_bytes(xs.chunks);
-  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, DMA ? 3 : 4, DMA, KW>,
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, DMA ? 3 : 4, DMA, KW, false, THROUGH>,
           dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), lds, s, a, xs);
   return launch_status();
+}
+// Tiles that are chosen for outputs of any size (several wave groups: up to 256 and 512 tiles).
+template <int BM, int BN, int WM, int WN, int MODE, bool DMA, class XSRC>
+int launch_conv_gemm_any_size(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
+  if constexpr (MODE != kOutAcc32) {
+    if (!bytes_through(a)) return launch_conv_gemm<BM, BN, WM, WN, MODE, DMA, 1, false>(a, xs, s);
+  }
+  return launch_conv_gemm<BM, BN, WM, WN, MODE, DMA>(a, xs, s);
 }
 
 // Tiles of the implicit GEMM.  kConvGroups2/4, kConvTall2: k-split wave groups, register staging (64 x 64 and 128 x 64).
@@ -412,12 +420,12 @@ bool pointwise_gemm_first(const ConvShape& s, const PostOps& po, int64_t halo_ro
 template <int MODE>
 int launch_conv_gemm_tile(ConvGemmTile tile, const GemmArgs& a, const XConvTable& xs, hipStream_t s) {
   switch (tile) {
-    case kConv64: return launch_conv_gemm<64, 64, 2, 2, MODE, true>(a, xs, s);
+    case kConv64: return launch_conv_gemm_any_size<64, 64, 2, 2, MODE, true>(a, xs, s);
     case kConvGroups2: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
     case kConvGroups4: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 4>(a, xs, s);
     case kConvTall2: return launch_conv_gemm<128, 64, 2, 2, MODE, false, 2>(a, xs, s);
-    case kConv128: return launch_conv_gemm<128, 128, 2, 2, MODE, true>(a, xs, s);
-    case kConv256: return launch_conv_gemm<128, 256, 2, 4, MODE, true>(a, xs, s);
+    case kConv128: return launch_conv_gemm_any_size<128, 128, 2, 2, MODE, true>(a, xs, s);
+    case kConv256: return launch_conv_gemm_any_size<128, 256, 2, 4, MODE, true>(a, xs, s);
     case kConvRows256: break;
   }
   return TMQ_ERR_UNSUPPORTED;
@@ -439,12 +447,12 @@ ConvGemmTile conv_walk_tile(int64_t M, int64_t N, int64_t stages) {
 template <int MODE>
 int launch_conv_gemm_walk(ConvGemmTile tile, const GemmArgs& a, const XConv& xs, hipStream_t s) {
   switch (tile) {
-    case kConv64: return launch_conv_gemm<64, 64, 2, 2, MODE, false>(a, xs, s);
+    case kConv64: return launch_conv_gemm_any_size<64, 64, 2, 2, MODE, false>(a, xs, s);
     case kConvGroups2: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 2>(a, xs, s);
     case kConvGroups4: return launch_conv_gemm<64, 64, 2, 2, MODE, false, 4>(a, xs, s);
     case kConvTall2: return launch_conv_gemm<128, 64, 2, 2, MODE, false, 2>(a, xs, s);
-    case kConvRows256: return launch_conv_gemm<256, 64, 4, 1, MODE, false>(a, xs, s);
-    case kConv128: return launch_conv_gemm<128, 128, 2, 2, MODE, false>(a, xs, s);
+    case kConvRows256: return launch_conv_gemm_any_size<256, 64, 4, 1, MODE, false>(a, xs, s);
+    case kConv128: return launch_conv_gemm_any_size<128, 128, 2, 2, MODE, false>(a, xs, s);
     case kConv256: break;
   }
   return TMQ_ERR_UNSUPPORTED;

@@ -162,6 +162,19 @@ struct GemmArgs {
   int64_t split_stride = 0;
 };
 
+// Whether a product's whole 16 bytes leave past the L2s (st16_through).  Us without | with: 4096 x 1024 -> 1024 11.1 | 10.0,
+// 8192 x 512 -> 2048 19.8 | 17.2, 1024 x 1024 -> 4096 11.8 | 10.8, 384 x 768 -> 3072 5.2 | 5.1, 512 x 1024 -> 1024 level.
+// Channels off the 64-byte grid: several blocks write parts of a line, which an L2 merges where it keeps the line for a while;
+// past it each part travels by itself.  Up to 24 MiB 3 % ahead on average (33088 x 320 -> 304 10 MB 9 %; pixels likewise, 288 ->
+// 240 on 32 x 56 x 56 24 MB 21.5 | 18.4), then level or far behind from one part to the next (320 -> 272 on 32 x 56 x 56 27 MB
+// 28.6 | 28.3, on another part 29.6 | 34.8), and behind from 30 MB on (183823 x 320 -> 272 50 MB 1.4 times, 152777 x 96 -> 720
+// 110 MB 1.27 times, 320 -> 528 on 32 x 80 x 80 85 | 105).  On that grid 2 to 10 % ahead up to 52 MiB (with a dequantizer
+// behind them 2 to 5 % up to 28 MiB and level from there), 1 % behind past 80 MB.
+// The host tells: a test in the kernel takes 0.05 us and 1 % of a longer one.
+constexpr int64_t kThroughLines = int64_t{52} << 20, kThroughParts = int64_t{24} << 20;
+inline bool whole_lines(const GemmArgs& a) { return a.N % 64 == 0 && a.ldy % 64 == 0 && a.n_off % 64 == 0; }
+inline bool bytes_through(const GemmArgs& a) { return a.M * a.N <= (whole_lines(a) ? kThroughLines : kThroughParts); }
+
 struct XQuant {
   float scale;
   int32_t coef;  // multiplies colsum[n] into the accumulator start
@@ -616,8 +629,9 @@ __device__ __forceinline__ uint32_t requant4_post(const int (&raw)[4], v4f bdiv,
 // all walk the longest run; a group whose run is shorter (the stage count is no
 // multiple of KW) stores zeros for the activations of the stages it lacks.  Every
 // group has at least one stage of its own.
+// THROUGH: byte outputs on the 16-byte grid leave past the L2s (bytes_through).
 template <int BM, int BN, int WM, int WN, int MODE, class XSRC, int PD = 4, bool WDMA = false, int KW = 1,
-          bool XWIDE = false>
+          bool XWIDE = false, bool THROUGH = true>
 __global__ __launch_bounds__(WM* WN* KW* kWave, (WDMA && WM * WN == 4 && (BM / WM) * (BN / WN) <= 128 * 64) ? 2 : 1)
 void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
   constexpr int NT = WM * WN * kWave;   // threads of one group
@@ -1393,8 +1407,6 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       requant_tile(std::true_type{});
     }
     __syncthreads();
-    // Whole 16 bytes leave past the L2 (us without | with: 4096 x 1024 -> 1024 11.1 | 10.0, 8192 x 512 -> 2048 19.8 | 17.2,
-    // 1024 x 1024 -> 4096 11.8 | 10.8, 384 x 768 -> 3072 5.2 | 5.1, 512 x 1024 -> 1024 and 4096 x 4096 -> 11008 level).
     uint8_t* y = static_cast<uint8_t*>(a.y) + a.n_off;
     const bool vec_ok = ((a.ldy & 15) == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
     constexpr int kRowChunks = BN / 16;
@@ -1406,7 +1418,8 @@ void gemm_i8_kernel(GemmArgs a, XSRC xsrc) {
       const v4i v = ld16(&smem[row * kOutPitch + cc * 16]);
       uint8_t* dst = y + m * a.ldy + n;
       if (vec_ok && n + 16 <= a.N) {
-        st16_through(dst, v);
+        if constexpr (THROUGH) st16_through(dst, v);
+        else *reinterpret_cast<v4i*>(dst) = v;
       } else if (n + 16 <= a.N) {
         st16_any(dst, v);  // (a row pitch or pointer off the 16-byte grid)
       } else {

@@ -283,7 +283,7 @@ __global__ __launch_bounds__(BN * 4) void gemm_i8_onepass_kernel(GemmArgs a, XLi
       const v4i v = ld16(&sW[row * kPitch + cc * 16]);
       uint8_t* dst = y + m * a.ldy + n;
       if (vec_ok && n + 16 <= a.N) {
-        st16_through(dst, v);
+        st16_through(dst, v);  // (2 MB at most: see bytes_through)
       } else if (n + 16 <= a.N) {
         st16_any(dst, v);  // (a row pitch or pointer off the 16-byte grid)
       } else {

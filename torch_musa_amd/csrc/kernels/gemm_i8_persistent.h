@@ -31,7 +31,7 @@ namespace tmq {
 
 constexpr int kPersistThreads = 512;
 
-template <int MODE>
+template <int MODE, bool THROUGH>
 __global__ __launch_bounds__(kPersistThreads, 1) void gemm_i8_persistent_kernel(GemmArgs a, XLinear xsrc) {
   static_assert(MODE == kOutU8 || MODE == kOutS8 || MODE == kOutF32, "byte or float outputs");
   constexpr int BM = 256, BN = 256, WM = 2, WN = 4;
@@ -335,7 +335,8 @@ __global__ __launch_bounds__(kPersistThreads, 1) void gemm_i8_persistent_kernel(
         if (m < a.M && n < a.N) {
           uint8_t* dst = ybase + m * a.ldy + n;
           if (vec_ok && n + 16 <= a.N) {
-            st16_through(dst, v);  // (4096 x 1024 -> 4096 23.2 -> 21.3 us, 4096 x 11008 -> 4096 149.5 -> 147.7)
+            if constexpr (THROUGH) st16_through(dst, v);
+            else *reinterpret_cast<v4i*>(dst) = v;
           } else if (n + 16 <= a.N) {
             st16_any(dst, v);  // (a row pitch or pointer off the 16-byte grid)
           } else {

@@ -576,14 +576,22 @@ __global__ __launch_bounds__(256) void linear_plain_kernel(GemmArgs a, XLinear x
 }
 
 template <int BM, int BN, int WM, int WN, int MODE, int PD = 4, bool WDMA = false, int KW = 1, bool XWIDE = false,
-          class XSRC = XLinear>
+          bool THROUGH = true, class XSRC = XLinear>
 int launch_gemm(const GemmArgs& a, const XSRC& xs, hipStream_t s) {
   const int64_t blocks = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (blocks > 0x7fffffff) return TMQ_ERR_UNSUPPORTED;
   if (ceil_div(a.K, kBK) < KW) return TMQ_ERR_UNSUPPORTED;  // a stage for every wave group
-  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, PD, WDMA, KW, XWIDE>,
+  enqueue(gemm_i8_kernel<BM, BN, WM, WN, MODE, XSRC, PD, WDMA, KW, XWIDE, THROUGH>,
           dim3(static_cast<unsigned>(blocks)), dim3(WM * WN * KW * kWave), 0, s, a, xs);
   return launch_status();
+}
+// Tiles that are chosen for outputs of any size (the others run a round or a few of them, 13 MB at most).
+template <int BM, int BN, int WM, int WN, int MODE, int PD = 4, bool WDMA = false, bool XWIDE = false>
+int launch_gemm_any_size(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
+  if constexpr (MODE == kOutU8 || MODE == kOutS8) {
+    if (!bytes_through(a)) return launch_gemm<BM, BN, WM, WN, MODE, PD, WDMA, 1, XWIDE, false>(a, xs, s);
+  }
+  return launch_gemm<BM, BN, WM, WN, MODE, PD, WDMA, 1, XWIDE>(a, xs, s);
 }
 
 // 64 x 64 (64 x 128) tiles with all of K in LDS (K <= 1024; the caller checked the address ranges).
@@ -687,7 +695,17 @@ int launch_gemm_persistent(const GemmArgs& a, const XLinear& xs, hipStream_t s) 
     // several rounds: a multiple of 8 blocks, so that the tile sequence deals
     // every XCD its own run of tiles
     const int64_t grid = tiles <= cus ? tiles : cus / 8 * 8;
-    enqueue(gemm_i8_persistent_kernel<MODE>, dim3(static_cast<unsigned>(grid)), dim3(kPersistThreads), 0, s, a, xs);
+    const dim3 blocks(static_cast<unsigned>(grid)), threads(kPersistThreads);
+    // Whole lines leave past the L2s at any size, beside the next tile's products (us without | with: 4096 x 1024 -> 4096 23.2 |
+    // 21.3, 4096 x 11008 -> 4096 149.5 | 147.7, 4096 x 512 -> 11008 45 MB 42.7 | 37.7; 112 shapes of 6 to 120 MB 7 % ahead,
+    // none behind); parts of lines as for the other tiles (173660 x 768 -> 144 25 MB 46.6 | 52.2).
+    if constexpr (MODE != kOutF32) {
+      if (!whole_lines(a) && !bytes_through(a)) {
+        enqueue(gemm_i8_persistent_kernel<MODE, false>, blocks, threads, 0, s, a, xs);
+        return launch_status();
+      }
+    }
+    enqueue(gemm_i8_persistent_kernel<MODE, true>, blocks, threads, 0, s, a, xs);
     return launch_status();
   } else {
     return TMQ_ERR_UNSUPPORTED;
@@ -1546,14 +1564,14 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     }
     case 13: return run_split<MODE>(a, xs, c.split, workspace, dma_limits_ok(a.K, xs.ldx), s);
     case 0: return launch_gemm<256, 256, 2, 2, MODE>(a, xs, s);
-    case 1: return dma_limits_ok(a.K, xs.ldx) ? launch_gemm<128, 128, 2, 2, MODE, 3, true>(a, xs, s)
-                                              : launch_gemm<128, 128, 2, 2, MODE>(a, xs, s);
+    case 1: return dma_limits_ok(a.K, xs.ldx) ? launch_gemm_any_size<128, 128, 2, 2, MODE, 3, true>(a, xs, s)
+                                              : launch_gemm_any_size<128, 128, 2, 2, MODE>(a, xs, s);
     case 2: return c.groups == 2                  ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s)
                    : one_round_ring(a.M, a.N, a.K) && dma_limits_ok(a.K, xs.ldx)
                        ? launch_gemm<64, 64, 2, 2, MODE, 6, true>(a, xs, s)
-                   : dma_limits_ok(a.K, xs.ldx) ? launch_gemm<64, 64, 2, 2, MODE, 3, true>(a, xs, s)
-                                                : launch_gemm<64, 64, 2, 2, MODE>(a, xs, s);
-    case 3: return launch_gemm<256, 256, 2, 4, MODE, 3>(a, xs, s);
+                   : dma_limits_ok(a.K, xs.ldx) ? launch_gemm_any_size<64, 64, 2, 2, MODE, 3, true>(a, xs, s)
+                                                : launch_gemm_any_size<64, 64, 2, 2, MODE>(a, xs, s);
+    case 3: return launch_gemm_any_size<256, 256, 2, 4, MODE, 3>(a, xs, s);
     case 4: return launch_gemm<128, 256, 2, 2, MODE>(a, xs, s);
     case 5: return launch_gemm<256, 128, 2, 2, MODE>(a, xs, s);
     case 6: return launch_gemm<256, 256, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
@@ -1562,11 +1580,11 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     // stages: M = 1160, N = 2048, K = 11008 59.4 | 58 | 41.7; M = 1062, N = 2496, K = 6016 35.5 | - | 26.8; M = 617, N = 5952,
     // K = 1728 14.2 | 13.7 | 13.0; M = 752, N = 4800, K = 960 8.7 | 8.0 | 8.4; M = 254, N = 11264, K = 2480 20.3 | 19.8 | 23.5)
     case 7: return ceil_div(a.M, 128) * ceil_div(a.N, 128) > 256
-                       ? launch_gemm<128, 128, 2, 2, MODE, 3, true, 1, true>(a, xs, s)
+                       ? launch_gemm_any_size<128, 128, 2, 2, MODE, 3, true, true>(a, xs, s)
                    : a.K >= 1536 && a.K % kBK == 0 ? launch_gemm<128, 128, 2, 4, MODE, 6, true>(a, xs, s)
                                                    : launch_gemm<128, 128, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
     case 14: return launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, xs, s);
-    case 17: return launch_gemm<128, 256, 2, 4, MODE, 3, true>(a, xs, s);
+    case 17: return launch_gemm_any_size<128, 256, 2, 4, MODE, 3, true>(a, xs, s);
     case 19: return launch_gemm<128, 256, 2, 4, MODE, 3, true, 1, true>(a, xs, s);
     case 20: return launch_gemm_persistent<MODE>(a, xs, s);
     case 22: return oblong_ring(a.M, a.N, a.K, xs.ldx, 128, 64) ? launch_gemm<128, 64, 2, 2, MODE, 6, true>(a, xs, s)
