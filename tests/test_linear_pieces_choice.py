@@ -29,3 +29,11 @@ def test_choice_and_scratch():
         assert cabi.lib().tmq_linear_scratch_bytes(m, n, k - 1, 0) == _ceil(m * k, 256) * 256, what
         seen.add(c["tile_channels"])
     assert seen == {32, 64}
+
+
+def test_lines_between_128_x_128_and_128_x_256_tiles():
+    # (just past a round of the former, of many rows: the shapes that were measured on either side)
+    for m, n, k, kernel in ((1779, 2544, 7424, 7), (2018, 2432, 7616, 7), (1732, 2768, 7168, 7), (1979, 2496, 6528, 7),
+                            (1751, 2496, 5824, 19), (2613, 1792, 6800, 19), (3379, 1344, 7760, 19), (2798, 1536, 4160, 19),
+                            (1234, 3440, 4992, 7), (1650, 2512, 8960, 7), (479, 9984, 2816, 19), (640, 8192, 4096, 7)):
+        assert cabi.linear_kernel_choice(m, n, k, workspace=True)["kernel"] - 1 == kernel, (m, n, k)

@@ -1362,6 +1362,11 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     // against 31.0 us; N = 11008, K = 4096: 20.2 against 21.2 us)
     const int cfg_half =
         nblk(128, 64) <= 256 && (nblk(128, 64) > nblk(64, 128) || (M <= 96 && nblk(128, 64) == nblk(64, 128))) ? 22 : 23;
+    // Just past a round of 128 x 128 tiles, half a round of 128 x 256 ones is ahead behind many rows (us, 128 x 128 | 128 x 256:
+    // M = 2798, N = 1536, K = 4160 0.80 of the time, M = 3613, N = 1216, K = 4288 33.5 | 26.3; M = 2613, N = 1792, K = 6800 0.87, M =
+    // 3379, N = 1344, K = 7760 0.73), up to 2560 of them while K is no longer than 6144 (M = 1779, N = 2544, K = 7424 49.3 | 51.8,
+    // M = 2018, N = 2432, K = 7616 1.04 times, M = 1732, N = 2768, K = 7168 48.2 | 49.6).
+    const bool rows_ahead = M >= 1536 && K <= (M < 2560 ? 6144 : 8192);
     // Many rows against a short K are bound by the epilogue, and 256-channel tiles requantise the padding behind
     // N as well: 128 x 128 tiles where those pad a quarter less (M = 100352 pixels of a 56 x 56 feature map at batch
     // 32: N = 384, K = 96: 35.1 -> 27 us; N = 96, K = 384: 20.9 -> 15.7 us; N = 512, K = 128 has nothing to gain and
@@ -1372,9 +1377,9 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     else if (t128x256 > 256 && rows_used(256))
       cfg = t256 > 256 && t256 <= 400 ? 17 : 6;  // 6: 8 waves of 128x64, operands copied straight into LDS
     else if (t128x256 >= 160 && rows_used(128))
-      // (barely more than half a round of them, against a long K and fewer than 1536 rows: 128x128 tiles, at most 320 (304),
+      // (barely more than half a round of them, against a long K and not too many rows: 128x128 tiles, at most 320 (304),
       // all resident at once; the branch of 128x128 tiles below has the figures)
-      cfg = K >= 4096 && nblk(128, 128) <= (M < 576 ? 304 : 320) && (M < 1536 || K > 8192) ? 7 : cfg128x256;
+      cfg = K >= 4096 && nblk(128, 128) <= (M < 576 ? 304 : 320) && !rows_ahead ? 7 : cfg128x256;
     else if (N >= 2048 && (N >= 4096 || K >= 4096) && nblk(64, 64) > 256 && (nblk(64, 128) <= 256 || M <= 64))
       // a few hundred rows whose 128 x 128 tiles would leave half the chip idle and whose
       // 64 x 64 tiles need a second round: 64 rows x 128 channels, one round (K = N = 4096,
@@ -1390,13 +1395,15 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     else if (nblk(128, 128) >= 128 && M > 64)  // (64 tiles: 64x64 wins, 15.2 against 17.9 us at M = 256, K = N = 4096;
                                                // up to 64 rows half of every tile is padding: M = 64, N = 16384, K = 4096:
                                                // 27.5 us against 17.5 us for the 64 x 64 tiles that walk K in phases)
-      // (just past a round of them 128 x 256 ones are more than half a round: behind up to 320 tiles (304 below 576 rows) of
-      // fewer rows against many channels or of K beyond 8192, 128 x 128 | 128 x 256: M = 374, N = 12208, K = 8304 65 | 76, M = 887, N = 5280,
-      // K = 3520 28.7 | 30.3, M = 1234, N = 3440, K = 4992 33.8 | 36.5, M = 640, N = 8192, K = 4096 29.3 | 31.3, M = 1650, N = 2512, K = 8960 55.2 | 61.3; ahead with
-      // more rows or tiles: M = 3613, N = 1216, K = 4288 33.5 | 26.3, M = 2547, N = 1680, K = 4592 39.0 | 27.9, M = 4591,
-      // N = 944, K = 7552 45.8 | 40.6, M = 479, N = 9984, K = 2816 27.8 | 24.9, M = 490, N = 10032, K = 5440
-      // 50.1 | 46.0, M = 695, N = 8688, K = 5824 53.1 | 47.2)
-      cfg = K > 2560 && nblk(128, 128) > 256 && rows_used(128) && (nblk(128, 128) > (M < 576 ? 304 : 320) || (M >= 1536 && K <= 8192)) ? cfg128x256 : 7;
+      // (just past a round of them 128 x 256 ones are more than half a round.  Up to 320 tiles (304 below 576 rows), us, 128 x 128 |
+      // 128 x 256: M = 374, N = 12208, K = 8304 65 | 76, M = 887, N = 5280, K = 3520 28.7 | 30.3, M = 1234, N = 3440, K = 4992 33.8 | 36.5,
+      // M = 640, N = 8192, K = 4096 29.3 | 31.3, M = 1650, N = 2512, K = 8960 55.2 | 61.3; on 118 drawn shapes of that kind 128 x 128
+      // are 1 % ahead on average, 12 % at most, and up to 44 % behind with 1040 to 1536 rows at K below 4000 (M = 1209, N = 3328,
+      // K = 3520 28.1 | 22.9, M = 1168, N = 3728, K = 2640 24.7 | 22.0) or more than 2688 past K = 8192 (M = 2722, N = 1456, K =
+      // 9232 73 | 51), which no line here tells apart yet.  The other side of the lines: 11 % ahead on 176, 6 % behind at most;
+      // M = 479, N = 9984, K = 2816 27.8 | 24.9, M = 490, N = 10032, K = 5440
+      // 50.1 | 46.0, M = 695, N = 8688, K = 5824 53.1 | 47.2, M = 2547, N = 1680, K = 4592 39.0 | 27.9)
+      cfg = K > 2560 && nblk(128, 128) > 256 && rows_used(128) && (nblk(128, 128) > (M < 576 ? 304 : 320) || rows_ahead) ? cfg128x256 : 7;
     else if (onepass_ok && K >= 3072 && K <= kWringMaxK && nblk(64, 64) <= 256 && N * K <= (int64_t{3} << 23))
       // one round of 64 x 64 tiles against a long K: eight waves split K, weights through
       // registers, activations through a ring per wave, no barrier before the partial tiles
