@@ -898,13 +898,16 @@ bool phased_ring_preferred(int64_t M, int64_t N, int64_t K) {
 //     289 x 12128 -> 1600 28.6 | 21.5; not for more than 32 Mi weights, near level (54 x 5440 -> 7616 18.2 | 17.1), nor
 //     from K = 9216 on more than 20 Mi, where a split along K into two launches is ahead (114 x 10576 -> 2304 20.6 | 22.3);
 //   up to 48 rows weights stream as fast (41 x 5712 -> 144 9.0 | 10.0, 37 x 6592 -> 1664 10.6 | 12.0, 23 x 8128 -> 448
-//     8.5 | 9.9) but for more than 32 from K = 7680 on: 38 x 9408 -> 432 14.4 | 12.2, 46 x 8960 -> 768 13.7 | 10.6.
-// The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and 32 Mi weights: their tests hold them to it, although
-// 116 x 4480 -> 1728 takes 15.2 | 12.2 (117 x 6272 -> 1472 15.5 | 10.4).  Measured up to K = 12288.  Returns the channels per
-// tile, 0: not such a shape.
+//     8.5 | 9.9) but for more than 32 from K = 7680 on: 38 x 9408 -> 432 14.4 | 12.2, 46 x 8960 -> 768 13.7 | 10.6; up to 40 rows
+//     not against more than 17 Mi weights short of K = 10240 (34 x 7808 -> 3504 11.6 | 12.4, 34 x 9536 -> 3216 14.9 | 15.9, 40 x
+//     7872 -> 2816 11.8 | 12.4; 35 x 8768 -> 1584 0.80 of the time, 36 x 10752 -> 2304 0.90).
+// The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and 32 Mi weights, which their tests hold as the
+// automatic choice; measured, this kernel is ahead there throughout (128 x 4608 -> 256 14.7 | 7.3, 128 x 4288 -> 1296 14.4 | 8.7, 116 x
+// 4480 -> 1728 15.2 | 12.2).  Measured up to K = 12288.  Returns the channels per tile, 0: not such a shape.
 constexpr int64_t kWloopMaxK = 12288, kWloopRingMinK = 5632;
 int wloop_tile(int64_t M, int64_t N, int64_t K) {
   if (M <= (K >= 7680 ? 32 : 48) || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
+  if (M <= 40 && N * K > int64_t{17} << 20 && K < 10240) return 0;
   if (K < kWloopRingMinK && phased_ring_preferred(M, N, K)) return 0;
   if (ceil_div(M, 32) * ceil_div(N, 32) <= 256) return 32;
   if (M > 48 && ceil_div(M, 32) * ceil_div(N, 64) <= 256 && N * K <= int64_t{K < 9216 ? 32 : 20} << 20) return 64;
