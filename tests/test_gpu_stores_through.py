@@ -1,64 +1,96 @@
-"""Outputs large enough that their bytes leave past the L2s, against the same images (rows) in calls too small for that: the
-same bytes.  Either side of each line in sizes and channel counts; what the small calls give is compared with the oracle
-elsewhere."""
+"""Outputs whose bytes leave past the L2s, on either side of each rule's lines in sizes and channel counts, against ordinary
+stores of the same values: an output pointer off the 16-byte grid, the plain kernel, calls short of the line, or torch's own
+pooling.  The values themselves are compared with the oracle elsewhere."""
 import pytest
 import torch
 
-import torch_musa_amd  # noqa: F401  (registers the operators)
 from gpu_util import say
+from torch_musa_amd import cabi
 
 pytestmark = pytest.mark.gpu
-OPS = torch.ops.quantized
 
 
-def feature_map(gen, b, h, w, c):
-    x = torch.relu(torch.randn(b, h, w, c, device="cuda", generator=gen)).permute(0, 3, 1, 2)
-    return torch.quantize_per_tensor(x, 4.0 / 255, 0, torch.quint8)
-
-
-def weight(gen, *shape):
-    w = torch.randn(*shape, device="cuda", generator=gen)
-    scales = w.abs().flatten(1).amax(1).double() / 127
-    return torch.quantize_per_channel(w, scales, torch.zeros(shape[0], dtype=torch.long, device="cuda"), 0, torch.qint8)
+def off_grid(shape, dtype):
+    """An uninitialised output one byte past the grid, and the bytes around it, which have to stay."""
+    n = 1
+    for d in shape:
+        n *= d
+    flat = torch.full((n + 64,), 77, dtype=dtype, device="cuda")
+    return flat[1:n + 1].view(shape), [flat[:1], flat[n + 1:]]
 
 
 @pytest.mark.parametrize("b,h,w,ic,oc,k,groups,post", [
-    (10, 56, 53, 24, 56, 1, 1, ""),          # 1.7 MB, channels off the grid
-    (10, 56, 53, 24, 64, 1, 1, "relu"),      # 1.9 MB, a block of 64 channels
-    (30, 56, 53, 20, 24, 1, 1, "relu"),      # 2.1 MB, eight channels a lane
-    (17, 41, 57, 64, 80, 1, 1, "add"),       # a last block of 16 channels
+    (10, 56, 53, 24, 56, 1, 1, "none"),       # channels off the grid: never past the L2s
+    (10, 56, 53, 24, 64, 1, 1, "relu"),       # pointwise: a block of 64 channels
+    (30, 56, 53, 20, 24, 1, 1, "relu"),       # eight channels a lane
+    (17, 41, 57, 64, 80, 1, 1, "add"),        # a last block of 16 channels
     (17, 41, 57, 64, 96, 1, 1, "silu"),
-    (33, 56, 57, 24, 208, 1, 1, "relu"),     # past 20 MB, channel blocks on several CUs
-    (27, 56, 57, 24, 256, 1, 1, "relu"),     # past 20 MB, on one
-    (16, 41, 37, 64, 64, 3, 1, "relu"),      # halo tiles
+    (27, 56, 57, 24, 144, 1, 1, "relu"),      # parts of lines, 12.4 MB
+    (28, 56, 57, 24, 144, 1, 1, "relu"),      # 12.9 MB, past 12 MiB: ordinary stores
+    (28, 56, 57, 24, 144, 1, 1, "silu"),      # ... but behind SiLU
+    (34, 56, 57, 24, 192, 1, 1, "relu"),      # whole lines, 20.8 MB
+    (35, 56, 57, 24, 192, 1, 1, "relu"),      # 21.5 MB, past 20 MiB: ordinary
+    (27, 56, 57, 24, 256, 1, 1, "relu"),      # ... but where a pixel's channel blocks are one CU's
+    (18, 56, 57, 256, 384, 1, 1, "relu"),     # ... or the layer is wide
+    (16, 41, 37, 64, 64, 3, 1, "relu"),       # halo tiles
     (16, 41, 37, 64, 80, 3, 1, "add"),
-    (33, 56, 57, 64, 96, 3, 1, "relu"),      # past 8 MB, lines of several blocks
-    (30, 56, 57, 60, 60, 3, 60, "relu"),     # depthwise, 5.7 MB
-    (30, 56, 57, 66, 66, 3, 66, "relu"),     # off the 4-channel grid
-    (16, 29, 31, 256, 272, 3, 1, "relu"),    # implicit GEMM
-    (20, 61, 67, 3, 24, 3, 1, "relu"),       # images
+    (27, 56, 57, 64, 96, 3, 1, "relu"),       # lines of several blocks, 8.3 MB
+    (28, 56, 57, 64, 96, 3, 1, "relu"),       # 8.6 MB, past 8 MiB: ordinary
+    (24, 56, 57, 60, 60, 3, 60, "relu"),      # depthwise, 4.6 MB: ordinary below 4.5 MiB
+    (25, 56, 57, 60, 60, 3, 60, "relu"),      # 4.8 MB
+    (54, 56, 57, 96, 96, 5, 96, "relu"),      # 16.5 MB
+    (55, 56, 57, 96, 96, 5, 96, "relu"),      # 16.9 MB, past 16 MiB: ordinary
+    (30, 56, 57, 66, 66, 3, 66, "relu"),      # off the 4-channel grid
+    (30, 56, 57, 60, 60, 7, 60, "silu"),
+    (16, 29, 31, 256, 272, 3, 1, "relu"),     # implicit GEMM
+    (20, 61, 67, 3, 24, 3, 1, "relu"),        # images, of any size
     (3, 61, 67, 3, 64, 7, 1, "relu"),
-    (20, 61, 67, 1, 48, 3, 1, "relu"),       # byte runs
+    (20, 61, 67, 1, 48, 3, 1, "relu"),        # byte runs
 ])
-def test_conv(b, h, w, ic, oc, k, groups, post):
-    say("conv", b, h, w, ic, oc, k, groups, post)
+@pytest.mark.parametrize("out_signed", [False, True])
+def test_conv(b, h, w, ic, oc, k, groups, post, out_signed):
+    say("conv", b, h, w, ic, oc, k, groups, post, out_signed)
     gen = torch.Generator("cuda").manual_seed(b + oc)
-    x, accum = feature_map(gen, b, h, w, ic), feature_map(gen, b, h, w, oc)
-    packed = OPS.conv2d_prepack(weight(gen, oc, ic // groups, k, k), torch.randn(oc, device="cuda", generator=gen),
-                                [1, 1], [k // 2, k // 2], [1, 1], groups)
-    scale = 8 * (ic // groups * k * k) ** 0.5 / 255
+    x = torch.randint(0, 256, (b, h, w, ic), generator=gen, device="cuda").to(torch.uint8)
+    wq = torch.randint(-127, 128, (oc, k, k, ic // groups), generator=gen, device="cuda").to(torch.int8)
+    ws = torch.rand(oc, generator=gen, device="cuda") * 1e-3 + 1e-4
+    bias = torch.randn(oc, generator=gen, device="cuda") * 0.1
+    accum = torch.randint(0, 256, (b, h, w, oc), generator=gen, device="cuda").to(torch.uint8) if post == "add" else None
+    g = cabi.conv_geom(tuple(x.shape), tuple(wq.shape), (1, 1), (k // 2, k // 2), (1, 1), groups)
+    pw = cabi.PackedConv2d(wq, g)
+    scale, zp = (ic // groups * k * k) ** 0.5 / 400, 0 if out_signed else 100
+    dtype = torch.int8 if out_signed else torch.uint8
 
-    def run(lo, hi):
-        xs = x[lo:hi]
-        if post == "add":
-            return OPS.conv2d_add_relu(xs, accum[lo:hi], packed, scale, 3).int_repr()
-        op = {"": OPS.conv2d, "relu": OPS.conv2d_relu, "silu": OPS.conv2d_silu}[post]
-        return op(xs, packed, scale, 3).int_repr()
+    def run(out):
+        return cabi.conv2d_fused(x, pw, g, 0.03, 128, ws, bias, scale, zp, accum=accum, accum_scale=0.02, accum_zp=100,
+                                 activation="relu" if post == "add" else post, out_signed=out_signed, out=out)
 
-    whole = run(0, b)
-    for i in range(b):
-        assert torch.equal(whole[i:i + 1], run(i, i + 1)), i
-    assert whole.unique().numel() > 50
+    plain, around = off_grid((b, h, w, oc), dtype)
+    run(plain)
+    assert all(bool((a == 77).all()) for a in around)
+    on_grid = run(torch.full((b, h, w, oc), 77, dtype=dtype, device="cuda"))
+    assert torch.equal(on_grid, plain)
+    assert on_grid.unique().numel() > 50
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (700, 1024, 2304), (1000, 512, 1600), (1000, 512, 1610), (384, 768, 3072),   # tiles that are never large
+    (1000, 512, 1000), (517, 1008, 2048), (130, 640, 130),                       # all of K in LDS
+    (4133, 1024, 1040), (2048, 128, 2048), (401, 4096, 4096), (5000, 1024, 4096),
+])
+def test_products(m, k, n):
+    say("product", m, k, n)
+    gen = torch.Generator("cuda").manual_seed(m + n)
+    x = torch.randint(0, 256, (m, k), generator=gen, device="cuda").to(torch.uint8)
+    pw = cabi.PackedLinear(torch.randint(-127, 128, (n, k), generator=gen, device="cuda").to(torch.int8))
+    ws = torch.rand(n, generator=gen, device="cuda") * 1e-3 + 1e-4
+    bias = torch.randn(n, generator=gen, device="cuda")
+    plain, around = off_grid((m, n), torch.uint8)
+    outs = [cabi.linear(x, pw, 0.05, 128, ws, bias, k ** 0.5 / 100, 100, out=out)
+            for out in (plain, torch.full((m, n), 77, dtype=torch.uint8, device="cuda"))]
+    assert all(bool((a == 77).all()) for a in around)
+    assert torch.equal(*outs)
+    assert plain.unique().numel() > 100
 
 
 # Products whose tiles may write outputs of any size: past the L2s up to 24 MiB, where channels lie on the 64-byte grid up to
@@ -67,7 +99,6 @@ def test_conv(b, h, w, ic, oc, k, groups, post):
 @pytest.mark.parametrize("cfg,k", [(1, 384), (2, 384), (3, 384), (7, 384), (17, 384), (20, 384), (1, 64), (2, 64)])
 @pytest.mark.parametrize("x_signed", [False, True])
 def test_products_on_either_side_of_the_lines(n, rows, cfg, k, x_signed):
-    from torch_musa_amd import cabi
     lo, hi, dt = (-128, 128, torch.int8) if x_signed else (0, 256, torch.uint8)
     gen = torch.Generator("cuda").manual_seed(n + k)
     pw = cabi.PackedLinear(torch.randint(-127, 128, (n, k), generator=gen, device="cuda").to(torch.int8))
@@ -97,7 +128,6 @@ def test_products_on_either_side_of_the_lines(n, rows, cfg, k, x_signed):
     (513, 512, 32, 48, (0, 0)), (397, 397, 32, 80, (0, 0)),              # the k order walked, 256 x 64 and 128 x 128
 ])
 def test_implicit_gemm_on_either_side_of_the_lines(h, w, ic, oc, tile):
-    from torch_musa_amd import cabi
     say("implicit GEMM", h, w, ic, oc, tile)
     gen = torch.Generator("cuda").manual_seed(oc + ic)
     x = torch.randint(0, 256, (2, h, w, ic), generator=gen, device="cuda").to(torch.uint8)
@@ -121,26 +151,34 @@ def test_implicit_gemm_on_either_side_of_the_lines(h, w, ic, oc, tile):
     assert whole.unique().numel() > 100
 
 
-@pytest.mark.parametrize("rows,cols,axis", [(7168, 4096, 0), (7167, 4096, 0), (4100, 8196, 0), (28001, 1050, 0)])
-def test_quantize(rows, cols, axis):
+# 28 Mi codes and more (per tensor short of 96 Mi) leave past the L2s: the whole against runs of rows short of that.
+@pytest.mark.parametrize("rows,cols", [(7168, 4096), (7167, 4096), (4100, 8196), (28001, 1050), (24575, 4096), (24576, 4096)])
+def test_quantize(rows, cols):
     say("quantize", rows, cols)
     gen = torch.Generator("cuda").manual_seed(rows)
     x = torch.randn(rows, cols, device="cuda", generator=gen)
-    scales = x.abs().amax(1).double() / 127
-    zps = torch.zeros(rows, dtype=torch.long, device="cuda")
-    whole, channels = torch.quantize_per_tensor(x, 0.03, 5, torch.qint8), torch.quantize_per_channel(x, scales, zps, axis, torch.qint8)
-    step = 3001
+    scales = x.abs().amax(1) / 127
+    zps = torch.randint(-5, 6, (rows,), generator=gen, device="cuda")
+
+    def codes(lo, hi):
+        xs, sc, zp = x[lo:hi], scales[lo:hi].clone(), zps[lo:hi].clone()   # (whole rows: contiguous, on the grid of the whole)
+        return (cabi.quantize_per_tensor(xs, 0.03, 5, True), cabi.quantize_per_channel(xs, sc.double(), zp, 0, True),
+                cabi.quantize_per_channel_float_qparams(xs, sc, zp.float() + 0.25, 0, True))
+
+    whole, step = codes(0, rows), 3000
     for lo in range(0, rows, step):
-        part = x[lo:lo + step].contiguous()
-        assert torch.equal(whole.int_repr()[lo:lo + step], torch.quantize_per_tensor(part, 0.03, 5, torch.qint8).int_repr())
-        few = torch.quantize_per_channel(part, scales[lo:lo + step].contiguous(), zps[lo:lo + step].contiguous(), axis, torch.qint8)
-        assert torch.equal(channels.int_repr()[lo:lo + step], few.int_repr())
+        for a, few in zip(whole, codes(lo, min(lo + step, rows))):
+            assert torch.equal(a[lo:lo + step], few), lo
+    assert all(a.unique().numel() > 100 for a in whole)
 
 
-@pytest.mark.parametrize("c", [48, 56])
-def test_max_pool(c):
+# Up to 3 MiB of maxima on the 16-channel grid (2.6, 3.1 and 3.0 MB); 3.4 MB and off that grid by ordinary stores.
+@pytest.mark.parametrize("b,c", [(9, 48), (11, 48), (8, 64), (9, 64), (9, 56)])
+@pytest.mark.parametrize("dtype", [torch.quint8, torch.qint8])
+def test_max_pool(b, c, dtype):
+    say("max pool", b, c, dtype)
     gen = torch.Generator("cuda").manual_seed(c)
-    x = feature_map(gen, 9, 147, 159, c)  # 2.6 and 3.1 MB of maxima in all
-    whole = torch.nn.functional.max_pool2d(x, 3, 2, 1).int_repr()
-    for i in range(9):
-        assert torch.equal(whole[i:i + 1], torch.nn.functional.max_pool2d(x[i:i + 1], 3, 2, 1).int_repr())
+    x = torch.randn(b, 147, 159, c, device="cuda", generator=gen).permute(0, 3, 1, 2)
+    q = torch.quantize_per_tensor(x, 6.0 / 255, 128 if dtype == torch.quint8 else 0, dtype)
+    expected = torch.nn.functional.max_pool2d(q.int_repr().float(), 3, 2, 1)
+    assert torch.equal(torch.nn.functional.max_pool2d(q, 3, 2, 1).int_repr().float(), expected)
