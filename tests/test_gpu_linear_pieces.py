@@ -64,12 +64,16 @@ def test_the_choice(cabi, m, n, k, x_signed):  # noqa: F811
     scratch = cabi.lib().tmq_linear_scratch_bytes(m, n, k, int(k % 16 == 0))
     for cfg, room in ((9, 0), (-1, 0), (-1, scratch)):
         cabi.force_linear_config(cfg)
-        cabi.linear_workspace = torch.empty(room, dtype=torch.uint8, device="cuda") if room else None
+        work = torch.full((room,), 0xab, dtype=torch.uint8, device="cuda") if room else None
+        cabi.linear_workspace, cabi.use_linear_workspace = work, room > 0
         try:
             outs.append((cabi.linear(x, pw, 0.05, 3, ws, bias, 0.4, 10), cabi.linear_f32(x, pw, 0.05, 3, ws, bias)))
         finally:
             cabi.force_linear_config(-1)
-            cabi.linear_workspace = None
+            cabi.linear_workspace, cabi.use_linear_workspace = None, True
+        if room and k % 16:                    # the rows were copied onto the grid first
+            pitch = (k + 15) // 16 * 16
+            assert torch.equal(work[:m * pitch].view(dt).view(m, pitch)[:, :k], x)
     for bytes_, floats in outs[1:]:
         assert torch.equal(bytes_, outs[0][0])
         assert torch.equal(floats, outs[0][1])

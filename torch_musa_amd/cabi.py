@@ -361,16 +361,18 @@ def _linear_desc(x, pw, x_scale, x_zp, w_scales, bias, out_scale, out_zp, out_si
     d.kernel = _linear_config + 1
     if y is not None:
         d.y, d.ldy = y.data_ptr(), y.stride(0)
-    nbytes = lib().tmq_linear_workspace_bytes(d.M, d.N, d.K) if use_linear_workspace else 0
-    if nbytes > 0:
-        # split-K scratch, from the caching allocator; the descriptor keeps it
-        # alive until the call is queued on the current stream
+    if use_linear_workspace:
+        nbytes = lib().tmq_linear_workspace_bytes(d.M, d.N, d.K)
+        # split-K scratch, from the caching allocator, or the shared tensor (which may be larger: room for
+        # tmq_linear_scratch_bytes); the descriptor keeps it alive until the call is queued on the current stream
         shared = linear_workspace
-        if shared is not None and shared.device == x.device and shared.numel() >= nbytes:
+        if shared is not None and shared.device == x.device and shared.numel() >= max(nbytes, 1):
             d._workspace = shared
-        else:
+        elif nbytes > 0:
             d._workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-        d.workspace, d.workspace_bytes = d._workspace.data_ptr(), nbytes
+        else:
+            return d
+        d.workspace, d.workspace_bytes = d._workspace.data_ptr(), d._workspace.numel()
     return d
 
 
