@@ -25,6 +25,8 @@ def off_grid(shape, dtype):
     (30, 56, 53, 20, 24, 1, 1, "relu"),       # eight channels a lane
     (17, 41, 57, 64, 80, 1, 1, "add"),        # a last block of 16 channels
     (17, 41, 57, 64, 96, 1, 1, "silu"),
+    (5, 41, 57, 128, 80, 1, 1, "silu"),       # 0.93 MB behind SiLU and 65 to 128 channels: ordinary
+    (6, 41, 57, 128, 80, 1, 1, "silu"),       # 1.1 MB
     (27, 56, 57, 24, 144, 1, 1, "relu"),      # parts of lines, 12.4 MB
     (28, 56, 57, 24, 144, 1, 1, "relu"),      # 12.9 MB, past 12 MiB: ordinary stores
     (28, 56, 57, 24, 144, 1, 1, "silu"),      # ... but behind SiLU

@@ -749,8 +749,12 @@ bool image_through(const ConvShape& s, const void* out) { return lanes_on_grid(s
 // 38.5 MB 14.4 | 15.3); not so where a pixel's channel blocks are one CU's (64 -> 256 25.7 MB 15.2 | 14.4, 24 -> 512 19.7 |
 // 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6; 256 -> 384 23.3 | 21.9).  Blocks that
 // begin inside a line, past 12 MB (24 -> 112 11.2 MB 9.6 | 6.2, 24 -> 144 14.5 MB 9.9 | 11.2, 144 -> 864 18.3 MB 13.3 | 15.0).
+// Nor for SiLU behind 65 to 128 channels short of 1 MiB: that kernel keeps five registers in memory and waits for them behind
+// its stores (222 layers, 2.3 to 2.9 % behind below, 0.5 % ahead up to 2 MB, 2 to 7 % from there; every other kernel is level at
+// 0.1 MB and 2 to 11 % ahead from 1 MB on).
 bool pointwise_through(const ConvShape& s, bool silu, const void* out) {
   const int64_t bytes = out_bytes(s);
+  if (silu && s.runs_KS == 2 && bytes < int64_t{1} << 20) return false;
   const bool lines = s.OC % 64 == 0;
   return lanes_on_grid(s, out) &&
          (silu || bytes <= int64_t{lines ? 20 : 12} << 20 || s.OC % 256 == 0 || (lines && s.runs_KS > 2));
@@ -892,10 +896,7 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.RL = static_cast<int>(s.runs_RL); a.RP = static_cast<int>(s.runs_RP); a.KS = static_cast<int>(s.runs_KS);
   const int64_t pieces = ceil_div(s.B * s.H * s.W, 16);
   a.tiles = static_cast<int32_t>(pieces);
-  if constexpr (MODE == kOutAcc32)
-    a.vec = aligned(out, 16) && s.OC % 4 == 0 ? 1 : 0;
-  else
-    a.through = pointwise_through(s, po.silu, out) ? 1 : 0;
+  if constexpr (MODE == kOutAcc32) a.vec = aligned(out, 16) && s.OC % 4 == 0 ? 1 : 0;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
   a.x_xor = d->x_signed ? 0u : 0x80808080u;
   a.acc_coef = (d->x_signed ? 0 : 128) - d->x_zero_point;
@@ -927,15 +928,21 @@ int launch_conv_pointwise_rows(const tmq_conv2d_desc* d, const ConvShape& s, con
   a.deal_shift = deal ? 3 : 0;
   a.deal_mask = deal ? 7 : 0;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kCrThreads);
-  const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
+  const auto launch_as = [&](auto post_tag, auto nt_tag, auto plain_tag, auto through_tag) {
     constexpr int kP = decltype(post_tag)::value, kNT = decltype(nt_tag)::value;
-    constexpr bool kPlain = decltype(plain_tag)::value;
+    constexpr bool kPlain = decltype(plain_tag)::value, kThrough = decltype(through_tag)::value;
     if (s.runs_KS == 1)
-      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 1, kPlain>, grid, block, 0, stream, a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 1, kPlain, kThrough>, grid, block, 0, stream, a);
     else if (s.runs_KS == 2)
-      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 2, kPlain>, grid, block, 0, stream, a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 2, kPlain, kThrough>, grid, block, 0, stream, a);
     else
-      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 4, kPlain>, grid, block, 0, stream, a);
+      enqueue(conv_runs_pointwise_kernel<MODE, kP, kNT, 4, kPlain, kThrough>, grid, block, 0, stream, a);
+  };
+  const auto launch = [&](auto post_tag, auto nt_tag, auto plain_tag) {
+    if constexpr (MODE != kOutAcc32) {
+      if (pointwise_through(s, po.silu, out)) return launch_as(post_tag, nt_tag, plain_tag, std::true_type{});
+    }
+    launch_as(post_tag, nt_tag, plain_tag, std::false_type{});
   };
   const auto launch_tiles = [&](auto nt_tag) {
     if constexpr (MODE != kOutAcc32) {

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_image_kernel(ConvRunArgs a
             acc[nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[nt][ks], xv, acc[nt], 0, 0, 0);
         }
       }
-      if (live) runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, mult, bdiv, bmul, accw);
+      if (live) runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, mult, bdiv, bmul, accw, a.through != 0);
     }
     __syncthreads();  // the staged rows are overwritten by the next tile
   }

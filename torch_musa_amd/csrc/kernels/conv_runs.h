@@ -64,7 +64,7 @@ struct ConvRunArgs {
   };
   union {
     int vec;                 // (int32 outputs) 16-byte stores per 4 channels are aligned
-    int through;             // (bytes) the stores of whole lanes are st16_through / st8_through
+    int through;             // (bytes, conv_runs_kernel and conv_image_kernel) those of whole lanes: st16_through / st8_through
   };
   int whole;                 // (pointwise) pieces all of whose reads and stores lie inside the tensors
   int nblk, groups;          // (pointwise) channel blocks, and waves on each of them
@@ -194,7 +194,7 @@ __device__ __forceinline__ void runs_store_some(uint8_t* dst, const uint32_t (&p
 template <int MODE, int POST, int NT, bool PLAIN = false>
 __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v4i (&acc)[NT], int64_t off, int cb,
                                                    const float* mult_cb, const float* bdiv_cb, float bmul,
-                                                   const RunsResidual<NT>& accw) {
+                                                   const RunsResidual<NT>& accw, bool through) {
   constexpr int kLaneCh = 4 * NT;
   if constexpr (MODE == kOutAcc32) {
 #pragma unroll
@@ -213,7 +213,7 @@ __device__ __forceinline__ void runs_requant_store(const ConvRunArgs& a, const v
     runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult_cb, bdiv_cb, bmul, accw, packed);
     uint8_t* const dst = static_cast<uint8_t*>(a.y) + off;
     if (cb + kLaneCh <= a.OC)
-      runs_store<NT>(dst, packed, a.through != 0);
+      runs_store<NT>(dst, packed, through);
     else
       runs_store_some<NT>(dst, packed, a.OC - cb);
   }
@@ -423,7 +423,8 @@ __global__ __launch_bounds__(kCrThreads, 3) void conv_runs_kernel(ConvRunArgs a)
       const int64_t off = opix * a.OC + cb;
       RunsResidual<NT> accw{};
       if (POST == 1 || (POST == 2 && a.post.accum != nullptr)) accw = runs_residual<NT>(a, off, cb);
-      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, &s_mult[kLaneCh * pq], &s_bdiv[kLaneCh * pq], bmul, accw);
+      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cb, &s_mult[kLaneCh * pq], &s_bdiv[kLaneCh * pq], bmul, accw,
+                                                a.through != 0);
     }
     __syncthreads();  // the staged rows are overwritten by the next tile
   }
@@ -457,7 +458,10 @@ template <int KSN>
 constexpr int kCrPointwiseDepth = KSN == 1 ? 4 : 2;
 constexpr int kCrXcdBlocks = 8;  // channel blocks from which on the waves of a group of pixels sit on one XCD
 
-template <int MODE, int POST, int NT, int KSN, bool PLAIN = false>
+// THROUGH: the stores of whole lanes are st16_through / st8_through.  (As a branch in the kernel it took registers: SiLU
+// behind 65 to 128 channels spilled ten instead of five and was 5 to 8 % slower, 4.2 | 4.5 us at 128 -> 192 on 37 x 38, and
+// 16 to 64 channels without a residual had three waves a SIMD instead of four.)
+template <int MODE, int POST, int NT, int KSN, bool PLAIN, bool THROUGH>
 __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointwise_kernel(ConvRunArgs a) {
   constexpr int kCrBN = 16 * NT;   // output channels per channel block
   constexpr int kLaneCh = 4 * NT;  // consecutive channels of one pixel in a lane
@@ -601,13 +605,13 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
     fetch(n + D, xr[i], rr[i]);
     const int64_t base = static_cast<int64_t>(g + n * groups) * (16 * a.OC);
     if constexpr (MODE == kOutAcc32) {
-      if (cl < a.OC) runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, base + yo, cl, mult, bdiv, bmul, accw);
+      if (cl < a.OC) runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, base + yo, cl, mult, bdiv, bmul, accw, false);
     } else {
       uint32_t packed[NT];
       uint8_t* const dst = static_cast<uint8_t*>(a.y) + base;
       if constexpr (decltype(all_ch_tag)::value) {
         runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
-        runs_store<NT>(dst + yo, packed, a.through != 0);
+        runs_store<NT>(dst + yo, packed, THROUGH);
       } else {
         if (residual && over > 0 && over < kLaneCh) {
           v4i v = {0, 0, 0, 0};
@@ -619,7 +623,7 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
         }
         runs_requant<MODE, POST, NT, PLAIN>(a, acc, mult, bdiv, bmul, accw, packed);
         if (over <= 0)
-          runs_store<NT>(dst + yo, packed, a.through != 0);
+          runs_store<NT>(dst + yo, packed, THROUGH);
         else if (over < kLaneCh)
           runs_store_some<NT>(dst + yo, packed, kLaneCh - over);
       }
@@ -657,7 +661,7 @@ __global__ __launch_bounds__(kCrThreads, KSN == 4 ? 2 : 3) void conv_runs_pointw
       const int64_t off = static_cast<int64_t>(pix) * a.OC + cl;
       RunsResidual<NT> accw{};
       if (residual) accw = runs_residual<NT>(a, off, cl);
-      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cl, mult, bdiv, bmul, accw);
+      runs_requant_store<MODE, POST, NT, PLAIN>(a, acc, off, cl, mult, bdiv, bmul, accw, THROUGH);
     }
   }
 }
