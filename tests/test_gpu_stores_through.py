@@ -40,14 +40,20 @@ def off_grid(shape, dtype):
     (28, 56, 57, 64, 96, 3, 1, "relu"),       # 8.6 MB, past 8 MiB: ordinary
     (24, 56, 57, 60, 60, 3, 60, "relu"),      # depthwise, 4.6 MB: ordinary below 4.5 MiB
     (25, 56, 57, 60, 60, 3, 60, "relu"),      # 4.8 MB
+    (25, 56, 57, 60, 60, 5, 60, "silu"),      # ... ordinary under a larger window
+    (25, 56, 57, 60, 60, 7, 60, "relu"),
+    (25, 56, 57, 60, 60, 3, 60, "silu"),
     (54, 56, 57, 96, 96, 5, 96, "relu"),      # 16.5 MB
     (55, 56, 57, 96, 96, 5, 96, "relu"),      # 16.9 MB, past 16 MiB: ordinary
     (30, 56, 57, 66, 66, 3, 66, "relu"),      # off the 4-channel grid
-    (30, 56, 57, 60, 60, 7, 60, "silu"),
     (16, 29, 31, 256, 272, 3, 1, "relu"),     # implicit GEMM
     (20, 61, 67, 3, 24, 3, 1, "relu"),        # images, of any size
     (3, 61, 67, 3, 64, 7, 1, "relu"),
-    (20, 61, 67, 1, 48, 3, 1, "relu"),        # byte runs
+    (3, 61, 67, 3, 64, 7, 1, "silu"),         # but SiLU behind 7 x 7 short of 1 MiB
+    (5, 61, 67, 3, 64, 7, 1, "silu"),
+    (20, 61, 67, 1, 48, 3, 1, "relu"),        # byte runs, 3.9 MB
+    (10, 61, 67, 1, 48, 3, 1, "relu"),        # 2.0 MB, short of 2 MiB: ordinary
+    (27, 56, 57, 24, 592, 1, 1, "silu"),      # parts of lines behind SiLU past 48 MiB: ordinary
 ])
 @pytest.mark.parametrize("out_signed", [False, True])
 def test_conv(b, h, w, ic, oc, k, groups, post, out_signed):

@@ -742,12 +742,16 @@ bool plan_runs(const ConvShape& s, int forced_rows, RunPlan* p) {
 int64_t out_bytes(const ConvShape& s) { return s.B * s.OH * s.OW * s.OC; }
 bool lanes_on_grid(const ConvShape& s, const void* out) { return aligned(out, 16) && s.OC % (s.OC <= 32 ? 8 : 16) == 0; }
 // From an image, of any size (us without | with them: 3 -> 64, 7 x 7, [32, 3, 224, 224] 19.4 | 15.9, one image 5.2 | 4.9;
-// 3 -> 32, 3 x 3, 12.6 | 9.4 and 4.2 | 4.0).
-bool image_through(const ConvShape& s, const void* out) { return lanes_on_grid(s, out); }
+// 3 -> 32, 3 x 3, 12.6 | 9.4 and 4.2 | 4.0), but for SiLU behind 7 x 7 and more than 32 channels short of 1 MiB, whose kernel
+// waits for registers that it keeps in memory behind its stores (5.62 | 5.75).
+bool image_through(const ConvShape& s, bool silu, const void* out) {
+  return lanes_on_grid(s, out) && !(silu && s.KH * s.KW > 9 && s.OC > 32 && out_bytes(s) < int64_t{1} << 20);
+}
 // Pointwise rows: 64 -> 64 with a residual 6.4 MB 8.2 | 6.6, 64 -> 128 12.8 MB 13.1 | 10.0, 256 -> 128 12.5 | 10.7.  Where the
 // lines leave the L2s during the kernel anyway, past 20 MB, those that several CUs write leave more than once (64 -> 384
 // 38.5 MB 14.4 | 15.3); not so where a pixel's channel blocks are one CU's (64 -> 256 25.7 MB 15.2 | 14.4, 24 -> 512 19.7 |
-// 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6; 256 -> 384 23.3 | 21.9).  Blocks that
+// 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6, off the 64-channel grid up to 48 MiB,
+// 208 -> 592 with a residual 85 MB 82 | 91; 256 -> 384 23.3 | 21.9).  Blocks that
 // begin inside a line, past 12 MB (24 -> 112 11.2 MB 9.6 | 6.2, 24 -> 144 14.5 MB 9.9 | 11.2, 144 -> 864 18.3 MB 13.3 | 15.0).
 // Nor for SiLU behind 65 to 128 channels short of 1 MiB: that kernel keeps five registers in memory and waits for them behind
 // its stores (222 layers, 2.3 to 2.9 % behind below, 0.5 % ahead up to 2 MB, 2 to 7 % from there; every other kernel is level at
@@ -757,7 +761,12 @@ bool pointwise_through(const ConvShape& s, bool silu, const void* out) {
   if (silu && s.runs_KS == 2 && bytes < int64_t{1} << 20) return false;
   const bool lines = s.OC % 64 == 0;
   return lanes_on_grid(s, out) &&
-         (silu || bytes <= int64_t{lines ? 20 : 12} << 20 || s.OC % 256 == 0 || (lines && s.runs_KS > 2));
+         (bytes <= int64_t{silu ? 48 : lines ? 20 : 12} << 20 || s.OC % 256 == 0 || (lines && (silu || s.runs_KS > 2)));
+}
+// Byte runs: the same from 2 MiB on, 2 to 4 % ahead; below level on average and up to 6 % behind (12 -> 16 on 8 x 96 x 97 1.2 MB
+// 9.7 | 10.1, 24 -> 160 on 16 x 15 x 17 0.6 MB 7.9 | 8.4).
+bool runs_through(const ConvShape& s, bool silu, const void* out) {
+  return out_bytes(s) >= int64_t{2} << 20 && pointwise_through(s, silu, out);
 }
 // Halo tiles: a block has 64 channels of its pixels.  64 -> 64 on 32 x 56 x 56 11.6 | 10.2, on 16 x 56 x 56 7.2 | 6.7, one
 // image 5.2 | 5.1; where other blocks write the rest of a line, up to 8 MB (96 channels 4.8 MB 11.3 | 9.7, 9.6 MB 16.8 | 17.4).
@@ -765,10 +774,13 @@ bool tiles_through(const ConvShape& s, const void* out) {
   return aligned(out, 16) && s.OC % 16 == 0 && (s.OC <= 64 || s.OC % 64 == 0 || out_bytes(s) <= int64_t{8} << 20);
 }
 // Depthwise, four bytes a lane: 96 channels on 4 x 56 x 56 1.2 MB 4.9 | 5.4, 60 on 32 x 56 x 56 6 MB 10.0 | 8.4, 144 on
-// 16 x 56 x 56 7.2 MB 11.1 | 9.6, 192 on 32 x 56 x 56 19.3 MB 15.3 | 15.8.
-bool depthwise_through(const ConvShape& s, const void* out) {
+// 16 x 56 x 56 7.2 MB 11.1 | 9.6, 192 on 32 x 56 x 56 19.3 MB 15.3 | 15.8.  Not where the arithmetic covers the stores: 7 x 7 is
+// level (relu) and 1 % behind (SiLU), 5 x 5 with SiLU level on average and up to 6 % behind (448 channels on 2 x 80 x 75 14.6 |
+// 15.4); 5 x 5 without is 2 to 4 % ahead.
+bool depthwise_through(const ConvShape& s, bool silu, const void* out) {
   const int64_t bytes = out_bytes(s);
-  return aligned(out, 4) && s.OC % 4 == 0 && bytes >= int64_t{9} << 19 && bytes <= int64_t{16} << 20;
+  return aligned(out, 4) && s.OC % 4 == 0 && bytes >= int64_t{9} << 19 && bytes <= int64_t{16} << 20 && s.KH == s.KW &&
+         (s.KH == 3 || (s.KH == 5 && !silu));
 }
 
 template <int MODE>
@@ -796,7 +808,7 @@ int launch_conv_runs(const tmq_conv2d_desc* d, const ConvShape& s, const RunPlan
   if constexpr (MODE == kOutAcc32)
     a.vec = aligned(out, 16) && s.OC % 4 == 0 ? 1 : 0;
   else
-    a.through = (s.pixels4 ? image_through(s, out) : pointwise_through(s, po.silu, out)) ? 1 : 0;
+    a.through = (s.pixels4 ? image_through(s, po.silu, out) : runs_through(s, po.silu, out)) ? 1 : 0;
   a.w_scale_stride = d->w_per_channel ? 1 : 0;
   a.x_xor = d->x_signed ? 0u : 0x80808080u;
   a.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
@@ -1016,13 +1028,13 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
     else if (s.KH == 5 && s.KW == 5)
       enqueue(conv_depthwise_kernel<MODE, kP, 5, kThrough>, grid, block, 0, stream, a);
     else if (s.KH == 7 && s.KW == 7)
-      enqueue(conv_depthwise_kernel<MODE, kP, 7, kThrough>, grid, block, 0, stream, a);
+      enqueue(conv_depthwise_kernel<MODE, kP, 7, false>, grid, block, 0, stream, a);
     else
       enqueue(conv_depthwise_kernel<MODE, kP, 0, false>, grid, block, 0, stream, a);
   };
   const auto launch = [&](auto post_tag) {
     if constexpr (MODE != kOutAcc32) {
-      if (depthwise_through(s, out)) return launch_as(post_tag, std::true_type{});
+      if (depthwise_through(s, po.silu, out)) return launch_as(post_tag, std::true_type{});
     }
     launch_as(post_tag, std::false_type{});
   };
