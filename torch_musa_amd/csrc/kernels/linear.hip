@@ -1232,9 +1232,10 @@ constexpr TileRate kRates[] = {
 bool oblong_ring(int64_t M, int64_t N, int64_t K, int64_t ldx, int bm, int bn) {
   return ceil_div(M, bm) * ceil_div(N, bn) <= 256 && K > 5 * kBK && dma_limits_ok(K, ldx) && (bm == 64 || K % kBK == 0);
 }
-// ... and ahead of every other tile there from K = 1280 on, where 64 x 64 tiles are more than a round (us, the choice before |
-// 64 x 128 in a ring: M = 1829, N = 800, K = 1552 9.9 | 8.3; M = 875, N = 1600, K = 1680 10.8 | 8.8; M = 2718, N = 304, K = 3024
-// 14.8 | 11.5; M = 3628, N = 432, K = 5360 26.1 | 17.6; level at M = 731, N = 1472, K = 1856 9.1 | 8.9; behind below, M = 1135,
+// ... and taken there from K = 1280 on, where 64 x 64 tiles are more than a round (us, the choice before | 64 x 128 in a
+// ring: M = 1829, N = 800, K = 1552 9.9 | 8.3; M = 875, N = 1600, K = 1680 10.8 | 8.8; M = 2718, N = 304, K = 3024 14.8 | 11.5; M =
+// 3628, N = 432, K = 5360 26.1 | 17.6; 181 drawn shapes: 0.88 of the time, the fastest of all kernels on 163, 13 % behind at most;
+// up to 576 channels at K < 1600 2 to 5 % behind 64 x 64 ones, M = 2469, N = 448, K = 1280 7.1 | 7.4; behind below, M = 1135,
 // N = 1024, K = 1216 7.2 | 7.4, and where a round of 64 x 64 tiles holds the product, M = 182, N = 4480, K = 1984 7.6 | 9.1).
 bool oblong_ring_first(int64_t M, int64_t N, int64_t K, int64_t ldx) {
   return K >= 1280 && ceil_div(M, 64) * ceil_div(N, 64) > 256 && oblong_ring(M, N, K, ldx, 64, 128);

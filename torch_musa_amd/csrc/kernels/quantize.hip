@@ -135,7 +135,7 @@ __device__ __forceinline__ void report_range(const RangeReport& r, float mn, flo
 // the caches.  The codes are written with ordinary stores, so a consumer that
 // follows on the stream (dequantize, a GEMM) finds them in the last-level cache --
 // unless there are more of them than that cache has bytes, 256 Mi: then they leave
-// with non-temporal stores as well (STREAM_OUT).  Quantize and dequantize of 2**28
+// with non-temporal stores as well (kQStream).  Quantize and dequantize of 2**28
 // values, us, non-temporal | ordinary: 407 | 375 with one buffer of codes call after
 // call, 405 | 386 with three in turn (2**27: 204 | 195; the quantizer by itself,
 // three buffers: 199 | 208); of 1.5 * 2**28: 606 | 640, 2**29: 808 | 853.
