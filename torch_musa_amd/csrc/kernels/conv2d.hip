@@ -750,12 +750,12 @@ bool image_through(const ConvShape& s, bool silu, const void* out) {
 // Pointwise rows: 64 -> 64 with a residual 6.4 MB 8.2 | 6.6, 64 -> 128 12.8 MB 13.1 | 10.0, 256 -> 128 12.5 | 10.7.  Where the
 // lines leave the L2s during the kernel anyway, past 20 MB, those that several CUs write leave more than once (64 -> 384
 // 38.5 MB 14.4 | 15.3); not so where a pixel's channel blocks are one CU's (64 -> 256 25.7 MB 15.2 | 14.4, 24 -> 512 19.7 |
-// 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6, off the 64-channel grid up to 48 MiB,
-// 208 -> 592 with a residual 85 MB 82 | 91; 256 -> 384 23.3 | 21.9).  Blocks that
-// begin inside a line, past 12 MB (24 -> 112 11.2 MB 9.6 | 6.2, 24 -> 144 14.5 MB 9.9 | 11.2, 144 -> 864 18.3 MB 13.3 | 15.0).
+// 18.9), nor where the kernel is no faster than the memory (SiLU: 64 -> 272 29.6 | 26.6, 256 -> 384 23.3 | 21.9; off the
+// 64-channel grid up to 48 MiB, 208 -> 592 with a residual 85 MB 82 | 91).  Blocks that begin inside a line, past 12 MB (24 ->
+// 112 11.2 MB 9.6 | 6.2, 24 -> 144 14.5 MB 9.9 | 11.2, 144 -> 864 18.3 MB 13.3 | 15.0).
 // Nor for SiLU behind 65 to 128 channels short of 1 MiB: that kernel keeps five registers in memory and waits for them behind
-// its stores (222 layers, 2.3 to 2.9 % behind below, 0.5 % ahead up to 2 MB, 2 to 7 % from there; every other kernel is level at
-// 0.1 MB and 2 to 11 % ahead from 1 MB on).
+// its stores (206 layers: 2.3 to 2.9 % behind below, level up to 2 MB, 2 to 7 % ahead from there; every other kernel is level
+// below 0.25 MB and 2 to 11 % ahead from 2 MB on).
 bool pointwise_through(const ConvShape& s, bool silu, const void* out) {
   const int64_t bytes = out_bytes(s);
   if (silu && s.runs_KS == 2 && bytes < int64_t{1} << 20) return false;

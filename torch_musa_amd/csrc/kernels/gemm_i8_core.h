@@ -166,8 +166,8 @@ struct GemmArgs {
 // 8192 x 512 -> 2048 19.8 | 17.2, 1024 x 1024 -> 4096 11.8 | 10.8, 384 x 768 -> 3072 5.2 | 5.1, 512 x 1024 -> 1024 level.
 // Channels off the 64-byte grid: several blocks write parts of a line, which an L2 merges where it keeps the line for a while;
 // past it each part travels by itself.  Up to 24 MiB 3 % ahead on average (33088 x 320 -> 304 10 MB 9 %; pixels likewise, 288 ->
-// 240 on 32 x 56 x 56 24 MB 21.5 | 18.4), then level or far behind from one part to the next (320 -> 272 on 32 x 56 x 56 27 MB
-// 28.6 | 28.3, on another part 29.6 | 34.8), and behind from 30 MB on (183823 x 320 -> 272 50 MB 1.4 times, 152777 x 96 -> 720
+// 240 on 32 x 56 x 56 24 MB 21.5 | 18.4), then level or far behind from one device to the next (320 -> 272 on 32 x 56 x 56 27 MB
+// 28.6 | 28.3, on another 29.6 | 34.8), and behind from 30 MB on (183823 x 320 -> 272 50 MB 1.4 times, 152777 x 96 -> 720
 // 110 MB 1.27 times, 320 -> 528 on 32 x 80 x 80 85 | 105).  On that grid 2 to 10 % ahead up to 52 MiB (with a dequantizer
 // behind them 2 to 5 % up to 28 MiB and level from there), 1 % behind past 80 MB.
 // The host tells: a test in the kernel takes 0.05 us and 1 % of a longer one.
