@@ -101,11 +101,13 @@ int tmq_quantize_per_tensor_dev(const float* x, void* q, int64_t n,
                                 const tmq_qparams* qparams, int q_signed,
                                 tmq_stream_t stream);
 /* The whole dynamic quantization on the device: min/max over x, the parameters
- * into *qparams (device memory), the codes into q.  Small inputs (at most
- * 98304 elements) take one launch, inputs of up to 2**25 elements two (the
- * quantizer's workgroups finish the range reduction themselves), larger or
- * unaligned ones three; `workspace` as for tmq_minmax (unused, and may be NULL,
- * for the small case).
+ * into *qparams (device memory), the codes into q.  One launch up to 2**26
+ * elements (from 32768 on its workgroups exchange their ranges through the
+ * workspace, which no other call may use meanwhile).  Where that is not possible -- a stream that is being
+ * captured, whose launches run again with the same arguments, x off the 16-byte
+ * or the workspace off the 16-byte grid, signed codes with TMQ_ROUND_FUSED -- one
+ * launch up to 98304 elements, two up to 2**25, else three.  `workspace` as for
+ * tmq_minmax (unused, and may be NULL, up to 32768 elements).
  * rounding = TMQ_ROUND_PRODUCT: q = clamp(rne(fl(x * inv)) + zp), the same
  * results as tmq_minmax + tmq_choose_qparams_dev + tmq_quantize_per_tensor_dev
  * (aten::quantize_per_tensor_dynamic).
@@ -153,10 +155,17 @@ int tmq_quantize_per_tensor_dynamic_parts(const float* x, void* q, int64_t n, in
 /* The same for M rows of K values -> rows of `pitch` codes, pitch a multiple of
  * 16 that is at least K: what tmq_linear wants of activations whose K is not.
  * The codes behind a row's end are undefined (the packed weights are zero there).
- * One launch up to 98304 values, else two; `workspace` 8-byte aligned. */
+ * One launch or, where ranges are not exchanged (see above; also TMQ_ROUND_PRODUCT and K < 4), two from 98305
+ * values on; `workspace` 8-byte aligned. */
 int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
                                   int reduce_range, int rounding, tmq_qparams* qparams,
                                   void* workspace, size_t workspace_bytes, tmq_stream_t stream);
+/* The launch that exchanges ranges, pinned, for tests: at most `blocks` workgroups, of which each reads the others'
+ * ranges polls + 1 times before it finds a missing one itself.  pitch == K: M * K values in a row.
+ * TMQ_ERR_UNSUPPORTED where the calls above take other kernels whatever the size. */
+int tmq_quantize_dynamic_exchange(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
+                                  int reduce_range, int rounding, tmq_qparams* qparams, void* workspace,
+                                  size_t workspace_bytes, int blocks, int polls, tmq_stream_t stream);
 /* Host-side ChooseQuantizationParams, same arithmetic (pure CPU, no GPU call). */
 int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
                             double* scale, int32_t* zero_point);

@@ -25,7 +25,7 @@ DECLARED_SYMBOLS = [
     "tmq_quantize_per_channel_float_qparams", "tmq_dequantize_per_channel_float_qparams",
     "tmq_linear_packed_kchunks", "tmq_linear_packed_bytes", "tmq_linear_prepack",
     "tmq_linear_unpack", "tmq_linear", "tmq_linear_workspace_bytes", "tmq_linear_split_plan", "tmq_linear_kernel_choice", "tmq_linear_static_workspace", "tmq_linear_acc32", "tmq_linear_f32", "tmq_linear_dynamic_small", "tmq_linear_dynamic_small_takes", "tmq_quantize_per_tensor_dynamic_dev",
-    "tmq_quantize_per_tensor_dynamic_report", "tmq_quantize_per_tensor_dynamic_parts", "tmq_quantize_rows_dynamic_dev", "tmq_linear_scratch_bytes", "tmq_linear_float", "tmq_per_channel",
+    "tmq_quantize_per_tensor_dynamic_report", "tmq_quantize_per_tensor_dynamic_parts", "tmq_quantize_rows_dynamic_dev", "tmq_quantize_dynamic_exchange", "tmq_linear_scratch_bytes", "tmq_linear_float", "tmq_per_channel",
     "tmq_conv2d_packed_bytes", "tmq_conv2d_prepack", "tmq_conv2d_out_hw", "tmq_conv2d_workspace_bytes",
     "tmq_conv2d", "tmq_conv2d_acc32", "tmq_conv2d_fused",
     "tmq_qadd", "tmq_qrelu", "tmq_qcat_rows", "tmq_planes_to_pixels", "tmq_qmaxpool2d", "tmq_qadaptive_avgpool2d", "tmq_qunary",
@@ -142,6 +142,10 @@ def lib() -> C.CDLL:
         l.tmq_quantize_per_tensor_dynamic_dev.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v]
         l.tmq_quantize_per_tensor_dynamic_report.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v,
                                                              C.c_uint32, C.c_uint32, v]
+        l.tmq_quantize_rows_dynamic_dev.argtypes = [v, v, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, v, v,
+                                                    C.c_size_t, v]
+        l.tmq_quantize_dynamic_exchange.argtypes = [v, v, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, v, v,
+                                                    C.c_size_t, C.c_int, C.c_int, v]
         l.tmq_conv2d_prepack.argtypes = [v, C.POINTER(Conv2dGeom), v, v, v]
         l.tmq_conv2d_out_hw.argtypes = [C.POINTER(Conv2dGeom), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]
         l.tmq_conv2d.argtypes = [C.POINTER(Conv2dDesc), v]
@@ -266,6 +270,20 @@ def quantize_per_tensor_dynamic_report(x: torch.Tensor, signed: bool, reduce_ran
                                                        int(reduce_range), 0, qp.data_ptr(), ws.data_ptr(), ws.numel(),
                                                        report.data_ptr(), ticket, slot, stream_ptr()),
           "tmq_quantize_per_tensor_dynamic_report")
+    return q, qp
+
+
+def quantize_dynamic_exchange(x: torch.Tensor, pitch: int, signed: bool, reduce_range: bool, fused: bool, blocks: int = 256,
+                              polls: int = 32):
+    """The launch whose blocks exchange their ranges, over rows x [M, K] -> (codes [M, pitch], 16 device bytes of qparams)."""
+    assert x.dtype == torch.float32 and x.is_contiguous() and x.dim() == 2
+    m, k = x.shape
+    q = torch.empty((m, pitch), dtype=torch.int8 if signed else torch.uint8, device=x.device)
+    qp = torch.empty(16, dtype=torch.uint8, device=x.device)
+    ws = minmax_workspace(x.device)
+    check(lib().tmq_quantize_dynamic_exchange(x.data_ptr(), q.data_ptr(), m, k, pitch, int(signed), int(reduce_range), int(fused),
+                                              qp.data_ptr(), ws.data_ptr(), ws.numel(), blocks, polls, stream_ptr()),
+          "tmq_quantize_dynamic_exchange")
     return q, qp
 
 

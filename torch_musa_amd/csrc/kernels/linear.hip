@@ -3,6 +3,7 @@
 // shapes the vector paths do not take (K not a multiple of 16, unaligned rows).
 #include <atomic>
 
+#include "device_info.h"
 #include "gemm_i8_core.h"
 #include "gemm_i8_onepass.h"
 #include "gemm_i8_persistent.h"
@@ -666,22 +667,6 @@ int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream
   if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2>, grid, block, 0, s, a, xs);
   else enqueue(gemm_i8_wloop_kernel<MODE, 1>, grid, block, 0, s, a, xs);
   return launch_status();
-}
-
-constexpr int kMaxDevices = 64;
-
-// Compute units of the current device (cached per device; two threads that race
-// on a device's first call store the same value).
-int cu_count() {
-  static std::atomic<int> cache[kMaxDevices];
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
-  int v = cache[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cache[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
 }
 
 // One block per CU walks the 256 x 256 tiles (byte or float outputs, direct copies two

@@ -9,12 +9,18 @@
 // Numerics follow PyTorch's CPU quantizer (fbgemm/QuantUtils.h:67-101,155-158):
 // multiply by the fp32 reciprocal of the fp32 scale, round half to even, add
 // the zero point, clamp.  Compiled with -ffp-contract=off.
+#include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <limits>
 #include <type_traits>
 
 #include "common.h"
+#include "device_info.h"
+#include "host_report.h"
 #include "qparams.h"
+#include "quantize_held.h"
 #include "stores_through.h"
 
 namespace tmq {
@@ -109,24 +115,6 @@ __device__ __forceinline__ void resolve(const QParamsArg& a, float& inv, float& 
     inv = a.inv;
     zp_f = a.zp_f;
   }
-}
-
-// What the host waits for goes to it as one or two 8-byte words in pinned host memory, a
-// ticket in the upper half and the payload in the lower one: each word is a single store,
-// so the host needs no order between them and the device no fence (a system-scope release
-// would write back the L2s first).
-__device__ __forceinline__ void report_word(uint64_t* word, uint32_t ticket, uint32_t payload) {
-  __hip_atomic_store(word, (static_cast<uint64_t>(ticket) << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-struct RangeReport {
-  tmq_host_report* to;
-  uint32_t ticket;
-  uint32_t slot;  // below TMQ_HOST_REPORTS, this report's own among the calls in flight
-};
-__device__ __forceinline__ void report_range(const RangeReport& r, float mn, float mx) {
-  if (r.to == nullptr) return;
-  report_word(&r.to->word[0], r.ticket, __builtin_bit_cast(uint32_t, mn));
-  report_word(&r.to->word[1], r.ticket, __builtin_bit_cast(uint32_t, mx));
 }
 
 // x4/q4 view the first 4*n4 elements; the block with index 0 also converts the
@@ -284,8 +272,7 @@ __device__ unsigned int g_range_arrivals[TMQ_HOST_REPORTS];
 // KEEP: ordinary loads instead of non-temporal ones, for an input that a second pass on
 // the stream reads again while the last-level cache still holds it.
 // With a report, the last block to arrive reduces the partial pairs and tells the host the
-// range, one launch earlier than the pass behind this one could (quantize_per_tensor_dynamic
-// and dequantize of 32 Ki ... 600 Ki values: 16.8 -> 15.0 us).
+// range, one launch earlier than the pass behind this one could.
 template <bool KEEP = false>
 __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
     const v4f* __restrict__ x4, int64_t n4, const float* __restrict__ x, int64_t head,
@@ -369,61 +356,6 @@ __global__ __launch_bounds__(kThreads) void minmax_partial_kernel(
   if (threadIdx.x == 0) report_range(report, s_mm[0], s_mm[1]);
 }
 
-// The range pass of a call whose host waits for the range, where a few dozen blocks are enough to read the input: every
-// block tells the host the range of its own part with one store, and the host puts the parts together.  The kernel above
-// spends two trips to where all XCDs see its count, and a third to read the other blocks' pairs, before the host hears a word;
-// here the host reads up to eight cache lines instead.  (quantize_per_tensor_dynamic and dequantize of 128 x 1024 values
-// 16.6 -> 15.6 us, of 1000 x 1000 17.9 -> 16.4, of 2048 x 1024 19.2 -> 16.7.  Against the one launch of
-// dynamic_quantize_repeat_kernel, whose blocks each read everything before the first of them reports: 32 Ki values 15.9 | 14.9,
-// 64 Ki level at 16.0, 80 Ki 15.8 | 16.9, 96 Ki 15.9 | 17.0.)
-constexpr int kPartsThreads = 1024;
-constexpr int64_t kPartsMin = TMQ_HOST_PARTS_ABOVE, kPartsMax = TMQ_HOST_PARTS_UP_TO;
-__global__ __launch_bounds__(kPartsThreads) void minmax_parts_kernel(const v4f* __restrict__ x4, int32_t n4,
-                                                                     const float* __restrict__ x, int32_t n,
-                                                                     float* __restrict__ partials, uint64_t* parts) {
-  constexpr int kWaves = kPartsThreads / kWave, kAhead = 4;
-  __shared__ float s_mn[kWaves], s_mx[kWaves];
-  const int t = threadIdx.x, step = static_cast<int>(gridDim.x) * kPartsThreads;
-  float mn = std::numeric_limits<float>::infinity();
-  float mx = -std::numeric_limits<float>::infinity();
-  // (indices past the end read the last group again, which no minimum or maximum minds)
-  for (int base = static_cast<int>(blockIdx.x) * kPartsThreads; base < n4; base += kAhead * step) {
-    v4f v[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int i = base + u * step + t;
-      v[u] = x4[i < n4 ? i : n4 - 1];
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      mn = fminf(fminf(mn, v[u].x), fminf(v[u].y, fminf(v[u].z, v[u].w)));
-      mx = fmaxf(fmaxf(mx, v[u].x), fmaxf(v[u].y, fmaxf(v[u].z, v[u].w)));
-    }
-  }
-  if (blockIdx.x == 0 && t < n - 4 * n4) {
-    mn = fminf(mn, x[4 * n4 + t]);
-    mx = fmaxf(mx, x[4 * n4 + t]);
-  }
-  wave_minmax(mn, mx);
-  if (t % kWave == 0) {
-    s_mn[t / kWave] = mn;
-    s_mx[t / kWave] = mx;
-  }
-  __syncthreads();
-  if (t >= kWave) return;
-  mn = t < kWaves ? s_mn[t] : std::numeric_limits<float>::infinity();
-  mx = t < kWaves ? s_mx[t] : -std::numeric_limits<float>::infinity();
-  wave_minmax(mn, mx);
-  if (t == 0) {
-    // (one store of eight bytes: complete or not there; the host needs no order between the parts)
-    __hip_atomic_store(&parts[blockIdx.x],
-                       (static_cast<uint64_t>(__builtin_bit_cast(uint32_t, mx)) << 32) | __builtin_bit_cast(uint32_t, mn),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    partials[2 * blockIdx.x] = mn;
-    partials[2 * blockIdx.x + 1] = mx;
-  }
-}
-
 __global__ __launch_bounds__(kThreads) void minmax_final_kernel(
     const float* __restrict__ partials, int count, float* __restrict__ out) {
   float mn = std::numeric_limits<float>::infinity();
@@ -470,7 +402,8 @@ __global__ __launch_bounds__(kThreads) void minmax_final_choose_kernel(
   }
 }
 
-// Second launch of a dynamic quantization: every block first finishes the range
+// Second launch of a dynamic quantization that takes two (quantize_held.h has the one that takes one, which a
+// captured stream cannot run): every block first finishes the range
 // reduction for itself -- the partial {min, max} pairs of the pass before it (at most
 // kDynPartials of them, 4 KB from the L2s), ChooseQuantizationParams in one thread --
 // while the loads of its first elements are already in flight, then quantizes its
@@ -612,7 +545,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_after_minmax_kernel(
 // into every CU, 2.7 us at 64 bytes a clock, about what the launch and the gap between two launches
 // cost (a dynamically quantized linear of 55 rows, 704 -> 480: 12.2 -> 8.6 us; of 283 rows, 392 -> 192,
 // 111 Ki values: level; quantize and dequantize of 130 x 384 values 16.7 -> 15.6 us, of 581 x 221
-// 16.3 -> 17.4 us, hence the limit).
+// 16.3 -> 17.4 us, hence the limit; above 32 Ki values it only runs where ranges cannot be exchanged, see kHeldAbove).
 // Rows: `K` values each, written at a pitch of 4 pitch4 codes (pitch4 = 0: one row, no pitch).  x is read as
 // 16 bytes at any 4-byte alignment.
 constexpr int kDynRepeatThreads = 1024;
@@ -1330,6 +1263,93 @@ TMQ_EXPORT int tmq_choose_qparams_dev(const float* minmax, int q_signed, int red
 
 namespace tmq {
 namespace {
+
+// ---------------------------------------------------------------------------
+// Dynamic quantization in one launch whose blocks exchange their ranges (quantize_held.h): where it is taken and how.
+// ---------------------------------------------------------------------------
+// Above 32 Ki values; up to there dynamic_quantize_repeat_kernel (us, that | this: 16 Ki 3.5 | 3.3, 32 Ki 3.6 | 3.7, 64 Ki
+// 4.8 | 4.0, 96 Ki 5.8 | 3.9).  Up to 64 Mi values; beyond, range and codes stream past the caches in three launches (64 Mi
+// 94 | 87, 256 Mi 372 | 478: one block per CU has too little on its way for what it does not hold).
+constexpr int64_t kHeldAbove = 32768, kHeldUpTo = int64_t{1} << 26;
+constexpr int kHeldPolls = 32;  // of about a microsecond each: more than the blocks of one launch are apart on an idle chip
+
+// What no other launch of this process has (a permutation of a counter; its start differs from process to process).
+uint64_t next_range_tag() {
+  static std::atomic<uint64_t> count{static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
+  uint64_t z = count.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  return z ^ (z >> 31);
+}
+
+// A captured launch keeps its arguments: its tag would be in the words already when the graph runs again.
+bool replayed(hipStream_t s) {
+  if (s == nullptr) return false;  // (the null stream cannot be captured)
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;  // unknown: as if it were
+}
+
+struct HeldCall {
+  const float* x;
+  void* q;
+  int64_t M, K, pitch;  // pitch == K: dense, M * K values
+  int q_signed;
+  bool fused;
+  int reduce_range;
+  tmq_qparams* qparams;
+  void* workspace;
+  size_t workspace_bytes;
+};
+// What the kernel needs of a call, whatever its size.
+bool held_runs(const HeldCall& c, hipStream_t s) {
+  const bool rows = c.pitch != c.K;
+  if (c.fused && c.q_signed) return false;
+  if (!aligned(c.q, 4) || !aligned(c.x, rows ? 4 : 16) || (rows && (!c.fused || c.K < 4 || c.M * (c.pitch / 4) > (1 << 30)))) return false;
+  if (c.M * c.K < 4 || c.M * c.K > kHeldUpTo) return false;
+  if (c.workspace == nullptr || c.workspace_bytes < kHeldBlocks * sizeof(v4u) || !aligned(c.workspace, 16)) return false;
+  return cu_count() > 0 && !replayed(s);
+}
+template <bool FUSED, bool ROWS>
+auto held_kernel(int held) {
+  switch (held) {
+    case 1: return dynamic_quantize_held_kernel<FUSED, ROWS, 1>;
+    case 2: return dynamic_quantize_held_kernel<FUSED, ROWS, 2>;
+    case 3: return dynamic_quantize_held_kernel<FUSED, ROWS, 3>;
+    case 4: return dynamic_quantize_held_kernel<FUSED, ROWS, 4>;
+    case 6: return dynamic_quantize_held_kernel<FUSED, ROWS, 6>;
+    case 8: return dynamic_quantize_held_kernel<FUSED, ROWS, 8>;
+    case 12: return dynamic_quantize_held_kernel<FUSED, ROWS, 12>;
+    case 16: return dynamic_quantize_held_kernel<FUSED, ROWS, 16>;
+    case 24: return dynamic_quantize_held_kernel<FUSED, ROWS, 24>;
+    default: return dynamic_quantize_held_kernel<FUSED, ROWS, kHeldMost>;
+  }
+}
+// The host takes the range of up to TMQ_HOST_PARTS_UP_TO values in parts, from as many blocks as it has words for: each
+// tells it its own, 1.5 us before any block knows all of them (with dequantize, against range pass and quantizer in two
+// launches: 874 x 2752 values 19.5 -> 16.4 us, 128 x 1024 level at 13.9, where the host's own work is the time).
+int launch_held(const HeldCall& c, int most_blocks, int polls, const RangeReport& report, uint64_t* parts, int32_t* parts_count,
+                hipStream_t s) {
+  const bool rows = c.pitch != c.K;
+  const int64_t n = c.M * c.K, total = rows ? c.M * (c.pitch / 4) : n / 4;
+  int64_t blocks = ceil_div(total, kHeldThreads);
+  blocks = std::min({blocks, int64_t{most_blocks}, int64_t{kHeldBlocks}, int64_t{cu_count()}});
+  const int64_t per_thread = ceil_div(total, blocks * kHeldThreads);
+  int held = kHeldMost;
+  for (const int h : {24, 16, 12, 8, 6, 4, 3, 2, 1})
+    if (h >= per_thread) held = h;
+  const int32_t more = static_cast<int32_t>(per_thread > held ? per_thread - held : 0);
+  const auto kernel = rows ? held_kernel<true, true>(held) : c.fused ? held_kernel<true, false>(held) : held_kernel<false, false>(held);
+  const HeldRange range{static_cast<v4u*>(c.workspace), next_range_tag(), polls};
+  if (parts != nullptr) *parts_count = static_cast<int32_t>(blocks);
+  enqueue(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHeldThreads), 0, s, c.x, static_cast<uint32_t*>(c.q),
+          static_cast<int32_t>(total), static_cast<int32_t>(rows ? c.K : 0), static_cast<int32_t>(rows ? c.pitch / 4 : 1),
+          static_cast<int32_t>(rows ? 0 : n % 4), range, more, c.q_signed ? 0x80808080u : 0u, c.q_signed ? -128 : 0,
+          c.q_signed ? 127 : 255, c.reduce_range, c.qparams, report, parts);
+  return launch_status();
+}
+
 int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduce_range, int rounding,
                      tmq_qparams* qparams, void* workspace, size_t workspace_bytes, RangeReport report,
                      tmq_stream_t stream, uint64_t* parts = nullptr, int32_t* parts_count = nullptr) {
@@ -1341,7 +1361,13 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
   const bool vec_ok = aligned(x, 16) && aligned(q, 4);
   const bool two_ok = workspace != nullptr && workspace_bytes >= tmq_minmax_workspace_bytes(n) && aligned(workspace, 8);
-  if (n <= kDynRepeatMax && !(parts != nullptr && n > kPartsMin && vec_ok && two_ok)) {
+  const HeldCall held{x, q, 1, n, n, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
+  if (n > kHeldAbove && held_runs(held, s)) {
+    const bool in_parts = parts != nullptr && n > TMQ_HOST_PARTS_ABOVE && n <= TMQ_HOST_PARTS_UP_TO;
+    return launch_held(held, in_parts ? TMQ_HOST_PARTS : kHeldBlocks, kHeldPolls, in_parts ? RangeReport{nullptr, 0, 0} : report,
+                       in_parts ? parts : nullptr, parts_count, s);
+  }
+  if (n <= kDynRepeatMax) {
     const int32_t n32 = static_cast<int32_t>(n);
     // (nothing to quantize: one block still publishes the parameters)
     return launch_dynamic_repeat(q_signed != 0, fused, n > 0 ? ceil_div(n, 4) : 1, s, x, static_cast<uint8_t*>(q), n32, n32, 0,
@@ -1359,16 +1385,9 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
     // the reduction themselves.
     const RangeReport early = n <= kDynEarlyMax ? report : none, late = n <= kDynEarlyMax ? none : report;
     const int64_t n4 = n / 4;
-    const bool in_parts = parts != nullptr && n <= kPartsMax;
-    const unsigned g = in_parts ? grid_for(n4, kPartsThreads, TMQ_HOST_PARTS) : grid_for(n4, kThreads * kUnroll, kDynPartials);
+    const unsigned g = grid_for(n4, kThreads * kUnroll, kDynPartials);
     const v4f* x4 = reinterpret_cast<const v4f*>(x);
-    if (in_parts) {
-      *parts_count = static_cast<int32_t>(g);
-      enqueue(minmax_parts_kernel, dim3(g), dim3(kPartsThreads), 0, s, x4, static_cast<int32_t>(n4), x, static_cast<int32_t>(n),
-              partials, parts);
-    } else {
-      enqueue(minmax_partial_kernel<true>, dim3(g), dim3(kThreads), 0, s, x4, n4, x, 0, n, partials, early);
-    }
+    enqueue(minmax_partial_kernel<true>, dim3(g), dim3(kThreads), 0, s, x4, n4, x, 0, n, partials, early);
     if (launch_status() != TMQ_OK) return TMQ_ERR_LAUNCH;
     const dim3 grid(grid_for(n4, kThreads * kUnrollQD, kDynQBlocks)), block(kThreads);
     uint32_t* q4 = static_cast<uint32_t*>(q);
@@ -1452,6 +1471,9 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
   const int qmin = q_signed ? -128 : 0, qmax = q_signed ? 127 : 255;
   const bool fused = rounding == TMQ_ROUND_FUSED;
   const int64_t n = M * K;
+  const HeldCall held{x, q, M, K, pitch, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
+  if (n > kHeldAbove && held_runs(held, s))
+    return launch_held(held, kHeldBlocks, kHeldPolls, RangeReport{nullptr, 0, 0}, nullptr, nullptr, s);
   if (n <= kDynRepeatMax)
     return launch_dynamic_repeat(q_signed != 0, fused, M * (pitch / 4), s, x, static_cast<uint8_t*>(q), static_cast<int32_t>(n),
                                  static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4), qmin, qmax, reduce_range, true,
@@ -1474,6 +1496,18 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
   };
   if (q_signed) return fused ? go(quantize_rows_after_minmax_kernel<true, true>) : go(quantize_rows_after_minmax_kernel<true, false>);
   return fused ? go(quantize_rows_after_minmax_kernel<false, true>) : go(quantize_rows_after_minmax_kernel<false, false>);
+}
+
+TMQ_EXPORT int tmq_quantize_dynamic_exchange(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
+                                            int reduce_range, int rounding, tmq_qparams* qparams, void* workspace,
+                                            size_t workspace_bytes, int blocks, int polls, tmq_stream_t stream) {
+  if (M < 1 || K < 1 || K > 0x7fffff00 || pitch < K || (pitch != K && pitch % 16 != 0) || x == nullptr || q == nullptr ||
+      qparams == nullptr || blocks < 1 || polls < 0 || M > (int64_t{1} << 40) / K)
+    return TMQ_ERR_INVALID_ARGUMENT;
+  if (rounding != TMQ_ROUND_PRODUCT && rounding != TMQ_ROUND_FUSED) return TMQ_ERR_INVALID_ARGUMENT;
+  const HeldCall held{x, q, M, K, pitch, q_signed, rounding == TMQ_ROUND_FUSED, reduce_range, qparams, workspace, workspace_bytes};
+  if (!held_runs(held, as_stream(stream))) return TMQ_ERR_UNSUPPORTED;
+  return launch_held(held, blocks, polls, RangeReport{nullptr, 0, 0}, nullptr, nullptr, as_stream(stream));
 }
 
 TMQ_EXPORT int tmq_choose_qparams_host(float min, float max, int q_signed, int reduce_range,
