@@ -1,23 +1,29 @@
-// int8 MFMA GEMM for grids smaller than the chip against a long K (gfx950): tiles of 32 rows x 32 or 64 channels whose
-// eight waves split K, each walking its share in pieces through registers, with no barrier before the partial tiles meet.
+// int8 MFMA GEMM for grids smaller than the chip and K beyond what fits LDS at once (gfx950): tiles of 32 rows x 32 or 64
+// channels whose eight waves split K, each walking its share in pieces through registers, with no barrier before the partial
+// tiles meet.
 //
-// What bounds these products is what a CU pulls from the L2s and memory, about 60 bytes a nanosecond, and before that how
+// What bounds these products is what a CU pulls from the L2s, 100 to 110 bytes a nanosecond here where few tiles share them
+// (a loop of copies alone reaches 120 to 150 where an XCD's CUs read the same lines), and before that how
 // much of it is on its way: the pipelined tiles of gemm_i8_core.h request a 64-byte stage at a time for all waves
-// behind one barrier (M = 174, N = 1088, K = 4544 on 51 tiles of 64 x 64 with two wave groups: 0.14 us a stage), and the kernels that
-// have all of a wave's share in registers and LDS at once (gemm_i8_wstream_kernel, gemm_i8_wring_kernel) end at K = 4096.
+// behind one barrier (M = 174, N = 1088, K = 4544 on 51 tiles of 64 x 64 with two wave groups: 0.14 us a stage).
 // Here a wave holds two pieces of both operands: 256 bytes of K by 32 rows and 32 channels, or 128 bytes by 32 and 64: 16
 // (12) requests of 1 KB each, 256 (192) KB a CU in flight.  A piece's activations go to the wave's own LDS (whole
 // lines of a row per request, the MFMA layout back out), its weights stay in registers in the packed layout, and as soon
 // as it has been multiplied the piece after the next is requested into the same registers.
 // The sign flip of unsigned activations and the zeros behind K are applied on the way into LDS.
+// A wave's pieces are every eighth one and not a run of its own, and nothing is requested that is not multiplied: with runs,
+// and the pieces past a wave's last fetched again so that every turn of the loop was alike, 482 x 5232 -> 768 took 12.6 us for
+// 10.1 now, 1437 x 5184 -> 256 12.6 | 10.3, 76 x 5824 -> 128 8.9 | 7.2, 196 x 2304 -> 256 7.0 | 4.6 (of 266 x 6592 -> 1600's 13.4 ->
+// 10.7 us the order alone is 1.0: rows off the 128-byte grid share a line between neighbouring pieces).
 //
-// Measured (us, weights from memory, the best other kernel | this one): M = 174, N = 1088, K = 4544 12.5 | 8.6;
-// M = 102, N = 1280, K = 6784 16.2 | 10.1; M = 267, N = 256, K = 8704 19.6 | 10.3; M = 364, N = 320, K = 11968 24.7 | 14.8.
-// At those a block pulls 64 K bytes at 48 ... 60 bytes a nanosecond behind 2 us of launch and first bytes.  Tried: 64 x 64
-// tiles the same way (never the best: M = 561, N = 1920, K = 6528 33 against 27); rows off the 16-byte grid read where
-// they lie (M = 1633, N = 163, K = 5834 20.9 against 17.2 for the tiles that stage them), which are copied onto the grid
-// instead; 32 x 32 tiles of four waves, two blocks a CU, where there are more than 256 (M = 2129, N = 192, K = 7104 21.9
-// against 15.6 for 32 x 64 tiles of eight).
+// Measured (us, weights from memory, the best other kernel | this one): M = 56, N = 1920, K = 4752 12.8 | 8.4; M = 63, N = 107,
+// K = 5376 11.5 | 7.4; M = 407, N = 154, K = 6080 10.9 (its former self) | 8.2; M = 364, N = 320, K = 11968 24.7 | 14.8 before.
+// Tried: 64 x 64 tiles the same way (256 registers; 273 x 5760 -> 2432 14.0 against 13.9 for lone 64 x 64 tiles in a ring of six
+// stages, 482 x 5232 -> 768 14.4); K split over two to sixteen blocks as well, the last to arrive adding the others' partial sums
+// (51 x 8384 -> 256 8.5 -> 7.9 with three, otherwise level or behind: the sums' way through memory costs 2.5 us); rows off
+// the 16-byte grid read where they lie (M = 1633, N = 163, K = 5834 20.9 against 17.2 for the tiles that stage them), which are
+// copied onto the grid instead; tiles of four waves, two blocks a CU, where there are more than 256 (1445 x 1472 -> 288 6.9
+// against 5.9 for 32 x 64 tiles of eight).
 #pragma once
 
 #include "gemm_i8_onepass.h"
@@ -25,6 +31,15 @@
 namespace tmq {
 
 constexpr int kWloopWaves = 8;
+
+// What the epilogue reads of the kernel's arguments, into scalar registers: called with a wave's requests on their way, so that
+// the argument buffer's latency passes under theirs and not behind the last barrier.
+__device__ __forceinline__ GemmArgs epilogue_args(const GemmArgs& a) {
+  GemmArgs e = a;
+  asm volatile("" : "+s"(e.M), "+s"(e.N), "+s"(e.bias), "+s"(e.w_scale_stride), "+s"(e.out_scale), "+s"(e.zp_f), "+s"(e.lo_f),
+                    "+s"(e.hi_f), "+s"(e.y), "+s"(e.ldy), "+s"(e.n_off), "+s"(e.f_kind));
+  return e;
+}
 
 // Tiles of 32 rows x 32 CT channels, PB bytes of K a piece.
 template <int MODE, int CT>
@@ -47,10 +62,9 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   const int K = static_cast<int>(a.K);
   const int KC = K >> 4;                     // 16-byte chunks of a row (K is a multiple of 16)
   const int pieces = (K + PB - 1) / PB;
-  // this wave's pieces: an equal run of them
-  const int each = pieces / WAVES, more = pieces - each * WAVES;
-  const int first = wave_u * each + (wave_u < more ? wave_u : more);
-  const int last = first + each + (wave_u < more ? 1 : 0);
+  // this wave's pieces: every eighth, so that neighbouring ones, which share the lines that rows off the 128-byte grid
+  // have at a piece's ends, are asked for together
+  int p = wave_u, left = wave_u < pieces ? (pieces - wave_u + WAVES - 1) / WAVES : 0;
 
   const uint8_t* const xtile = xs.x + m0 * xs.ldx;
   const int slot = lane % kLPR;
@@ -76,20 +90,21 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   struct Piece {
     v4i x[kNX], w[CT][kSteps];
   };
-  // (pieces past this wave's last fetch that one again and are not multiplied; chunks past K: bytes of the row, zeroed below)
+  // (chunks past K: bytes of the row, zeroed below)
   const auto request = [&](int p, Piece& pc) {
-    const int pp = p < last ? p : last > 0 ? last - 1 : 0;
-    const int c = pp * kLPR + slot;
+    __builtin_amdgcn_sched_barrier(0);
+    const int c = p * kLPR + slot;
     const uint32_t off = static_cast<uint32_t>(c < KC ? c : KC - 1) * 16u;
 #pragma unroll
     for (int i = 0; i < kNX; ++i) pc.x[i] = ld16(xtile + (xrow[i] + off));
 #pragma unroll
     for (int j = 0; j < kSteps; ++j) {
-      const int kc = pp * kLPR + 2 * j + half;
+      const int kc = p * kLPR + 2 * j + half;
       const int64_t woff = static_cast<int64_t>(kc < kc_last ? kc : kc_last) * 256;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) pc.w[ct][j] = ld16(wlane[ct] + woff);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
   // (the tile's constants first: nothing behind them is waited for when they are put down at the end)
   const int64_t n_raw = (n0 + t % BN < a.N ? n0 + t % BN : a.N - 1) + a.n_off;
@@ -100,11 +115,6 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
     bias = __float_as_int((a.bias != nullptr ? a.bias : a.w_scales)[a.bias != nullptr ? n_raw : 0]);
   }
   Piece pc[2];
-  __builtin_amdgcn_sched_barrier(0);
-  request(first, pc[0]);
-  __builtin_amdgcn_sched_barrier(0);
-  request(first + 1, pc[1]);
-  __builtin_amdgcn_sched_barrier(0);
   v16i acc[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct)
@@ -121,7 +131,7 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
     for (int i = 0; i < kNX; ++i) {
       const int r = i * kRPL + lane / kLPR;
       v4i v = pc.x[i];
-      const int keep = c < KC && p < last ? -1 : 0;
+      const int keep = c < KC ? -1 : 0;
       v = (v ^ v4i{flip, flip, flip, flip}) & v4i{keep, keep, keep, keep};
       *reinterpret_cast<v4i*>(mine + r * PB + ((slot ^ swizzle(r)) << 4)) = v;
     }
@@ -134,16 +144,37 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
     }
     wave_sync_lds();                         // (the next piece is written over this one)
   };
-  // (both pieces in every turn, an odd last one with zeros: the counts of outstanding requests stay exact)
-  for (int p = first; p < last; p += 2) {
+  // Straight code for the pieces that are left, so that nothing is fetched that is not multiplied and the compiler knows
+  // how many requests are behind the one it waits for.
+  constexpr int kNext = WAVES;
+  XQuant xq;
+  GemmArgs e;
+  const auto arguments = [&] {
+    xq = x_quant(a);
+    e = epilogue_args(a);
+  };
+  if (left >= 2) {
+    request(p, pc[0]);
+    request(p + kNext, pc[1]);
+    arguments();
+    for (; left >= 4; left -= 2, p += 2 * kNext) {
+      multiply(p, pc[0]);
+      request(p + 2 * kNext, pc[0]);
+      multiply(p + kNext, pc[1]);
+      request(p + 3 * kNext, pc[1]);
+    }
     multiply(p, pc[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    request(p + 2, pc[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(p + 1, pc[1]);
-    __builtin_amdgcn_sched_barrier(0);
-    request(p + 3, pc[1]);
-    __builtin_amdgcn_sched_barrier(0);
+    if (left == 3) {
+      request(p + 2 * kNext, pc[0]);
+      multiply(p + kNext, pc[1]);
+      multiply(p + 2 * kNext, pc[0]);
+    } else {
+      multiply(p + kNext, pc[1]);
+    }
+  } else {
+    if (left == 1) request(p, pc[0]);
+    arguments();
+    if (left == 1) multiply(p, pc[0]);
   }
   if (t < BN) {
     s_raw[0][t] = colsum;
@@ -162,7 +193,7 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   __syncthreads();
 #pragma unroll
   for (int idx = t; idx < BM * BN / 4; idx += WAVES * kWave)
-    ksplit_finish_four<MODE, BN, WAVES>(a, &sX[0][0], kWaveLds, s_raw, m0, n0, idx);
+    ksplit_finish_four<MODE, BN, WAVES>(e, &sX[0][0], kWaveLds, s_raw, xq, m0, n0, idx);
 }
 
 }  // namespace tmq

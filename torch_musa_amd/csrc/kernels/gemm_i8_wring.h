@@ -213,9 +213,10 @@ __global__ __launch_bounds__(kWringThreads) void gemm_i8_wring_kernel(GemmArgs a
         *reinterpret_cast<v4i*>(&sX[wave_u][(32 * rt + li) * kRedPitch + (32 * ct + 8 * g + 4 * half) * 4]) = part;
       }
   __syncthreads();
+  const XQuant xq = x_quant(a);  // (not in front: the waits above count requests)
 #pragma unroll
   for (int idx = t; idx < BM * BN / 4; idx += kWringThreads)
-    ksplit_finish_four<MODE, BN, WAVES>(a, &sX[0][0], kWaveLds, s_raw, m0, n0, idx);
+    ksplit_finish_four<MODE, BN, WAVES>(a, &sX[0][0], kWaveLds, s_raw, xq, m0, n0, idx);
 }
 
 }  // namespace tmq

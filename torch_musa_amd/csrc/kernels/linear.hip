@@ -625,27 +625,6 @@ int launch_gemm_ksplit(const GemmArgs& a, const XLinear& xs, hipStream_t s) {
   return launch_status();
 }
 
-// Tiles of 32 rows whose waves split K, weights through registers (K <= 4096; the caller
-// checked the address ranges).  wide: 64 channels per tile instead of 32.
-template <int MODE, bool RUNS>
-int launch_gemm_wstream_as(const GemmArgs& a, const XLinear& xs, bool wide, dim3 grid, hipStream_t s) {
-  if (!wide && a.K <= 2048)
-    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 16>, grid, dim3(256), 0, s, a, xs);
-  else if (!wide)
-    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 32>, grid, dim3(256), 0, s, a, xs);
-  else
-    enqueue(gemm_i8_wstream_kernel<MODE, RUNS, 16, 2, 8>, grid, dim3(512), 0, s, a, xs);
-  return launch_status();
-}
-template <int MODE>
-int launch_gemm_wstream(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
-  const int64_t tiles_m = ceil_div(a.M, 32), tiles_n = ceil_div(a.N, wide ? 64 : 32);
-  if (tiles_n > 0x7fffffff || tiles_m > 65535 || a.K > 4096) return TMQ_ERR_UNSUPPORTED;
-  const dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
-  return tiles_n * tiles_m <= 0x7fffffff && tile_runs(tiles_m, tiles_n, a) ? launch_gemm_wstream_as<MODE, true>(a, xs, wide, grid, s)
-                                                                           : launch_gemm_wstream_as<MODE, false>(a, xs, wide, grid, s);
-}
-
 // 64 x 64 tiles whose eight waves split K, weights through registers, activations through
 // a ring per wave (K <= 4096; the caller checked the address ranges).
 template <int MODE>
@@ -667,6 +646,13 @@ int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream
   if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2>, grid, block, 0, s, a, xs);
   else enqueue(gemm_i8_wloop_kernel<MODE, 1>, grid, block, 0, s, a, xs);
   return launch_status();
+}
+
+// The same for K up to 4096 (cfg 25, 26), two tiles of 32 channels side by side in a block where one round holds those only
+// (us, weights from memory, four waves a tile and two blocks a CU | pairs: 71 x 1120 -> 3200 5.6 | 4.6, 1445 x 1472 -> 288 7.4 |
+// 5.3, 512 x 2048 -> 1024 6.7 | 6.1).
+bool wstream_pairs(int64_t M, int64_t N) {
+  return ceil_div(M, 32) * ceil_div(N, 32) > 256 && ceil_div(M, 32) * ceil_div(N, 64) <= 256;
 }
 
 // One block per CU walks the 256 x 256 tiles (byte or float outputs, direct copies two
@@ -845,20 +831,14 @@ bool two_wave_groups_fit(int64_t M, int64_t N, int64_t K) {
 SplitPlan plan_split_tiles(int64_t M, int64_t N, int64_t K);
 
 // Shapes for the tiles of 32 rows whose waves split K and stream their weights through
-// registers: K beyond what the kernels with all operands in LDS take, one round of
-// blocks (two blocks share a CU while a block's activations, 32 rows x K, are at
-// most 64 KB).  With more blocks than that it loses to the larger tiles (K = 4096:
-// N = 4096, M = 96: 13.7 against 12.8 us; K = 2048, N = 4096, M = 256: 10.7 against 9.7 us).
-// Returns the channels per tile: 32; 64 (eight waves, K > 2048 only: at K <= 2048 it
-// never beat the 32 x 32 tiles where they fit nor the larger tiles where they do not)
-// when only those fit one round (K = N = 4096: M = 96 12.8 -> 9.9 us, M = 128 14.1 -> 10.0 us;
-// N = 8192, M = 64: 15.7 -> 11.5 us; N = 2048, M = 256: 13.6 -> 9.5 us; where both fit, 32
-// channels are 1.5 us ahead); 0: neither.
+// registers (gemm_i8_wloop.h): K beyond what the kernels with all operands in LDS take, one round of blocks of 32 or 64
+// channels.  With more than that it loses to the larger tiles.  Returns the channels per tile: 32 (K <= 2048: by pairs
+// where single ones are more than a round, wstream_pairs), 64; 0: neither.
 int wstream_tile(int64_t M, int64_t N, int64_t K) {
   if (K <= kOnePassMaxK || K > 4096) return 0;
-  if (ceil_div(M, 32) * ceil_div(N, 32) <= (K <= 2048 ? 512 : 256)) return 32;
-  if (K > 2048 && ceil_div(M, 32) * ceil_div(N, 64) <= 256) return 64;
-  return 0;
+  const bool pairs = ceil_div(M, 32) * ceil_div(N, 64) <= 256;
+  if (ceil_div(M, 32) * ceil_div(N, 32) <= 256 || (K <= 2048 && pairs)) return 32;
+  return pairs ? 64 : 0;
 }
 
 // One round of 64 x 64 tiles against K > 4096 whose last row tile is at least three
@@ -874,40 +854,34 @@ bool phased_ring_preferred(int64_t M, int64_t N, int64_t K) {
   return K > 4096 ? M <= 128 : (K == 4096 && M <= 64 && N >= 10240);
 }
 
-// More than 48 (32) rows against K beyond what the kernels above hold at once, one round of tiles of 32 rows: eight waves a
-// tile that walk their shares of K (gemm_i8_wloop.h).  Us, the best other kernel | it, weights from memory:
-//   up to 256 tiles of 32 x 32: 526 x 11936 -> 464 33.3 | 16.5; 373 x 8832 -> 576 19.9 | 11.5; 322 x 4352 -> 384 12.1 | 8.0;
-//     58 x 11840 -> 2944 20.3 | 18.3; 53 x 10832 -> 96 level at 13.0; at K = 4096 and below behind those that hold K at
-//     once (593 x 4096 -> 384 7.1 | 8.3);
-//   up to 256 of 32 x 64: 225 x 4992 -> 1392 13.3 | 10.6; 250 x 6720 -> 1216 19.8 | 12.7; 111 x 7808 -> 2576 21.2 | 16.3;
-//     289 x 12128 -> 1600 28.6 | 21.5; not for more than 32 Mi weights, near level (54 x 5440 -> 7616 18.2 | 17.1), nor
-//     from K = 9216 on more than 20 Mi, where a split along K into two launches is ahead (114 x 10576 -> 2304 20.6 | 22.3);
-//   up to 48 rows weights stream as fast (41 x 5712 -> 144 9.0 | 10.0, 37 x 6592 -> 1664 10.6 | 12.0, 23 x 8128 -> 448
-//     8.5 | 9.9) but for more than 32 from K = 7680 on: 38 x 9408 -> 432 14.4 | 12.2, 46 x 8960 -> 768 13.7 | 10.6; up to 40 rows
-//     not against more than 17 Mi weights short of K = 10240 (34 x 7808 -> 3504 11.6 | 12.4, 34 x 9536 -> 3216 14.9 | 15.9, 40 x
-//     7872 -> 2816 11.8 | 12.4; 35 x 8768 -> 1584 0.80 of the time, 36 x 10752 -> 2304 0.90).
-// The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and 32 Mi weights, which their tests hold as the
-// automatic choice; measured, this kernel is ahead there throughout (128 x 4608 -> 256 14.7 | 7.3, 128 x 4288 -> 1296 14.4 | 8.7, 116 x
-// 4480 -> 1728 15.2 | 12.2).  Measured up to K = 12288.  Returns the channels per tile, 0: not such a shape.
+// More than 32 rows against K beyond 4096, one round of tiles of 32 rows: eight waves a tile that walk K in pieces
+// (gemm_i8_wloop.h).  Us, the best other kernel | it, weights from memory:
+//   up to 256 tiles of 32 x 32: 63 x 5376 -> 107 11.5 | 7.35; 49 x 4160 -> 430 9.9 | 6.35; 76 x 9168 -> 2336 17.8 | 12.0; 37 x 4624 -> 304
+//     8.9 | 6.3; 135 x 11552 -> 1488 21.1 | 13.5;
+//   up to 256 of 32 x 64: 71 x 5936 -> 3504 16.0 | 12.0; 127 x 4576 -> 4080 15.7 | 10.8; 42 x 6704 -> 6624 19.4 | 14.4; 74 x 8752 -> 5040
+//     21.7 | 16.8; 65 x 10496 -> 4880 22.8 | 17.9; 85 x 11296 -> 2736 21.2 | 20.6;
+//   up to 32 rows weights stream as fast (18 x 5296 -> 1584 7.2 | 8.3, 26 x 8144 -> 192 8.0 | 8.8; 30 x 4656 -> 128 6.9 | 6.1), up to
+//     40 against more than 17 Mi weights short of K = 10240 likewise when that line was drawn (now ahead, 36 x 6288 -> 5632 17.7 | 12.9).
+// The tiles that walk K as a ring of phases keep their shapes up to K = 5632 and, of 64 channels, those of more than 32 Mi weights,
+// which their tests hold as the automatic choice; measured, this kernel is ahead there throughout (128 x 4608 -> 256 14.7 | 6.6,
+// 48 x 4288 -> 5024 15.0 | 10.3).  Measured up to K = 12288.  Returns the channels per tile, 0: not such a shape.
 constexpr int64_t kWloopMaxK = 12288, kWloopRingMinK = 5632;
 int wloop_tile(int64_t M, int64_t N, int64_t K) {
-  if (M <= (K >= 7680 ? 32 : 48) || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
+  if (M <= 32 || K <= 4096 || K > kWloopMaxK || K % 16 != 0) return 0;
   if (M <= 40 && N * K > int64_t{17} << 20 && K < 10240) return 0;
-  if (K < kWloopRingMinK && phased_ring_preferred(M, N, K)) return 0;
+  const bool ring = phased_ring_preferred(M, N, K);
+  if (ring && K < kWloopRingMinK) return 0;
   if (ceil_div(M, 32) * ceil_div(N, 32) <= 256) return 32;
-  if (M > 48 && ceil_div(M, 32) * ceil_div(N, 64) <= 256 && N * K <= int64_t{K < 9216 ? 32 : 20} << 20) return 64;
-  return 0;
+  return ceil_div(M, 32) * ceil_div(N, 64) <= 256 && !(ring && N * K > int64_t{32} << 20) ? 64 : 0;
 }
 
 SmallRows small_rows_path(int64_t M, int64_t N, int64_t K, bool workspace) {
-  // Where the 32 x 32 tiles with the weights through registers fit, they are measured
-  // directly against the weight-streaming kernel (us at M = 17 / 32 / 40 / 64, tiles | streaming):
-  //   K = 2048, N = 4096:  5.2 / 5.4 / 5.5 / 5.5 | 5.7 / 5.9 / 7.2 / 9.3    K = 4096, N = 1024:  6.7 / 6.7 / 6.7 / 6.7 | 5.3 / 5.5 / 6.9 / 8.6
-  //   K = 4096, N = 4096:  8.4 / 8.5 / 8.6 / 8.7 | 6.4 / 7.5 / 8.6 / 11.3   K = 3072, N = 3072:  7.2 / 7.2 / 7.2 / 7.4 | 5.5 / 6.1 / 7.2 / 10.0
-  //   K = 3072, N = 4096:  7.4 / 7.4 / 7.5 / 7.7 | 5.9 / 6.5 / 7.7 / 10.9   K = 4096, N = 8192: 10.8 / 10.9 / -   / -   | 11.1 / 12.2 / 14.5 / 20.6
-  // streaming keeps K > 2048 up to 32 rows (two row groups) while its blocks fit one round.
+  // Where the tiles of 32 rows with the weights through registers fit, they are measured directly against the
+  // weight-streaming kernel, which keeps K > 3008 up to 32 rows (two row groups) while its blocks fit one round (us, tiles |
+  // streaming: 18 x 2176 -> 545 4.4 | 5.0, 28 x 2288 -> 2000 4.5 | 5.1, 20 x 2576 -> 144 4.4 | 4.8, 32 x 3024 -> 544 level at 5.0,
+  // 29 x 3744 -> 160 5.5 | 5.0, 24 x 3696 -> 2661 7.2 | 5.9, 31 x 4096 -> 1600 6.1 | 5.4; 24 x 2784 -> 4864 6.4 | 8.9).
   if (wstream_tile(M, N, K) != 0)
-    return K > 2048 && M <= 32 && N <= 4096 ? SmallRows::kStream : SmallRows::kTiles;
+    return K > 3008 && M <= 32 && N <= 4096 ? SmallRows::kStream : SmallRows::kTiles;
   const double mib = static_cast<double>(N) * static_cast<double>(K) / 1048576.0;
   const double stages = static_cast<double>(ceil_div(K, kBK));
   const double rows = static_cast<double>(M);
@@ -1590,8 +1564,8 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
                                                                   : launch_gemm<64, 128, 2, 2, MODE>(a, xs, s);
     case 21: return launch_gemm_onepass<MODE>(a, xs, s);
     case 24: return launch_gemm_ksplit<MODE>(a, xs, s);
-    case 25: return launch_gemm_wstream<MODE>(a, xs, false, s);
-    case 26: return launch_gemm_wstream<MODE>(a, xs, true, s);
+    case 25: return launch_gemm_wloop<MODE>(a, xs, wstream_pairs(a.M, a.N), s);
+    case 26: return launch_gemm_wloop<MODE>(a, xs, true, s);
     case 27: return launch_gemm_wring<MODE>(a, xs, s);
     case 29: case 30: return launch_gemm_wloop<MODE>(a, xs, c.cfg == 30, s);
     default: return TMQ_ERR_UNSUPPORTED;
@@ -1725,7 +1699,8 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     case 5: bm = 256, bn = 128; break;
     case 22: bm = 128, bn = 64; break;
     case 23: bm = 64, bn = 128, waves = c.onepass ? 8 : 4; break;
-    case 24: case 25: bm = 32, bn = 32; break;
+    case 24: bm = 32, bn = 32; break;
+    case 25: bm = 32, bn = 32, waves = kWloopWaves; break;
     case 26: bm = 32, bn = 64, waves = 8; break;
     case 27: bm = 64, bn = 64, waves = 8; break;
     case 29: bm = 32, bn = 32, waves = kWloopWaves; break;
@@ -1746,6 +1721,7 @@ TMQ_EXPORT int tmq_linear_kernel_choice(int64_t M, int64_t N, int64_t K, int64_t
     out->tiles = ceil_div(M, bm) * ceil_div(N, bn) * c.split.splits;
     out->blocks = out->tiles;
     if (c.cfg == 20 && out->tiles > compute_units) out->blocks = compute_units / 8 * 8;
+    if (c.cfg == 25 && wstream_pairs(M, N)) out->blocks = ceil_div(M, 32) * ceil_div(N, 64);
     if (c.cfg == 28) out->blocks = std::min<int64_t>(out->tiles, (waves == 8 ? 2 : 1) * static_cast<int64_t>(compute_units));
   }
   return TMQ_OK;
