@@ -939,6 +939,13 @@ SplitPlan plan_split_tiles(int64_t M, int64_t N, int64_t K) {
 
 // The plan the automatic choice follows: none for the rows that stream the
 // weights, and for 17 ... 64 rows only where the estimate above prefers it.
+// Not where one round holds the product in 64 x 64 tiles but not in tiles of 32 rows: the lone tiles' ring is ahead up to
+// K = 10752, and beyond against more than 550 thousand outputs (us, split | ring, weights from memory: 661 x 8544 -> 1408 28.4 |
+// 21.1, 478 x 8736 -> 1152 25.9 | 21.3, 168 x 8656 -> 4736 27.2 | 23.3, 1110 x 11504 -> 794 33.7 | 27.2, 683 x 11872 -> 832 27.8 |
+// 28.8; 194 x 10976 -> 2560 23.2 | 26.0, 180 x 13024 -> 2752 26.8 | 34.7, 80 x 12896 -> 5632 27.0 | 31.0).
+bool ring_ahead_of_split(int64_t M, int64_t N, int64_t K) {
+  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && ceil_div(M, 32) * ceil_div(N, 64) > 256 && (K < 10752 || M * N > 550000);
+}
 SplitPlan plan_split(int64_t M, int64_t N, int64_t K) {
   if (M > kDecodeRowsAuto && M <= kDecodeMaxRows && small_rows_path(M, N, K, true) != SmallRows::kSplit)
     return SplitPlan{};
@@ -1237,6 +1244,15 @@ int tile_by_rounds(int cfg, bool onepass, int64_t M, int64_t N, int64_t K) {
   return best == 17 && (cfg == 19 || (K >= 1104 && ceil_div(M, 128) * ceil_div(N, 256) <= 256)) ? 19 : best;
 }
 
+// One round of 64 x 64 tiles beyond the shapes that tile_by_rounds models: the lone tile's ring of six stages is ahead of two
+// wave groups (cfg 2, 14) and of the kernel whose waves take their weights through registers (27), which wait for their
+// stages in registers or for the weights they asked for at once (us, weights from memory, those | the ring: 1452 x 4016 -> 369
+// 14.1 | 11.3, 759 x 4432 -> 960 13.6 | 11.6, 173 x 7264 -> 4026 22.9 | 20.3, 1418 x 7088 -> 512 19.4 | 16.5, 49 x 3408 -> 8256 15.3 |
+// 13.0, 88 x 4352 -> 8192 level at 14.0; 70 shapes drawn over K = 1100 ... 14000: never more than 3 % behind, 6 % ahead on average).
+bool lone_ring_first(int cfg, const LinearQuery& q) {
+  return (cfg == 2 || cfg == 14 || cfg == 27) && one_round_ring(q.M, q.N, q.K) && dma_limits_ok(q.K, q.ldx);
+}
+
 // forced: tmq_linear_desc::kernel - 1 (-1 = automatic choice).
 LinearChoice choose_linear(const LinearQuery& q, int forced) {
   LinearChoice c;
@@ -1267,7 +1283,8 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
   const bool dma_ok = dma_limits_ok(q.K, q.ldx);
   if (forced < 0 || forced == 13) {
     const SplitPlan p = forced == 13 ? plan_split_tiles(q.M, q.N, q.K) : plan_split(q.M, q.N, q.K);
-    if (p.splits > 1 && q.workspace_bytes >= split_workspace_bytes(p, q.M)) {
+    if (p.splits > 1 && q.workspace_bytes >= split_workspace_bytes(p, q.M) &&
+        (forced == 13 || q.mode == kOutAcc32 || !ring_ahead_of_split(q.M, q.N, q.K))) {
       c.cfg = 13;
       c.split = p;
       return c;
@@ -1391,6 +1408,10 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
     if (by_rounds != cfg) c.onepass = false;
     if (by_rounds == 2 && rounds_modelled(M, N, K)) c.groups = 1;
     cfg = by_rounds;
+  }
+  if (forced < 0 && q.mode != kOutAcc32 && lone_ring_first(cfg, q)) {
+    cfg = 2;
+    c.groups = 1;
   }
   if (forced < 0 && q.mode != kOutAcc32 && (cfg == 1 || cfg == 2 || cfg == 7 || cfg == 14 || cfg == 17) &&
       oblong_ring_first(M, N, K, q.ldx)) {
