@@ -381,8 +381,8 @@ int tmq_linear_float(const tmq_linear_desc* desc, const tmq_qparams* x_qparams_d
  * fp32 x [M, ldx] -> fp32 y [M, ldy] with M <= 16, K >= 16, and (K rounded up to
  * a multiple of 4) either M * K <= 16384 (every block of the
  * weight-streaming kernel derives the activation range, parameters and codes
- * itself while its weights are on their way) or M * K <= 32768 with
- * 64 <= K <= 8192 (one block per CU does so once, keeps the codes in LDS and
+ * itself while its weights are on their way) or M * K <= 32768 -- 65536 from
+ * N = 10240 on -- with 64 <= K <= 8192 (one block per CU does so once, keeps the codes in LDS and
  * streams the channel groups it owns; the library picks between the two where
  * both apply).  TMQ_ERR_UNSUPPORTED otherwise: use
  * tmq_quantize_per_tensor_dynamic_dev + tmq_linear_f32, which give the same

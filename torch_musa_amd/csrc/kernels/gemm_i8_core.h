@@ -263,18 +263,6 @@ __device__ __forceinline__ v4i shift_up_bytes(v4i v, int s) {
   const uint64_t nlo = b < 64 ? lo << b : 0;
   return v4i{static_cast<int>(nlo), static_cast<int>(nlo >> 32), static_cast<int>(nhi), static_cast<int>(nhi >> 32)};
 }
-// Four fp32 values 4 c4 ... 4 c4 + 3 of a row of K >= 4 values (4-byte aligned), zeros behind its
-// end, by the same clamped load.  (A zero does not change the range of a dynamic quantization:
-// ChooseQuantizationParams extends every range to hold 0.)
-struct __attribute__((packed, aligned(4))) V4fRow {
-  v4f v;
-};
-__device__ __forceinline__ v4f load_row4(const float* row, int c4, int K) {
-  const int at = 4 * c4 < K - 4 ? 4 * c4 : K - 4, s = 4 * c4 - at;
-  const v4f v = reinterpret_cast<const V4fRow*>(row + at)->v;
-  return v4f{s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w, s == 0 ? v.y : s == 1 ? v.z : s == 2 ? v.w : 0.f,
-             s == 0 ? v.z : s == 1 ? v.w : 0.f, s == 0 ? v.w : 0.f};
-}
 typedef int v2i __attribute__((ext_vector_type(2)));
 struct __attribute__((packed, aligned(1))) V2iAnyAlignment {
   v2i v;

@@ -348,8 +348,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
   static_assert(kHeld * 4 * kWaves * kWave <= kDynSmallMaxValues, "held values");
   extern __shared__ __attribute__((aligned(16))) uint8_t sx[];  // [M][pitch] activation codes
   __shared__ int s_sum[4][kWave];  // the waves' partial sums, added with LDS atomics (see linear_decode_kernel)
-  __shared__ float s_mn[kWaves], s_mx[kWaves];
-  __shared__ float s_scale, s_inv, s_zp;
+  __shared__ float s_range[2 * kWaves + 3];
   const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
   const int lr = lane & 15, lc = lane >> 4;
   const int64_t nb = blockIdx.x;
@@ -374,16 +373,8 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
   // ---- the input: requested first (loads return in order: behind the weight
   // stream it would arrive only after it), held in registers between the range
   // pass and the quantization
-  const int k4 = (K + 3) / 4;
-  const int total4 = static_cast<int>(a.M) * k4;
-  v4f held[kHeld];
-#pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int e = t + u * (kWaves * kWave);
-    const int ec = e < total4 ? e : 0;  // unconditional loads keep the load counter exact
-    const int row = ec / k4, c4 = ec - row * k4;
-    held[u] = load_row4(x + row * ldxf, c4, K);
-  }
+  HeldRows<kHeld, kWaves * kWave> rows;
+  rows.load(x, ldxf, static_cast<int>(a.M), K, t);
   // then the first batch of weights: on its way while the input is processed
   v4i wf[kBatch];
 #pragma unroll
@@ -393,60 +384,12 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
     wf[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wp + kbc * 1024));
   }
   __builtin_amdgcn_sched_barrier(0);
-  float mn = __builtin_inff(), mx = -__builtin_inff();
-#pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int e = t + u * (kWaves * kWave);
-    if (e < total4) {
-      const v4f v = held[u];
-      mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
-      mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
-    }
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    mn = fminf(mn, __shfl_xor(mn, off, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-  }
-  if (lane == 0) {
-    s_mn[wave] = mn;
-    s_mx[wave] = mx;
-  }
   if (t < 4 * kWave) (&s_sum[0][0])[t] = 0;  // (two barriers before the first addition)
-  __syncthreads();
-  if (t == 0) {
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
-      mn = fminf(mn, s_mn[w]);
-      mx = fmaxf(mx, s_mx[w]);
-    }
-    double sc;
-    int32_t zp;
-    choose_qparams(mn, mx, 0, 255, reduce_range != 0, &sc, &zp);
-    const float scf = static_cast<float>(sc);
-    s_scale = scf;
-    s_inv = 1.0f / scf;  // IEEE division, as the separate quantize kernels
-    s_zp = static_cast<float>(zp);
-  }
-  __syncthreads();
-  const float inv = s_inv, zp_f = s_zp;
-#pragma unroll
-  for (int u = 0; u < kHeld; ++u) {
-    const int e = t + u * (kWaves * kWave);
-    if (e < total4) {
-      const int row = e / k4, c4 = e - row * k4;
-      const v4f v = held[u];
-      uint32_t q = 0;
-      const float f[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float r = __builtin_rintf(__builtin_fmaf(f[j], inv, zp_f));
-        r = fminf(fmaxf(r, 0.f), 255.f);
-        q |= static_cast<uint32_t>(static_cast<int>(r)) << (8 * j);
-      }
-      *reinterpret_cast<uint32_t*>(sx + row * pitch + c4 * 4) = q;
-    }
-  }
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  rows.range(mn, mx);
+  float scale, inv, zp_f;
+  block_qparams<kWaves>(mn, mx, s_range, t, reduce_range != 0, [] { __syncthreads(); }, scale, inv, zp_f);
+  rows.codes(inv, zp_f, [&](int row, int c4, uint32_t q) { *reinterpret_cast<uint32_t*>(sx + row * pitch + c4 * 4) = q; });
   __syncthreads();
   // ---- the product, activation operands from LDS (rows past M are zero)
   const v4i xmask = {static_cast<int>(0x80808080u), static_cast<int>(0x80808080u), static_cast<int>(0x80808080u),
@@ -484,7 +427,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void linear_decode_dynamic_ker
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       acc0[j] = coef * c_cs[j];
-      mult[j] = s_scale * c_ws[j];
+      mult[j] = scale * c_ws[j];
       bias[j] = c_b[j];
     }
   }
@@ -1890,16 +1833,18 @@ TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qpa
   return tmq_linear_float(d, x_qparams_dev, y, ldy, TMQ_FLOAT_F32, stream);
 }
 
-// The float rows of the one-launch dynamic linear as the resident kernel holds them: 16 waves x 64
-// lanes x up to 8 groups of four values (16 groups -- M = 16 at K = 4096 -- spill registers and every
-// CU then reads 256 KB of rows: 14.2 us against 11.0 us for the two launches at N = 4096).
-constexpr int64_t kDynResidentMaxValues = 32768;
+// The float rows of the one-launch dynamic linear as the resident kernel holds them: 16 waves x 64 lanes x up to 16 groups of
+// four values.  More than 8 groups only against many channels, whose stream is what the block's work on the rows passes under
+// (us, two launches | one: 16 x 4096 -> 11008 14.2 | 13.7, 10 x 4096 -> 11008 13.85 | 13.1, 12 x 3072 -> 11008 12.5 | 11.9, 16 x 2560
+// -> 11008 11.7 | 11.55; -> 8192 0.95 to 1.03 of the time, 16 x 4096 -> 4096 9.5 | 10.6, -> 256 8.15 | 9.2).
+constexpr int64_t kDynResidentMaxValues = 32768, kDynResidentMostValues = 65536, kDynResidentManyChannels = 10240;
 
 namespace {
 // Groups of four values, the last one of a row perhaps partly behind its end.
 int64_t dyn_groups(int64_t M, int64_t K) { return M * ceil_div(K, 4); }
 bool dyn_resident_ok(int64_t M, int64_t N, int64_t K, int cus) {
-  return 4 * dyn_groups(M, K) <= kDynResidentMaxValues && resident_limits_ok(M, N, round_up(K, 16), K, cus);
+  return 4 * dyn_groups(M, K) <= (N < kDynResidentManyChannels ? kDynResidentMaxValues : kDynResidentMostValues) &&
+         resident_limits_ok(M, N, round_up(K, 16), K, cus);
 }
 }  // namespace
 
@@ -1937,7 +1882,7 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
   a.ldy = ldy;
   hipStream_t s = as_stream(stream);
   // Two kernels: a block per 16 channels that repeats the work on the input (up to 16384 values), and
-  // one block per CU that does it once for all its channel groups (up to 32768 values, K <= 8192).
+  // one block per CU that does it once for all its channel groups (dyn_resident_ok).
   // desc->kernel pins one for tests: 9 the first, 29 the second.
   const int cus = cu_count();
   const bool resident_ok = dyn_resident_ok(d->M, d->N, d->K, cus);
@@ -1954,8 +1899,10 @@ TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x
       enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 2>, grid, block, 0, s, a, none, x, ldx, reduce_range);
     else if (held <= 4)
       enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 4>, grid, block, 0, s, a, none, x, ldx, reduce_range);
-    else
+    else if (held <= 8)
       enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 8>, grid, block, 0, s, a, none, x, ldx, reduce_range);
+    else
+      enqueue(linear_resident_kernel<kOutF32, 1, kResidentWaves, 16>, grid, block, 0, s, a, none, x, ldx, reduce_range);
     return launch_status();
   }
   const size_t lds = static_cast<size_t>(d->M) * static_cast<size_t>(round_up(d->K, 16) + 16);

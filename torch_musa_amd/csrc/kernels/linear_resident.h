@@ -25,15 +25,18 @@
 //
 // HELD > 0: the dynamically quantized linear in one launch (float rows in, float out, up to
 // 16 rows and HELD x 4096 values): the block reads the float rows instead of codes -- every
-// thread holds HELD groups of four values in registers --, reduces their range, one thread
+// thread holds HELD groups of four values in registers --, reduces their range, one wave
 // derives the parameters (ChooseQuantizationParams), and the held values are quantized into
 // the same LDS operand layout, product and zero point rounded once, as PyTorch's CPU
 // quantized::linear_dynamic does while packing.  All of it runs under the latency of the
-// first weight requests; the stream that follows is the same.
+// first weight requests; the stream that follows is the same.  The vector unit bounds that part: every CU works on all
+// values.  With a division per group of values for its row and a clamp, a conversion and shifts per code, 10 x 2616 -> 320 took
+// 8.1 us for 6.3 now, 14 x 1271 -> 1552 7.65 | 6.1, 4 x 3912 -> 192 6.6 | 5.7, 11 x 768 -> 1792 5.6 | 5.0 (dynamic_rows.h), and 16
+// groups a thread, which that left no registers for, 16 x 4096 -> 256 13.0 | 9.2.
 #pragma once
 
+#include "dynamic_rows.h"
 #include "gemm_i8_core.h"
-#include "qparams.h"
 
 namespace tmq {
 
@@ -65,8 +68,7 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
   __shared__ __attribute__((aligned(16))) float s_mult[kGroups * 16];
   __shared__ __attribute__((aligned(16))) float s_bdiv[kGroups * 16];
   __shared__ float s_bmul;
-  __shared__ float s_mn[W], s_mx[W];
-  __shared__ float s_scale, s_inv, s_zp;
+  __shared__ float s_range[2 * W + 3];
 
   const int t = threadIdx.x, lane = t % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
@@ -87,18 +89,10 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
   // (four lanes ask for one cache line); pieces are dealt round-robin to the waves
   constexpr int kXPieces = HELD > 0 ? 1 : kXBytes / 1024 / W;  // per wave, at most
   v4i xr[kXPieces];
-  constexpr int kHeldN = HELD > 0 ? HELD : 1;
-  v4f held[kHeldN];
+  HeldRows<(HELD > 0 ? HELD : 1), kThreads> rows;
   const int sr = lane >> 2, sp = lane & 3;
-  const int k4 = (K + 3) >> 2, total4 = M * k4;    // (dynamic form) groups of four float values
   if constexpr (HELD > 0) {
-#pragma unroll
-    for (int u = 0; u < HELD; ++u) {
-      const int e = t + u * kThreads;
-      const int ec = e < total4 ? e : 0;           // unconditional loads keep the load counter exact
-      const int row = ec / k4, c4 = ec - row * k4;
-      held[u] = load_row4(xf + row * ldxf, c4, K);
-    }
+    rows.load(xf, ldxf, M, K, t);
   } else {
 #pragma unroll
     for (int j = 0; j < kXPieces; ++j) {
@@ -142,8 +136,9 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
     return w;
   };
   v4i wf[D];
+  constexpr int kFirst = HELD > 8 ? 4 : D;         // (the rest once the held values have left their registers)
 #pragma unroll
-  for (int j = 0; j < D; ++j)
+  for (int j = 0; j < kFirst; ++j)
     if (j < Q) wf[j] = next_weights();
 
   // ---- activations into LDS: piece (mg, kb), chunk c of row r -> ((4 kb + c) * 16 MG + 16 mg + r) * 16
@@ -153,59 +148,17 @@ __global__ __launch_bounds__(W * kWave, 4) void linear_resident_kernel(GemmArgs 
     // rows past M and bytes past K stay zero: clear the area, then write the codes over it
     for (int i = t; i < KBP * 64; i += kThreads) *reinterpret_cast<v4i*>(&s_x[i * 16]) = v4i{0, 0, 0, 0};
     float mn = __builtin_inff(), mx = -__builtin_inff();
+    rows.range(mn, mx);
+    float scale, inv, zp_f;
+    block_qparams<W>(mn, mx, s_range, t, reduce_range != 0, [] { resident_barrier(); }, scale, inv, zp_f);
+    rows.codes(inv, zp_f, [&](int row, int c4, uint32_t q) {
+      // bytes 4 c4 .. 4 c4 + 3 of the row: k-block c4 / 16, chunk (c4 / 4) % 4, byte 4 (c4 % 4) of the chunk
+      *reinterpret_cast<uint32_t*>(&s_x[((c4 >> 2) * 16 + row) * 16 + (c4 & 3) * 4]) = q ^ 0x80808080u;
+    });
+    xq = XQuant{scale, 128 - static_cast<int>(zp_f)};
 #pragma unroll
-    for (int u = 0; u < HELD; ++u) {
-      if (t + u * kThreads < total4) {
-        const v4f v = held[u];
-        mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
-        mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
-      }
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      mn = fminf(mn, __shfl_xor(mn, off, kWave));
-      mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-    }
-    if (lane == 0) {
-      s_mn[wave] = mn;
-      s_mx[wave] = mx;
-    }
-    resident_barrier();
-    if (t == 0) {
-#pragma unroll
-      for (int w = 1; w < W; ++w) {
-        mn = fminf(mn, s_mn[w]);
-        mx = fmaxf(mx, s_mx[w]);
-      }
-      double sc;
-      int32_t zp;
-      choose_qparams(mn, mx, 0, 255, reduce_range != 0, &sc, &zp);
-      const float scf = static_cast<float>(sc);
-      s_scale = scf;
-      s_inv = 1.0f / scf;  // IEEE division, as the separate quantize kernels
-      s_zp = static_cast<float>(zp);
-    }
-    resident_barrier();
-    const float inv = s_inv, zp_f = s_zp;
-#pragma unroll
-    for (int u = 0; u < HELD; ++u) {
-      const int e = t + u * kThreads;
-      if (e < total4) {
-        const int row = e / k4, c4 = e - row * k4;
-        const v4f v = held[u];
-        uint32_t q = 0;
-        const float f[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float r = __builtin_rintf(__builtin_fmaf(f[j], inv, zp_f));
-          r = fminf(fmaxf(r, 0.f), 255.f);
-          q |= static_cast<uint32_t>(static_cast<int>(r)) << (8 * j);
-        }
-        // bytes 4 c4 .. 4 c4 + 3 of the row: k-block c4 / 16, chunk (c4 / 4) % 4, byte 4 (c4 % 4) of the chunk
-        *reinterpret_cast<uint32_t*>(&s_x[((c4 >> 2) * 16 + row) * 16 + (c4 & 3) * 4]) = q ^ 0x80808080u;
-      }
-    }
-    xq = XQuant{s_scale, 128 - static_cast<int>(zp_f)};
+    for (int j = kFirst; j < D; ++j)
+      if (j < Q) wf[j] = next_weights();
   } else {
     const int xor_word = static_cast<int>(a.x_xor);
     const v4i xmask = {xor_word, xor_word, xor_word, xor_word};

@@ -4,6 +4,7 @@
 #include <limits>
 
 #include "common.h"
+#include "dynamic_rows.h"
 #include "host_report.h"
 #include "qparams.h"
 #include "stores_through.h"
@@ -40,33 +41,6 @@ struct HeldRange {
   int polls;  // of the words, before a block sees to what is missing itself
 };
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_float(float v) {  // (lanes without a source keep their own value)
-  const int i = __builtin_bit_cast(int, v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
-}
-template <int CTRL>
-__device__ __forceinline__ void minmax_step(float& mn, float& mx) {
-  mn = fminf(mn, dpp_float<CTRL>(mn));
-  mx = fmaxf(mx, dpp_float<CTRL>(mx));
-}
-// Minimum and maximum of each 16 lanes in the last of them (row_shr 1, 2, 4, 8) ...
-__device__ __forceinline__ void row_minmax(float& mn, float& mx) {
-  minmax_step<0x111>(mn, mx);
-  minmax_step<0x112>(mn, mx);
-  minmax_step<0x114>(mn, mx);
-  minmax_step<0x118>(mn, mx);
-}
-// ... and of the wave in its last lane (row_bcast 15, 31).
-__device__ __forceinline__ void wave_minmax_last(float& mn, float& mx) {
-  row_minmax(mn, mx);
-  minmax_step<0x142>(mn, mx);
-  minmax_step<0x143>(mn, mx);
-}
-__device__ __forceinline__ float lane_float(float v, int lane) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-
 // `total` words of four codes, H + more of them for each thread.  Dense (not ROWS): x on the 16-byte grid, `tail` values
 // (below four) behind the last word.  ROWS: rows of K >= 4 values at any 4-byte alignment -> rows of pitch4 words; the codes
 // behind a row's end are whatever its last values give.  sign_flip 0x80808080 for signed codes, which FUSED does not have
@@ -82,9 +56,6 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
   __shared__ int s_missing;
   const int t = threadIdx.x, own = static_cast<int>(blockIdx.x), blocks = static_cast<int>(gridDim.x);
   const int step = blocks * kHeldThreads;
-  struct __attribute__((packed, aligned(4))) Four {
-    v4f v;
-  };
   // a thread's words: its first, then one every `step`
   struct Place {
     int i, row, c4;
@@ -114,14 +85,10 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     if (ROWS) {
       const bool in = p.i < total;
       const int c = in ? 4 * p.c4 : 0;
-      return reinterpret_cast<const Four*>(x + static_cast<int64_t>(in ? p.row : 0) * K + (c + 4 <= K ? c : K - 4))->v;
+      return reinterpret_cast<const FourFloats*>(x + static_cast<int64_t>(in ? p.row : 0) * K + (c + 4 <= K ? c : K - 4))->v;
     }
     const v4f* src = reinterpret_cast<const v4f*>(x) + (p.i < total ? p.i : total - 1);
     return H >= kHeldStream ? __builtin_nontemporal_load(src) : *src;
-  };
-  const auto take = [](const v4f& v, float& mn, float& mx) {
-    mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
-    mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
   };
   const auto take_tail = [&](int block, float& mn, float& mx) {
     if (!ROWS && block == 0 && t < tail) {
@@ -168,7 +135,7 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
         advance(p);
       }
 #pragma unroll
-      for (int j = 0; j < kAhead; ++j) take(v[j], mn, mx);
+      for (int j = 0; j < kAhead; ++j) take_four(v[j], mn, mx);
     }
   }
   v4f held[H];
@@ -178,7 +145,7 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     advance(at);
   }
 #pragma unroll
-  for (int u = 0; u < H; ++u) take(held[u], mn, mx);
+  for (int u = 0; u < H; ++u) take_four(held[u], mn, mx);
   take_tail(own, mn, mx);
   publish(own, mn, mx, parts == nullptr ? nullptr : parts + own);
 
@@ -252,7 +219,7 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     Place p = place(missing);
 #pragma unroll 1
     for (int u = 0; u < H + more; ++u) {
-      take(load(p), a, b);
+      take_four(load(p), a, b);
       advance(p);
     }
     take_tail(missing, a, b);
