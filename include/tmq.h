@@ -296,6 +296,9 @@ int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * vector kernels run them.  Without it such products fall back to a byte-wise
  * kernel, a hundred times slower; up to 16 rows of 16 and more bytes need none. */
 int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid);
+/* 1: rows off the grid need no copy for this size, the call is faster without the
+ * room for one (which it uses where tmq_linear_scratch_bytes names it).  0: see there. */
+int tmq_linear_rows_in_place(int64_t M, int64_t N, int64_t K);
 /* The split behind that figure: *splits runs of *stages k-stages (64 bytes of K
  * each), the last run taking everything that is left; *splits == 1: no split.
  * Pure host arithmetic, no GPU call. */

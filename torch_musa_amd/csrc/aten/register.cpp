@@ -104,6 +104,7 @@ void check_status(int status, const char* what) {
 // the descriptor, kept alive by the returned tensor until the call is queued.
 at::Tensor attach_linear_workspace(tmq_linear_desc& d, const at::Tensor& like) {
   const bool on_grid = d.ldx % 16 == 0 && reinterpret_cast<uintptr_t>(d.x) % 16 == 0;
+  if (!(on_grid && d.K % 16 == 0) && tmq_linear_rows_in_place(d.M, d.N, d.K) != 0) return at::Tensor();
   const int64_t bytes = tmq_linear_scratch_bytes(d.M, d.N, d.K, on_grid);
   if (bytes <= 0) return at::Tensor();
   at::Tensor ws = empty_bytes(bytes, like);

@@ -18,11 +18,16 @@
 //
 // Measured (us, weights from memory, the best other kernel | this one): M = 56, N = 1920, K = 4752 12.8 | 8.4; M = 63, N = 107,
 // K = 5376 11.5 | 7.4; M = 407, N = 154, K = 6080 10.9 (its former self) | 8.2; M = 364, N = 320, K = 11968 24.7 | 14.8 before.
+// RAGGED: rows of any K >= 16, pitch and address are read where they lie, by requests of any alignment; a row's last chunk as its
+// last 16 bytes, shifted to their place.  On a round of tiles that beats staging them for 64 x 64 tiles, whose chain of stages is
+// as long as K, and the copy onto the grid with its launch (us, those | these: 39 x 1098 -> 64 6.1 | 4.3, 137 x 1246 -> 203 6.9 | 4.7,
+// 244 x 2680 -> 266 9.5 | 5.0, 1523 x 2982 -> 72 10.7 | 6.2, 542 x 745 -> 945 6.0 | 4.7, 50 x 270 -> 88 4.0 | 3.5, 71 x 7470 -> 512
+// 11.1 | 10.6, 1073 x 5823 -> 320 18.2 | 13.1).  Beyond one round the larger tiles are ahead: 517 x 2051 -> 1000 8.9 | 10.5.
+//
 // Tried: 64 x 64 tiles the same way (256 registers; 273 x 5760 -> 2432 14.0 against 13.9 for lone 64 x 64 tiles in a ring of six
 // stages, 482 x 5232 -> 768 14.4); K split over two to sixteen blocks as well, the last to arrive adding the others' partial sums
-// (51 x 8384 -> 256 8.5 -> 7.9 with three, otherwise level or behind: the sums' way through memory costs 2.5 us); rows off
-// the 16-byte grid read where they lie (M = 1633, N = 163, K = 5834 20.9 against 17.2 for the tiles that stage them), which are
-// copied onto the grid instead; tiles of four waves, two blocks a CU, where there are more than 256 (1445 x 1472 -> 288 6.9
+// (51 x 8384 -> 256 8.5 -> 7.9 with three, otherwise level or behind: the sums' way through memory costs 2.5 us); off the
+// grid 517 x 1000 -> 2051 11.0 against 7.8); tiles of four waves, two blocks a CU, where there are more than 256 (1445 x 1472 -> 288 6.9
 // against 5.9 for 32 x 64 tiles of eight).
 #pragma once
 
@@ -42,7 +47,7 @@ __device__ __forceinline__ GemmArgs epilogue_args(const GemmArgs& a) {
 }
 
 // Tiles of 32 rows x 32 CT channels, PB bytes of K a piece.
-template <int MODE, int CT>
+template <int MODE, int CT, bool RAGGED = false>
 __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(GemmArgs a, XLinear xs) {
   constexpr int BM = 32, BN = 32 * CT, PB = 256 / CT, WAVES = kWloopWaves;
   constexpr int kLPR = PB / 16;              // 16-byte chunks (lanes) of a row in a piece
@@ -94,9 +99,15 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   const auto request = [&](int p, Piece& pc) {
     __builtin_amdgcn_sched_barrier(0);
     const int c = p * kLPR + slot;
-    const uint32_t off = static_cast<uint32_t>(c < KC ? c : KC - 1) * 16u;
+    if constexpr (RAGGED) {
+      const uint32_t off = static_cast<uint32_t>(16 * c + 16 <= K ? 16 * c : K - 16);
 #pragma unroll
-    for (int i = 0; i < kNX; ++i) pc.x[i] = ld16(xtile + (xrow[i] + off));
+      for (int i = 0; i < kNX; ++i) pc.x[i] = ld16_any(xtile + (xrow[i] + off));
+    } else {
+      const uint32_t off = static_cast<uint32_t>(c < KC ? c : KC - 1) * 16u;
+#pragma unroll
+      for (int i = 0; i < kNX; ++i) pc.x[i] = ld16(xtile + (xrow[i] + off));
+    }
 #pragma unroll
     for (int j = 0; j < kSteps; ++j) {
       const int kc = p * kLPR + 2 * j + half;
@@ -127,11 +138,16 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   const int flip = static_cast<int>(a.x_xor);
   const auto multiply = [&](int p, Piece& pc) {
     const int c = p * kLPR + slot;
+    const int keep = (RAGGED ? 16 * c < K : c < KC) ? -1 : 0;
+    if (RAGGED && p == pieces - 1) {         // (a row's last chunk was read where its last 16 bytes are)
+      const int past = 16 * c - (K - 16);
+#pragma unroll
+      for (int i = 0; i < kNX; ++i) pc.x[i] = shift_down_bytes(pc.x[i], past > 0 && past < 16 ? past : 0);
+    }
 #pragma unroll
     for (int i = 0; i < kNX; ++i) {
       const int r = i * kRPL + lane / kLPR;
       v4i v = pc.x[i];
-      const int keep = c < KC ? -1 : 0;
       v = (v ^ v4i{flip, flip, flip, flip}) & v4i{keep, keep, keep, keep};
       *reinterpret_cast<v4i*>(mine + r * PB + ((slot ^ swizzle(r)) << 4)) = v;
     }

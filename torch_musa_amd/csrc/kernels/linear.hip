@@ -590,6 +590,14 @@ int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream
   else enqueue(gemm_i8_wloop_kernel<MODE, 1>, grid, block, 0, s, a, xs);
   return launch_status();
 }
+// ... and for rows off the 16-byte grid.
+template <int MODE>
+int launch_gemm_wloop_ragged(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(a.N, wide ? 64 : 32)), static_cast<unsigned>(ceil_div(a.M, 32)));
+  if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2, true>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
+  else enqueue(gemm_i8_wloop_kernel<MODE, 1, true>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
+  return launch_status();
+}
 
 // The same for K up to 4096 (cfg 25, 26), two tiles of 32 channels side by side in a block where one round holds those only
 // (us, weights from memory, four waves a tile and two blocks a CU | pairs: 71 x 1120 -> 3200 5.6 | 4.6, 1445 x 1472 -> 288 7.4 |
@@ -1404,7 +1412,19 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
   return c;
 }
 
-// More than 16 rows off the 16-byte grid: 64 x 64 tiles that read the rows where they lie, or a copy
+// More than 16 rows off the 16-byte grid, one round of tiles of 32 rows: eight waves a tile that walk K in pieces and read the rows
+// where they lie (gemm_i8_wloop.h has both sides).  Tiles of 64 channels, whose pieces are half as long, where not every wave would
+// have one otherwise (us, 32 | 64 channels: 24 x 276 -> 65 3.8 | 3.6, 1279 x 378 -> 64 4.0 | 3.8; 523 x 360 -> 322 level; 205 x 684
+// -> 640 4.0 | 4.1) and where 32 do not fit a round.  Two stages and less stay with the 64 x 64 tiles (those | these: 172 x 84 -> 64
+// 3.3 | 3.6, 1897 x 76 -> 128 3.5 | 3.7, 136 x 88 -> 1043 3.7 | 3.9; 97 x 152 -> 64 3.6 | 3.4, 26 x 132 -> 8064 4.1 | 3.7).  Returns the
+// channels per tile, 0: not such a shape.
+constexpr int64_t kWloopRaggedMinK = 2 * kBK, kWloopRaggedShortK = 512;
+int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
+  if (M <= kDecodeRowsAuto || K <= kWloopRaggedMinK || K > kWloopMaxK || ceil_div(M, 32) * ceil_div(N, 64) > 256) return 0;
+  return K > kWloopRaggedShortK && ceil_div(M, 32) * ceil_div(N, 32) <= 256 ? 32 : 64;
+}
+
+// More than that: 64 x 64 tiles that read the rows where they lie, or a copy
 // onto the grid and the padded shape's own kernel.  The copy is a launch (2.2 us and a scratch
 // allocation); the larger tiles it opens earn that back from 512 tiles on, later where K is short
 // (us, direct | copy, weights in the caches: M = 517: K = 1000, N = 2051 8.1 | 9.8, K = 2051, N = 1000 9.3 | 10.7; K = 3907,
@@ -1412,11 +1432,7 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
 // 19.4 | 18.6; K = 1480, N = 5664, M = 611 (890) 18.9 | 14.7; K = 700, N = 2000, M = 2048 (1024) 11.3 | 12.6; K = 741,
 // N = 3952, M = 1560 (1550) 21.4 | 14.8; K = 500, N = 2000, M = 3000 (1504) 12.8 | 12.3; K = 100, N = 1000, M = 8000 (2000)
 // 10.4 | 12.8; K = 120, N = 8000, M = 4096 (8000) 26.3 | 22.1).  Few outputs leave the copy behind further on (K = 1204,
-// N = 646, M = 2983, 517 tiles, 11.3 | 14.9).  Few rows against K beyond 1200 have kernels on the grid that make up for it
-// on the device (M = 67, N = 2383, K = 2901 11.1 | 9.0, M = 40, N = 1308, K = 1413 7.7 | 6.8), but not on the host, which
-// takes longer over the copy's launch and memory than the device gains: two layers, quantize and dequantize, M = 67,
-// 2901 -> 2383 -> 1001 25.1 | 25.0, M = 40, 1413 -> 1308 -> 1413 18.7 | 25.4, M = 109, 3298 -> 74 -> 3298 20.3 | 24.5.  Rows few
-// enough for the streaming kernel keep it (M = 40, K = 4100, N = 512: 10.5).
+// N = 646, M = 2983, 517 tiles, 11.3 | 14.9).
 bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
   if (K < 16 || K > 0x7fffff00) return false;
   if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return false;
@@ -1425,10 +1441,10 @@ bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
 }
 
 // ... and where the copy comes first, if there is room for it: K so long that the padded shape's kernel earns it back (two
-// layers, quantize and dequantize as a program calls them, direct | copy, us).  Waves that walk their shares of K: 840 x 8155
-// -> 192 39.0 | 33.8, 59 x 6040 -> 384 26.8 | 21.5, 200 x 5001 -> 1000 29.7 | 25.2, 1237 x 6284 -> 212 36.7 | 34.1, 1633 x
-// 5834 -> 163 35.6 | 35.4.  64 x 128 tiles in a ring: 600 x 6001 -> 2000 45.3 | 34.6, 700 x 3001 -> 1500 30.8 | 26.8, 1500 x
-// 2501 -> 900 31.4 | 29.7; 1000 x 2051 -> 2051 28.5 | 29.3, 2048 x 1310 -> 1024 25.6 | 26.9.
+// layers, quantize and dequantize as a program calls them, direct | copy, us).  64 x 128 tiles in a ring: 600 x 6001 -> 2000
+// 45.3 | 34.6, 700 x 3001 -> 1500 30.8 | 26.8, 1500 x 2501 -> 900 31.4 | 29.7; 1000 x 2051 -> 2051 28.5 | 29.3, 2048 x 1310 ->
+// 1024 25.6 | 26.9.  One round of tiles of 32 rows against K > 4096 reads the rows in place where there is no room (wloop_ragged_tile),
+// which is faster still and needs none; a caller that gives the room tmq_linear_scratch_bytes names has them copied.
 bool ragged_copy_first(int64_t M, int64_t N, int64_t K) {
   const int64_t pitch = regrid_pitch(K);
   return wloop_tile(M, N, pitch) != 0 || (K >= 2304 && oblong_ring_first(M, N, pitch, pitch));
@@ -1457,7 +1473,11 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
       return launch_linear_decode_ragged<MODE>(a, xs, s);
     const int64_t room = regrid_bytes(a.M, a.K);
     const bool copy_ok = regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room;
-    if (ragged_tiles_preferred(a.M, a.N, a.K) && a.w_kchunks == packed_kchunks(a.K) &&
+    const bool zero_padded = a.w_kchunks == packed_kchunks(a.K);
+    if (const int tile = wloop_ragged_tile(a.M, a.N, a.K); tile != 0 && zero_padded && xs.ldx <= (int64_t{1} << 23) &&
+        a.N + a.n_off < (int64_t{1} << 29) && !(copy_ok && wloop_tile(a.M, a.N, regrid_pitch(a.K)) != 0))
+      return launch_gemm_wloop_ragged<MODE>(a, xs, tile == 64, s);
+    if (ragged_tiles_preferred(a.M, a.N, a.K) && zero_padded &&
         !(copy_ok && ragged_copy_first(a.M, a.N, a.K))) {
       const XLinearRagged rows{xs.x, xs.ldx};
       return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
@@ -1616,8 +1636,13 @@ TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int
   // (the plan of a split along K is there for pinned kernels where the automatic choice is another one)
   const int64_t split = wloop_tile(M, N, regrid_pitch(K)) != 0 ? 0 : tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
   if (K % 16 == 0 && on_grid) return split;
+  if (wloop_ragged_tile(M, N, K) != 0 && wloop_tile(M, N, regrid_pitch(K)) == 0) return 0;
   if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_tiles_preferred(M, N, K) && !ragged_copy_first(M, N, K)) || !regrid_limits_ok(M, K)) return 0;
   return regrid_bytes(M, K) + split;
+}
+
+TMQ_EXPORT int tmq_linear_rows_in_place(int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && wloop_ragged_tile(M, N, K) != 0 ? 1 : 0;
 }
 
 TMQ_EXPORT int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int32_t* stages) {
