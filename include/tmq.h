@@ -478,6 +478,9 @@ int tmq_conv2d(const tmq_conv2d_desc* desc, tmq_stream_t stream);
  * reference: muDNN allocates its own scratch through the InternalMemAlloc
  * callback (torch_musa/csrc/aten/utils/Utils.cpp:79-153). */
 int64_t tmq_conv2d_workspace_bytes(const tmq_conv2d_geom* g);
+/* What the automatic choice makes use of: the same, but 0 where a layer of few
+ * pixels has a kernel that needs no patch rows. */
+int64_t tmq_conv2d_scratch_bytes(const tmq_conv2d_geom* g);
 /* Zero-point-corrected accumulators, [B,OH,OW,OC] int32:
  * acc = sum over in-image taps of (x - x_zp) * w. */
 int tmq_conv2d_acc32(const tmq_conv2d_desc* desc, int32_t* acc, tmq_stream_t stream);

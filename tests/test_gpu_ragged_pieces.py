@@ -1,7 +1,5 @@
 """quantized::linear on one round of tiles of 32 rows whose activation rows lie off the 16-byte grid: tile and piece edges and a
 last chunk of 1 to 15 bytes, rows of any pitch and address with the storage's ends at the first and last byte, against the oracle."""
-import ctypes
-
 import numpy as np
 import pytest
 import torch
@@ -12,7 +10,7 @@ from test_gpu_linear import _check, _run, _tile_case, cabi  # noqa: F401
 
 
 def _in_place(cabi, m, n, k):
-    return cabi.lib().tmq_linear_rows_in_place(*(ctypes.c_int64(v) for v in (m, n, k)))
+    return cabi.lib().tmq_linear_rows_in_place(m, n, k)
 
 
 @pytest.mark.gpu

@@ -26,7 +26,7 @@ DECLARED_SYMBOLS = [
     "tmq_linear_packed_kchunks", "tmq_linear_packed_bytes", "tmq_linear_prepack",
     "tmq_linear_unpack", "tmq_linear", "tmq_linear_workspace_bytes", "tmq_linear_split_plan", "tmq_linear_kernel_choice", "tmq_linear_static_workspace", "tmq_linear_acc32", "tmq_linear_f32", "tmq_linear_dynamic_small", "tmq_linear_dynamic_small_takes", "tmq_quantize_per_tensor_dynamic_dev",
     "tmq_quantize_per_tensor_dynamic_report", "tmq_quantize_per_tensor_dynamic_parts", "tmq_quantize_rows_dynamic_dev", "tmq_quantize_dynamic_exchange", "tmq_linear_scratch_bytes", "tmq_linear_rows_in_place", "tmq_linear_float", "tmq_per_channel",
-    "tmq_conv2d_packed_bytes", "tmq_conv2d_prepack", "tmq_conv2d_out_hw", "tmq_conv2d_workspace_bytes",
+    "tmq_conv2d_packed_bytes", "tmq_conv2d_prepack", "tmq_conv2d_out_hw", "tmq_conv2d_workspace_bytes", "tmq_conv2d_scratch_bytes",
     "tmq_conv2d", "tmq_conv2d_acc32", "tmq_conv2d_fused",
     "tmq_qadd", "tmq_qrelu", "tmq_qcat_rows", "tmq_planes_to_pixels", "tmq_qmaxpool2d", "tmq_qadaptive_avgpool2d", "tmq_qunary",
 ]
@@ -119,6 +119,9 @@ def lib() -> C.CDLL:
         l.tmq_conv2d_packed_bytes.argtypes = [C.POINTER(Conv2dGeom)]
         l.tmq_conv2d_workspace_bytes.restype = C.c_int64
         l.tmq_conv2d_workspace_bytes.argtypes = [C.POINTER(Conv2dGeom)]
+        l.tmq_conv2d_scratch_bytes.restype = C.c_int64
+        l.tmq_conv2d_scratch_bytes.argtypes = [C.POINTER(Conv2dGeom)]
+        l.tmq_linear_rows_in_place.argtypes = [C.c_int64, C.c_int64, C.c_int64]
         v = C.c_void_p
         l.tmq_quantize_per_tensor.argtypes = [v, v, C.c_int64, C.c_double, C.c_int64, C.c_int, v]
         l.tmq_dequantize_per_tensor.argtypes = [v, v, C.c_int64, C.c_double, C.c_int64, C.c_int, v]

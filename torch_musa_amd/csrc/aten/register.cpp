@@ -833,7 +833,7 @@ struct PackedConvWeightTmq final : public ConvPackedParamsBase<2> {
     // scratch for the layers that run on their patch rows or on a channel-padded copy of the
     // input (from the caching allocator: safe under stream capture, freed for reuse in stream order)
     at::Tensor workspace;
-    const int64_t ws_bytes = tmq_conv2d_workspace_bytes(&g);
+    const int64_t ws_bytes = tmq_conv2d_scratch_bytes(&g);
     if (ws_bytes > 0) {
       workspace = empty_bytes(ws_bytes, x);
       d.workspace = workspace.data_ptr();
@@ -1601,7 +1601,7 @@ at::Tensor qconv_plain(const at::Tensor& act, double act_scale, int64_t act_zero
     TORCH_CHECK(accum->sizes() == c10::IntArrayRef(out_shape) && accum->device() == act.device(), what,
                 ": accum must have the output's shape ", c10::IntArrayRef(out_shape), " and device");
   at::Tensor workspace;  // (as in PackedConvWeightTmq::apply)
-  const int64_t ws_bytes = tmq_conv2d_workspace_bytes(&g);
+  const int64_t ws_bytes = tmq_conv2d_scratch_bytes(&g);
   if (ws_bytes > 0) {
     workspace = at::empty({ws_bytes}, act.options().dtype(at::kByte));
     d.workspace = workspace.data_ptr();

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "conv_image.h"
+#include "gemm_i8_wloop.h"
 #include "conv_runs.h"
 #include "conv_depthwise.h"
 #include "conv_tile.h"
@@ -1066,6 +1067,66 @@ int run_as_linear(const tmq_conv2d_desc* d, int64_t rows, int64_t OC, int64_t K,
   return tmq_linear(&l, reinterpret_cast<tmq_stream_t>(stream));
 }
 
+// Operands of the implicit GEMM (of a layer's first group).
+void conv_gemm_operands(const tmq_conv2d_desc* d, const ConvShape& s, const PostOps& po, float zp_f, float lo_f, float hi_f,
+                        void* out, GemmArgs* args, XConvTable* source) {
+  XConvTable& xs = *source;
+  xs.x = static_cast<const uint8_t*>(d->x);
+  xs.H = static_cast<int>(s.H); xs.W = static_cast<int>(s.W); xs.IC = static_cast<int>(s.IC);
+  xs.OH = static_cast<int>(s.OH); xs.OW = static_cast<int>(s.OW);
+  xs.KW = static_cast<int>(s.KW); xs.icb = static_cast<int>(s.ICgp / 16);
+  xs.stride_h = static_cast<int>(s.sh); xs.stride_w = static_cast<int>(s.sw);
+  xs.pad_h = static_cast<int>(s.ph); xs.pad_w = static_cast<int>(s.pw);
+  xs.dil_h = static_cast<int>(s.dh); xs.dil_w = static_cast<int>(s.dw);
+  xs.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
+  xs.KH = static_cast<int>(s.KH);
+  xs.chunks = static_cast<int>(s.Kp / 16);
+  xs.step_w = static_cast<int>(s.dw * s.IC - 16 * (s.ICgp / 16));
+  xs.step_h = static_cast<int>(s.dh * s.W * s.IC - s.KW * s.dw * s.IC);
+
+  GemmArgs& a = *args;
+  a.M = s.B * s.OH * s.OW;
+  a.N = s.OCg;
+  a.K = s.Kp;
+  a.w_packed = static_cast<const uint8_t*>(d->w_packed);
+  a.w_kchunks = s.KC;
+  a.colsum = d->w_colsum;
+  a.w_scales = d->w_scales;
+  a.bias = d->bias;
+  a.w_scale_stride = d->w_per_channel ? 1 : 0;
+  a.x_xor = d->x_signed ? 0u : 0x80808080u;
+  a.acc_coef = (d->x_signed ? 0 : 128) - d->x_zero_point;
+  a.x_scale = d->x_scale;
+  a.out_scale = d->out_scale;
+  a.zp_f = zp_f; a.lo_f = lo_f; a.hi_f = hi_f;
+  a.y = out;
+  a.ldy = s.OC;
+  a.post = po;
+}
+
+template <int MODE>
+int launch_conv_waves(const GemmArgs& a, const XConvTable& xs, int tile, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(a.N, tile)), static_cast<unsigned>(ceil_div(a.M, 32)));
+  if (tile == 32) enqueue(gemm_i8_wloop_kernel<MODE, 1, XConvTable>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
+  else enqueue(gemm_i8_wloop_kernel<MODE, 2, XConvTable>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
+  return launch_status();
+}
+// Layers of one group whose pixels and channels make one round of tiles of 32 rows: their eight waves walk K in pieces, the windows'
+// chunks gathered straight into registers (gemm_i8_wloop.h).  Everything else that takes such a layer has a chain as long as K on a
+// few blocks, or a copy in front: us, the best before | these, 3 x 3: 512 -> 398 on 8 x 9 x 10 15.2 | 9.6, 256 -> 256 on one 28 x 28
+// 9.4 | 6.0, 512 -> 512 on one 14 x 14 (patch rows) 14.6 | 7.0, 192 -> 192 on 2 x 20 x 67 8.7 | 7.0, 112 -> 48 with SiLU on 8 x 10 x 19 (halo
+// tiles) 6.9 | 4.8; 1 x 1 with SiLU, 624 -> 304 on 2 x 24 x 23 6.5 | 5.5; 960 -> 187 with SiLU on 3 x 7 x 34 22.7 | 10.4.  Of 240 drawn
+// layers (K = 144 ... 23040) 32 channels a tile take 0.40 to 0.98 of the time where they fit a round, but for K short of 576 without
+// a residual or SiLU (0.96 to 1.13, halo tiles and patches in registers); 64 channels, where only those fit, 0.56 to 0.99 from K = 720
+// (400 with a residual or SiLU) on, below 0.86 to 1.2.  A second round is behind: 1.0 to 1.9.
+// Returns the channels per tile, 0: not such a layer.
+int conv_waves_tile(const ConvShape& s, const tmq_conv2d_geom& g, bool post) {
+  if (g.groups != 1 || s.groups != 1 || s.ICg % 16 != 0 || !conv_table_takes(s)) return 0;
+  const int64_t rows = ceil_div(s.B * s.OH * s.OW, 32);
+  if (rows * ceil_div(s.OC, 32) <= 256) return post || s.Kp >= 576 ? 32 : 0;
+  return rows * ceil_div(s.OC, 64) <= 256 && s.Kp >= (post ? 400 : 720) ? 64 : 0;
+}
+
 template <int MODE>
 int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, hipStream_t stream) {
   ConvShape s;
@@ -1126,6 +1187,15 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     if (forced == 5 && !pointwise) return TMQ_ERR_UNSUPPORTED;
     if (forced == 5 || (forced < 0 && pointwise && !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, false)))) {
       return run_as_linear(d, rows, s.OC, s.IC, d->x, relu, out, stream);
+    }
+  }
+  if constexpr (MODE != kOutAcc32) {
+    const int tile = forced < 0 && aligned(d->x, 16) ? conv_waves_tile(s, d->geom, po.any()) : 0;
+    if (tile != 0 && !(pointwise_rows_ok(d->geom, s) && pointwise_rows_first(s, po.any()))) {
+      GemmArgs a{};
+      XConvTable xs{};
+      conv_gemm_operands(d, s, po, zp_f, lo_f, hi_f, out, &a, &xs);
+      return launch_conv_waves<MODE>(a, xs, tile, stream);
     }
   }
   // Few output pixels against a long K and a weight slice the halo tiles cannot hold: with a
@@ -1284,38 +1354,10 @@ int run_conv(const tmq_conv2d_desc* d, const tmq_conv2d_post* post, void* out, h
     return launch_conv_tiles<MODE>(s, plan, t, stream);
   }
 
-  XConvTable xs{};
-  xs.x = static_cast<const uint8_t*>(d->x);
-  xs.H = static_cast<int>(s.H); xs.W = static_cast<int>(s.W); xs.IC = static_cast<int>(s.IC);
-  xs.OH = static_cast<int>(s.OH); xs.OW = static_cast<int>(s.OW);
-  xs.KW = static_cast<int>(s.KW); xs.icb = static_cast<int>(s.ICgp / 16);
-  xs.stride_h = static_cast<int>(s.sh); xs.stride_w = static_cast<int>(s.sw);
-  xs.pad_h = static_cast<int>(s.ph); xs.pad_w = static_cast<int>(s.pw);
-  xs.dil_h = static_cast<int>(s.dh); xs.dil_w = static_cast<int>(s.dw);
-  xs.pad_word = 0x01010101u * static_cast<uint32_t>(static_cast<uint8_t>(d->x_zero_point));
-  xs.KH = static_cast<int>(s.KH);
-  xs.chunks = static_cast<int>(s.Kp / 16);
-  const bool table = conv_table_takes(s);
-  xs.step_w = static_cast<int>(s.dw * s.IC - 16 * (s.ICgp / 16));
-  xs.step_h = static_cast<int>(s.dh * s.W * s.IC - s.KW * s.dw * s.IC);
-
   GemmArgs a{};
-  a.M = rows;
-  a.N = s.OCg;
-  a.K = s.Kp;
-  a.w_kchunks = s.KC;
-  a.colsum = d->w_colsum;
-  a.w_scales = d->w_scales;
-  a.bias = d->bias;
-  a.w_scale_stride = d->w_per_channel ? 1 : 0;
-  a.x_xor = d->x_signed ? 0u : 0x80808080u;
-  a.acc_coef = (d->x_signed ? 0 : 128) - d->x_zero_point;
-  a.x_scale = d->x_scale;
-  a.out_scale = d->out_scale;
-  a.zp_f = zp_f; a.lo_f = lo_f; a.hi_f = hi_f;
-  a.y = out;
-  a.ldy = s.OC;
-  a.post = po;
+  XConvTable xs{};
+  conv_gemm_operands(d, s, po, zp_f, lo_f, hi_f, out, &a, &xs);
+  const bool table = conv_table_takes(s);
   const int64_t stages = ceil_div(s.Kp, kBK);
   ConvGemmTile tile = table ? conv_gemm_tile(rows, s.OCg, stages, po.any()) : conv_walk_tile(rows, s.OCg, stages);
   if (forced == 2 && !pinned_conv_tile(d->tile_rows, d->tile_cols, stages, &tile)) return TMQ_ERR_UNSUPPORTED;
@@ -1347,6 +1389,11 @@ TMQ_EXPORT int64_t tmq_conv2d_workspace_bytes(const tmq_conv2d_geom* g) {
   const int64_t need = patch_rows_bytes(*g, s, false);
   if (need > 0 && !(s.ICg % 16 == 0 && plan_tiles(s, false, 0, 0, &tp))) return need;
   return padded_input_bytes(*g, s, false);
+}
+
+TMQ_EXPORT int64_t tmq_conv2d_scratch_bytes(const tmq_conv2d_geom* g) {
+  ConvShape s;
+  return make_shape(g, &s) == TMQ_OK && conv_waves_tile(s, *g, false) != 0 ? 0 : tmq_conv2d_workspace_bytes(g);
 }
 
 TMQ_EXPORT int tmq_conv2d_out_hw(const tmq_conv2d_geom* g, int64_t* OH, int64_t* OW) {

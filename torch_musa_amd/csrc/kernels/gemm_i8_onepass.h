@@ -297,7 +297,7 @@ __global__ __launch_bounds__(BN * 4) void gemm_i8_onepass_kernel(GemmArgs a, XLi
 }
 
 // (one thread's share of ksplit_finish: row idx / (BN / 4), channels 4 (idx % (BN / 4)) ... + 3)
-template <int MODE, int BN, int WAVES>
+template <int MODE, int BN, int WAVES, bool POST = false>
 __device__ __forceinline__ void ksplit_finish_four(const GemmArgs& a, const uint8_t* red, int red_stride,
                                                    const int (*s_raw)[kWave], const XQuant& xq, int64_t m0, int64_t n0,
                                                    int idx) {
@@ -336,8 +336,15 @@ __device__ __forceinline__ void ksplit_finish_four(const GemmArgs& a, const uint
     const float bmul = bias_mul(a.w_scale_stride == 0, xq.scale * __int_as_float(s_raw[1][0]));
     const bool plain_u8 = MODE == kOutU8 && a.lo_f <= 0.f && a.hi_f >= 255.f;
     // unsigned output without ReLU: the saturating conversion is the clamp
-    const uint32_t q4 = plain_u8 ? requant4<MODE, false>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f)
-                                 : requant4<MODE, true>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
+    uint32_t q4;
+    if (POST && a.post.any()) {
+      const int nvalid = a.N - n < 4 ? static_cast<int>(a.N - n) : 4;
+      const uint32_t accw = a.post.accum != nullptr ? load_accum4(a.post, m * a.ldy + a.n_off + n, nvalid) : 0u;
+      q4 = requant4_post<MODE>(raw, bdiv, bmul, mult, a.post, accw, a.zp_f, a.lo_f, a.hi_f);
+    } else {
+      q4 = plain_u8 ? requant4<MODE, false>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f)
+                    : requant4<MODE, true>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
+    }
     uint8_t* const dst = static_cast<uint8_t*>(a.y) + a.n_off + m * a.ldy + n;
     if ((reinterpret_cast<uintptr_t>(dst) & 3) == 0 && n + 4 <= a.N) {
       *reinterpret_cast<uint32_t*>(dst) = q4;

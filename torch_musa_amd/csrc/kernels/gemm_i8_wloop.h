@@ -23,6 +23,10 @@
 // as long as K, and the copy onto the grid with its launch (us, those | these: 39 x 1098 -> 64 6.1 | 4.3, 137 x 1246 -> 203 6.9 | 4.7,
 // 244 x 2680 -> 266 9.5 | 5.0, 1523 x 2982 -> 72 10.7 | 6.2, 542 x 745 -> 945 6.0 | 4.7, 50 x 270 -> 88 4.0 | 3.5, 71 x 7470 -> 512
 // 11.1 | 10.6, 1073 x 5823 -> 320 18.2 | 13.1).  Beyond one round the larger tiles are ahead: 517 x 2051 -> 1000 8.9 | 10.5.
+// XConvTable: a convolution's windows.  One thread a row works out where its window lies and which taps are inside the image, two
+// divisions a piece give a lane its chunk's tap, and the zero point goes in for what is outside on the way into LDS: no table of
+// the k order, no barrier but the one behind the windows.  Pieces of 128 bytes here also for 32 channels a tile (with 256 the row
+// offsets and masks left 11 registers in memory).  conv_waves_tile (conv2d.hip) has what it is worth.
 //
 // Tried: 64 x 64 tiles the same way (256 registers; 273 x 5760 -> 2432 14.0 against 13.9 for lone 64 x 64 tiles in a ring of six
 // stages, 482 x 5232 -> 768 14.4); K split over two to sixteen blocks as well, the last to arrive adding the others' partial sums
@@ -47,9 +51,10 @@ __device__ __forceinline__ GemmArgs epilogue_args(const GemmArgs& a) {
 }
 
 // Tiles of 32 rows x 32 CT channels, PB bytes of K a piece.
-template <int MODE, int CT, bool RAGGED = false>
-__global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(GemmArgs a, XLinear xs) {
-  constexpr int BM = 32, BN = 32 * CT, PB = 256 / CT, WAVES = kWloopWaves;
+template <int MODE, int CT, class XSRC = XLinear>
+__global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(GemmArgs a, XSRC xs) {
+  constexpr bool kConv = std::is_same<XSRC, XConvTable>::value, RAGGED = std::is_same<XSRC, XLinearRagged>::value;
+  constexpr int BM = 32, BN = 32 * CT, PB = kConv ? 128 : 256 / CT, WAVES = kWloopWaves;
   constexpr int kLPR = PB / 16;              // 16-byte chunks (lanes) of a row in a piece
   constexpr int kRPL = kWave / kLPR;         // rows per request
   constexpr int kNX = BM / kRPL;             // activation requests of a piece
@@ -71,10 +76,32 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   // have at a piece's ends, are asked for together
   int p = wave_u, left = wave_u < pieces ? (pieces - wave_u + WAVES - 1) / WAVES : 0;
 
-  const uint8_t* const xtile = xs.x + m0 * xs.ldx;
+  const uint8_t* xtile;
   const int slot = lane % kLPR;
   uint32_t xrow[kNX];
-  {
+  uint64_t inside[kNX];                      // (convolutions) XLoader<XConvTable>
+  if constexpr (kConv) {
+    // the windows of the tile's rows, one thread each: offset of the corner from the tile's first image, taps inside the image
+    struct Window {
+      uint32_t off, unused;
+      uint64_t inside;
+    };
+    __shared__ Window s_window[BM];
+    const uint32_t image = static_cast<uint32_t>(m0) / static_cast<uint32_t>(xs.OH * xs.OW);
+    xtile = xs.x + static_cast<int64_t>(image) * xs.H * xs.W * xs.IC + xs.ic_off;
+    if (t < BM) {
+      XLoader<XConvTable> row;
+      row.init(xs, m0 + t, a.M);
+      s_window[t] = Window{static_cast<uint32_t>(row.img - xtile) + static_cast<uint32_t>(row.off0), 0, row.inside};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kNX; ++i) {
+      xrow[i] = s_window[i * kRPL + lane / kLPR].off;
+      inside[i] = s_window[i * kRPL + lane / kLPR].inside;
+    }
+  } else {
+    xtile = xs.x + m0 * xs.ldx;
     const int64_t m_last = a.M - 1 - m0;     // rows past M: clamped, never stored
 #pragma unroll
     for (int i = 0; i < kNX; ++i) {
@@ -94,12 +121,26 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   }
   struct Piece {
     v4i x[kNX], w[CT][kSteps];
+    uint32_t outside;                        // (convolutions) bit i: x[i] lies outside the image
   };
   // (chunks past K: bytes of the row, zeroed below)
   const auto request = [&](int p, Piece& pc) {
     __builtin_amdgcn_sched_barrier(0);
     const int c = p * kLPR + slot;
-    if constexpr (RAGGED) {
+    if constexpr (kConv) {
+      // (chunks past K: no tap)
+      const uint32_t tap = c < KC ? static_cast<uint32_t>(c) / static_cast<uint32_t>(xs.icb) : kConvMaxTaps;
+      const int kh = static_cast<int>(tap / static_cast<uint32_t>(xs.KW));
+      const uint32_t off = static_cast<uint32_t>(
+          (kh * xs.dil_h * xs.W + (static_cast<int>(tap) - kh * xs.KW) * xs.dil_w) * xs.IC + (c - static_cast<int>(tap) * xs.icb) * 16);
+      pc.outside = 0;
+#pragma unroll
+      for (int i = 0; i < kNX; ++i) {
+        const uint32_t in = static_cast<uint32_t>(inside[i] >> tap) & 1u;
+        pc.outside |= (in ^ 1u) << i;
+        pc.x[i] = ld16(xtile + ((xrow[i] + off) & (0u - in)));
+      }
+    } else if constexpr (RAGGED) {
       const uint32_t off = static_cast<uint32_t>(16 * c + 16 <= K ? 16 * c : K - 16);
 #pragma unroll
       for (int i = 0; i < kNX; ++i) pc.x[i] = ld16_any(xtile + (xrow[i] + off));
@@ -148,6 +189,10 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
     for (int i = 0; i < kNX; ++i) {
       const int r = i * kRPL + lane / kLPR;
       v4i v = pc.x[i];
+      if constexpr (kConv) {
+        const int pad = static_cast<int>(xs.pad_word);
+        if ((pc.outside >> i) & 1u) v = v4i{pad, pad, pad, pad};
+      }
       v = (v ^ v4i{flip, flip, flip, flip}) & v4i{keep, keep, keep, keep};
       *reinterpret_cast<v4i*>(mine + r * PB + ((slot ^ swizzle(r)) << 4)) = v;
     }
@@ -209,7 +254,7 @@ __global__ __launch_bounds__(kWloopWaves* kWave, 2) void gemm_i8_wloop_kernel(Ge
   __syncthreads();
 #pragma unroll
   for (int idx = t; idx < BM * BN / 4; idx += WAVES * kWave)
-    ksplit_finish_four<MODE, BN, WAVES>(e, &sX[0][0], kWaveLds, s_raw, xq, m0, n0, idx);
+    ksplit_finish_four<MODE, BN, WAVES, kConv>(e, &sX[0][0], kWaveLds, s_raw, xq, m0, n0, idx);
 }
 
 }  // namespace tmq

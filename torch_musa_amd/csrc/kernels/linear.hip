@@ -594,8 +594,9 @@ int launch_gemm_wloop(const GemmArgs& a, const XLinear& xs, bool wide, hipStream
 template <int MODE>
 int launch_gemm_wloop_ragged(const GemmArgs& a, const XLinear& xs, bool wide, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(ceil_div(a.N, wide ? 64 : 32)), static_cast<unsigned>(ceil_div(a.M, 32)));
-  if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2, true>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
-  else enqueue(gemm_i8_wloop_kernel<MODE, 1, true>, grid, dim3(kWloopWaves * kWave), 0, s, a, xs);
+  const XLinearRagged rows{xs.x, xs.ldx};
+  if (wide) enqueue(gemm_i8_wloop_kernel<MODE, 2, XLinearRagged>, grid, dim3(kWloopWaves * kWave), 0, s, a, rows);
+  else enqueue(gemm_i8_wloop_kernel<MODE, 1, XLinearRagged>, grid, dim3(kWloopWaves * kWave), 0, s, a, rows);
   return launch_status();
 }
 
