@@ -346,8 +346,11 @@ __device__ __forceinline__ void ksplit_finish_four(const GemmArgs& a, const uint
                     : requant4<MODE, true>(raw, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);
     }
     uint8_t* const dst = static_cast<uint8_t*>(a.y) + a.n_off + m * a.ldy + n;
-    if ((reinterpret_cast<uintptr_t>(dst) & 3) == 0 && n + 4 <= a.N) {
-      *reinterpret_cast<uint32_t*>(dst) = q4;
+    struct __attribute__((packed, aligned(1))) FourBytes {
+      uint32_t v;
+    };
+    if (n + 4 <= a.N) {
+      reinterpret_cast<FourBytes*>(dst)->v = q4;
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
