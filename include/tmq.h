@@ -393,6 +393,14 @@ int tmq_linear_float(const tmq_linear_desc* desc, const tmq_qparams* x_qparams_d
  * aside).  Uses M, N, K, w_*, relu, bias of `desc`; desc->kernel = 9 / 29 pins
  * the first / second kernel for tests.  Same reference note as tmq_linear_f32. */
 int tmq_linear_dynamic_small_takes(int64_t M, int64_t N, int64_t K);
+/* The same for more than 16 rows that make one round of tiles: bytes of `workspace`
+ * the call needs (0: none), or -1 where the size is not such a one. */
+int64_t tmq_linear_dynamic_tiles_workspace(int64_t M, int64_t N, int64_t K);
+/* polls: of the other blocks' ranges, before a block finds a missing one itself
+ * (negative: the default).  TMQ_ERR_UNSUPPORTED for other sizes, too little
+ * workspace, and more than 32 rows on a stream that is being captured. */
+int tmq_linear_dynamic_tiles(const tmq_linear_desc* desc, const float* x, int64_t ldx, int reduce_range, float* y,
+                             int64_t ldy, int polls, tmq_stream_t stream);
 int tmq_linear_dynamic_small(const tmq_linear_desc* desc, const float* x, int64_t ldx, int reduce_range,
                              float* y, int64_t ldy, tmq_stream_t stream);
 

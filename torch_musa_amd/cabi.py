@@ -24,7 +24,7 @@ DECLARED_SYMBOLS = [
     "tmq_quantize_per_channel", "tmq_dequantize_per_channel",
     "tmq_quantize_per_channel_float_qparams", "tmq_dequantize_per_channel_float_qparams",
     "tmq_linear_packed_kchunks", "tmq_linear_packed_bytes", "tmq_linear_prepack",
-    "tmq_linear_unpack", "tmq_linear", "tmq_linear_workspace_bytes", "tmq_linear_split_plan", "tmq_linear_kernel_choice", "tmq_linear_static_workspace", "tmq_linear_acc32", "tmq_linear_f32", "tmq_linear_dynamic_small", "tmq_linear_dynamic_small_takes", "tmq_quantize_per_tensor_dynamic_dev",
+    "tmq_linear_unpack", "tmq_linear", "tmq_linear_workspace_bytes", "tmq_linear_split_plan", "tmq_linear_kernel_choice", "tmq_linear_static_workspace", "tmq_linear_acc32", "tmq_linear_f32", "tmq_linear_dynamic_small", "tmq_linear_dynamic_small_takes", "tmq_linear_dynamic_tiles", "tmq_linear_dynamic_tiles_workspace", "tmq_quantize_per_tensor_dynamic_dev",
     "tmq_quantize_per_tensor_dynamic_report", "tmq_quantize_per_tensor_dynamic_parts", "tmq_quantize_rows_dynamic_dev", "tmq_quantize_dynamic_exchange", "tmq_linear_scratch_bytes", "tmq_linear_rows_in_place", "tmq_linear_float", "tmq_per_channel",
     "tmq_conv2d_packed_bytes", "tmq_conv2d_prepack", "tmq_conv2d_out_hw", "tmq_conv2d_workspace_bytes", "tmq_conv2d_scratch_bytes",
     "tmq_conv2d", "tmq_conv2d_acc32", "tmq_conv2d_fused",
@@ -142,6 +142,9 @@ def lib() -> C.CDLL:
         l.tmq_linear_f32.argtypes = [C.POINTER(LinearDesc), v, v, C.c_int64, v]
         l.tmq_linear_dynamic_small.argtypes = [C.POINTER(LinearDesc), v, C.c_int64, C.c_int, v, C.c_int64, v]
         l.tmq_linear_dynamic_small_takes.argtypes = [C.c_int64, C.c_int64, C.c_int64]
+        l.tmq_linear_dynamic_tiles.argtypes = [C.POINTER(LinearDesc), v, C.c_int64, C.c_int, v, C.c_int64, C.c_int, v]
+        l.tmq_linear_dynamic_tiles_workspace.restype = C.c_int64
+        l.tmq_linear_dynamic_tiles_workspace.argtypes = [C.c_int64, C.c_int64, C.c_int64]
         l.tmq_quantize_per_tensor_dynamic_dev.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v]
         l.tmq_quantize_per_tensor_dynamic_report.argtypes = [v, v, C.c_int64, C.c_int, C.c_int, C.c_int, v, v, C.c_size_t, v,
                                                              C.c_uint32, C.c_uint32, v]

@@ -591,6 +591,29 @@ struct PackedLinearWeightTmq final : public LinearPackedParamsBase {
                    "tmq_linear_dynamic_small");
       return y;
     }
+    if (const int64_t words = tmq_linear_dynamic_tiles_workspace(M, N_, K_); words >= 0) {
+      // one round of tiles: the same, with the ranges exchanged on the way (not on a stream that is captured)
+      tmq_linear_desc d{};
+      d.M = M;
+      d.N = N_;
+      d.K = K_;
+      d.w_packed = packed_.const_data_ptr();
+      d.w_colsum = cptr<int32_t>(colsum_);
+      d.w_scales = cptr<float>(wp_.scales_f32);
+      d.w_per_channel = wp_.per_channel;
+      d.relu = relu;
+      d.bias = bias_.has_value() ? cptr<float>(*bias_) : nullptr;
+      const at::Tensor ranges = words > 0 ? empty_bytes(words, x) : at::Tensor();
+      if (words > 0) {
+        d.workspace = ranges.data_ptr();
+        d.workspace_bytes = words;
+      }
+      const int status = tmq_linear_dynamic_tiles(&d, cptr<float>(x), K_, reduce_range, mptr<float>(y), N_, -1, stream);
+      if (status != TMQ_ERR_UNSUPPORTED) {
+        check_status(status, "tmq_linear_dynamic_tiles");
+        return y;
+      }
+    }
     // one allocation: the codes (rows on the 16-byte grid), the partial ranges, the parameters
     const int64_t pitch = (K_ + 15) / 16 * 16;
     const int64_t code_bytes = (M * pitch + 255) / 256 * 256;

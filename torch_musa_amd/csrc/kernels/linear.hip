@@ -9,6 +9,7 @@
 #include "gemm_i8_persistent.h"
 #include "gemm_i8_wring.h"
 #include "gemm_i8_wloop.h"
+#include "linear_dynamic_tiles.h"
 #include "linear_resident.h"
 #include "qparams.h"
 
@@ -1879,6 +1880,72 @@ TMQ_EXPORT int tmq_linear_dynamic_small_takes(int64_t M, int64_t N, int64_t K) {
   if (4 * dyn_groups(M, K) <= kDynSmallMaxValues) return 1;
   const int cus = cu_count();
   return dyn_resident_ok(M, N, K, cus > 0 ? cus : 256) ? 1 : 0;
+}
+
+namespace tmq {
+namespace {
+
+constexpr int64_t kDynTilesMaxK = 2048;
+// Channels per tile of the one-launch dynamic linear of more than 16 rows, 0: not such a shape.  All its blocks have to be on the chip
+// together (one that waits for a block behind it finds that one's range itself, but late): one a CU, two up to K = 512, where
+// their registers and LDS allow that (us, two launches | 64 channels on 257 to 512 tiles: 135 x 64 -> 5104 7.8 | 6.1, 79 x 263 -> 10799
+// 9.6 | 7.0, 3041 x 256 -> 184 8.5 | 6.6, 2825 x 448 -> 296 10.2 | 8.2; 32 channels there, where 64 have one a CU, 3370 x 344 -> 111 7.5
+// against 5.9).
+int dyn_tile(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16 || M > 32 * kRangeParts || N <= 0 || N >= (int64_t{1} << 29) || K < 16 || K > kDynTilesMaxK) return 0;
+  const int64_t tiles_m = ceil_div(M, 32), cus = cu_count() > 0 ? cu_count() : 256;
+  return tiles_m * ceil_div(N, 32) <= cus ? 32 : tiles_m * ceil_div(N, 64) <= (K <= 512 ? 2 * cus : cus) ? 64 : 0;
+}
+template <int CT>
+auto dyn_tiles_kernel(int64_t K) {
+  return K <= 256    ? linear_dynamic_tiles_kernel<CT, 32>
+         : K <= 512  ? linear_dynamic_tiles_kernel<CT, 64>
+         : K <= 1024 ? linear_dynamic_tiles_kernel<CT, 128>
+                     : linear_dynamic_tiles_kernel<CT, 256>;
+}
+
+}  // namespace
+}  // namespace tmq
+
+TMQ_EXPORT int64_t tmq_linear_dynamic_tiles_workspace(int64_t M, int64_t N, int64_t K) {
+  return dyn_tile(M, N, K) == 0 ? -1 : M <= 32 ? 0 : ceil_div(M, 32) * static_cast<int64_t>(sizeof(v4u));
+}
+
+TMQ_EXPORT int tmq_linear_dynamic_tiles(const tmq_linear_desc* d, const float* x, int64_t ldx, int reduce_range, float* y,
+                                        int64_t ldy, int polls, tmq_stream_t stream) {
+  if (d == nullptr) return TMQ_ERR_INVALID_ARGUMENT;
+  const int tile = dyn_tile(d->M, d->N, d->K);
+  if (tile == 0) return TMQ_ERR_UNSUPPORTED;
+  if (x == nullptr || y == nullptr || d->w_packed == nullptr || d->w_colsum == nullptr || d->w_scales == nullptr || ldx < d->K ||
+      ldy < d->N)
+    return TMQ_ERR_INVALID_ARGUMENT;
+  if (!aligned(x, 4) || !aligned(d->w_packed, 16) || !aligned(y, 4)) return TMQ_ERR_UNSUPPORTED;
+  hipStream_t s = as_stream(stream);
+  const int64_t tiles_m = ceil_div(d->M, 32), tiles_n = ceil_div(d->N, tile);
+  if (tiles_m > 1 && (d->workspace == nullptr || d->workspace_bytes < tiles_m * static_cast<int64_t>(sizeof(v4u)) ||
+                      !aligned(d->workspace, 16) || replayed(s)))
+    return TMQ_ERR_UNSUPPORTED;
+  GemmArgs a{};
+  a.M = d->M;
+  a.N = d->N;
+  a.K = d->K;
+  a.w_packed = static_cast<const uint8_t*>(d->w_packed);
+  a.w_kchunks = packed_kchunks(d->K);
+  a.colsum = d->w_colsum;
+  a.w_scales = d->w_scales;
+  a.w_scale_stride = d->w_per_channel ? 1 : 0;
+  a.bias = d->bias;
+  a.lo_f = d->relu ? 0.f : -__builtin_inff();
+  a.y = y;
+  a.ldy = ldy;
+  const bool by_rows = 4 * d->M >= d->N;
+  const int64_t minor = by_rows ? tiles_n : tiles_m;
+  const DynTileOrder order{static_cast<uint32_t>(tiles_m), static_cast<uint32_t>(tiles_n),
+                           minor == 1 ? 0u : static_cast<uint32_t>(((int64_t{1} << 32) + minor - 1) / minor), by_rows ? 1 : 0};
+  const RangeWords range{static_cast<v4u*>(d->workspace), tiles_m > 1 ? next_range_tag() : 0, polls < 0 ? kRangePolls : polls};
+  enqueue(tile == 32 ? dyn_tiles_kernel<1>(d->K) : dyn_tiles_kernel<2>(d->K), dim3(static_cast<unsigned>(tiles_m * tiles_n)),
+          dim3(kDynTileThreads), 0, s, a, x, ldx, reduce_range, range, order);
+  return launch_status();
 }
 
 TMQ_EXPORT int tmq_linear_dynamic_small(const tmq_linear_desc* d, const float* x, int64_t ldx, int reduce_range,

@@ -10,8 +10,6 @@
 // multiply by the fp32 reciprocal of the fp32 scale, round half to even, add
 // the zero point, clamp.  Compiled with -ffp-contract=off.
 #include <algorithm>
-#include <atomic>
-#include <chrono>
 #include <cmath>
 #include <limits>
 #include <type_traits>
@@ -1271,25 +1269,6 @@ namespace {
 // 4.8 | 4.0, 96 Ki 5.8 | 3.9).  Up to 64 Mi values; beyond, range and codes stream past the caches in three launches (64 Mi
 // 94 | 87, 256 Mi 372 | 478: one block per CU has too little on its way for what it does not hold).
 constexpr int64_t kHeldAbove = 32768, kHeldUpTo = int64_t{1} << 26;
-constexpr int kHeldPolls = 32;  // of about a microsecond each: more than the blocks of one launch are apart on an idle chip
-
-// What no other launch of this process has (a permutation of a counter; its start differs from process to process).
-uint64_t next_range_tag() {
-  static std::atomic<uint64_t> count{static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
-  uint64_t z = count.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;
-  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-  return z ^ (z >> 31);
-}
-
-// A captured launch keeps its arguments: its tag would be in the words already when the graph runs again.
-bool replayed(hipStream_t s) {
-  if (s == nullptr) return false;  // (the null stream cannot be captured)
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;  // unknown: as if it were
-}
 
 struct HeldCall {
   const float* x;
@@ -1341,7 +1320,7 @@ int launch_held(const HeldCall& c, int most_blocks, int polls, const RangeReport
     if (h >= per_thread) held = h;
   const int32_t more = static_cast<int32_t>(per_thread > held ? per_thread - held : 0);
   const auto kernel = rows ? held_kernel<true, true>(held) : c.fused ? held_kernel<true, false>(held) : held_kernel<false, false>(held);
-  const HeldRange range{static_cast<v4u*>(c.workspace), next_range_tag(), polls};
+  const RangeWords range{static_cast<v4u*>(c.workspace), next_range_tag(), polls};
   if (parts != nullptr) *parts_count = static_cast<int32_t>(blocks);
   enqueue(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHeldThreads), 0, s, c.x, static_cast<uint32_t*>(c.q),
           static_cast<int32_t>(total), static_cast<int32_t>(rows ? c.K : 0), static_cast<int32_t>(rows ? c.pitch / 4 : 1),
@@ -1364,7 +1343,7 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   const HeldCall held{x, q, 1, n, n, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
   if (n > kHeldAbove && held_runs(held, s)) {
     const bool in_parts = parts != nullptr && n > TMQ_HOST_PARTS_ABOVE && n <= TMQ_HOST_PARTS_UP_TO;
-    return launch_held(held, in_parts ? TMQ_HOST_PARTS : kHeldBlocks, kHeldPolls, in_parts ? RangeReport{nullptr, 0, 0} : report,
+    return launch_held(held, in_parts ? TMQ_HOST_PARTS : kHeldBlocks, kRangePolls, in_parts ? RangeReport{nullptr, 0, 0} : report,
                        in_parts ? parts : nullptr, parts_count, s);
   }
   if (n <= kDynRepeatMax) {
@@ -1473,7 +1452,7 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
   const int64_t n = M * K;
   const HeldCall held{x, q, M, K, pitch, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
   if (n > kHeldAbove && held_runs(held, s))
-    return launch_held(held, kHeldBlocks, kHeldPolls, RangeReport{nullptr, 0, 0}, nullptr, nullptr, s);
+    return launch_held(held, kHeldBlocks, kRangePolls, RangeReport{nullptr, 0, 0}, nullptr, nullptr, s);
   if (n <= kDynRepeatMax)
     return launch_dynamic_repeat(q_signed != 0, fused, M * (pitch / 4), s, x, static_cast<uint8_t*>(q), static_cast<int32_t>(n),
                                  static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4), qmin, qmax, reduce_range, true,

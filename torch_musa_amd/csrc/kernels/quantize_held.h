@@ -4,10 +4,9 @@
 #include <limits>
 
 #include "common.h"
-#include "dynamic_rows.h"
 #include "host_report.h"
 #include "qparams.h"
-#include "stores_through.h"
+#include "range_exchange.h"
 
 namespace tmq {
 namespace {
@@ -27,19 +26,9 @@ namespace {
 // is not read twice, and the caches are left to what is (4096 x 4096 18.1 -> 15.0 ... 17.5; 16 groups and fewer measured slower
 // that way when the same input comes again, 9.2 -> 9.4).
 constexpr int kHeldThreads = 512;
-constexpr int kHeldBlocks = 256;
+constexpr int kHeldBlocks = kRangeParts;
 constexpr int kHeldMost = 32;
 constexpr int kHeldStream = 24;
-
-// Where the blocks tell each other the ranges of their parts: a word of 16 bytes for each, {minimum, low half of the tag,
-// maximum, high half of the tag}.  Either half of a word is whole if its half of the tag is this launch's; no other launch
-// of the process has that tag, so what the memory held before need not be cleared.
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-struct HeldRange {
-  v4u* words;
-  uint64_t tag;
-  int polls;  // of the words, before a block sees to what is missing itself
-};
 
 // `total` words of four codes, H + more of them for each thread.  Dense (not ROWS): x on the 16-byte grid, `tail` values
 // (below four) behind the last word.  ROWS: rows of K >= 4 values at any 4-byte alignment -> rows of pitch4 words; the codes
@@ -48,11 +37,11 @@ struct HeldRange {
 template <bool FUSED, bool ROWS, int H>
 __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     const float* __restrict__ x, uint32_t* __restrict__ q4, int32_t total, int32_t K, int32_t pitch4, int32_t tail,
-    HeldRange range, int32_t more, uint32_t sign_flip, int qmin, int qmax, int reduce_range, tmq_qparams* __restrict__ out,
+    RangeWords range, int32_t more, uint32_t sign_flip, int qmin, int qmax, int reduce_range, tmq_qparams* __restrict__ out,
     RangeReport report, uint64_t* parts) {
   constexpr int kWaves = kHeldThreads / kWave;
   constexpr int kAhead = H >= 16 ? 16 : 4;  // (of the words that are not held; only H = kHeldMost has any)
-  __shared__ float s_mn[kWaves], s_mx[kWaves], s_inv, s_zp;
+  __shared__ float s_range[2 * kWaves], s_inv, s_zp;
   __shared__ int s_missing;
   const int t = threadIdx.x, own = static_cast<int>(blockIdx.x), blocks = static_cast<int>(gridDim.x);
   const int step = blocks * kHeldThreads;
@@ -99,25 +88,12 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
   };
   // The range of a block's part, to where all blocks see it (and to the host).
   const auto publish = [&](int block, float mn, float mx, uint64_t* part) {
-    wave_minmax_last(mn, mx);
-    if (t % kWave == kWave - 1) {
-      s_mn[t / kWave] = mn;
-      s_mx[t / kWave] = mx;
-    }
-    __syncthreads();
-    if (t < kWave) {
-      static_assert(kWaves <= 16 && 16 % kWaves == 0);
-      mn = s_mn[t % kWaves];
-      mx = s_mx[t % kWaves];
-      row_minmax(mn, mx);
-      const uint32_t lo = __builtin_bit_cast(uint32_t, lane_float(mn, 15));
-      const uint32_t hi = __builtin_bit_cast(uint32_t, lane_float(mx, 15));
-      if (t == 0) {
-        const v4u word = {lo, static_cast<uint32_t>(range.tag), hi, static_cast<uint32_t>(range.tag >> 32)};
-        st16_through(range.words + block, __builtin_bit_cast(v4i, word));
-        if (part != nullptr)  // (one store of eight bytes: complete or not there)
-          __hip_atomic_store(part, (static_cast<uint64_t>(hi) << 32) | lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      }
+    block_range<kWaves>(mn, mx, s_range, t);
+    if (t == 0) {
+      put_range(range, block, mn, mx);
+      if (part != nullptr)  // (one store of eight bytes: complete or not there)
+        __hip_atomic_store(part, (static_cast<uint64_t>(__builtin_bit_cast(uint32_t, mx)) << 32) | __builtin_bit_cast(uint32_t, mn),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   };
 
@@ -152,36 +128,8 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
   // All ranges, and the parameters from them.
   for (;;) {
     if (t < kWave) {
-      constexpr int kPer = kHeldBlocks / kWave;
-      uint64_t absent[kPer];
-      bool there;
-      for (int poll = 0;; ++poll) {
-        v4u w[kPer];
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-          const int i = j * kWave + t;
-          w[j] = __builtin_amdgcn_global_load_b128(
-              (__attribute__((address_space(1))) v4u_global*)(range.words + (i < blocks ? i : blocks - 1)), "agent");
-        }
-        mn = std::numeric_limits<float>::infinity();
-        mx = -std::numeric_limits<float>::infinity();
-        there = true;
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-          absent[j] = __builtin_amdgcn_ballot_w64(w[j].y != static_cast<uint32_t>(range.tag) ||
-                                                  w[j].w != static_cast<uint32_t>(range.tag >> 32));
-          there = there && absent[j] == 0;
-          const uint32_t lo = w[j].x, hi = w[j].z;  // (__builtin_bit_cast of a vector's element takes its first one)
-          mn = fminf(mn, __builtin_bit_cast(float, lo));
-          mx = fmaxf(mx, __builtin_bit_cast(float, hi));
-        }
-        if (there || poll >= range.polls) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      if (there) {
-        wave_minmax_last(mn, mx);
-        mn = lane_float(mn, kWave - 1);
-        mx = lane_float(mx, kWave - 1);
+      const int missing = get_ranges(range, blocks, own, mn, mx);
+      if (missing < 0) {
         if (own == 0 && t == 0) report_range(report, mn, mx);
         double s;
         int32_t z;
@@ -194,26 +142,14 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
           }
           s_inv = 1.0f / static_cast<float>(s);  // IEEE division, as in resolve()
           s_zp = static_cast<float>(z);
-          s_missing = -1;
         }
-      } else if (t == 0) {
-        // the next absent block behind this one: blocks that wait together see to different ones
-        int first = -1, next = -1;
-        for (int j = 0; j < kPer; ++j)
-          for (uint64_t m = absent[j]; m != 0; m &= m - 1) {
-            int i = j * kWave + __builtin_ctzll(m);
-            i = i < blocks ? i : blocks - 1;
-            if (first < 0) first = i;
-            if (next < 0 && i > own) next = i;
-          }
-        s_missing = next >= 0 ? next : first;
       }
+      if (t == 0) s_missing = missing;
     }
     __syncthreads();
     const int missing = s_missing;
     if (missing < 0) break;
-    // That block has not run yet -- the chip is not this launch's alone -- or not for this long.  Any block can find its
-    // range, and the word says the same whoever writes it: every block ends whether or not the others run beside it.
+    // That block has not run yet -- the chip is not this launch's alone -- or not for this long.
     float a = std::numeric_limits<float>::infinity();
     float b = -std::numeric_limits<float>::infinity();
     Place p = place(missing);
