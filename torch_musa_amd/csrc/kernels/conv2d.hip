@@ -1002,12 +1002,22 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
   int64_t strip = pinned_strip ? d->tile_rows : kDwStripMax;
   // (images of 9 to 14 rows in two strips: 5 x 5 over 672 channels on 14 x 14 9.9 against 10.8 us in one)
   if (!pinned_strip && s.KH >= 5 && s.OH > 8) strip = ceil_div(s.OH, s.OH <= 14 ? 2 : ceil_div(s.OH, 14));
+  // Two columns a lane for 3 x 3 at stride 1 where strips of eight rows are four waves a SIMD and more of one column (us, one | two: 624
+  // channels on 15 x 42 x 26 12.3 | 10.7, 768 on 15 x 55 x 27 17.6 | 15.1, 864 on 28 x 100 x 44 85 | 72; with the layers around it,
+  // 768 on 14 x 26 x 59 33.4 | 29.8, 816 on 4 x 106 x 74 56.7 | 53.2, 288 on 23 x 69 x 53 46.1 | 44.4; below, what is left over of the
+  // last wave decides, 288 on 25 x 7 x 110 23.1 | 23.8).  From 256 channels on: fewer leave a line in two parts, which what follows pays
+  // for (234 on 15 x 33 x 97 30.5 | 31.4, 120 on 27 x 38 x 69 32.1 | 33.0); and no odd width that wastes more than a sixteenth (768 on
+  // 18 x 55 x 13 30.1 | 30.4).
+  const bool pairs = !pinned_strip && s.KH == 3 && s.KW == 3 && s.sh == 1 && s.sw == 1 && s.dh == 1 && s.dw == 1 && s.IC >= 256 &&
+                     (s.OW % 2 == 0 || s.OW > 16) &&
+                     s.B * ceil_div(s.OH, kDwStripMax) * s.OW * ceil_div(s.IC, 4) >= int64_t{1} << 18;
+  const int64_t across = pairs ? ceil_div(s.OW, 2) : s.OW;
   const int64_t lanes_wanted = int64_t{1} << (s.KH == 7 && s.KW == 7 ? 15 : 16);
   if (!pinned_strip)
-    while (strip > 1 && s.B * ceil_div(s.OH, strip) * s.OW * ceil_div(s.IC, 4) < lanes_wanted) strip = ceil_div(strip, 2);
+    while (strip > 1 && s.B * ceil_div(s.OH, strip) * across * ceil_div(s.IC, 4) < lanes_wanted) strip = ceil_div(strip, 2);
   if (strip > s.OH) strip = s.OH;
   a.strip = static_cast<int>(strip);
-  const int64_t per_image = ceil_div(s.OH, strip) * s.OW * ceil_div(s.IC, 4);
+  const int64_t per_image = ceil_div(s.OH, strip) * across * ceil_div(s.IC, 4);
   const int64_t blocks_per_image = ceil_div(per_image, kDwThreads);
   a.per_image = static_cast<uint32_t>(per_image);
   a.blocks_per_image = static_cast<uint32_t>(blocks_per_image);
@@ -1024,7 +1034,9 @@ int launch_conv_depthwise(const tmq_conv2d_desc* d, const ConvShape& s, const Po
   const dim3 grid(static_cast<unsigned>(blocks)), block(kDwThreads);
   const auto launch_as = [&](auto post_tag, auto through_tag) {
     constexpr bool kP = decltype(post_tag)::value, kThrough = decltype(through_tag)::value;
-    if (s.KH == 3 && s.KW == 3)
+    if (pairs)
+      enqueue(conv_depthwise_kernel<MODE, kP, 3, kThrough, 2>, grid, block, 0, stream, a);
+    else if (s.KH == 3 && s.KW == 3)
       enqueue(conv_depthwise_kernel<MODE, kP, 3, kThrough>, grid, block, 0, stream, a);
     else if (s.KH == 5 && s.KW == 5)
       enqueue(conv_depthwise_kernel<MODE, kP, 5, kThrough>, grid, block, 0, stream, a);

@@ -85,13 +85,19 @@ __device__ __forceinline__ void transpose_4x4_bytes(uint32_t a0, uint32_t a1, ui
 // load sits behind a branch -- and the zero point replaces what came back, chosen by bits (a
 // select would let the compiler move the load behind a branch again).
 // THROUGH: bytes on the 4-byte grid leave past the L2 (a branch on that in the row loop costs 0.6 of 6.4 us).
-template <int MODE, bool POST, int KS, bool THROUGH>
+// COLS = 2 (3 x 3 at stride 1, no dilation): a lane has two neighbouring output columns.  Their four pixels a row are one transposition,
+// the second column's weights the first's moved up by a byte, so that a row of eight values takes four loads and eight permutes
+// where it took six and sixteen: the vector unit bounds large layers (launch_conv_depthwise has the figures).  A second row on its
+// way made no difference.
+template <int MODE, bool POST, int KS, bool THROUGH, int COLS = 1>
 __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_depthwise_kernel(DepthwiseArgs a) {
+  static_assert(COLS == 1 || (COLS == 2 && KS == 3), "two columns' taps in one dword");
   const uint32_t b = blockIdx.x / a.blocks_per_image;
   const uint32_t q0 = (blockIdx.x - b * a.blocks_per_image) * kDwThreads, q = q0 + threadIdx.x;
   const uint32_t C4 = (static_cast<uint32_t>(a.C) + 3) >> 2, c_last = static_cast<uint32_t>(a.C) - 4;
   const uint32_t rest = q / C4, cg = q - rest * C4;
-  const uint32_t strip = rest / static_cast<uint32_t>(a.OW), ow = rest - strip * static_cast<uint32_t>(a.OW);
+  const uint32_t across = (static_cast<uint32_t>(a.OW) + COLS - 1) / COLS;
+  const uint32_t strip = rest / across, ow = (rest - strip * across) * COLS;
   const uint32_t c = cg * 4 < c_last ? cg * 4 : c_last;
   constexpr int kSide = KS > 0 ? KS : 1;
   constexpr int kGroups = (kSide + 3) / 4;  // dwords of four taps per kernel row
@@ -170,46 +176,50 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
   const int oh_end = oh_first + a.strip < a.OH ? oh_first + a.strip : a.OH;
   uint32_t yoff = ((b * static_cast<uint32_t>(a.OH) + oh_first) * static_cast<uint32_t>(a.OW) + ow) * static_cast<uint32_t>(a.C) + c;
   const uint32_t ystep = static_cast<uint32_t>(a.OW * a.C);
-  const auto finish = [&](const int (&acc)[4]) {
+  const auto finish_at = [&](const int (&acc)[4], uint32_t at) {
     if constexpr (MODE == kOutAcc32) {
-      reinterpret_cast<DwFour*>(static_cast<int32_t*>(a.y) + yoff)->v = v4i{acc[0], acc[1], acc[2], acc[3]};
+      reinterpret_cast<DwFour*>(static_cast<int32_t*>(a.y) + at)->v = v4i{acc[0], acc[1], acc[2], acc[3]};
     } else {
       uint32_t packed;
       if constexpr (POST) {
-        const uint32_t accw = a.post.accum != nullptr ? dw_load(a.post.accum + yoff) : 0u;
+        const uint32_t accw = a.post.accum != nullptr ? dw_load(a.post.accum + at) : 0u;
         packed = requant4_post<MODE>(acc, bdiv, bmul, mult, a.post, accw, a.zp_f, a.lo_f, a.hi_f);
       } else {
         packed = requant4<MODE, true, 2>(acc, bdiv, bmul, mult, a.zp_f, a.lo_f, a.hi_f);  // (tested here: 11.8 -> 10.8 us where it holds, level where not)
       }
-      uint8_t* const dst = static_cast<uint8_t*>(a.y) + yoff;
+      uint8_t* const dst = static_cast<uint8_t*>(a.y) + at;
       if constexpr (THROUGH) st4_through(dst, packed);
       else reinterpret_cast<DwWord*>(dst)->v = packed;
     }
+  };
+  const auto finish = [&](const int (&acc)[4]) {
+    finish_at(acc, yoff);
     yoff += ystep;
   };
 
   if constexpr (KS > 0) {
     // the window's columns: fixed for the lane (masks: all ones where the tap is inside the image)
-    uint32_t col[KS], col_in[KS];
+    constexpr int kTaps = KS + COLS - 1;
+    uint32_t col[kTaps], col_in[kTaps];
 #pragma unroll
-    for (int kw = 0; kw < KS; ++kw) {
+    for (int kw = 0; kw < kTaps; ++kw) {
       const int iw = iw0 + kw * a.dw;
       col_in[kw] = static_cast<unsigned>(iw) < static_cast<unsigned>(a.W) ? ~0u : 0u;
       col[kw] = lane_base + (static_cast<uint32_t>(iw * a.C) & col_in[kw]);
     }
     // loads of one window row (what comes back is not looked at here) ...
-    const auto request_row = [&](int ih, int pos, uint32_t (&raw)[KS], uint32_t& row_in) {
+    const auto request_row = [&](int ih, int pos, uint32_t (&raw)[kTaps], uint32_t& row_in) {
       row_in = static_cast<unsigned>(ih) < static_cast<unsigned>(a.H) ? ~0u : 0u;
       const uint32_t rp = static_cast<uint32_t>(pos) & row_in;
 #pragma unroll
-      for (int kw = 0; kw < KS; ++kw) raw[kw] = dw_load(a.x + (rp + col[kw]));
+      for (int kw = 0; kw < kTaps; ++kw) raw[kw] = dw_load(a.x + (rp + col[kw]));
     };
     // ... and the row they make: [channel][group of four taps]
-    const auto settle_row = [&](const uint32_t (&raw)[KS], uint32_t row_in, uint32_t (&row)[4][kGroups]) {
+    const auto settle_row = [&](const uint32_t (&raw)[kTaps], uint32_t row_in, uint32_t (&row)[4][kGroups]) {
       uint32_t v[4 * kGroups];
 #pragma unroll
       for (int kw = 0; kw < 4 * kGroups; ++kw) {
-        if (kw < KS) {
+        if (kw < kTaps) {
           const uint32_t in = row_in & col_in[kw];
           v[kw] = ((raw[kw] & in) | (a.pad_word & ~in)) ^ a.x_xor;
         } else {
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
     };
     uint32_t win[KS][4][kGroups];
     // window row kh of the current output row is win[(kh + ROT) % KS]
-    const auto window_sums = [&](auto rot_tag, int (&acc)[4]) {
+    const auto window_sums = [&](auto rot_tag, int (&acc)[4], const uint32_t (&weights)[kSide][4][kGroups]) {
       constexpr int ROT = decltype(rot_tag)::value;
 #pragma unroll
       for (int kh = 0; kh < KS; ++kh)
@@ -234,14 +244,22 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int g = 0; g < kGroups; ++g)
-            acc[j] = __builtin_amdgcn_sdot4(static_cast<int>(win[(kh + ROT) % KS][j][g]), static_cast<int>(wreg[kh][j][g]), acc[j], false);
+            acc[j] = __builtin_amdgcn_sdot4(static_cast<int>(win[(kh + ROT) % KS][j][g]), static_cast<int>(weights[kh][j][g]), acc[j], false);
     };
+    // (the second column's weights: the same taps one pixel further on)
+    uint32_t wnext[kSide][4][kGroups];
+    if constexpr (COLS == 2)
+#pragma unroll
+      for (int kh = 0; kh < KS; ++kh)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wnext[kh][j][0] = wreg[kh][j][0] << 8;
+    const bool second = ow + 1 < static_cast<uint32_t>(a.OW);
     const int ih_first = oh_first * a.sh - a.ph;
-    if (a.sh == 1 && a.dh == 1) {
+    if (COLS == 2 || (a.sh == 1 && a.dh == 1)) {
       // Stride 1: the window moves down one image row per output row.  The fences keep the
       // compiler's scheduler from moving the entering row's loads down to their use.
       {
-        uint32_t raw[KS][KS], row_in[KS];
+        uint32_t raw[KS][kTaps], row_in[KS];
 #pragma unroll
         for (int kh = 0; kh < KS; ++kh) request_row(ih_first + kh, (ih_first + kh) * static_cast<int>(row_bytes), raw[kh], row_in[kh]);
 #pragma unroll
@@ -253,13 +271,18 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
       // image read row 0, and nothing uses them) takes the place of the window's row 0
       const auto step = [&](auto rot_tag) {
         constexpr int ROT = decltype(rot_tag)::value;
-        uint32_t raw[KS], row_in;
+        uint32_t raw[kTaps], row_in;
         request_row(ih_next, pos_next, raw, row_in);
         ih_next += 1;
         pos_next += static_cast<int>(row_bytes);
         __builtin_amdgcn_sched_barrier(0);
         int acc[4] = {acc0[0], acc0[1], acc0[2], acc0[3]};
-        window_sums(rot_tag, acc);
+        window_sums(rot_tag, acc, wreg);
+        if constexpr (COLS == 2) {
+          int next[4] = {acc0[0], acc0[1], acc0[2], acc0[3]};
+          window_sums(rot_tag, next, wnext);
+          if (second) finish_at(next, yoff + static_cast<uint32_t>(a.C));
+        }
         finish(acc);
         __builtin_amdgcn_sched_barrier(0);
         settle_row(raw, row_in, win[ROT]);
@@ -289,13 +312,13 @@ __global__ __launch_bounds__(kDwThreads, KS == 7 && !POST ? 3 : 1) void conv_dep
       // any stride and dilation: the whole window per output row
       for (int oh = oh_first; oh < oh_end; ++oh) {
         const int ih0 = oh * a.sh - a.ph;
-        uint32_t raw[KS][KS], row_in[KS];
+        uint32_t raw[KS][kTaps], row_in[KS];
 #pragma unroll
         for (int kh = 0; kh < KS; ++kh) request_row(ih0 + kh * a.dh, (ih0 + kh * a.dh) * static_cast<int>(row_bytes), raw[kh], row_in[kh]);
 #pragma unroll
         for (int kh = 0; kh < KS; ++kh) settle_row(raw[kh], row_in[kh], win[kh]);
         int acc[4] = {acc0[0], acc0[1], acc0[2], acc0[3]};
-        window_sums(std::integral_constant<int, 0>{}, acc);
+        window_sums(std::integral_constant<int, 0>{}, acc, wreg);
         finish(acc);
       }
     }
