@@ -193,15 +193,15 @@ __device__ __forceinline__ uint32_t bf16_bits(float f) {
 __device__ __forceinline__ uint32_t fp16_bits(float f) {
   return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
 }
-// Stores four results of one output row, channels n .. n+3 (those below N), as a.f_kind asks.
-// STREAM: past the caches.  The 16-bit kinds leave the kernel instead of an fp32 tensor that
-// a second launch reads and converts.
-template <class V>
 // Rows whose length is no multiple of four: one store at any address, where four of a value each held up the end of the kernel (us, fp32
 // from 64 x 64 tiles: 592 x 192 -> 3581 8.1 | 6.0, 3821 x 160 -> 699 8.5 | 6.4, from 128 x 128 ones 217 x 2080 -> 10027 15.7 | 13.7).
+template <class V>
 struct __attribute__((packed, aligned(2))) FourOfAnyRow {
   V v;
 };
+// Stores four results of one output row, channels n .. n+3 (those below N), as a.f_kind asks.
+// STREAM: past the caches.  The 16-bit kinds leave the kernel instead of an fp32 tensor that
+// a second launch reads and converts.
 template <bool STREAM = false>
 __device__ __forceinline__ void put_f32x4(const GemmArgs& a, int64_t m, int64_t n, v4f v) {
   const int64_t at = m * a.ldy + a.n_off + n;
