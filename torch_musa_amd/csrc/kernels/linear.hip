@@ -1426,30 +1426,61 @@ int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
   return K > kWloopRaggedShortK && ceil_div(M, 32) * ceil_div(N, 32) <= 256 ? 32 : 64;
 }
 
-// More than that: 64 x 64 tiles that read the rows where they lie, or a copy
-// onto the grid and the padded shape's own kernel.  The copy is a launch (2.2 us and a scratch
-// allocation); the larger tiles it opens earn that back from 512 tiles on, later where K is short
-// (us, direct | copy, weights in the caches: M = 517: K = 1000, N = 2051 8.1 | 9.8, K = 2051, N = 1000 9.3 | 10.7; K = 3907,
-// N = 193, M = 2889 13.6 | 25.3; K = 4100, N = 3900, M = 500 (488 tiles) 22.6 | 23.9; K = 2051, N = 2051, M = 1000 (528)
-// 19.4 | 18.6; K = 1480, N = 5664, M = 611 (890) 18.9 | 14.7; K = 700, N = 2000, M = 2048 (1024) 11.3 | 12.6; K = 741,
-// N = 3952, M = 1560 (1550) 21.4 | 14.8; K = 500, N = 2000, M = 3000 (1504) 12.8 | 12.3; K = 100, N = 1000, M = 8000 (2000)
-// 10.4 | 12.8; K = 120, N = 8000, M = 4096 (8000) 26.3 | 22.1).  Few outputs leave the copy behind further on (K = 1204,
-// N = 646, M = 2983, 517 tiles, 11.3 | 14.9).
-bool ragged_tiles_preferred(int64_t M, int64_t N, int64_t K) {
-  if (K < 16 || K > 0x7fffff00) return false;
-  if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return false;
-  const int64_t tiles = ceil_div(M, 64) * ceil_div(N, 64);
-  return tiles <= (K <= 128 ? 3072 : K <= 768 ? 1024 : 512);
+// More than that: tiles that read the rows where they lie, or a copy onto the grid and the padded shape's own kernel.  The copy is a
+// launch (2.2 us and a scratch allocation).
+//
+// 64 x 64 tiles request every row once per 64 channels, and what bounds them is those unaligned requests; larger tiles halve them and
+// cost idle CUs where their grid is short.  So each tile is taken while its own grid makes one round and the smaller one's does not (us,
+// the route before (64 x 64, from 512 of them on the copy, K <= 768: 1024) | this one; 200 shapes drawn over M = 100 ... 4096, K = 141 ...
+// 4000, N = 240 ... 12000, 65 ... 4200 tiles of 64 x 64; bytes where nothing else is said, floats the same but for the lines that name them):
+//   64 x 128 from K = 1200 on (floats 1536: 183 x 1288 -> 6551 9.3 | 10.1, 183 x 1791 -> 5724 11.8 | 11.6): 2106 x 2839 -> 539 19.1 |
+//     14.1, 746 x 2053 -> 2555 13.7 | 11.9, 212 x 1481 -> 6574 11.5 | 10.2, 168 x 3495 -> 8678 level at 15.8; below, 64 x 64 are level
+//     or up to 12 % ahead (517 x 1000 -> 2051 7.8 | 8.0, 456 x 200 -> 3197 4.9 | 5.5);
+//   128 x 128, eight waves: 3931 x 2345 -> 881 24.7 | 16.9, 3819 x 1352 -> 998 19.1 | 12.3, 1989 x 375 -> 1580 9.3 | 7.2, 1019 x 1685 -> 2890
+//     15.3 | 13.8, 823 x 3208 -> 3743 21.6 | 19.7; beyond K = 3300 the copy, which floats want (275 x 3317 -> 7349 20.4 | 22.4); up to 288
+//     tiles of 64 x 128 at K <= 640 64 x 64 (230 x 264 -> 9105 5.7 | 6.0), up to 370 at K <= 330 (837 x 312 -> 2930 5.8 | 6.2; 1550 x
+//     279 -> 2151, 425 of them, 7.6 | 6.7);
+//   128 x 256, eight waves: 1860 x 574 -> 3469 17.8 | 11.8, 4022 x 1928 -> 1556 28.2 | 21.7, 446 x 1309 -> 10760
+//     16.8 | 15.8; up to 700 tiles of 64 x 128 at K < 480 those (516 x 372 -> 7244 10.7 | 8.0, with 128 x 256 9.4);
+//   beyond one round of those 128 x 128 where the copy is not ahead, K = 250 ... 640 (1356 x 344 -> 7817 17.3 | 14.4, 3508 x 252 -> 4716
+//     20.4 | 17.2; 1258 x 333 -> 9024 12.9 | 13.4; 7202 x 245 -> 1879 15.9 | 16.7, 2759 x 2023 -> 3364 34.9 | 38.1).
+// Elsewhere 64 x 64 up to 512 tiles, later where K is short, beyond that the copy (direct | copy: K = 2051, N = 1000, M = 517 9.3 |
+// 10.7; K = 4100, N = 3900, M = 500 22.6 | 23.9; K = 3907, N = 193, M = 2889 13.6 | 25.3; K = 100, N = 1000, M = 8000 10.4 | 12.8; K = 120,
+// N = 8000, M = 4096 26.3 | 22.1).
+enum class RaggedTile { kCopy, k64, k64x128, k128, k128x256 };
+constexpr int64_t kRaggedLargeMaxTiles = 4096, kRaggedLargeMaxK = 4000, kRagged128MaxK = 3300;
+RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
+  if (K < 16 || K > 0x7fffff00) return RaggedTile::kCopy;
+  if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return RaggedTile::kCopy;
+  const int64_t rows64 = ceil_div(M, 64), rows128 = ceil_div(M, 128);
+  const int64_t tiles = rows64 * ceil_div(N, 64), oblong = rows64 * ceil_div(N, 128);
+  // (at least 96 rows and 384 channels: fewer are padding in the larger tiles, 9974 x 296 -> 289 8.1 | 8.5)
+  if (tiles > 256 && tiles <= kRaggedLargeMaxTiles && M >= 96 && N >= 384 && K > 2 * kBK &&
+      K <= (oblong <= 256 ? kRaggedLargeMaxK : kRagged128MaxK)) {
+    if (oblong <= 256) {
+      if (K > (floats ? 1536 : 1200)) return RaggedTile::k64x128;
+    } else if (rows128 * ceil_div(N, 128) <= 256) {
+      if (K > 640 || oblong > (K > 330 ? 288 : 370)) return RaggedTile::k128;
+    } else if (rows128 * ceil_div(N, 256) <= 256) {
+      return K >= 480 || oblong > 700 ? RaggedTile::k128x256 : RaggedTile::k64x128;
+    } else if (K >= 250 && K <= 640) {
+      return RaggedTile::k128;
+    }
+  }
+  return tiles <= (K <= 128 ? 3072 : K <= 768 ? 1024 : 512) ? RaggedTile::k64 : RaggedTile::kCopy;
 }
 
-// ... and where the copy comes first, if there is room for it: K so long that the padded shape's kernel earns it back (two
-// layers, quantize and dequantize as a program calls them, direct | copy, us).  64 x 128 tiles in a ring: 600 x 6001 -> 2000
-// 45.3 | 34.6, 700 x 3001 -> 1500 30.8 | 26.8, 1500 x 2501 -> 900 31.4 | 29.7; 1000 x 2051 -> 2051 28.5 | 29.3, 2048 x 1310 ->
-// 1024 25.6 | 26.9.  One round of tiles of 32 rows against K > 4096 reads the rows in place where there is no room (wloop_ragged_tile),
+// ... and where the copy comes before 64 x 64 tiles, if there is room for it: K so long that the padded shape's kernel earns it back (two
+// layers, quantize and dequantize as a program calls them, direct | copy, us; 64 x 128 tiles in a ring: 600 x 6001 -> 2000
+// 45.3 | 34.6).  One round of tiles of 32 rows against K > 4096 reads the rows in place where there is no room (wloop_ragged_tile),
 // which is faster still and needs none; a caller that gives the room tmq_linear_scratch_bytes names has them copied.
 bool ragged_copy_first(int64_t M, int64_t N, int64_t K) {
   const int64_t pitch = regrid_pitch(K);
   return wloop_tile(M, N, pitch) != 0 || (K >= 2304 && oblong_ring_first(M, N, pitch, pitch));
+}
+RaggedTile ragged_route(int64_t M, int64_t N, int64_t K, bool floats, bool copy_ok) {
+  const RaggedTile tile = ragged_tile(M, N, K, floats);
+  return tile == RaggedTile::k64 && copy_ok && ragged_copy_first(M, N, K) ? RaggedTile::kCopy : tile;
 }
 
 template <int MODE>
@@ -1468,7 +1499,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
   if (a.splits != 1) return TMQ_ERR_INVALID_ARGUMENT;  // the split is this function's to plan
   if (!vec_ok && forced < 0) {
     // Off the 16-byte grid: up to 16 rows stream the weights as they are (the copy would cost a
-    // launch, more than any other kernel's advantage at so few rows); more rows take 64 x 64 tiles
+    // launch, more than any other kernel's advantage at so few rows); more rows take tiles
     // that read them where they lie, or are copied onto the grid if the caller left room for that
     // and take the kernel of the padded shape.
     if (a.M <= kDecodeRowsAuto && a.K >= 16 && stream_limits_ok(q) && a.w_kchunks == packed_kchunks(a.K))
@@ -1479,11 +1510,15 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     if (const int tile = wloop_ragged_tile(a.M, a.N, a.K); tile != 0 && zero_padded && xs.ldx <= (int64_t{1} << 23) &&
         a.N + a.n_off < (int64_t{1} << 29) && !(copy_ok && wloop_tile(a.M, a.N, regrid_pitch(a.K)) != 0))
       return launch_gemm_wloop_ragged<MODE>(a, xs, tile == 64, s);
-    if (ragged_tiles_preferred(a.M, a.N, a.K) && zero_padded &&
-        !(copy_ok && ragged_copy_first(a.M, a.N, a.K))) {
-      const XLinearRagged rows{xs.x, xs.ldx};
-      return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
-                                                : launch_gemm<64, 64, 2, 2, MODE>(a, rows, s);
+    const XLinearRagged rows{xs.x, xs.ldx};
+    switch (zero_padded ? ragged_route(a.M, a.N, a.K, MODE == kOutF32, copy_ok) : RaggedTile::kCopy) {
+      case RaggedTile::k64:
+        return two_wave_groups_fit(a.M, a.N, a.K) ? launch_gemm<64, 64, 2, 2, MODE, 4, false, 2>(a, rows, s)
+                                                  : launch_gemm<64, 64, 2, 2, MODE>(a, rows, s);
+      case RaggedTile::k64x128: return launch_gemm<64, 128, 2, 2, MODE>(a, rows, s);
+      case RaggedTile::k128: return launch_gemm<128, 128, 2, 4, MODE>(a, rows, s);
+      case RaggedTile::k128x256: return launch_gemm<128, 256, 2, 4, MODE>(a, rows, s);
+      case RaggedTile::kCopy: break;
     }
     if (copy_ok) {
       const int rc = launch_regrid(xs, a.M, a.K, workspace, s);
@@ -1639,7 +1674,7 @@ TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int
   const int64_t split = wloop_tile(M, N, regrid_pitch(K)) != 0 ? 0 : tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
   if (K % 16 == 0 && on_grid) return split;
   if (wloop_ragged_tile(M, N, K) != 0 && wloop_tile(M, N, regrid_pitch(K)) == 0) return 0;
-  if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_tiles_preferred(M, N, K) && !ragged_copy_first(M, N, K)) || !regrid_limits_ok(M, K)) return 0;
+  if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_route(M, N, K, false, true) != RaggedTile::kCopy && ragged_route(M, N, K, true, true) != RaggedTile::kCopy) || !regrid_limits_ok(M, K)) return 0;
   return regrid_bytes(M, K) + split;
 }
 
