@@ -1437,7 +1437,8 @@ int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
 //     14.1, 746 x 2053 -> 2555 13.7 | 11.9, 212 x 1481 -> 6574 11.5 | 10.2, 168 x 3495 -> 8678 level at 15.8; below, 64 x 64 are level
 //     or up to 12 % ahead (517 x 1000 -> 2051 7.8 | 8.0, 456 x 200 -> 3197 4.9 | 5.5);
 //   128 x 128, eight waves: 3931 x 2345 -> 881 24.7 | 16.9, 3819 x 1352 -> 998 19.1 | 12.3, 1989 x 375 -> 1580 9.3 | 7.2, 1019 x 1685 -> 2890
-//     15.3 | 13.8, 823 x 3208 -> 3743 21.6 | 19.7; beyond K = 3300 the copy, which floats want (275 x 3317 -> 7349 20.4 | 22.4); up to 288
+//     15.3 | 13.8, 823 x 3208 -> 3743 21.6 | 19.7; beyond K = 3300 the copy, which floats want (275 x 3317 -> 7349 20.4 | 22.4),
+//     up to 256 rows beyond K = 2000 (210 x 2773 -> 11089 17.3 | 18.4, 221 x 2102 -> 8984 14.0 | 14.7); up to 288
 //     tiles of 64 x 128 at K <= 640 64 x 64 (230 x 264 -> 9105 5.7 | 6.0), up to 370 at K <= 330 (837 x 312 -> 2930 5.8 | 6.2; 1550 x
 //     279 -> 2151, 425 of them, 7.6 | 6.7);
 //   128 x 256, eight waves: 1860 x 574 -> 3469 17.8 | 11.8, 4022 x 1928 -> 1556 28.2 | 21.7, 446 x 1309 -> 10760
@@ -1448,7 +1449,7 @@ int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
 // 10.7; K = 4100, N = 3900, M = 500 22.6 | 23.9; K = 3907, N = 193, M = 2889 13.6 | 25.3; K = 100, N = 1000, M = 8000 10.4 | 12.8; K = 120,
 // N = 8000, M = 4096 26.3 | 22.1).
 enum class RaggedTile { kCopy, k64, k64x128, k128, k128x256 };
-constexpr int64_t kRaggedLargeMaxTiles = 4096, kRaggedLargeMaxK = 4000, kRagged128MaxK = 3300;
+constexpr int64_t kRaggedLargeMaxTiles = 4096, kRaggedLargeMaxK = 4000, kRagged128MaxK = 3300, kRagged128FewRowsMaxK = 2000;
 RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
   if (K < 16 || K > 0x7fffff00) return RaggedTile::kCopy;
   if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return RaggedTile::kCopy;
@@ -1456,7 +1457,7 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
   const int64_t tiles = rows64 * ceil_div(N, 64), oblong = rows64 * ceil_div(N, 128);
   // (at least 96 rows and 384 channels: fewer are padding in the larger tiles, 9974 x 296 -> 289 8.1 | 8.5)
   if (tiles > 256 && tiles <= kRaggedLargeMaxTiles && M >= 96 && N >= 384 && K > 2 * kBK &&
-      K <= (oblong <= 256 ? kRaggedLargeMaxK : kRagged128MaxK)) {
+      K <= (oblong <= 256 ? kRaggedLargeMaxK : M > 256 ? kRagged128MaxK : kRagged128FewRowsMaxK)) {
     if (oblong <= 256) {
       if (K > (floats ? 1536 : 1200)) return RaggedTile::k64x128;
     } else if (rows128 * ceil_div(N, 128) <= 256) {
