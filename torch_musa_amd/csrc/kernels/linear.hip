@@ -1439,8 +1439,8 @@ int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
 //   128 x 128, eight waves: 3931 x 2345 -> 881 24.7 | 16.9, 3819 x 1352 -> 998 19.1 | 12.3, 1989 x 375 -> 1580 9.3 | 7.2, 1019 x 1685 -> 2890
 //     15.3 | 13.8, 823 x 3208 -> 3743 21.6 | 19.7; beyond K = 3300 the copy, which floats want (275 x 3317 -> 7349 20.4 | 22.4),
 //     up to 256 rows beyond K = 2000 (210 x 2773 -> 11089 17.3 | 18.4, 221 x 2102 -> 8984 14.0 | 14.7); up to 288
-//     tiles of 64 x 128 at K <= 640 64 x 64 (230 x 264 -> 9105 5.7 | 6.0), up to 370 at K <= 330 (837 x 312 -> 2930 5.8 | 6.2; 1550 x
-//     279 -> 2151, 425 of them, 7.6 | 6.7);
+//     tiles of 64 x 128 at K <= 640 64 x 64 (230 x 264 -> 9105 5.7 | 6.0), up to 370 at K <= 330 and of floats (837 x 312 -> 2930
+//     5.8 | 6.2, bf16 2764 x 417 -> 949 8.7 | 9.2; 1550 x 279 -> 2151, 425 of them, 7.6 | 6.7);
 //   128 x 256, eight waves: 1860 x 574 -> 3469 17.8 | 11.8, 4022 x 1928 -> 1556 28.2 | 21.7, 446 x 1309 -> 10760
 //     16.8 | 15.8; up to 700 tiles of 64 x 128 at K < 480 those (516 x 372 -> 7244 10.7 | 8.0, with 128 x 256 9.4);
 //   beyond one round of those 128 x 128 where the copy is not ahead, K = 250 ... 640 (1356 x 344 -> 7817 17.3 | 14.4, 3508 x 252 -> 4716
@@ -1461,7 +1461,7 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
     if (oblong <= 256) {
       if (K > (floats ? 1536 : 1200)) return RaggedTile::k64x128;
     } else if (rows128 * ceil_div(N, 128) <= 256) {
-      if (K > 640 || oblong > (K > 330 ? 288 : 370)) return RaggedTile::k128;
+      if (K > 640 || oblong > (K > 330 && !floats ? 288 : 370)) return RaggedTile::k128;
     } else if (rows128 * ceil_div(N, 256) <= 256) {
       return K >= 480 || oblong > 700 ? RaggedTile::k128x256 : RaggedTile::k64x128;
     } else if (K >= 250 && K <= 640) {
