@@ -102,10 +102,11 @@ int tmq_quantize_per_tensor_dev(const float* x, void* q, int64_t n,
                                 tmq_stream_t stream);
 /* The whole dynamic quantization on the device: min/max over x, the parameters
  * into *qparams (device memory), the codes into q.  One launch up to 2**26
- * elements (from 32768 on its workgroups exchange their ranges through the
- * workspace, which no other call may use meanwhile).  Where that is not possible -- a stream that is being
- * captured, whose launches run again with the same arguments, x off the 16-byte
- * or the workspace off the 16-byte grid, signed codes with TMQ_ROUND_FUSED -- one
+ * elements (beyond 32768 its workgroups exchange their ranges through the
+ * workspace, which no other call may use meanwhile: up to 98304 elements that costs
+ * time only).  Where that is not possible -- a stream that is being captured, whose
+ * launches run again with the same arguments, x off the 16-byte or the workspace
+ * off the 16-byte grid, signed codes with TMQ_ROUND_FUSED -- one
  * launch up to 98304 elements, two up to 2**25, else three.  `workspace` as for
  * tmq_minmax (unused, and may be NULL, up to 32768 elements).
  * rounding = TMQ_ROUND_PRODUCT: q = clamp(rne(fl(x * inv)) + zp), the same

@@ -96,9 +96,10 @@ __global__ __launch_bounds__(kDynTileThreads, S <= 64 ? 4 : 2) void linear_dynam
   for (int i = 0; i < R; ++i) take_four(held[i], mn, mx);
   block_range<WAVES>(mn, mx, s_range, t);
   if (tiles_m > 1 && tile_n == 0 && t == 0) put_range(range, tile_m, mn, mx);
-  for (;;) {
+  RangeView view(tiles_m);
+  for (int polls = range.polls;; polls = 0) {
     if (t < kWave) {
-      const int missing = tiles_m > 1 ? get_ranges(range, tiles_m, tile_m, mn, mx) : -1;
+      const int missing = tiles_m > 1 ? get_ranges(range, tiles_m, static_cast<int>(tile), polls, view, mn, mx) : -1;
       if (missing < 0) {
         double s;
         int32_t z;
@@ -117,16 +118,21 @@ __global__ __launch_bounds__(kDynTileThreads, S <= 64 ? 4 : 2) void linear_dynam
     // Those rows' block has not run yet, or not for this long: their range, read here.
     mn = __builtin_inff();
     mx = -__builtin_inff();
-    const int64_t first = static_cast<int64_t>(missing) * BM;
-    const int rows = static_cast<int>(a.M - first < BM ? a.M - first : BM);
+    const int64_t first = static_cast<int64_t>(missing) * BM, last = a.M - 1;
 #pragma unroll 1
-    for (int r = wave_u; r < rows; r += WAVES) {
-      const float* const row = x + (first + r) * ldx;
-#pragma unroll 1
-      for (int k = 4 * lane; k < K; k += 4 * kWave) take_four(reinterpret_cast<const FourFloats*>(row + (k + 4 <= K ? k : K - 4))->v, mn, mx);
+    for (int k = 4 * lane; k < K; k += 4 * kWave) {
+      v4f v[BM / WAVES];
+#pragma unroll
+      for (int j = 0; j < BM / WAVES; ++j) {  // (rows past M: the last one again)
+        const int64_t row = first + wave_u + j * WAVES;
+        v[j] = reinterpret_cast<const FourFloats*>(x + (row < last ? row : last) * ldx + (k + 4 <= K ? k : K - 4))->v;
+      }
+#pragma unroll
+      for (int j = 0; j < BM / WAVES; ++j) take_four(v[j], mn, mx);
     }
     block_range<WAVES>(mn, mx, s_range, t);
     if (t == 0) put_range(range, missing, mn, mx);
+    if (t < kWave) view.add(missing, mn, mx);
     __syncthreads();                         // (s_missing is written again)
   }
 

@@ -1308,6 +1308,7 @@ auto held_kernel(int held) {
 // The host takes the range of up to TMQ_HOST_PARTS_UP_TO values in parts, from as many blocks as it has words for: each
 // tells it its own, 1.5 us before any block knows all of them (with dequantize, against range pass and quantizer in two
 // launches: 874 x 2752 values 19.5 -> 16.4 us, 128 x 1024 level at 13.9, where the host's own work is the time).
+// polls: negative for as many as kRangePolls says.
 int launch_held(const HeldCall& c, int most_blocks, int polls, const RangeReport& report, uint64_t* parts, int32_t* parts_count,
                 hipStream_t s) {
   const bool rows = c.pitch != c.K;
@@ -1320,7 +1321,7 @@ int launch_held(const HeldCall& c, int most_blocks, int polls, const RangeReport
     if (h >= per_thread) held = h;
   const int32_t more = static_cast<int32_t>(per_thread > held ? per_thread - held : 0);
   const auto kernel = rows ? held_kernel<true, true>(held) : c.fused ? held_kernel<true, false>(held) : held_kernel<false, false>(held);
-  const RangeWords range{static_cast<v4u*>(c.workspace), next_range_tag(), polls};
+  const RangeWords range{static_cast<v4u*>(c.workspace), next_range_tag(), polls >= 0 ? polls : more > 0 ? 2 * kRangePolls : kRangePolls};
   if (parts != nullptr) *parts_count = static_cast<int32_t>(blocks);
   enqueue(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHeldThreads), 0, s, c.x, static_cast<uint32_t*>(c.q),
           static_cast<int32_t>(total), static_cast<int32_t>(rows ? c.K : 0), static_cast<int32_t>(rows ? c.pitch / 4 : 1),
@@ -1343,7 +1344,7 @@ int quantize_dynamic(const float* x, void* q, int64_t n, int q_signed, int reduc
   const HeldCall held{x, q, 1, n, n, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
   if (n > kHeldAbove && held_runs(held, s)) {
     const bool in_parts = parts != nullptr && n > TMQ_HOST_PARTS_ABOVE && n <= TMQ_HOST_PARTS_UP_TO;
-    return launch_held(held, in_parts ? TMQ_HOST_PARTS : kHeldBlocks, kRangePolls, in_parts ? RangeReport{nullptr, 0, 0} : report,
+    return launch_held(held, in_parts ? TMQ_HOST_PARTS : kHeldBlocks, -1, in_parts ? RangeReport{nullptr, 0, 0} : report,
                        in_parts ? parts : nullptr, parts_count, s);
   }
   if (n <= kDynRepeatMax) {
@@ -1452,7 +1453,7 @@ TMQ_EXPORT int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M,
   const int64_t n = M * K;
   const HeldCall held{x, q, M, K, pitch, q_signed, fused, reduce_range, qparams, workspace, workspace_bytes};
   if (n > kHeldAbove && held_runs(held, s))
-    return launch_held(held, kHeldBlocks, kRangePolls, RangeReport{nullptr, 0, 0}, nullptr, nullptr, s);
+    return launch_held(held, kHeldBlocks, -1, RangeReport{nullptr, 0, 0}, nullptr, nullptr, s);
   if (n <= kDynRepeatMax)
     return launch_dynamic_repeat(q_signed != 0, fused, M * (pitch / 4), s, x, static_cast<uint8_t*>(q), static_cast<int32_t>(n),
                                  static_cast<int32_t>(K), static_cast<int32_t>(pitch / 4), qmin, qmax, reduce_range, true,

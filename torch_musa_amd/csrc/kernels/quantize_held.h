@@ -40,6 +40,7 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     RangeWords range, int32_t more, uint32_t sign_flip, int qmin, int qmax, int reduce_range, tmq_qparams* __restrict__ out,
     RangeReport report, uint64_t* parts) {
   constexpr int kWaves = kHeldThreads / kWave;
+  constexpr int kRepairAhead = 4;
   constexpr int kAhead = H >= 16 ? 16 : 4;  // (of the words that are not held; only H = kHeldMost has any)
   __shared__ float s_range[2 * kWaves], s_inv, s_zp;
   __shared__ int s_missing;
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     }
   };
   // The range of a block's part, to where all blocks see it (and to the host).
-  const auto publish = [&](int block, float mn, float mx, uint64_t* part) {
+  const auto publish = [&](int block, float& mn, float& mx, uint64_t* part) {
     block_range<kWaves>(mn, mx, s_range, t);
     if (t == 0) {
       put_range(range, block, mn, mx);
@@ -126,9 +127,10 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
   publish(own, mn, mx, parts == nullptr ? nullptr : parts + own);
 
   // All ranges, and the parameters from them.
-  for (;;) {
+  RangeView view(blocks);
+  for (int polls = range.polls;; polls = 0) {
     if (t < kWave) {
-      const int missing = get_ranges(range, blocks, own, mn, mx);
+      const int missing = get_ranges(range, blocks, own, polls, view, mn, mx);
       if (missing < 0) {
         if (own == 0 && t == 0) report_range(report, mn, mx);
         double s;
@@ -154,12 +156,19 @@ __global__ __launch_bounds__(kHeldThreads) void dynamic_quantize_held_kernel(
     float b = -std::numeric_limits<float>::infinity();
     Place p = place(missing);
 #pragma unroll 1
-    for (int u = 0; u < H + more; ++u) {
-      take_four(load(p), a, b);
-      advance(p);
+    for (int u = 0; u < H + more; u += kRepairAhead) {  // (past the part's end: of another one, or the last word again)
+      v4f v[kRepairAhead];
+#pragma unroll
+      for (int j = 0; j < kRepairAhead; ++j) {
+        v[j] = load(p);
+        advance(p);
+      }
+#pragma unroll
+      for (int j = 0; j < kRepairAhead; ++j) take_four(v[j], a, b);
     }
     take_tail(missing, a, b);
     publish(missing, a, b, nullptr);
+    if (t < kWave) view.add(missing, a, b);
     __syncthreads();
   }
 
