@@ -40,3 +40,16 @@ def test_lines_between_128_x_128_and_128_x_256_tiles():
                             (1751, 2496, 5824, 19), (2613, 1792, 6800, 19), (3379, 1344, 7760, 19), (2798, 1536, 4160, 19),
                             (1234, 3440, 4992, 7), (1650, 2512, 8960, 7), (479, 9984, 2816, 19), (640, 8192, 4096, 7)):
         assert cabi.linear_kernel_choice(m, n, k, workspace=True)["kernel"] - 1 == kernel, (m, n, k)
+
+
+def test_split_along_k_where_the_ring_of_phases_would_run():
+    # (us, split | phases: 34.5 | 35.6, 26.2 | 32.1, 27.2 | 29.0, 35.7 | 40.6, 23.4 | 26.5; the others, split | lone tiles' ring: 28.4 | 21.1,
+    # 25.9 | 21.3, 27.2 | 23.3)
+    for m, n, k in ((128, 7038, 10960), (114, 4815, 10576), (119, 6172, 9056), (123, 7505, 13184), (128, 4200, 8240)):
+        assert cabi.linear_kernel_choice(m, n, k, workspace=True)["kernel"] - 1 == 13, (m, n, k)
+        assert cabi.linear_kernel_choice(m, n, k, workspace=False)["kernel"] - 1 == 21, (m, n, k)
+    for m, n, k in ((661, 1408, 8544), (478, 1152, 8736), (168, 4736, 8656)):
+        for workspace in (False, True):
+            assert cabi.linear_kernel_choice(m, n, k, workspace=workspace)["kernel"] - 1 == 2, (m, n, k)
+    # rows too far apart for the ring's copies: the split, as a workspace asks for
+    assert cabi.linear_kernel_choice(478, 1152, 8736, ldx=2 ** 23 + 16, workspace=True)["kernel"] - 1 == 13

@@ -890,15 +890,19 @@ SplitPlan plan_split_tiles(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
-// The plan the automatic choice follows: none for the rows that stream the
-// weights, and for 17 ... 64 rows only where the estimate above prefers it.
-// Not where one round holds the product in 64 x 64 tiles but not in tiles of 32 rows: the lone tiles' ring is ahead up to
+// Bytes and floats are not split where one round holds the product in 64 x 64 tiles but not in tiles of 32 rows: the lone tiles' ring is ahead up to
 // K = 10752, and beyond against more than 550 thousand outputs (us, split | ring, weights from memory: 661 x 8544 -> 1408 28.4 |
 // 21.1, 478 x 8736 -> 1152 25.9 | 21.3, 168 x 8656 -> 4736 27.2 | 23.3, 1110 x 11504 -> 794 33.7 | 27.2, 683 x 11872 -> 832 27.8 |
-// 28.8; 194 x 10976 -> 2560 23.2 | 26.0, 180 x 13024 -> 2752 26.8 | 34.7, 80 x 12896 -> 5632 27.0 | 31.0).
+// 28.8; 194 x 10976 -> 2560 23.2 | 26.0, 180 x 13024 -> 2752 26.8 | 34.7, 80 x 12896 -> 5632 27.0 | 31.0).  The split stays where
+// it would go to the ring of phases (split | phases | lone ring: 128 x 10960 -> 7038 34.5 | 35.6 | 35.9, 114 x 10576 -> 4815 26.2 |
+// 32.1 | 31.1, 119 x 9056 -> 6172 27.2 | 29.0 | 28.1, 123 x 13184 -> 7505 35.7 | 40.6 | 40.1, 128 x 8240 -> 4200 23.4 | 26.5 | 26.7).
 bool ring_ahead_of_split(int64_t M, int64_t N, int64_t K) {
-  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && ceil_div(M, 32) * ceil_div(N, 64) > 256 && (K < 10752 || M * N > 550000);
+  return ceil_div(M, 64) * ceil_div(N, 64) <= 256 && ceil_div(M, 32) * ceil_div(N, 64) > 256 && (K < 10752 || M * N > 550000) &&
+         !phased_ring_preferred(M, N, K);
 }
+
+// The plan the automatic choice follows: none for the rows that stream the
+// weights, and for 17 ... 64 rows only where the estimate above prefers it.
 SplitPlan plan_split(int64_t M, int64_t N, int64_t K) {
   if (M > kDecodeRowsAuto && M <= kDecodeMaxRows && small_rows_path(M, N, K, true) != SmallRows::kSplit)
     return SplitPlan{};
@@ -1237,7 +1241,7 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
   if (forced < 0 || forced == 13) {
     const SplitPlan p = forced == 13 ? plan_split_tiles(q.M, q.N, q.K) : plan_split(q.M, q.N, q.K);
     if (p.splits > 1 && q.workspace_bytes >= split_workspace_bytes(p, q.M) &&
-        (forced == 13 || q.mode == kOutAcc32 || !ring_ahead_of_split(q.M, q.N, q.K))) {
+        (forced == 13 || q.mode == kOutAcc32 || !dma_ok || !ring_ahead_of_split(q.M, q.N, q.K))) {
       c.cfg = 13;
       c.split = p;
       return c;
