@@ -291,14 +291,17 @@ int tmq_linear(const tmq_linear_desc* desc, tmq_stream_t stream);
  * single-launch kernel is ahead of that, and always when the split is pinned.  No counterpart in the reference: muDNN allocates its own scratch
  * through the InternalMemAlloc callback (torch_musa/csrc/aten/utils/Utils.cpp:79-153). */
 int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
-/* Everything the call can make use of as `workspace`: the above, and for
- * activations off the 16-byte grid (K no multiple of 16, or on_grid == 0: their
+/* Everything tmq_linear / tmq_linear_f32 make use of as `workspace`: the above
+ * where the automatic choice splits (tmq_linear_acc32 may where they do not), and
+ * for activations off the 16-byte grid (K no multiple of 16, or on_grid == 0: their
  * pointer or row pitch is none) room for a copy of the rows on it, which lets the
  * vector kernels run them.  Without it such products fall back to a byte-wise
- * kernel, a hundred times slower; up to 16 rows of 16 and more bytes need none. */
+ * kernel, a hundred times slower; up to 16 rows of 16 and more bytes need none,
+ * and for activations off the grid ask tmq_linear_rows_in_place first. */
 int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid);
-/* 1: rows off the grid need no copy for this size, the call is faster without the
- * room for one (which it uses where tmq_linear_scratch_bytes names it).  0: see there. */
+/* 1: rows off the grid, at most 2**23 bytes apart, need no copy for this size, and
+ * the call is faster without the room for one (which it uses where
+ * tmq_linear_scratch_bytes names it): attach no workspace.  0: see there. */
 int tmq_linear_rows_in_place(int64_t M, int64_t N, int64_t K);
 /* The split behind that figure: *splits runs of *stages k-stages (64 bytes of K
  * each), the last run taking everything that is left; *splits == 1: no split.
@@ -321,7 +324,8 @@ typedef struct tmq_linear_choice {
   int32_t splits;        /* runs of k-stages (1: no split along K) */
   int32_t split_stages;  /* k-stages per run */
   int64_t tiles;         /* tiles of the product (x splits for split K) */
-  int64_t blocks;        /* workgroups launched (the persistent kernel: fewer than tiles) */
+  int64_t blocks;        /* workgroups launched (fewer than tiles where one takes several: the persistent
+                            kernels, and tiles of 32 channels dealt in pairs) */
   int64_t k_stages;      /* 64-byte stages of K */
 } tmq_linear_choice;
 enum tmq_linear_output_kind { TMQ_LINEAR_OUT_BYTES = 0, TMQ_LINEAR_OUT_F32 = 1, TMQ_LINEAR_OUT_ACC32 = 2 };

@@ -53,3 +53,20 @@ def test_split_along_k_where_the_ring_of_phases_would_run():
             assert cabi.linear_kernel_choice(m, n, k, workspace=workspace)["kernel"] - 1 == 2, (m, n, k)
     # rows too far apart for the ring's copies: the split, as a workspace asks for
     assert cabi.linear_kernel_choice(478, 1152, 8736, ldx=2 ** 23 + 16, workspace=True)["kernel"] - 1 == 13
+
+
+def test_no_room_for_a_split_that_is_not_made():
+    rng = np.random.default_rng(11)
+    asked = spared = 0
+    for _ in range(20000):
+        m, n, k = int(2 ** rng.uniform(4, 12)), int(2 ** rng.uniform(4, 14)), 16 * int(2 ** rng.uniform(6, 10))
+        plan = cabi.lib().tmq_linear_workspace_bytes(m, n, k)
+        uses = any(cabi.linear_kernel_choice(m, n, k, out=out, workspace=True)["kernel"] !=
+                   cabi.linear_kernel_choice(m, n, k, out=out, workspace=False)["kernel"] for out in ("bytes", "f32"))
+        assert cabi.lib().tmq_linear_scratch_bytes(m, n, k, 1) == (plan if uses else 0), (m, n, k)
+        assert not uses or plan > 0
+        asked, spared = asked + uses, spared + (plan > 0 and not uses)
+    assert asked > 100 and spared > 100, (asked, spared)
+    # (15.4 and 11.2 MB that nothing read)
+    for m, n, k in ((478, 1152, 8736), (661, 1408, 8544)):
+        assert cabi.lib().tmq_linear_workspace_bytes(m, n, k) > 11 * 10 ** 6 and cabi.lib().tmq_linear_scratch_bytes(m, n, k, 1) == 0

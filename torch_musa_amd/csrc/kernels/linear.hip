@@ -1673,10 +1673,35 @@ TMQ_EXPORT int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return split_workspace_bytes(plan_split(M, N, K), M);
 }
 
+namespace tmq {
+namespace {
+
+// Bytes of a split along K that products of bytes or floats on the grid make use of: none where the automatic choice is the
+// same kernel with and without them (the plan is there for pinned kernels and raw accumulators).
+int64_t split_bytes_used(int64_t M, int64_t N, int64_t K) {
+  LinearQuery q;
+  q.M = M;
+  q.N = N;
+  q.K = q.ldx = K;
+  q.vec_ok = q.workspace_attached = true;
+  q.workspace_bytes = split_workspace_bytes(plan_split(M, N, K), M);
+  if (q.workspace_bytes == 0) return 0;
+  for (const int mode : {kOutU8, kOutF32}) {
+    q.mode = mode;
+    LinearQuery without = q;
+    without.workspace_attached = false;
+    without.workspace_bytes = 0;
+    if (choose_linear(q, -1).cfg != choose_linear(without, -1).cfg) return q.workspace_bytes;
+  }
+  return 0;
+}
+
+}  // namespace
+}  // namespace tmq
+
 TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  // (the plan of a split along K is there for pinned kernels where the automatic choice is another one)
-  const int64_t split = wloop_tile(M, N, regrid_pitch(K)) != 0 ? 0 : tmq_linear_workspace_bytes(M, N, regrid_pitch(K));
+  const int64_t split = split_bytes_used(M, N, regrid_pitch(K));
   if (K % 16 == 0 && on_grid) return split;
   if (wloop_ragged_tile(M, N, K) != 0 && wloop_tile(M, N, regrid_pitch(K)) == 0) return 0;
   if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_route(M, N, K, false, true) != RaggedTile::kCopy && ragged_route(M, N, K, true, true) != RaggedTile::kCopy) || !regrid_limits_ok(M, K)) return 0;
