@@ -69,9 +69,9 @@ def test_dynamic_range_report_by_each_pass(n, offset, dtype):
         torch.quantize_per_tensor_dynamic(xg.fill_(float("nan")), dtype, False)
 
 
-@pytest.mark.parametrize("n,offset", [(1, 0), (65537, 0), (98304, 0),            # by the one launch
-                                      (98305, 0), (200003, 0), (1 << 21, 0),     # by the range pass's last block
-                                      ((1 << 21) + 1, 0), (98305, 1)])
+@pytest.mark.parametrize("n,offset", [(1, 0), (65537, 0), (98304, 0),            # by the one launch, from 32769 on by its first block once it has
+                                      (98305, 0), (200003, 0), (1 << 21, 0),     # all ranges
+                                      ((1 << 21) + 1, 0), (98305, 1)])           # (off the grid: by the launch behind the range pass)
 def test_range_reported_as_a_whole(n, offset):
     """The C entry point whose range comes in one piece at every size."""
     x = torch.randn(n, generator=torch.Generator().manual_seed(n)) * 2
@@ -79,7 +79,7 @@ def test_range_reported_as_a_whole(n, offset):
     xg = torch.empty(n + offset, device="cuda")[offset:].copy_(x.cuda())
     want = torch.quantize_per_tensor_dynamic(x, torch.quint8, False)
     report = torch.zeros(2, dtype=torch.int64).pin_memory()
-    for ticket in (7, 8):     # the block count of the slot is ready for the next call
+    for ticket in (7, 8):     # the slot is ready for the next call
         q, qp = cabi.quantize_per_tensor_dynamic_report(xg, False, False, report, ticket, 63)
         torch.cuda.synchronize()
         assert [w >> 32 for w in report.tolist()] == [ticket, ticket]

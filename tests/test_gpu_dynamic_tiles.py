@@ -1,11 +1,14 @@
 """quantized::linear_dynamic of more than 16 rows in one launch: rows, channels and K at the edges of tiles and of the waves' shares,
-blocks that wait for the others' ranges and blocks that find them themselves, against the launches it replaces."""
+blocks that wait for the others' ranges and blocks that find them themselves, against the oracle and the launches that quantize the
+rows first (which exchange ranges themselves above 32768 values)."""
 import ctypes as C
 
+import numpy as np
 import pytest
 import torch
 
-from gpu_util import say
+import oracle
+from gpu_util import dev, host, say
 from torch_musa_amd import cabi
 
 
@@ -44,6 +47,25 @@ def test_edges(m, n, k):
         assert status == 0
         assert torch.equal(y[:, :n], want), polls
         assert bool((y[:, n:] == 77).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(17, 33, 2048), (33, 70, 1026), (64, 65, 515), (257, 70, 1024), (97, 129, 2047), (1100, 40, 256),
+                                   (4100, 64, 19), (2000, 250, 100)])
+def test_against_the_oracle(m, n, k):
+    say("dynamic tiles, oracle", m, n, k)
+    rng = np.random.default_rng(m * n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32) + np.float32(0.3)
+    x[m - 1, k - 1], x[m // 2, 0] = 9.0, -7.0
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    scales = (rng.random(n) * 1e-3 + 1e-4).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32) if k % 3 else None
+    want = oracle.linear_dynamic(x, w, scales.astype(np.float64), bias, bool(m & 1), bool(k & 1))
+    pw, xd, sd, bd = cabi.PackedLinear(dev(w)), dev(x), dev(scales), None if bias is None else dev(bias)
+    for polls in (-1, 0):
+        status, y = _call(xd, pw, sd, bd, m & 1, k & 1, polls, 0)
+        assert status == 0
+        np.testing.assert_array_equal(host(y)[:, :n], want)
 
 
 @pytest.mark.gpu

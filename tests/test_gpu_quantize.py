@@ -335,10 +335,10 @@ def test_qadaptive_avgpool_resnet_head_sized(cabi):
                                       (1 << 20, 0), ((1 << 20) + 3, 1), ((1 << 23) + 1029, 0), ((1 << 25) + 4, 0)])
 @pytest.mark.parametrize("signed,reduce_range", [(False, False), (False, True), (True, False)])
 def test_quantize_dynamic_on_device(cabi, n, offset, signed, reduce_range):
-    # one call: range, parameters (left in device memory) and codes; small inputs take the
-    # single-block kernel, aligned ones of up to 2**25 elements two launches (the quantizer's
-    # blocks finish the reduction; 2**23 + 1029 walks its grid-stride loop more than once and
-    # ends inside a chunk), larger or unaligned ones the three-launch chain -- same results
+    # one call: range, parameters (left in device memory) and codes; up to 32768 elements the
+    # launch whose blocks read everything, aligned ones beyond the launch whose blocks exchange
+    # their ranges, unaligned ones the three-launch chain -- same results
+    # (test_gpu_range_launches.py has the launches of streams that are captured)
     say("dynamic dev", n, offset, signed, reduce_range)
     rng = np.random.default_rng(n + offset)
     x = (rng.standard_normal(n + offset) * 2.5 + 0.4).astype(np.float32)
