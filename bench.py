@@ -15,7 +15,10 @@ resident in HBM.  The last line of stdout is one JSON object:
                    model, the scalar C oracle port and the other configurations
   secondary        the other benchmark configurations: quantize / dequantize / min-max
                    over 2**28 fp32 (HBM bound), decode-shaped linear (weight
-                   read bound), conv2d NHWC
+                   read bound), conv2d NHWC: their times and rates, so that the
+                   line stays short enough for whoever keeps the end of an
+                   output; --details FILE has all of each (methods, byte and
+                   operation counts, rooflines, layer tables)
 
 Everything here is synthetic data of the benchmark shapes and distributions
 ("N(0,s)" read as standard deviation s).
@@ -161,6 +164,12 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
+def in_short(figures):
+    """The times and rates of a secondary configuration, without its counts, method and tables."""
+    return {k: v for k, v in figures.items()
+            if k in ("value", "unit", "torch_int_mm_us") or k.endswith(("launch_us", "call_us", "total_us", "kernel_us"))}
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -168,6 +177,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=50)
     ap.add_argument("--skip-secondary", action="store_true")
     ap.add_argument("--skip-cpu", action="store_true")
+    ap.add_argument("--details", metavar="FILE", help="write the same object there with all of `secondary`")
     ap.add_argument("--no-power", action="store_true",
                     help="do not start the child process that samples the socket power (for runs under a profiler, "
                          "whose library has initialised the GPU before this program starts)")
@@ -1514,6 +1524,10 @@ def main():
         "device": torch.cuda.get_device_name(0),
     }
     stop_power_sampler()
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f)
+    out["secondary"] = {name: in_short(figures) for name, figures in secondary.items()}
     print(json.dumps(out))
 
 
