@@ -512,8 +512,9 @@ struct PackedLinearWeightTmq final : public LinearPackedParamsBase {
   }
   // The reference declares these and throws (mudnn/Linear.h:35-46).  Here:
   // min/max -> qparams -> quint8 activations -> int8 product -> fp32 output on
-  // the current stream (one launch where a kernel does all of it, two otherwise, three past 2^26 values; a
-  // captured stream up to four), the parameters never visit the host.
+  // the current stream (one launch where a kernel does all of it; else the codes, in one launch, two where ranges are
+  // not exchanged and three for dense rows past 2^26 or, captured, 2^25 values, and the product, two where it is split
+  // along K), the parameters never visit the host.
   at::Tensor apply_dynamic(at::Tensor input, bool reduce_range) override {
     return apply_dynamic_impl(input, reduce_range, false);
   }

@@ -1,5 +1,6 @@
 // int8 MFMA GEMM on 64 x 64 tiles for a few hundred rows against 2048 < K <= 4096
-// (gfx950): eight waves split K, the weights go through registers, the activations
+// (gfx950), raw accumulators unless it is pinned (bytes and floats have the lone tiles' ring of
+// six stages, linear.hip): eight waves split K, the weights go through registers, the activations
 // through a ring in LDS that belongs to the wave.
 //
 // What bounds these shapes is what a CU can pull from the L2s (about 45 bytes per

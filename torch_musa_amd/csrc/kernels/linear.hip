@@ -828,6 +828,8 @@ int wloop_tile(int64_t M, int64_t N, int64_t K) {
   return ceil_div(M, 32) * ceil_div(N, 64) <= 256 && !(ring && N * K > int64_t{32} << 20) ? 64 : 0;
 }
 
+// (`tiles` beyond K = 1024 prices one round as two wave groups and the ring of phases: the lone tiles' ring that runs now is
+// up to a tenth faster, and the kernel in pieces is not priced here at all)
 SmallRows small_rows_path(int64_t M, int64_t N, int64_t K, bool workspace) {
   // Where the tiles of 32 rows with the weights through registers fit, they are measured directly against the
   // weight-streaming kernel, which keeps K > 3008 up to 32 rows (two row groups) while its blocks fit one round (us, tiles |
@@ -1348,13 +1350,14 @@ LinearChoice choose_linear(const LinearQuery& q, int forced) {
       // M = 256 14.3 -> 13.6 us; N = 2048: M = 512 14.0 -> 13.0 us; K = 3072: M = 192
       // 13.0 -> 12.1 us; behind the two wave groups at K = 2560 (12.3 against 11.7 us) and
       // against 32 MB of weights, N = 8192: 15.3 against 14.6 us; 24 MB, N = 6144, K = 4096,
-      // M = 128: 13.7 against 15.0 us)
+      // M = 128: 13.7 against 15.0 us).  Raw accumulators; lone_ring_first takes bytes and floats
       cfg = 27;
     else if (onepass_ok && phased_ring_preferred(M, N, K))
       cfg = 21;
     else if (nblk(64, 64) <= 256 && ceil_div(K, kBK) >= 32 && ceil_div(K, kBK) % 2 == 0)
       cfg = 14;  // at most one block per CU and a long k loop: two wave groups halve it (14.7 -> 11.7 us
-                 // at M = 128, K = N = 4096; four groups run into the L2's bandwidth: 12.3 us)
+                 // at M = 128, K = N = 4096; four groups run into the L2's bandwidth: 12.3 us); raw
+                 // accumulators here and below, lone_ring_first takes bytes and floats
     else {
       cfg = 2;
       c.groups = two_wave_groups_fit(M, N, K) ? 2 : 1;  // (an odd number of stages, or a shorter loop)
@@ -1926,9 +1929,13 @@ TMQ_EXPORT int tmq_linear_f32(const tmq_linear_desc* d, const tmq_qparams* x_qpa
 }
 
 // The float rows of the one-launch dynamic linear as the resident kernel holds them: 16 waves x 64 lanes x up to 16 groups of
-// four values.  More than 8 groups only against many channels, whose stream is what the block's work on the rows passes under
-// (us, two launches | one: 16 x 4096 -> 11008 14.2 | 13.7, 10 x 4096 -> 11008 13.85 | 13.1, 12 x 3072 -> 11008 12.5 | 11.9, 16 x 2560
-// -> 11008 11.7 | 11.55; -> 8192 0.95 to 1.03 of the time, 16 x 4096 -> 4096 9.5 | 10.6, -> 256 8.15 | 9.2).
+// four values.  More than 8 groups only against many channels, whose stream is what the block's work on the rows passes under.
+// One launch over two, each queued behind the one before, of 16 x 2560, 9 x 4096, 16 x 4096, 12 x 5120, 8 x 8192, 5 x 8192 and 14 x 3000,
+// whose rows are off the 16-byte grid: N = 4096 0.97, 0.97, 1.06, 0.94, 1.01, 1.00, 0.91; 6144 0.95, 0.95, 0.97, 0.94, 0.92, 0.96, 0.87;
+// 8192 0.91, 1.04, 0.95, 0.95, 0.99, 1.04, 0.87; 10240 0.90, 0.92, 0.92, 0.93, 0.95, 0.94, 0.84; 12288 0.92, 0.93, 0.94, 0.94, 0.99, 0.96,
+// 0.85; 16384 0.96, 0.96, 0.95, 0.97, 0.96, 0.95, 0.84; 24576 0.97, 1.00, 0.98, 0.96, 0.95, 0.95, 0.78 (16 x 4096 -> 10240 15.3 | 14.0 us).
+// From 10240 on never behind, below by up to 6 %; the line follows N, not the weights' bytes (5 x 8192 -> 8192, 64 Mi: 1.04; 16 x 2560 ->
+// 10240, 25 Mi: 0.90).
 constexpr int64_t kDynResidentMaxValues = 32768, kDynResidentMostValues = 65536, kDynResidentManyChannels = 10240;
 
 namespace {

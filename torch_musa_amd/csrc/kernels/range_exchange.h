@@ -34,7 +34,8 @@ constexpr int kRangeParts = 256;  // at most
 // 160 us: 4 looks 61, 8 55, 16 58, 32 66 us).
 constexpr int kRangePolls = 16;
 
-// What no other launch of this process has (a permutation of a counter; its start differs from process to process).
+// What no other launch of this process has: SplitMix64 (Steele, Lea and Flood, "Fast splittable pseudorandom number generators"),
+// whose output is a permutation of its counter; the counter's start differs from process to process.
 inline uint64_t next_range_tag() {
   static std::atomic<uint64_t> count{static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
   uint64_t z = count.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;
