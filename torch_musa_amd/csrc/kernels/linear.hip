@@ -1001,6 +1001,7 @@ int run_split(const GemmArgs& a, const XLinear& xs, const SplitPlan& p, void* wo
   GemmArgs part = a;  // first kernel: pure sums of (x ^ flip) * w, no zero-point term
   part.acc_coef = 0;
   part.acc_base = 0;
+  part.f_kind = TMQ_FLOAT_F32;  // (32-bit words whatever kind of float the second kernel writes)
   part.x_qp_dev = nullptr;
   part.y = workspace;
   part.ldy = p.ldp;
