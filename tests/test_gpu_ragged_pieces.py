@@ -63,3 +63,32 @@ def test_route():
     for m, n, k, one in ((16, 64, 1001, 0), (17, 64, 1001, 1), (17, 64, 127, 0), (17, 64, 129, 1), (512, 1024, 1000, 1),
                          (513, 1024, 1000, 0), (64, 64, 12287, 1), (64, 64, 12289, 0), (0, 64, 1001, 0)):
         assert _in_place(cabi, m, n, k) == one, (m, n, k)
+
+
+FEW_ROWS = [(17, 2600, 6001, 1), (24, 64, 8001, 1), (24, 1000, 11001, 1), (24, 300, 7001, 1), (28, 2600, 10002, 1),
+            (29, 2600, 6001, 0), (25, 300, 7001, 0), (24, 2600, 5631, 0), (24, 64, 8193, 0), (24, 300, 10002, 0), (24, 2600, 8004, 0), (17, 17, 12001, 0)]
+
+
+def test_few_long_rows_are_copied_first():
+    from torch_musa_amd import cabi
+    for m, n, k, copied in FEW_ROWS:
+        assert _in_place(cabi, m, n, k) == 1 - copied, (m, n, k)
+        room = cabi.lib().tmq_linear_scratch_bytes(m, n, k, 0)
+        assert room == (-(-(m * (-(-k // 16) * 16)) // 256) * 256 if copied else 0), (m, n, k, room)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [s[:3] for s in FEW_ROWS[:5]])
+def test_few_long_rows(cabi, m, n, k):  # noqa: F811
+    """With the room for a copy and, read where they lie, without: the plain kernel's bytes."""
+    say("few long rows", m, n, k)
+    c = _tile_case(m, n, k, seed=m + n + k, x_signed=bool(m & 1), relu=False, bias=True, per_channel=True)
+    want, _, _ = _run(cabi, c, 9)
+    got, _, _ = _run(cabi, c, -1)
+    np.testing.assert_array_equal(got, want)
+    keep, cabi.linear_workspace = cabi.linear_workspace, torch.empty(cabi.lib().tmq_linear_scratch_bytes(m, n, k, 0), dtype=torch.uint8, device="cuda")
+    try:
+        got, _, _ = _run(cabi, c, -1)
+    finally:
+        cabi.linear_workspace = keep
+    np.testing.assert_array_equal(got, want)

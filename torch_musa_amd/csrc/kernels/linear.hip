@@ -1434,6 +1434,22 @@ int wloop_ragged_tile(int64_t M, int64_t N, int64_t K) {
   return K > kWloopRaggedShortK && ceil_div(M, 32) * ceil_div(N, 32) <= 256 ? 32 : 64;
 }
 
+// ... but for rows that the streaming kernel takes on the grid: a copy in front of that is ahead, if there is room for it, where rows
+// off the 4-byte grid, whose requests cost twice as much, are long and the weights many (an operator's call after the other, us, in
+// place | copied: 24 x 8001 -> 2600 15.7 | 13.0, 17 x 6001 -> 2600 11.1 | 9.8, 24 x 11001 -> 1000 18.0 | 14.4, 24 x 12001 -> 4000 22.1 |
+// 18.9, 28 x 10001 -> 2600 18.5 | 16.7; at odd lengths up to 8192 of few weights as well, 24 x 8001 -> 64 12.8 | 11.2, 22 x 7929 -> 37 12.6 |
+// 10.4, 20 x 7001 -> 300 11.6 | 10.4, 17 x 8001 -> 17 10.4 | 10.2).  The other side: 28 x 7001 -> 1000 11.6 | 12.1; on the device 24 x 5001 ->
+// 2600 11.1 | 11.4, 32 x 10001 -> 2600 19.0 | 18.5, 32 x 8001 -> 64 12.8 | 13.9, 24 x 9001 -> 1000 14.2 | 15.1, 24 x 10002 -> 300 13.9 |
+// 14.6, and rows on the 4-byte grid, 20 x 5784 -> 51 7.7 | 10.0, 25 x 10116 -> 287 10.7 | 15.4, 22 x 10156 -> 2618 15.4 | 16.5.
+constexpr int64_t kFewRowsCopied = 28, kFewRowsCopiedMinK = 5632, kFewerRowsCopied = 24, kFewerRowsCopiedMaxK = 8192;
+bool few_rows_copied(int64_t M, int64_t N, int64_t K) {
+  return M > kDecodeRowsAuto && M <= kFewRowsCopied && K > kFewRowsCopiedMinK && K % 4 != 0 &&
+         (N * K > int64_t{10} << 20 || (K % 2 != 0 && K <= kFewerRowsCopiedMaxK && M <= kFewerRowsCopied)) &&
+         small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream;
+}
+// Whether a copy, if there is room for it, comes before the tiles that wloop_ragged_tile names.
+bool wloop_ragged_copied(int64_t M, int64_t N, int64_t K) { return wloop_tile(M, N, regrid_pitch(K)) != 0 || few_rows_copied(M, N, K); }
+
 // More than that: tiles that read the rows where they lie, or a copy onto the grid and the padded shape's own kernel.  The copy is a
 // launch (2.2 us and a scratch allocation).
 //
@@ -1517,7 +1533,7 @@ int dispatch_linear(const GemmArgs& a, const XLinear& xs, int x_signed, bool vec
     const bool copy_ok = regrid_limits_ok(a.M, a.K) && q.workspace_bytes >= room;
     const bool zero_padded = a.w_kchunks == packed_kchunks(a.K);
     if (const int tile = wloop_ragged_tile(a.M, a.N, a.K); tile != 0 && zero_padded && xs.ldx <= (int64_t{1} << 23) &&
-        a.N + a.n_off < (int64_t{1} << 29) && !(copy_ok && wloop_tile(a.M, a.N, regrid_pitch(a.K)) != 0))
+        a.N + a.n_off < (int64_t{1} << 29) && !(copy_ok && wloop_ragged_copied(a.M, a.N, a.K)))
       return launch_gemm_wloop_ragged<MODE>(a, xs, tile == 64, s);
     const XLinearRagged rows{xs.x, xs.ldx};
     switch (zero_padded ? ragged_route(a.M, a.N, a.K, MODE == kOutF32, copy_ok) : RaggedTile::kCopy) {
@@ -1705,15 +1721,14 @@ int64_t split_bytes_used(int64_t M, int64_t N, int64_t K) {
 
 TMQ_EXPORT int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int64_t split = split_bytes_used(M, N, regrid_pitch(K));
-  if (K % 16 == 0 && on_grid) return split;
-  if (wloop_ragged_tile(M, N, K) != 0 && wloop_tile(M, N, regrid_pitch(K)) == 0) return 0;
+  if (K % 16 == 0 && on_grid) return split_bytes_used(M, N, K);
+  if (wloop_ragged_tile(M, N, K) != 0 && !wloop_ragged_copied(M, N, K)) return 0;
   if ((M <= kDecodeRowsAuto && K >= 16) || (ragged_route(M, N, K, false, true) != RaggedTile::kCopy && ragged_route(M, N, K, true, true) != RaggedTile::kCopy) || !regrid_limits_ok(M, K)) return 0;
-  return regrid_bytes(M, K) + split;
+  return regrid_bytes(M, K) + split_bytes_used(M, N, regrid_pitch(K));
 }
 
 TMQ_EXPORT int tmq_linear_rows_in_place(int64_t M, int64_t N, int64_t K) {
-  return M > 0 && N > 0 && wloop_ragged_tile(M, N, K) != 0 ? 1 : 0;
+  return M > 0 && N > 0 && wloop_ragged_tile(M, N, K) != 0 && !few_rows_copied(M, N, K) ? 1 : 0;
 }
 
 TMQ_EXPORT int tmq_linear_split_plan(int64_t M, int64_t N, int64_t K, int32_t* splits, int32_t* stages) {
