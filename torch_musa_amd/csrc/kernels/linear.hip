@@ -1466,7 +1466,10 @@ bool wloop_ragged_copied(int64_t M, int64_t N, int64_t K) { return wloop_tile(M,
 //     tiles of 64 x 128 at K <= 640 64 x 64 (230 x 264 -> 9105 5.7 | 6.0), up to 370 at K <= 330 and of floats (837 x 312 -> 2930
 //     5.8 | 6.2, bf16 2764 x 417 -> 949 8.7 | 9.2; 1550 x 279 -> 2151, 425 of them, 7.6 | 6.7);
 //   128 x 256, eight waves: 1860 x 574 -> 3469 17.8 | 11.8, 4022 x 1928 -> 1556 28.2 | 21.7, 446 x 1309 -> 10760
-//     16.8 | 15.8; up to 700 tiles of 64 x 128 at K < 480 those (516 x 372 -> 7244 10.7 | 8.0, with 128 x 256 9.4);
+//     16.8 | 15.8; up to 700 tiles of 64 x 128 at K < 480 those (516 x 372 -> 7244 10.7 | 8.0, with 128 x 256 9.4); up to 512 rows beyond
+//     K = 2000 the copy, whose time follows the rows (copied | 128 x 256: 264 x 2227 -> 12681 23.7 | 25.6, 399 x 2179 -> 12067 24.5 | 26.2,
+//     471 x 3206 -> 8959 32.3 | 36.0, 500 x 2302 -> 11735 26.4 | 28.9, 499 x 2209 -> 11550 level, 494 x 3272 -> 15876 38.8 | 39.2; the other
+//     side 449 x 1113 -> 11446 18.2 | 17.0, 566 x 2942 -> 10913 34.0 | 32.5, 654 x 3138 -> 6707 31.4 | 32.5);
 //   beyond one round of those 128 x 128 where the copy is not ahead, K = 250 ... 640 (1356 x 344 -> 7817 17.3 | 14.4, 3508 x 252 -> 4716
 //     20.4 | 17.2; 1258 x 333 -> 9024 12.9 | 13.4; 7202 x 245 -> 1879 15.9 | 16.7, 2759 x 2023 -> 3364 34.9 | 38.1).
 // Elsewhere 64 x 64 up to 512 tiles, later where K is short, beyond that the copy (direct | copy: K = 2051, N = 1000, M = 517 9.3 |
@@ -1479,12 +1482,13 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
   if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return RaggedTile::kCopy;
   const int64_t rows64 = ceil_div(M, 64), rows128 = ceil_div(M, 128);
   const int64_t tiles = rows64 * ceil_div(N, 64), oblong = rows64 * ceil_div(N, 128);
+  const bool one128 = rows128 * ceil_div(N, 128) <= 256;
   // (at least 96 rows and 384 channels: fewer are padding in the larger tiles, 9974 x 296 -> 289 8.1 | 8.5)
   if (tiles > 256 && tiles <= kRaggedLargeMaxTiles && M >= 96 && N >= 384 && K > 2 * kBK &&
-      K <= (oblong <= 256 ? kRaggedLargeMaxK : M > 256 ? kRagged128MaxK : kRagged128FewRowsMaxK)) {
+      K <= (oblong <= 256 ? kRaggedLargeMaxK : M > (one128 ? 256 : 512) ? kRagged128MaxK : kRagged128FewRowsMaxK)) {
     if (oblong <= 256) {
       if (K > (floats ? 1536 : 1200)) return RaggedTile::k64x128;
-    } else if (rows128 * ceil_div(N, 128) <= 256) {
+    } else if (one128) {
       if (K > 640 || oblong > (K > 330 && !floats ? 288 : 370)) return RaggedTile::k128;
     } else if (rows128 * ceil_div(N, 256) <= 256) {
       return K >= 480 || oblong > 700 ? RaggedTile::k128x256 : RaggedTile::k64x128;
