@@ -51,6 +51,7 @@ def test_room_for_a_copy():
     for m, n, k, copies in ((1025, 1030, 1201, 0), (1025, 2049, 1000, 0), (1152, 2048, 639, 0), (2049, 2049, 1001, 0), (2113, 4097, 400, 0),
                             (2113, 4097, 1000, 1), (2113, 4097, 200, 1), (1025, 1030, 4001, 1), (2049, 2049, 3301, 1), (1025, 2049, 3301, 1), (256, 9000, 2001, 1), (256, 9000, 1999, 0),
                             (512, 11000, 2001, 1), (512, 11000, 1999, 0), (513, 11000, 2001, 0), (512, 8192, 2001, 0), (512, 8193, 2001, 1),
+                            (2034, 6687, 637, 1), (2034, 6687, 399, 0), (2034, 6401, 401, 1), (2034, 6400, 401, 0),
                            
                             (17000, 65, 1001, 1), (17000, 65, 701, 0)):
         assert (cabi.lib().tmq_linear_scratch_bytes(m, n, k, 0) > 0) == bool(copies), (m, n, k)

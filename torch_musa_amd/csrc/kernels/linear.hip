@@ -1471,7 +1471,12 @@ bool wloop_ragged_copied(int64_t M, int64_t N, int64_t K) { return wloop_tile(M,
 //     471 x 3206 -> 8959 32.3 | 36.0, 500 x 2302 -> 11735 26.4 | 28.9, 499 x 2209 -> 11550 level, 494 x 3272 -> 15876 38.8 | 39.2; the other
 //     side 449 x 1113 -> 11446 18.2 | 17.0, 566 x 2942 -> 10913 34.0 | 32.5, 654 x 3138 -> 6707 31.4 | 32.5);
 //   beyond one round of those 128 x 128 where the copy is not ahead, K = 250 ... 640 (1356 x 344 -> 7817 17.3 | 14.4, 3508 x 252 -> 4716
-//     20.4 | 17.2; 1258 x 333 -> 9024 12.9 | 13.4; 7202 x 245 -> 1879 15.9 | 16.7, 2759 x 2023 -> 3364 34.9 | 38.1).
+//     20.4 | 17.2; 1258 x 333 -> 9024 12.9 | 13.4; 7202 x 245 -> 1879 15.9 | 16.7, 2759 x 2023 -> 3364 34.9 | 38.1), of bytes beyond
+//     K = 400 only up to 200 tiles of 256 x 256, which on the grid fill a round from there on (their tiles: 216, 2034 x 637 -> 6687 22.1 |
+//     25.8; 216, 897 x 577 -> 13709 20.8 | 23.3; 220, 2546 x 635 -> 5628 22.4 | 25.1; 240, 3014 x 405 -> 4927 19.1 | 20.6; 245, 1655 x 537 ->
+//     8955 22.5 | 25.3; 280, 1037 x 421 -> 14325 18.7 | 21.7; the mean of 26 drawn ones 1.05; the other side: 204, 1356 x 561 -> 8586 21.0 |
+//     19.5; 215, 1151 x 504 -> 10801 19.6 | 17.4; 152, 965 x 332 -> 9627 17.7 | 14.6; 168, 1963 x 522 -> 5352 20.4 | 17.6; floats 0.59 to 0.89
+//     but for 3293 x 324 -> 2880 1.06).
 // Elsewhere 64 x 64 up to 512 tiles, later where K is short, beyond that the copy (direct | copy: K = 2051, N = 1000, M = 517 9.3 |
 // 10.7; K = 4100, N = 3900, M = 500 22.6 | 23.9; K = 3907, N = 193, M = 2889 13.6 | 25.3; K = 100, N = 1000, M = 8000 10.4 | 12.8; K = 120,
 // N = 8000, M = 4096 26.3 | 22.1).
@@ -1492,7 +1497,7 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
       if (K > 640 || oblong > (K > 330 && !floats ? 288 : 370)) return RaggedTile::k128;
     } else if (rows128 * ceil_div(N, 256) <= 256) {
       return K >= 480 || oblong > 700 ? RaggedTile::k128x256 : RaggedTile::k64x128;
-    } else if (K >= 250 && K <= 640) {
+    } else if (K >= 250 && K <= 640 && (floats || K <= 400 || ceil_div(M, 256) * ceil_div(N, 256) <= 200)) {
       return RaggedTile::k128;
     }
   }
