@@ -300,8 +300,9 @@ int64_t tmq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * and for activations off the grid ask tmq_linear_rows_in_place first. */
 int64_t tmq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int on_grid);
 /* 1: rows off the grid, at most 2**23 bytes apart, need no copy for this size, and
- * the call is faster without the room for one (which it uses where
- * tmq_linear_scratch_bytes names it): attach no workspace.  0: see there. */
+ * the call is as fast or faster without the room for one (which it uses where
+ * tmq_linear_scratch_bytes names it), a few per cent behind at odd K beyond 8000:
+ * attach no workspace.  0: see there. */
 int tmq_linear_rows_in_place(int64_t M, int64_t N, int64_t K);
 /* The split behind that figure: *splits runs of *stages k-stages (64 bytes of K
  * each), the last run taking everything that is left; *splits == 1: no split.

@@ -55,3 +55,22 @@ def test_room_for_a_copy():
                            
                             (17000, 65, 1001, 1), (17000, 65, 701, 0)):
         assert (cabi.lib().tmq_linear_scratch_bytes(m, n, k, 0) > 0) == bool(copies), (m, n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(300, 11010, 2003), (1290, 10505, 405)])
+def test_copied_where_there_is_room(cabi, m, n, k):  # noqa: F811
+    """The same bytes as the plain kernel's with the room for a copy and, in the tiles that need none, without it."""
+    room = cabi.lib().tmq_linear_scratch_bytes(m, n, k, 0)
+    assert room > 0
+    say("ragged tiles, room", m, n, k)
+    c = _tile_case(m, n, k, seed=m + n + k, x_signed=bool(m & 1), relu=False, bias=True, per_channel=True)
+    want, _, _ = _run(cabi, c, 9)
+    keep = cabi.linear_workspace
+    try:
+        for given in (None, torch.empty(room, dtype=torch.uint8, device="cuda")):
+            cabi.linear_workspace = given
+            got, _, _ = _run(cabi, c, -1)
+            np.testing.assert_array_equal(got, want)
+    finally:
+        cabi.linear_workspace = keep

@@ -1482,7 +1482,8 @@ bool wloop_ragged_copied(int64_t M, int64_t N, int64_t K) { return wloop_tile(M,
 // N = 8000, M = 4096 26.3 | 22.1).
 enum class RaggedTile { kCopy, k64, k64x128, k128, k128x256 };
 constexpr int64_t kRaggedLargeMaxTiles = 4096, kRaggedLargeMaxK = 4000, kRagged128MaxK = 3300, kRagged128FewRowsMaxK = 2000;
-RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
+// room: for the copy; without it the larger tiles take the last two kinds of shapes as well.
+RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats, bool room) {
   if (K < 16 || K > 0x7fffff00) return RaggedTile::kCopy;
   if (M <= kDecodeMaxRows && small_rows_path(M, N, regrid_pitch(K), true) == SmallRows::kStream) return RaggedTile::kCopy;
   const int64_t rows64 = ceil_div(M, 64), rows128 = ceil_div(M, 128);
@@ -1490,14 +1491,14 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
   const bool one128 = rows128 * ceil_div(N, 128) <= 256;
   // (at least 96 rows and 384 channels: fewer are padding in the larger tiles, 9974 x 296 -> 289 8.1 | 8.5)
   if (tiles > 256 && tiles <= kRaggedLargeMaxTiles && M >= 96 && N >= 384 && K > 2 * kBK &&
-      K <= (oblong <= 256 ? kRaggedLargeMaxK : M > (one128 ? 256 : 512) ? kRagged128MaxK : kRagged128FewRowsMaxK)) {
+      K <= (oblong <= 256 ? kRaggedLargeMaxK : M > (one128 || !room ? 256 : 512) ? kRagged128MaxK : kRagged128FewRowsMaxK)) {
     if (oblong <= 256) {
       if (K > (floats ? 1536 : 1200)) return RaggedTile::k64x128;
     } else if (one128) {
       if (K > 640 || oblong > (K > 330 && !floats ? 288 : 370)) return RaggedTile::k128;
     } else if (rows128 * ceil_div(N, 256) <= 256) {
       return K >= 480 || oblong > 700 ? RaggedTile::k128x256 : RaggedTile::k64x128;
-    } else if (K >= 250 && K <= 640 && (floats || K <= 400 || ceil_div(M, 256) * ceil_div(N, 256) <= 200)) {
+    } else if (K >= 250 && K <= 640 && (floats || !room || K <= 400 || ceil_div(M, 256) * ceil_div(N, 256) <= 200)) {
       return RaggedTile::k128;
     }
   }
@@ -1507,13 +1508,15 @@ RaggedTile ragged_tile(int64_t M, int64_t N, int64_t K, bool floats) {
 // ... and where the copy comes before 64 x 64 tiles, if there is room for it: K so long that the padded shape's kernel earns it back (two
 // layers, quantize and dequantize as a program calls them, direct | copy, us; 64 x 128 tiles in a ring: 600 x 6001 -> 2000
 // 45.3 | 34.6).  One round of tiles of 32 rows against K > 4096 reads the rows in place where there is no room (wloop_ragged_tile),
-// which is faster still and needs none; a caller that gives the room tmq_linear_scratch_bytes names has them copied.
+// which operators leave out there: a caller that gives the room tmq_linear_scratch_bytes names has them copied.  Copied over in place on
+// the device, 188 drawn shapes of more than 32 rows: even K 1.06 to 1.13 of the time by range of K, odd K 1.06 to 1.10 up to 6000, level up to
+// 8000, 0.93 to 0.97 beyond (0.81 to 1.28 there); the copy's launch and memory are the host's besides.
 bool ragged_copy_first(int64_t M, int64_t N, int64_t K) {
   const int64_t pitch = regrid_pitch(K);
   return wloop_tile(M, N, pitch) != 0 || (K >= 2304 && oblong_ring_first(M, N, pitch, pitch));
 }
 RaggedTile ragged_route(int64_t M, int64_t N, int64_t K, bool floats, bool copy_ok) {
-  const RaggedTile tile = ragged_tile(M, N, K, floats);
+  const RaggedTile tile = ragged_tile(M, N, K, floats, copy_ok);
   return tile == RaggedTile::k64 && copy_ok && ragged_copy_first(M, N, K) ? RaggedTile::kCopy : tile;
 }
 
