@@ -162,7 +162,8 @@ int tmq_quantize_rows_dynamic_dev(const float* x, void* q, int64_t M, int64_t K,
                                   int reduce_range, int rounding, tmq_qparams* qparams,
                                   void* workspace, size_t workspace_bytes, tmq_stream_t stream);
 /* The launch that exchanges ranges, pinned, for tests: at most `blocks` workgroups, of which each reads the others'
- * ranges polls + 1 times before it finds a missing one itself.  pitch == K: M * K values in a row.
+ * ranges polls + 1 times before it finds the missing ones itself, looking once between two of them.
+ * pitch == K: M * K values in a row.
  * TMQ_ERR_UNSUPPORTED where the calls above take other kernels whatever the size. */
 int tmq_quantize_dynamic_exchange(const float* x, void* q, int64_t M, int64_t K, int64_t pitch, int q_signed,
                                   int reduce_range, int rounding, tmq_qparams* qparams, void* workspace,
@@ -402,7 +403,7 @@ int tmq_linear_dynamic_small_takes(int64_t M, int64_t N, int64_t K);
 /* The same for more than 16 rows that make one round of tiles: bytes of `workspace`
  * the call needs (0: none), or -1 where the size is not such a one. */
 int64_t tmq_linear_dynamic_tiles_workspace(int64_t M, int64_t N, int64_t K);
-/* polls: of the other blocks' ranges, before a block finds a missing one itself
+/* polls: of the other blocks' ranges, before a block finds the missing ones itself
  * (negative: the default).  TMQ_ERR_UNSUPPORTED for other sizes, too little
  * workspace, and more than 32 rows on a stream that is being captured. */
 int tmq_linear_dynamic_tiles(const tmq_linear_desc* desc, const float* x, int64_t ldx, int reduce_range, float* y,
